@@ -27,6 +27,12 @@ int ncnn_moe_hip_sampler_debug_stream_only(
  * a kernel of their own before the replay, which then adds such a chunk in one step; off, the replay runs every chunk's
  * round itself.  Same results either way. */
 int ncnn_moe_hip_sampler_debug_chunk_steps(ncnn_moe_hip_sampler* sampler, int enabled);
+/* binned_sums (in this build off by default, so that the tests of the sort reach it; on in the shipped library): fp32 rows
+ * with no Top-K window, and rows of either type with one of 65 or more, are served without an order of their logits
+ * (sampler_bins.h); what that path leaves is sorted.  Same results either way.  binned_rows copies out, for the handle's
+ * first `rows` rows, 1 for a row that was finished that way the last time it was given to it. */
+int ncnn_moe_hip_sampler_debug_binned_sums(ncnn_moe_hip_sampler* sampler, int enabled);
+int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32_t* served, uint32_t rows);
 /* spread_sort (on by default): the radix sort of a long full-order row runs on several workgroups; off,
  * every row is sorted by one workgroup. */
 int ncnn_moe_hip_sampler_debug_spread_sort(ncnn_moe_hip_sampler* sampler, int enabled);

@@ -15,6 +15,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 using namespace ncnn_moe_hip;
@@ -37,6 +38,7 @@ struct ncnn_moe_hip_sampler
     hipEvent_t cut_done = nullptr;
     hipStream_t stream = nullptr;
 
+    void* device_memory = nullptr; // every device buffer below
     void* logits = nullptr;
     int logits_dtype = NCNN_MOE_LOGITS_F32;
     uint32_t logits_rows = 0;
@@ -79,6 +81,16 @@ struct ncnn_moe_hip_sampler
     uint32_t term_sum_parts = 0;
     uint32_t chunk_capacity = 0;
     int chunk_steps_enabled = 1;
+
+    BinArgs bins{};             // scratch of the binned sums (sampler_bins.h)
+    WindowArgs windows{};       // ... and of the window kernels (sampler_windows.h)
+    uint32_t* bin_list = nullptr;
+    uint32_t* window_list = nullptr;
+#ifdef NCNN_MOE_TESTING
+    int binned_sums = 0;        // (the tests of the sort reach it first)
+#else
+    int binned_sums = 1;        // rows that the first select leaves go to the binned sums first
+#endif
 
     int32_t* distribution_ids = nullptr;
     float* distribution_probabilities = nullptr;
@@ -279,6 +291,35 @@ struct SamplerPasses
     bool side_by_side = false; // the wide select on the handle's second stream, beside the full-order kernels
 };
 
+// Enqueues what follows the first select: the window kernels (sampler_windows.h) and the binned sums (sampler_bins.h) for
+// the rows that it left pending; by_options: for those that it leaves by their options.
+template <int DTYPE>
+void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool sums, bool by_options, hipStream_t stream)
+{
+    hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, by_options ? 1u : 0u,
+                       windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
+    if (windows)
+    {
+        WindowArgs w = s->windows;
+        w.a = a;
+        w.windows_are_selects = 1u;
+        hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
+        hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
+    }
+    if (sums)
+    {
+        BinArgs g = s->bins;
+        g.a = a;
+        g.windows_are_selects = windows ? 1u : 0u;
+        hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
+        hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
+        hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
+        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 0>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 1>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+    }
+}
+
 // Enqueues the sampling path for `rows` rows.
 int launch_sampler(
     ncnn_moe_hip_sampler* s, const void* logits, int dtype, uint32_t rows, uint32_t vocab, uint64_t row_stride,
@@ -335,6 +376,36 @@ int launch_sampler(
     const uint32_t sort_tiles = static_cast<uint32_t>((static_cast<uint64_t>(vocab) + kSortTile - 1) / kSortTile);
     const uint32_t sort_tiles_per_part = std::max<uint32_t>(1, (sort_tiles + kMaxSortParts - 1) / kMaxSortParts);
     const uint32_t sort_parts = std::max<uint32_t>(1, (sort_tiles + sort_tiles_per_part - 1) / sort_tiles_per_part);
+    // Rows with a window of 65 to 1024 go to the window kernels, fp32 rows without one to the binned sums (bf16 rows have a
+    // kernel of their own); what they leave pending goes to the full-order kernels.  A call that exports distributions
+    // needs the order itself.
+    const bool windows = passes.wide_select && vocab <= kWindowMaxVocab;
+    const bool sums = passes.full_order && dtype == NCNN_MOE_LOGITS_F32 && vocab <= kBinMaxVocab;
+    if (s->binned_sums != 0 && passes.select && !want_distribution && (windows || sums) && windows == passes.wide_select)
+    {
+        if (dtype == NCNN_MOE_LOGITS_F32)
+        {
+            launch_select<NCNN_MOE_LOGITS_F32>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
+            launch_later_rows<NCNN_MOE_LOGITS_F32>(s, a, windows, sums, passes.side_by_side, stream);
+        }
+        else
+        {
+            launch_select<NCNN_MOE_LOGITS_BF16>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
+            launch_later_rows<NCNN_MOE_LOGITS_BF16>(s, a, windows, false, passes.side_by_side, stream);
+        }
+        if (passes.full_order)
+        {
+            if (dtype == NCNN_MOE_LOGITS_F32)
+            {
+                hipLaunchKernelGGL((general_sort_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kSortThreads), 0, stream, a);
+                hipLaunchKernelGGL((general_replay_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kReplayThreads), 0, stream, a);
+            }
+            else
+                hipLaunchKernelGGL(bf16_counting_replay_kernel, dim3(rows), dim3(kSortThreads), 0, stream, a);
+        }
+        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        return NCNN_MOE_SAMPLER_SUCCESS;
+    }
     // fp32 rows whose sort is spread over the GPU are sorted only as far as their terms can move a sum
     // (full_order_cut_kernel); a row whose replay finds that guess too short stays pending, and a second launch of
     // the full-order kernels, behind the first, sorts it whole.
@@ -627,7 +698,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     s->max_segments = static_cast<uint32_t>(std::min<uint64_t>(
         static_cast<uint64_t>(kMaxSegments), (static_cast<uint64_t>(max_vocab) + 7 + kSegmentValuesF32 - 1) / kSegmentValuesF32));
     s->logits_stride_f32 = round_up(max_vocab, 8);
-    s->sort_stride = round_up(max_vocab, 4);
+    s->sort_stride = round_up(static_cast<uint64_t>(max_vocab) + 16, 8); // (the binned sums keep a row's terms from its 16-byte boundary on)
 
     auto destroy_and_return = [&](hipError_t error, const char* what) {
         std::fprintf(stderr, "ncnn_moe_hip_sampler_create: %s: %s\n", what, hipGetErrorString(error));
@@ -650,10 +721,89 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     CREATE_CHECK(hipEventCreateWithFlags(&s->cut_done, hipEventDisableTiming));
     const size_t rows = max_rows;
     const size_t slots = rows * s->max_segments;
-    CREATE_CHECK(hipMalloc(&s->logits, rows * s->logits_stride_f32 * sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->params, rows * sizeof(ncnn_moe_sample_params)));
-    CREATE_CHECK(hipMalloc(&s->uniforms, rows * sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->results, rows * sizeof(ncnn_moe_sample_result)));
+    // Device memory comes in one allocation (some forty buffers; an allocation of its own for each took half of the time
+    // that a handle takes to create), the buffers that a launch expects to find at zero side by side at its front.
+    size_t bytes = 0;
+    std::vector<std::pair<void**, size_t>> buffers;
+    const auto place = [&bytes, &buffers](auto** pointer, size_t size) {
+        buffers.emplace_back(reinterpret_cast<void**>(pointer), bytes);
+        bytes += round_up(std::max<size_t>(size, 1), 256);
+    };
+    // split path: records start untagged (epoch 0 tags nothing), every row at epoch 1
+    const size_t split_rows = std::min<size_t>(rows, static_cast<size_t>(kWholeRowBatch) - 1);
+    place(&s->split_records, split_rows * kSplitMaxSegments * kSplitRecordSlots * sizeof(unsigned long long));
+    place(&s->segment_counts, slots * sizeof(uint32_t));
+    place(&s->row_counter, rows * sizeof(unsigned long long));
+    place(&s->row_flags, rows * sizeof(uint32_t));
+    place(&s->row_state, rows * sizeof(uint32_t));
+    place(&s->windows.counts, rows * sizeof(uint32_t));
+    place(&s->windows.flags, rows * sizeof(uint32_t));
+    const size_t cleared = bytes;
+    place(&s->row_epoch, rows * sizeof(uint32_t));
+    place(&s->logits, rows * s->logits_stride_f32 * sizeof(float));
+    place(&s->params, rows * sizeof(ncnn_moe_sample_params));
+    place(&s->uniforms, rows * sizeof(float));
+    place(&s->results, rows * sizeof(ncnn_moe_sample_result));
+    place(&s->segment_values, slots * kSegmentRecordSlots * sizeof(float));
+    place(&s->segment_indices, slots * kSegmentRecordSlots * sizeof(int32_t));
+    for (int i = 0; i < 2; ++i)
+    {
+        place(&s->sort_keys[i], rows * s->sort_stride * sizeof(uint32_t));
+        place(&s->sort_indices[i], rows * s->sort_stride * sizeof(uint32_t));
+    }
+    place(&s->row_list, (rows + 1) * sizeof(uint32_t));
+    place(&s->sort_cuts, 4 * rows * sizeof(uint32_t));
+    place(&s->sort_part_counts, rows * kMaxSortParts * 256 * sizeof(uint32_t));
+    s->term_sum_parts = (max_vocab + kTermsThreads * kTermsPerThread - 1) / (kTermsThreads * kTermsPerThread);
+    s->chunk_capacity = max_vocab / kReplayChunk + 1;
+    place(&s->term_sums, rows * s->term_sum_parts * sizeof(double));
+    place(&s->chunk_steps, rows * s->chunk_capacity * sizeof(uint4));
+    place(&s->distribution_ids, static_cast<size_t>(max_vocab) * sizeof(int32_t));
+    place(&s->distribution_probabilities, static_cast<size_t>(max_vocab) * sizeof(float));
+    place(&s->distribution_count, sizeof(uint32_t));
+    constexpr size_t kVerifyRows = 2 * NCNN_MOE_MAX_DRAFT_TOKENS + 1;
+    place(&s->verify_ids, kVerifyRows * kVerifyCap * sizeof(int32_t));
+    place(&s->verify_probabilities, kVerifyRows * kVerifyCap * sizeof(float));
+    place(&s->verify_counts, kVerifyRows * sizeof(uint32_t));
+    // lists that hold whole rows and two dense vectors over the vocabulary, for steps whose filtered
+    // distributions are longer than kVerifyCap (a handle for fewer rows than a step needs never gets there)
+    if (max_rows >= 3)
+    {
+        const size_t long_rows = std::min<size_t>(kVerifyRows, rows);
+        place(&s->verify_long_ids, long_rows * max_vocab * sizeof(int32_t));
+        place(&s->verify_long_probabilities, long_rows * max_vocab * sizeof(float));
+        place(&s->verify_dense, 2 * static_cast<size_t>(max_vocab) * sizeof(float));
+    }
+    place(&s->single_params, sizeof(ncnn_moe_sample_params));
+    place(&s->single_uniform, sizeof(float));
+    place(&s->single_result, sizeof(ncnn_moe_sample_result));
+    // the binned sums: a launch covers its rows with kBinGrid workgroups, at most kMaxBinParts a row and at least one
+    const size_t pairs = std::max<size_t>(rows, std::min<size_t>(kBinGrid, rows * kMaxBinParts));
+    place(&s->bin_list, (rows + 1) * sizeof(uint32_t));
+    place(&s->bins.records, rows * sizeof(BinRow));
+    place(&s->bins.stats, pairs * sizeof(uint4));
+    place(&s->bins.counts, pairs * 2 * kBins * sizeof(uint32_t));
+    place(&s->bins.head_terms, rows * kBinListCap * sizeof(float));
+    place(&s->bins.head_tokens, rows * kBinListCap * sizeof(uint32_t));
+    for (int i = 0; i < 2; ++i)
+    {
+        place(&s->bins.steps[i], pairs * kBins * sizeof(uint32_t));
+        place(&s->bins.ties[i], pairs * 3 * kBinWords * sizeof(uint32_t));
+        place(&s->bins.masks[i], pairs * 2 * kBins * sizeof(uint32_t));
+        place(&s->bins.packed[i], rows * kBins * sizeof(uint32_t));
+        place(&s->bins.list_terms[i], rows * kBinListCap * sizeof(float));
+        place(&s->bins.list_tokens[i], rows * kBinListCap * sizeof(uint32_t));
+    }
+    place(&s->window_list, (rows + 1) * sizeof(uint32_t));
+    place(&s->windows.keys, rows * kWindowListCap * sizeof(uint32_t));
+    place(&s->windows.tokens, rows * kWindowListCap * sizeof(uint32_t));
+    CREATE_CHECK(hipMalloc(&s->device_memory, bytes));
+    for (const auto& [pointer, offset] : buffers)
+        *pointer = static_cast<uint8_t*>(s->device_memory) + offset;
+    s->bins.list = s->bin_list;
+    s->windows.list = s->window_list;
+    CREATE_CHECK(hipMemsetAsync(s->device_memory, 0, cleared, s->stream));
+    CREATE_CHECK(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(s->row_epoch), 1, rows, s->stream));
     s->input_uniforms_offset = rows * sizeof(ncnn_moe_sample_params);
     s->input_stops_offset = s->input_uniforms_offset + rows * sizeof(float);
     // room for stop ids: 64 per row, or one list as long as the vocabulary, whichever is more
@@ -663,58 +813,11 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->input_block_mapped), s->input_block_host, 0));
     CREATE_CHECK(hipHostMalloc(&s->results_host, rows * sizeof(ncnn_moe_sample_result), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->results_host_device), s->results_host, 0));
-    CREATE_CHECK(hipMalloc(&s->segment_values, slots * kSegmentRecordSlots * sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->segment_indices, slots * kSegmentRecordSlots * sizeof(int32_t)));
-    CREATE_CHECK(hipMalloc(&s->segment_counts, slots * sizeof(uint32_t)));
-    CREATE_CHECK(hipMalloc(&s->row_counter, rows * sizeof(unsigned long long)));
-    CREATE_CHECK(hipMalloc(&s->row_flags, rows * sizeof(uint32_t)));
-    CREATE_CHECK(hipMalloc(&s->row_state, rows * sizeof(uint32_t)));
-    // split path: records start untagged (epoch 0 tags nothing), every row at epoch 1
-    const size_t split_rows = std::min<size_t>(rows, static_cast<size_t>(kWholeRowBatch) - 1);
-    CREATE_CHECK(hipMalloc(&s->split_records, split_rows * kSplitMaxSegments * kSplitRecordSlots * sizeof(unsigned long long)));
-    CREATE_CHECK(hipMemset(s->split_records, 0, split_rows * kSplitMaxSegments * kSplitRecordSlots * sizeof(unsigned long long)));
-    CREATE_CHECK(hipMalloc(&s->row_epoch, rows * sizeof(uint32_t)));
-    CREATE_CHECK(hipMemsetD32(reinterpret_cast<hipDeviceptr_t>(s->row_epoch), 1, rows));
-    CREATE_CHECK(hipMemset(s->segment_counts, 0, slots * sizeof(uint32_t)));
-    CREATE_CHECK(hipMemset(s->row_counter, 0, rows * sizeof(unsigned long long)));
-    CREATE_CHECK(hipMemset(s->row_flags, 0, rows * sizeof(uint32_t)));
-    CREATE_CHECK(hipMemset(s->row_state, 0, rows * sizeof(uint32_t)));
-    for (int i = 0; i < 2; ++i)
-    {
-        CREATE_CHECK(hipMalloc(&s->sort_keys[i], rows * s->sort_stride * sizeof(uint32_t)));
-        CREATE_CHECK(hipMalloc(&s->sort_indices[i], rows * s->sort_stride * sizeof(uint32_t)));
-    }
-    CREATE_CHECK(hipMalloc(&s->row_list, (static_cast<size_t>(rows) + 1) * sizeof(uint32_t)));
-    CREATE_CHECK(hipMalloc(&s->sort_cuts, 4 * static_cast<size_t>(rows) * sizeof(uint32_t)));
-    CREATE_CHECK(hipMalloc(&s->sort_part_counts, rows * kMaxSortParts * 256 * sizeof(uint32_t)));
-    s->term_sum_parts = (max_vocab + kTermsThreads * kTermsPerThread - 1) / (kTermsThreads * kTermsPerThread);
-    s->chunk_capacity = max_vocab / kReplayChunk + 1;
-    CREATE_CHECK(hipMalloc(&s->term_sums, rows * s->term_sum_parts * sizeof(double)));
-    CREATE_CHECK(hipMalloc(&s->chunk_steps, rows * s->chunk_capacity * sizeof(uint4)));
-    CREATE_CHECK(hipMalloc(&s->distribution_ids, static_cast<size_t>(max_vocab) * sizeof(int32_t)));
-    CREATE_CHECK(hipMalloc(&s->distribution_probabilities, static_cast<size_t>(max_vocab) * sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->distribution_count, sizeof(uint32_t)));
-    constexpr size_t kVerifyRows = 2 * NCNN_MOE_MAX_DRAFT_TOKENS + 1;
-    CREATE_CHECK(hipMalloc(&s->verify_ids, kVerifyRows * kVerifyCap * sizeof(int32_t)));
-    CREATE_CHECK(hipMalloc(&s->verify_probabilities, kVerifyRows * kVerifyCap * sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->verify_counts, kVerifyRows * sizeof(uint32_t)));
-    // lists that hold whole rows and two dense vectors over the vocabulary, for steps whose filtered
-    // distributions are longer than kVerifyCap (a handle for fewer rows than a step needs never gets there)
-    if (max_rows >= 3)
-    {
-        const size_t long_rows = std::min<size_t>(kVerifyRows, rows);
-        CREATE_CHECK(hipMalloc(&s->verify_long_ids, long_rows * max_vocab * sizeof(int32_t)));
-        CREATE_CHECK(hipMalloc(&s->verify_long_probabilities, long_rows * max_vocab * sizeof(float)));
-        CREATE_CHECK(hipMalloc(&s->verify_dense, 2 * static_cast<size_t>(max_vocab) * sizeof(float)));
-    }
     CREATE_CHECK(hipHostMalloc(&s->verify_input_host, sizeof(ncnn_moe_hip_sampler::VerifyInput), hipHostMallocDefault));
     CREATE_CHECK(hipHostMalloc(&s->verify_output_host, sizeof(ncnn_moe_hip_sampler::VerifyOutput), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->verify_input_mapped), s->verify_input_host, 0));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->verify_output_mapped), s->verify_output_host, 0));
-    CREATE_CHECK(hipMalloc(&s->single_params, sizeof(ncnn_moe_sample_params)));
-    CREATE_CHECK(hipMalloc(&s->single_uniform, sizeof(float)));
-    CREATE_CHECK(hipMalloc(&s->single_result, sizeof(ncnn_moe_sample_result)));
-    CREATE_CHECK(hipDeviceSynchronize());
+    CREATE_CHECK(hipStreamSynchronize(s->stream));
 #undef CREATE_CHECK
     *out = s;
     return NCNN_MOE_SAMPLER_SUCCESS;
@@ -741,17 +844,8 @@ void ncnn_moe_hip_sampler_destroy(ncnn_moe_hip_sampler* s)
         (void)hipEventDestroy(s->side_join);
     if (s->cut_done != nullptr)
         (void)hipEventDestroy(s->cut_done);
-    void* buffers[] = {
-        s->logits, s->params, s->uniforms, s->results, s->segment_values, s->segment_indices,
-        s->segment_counts, s->row_counter, s->row_flags, s->row_state, s->split_records, s->row_epoch, s->sort_keys[0], s->sort_keys[1],
-        s->sort_indices[0], s->sort_indices[1], s->sort_part_counts, s->row_list, s->sort_cuts, s->term_sums, s->chunk_steps, s->distribution_ids, s->distribution_probabilities,
-        s->distribution_count, s->single_params, s->single_uniform, s->single_result, s->verify_ids,
-        s->verify_probabilities, s->verify_counts, s->verify_long_ids, s->verify_long_probabilities, s->verify_dense};
-    for (void* buffer : buffers)
-    {
-        if (buffer != nullptr)
-            (void)hipFree(buffer);
-    }
+    if (s->device_memory != nullptr)
+        (void)hipFree(s->device_memory);
     if (s->input_block_host != nullptr)
         (void)hipHostFree(s->input_block_host);
     if (s->results_host != nullptr)
@@ -1205,6 +1299,28 @@ int ncnn_moe_hip_sampler_debug_force_general(ncnn_moe_hip_sampler* s, int enable
     if (s == nullptr)
         return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
     s->force_general = enabled ? 1 : 0;
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+int ncnn_moe_hip_sampler_debug_binned_sums(ncnn_moe_hip_sampler* s, int enabled)
+{
+    if (s == nullptr)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    s->binned_sums = enabled ? 1 : 0;
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+// Which of the handle's first `rows` rows the binned sums finished the last time that they were given them.
+int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* s, uint32_t* served, uint32_t rows)
+{
+    if (s == nullptr || served == nullptr || rows > s->max_rows)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
+    SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+    std::vector<BinRow> records(rows);
+    SAMPLER_HIP_CHECK(s, hipMemcpy(records.data(), s->bins.records, rows * sizeof(BinRow), hipMemcpyDeviceToHost));
+    for (uint32_t row = 0; row < rows; ++row)
+        served[row] = records[row].served;
     return NCNN_MOE_SAMPLER_SUCCESS;
 }
 

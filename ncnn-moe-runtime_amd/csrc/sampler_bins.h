@@ -1,0 +1,2095 @@
+// Binned sums: the sampler's walk over a row whose order is never worked out.
+//
+// The CPU sampler adds the row's terms exp(logit/T - max) one by one in descending order, three times over (the
+// normaliser, the Top-P walk, the draw), and every partial sum is rounded to fp32.  While such a sum stays inside one
+// binade its mantissa grows by round(term / ulp) per term, which depends on the sum in one case only: a term that ends
+// exactly half an ulp above a multiple of it.  So the terms of a stretch of the sorted row in which the sum neither
+// leaves its binade nor meets such a term may be added in any order, as integers.  The rows served here (no Top-K
+// window, or one wider than the first select's) are therefore not sorted:
+//   * the terms fall into kBins bins by their bit pattern (0.4 to 0.8 % of a term wide; bins follow the sorted order);
+//   * the head of the row (the bins of its first few thousand elements) is sorted in LDS and added exactly as the
+//     CPU does, which takes the sum through most of its binades;
+//   * every other bin is one integer: the sum of its terms' steps at the exponent that the running sum will have there;
+//   * the few bins in which the order matters - the sum leaves its binade, a stop condition is met, the window or the
+//     Min-P cut ends - are fetched element by element and sorted: those that can be foreseen from the bins' masses by the
+//     pass that adds the others, the rest on demand by a pass over the row's terms;
+//   * a term that lies half way between two sums is rounded by the parity of the sum in front of it, which follows from
+//     the parities of the steps in front of it: between two such values every term of a bin has the same step, so one
+//     bit per step value and bin (the parity of the odd steps of that value) tells.
+// A term of 2^-25 or less never moves any of the three sums (the first term is 1, so half an ulp of the normaliser is
+// at least 2^-24; the other two sums start at the first term divided by the same numbers as every other): such terms
+// are in no bin.  A foreseen exponent is checked against the exact sum before a bin's integer is used.
+//
+// Five or six launches serve every row of a call, each workgroup a part of one row: (1) maximum and counts, (2) terms
+// and bin counts, (3) head fetched, steps of the normaliser's sum, (4) normaliser walked, steps of the Top-P sum,
+// (5) Top-P walked, steps of the draw's sum, (6) draw walked.  A row whose walks end inside its head is finished by (4).
+//
+// What bounds it: at few rows the chain of launches and, inside (4) to (6), the walk (some 5 to 10 us each, LDS and
+// dependent instructions); at a hundred rows and more the instructions per logit (some 40 for the exponential and its
+// bin, 25 to 40 for a step).
+#ifndef NCNN_MOE_HIP_SAMPLER_BINS_H
+#define NCNN_MOE_HIP_SAMPLER_BINS_H
+
+#include "sampler_full_order.h"
+
+namespace ncnn_moe_hip {
+
+constexpr int kBinThreads = 1024;
+constexpr int kBinWaves = kBinThreads / kWaveSize;
+constexpr int kWalkThreads = 512;                // the walk: half the waves cost half of what every wave of it does
+constexpr int kWalkWaves = kWalkThreads / kWaveSize;
+constexpr uint32_t kBinsPerBinade = 64;
+constexpr uint32_t kBinBinades = 25;
+constexpr uint32_t kBins = kBinBinades * kBinsPerBinade;
+constexpr uint32_t kBinWords = kBins / 32;
+constexpr uint32_t kBinQuads = kBins / 4;        // a thread of the row's scan holds four consecutive bins
+constexpr uint32_t kOneBits = 0x3f800000u;       // the largest term
+constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms of 2^-25 or less move no sum
+constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
+constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
+constexpr uint32_t kBinHead = 3072;              // elements of the sorted head at most (unless one bin or a window takes more) ...
+constexpr uint32_t kBinHeadDense = 1024;         // ... behind this many it takes only bins of
+constexpr uint32_t kBinHeadBin = 48;             // ... this many elements at most: dense bins cost their ordering and save little
+constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
+constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
+constexpr uint32_t kBinStops = 512;
+constexpr int kMaskedDifference = 14;            // so many binades below the sum a bin's terms (within a 64th of each other) take 18 different steps at most
+constexpr uint32_t kBinRequests = 64;            // ... and how often per walk
+constexpr uint32_t kMaxBinParts = 16;
+constexpr uint32_t kPartsAtATime = 8;            // loads of the parts' numbers in flight together
+constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
+constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
+constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
+constexpr float kForeseenFirst = 4e-4f;          // relative error allowed for the sums foreseen from the bins' masses
+constexpr float kForeseenLater = 4e-4f;          // ... and from the steps of the sum before
+static_assert(kBinQuads <= kWalkThreads && kBinListCap % kWalkThreads == 0 && kBinListCap <= 64 * kWaveSize, "the walk's thread and lane counts");
+
+// A bin as the walk sees it: kind (2 bits), biased exponent assumed for the running sum (8), elements in front of it (22).
+constexpr uint32_t kBinAdded = 0u;  // its elements' steps are added as one integer
+constexpr uint32_t kBinListed = 1u; // its elements are in the list
+constexpr uint32_t kBinBeyond = 2u; // behind the end of the sum
+constexpr uint32_t kBinWanted = 3u; // its elements are needed and not in the list: fetched on demand
+
+__device__ __forceinline__ uint32_t packed_kind(uint32_t packed) { return packed >> 30; }
+__device__ __forceinline__ uint32_t packed_exponent(uint32_t packed) { return (packed >> 22) & 0xffu; }
+__device__ __forceinline__ uint32_t packed_front(uint32_t packed) { return packed & 0x3fffffu; }
+
+enum BinRowState : uint32_t
+{
+    kBinRowLeft = 0,  // not (or no longer) served here: finished, or left to the full-order kernels
+    kBinRowGoesOn = 1 // the next launch goes on with it
+};
+
+// What the launches of a call keep of a row.  A launch reads what earlier ones wrote and writes other words (its own
+// workgroups read the row's record at different times).
+struct BinRow
+{
+    uint32_t state[4];      // after launches (2), (3), (4), (5)
+    uint32_t shift;         // a term's bin: (kOneBits - bits) >> shift
+    uint32_t window;        // elements of the Top-K window (finite logits at most)
+    uint32_t binned;        // elements in bins
+    uint32_t saw_nan;
+    uint32_t head_bins;     // bins [0, head_bins) are the head, head_count elements
+    uint32_t head_count;
+    uint32_t listed[3];     // elements in the list of each walk (the first walk's holds the head, the others' places behind it)
+    float normalizer;
+    float head_sum[2];      // the Top-P sum and the draw's behind the head
+    uint32_t limit[2];      // elements that those sums run over at most
+    uint32_t cut_bin;       // Min-P: the bin that holds the smallest term kept (kBins: no cut inside the bins), and that term
+    float cut_term;
+    uint32_t cut_in_tail;   // ... or it lies in no bin
+    float renormalizer;
+    uint32_t kept;
+    uint32_t served;        // the row was finished here
+};
+
+struct BinArgs
+{
+    SamplerArgs a;
+    const uint32_t* list;  // the rows served: [0] their number, then the rows
+    uint4* stats;          // [pairs] (row, part): largest and smallest finite logit, finite logits, flags
+    uint32_t* counts;      // [pairs][2][kBins]: terms in each bin, and the sum of their places in it (kOffsetBits)
+    uint32_t* steps[2];    // [pairs][kBins], of alternate launches
+    uint32_t* ties[2];     // [pairs][3][kBinWords]: bins with terms half way, with two of one value, and with some that their masks cannot hold
+    uint32_t* masks[2];    // [pairs][2][kBins]: parities of the odd steps, and the values half way, by step (see add_bin_steps)
+    uint32_t* packed[2];   // [rows][kBins]
+    float* list_terms[2];  // [rows][kBinListCap]
+    uint32_t* list_tokens[2];
+    float* head_terms;     // [rows][kBinListCap], sorted
+    uint32_t* head_tokens;
+    BinRow* records;       // [rows]
+    uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
+};
+
+// How a launch's workgroups cover the listed rows: all parts of a row on one XCD (workgroups are dealt out to the XCDs
+// in turn), so that what one launch leaves of a row is found in that XCD's L2 by the next.
+struct BinGrid
+{
+    uint32_t rows, parts, first_slot, slot_step, part;
+};
+
+__device__ __forceinline__ BinGrid bin_grid(const uint32_t* list, uint32_t vocab)
+{
+    BinGrid r;
+    r.rows = list[0];
+    const uint32_t per_xcd = kBinGrid / 8u;
+    const uint32_t slots_per_xcd = max(1u, (r.rows + 7u) / 8u);
+    const uint32_t most = min(kMaxBinParts, (vocab + kBinPartElements - 1u) / kBinPartElements);
+    r.parts = max(1u, min(most, per_xcd / slots_per_xcd));
+    const uint32_t lanes = per_xcd / r.parts; // slots in flight on an XCD
+    const uint32_t within = blockIdx.x >> 3;
+    r.part = within % r.parts;
+    r.first_slot = within / r.parts < lanes ? (within / r.parts) * 8u + (blockIdx.x & 7u) : 0xffffffffu;
+    r.slot_step = lanes * 8u;
+    return r;
+}
+
+// The stretch of a row that a part covers, in groups of eight positions; positions count from the 16-byte boundary
+// below the row, and [misalignment, end) hold its logits.
+struct BinStretch
+{
+    uint32_t misalignment, end, first, last;
+};
+
+template <int ELEMENT_BYTES>
+__device__ __forceinline__ BinStretch bin_stretch(const SamplerArgs& a, uint32_t row, uint32_t part, uint32_t parts)
+{
+    const char* pointer = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * ELEMENT_BYTES;
+    BinStretch s;
+    s.misalignment = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(pointer) & 15u) / ELEMENT_BYTES;
+    s.end = s.misalignment + a.vocab;
+    const uint32_t groups = (s.end + 7u) / 8u;
+    const uint32_t each = (groups + parts - 1u) / parts;
+    s.first = min(groups, part * each);
+    s.last = min(groups, s.first + each);
+    return s;
+}
+
+__device__ __forceinline__ bool counts_as_select(uint32_t windows_are_selects, uint32_t vocab, const ncnn_moe_sample_params& p)
+{
+    const uint32_t window = p.top_k == 0u || p.top_k >= vocab ? vocab : p.top_k;
+    return windows_are_selects != 0u && window <= static_cast<uint32_t>(kSelectTopK);
+}
+
+__device__ __forceinline__ float* bin_terms(const SamplerArgs& a, uint32_t row)
+{
+    return reinterpret_cast<float*>(a.sort_indices[0] + row * a.sort_stride);
+}
+
+// ---- (1) largest and smallest finite logit, number of finite logits, NaN and +inf seen
+template <int DTYPE>
+__global__ __launch_bounds__(kBinThreads) void bin_stats_kernel(BinArgs g)
+{
+    using Vector = LogitsVector<DTYPE>;
+    constexpr uint32_t kWidth = Vector::kWidth;
+    constexpr int kLoads = 4;
+    __shared__ uint4 wave_stats[kBinWaves];
+    const SamplerArgs& a = g.a;
+    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const int tid = threadIdx.x;
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = g.list[1u + slot];
+        const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
+        const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
+            static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
+        const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
+        float largest = -INFINITY, smallest = INFINITY;
+        uint32_t finite = 0, flags = 0;
+        for (uint32_t at = first + tid; at < last; at += kLoads * kBinThreads)
+        {
+            uint4 raw[kLoads];
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k)
+            {
+                const uint32_t v = min(at + k * kBinThreads, last - 1u);
+                raw[k] = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u);
+            }
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k)
+            {
+                const uint32_t v = at + k * kBinThreads;
+                float x[kWidth];
+                Vector::unpack(raw[k], x);
+                const uint32_t position = v * kWidth;
+                const bool whole = v < last && position >= s.misalignment && position + kWidth <= s.end;
+#pragma unroll
+                for (uint32_t c = 0; c < kWidth; ++c)
+                {
+                    const bool inside = whole || (v < last && position + c >= s.misalignment && position + c < s.end);
+                    const uint32_t magnitude = __float_as_uint(x[c]) & 0x7fffffffu;
+                    const bool counts = inside && magnitude < 0x7f800000u;
+                    largest = fmaxf(largest, counts ? x[c] : -INFINITY);
+                    smallest = fminf(smallest, counts ? x[c] : INFINITY);
+                    finite += counts ? 1u : 0u;
+                    flags |= inside && magnitude > 0x7f800000u ? static_cast<uint32_t>(kScanSawNan) : 0u;
+                    flags |= inside && __float_as_uint(x[c]) == 0x7f800000u ? static_cast<uint32_t>(kScanSawPositiveInfinity) : 0u;
+                }
+            }
+        }
+#pragma unroll
+        for (int distance = kWaveSize / 2; distance > 0; distance >>= 1)
+        {
+            largest = fmaxf(largest, __shfl_xor(largest, distance, kWaveSize));
+            smallest = fminf(smallest, __shfl_xor(smallest, distance, kWaveSize));
+            finite += __shfl_xor(finite, distance, kWaveSize);
+            flags |= __shfl_xor(flags, distance, kWaveSize);
+        }
+        if ((tid & (kWaveSize - 1)) == 0)
+            wave_stats[tid >> 6] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
+        __syncthreads();
+        if (tid == 0)
+        {
+            for (int w = 1; w < kBinWaves; ++w)
+            {
+                const uint4 other = wave_stats[w];
+                largest = fmaxf(largest, __uint_as_float(other.x));
+                smallest = fminf(smallest, __uint_as_float(other.y));
+                finite += other.z;
+                flags |= other.w;
+            }
+            g.stats[slot * grid.parts + grid.part] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
+        }
+        __syncthreads();
+    }
+}
+
+// ---- (2) the terms, in the row's order, and how many fall into each bin
+template <int DTYPE>
+__global__ __launch_bounds__(kBinThreads) void bin_terms_kernel(BinArgs g)
+{
+    using Vector = LogitsVector<DTYPE>;
+    constexpr uint32_t kWidth = Vector::kWidth;
+    constexpr int kLoads = DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2;
+    __shared__ __align__(16) uint32_t bins[2 * kBins];
+    __shared__ uint4 part_stats[kMaxBinParts];
+    __shared__ uint64_t exp2_table[32];
+    const SamplerArgs& a = g.a;
+    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const int tid = threadIdx.x;
+    if (tid < 32)
+        exp2_table[tid] = kExp2Table[tid];
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = g.list[1u + slot];
+        const ncnn_moe_sample_params p = a.params[row];
+        if (tid < static_cast<int>(grid.parts))
+            part_stats[tid] = g.stats[slot * grid.parts + tid];
+        if (tid < static_cast<int>(2u * kBinQuads))
+            reinterpret_cast<uint4*>(bins)[tid] = uint4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        float largest = -INFINITY, smallest = INFINITY;
+        uint32_t finite = 0, flags = 0;
+        for (uint32_t q = 0; q < grid.parts; ++q)
+        {
+            const uint4 other = part_stats[q];
+            largest = fmaxf(largest, __uint_as_float(other.x));
+            smallest = fminf(smallest, __uint_as_float(other.y));
+            finite += other.z;
+            flags |= other.w;
+        }
+        const float maximum = largest / p.temperature;
+        const bool rejected = finite == 0u || (flags & kScanSawPositiveInfinity) != 0u;
+        const bool served = !rejected && is_finite_f32(maximum);
+        // (the bins cover the row's range of terms, or the 25 binades that matter)
+        const float least = fmaxf(smallest / p.temperature - maximum, kTailArgument);
+        uint32_t distance = served ? kOneBits - __float_as_uint(expf_libm(least, exp2_table)) : 0u;
+        distance = min(distance, kTailDistance - 1u);
+        uint32_t shift = 0;
+        while ((distance >> shift) >= kBins)
+            ++shift;
+        const uint32_t place_mask = (1u << shift) - 1u;
+        const uint32_t place_shift = shift > kOffsetBits ? shift - kOffsetBits : 0u;
+        if (grid.part == 0u && tid == 0)
+        {
+            BinRow& record = g.records[row];
+            record.state[0] = served ? kBinRowGoesOn : kBinRowLeft;
+            record.shift = shift;
+            record.window = (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite;
+            record.served = 0u;
+            record.saw_nan = (flags & kScanSawNan) != 0u ? 1u : 0u;
+            if (rejected)
+            {
+                // no finite logit, or +inf among them: the CPU sampler rejects the row
+                uint32_t row_flags = counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH);
+                if ((flags & kScanSawNan) != 0u)
+                    row_flags |= NCNN_MOE_ROW_FLAG_HAS_NAN;
+                write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, static_cast<uint8_t>(row_flags));
+                a.row_state[row] = kRowDone;
+            }
+        }
+        if (served)
+        {
+            const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
+            const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
+                static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
+            float* terms = bin_terms(a, row);
+            const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
+            for (uint32_t at = first + tid; at < last; at += kLoads * kBinThreads)
+            {
+                uint4 raw[kLoads];
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k)
+                {
+                    const uint32_t v = min(at + k * kBinThreads, last - 1u);
+                    raw[k] = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u);
+                }
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k)
+                {
+                    const uint32_t v = at + k * kBinThreads;
+                    if (v >= last)
+                        break;
+                    float x[kWidth], t[kWidth];
+                    Vector::unpack(raw[k], x);
+                    const uint32_t position = v * kWidth;
+#pragma unroll
+                    for (uint32_t c = 0; c < kWidth; ++c)
+                    {
+                        const float argument = x[c] / p.temperature - maximum;
+                        // (a comparison that NaN fails as well)
+                        const bool matters = argument >= kTailArgument && position + c >= s.misalignment && position + c < s.end;
+                        t[c] = matters ? expf_of_small_argument(argument, exp2_table) : 0.0f;
+                        const uint32_t below = kOneBits - __float_as_uint(t[c]);
+                        if (below < kTailDistance)
+                        {
+                            atomicAdd(&bins[below >> shift], 1u);
+                            atomicAdd(&bins[kBins + (below >> shift)], (below & place_mask) >> place_shift);
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t c = 0; c < kWidth; c += 4u)
+                        *reinterpret_cast<float4*>(terms + position + c) = float4{t[c], t[c + 1], t[c + 2], t[c + 3]};
+                }
+            }
+            // (the last group of eight positions of the row may reach a vector further than the row does)
+            if (kWidth == 4u && tid == 0 && s.last * 2u > last && last > first)
+                *reinterpret_cast<float4*>(terms + last * 4u) = float4{0.0f, 0.0f, 0.0f, 0.0f};
+            __syncthreads();
+            if (tid < static_cast<int>(2u * kBinQuads))
+                reinterpret_cast<uint4*>(g.counts + static_cast<size_t>(slot * grid.parts + grid.part) * 2u * kBins)[tid] = reinterpret_cast<uint4*>(bins)[tid];
+        }
+        __syncthreads();
+    }
+}
+
+// Exclusive prefix sums over the workgroup's threads (and the totals) of some integers and a float.
+struct BinScanScratch
+{
+    uint32_t u[4][kBinWaves];
+    float f[kBinWaves];
+};
+
+__device__ __forceinline__ float wave_prefix_sum_f32(float value)
+{
+#define NCNN_MOE_ADD_STAGE(CONTROL, ROW_MASK) value += __uint_as_float(dpp_source<CONTROL, ROW_MASK>(__float_as_uint(value)));
+    NCNN_MOE_ADD_STAGE(0x111, 0xf)
+    NCNN_MOE_ADD_STAGE(0x112, 0xf)
+    NCNN_MOE_ADD_STAGE(0x114, 0xf)
+    NCNN_MOE_ADD_STAGE(0x118, 0xf)
+    NCNN_MOE_ADD_STAGE(0x142, 0xa)
+    NCNN_MOE_ADD_STAGE(0x143, 0xc)
+#undef NCNN_MOE_ADD_STAGE
+    return value;
+}
+
+template <int WAVES, int COUNT>
+__device__ __forceinline__ void bin_scan(uint32_t (&u)[COUNT], uint32_t (&totals)[COUNT], float& f, BinScanScratch& scratch, int tid)
+{
+    const int lane = tid & (kWaveSize - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t own[COUNT];
+    uint32_t inclusive[COUNT];
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i)
+    {
+        own[i] = u[i];
+        inclusive[i] = wave_prefix_sum_u32(u[i]);
+        if (lane == kWaveSize - 1)
+            scratch.u[i][wave] = inclusive[i];
+    }
+    const float inclusive_f = wave_prefix_sum_f32(f);
+    if (lane == kWaveSize - 1)
+        scratch.f[wave] = inclusive_f;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i)
+    {
+        const uint32_t through = wave_prefix_sum_u32(lane < WAVES ? scratch.u[i][lane] : 0u);
+        totals[i] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), WAVES - 1));
+        const uint32_t before = wave > 0 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), wave - 1)) : 0u;
+        u[i] = before + inclusive[i] - own[i];
+    }
+    const float through = wave_prefix_sum_f32(lane < WAVES ? scratch.f[lane] : 0.0f);
+    const float before = wave > 0 ? read_lane(through, wave - 1) : 0.0f;
+    f = before + (inclusive_f - f);
+    __syncthreads();
+}
+
+// The largest term that a bin can hold (the lower end of a bin is the upper end of the next).
+__device__ __forceinline__ float bin_top(uint32_t bin, uint32_t shift)
+{
+    return __uint_as_float(kOneBits - (bin << shift));
+}
+
+// Plans a sum over the bins behind the head: what becomes of each of the calling thread's four bins (from `bin` on).
+//   front          elements in front of each bin; front[4] behind the last
+//   mass           about what the sum holds in front of each bin
+//   limit          elements that the sum runs over; cut_bin: no bin behind it takes part, and the sum may end inside it
+//   bound          the sum may end once it reaches this; error: relative error of the masses
+struct BinPlan
+{
+    uint32_t kind[4];
+    uint32_t exponent[4];
+    uint32_t ends;   // bit j: the sum ends inside bin j
+    uint32_t listed; // elements of the four bins that should be in the list
+};
+
+__device__ __forceinline__ BinPlan plan_bins(
+    uint32_t bin, const uint32_t (&front)[5], const float (&mass)[5], uint32_t head_bins, uint32_t limit, uint32_t cut_bin, float bound, float error)
+{
+    BinPlan plan;
+    plan.listed = 0;
+    plan.ends = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        const uint32_t b = bin + j;
+        const uint32_t count = front[j + 1] - front[j];
+        const float low = mass[j] * (1.0f - error);
+        const float high = mass[j + 1] * (1.0f + error);
+        plan.exponent[j] = (__float_as_uint(mass[j]) >> 23) & 0xffu;
+        uint32_t kind = kBinAdded;
+        if (b < head_bins || front[j] >= limit || b > cut_bin || low > bound)
+            kind = kBinBeyond;
+        else if (count > 0u)
+        {
+            const bool ends = front[j + 1] > limit || b == cut_bin;
+            const bool leaves = ((__float_as_uint(low) ^ __float_as_uint(high)) >> 23) != 0u;
+            plan.ends |= ends ? 1u << j : 0u;
+            if (ends || leaves || high >= bound)
+            {
+                kind = kBinListed;
+                plan.listed += count;
+            }
+        }
+        plan.kind[j] = kind;
+    }
+    return plan;
+}
+
+// Where the thread's listed bins lie in the list (base: the position of the first); a bin that does not fit is not listed.
+__device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&front)[5], uint32_t base, uint32_t (&place)[4])
+{
+    uint32_t position = base;
+    uint32_t end_of_list = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        place[j] = position;
+        if (plan.kind[j] == kBinListed)
+        {
+            position += front[j + 1] - front[j];
+            if (position > kBinListCap)
+                plan.kind[j] = (plan.ends >> j & 1u) != 0u ? kBinWanted : kBinAdded;
+            else
+                end_of_list = position;
+        }
+    }
+    return end_of_list;
+}
+
+// Elements of a bin in the parts in front of the calling one.
+__device__ __forceinline__ uint32_t count_in_front_parts(const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t bin)
+{
+    uint32_t before = 0;
+#pragma unroll
+    for (uint32_t q = 0; q + 1u < kMaxBinParts; ++q)
+    {
+        if (q < grid.part)
+            before += g.counts[static_cast<size_t>(slot * grid.parts + q) * 2u * kBins + bin];
+    }
+    return before;
+}
+
+// Adds the steps of a part's terms to the bins' integers, and puts the terms of listed bins into the list.
+//   entries   per bin: bit 31 the bin is listed and the rest is the next place of this part in the list; bit 30 it takes
+//             no part in the sum; else the exponent assumed for the sum
+//   ties      bins with a term half way between two sums (its step is counted rounded up), with a second one of the same
+//             value, and with one that the masks cannot tell (the bin's terms take more than 32 steps)
+//   masks     per bin, for terms kMaskedDifference binades and more below the sum: bit (step / 2) % 32 the parity of the
+//             odd steps of that value; then bit step % 32 for a term half way between `step` and the next
+template <int PHASE, int THREADS>
+__device__ __forceinline__ void add_bin_steps(
+    const float* terms, const BinStretch& s, uint32_t shift, uint32_t first_bin, uint32_t bin_count, float divisor, float second_divisor,
+    uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, float* list_terms, uint32_t* list_tokens, int tid)
+{
+    constexpr int kLoads = 4;
+    const uint32_t first = s.first * 2u, last = s.last * 2u;
+    for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
+    {
+        float4 raw[kLoads];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k)
+            raw[k] = reinterpret_cast<const float4*>(terms)[min(at + k * THREADS, last - 1u)];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k)
+        {
+            const uint32_t v = at + k * THREADS;
+            if (v >= last)
+                break;
+            const float t[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+            {
+                const uint32_t below = kOneBits - __float_as_uint(t[c]);
+                const uint32_t bin = below >> shift;
+                if (below >= kTailDistance || bin - first_bin >= bin_count)
+                    continue;
+                const uint32_t entry = entries[bin];
+                if ((entry & 0xc0000000u) == 0u)
+                {
+                    float term = t[c];
+                    if (PHASE >= 1)
+                        term = term / divisor;
+                    if (PHASE >= 2)
+                        term = term / second_divisor;
+                    const uint32_t bits = __float_as_uint(term);
+                    const uint32_t mantissa = (bits & 0x7fffffu) | 0x800000u;
+                    const int difference = static_cast<int>(entry) - static_cast<int>(bits >> 23);
+                    const uint32_t down = static_cast<uint32_t>(min(max(difference, 1), 25));
+                    const uint32_t half = 1u << (down - 1u);
+                    const uint32_t rest = mantissa & (2u * half - 1u);
+                    const uint32_t step = (mantissa + half) >> down;
+                    atomicAdd(&steps[bin], step);
+                    if ((rest == half) || difference < 1)
+                    {
+                        const uint32_t bit = 1u << (bin & 31u);
+                        atomicOr(&ties[bin >> 5], bit);
+                        if (difference < kMaskedDifference)
+                            atomicOr(&ties[2u * kBinWords + (bin >> 5)], bit);
+                        else if ((atomicOr(&masks[kBins + bin], 1u << ((step - 1u) & 31u)) >> ((step - 1u) & 31u) & 1u) != 0u)
+                            atomicOr(&ties[kBinWords + (bin >> 5)], bit);
+                    }
+                    else if ((step & 1u) != 0u)
+                        atomicXor(&masks[bin], 1u << ((step >> 1) & 31u));
+                }
+                else if ((entry & 0x80000000u) != 0u)
+                {
+                    const uint32_t place = atomicAdd(&entries[bin], 1u) & 0x7fffffffu;
+                    list_terms[place] = t[c];
+                    list_tokens[place] = v * 4u + c - s.misalignment;
+                }
+            }
+        }
+    }
+}
+
+// ---- (3) the head and the bins whose order is foreseen to matter go to the list; the others' steps of the normaliser
+__global__ __launch_bounds__(kBinThreads) void bin_sum_kernel(BinArgs g, uint32_t element_bytes)
+{
+    __shared__ __align__(16) uint32_t entries[kBins];
+    __shared__ __align__(16) uint32_t steps[kBins];
+    __shared__ __align__(16) uint32_t masks[2 * kBins];
+    __shared__ uint32_t ties[3 * kBinWords];
+    __shared__ BinScanScratch scan;
+    __shared__ uint32_t head_bins_of_row, head_count_of_row, end_of_list;
+    const SamplerArgs& a = g.a;
+    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const int tid = threadIdx.x;
+    const uint32_t bin = 4u * static_cast<uint32_t>(tid);
+    const bool holds_bins = tid < static_cast<int>(kBinQuads);
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = g.list[1u + slot];
+        BinRow& record = g.records[row];
+        if (record.state[0] != kBinRowGoesOn)
+        {
+            if (grid.part == 0u && tid == 0)
+                record.state[1] = kBinRowLeft;
+            continue;
+        }
+        const uint32_t shift = record.shift;
+        const uint32_t window = record.window;
+        // counts of the thread's bins, of the whole row and of the parts in front of this one, and their masses
+        uint32_t count[4] = {0u, 0u, 0u, 0u}, before[4] = {0u, 0u, 0u, 0u};
+        uint32_t places[4] = {0u, 0u, 0u, 0u};
+        if (holds_bins)
+        {
+            const uint4* counts = reinterpret_cast<const uint4*>(g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins) + tid;
+            for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
+            {
+                uint4 of_part[kPartsAtATime], place_sums[kPartsAtATime];
+#pragma unroll
+                for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                {
+                    const uint4* from = counts + static_cast<size_t>(min(first + k, grid.parts - 1u)) * 2u * kBinQuads;
+                    of_part[k] = from[0];
+                    place_sums[k] = from[kBinQuads];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                {
+                    const uint32_t some = first + k < grid.parts ? 0xffffffffu : 0u;
+                    const uint32_t some_before = first + k < grid.part ? 0xffffffffu : 0u;
+                    const uint32_t c[4] = {of_part[k].x, of_part[k].y, of_part[k].z, of_part[k].w};
+                    const uint32_t o[4] = {place_sums[k].x, place_sums[k].y, place_sums[k].z, place_sums[k].w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                    {
+                        count[j] += c[j] & some;
+                        before[j] += c[j] & some_before;
+                        places[j] += o[j] & some; // (a bin's places add up to less than 2^22 x 2^12: only a bin of a million terms wraps, a wrong guess)
+                    }
+                }
+            }
+        }
+        if (tid == 0)
+            head_bins_of_row = head_count_of_row = end_of_list = 0u;
+        if (holds_bins)
+            reinterpret_cast<uint4*>(steps)[tid] = uint4{0u, 0u, 0u, 0u};
+        if (tid < static_cast<int>(2u * kBinQuads))
+            reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
+        if (tid < static_cast<int>(3u * kBinWords))
+            ties[tid] = 0u;
+        // elements and mass in front of the thread's bins: first the plain masses, then what the sum makes of them (a term
+        // of few ulps of the sum is rounded, the same way all over a bin: up to half an ulp a term, thousands of them)
+        uint32_t front[5];
+        float mass[5];
+        uint32_t binned;
+        {
+            uint32_t total[1] = {count[0] + count[1] + count[2] + count[3]};
+            uint32_t totals[1];
+            float own[4];
+            float masses = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const float top = bin_top(bin + j, shift);
+                const float width = top - bin_top(bin + j + 1u, shift);
+                own[j] = count[j] == 0u ? 0.0f
+                    : static_cast<float>(count[j]) * top - width * static_cast<float>(places[j]) * (shift > kOffsetBits ? 1.0f / (1u << kOffsetBits) : 1.0f / static_cast<float>(1u << shift));
+                masses += own[j];
+            }
+            bin_scan<kBinWaves>(total, totals, masses, scan, tid);
+            binned = totals[0];
+            front[0] = total[0];
+            mass[0] = masses;
+            float rounded = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                front[j + 1] = front[j] + count[j];
+                mass[j + 1] = mass[j] + own[j];
+                if (count[j] != 0u && mass[j] > 0.0f)
+                {
+                    const uint32_t exponent = __float_as_uint(mass[j]) >> 23; // (the sum is 1 or more: no denormal ulps)
+                    const float ulp = __uint_as_float((max(exponent, 24u) - 23u) << 23);
+                    const float steps_per_ulp = __uint_as_float((277u - min(max(exponent, 24u), 250u)) << 23); // 1 / ulp
+                    const float lowest = bin_top(bin + j + 1u, shift) * steps_per_ulp;
+                    const float span = bin_top(bin + j, shift) * steps_per_ulp - lowest;
+                    if (span < 1.0f)
+                    {
+                        const float whole = floorf(lowest + 0.5f);
+                        const float above = fminf(fmaxf((lowest + span - (whole + 0.5f)) / span, 0.0f), 1.0f);
+                        own[j] = static_cast<float>(count[j]) * (whole + above) * ulp;
+                    }
+                }
+                rounded += own[j];
+            }
+            uint32_t none[1] = {0u};
+            bin_scan<kBinWaves>(none, totals, rounded, scan, tid);
+            mass[0] = rounded;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                mass[j + 1] = mass[j] + own[j];
+        }
+        // the head: as many bins as hold kBinHead elements at most, or those that hold the whole of a window that narrow
+        const bool window_in_head = window <= kBinHead;
+        {
+            // (the bins of the head are the first ones: one that is not of it ends it)
+            uint32_t first_not = kBins;
+#pragma unroll
+            for (int j = 3; j >= 0; --j)
+            {
+                const bool in_head = window_in_head ? front[j] < window
+                    : front[j + 1] <= kBinHead && (front[j + 1] <= kBinHeadDense || count[j] <= kBinHeadBin);
+                if (!in_head && bin + j != 0u)
+                    first_not = bin + j;
+            }
+            if (!holds_bins)
+                first_not = kBins;
+            // smallest over the workgroup, through the largest of the complement
+            const uint32_t most = wave_max_u32(kBins - first_not);
+            if ((tid & (kWaveSize - 1)) == 0 && most != 0u)
+                atomicMax(&head_bins_of_row, most);
+        }
+        __syncthreads();
+        const uint32_t head_bins = kBins - head_bins_of_row;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            if (holds_bins && bin + j + 1u == head_bins)
+                head_count_of_row = front[j + 1];
+        }
+        __syncthreads();
+        const uint32_t head_count = head_count_of_row;
+        if (head_count == 0u || head_count > kBinListCap)
+        {
+            // thousands of equal terms at the row's top: left to the full-order kernels
+            if (grid.part == 0u && tid == 0)
+                record.state[1] = kBinRowLeft;
+            __syncthreads();
+            continue;
+        }
+        const bool beyond = window > head_count && binned > head_count; // the sum goes on behind the head
+        BinPlan plan = plan_bins(bin, front, mass, head_bins, beyond ? window : 0u, kBins, INFINITY, kForeseenFirst);
+        uint32_t listed[1] = {holds_bins ? plan.listed : 0u};
+        {
+            uint32_t totals[1];
+            float none = 0.0f;
+            bin_scan<kBinWaves>(listed, totals, none, scan, tid);
+        }
+        uint32_t place[4];
+        const uint32_t own_end = fit_plan(plan, front, head_count + listed[0], place);
+        if (holds_bins)
+        {
+            uint32_t packed[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const bool in_head = bin + j < head_bins;
+                packed[j] = (plan.kind[j] << 30) | (plan.exponent[j] << 22) | front[j];
+                entries[bin + j] = in_head ? (0x80000000u | (front[j] + before[j]))
+                    : plan.kind[j] == kBinListed ? (0x80000000u | (place[j] + before[j]))
+                    : plan.kind[j] == kBinAdded ? plan.exponent[j] : 0x40000000u;
+            }
+            if (grid.part == 0u)
+            {
+                reinterpret_cast<uint4*>(g.packed[0] + static_cast<size_t>(row) * kBins)[tid] = uint4{packed[0], packed[1], packed[2], packed[3]};
+                if (own_end != 0u)
+                    atomicMax(&end_of_list, own_end);
+            }
+        }
+        __syncthreads();
+        if (grid.part == 0u && tid == 0)
+        {
+            record.state[1] = kBinRowGoesOn;
+            record.binned = binned;
+            record.head_bins = head_bins;
+            record.head_count = head_count;
+            record.listed[0] = max(end_of_list, head_count);
+        }
+        const BinStretch s = element_bytes == 4u ? bin_stretch<4>(a, row, grid.part, grid.parts) : bin_stretch<2>(a, row, grid.part, grid.parts);
+        add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks,
+                                      g.list_terms[0] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[0] + static_cast<size_t>(row) * kBinListCap, tid);
+        __syncthreads();
+        if (beyond)
+        {
+            const size_t pair = slot * grid.parts + grid.part;
+            if (holds_bins)
+                reinterpret_cast<uint4*>(g.steps[0] + pair * kBins)[tid] = reinterpret_cast<uint4*>(steps)[tid];
+            if (tid < static_cast<int>(2u * kBinQuads))
+                reinterpret_cast<uint4*>(g.masks[0] + pair * 2u * kBins)[tid] = reinterpret_cast<uint4*>(masks)[tid];
+            if (tid < static_cast<int>(3u * kBinWords))
+                g.ties[0][pair * 3u * kBinWords + tid] = ties[tid];
+        }
+        __syncthreads();
+    }
+}
+
+// The terms at terms[0 .. count) (LDS, in descending order) added to `sum` by one wave, two consecutive ones a lane.
+struct WaveSum
+{
+    float sum;
+    uint32_t index; // of the term at which the stop condition first held
+    bool stopped;
+};
+
+template <int PHASE>
+__device__ __forceinline__ WaveSum wave_add_terms(
+    const float* terms, uint32_t count, float sum, int mode, float bound, float divisor, float second_divisor)
+{
+    constexpr uint32_t kPerLane = 2;
+    const uint32_t lane = static_cast<uint32_t>(lane_id());
+    for (uint32_t base = 0; base < count; base += kPerLane * kWaveSize)
+    {
+        const uint32_t own = base + lane * kPerLane;
+        float v[kPerLane];
+#pragma unroll
+        for (uint32_t j = 0; j < kPerLane; ++j)
+        {
+            v[j] = own + j < count ? terms[own + j] : 0.0f;
+            if (PHASE >= 1)
+                v[j] = v[j] / divisor;
+            if (PHASE >= 2)
+                v[j] = v[j] / second_divisor;
+        }
+        uint32_t start = base;
+        while (true)
+        {
+            int exponent;
+            uint32_t mantissa;
+            decode_sum(sum, exponent, mantissa);
+            const uint32_t stop_at = stop_mantissa(mode, bound, exponent);
+            const uint32_t limit = min(stop_at, kBinadeFull);
+            ParityStep steps[kPerLane];
+            ParityStep total{0u, 0u};
+#pragma unroll
+            for (uint32_t j = 0; j < kPerLane; ++j)
+            {
+                const ParityStep step = step_of_term(v[j], exponent);
+                const bool active = own + j >= start;
+                steps[j] = ParityStep{active ? step.even : 0u, active ? step.odd : 0u};
+                total = compose_steps(total, steps[j]);
+            }
+            const ParityStep through = wave_scan_steps(total);
+            ParityStep in_front{__shfl_up(through.even, 1, kWaveSize), __shfl_up(through.odd, 1, kWaveSize)};
+            if (lane == 0u)
+                in_front = ParityStep{0u, 0u};
+            uint32_t current = apply_step(mantissa, in_front);
+            const uint32_t behind = apply_step(mantissa, through);
+            const uint64_t reaching = __builtin_amdgcn_ballot_w64(behind >= limit);
+            if (reaching == 0ull)
+            {
+                sum = encode_sum(exponent, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(behind), kWaveSize - 1)));
+                break;
+            }
+            const int first = __builtin_ctzll(reaching);
+            // the first term of that lane that takes the mantissa to the limit
+            uint32_t at = 0, before = 0, after = 0;
+            float term = 0.0f;
+            bool hit = false;
+#pragma unroll
+            for (uint32_t j = 0; j < kPerLane; ++j)
+            {
+                const uint32_t next = apply_step(current, steps[j]);
+                const bool here = !hit && own + j >= start && next >= limit;
+                at = here ? own + j : at;
+                before = here ? current : before;
+                after = here ? next : after;
+                term = here ? v[j] : term;
+                hit = hit || here;
+                current = next;
+            }
+            at = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), first));
+            before = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(before), first));
+            after = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(after), first));
+            term = read_lane(term, first);
+            if (after < kBinadeFull)
+                return WaveSum{encode_sum(exponent, after), at, true};
+            sum = encode_sum(exponent, before) + term;
+            if ((mode == kStopAtOrAbove && sum >= bound) || (mode == kStopAbove && sum > bound))
+                return WaveSum{sum, at, true};
+            start = at + 1u;
+            if (start >= count)
+                break;
+        }
+    }
+    return WaveSum{sum, 0u, false};
+}
+
+// `count` additions of one term.
+template <int PHASE>
+__device__ __forceinline__ WaveSum wave_add_repeated(
+    float term, uint32_t count, float sum, int mode, float bound, float divisor, float second_divisor)
+{
+    if (PHASE >= 1)
+        term = term / divisor;
+    if (PHASE >= 2)
+        term = term / second_divisor;
+    uint32_t done = 0;
+    while (done < count)
+    {
+        int exponent;
+        uint32_t mantissa;
+        decode_sum(sum, exponent, mantissa);
+        const uint32_t stop_at = stop_mantissa(mode, bound, exponent);
+        const uint32_t limit = min(stop_at, kBinadeFull);
+        const ParityStep single = step_of_term(term, exponent);
+        const bool odd = (mantissa & 1u) != 0u;
+        const uint32_t left = count - done;
+        if (mantissa + repeated_step(odd, single, left) < limit)
+            return WaveSum{encode_sum(exponent, mantissa + repeated_step(odd, single, left)), 0u, false};
+        uint32_t none = 0, some = left; // `none` additions stay below the limit, `some` reach it
+        while (some - none > 1u)
+        {
+            const uint32_t middle = none + ((some - none) >> 1);
+            if (mantissa + repeated_step(odd, single, middle) >= limit)
+                some = middle;
+            else
+                none = middle;
+        }
+        const uint32_t before = mantissa + repeated_step(odd, single, none);
+        const uint32_t after = apply_step(before, single);
+        if (after < kBinadeFull)
+            return WaveSum{encode_sum(exponent, after), done + none, true};
+        sum = encode_sum(exponent, before) + term;
+        if ((mode == kStopAtOrAbove && sum >= bound) || (mode == kStopAbove && sum > bound))
+            return WaveSum{sum, done + none, true};
+        done += none + 1u;
+    }
+    return WaveSum{sum, 0u, false};
+}
+
+// Of the sums over a sorted stretch of terms in LDS (sum_chunks, sum_head): per 64 terms the sum in front of them (about),
+// and what they do to a sum of that exponent.
+struct HeadScratch
+{
+    float chunk_front[kWaveSize];
+    uint32_t chunk_exponent[kWaveSize], chunk_even[kWaveSize], chunk_odd[kWaveSize];
+    float sum;
+    uint32_t stop; // 0xffffffff: no element met the stop condition
+};
+
+constexpr uint32_t kBinMasks = 128;      // bins with terms half way whose masks the walk keeps
+constexpr uint32_t kHasMasks = 0x8000u;
+
+struct BinWalkShared
+{
+    alignas(16) uint32_t packed[kBins + 4]; // [kBins]: the elements in bins
+    alignas(16) uint32_t prefix[kBins + 4]; // steps added in front of each bin (modulo 2^32)
+    alignas(16) float terms[kBinListCap + kBinExtraCap];
+    alignas(16) uint32_t tokens[kBinListCap + kBinExtraCap];
+    uint16_t places[kBins];                 // where a listed bin's elements begin; kHasMasks + i: the bin's masks are the i-th
+    uint32_t bin_masks[2 * kBinMasks];      // of bins with terms half way
+    uint32_t mask_count;
+    uint32_t stop_bin[kBinStops];           // bins at which the walk looks closer, in order; bit 31: nothing but a new exponent
+    uint32_t ties[2 * kBinWords];           // bins with terms half way; those of them that the masks do not tell
+    BinScanScratch scan;
+    HeadScratch head;
+    // the walk's state between two fetches
+    uint32_t status; // 0: elements of bins [low, high] are wanted; 1: ended; 2: given up
+    uint32_t low, high;
+    uint32_t extra_count, extra_least, extra_most;
+    float sum;
+    uint32_t stopped;
+    uint32_t stop_rank;  // rank in the sorted row, and place in terms[], of the element the sum stopped at
+    uint32_t stop_at;
+    uint32_t taken;      // elements added when the sum ran to its end
+    uint32_t listed_end;
+    int32_t token;
+};
+
+constexpr uint32_t kBinExtraPlace = kBinListCap;
+
+__device__ __forceinline__ uint32_t same_in_all(uint32_t value)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(value)));
+}
+
+__device__ __forceinline__ float same_in_all(float value)
+{
+    return __uint_as_float(same_in_all(__float_as_uint(value)));
+}
+
+// Puts `count` elements (thread i % kWalkThreads holds element i, its term and token in registers) in descending order of
+// their terms at terms[place ..], tokens[place ..].  `fine` is about where each belongs (0 .. count - 1, falling with the
+// term): elements of one `fine` are neighbours, few of them unless they are equal, and are ranked against each other.
+// The place where the tokens go counts the elements of each `fine` first.  Every thread calls it.
+template <uint32_t PER_THREAD>
+__device__ __forceinline__ void order_elements(
+    BinWalkShared& shared, uint32_t place, uint32_t count, const float (&own)[PER_THREAD], const uint32_t (&token)[PER_THREAD],
+    const uint32_t (&fine)[PER_THREAD], int tid)
+{
+    constexpr uint32_t kMixed = 0x80000000u; // the elements of this `fine` are not all equal
+    uint32_t* const counters = shared.tokens + place;
+    float* const terms = shared.terms + place;
+    uint32_t turn[PER_THREAD];
+    for (uint32_t i = tid; i < count; i += kWalkThreads)
+        counters[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    {
+        if (k * kWalkThreads + tid < count)
+            turn[k] = atomicAdd(&counters[fine[k]], 1u);
+    }
+    __syncthreads();
+    {
+        const uint32_t each = (count + kWalkThreads - 1u) / kWalkThreads;
+        const uint32_t first = tid * each;
+        uint32_t held[PER_THREAD];
+        uint32_t total[1] = {0u};
+#pragma unroll
+        for (uint32_t k = 0; k < PER_THREAD; ++k)
+        {
+            held[k] = k < each && first + k < count ? counters[first + k] : 0u;
+            total[0] += held[k];
+        }
+        uint32_t totals[1];
+        float none = 0.0f;
+        bin_scan<kWalkWaves>(total, totals, none, shared.scan, tid);
+        uint32_t front = total[0];
+#pragma unroll
+        for (uint32_t k = 0; k < PER_THREAD; ++k)
+        {
+            if (k < each && first + k < count)
+                counters[first + k] = front;
+            front += held[k];
+        }
+    }
+    __syncthreads();
+    uint32_t at[PER_THREAD];
+#pragma unroll
+    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    {
+        at[k] = 0u;
+        if (k * kWalkThreads + tid < count)
+        {
+            at[k] = counters[fine[k]] + turn[k];
+            terms[at[k]] = own[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    {
+        if (k * kWalkThreads + tid < count && terms[at[k] - turn[k]] != own[k])
+            atomicOr(&counters[fine[k]], kMixed);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    {
+        if (k * kWalkThreads + tid < count && (counters[fine[k]] & kMixed) != 0u)
+        {
+            const uint32_t low = at[k] - turn[k];
+            const uint32_t high = fine[k] + 1u < count ? counters[fine[k] + 1u] & ~kMixed : count;
+            uint32_t rank = low;
+            for (uint32_t j = low; j < high; ++j)
+                rank += terms[j] > own[k] || (terms[j] == own[k] && j < at[k]) ? 1u : 0u;
+            at[k] = rank;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    {
+        if (k * kWalkThreads + tid < count)
+        {
+            terms[at[k]] = own[k];
+            counters[at[k]] = token[k];
+        }
+    }
+    __syncthreads();
+}
+
+// About where in a bin of `count` elements a term lies.
+__device__ __forceinline__ uint32_t fine_place(float term, uint32_t shift, uint32_t count)
+{
+    const uint32_t within = (kOneBits - __float_as_uint(term)) & ((1u << shift) - 1u);
+    return static_cast<uint32_t>((static_cast<uint64_t>(within) * count) >> shift);
+}
+
+// Fetches the elements of bins [shared.low, shared.high] (at most kBinExtraCap of them; shared.extra_count: how many there
+// are), in order, to shared.terms[kBinExtraPlace ..].
+__device__ __forceinline__ void fetch_bins(const float* terms, uint32_t positions, uint32_t misalignment, uint32_t shift, BinWalkShared& shared, int tid)
+{
+    constexpr int kLoads = 8;
+    if (tid == 0)
+    {
+        shared.extra_count = 0u;
+        shared.extra_least = 0xffffffffu;
+        shared.extra_most = 0u;
+    }
+    __syncthreads();
+    const uint32_t top = kOneBits - (shared.low << shift);        // bits of the largest term wanted
+    const uint32_t width = (shared.high + 1u - shared.low) << shift;
+    const uint32_t vectors = positions / 4u;
+    for (uint32_t at = tid; at < vectors; at += kLoads * kWalkThreads)
+    {
+        float4 raw[kLoads];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k)
+            raw[k] = reinterpret_cast<const float4*>(terms)[min(at + k * kWalkThreads, vectors - 1u)];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k)
+        {
+            const uint32_t v = at + k * kWalkThreads;
+            const float t[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+            {
+                const uint32_t bits = __float_as_uint(t[c]);
+                if (top - bits < width && kOneBits - bits < kTailDistance && v < vectors)
+                {
+                    const uint32_t at_place = atomicAdd(&shared.extra_count, 1u);
+                    atomicMin(&shared.extra_least, bits);
+                    atomicMax(&shared.extra_most, bits);
+                    if (at_place < kBinExtraCap)
+                    {
+                        shared.terms[kBinExtraPlace + at_place] = t[c];
+                        shared.tokens[kBinExtraPlace + at_place] = v * 4u + c - misalignment;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t count = shared.extra_count;
+    if (count <= kBinExtraCap)
+    {
+        constexpr uint32_t kPerThread = (kBinExtraCap + kWalkThreads - 1) / kWalkThreads;
+        float own[kPerThread];
+        uint32_t token[kPerThread], fine[kPerThread];
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            const uint32_t i = k * kWalkThreads + tid;
+            own[k] = 1.0f;
+            token[k] = fine[k] = 0u;
+            if (i < count)
+            {
+                own[k] = shared.terms[kBinExtraPlace + i];
+                token[k] = shared.tokens[kBinExtraPlace + i];
+                fine[k] = static_cast<uint32_t>((static_cast<uint64_t>(top - __float_as_uint(own[k])) * count) / width);
+            }
+        }
+        __syncthreads();
+        order_elements<kPerThread>(shared, kBinExtraPlace, count, own, token, fine, tid);
+    }
+}
+
+// The plain sums of the terms in front of each 64 of `count` (4096 at most).
+template <int WAVES>
+__device__ __forceinline__ void sum_chunks(HeadScratch& scratch, const float* terms, uint32_t count, int tid)
+{
+    const int lane = tid & (kWaveSize - 1);
+    const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
+    const uint32_t chunks = (count + kWaveSize - 1u) / kWaveSize;
+    for (uint32_t c = wave; c < chunks; c += WAVES)
+    {
+        const uint32_t i = c * kWaveSize + lane;
+        const float sum = wave_prefix_sum_f32(i < count ? terms[i] : 0.0f);
+        if (lane == kWaveSize - 1)
+            scratch.chunk_front[c] = sum;
+    }
+    __syncthreads();
+    const float own = static_cast<uint32_t>(lane) < chunks ? scratch.chunk_front[lane] : 0.0f;
+    const float through = wave_prefix_sum_f32(own);
+    __syncthreads();
+    if (wave == 0u)
+        scratch.chunk_front[lane] = through - own;
+    __syncthreads();
+}
+
+// The sum of `count` terms in descending order (scratch.sum, scratch.stop), exactly as a sequential loop makes it; every thread calls it.  The waves work
+// out what each 64 terms do to a sum of the exponent that it should have there (from sum_chunks), while the first wave adds the first
+// terms in order; it then takes the chunks whose exponent was right in one scan and looks into the others.
+template <int WAVES, int PHASE>
+__device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* terms, uint32_t count, int mode, float bound, float divisor, float second_divisor, int tid)
+{
+    constexpr uint32_t kInOrder = 4; // chunks added in order
+    const int lane = tid & (kWaveSize - 1);
+    const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
+    const uint32_t chunks = (count + kWaveSize - 1u) / kWaveSize;
+    const auto scaled = [&](float t) {
+        if (PHASE >= 1)
+            t = t / divisor;
+        if (PHASE >= 2)
+            t = t / second_divisor;
+        return t;
+    };
+    const float scale = PHASE == 0 ? 1.0f : PHASE == 1 ? 1.0f / divisor : 1.0f / (divisor * second_divisor);
+    for (uint32_t c = wave == 0u ? WAVES : wave; c < chunks; c += WAVES)
+    {
+        if (c < kInOrder)
+            continue;
+        const uint32_t i = c * kWaveSize + lane;
+        const uint32_t exponent = same_in_all(__float_as_uint(scratch.chunk_front[c] * scale) >> 23);
+        const ParityStep through = wave_scan_steps(step_of_term(scaled(i < count ? terms[i] : 0.0f), static_cast<int>(exponent)));
+        if (lane == kWaveSize - 1)
+        {
+            scratch.chunk_exponent[c] = exponent;
+            scratch.chunk_even[c] = through.even;
+            scratch.chunk_odd[c] = through.odd;
+        }
+    }
+    float sum = 0.0f;
+    uint32_t stop = 0xffffffffu;
+    if (wave == 0u)
+    {
+        const uint32_t in_order = min(count, kInOrder * kWaveSize);
+        for (uint32_t first = 0; first < in_order && stop == 0xffffffffu; first += kWaveSize)
+        {
+            const uint32_t i = first + lane;
+            float own = i < count ? scaled(terms[i]) : 0.0f;
+            own = lane == 0 ? sum + own : own;
+            const float sums = wave_sequential_sums(own);
+            const bool stops = i < count && ((mode == kStopAtOrAbove && sums >= bound) || (mode == kStopAbove && sums > bound));
+            const uint64_t stopping = __builtin_amdgcn_ballot_w64(stops);
+            sum = read_lane(sums, kWaveSize - 1);
+            if (stopping != 0ull)
+            {
+                const int at = __builtin_ctzll(stopping);
+                sum = read_lane(sums, at);
+                stop = first + static_cast<uint32_t>(at);
+            }
+        }
+    }
+    __syncthreads();
+    if (wave == 0u)
+    {
+        uint32_t c = kInOrder;
+        uint32_t own_exponent = 0, own_even = 0, own_odd = 0;
+        if (static_cast<uint32_t>(lane) < chunks && static_cast<uint32_t>(lane) >= kInOrder)
+        {
+            own_exponent = scratch.chunk_exponent[lane];
+            own_even = scratch.chunk_even[lane];
+            own_odd = scratch.chunk_odd[lane];
+        }
+        while (c < chunks && stop == 0xffffffffu)
+        {
+            int exponent;
+            uint32_t mantissa;
+            decode_sum(sum, exponent, mantissa);
+            const uint32_t goal = min(stop_mantissa(mode, bound, exponent), kBinadeFull);
+            const bool ahead = static_cast<uint32_t>(lane) >= c && static_cast<uint32_t>(lane) < chunks;
+            const bool usable = ahead && own_exponent == static_cast<uint32_t>(exponent);
+            const ParityStep through = wave_scan_steps(ParityStep{usable ? own_even : 0u, usable ? own_odd : 0u});
+            const uint32_t behind = apply_step(mantissa, through);
+            const uint64_t bad = __builtin_amdgcn_ballot_w64(ahead && !(usable && behind < goal));
+            const uint32_t first_bad = bad != 0ull ? static_cast<uint32_t>(__builtin_ctzll(bad)) : chunks;
+            if (first_bad > c)
+                sum = encode_sum(exponent, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(behind), static_cast<int>(first_bad - 1u))));
+            c = first_bad;
+            if (c >= chunks)
+                break;
+            const uint32_t first = c * kWaveSize;
+            const WaveSum result = wave_add_terms<PHASE>(terms + first, min(count - first, static_cast<uint32_t>(kWaveSize)), sum, mode, bound, divisor, second_divisor);
+            sum = result.sum;
+            if (result.stopped)
+                stop = first + result.index;
+            ++c;
+        }
+        if (lane == 0)
+        {
+            scratch.sum = sum;
+            scratch.stop = stop;
+        }
+    }
+    __syncthreads();
+}
+
+// The walk over the bins behind the head, from `sum` on: every thread calls it; the first wave walks, the workgroup
+// fetches what it asks for.  Ends with shared.status 1 (ended: sum, stopped, ...) or 2 (given up).
+//   limit     elements that the sum runs over at most; cut_bin, cut_term: it ends at the first term below cut_term,
+//             which lies in that bin (kBins: nowhere)
+template <int PHASE>
+__device__ __forceinline__ void walk_bins(
+    BinWalkShared& shared, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins,
+    uint32_t limit, uint32_t cut_bin, float cut_term, float start_sum, int mode, float bound, float divisor, float second_divisor, int tid)
+{
+    uint32_t cur = head_bins;
+    uint32_t stop = 0;
+    float sum = start_sum;
+    bool fetched = false;
+    const auto front_of = [&shared](uint32_t bin) { return packed_front(shared.packed[bin]); };
+    for (uint32_t requests = 0;; ++requests)
+    {
+        if (tid < kWaveSize)
+        {
+            uint32_t status = 3u;
+            const auto finish = [&](uint32_t outcome) {
+                status = outcome;
+                shared.status = outcome;
+                shared.sum = sum;
+            };
+            // of `count` elements from `place` on, of bins [bin, last_bin]: how many the sum takes
+            const auto share_of_sum = [&](uint32_t bin, uint32_t last_bin, uint32_t place, uint32_t count) {
+                uint32_t take = min(count, limit - min(limit, front_of(bin)));
+                if (cut_bin >= bin && cut_bin <= last_bin)
+                {
+                    const float* elements = shared.terms + place;
+                    take = min(take, wave_partition_point(count, [elements, cut_term](uint32_t i) { return elements[i] >= cut_term; }));
+                }
+                return take;
+            };
+            const auto end_at = [&](uint32_t taken) {
+                shared.stopped = 0u;
+                shared.taken = taken;
+                finish(1u);
+            };
+            const auto stopped_at = [&](uint32_t rank, uint32_t place) {
+                shared.stopped = 1u;
+                shared.stop_rank = rank;
+                shared.stop_at = place;
+                finish(1u);
+            };
+            const auto ask_for = [&](uint32_t low, uint32_t high) {
+                shared.low = low;
+                shared.high = high;
+                finish(requests < kBinRequests ? 0u : 2u);
+            };
+            if (fetched)
+            {
+                const uint32_t low = shared.low, high = shared.high, count = shared.extra_count;
+                const uint32_t front = front_of(low);
+                fetched = false;
+                if (count > kBinExtraCap && shared.extra_least != shared.extra_most)
+                    finish(2u);
+                else
+                {
+                    uint32_t take;
+                    WaveSum result;
+                    if (count > kBinExtraCap)
+                    {
+                        // thousands of equal terms
+                        const float term = __uint_as_float(shared.extra_least);
+                        take = min(count, limit - min(limit, front));
+                        take = cut_bin >= low && cut_bin <= high && term < cut_term ? 0u : take;
+                        result = wave_add_repeated<PHASE>(term, take, sum, mode, bound, divisor, second_divisor);
+                    }
+                    else
+                    {
+                        take = share_of_sum(low, high, kBinExtraPlace, count);
+                        result = wave_add_terms<PHASE>(shared.terms + kBinExtraPlace, take, sum, mode, bound, divisor, second_divisor);
+                    }
+                    sum = result.sum;
+                    if (result.stopped)
+                        stopped_at(front + result.index, count > kBinExtraCap ? 0xffffffffu : kBinExtraPlace + result.index);
+                    else if (take < count)
+                        end_at(front + take);
+                    cur = high + 1u;
+                    while ((shared.stop_bin[stop] & 0x7fffffffu) <= high)
+                        ++stop;
+                }
+            }
+            while (status == 3u)
+            {
+                const uint32_t stop_word = shared.stop_bin[stop];
+                const uint32_t stop_here = stop_word & 0x7fffffffu;
+                if (cur < stop_here)
+                {
+                    // bins that are one integer each
+                    const uint32_t front = front_of(cur);
+                    const uint32_t front_prefix = shared.prefix[cur];
+                    if (front_of(stop_here) == front)
+                    {
+                        cur = stop_here;
+                        continue;
+                    }
+                    int exponent;
+                    uint32_t mantissa;
+                    decode_sum(sum, exponent, mantissa);
+                    const uint32_t goal = min(stop_mantissa(mode, bound, exponent), kBinadeFull);
+                    if (packed_exponent(shared.packed[cur]) == static_cast<uint32_t>(exponent))
+                    {
+                        const uint32_t total = shared.prefix[stop_here] - front_prefix;
+                        if (mantissa + total < goal && total < kBinadeFull)
+                        {
+                            sum = encode_sum(exponent, mantissa + total);
+                            cur = stop_here;
+                            continue;
+                        }
+                        const uint32_t first = cur;
+                        const uint32_t* prefix = shared.prefix;
+                        const uint32_t good = wave_partition_point(stop_here - cur, [prefix, first, front_prefix, mantissa, goal](uint32_t i) {
+                            const uint32_t through = prefix[first + i + 1u] - front_prefix;
+                            return through < kBinadeFull && mantissa + through < goal;
+                        });
+                        if (good > 0u)
+                            sum = encode_sum(exponent, mantissa + (shared.prefix[cur + good] - front_prefix));
+                        cur += good;
+                        ask_for(cur, cur);
+                    }
+                    else
+                    {
+                        // the sum has another exponent than was foreseen: as many bins as can be fetched at a time
+                        const uint32_t first = cur;
+                        const uint32_t more = wave_partition_point(stop_here - cur, [&shared, first, front](uint32_t i) {
+                            return packed_front(shared.packed[first + i + 1u]) - front <= kBinExtraCap;
+                        });
+                        ask_for(cur, cur + max(more, 1u) - 1u);
+                    }
+                }
+                else if ((stop_word & 0x80000000u) != 0u)
+                    ++stop; // (a new exponent from this bin on)
+                else if (stop_here == kBins || packed_kind(shared.packed[stop_here]) == kBinBeyond)
+                    end_at(min(limit, front_of(stop_here)));
+                else if (packed_kind(shared.packed[stop_here]) != kBinListed)
+                {
+                    // terms half way: their roundings follow from the masks, unless the sum has another exponent than was
+                    // foreseen or leaves its binade (or stops) in this bin
+                    const uint32_t place = shared.places[stop_here];
+                    int exponent;
+                    uint32_t mantissa;
+                    decode_sum(sum, exponent, mantissa);
+                    const uint32_t goal = min(stop_mantissa(mode, bound, exponent), kBinadeFull);
+                    bool known = (place & kHasMasks) != 0u && packed_exponent(shared.packed[stop_here]) == static_cast<uint32_t>(exponent);
+                    if (known)
+                    {
+                        const uint32_t total = shared.prefix[stop_here + 1u] - shared.prefix[stop_here];
+                        const uint32_t parities = shared.bin_masks[2u * (place & ~kHasMasks)], halves = shared.bin_masks[2u * (place & ~kHasMasks) + 1u];
+                        float top = bin_top(stop_here, shift);
+                        if (PHASE >= 1)
+                            top = top / divisor;
+                        if (PHASE >= 2)
+                            top = top / second_divisor;
+                        // lane l: the terms of step highest - l, and the value half way between that step and the one below
+                        known = exponent - static_cast<int>(__float_as_uint(top) >> 23) >= kMaskedDifference;
+                        const uint32_t step = step_of_term(top, exponent).odd + 1u - static_cast<uint32_t>(lane_id());
+                        const bool in_range = lane_id() < 32;
+                        const uint64_t odd_steps = __builtin_amdgcn_ballot_w64(in_range && (step & 1u) != 0u && (parities >> ((step >> 1) & 31u) & 1u) != 0u);
+                        uint64_t half_way = __builtin_amdgcn_ballot_w64(in_range && (halves >> ((step - 1u) & 31u) & 1u) != 0u);
+                        const uint32_t highest = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(step), 0));
+                        uint32_t parity = mantissa, less = 0;
+                        while (half_way != 0ull)
+                        {
+                            const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(half_way));
+                            half_way &= half_way - 1ull;
+                            const uint32_t below = highest - l - 1u; // the value lies half way between this step and the next
+                            const uint32_t in_front = static_cast<uint32_t>(__popcll(odd_steps & ((2ull << l) - 1ull)));
+                            const uint32_t up = (parity + in_front + below) & 1u; // to the even neighbour
+                            parity += below + up;
+                            less += 1u - up;
+                        }
+                        known = known && total < kBinadeFull && mantissa + total < goal;
+                        if (known)
+                        {
+                            sum = encode_sum(exponent, mantissa + total - less);
+                            cur = stop_here + 1u;
+                            ++stop;
+                        }
+                    }
+                    if (!known)
+                        ask_for(stop_here, stop_here);
+                }
+                else
+                {
+                    const uint32_t place = shared.places[stop_here];
+                    const uint32_t front = front_of(stop_here);
+                    const uint32_t count = front_of(stop_here + 1u) - front;
+                    const uint32_t take = share_of_sum(stop_here, stop_here, place, count);
+                    const WaveSum result = wave_add_terms<PHASE>(shared.terms + place, take, sum, mode, bound, divisor, second_divisor);
+                    sum = result.sum;
+                    if (result.stopped)
+                        stopped_at(front + result.index, place + result.index);
+                    else if (take < count)
+                        end_at(front + take);
+                    cur = stop_here + 1u;
+                    ++stop;
+                }
+            }
+        }
+        __syncthreads();
+        if (shared.status != 0u)
+            return;
+        fetch_bins(row_terms, positions, misalignment, shift, shared, tid);
+        fetched = true;
+    }
+}
+
+// The token of the element at terms[at] of a list [list_first, list_end) in order: elements of equal term are in no
+// particular order, and are told apart by their logits and indices.
+template <int DTYPE>
+__device__ __forceinline__ int32_t token_of_listed(
+    const SamplerArgs& a, uint32_t row, BinWalkShared& shared, const uint32_t* tokens, uint32_t at, uint32_t list_first, uint32_t list_end, int tid)
+{
+    const float term = shared.terms[at];
+    const float* terms = shared.terms;
+    const uint32_t low = list_first + wave_partition_point(at - list_first, [terms, list_first, term](uint32_t i) { return terms[list_first + i] > term; });
+    const uint32_t high = at + 1u + wave_partition_point(list_end - at - 1u, [terms, at, term](uint32_t i) { return terms[at + 1u + i] >= term; });
+    if (high - low == 1u)
+        return static_cast<int32_t>(tokens[at]);
+    const char* pointer = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes;
+    // their keys, where the bins' words were
+    uint32_t* const keys = shared.packed;
+    const bool keys_fit = high - low <= 2u * kBins;
+    static_assert(offsetof(BinWalkShared, prefix) == sizeof(uint32_t) * (kBins + 4), "packed and prefix lie one behind the other");
+    const auto key_of = [&](uint32_t i) { return descending_key(load_logit<DTYPE>(pointer, tokens[i])); };
+    __syncthreads();
+    if (keys_fit)
+    {
+        for (uint32_t i = low + tid; i < high; i += kWalkThreads)
+            keys[i - low] = key_of(i);
+    }
+    __syncthreads();
+    for (uint32_t i = low + tid; i < high; i += kWalkThreads)
+    {
+        const uint32_t token = tokens[i];
+        const uint32_t key = keys_fit ? keys[i - low] : key_of(i);
+        uint32_t rank = 0;
+        for (uint32_t j = low; j < high; ++j)
+        {
+            const uint32_t other = keys_fit ? keys[j - low] : key_of(j);
+            rank += other < key || (other == key && tokens[j] < token) ? 1u : 0u;
+        }
+        if (rank == at - low)
+            shared.token = static_cast<int32_t>(token);
+    }
+    __syncthreads();
+    const int32_t token = shared.token;
+    __syncthreads();
+    return token;
+}
+
+// ---- (4), (5), (6): WALK 0 walks the normaliser and, inside the head, the Top-P sum and the draw, WALK 1 the Top-P sum
+// behind the head (and the draw inside it), WALK 2 the draw behind the head.  Each then has the bins' steps of the next
+// sum added for the calling part of the row, unless the row is finished.  Every part of a row walks for itself.
+template <int DTYPE, int WALK>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void bin_walk_kernel(BinArgs g)
+{
+    __shared__ BinWalkShared shared;
+    constexpr int kFrom = WALK & 1;      // which of the alternating buffers this launch reads
+    constexpr int kTo = kFrom ^ 1;
+    const SamplerArgs& a = g.a;
+    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const int tid = threadIdx.x;
+    const uint32_t bin = 4u * static_cast<uint32_t>(tid);
+    const bool holds_bins = tid < static_cast<int>(kBinQuads);
+    if (WALK == 2 && grid.part != 0u)
+        return;
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = same_in_all(g.list[1u + slot]);
+        BinRow& record = g.records[row];
+        const auto leave = [&](uint32_t state) {
+            if (WALK < 2 && grid.part == 0u && tid == 0)
+                record.state[WALK + 2] = state;
+        };
+        if (same_in_all(record.state[WALK + 1]) != kBinRowGoesOn)
+        {
+            leave(kBinRowLeft);
+            continue;
+        }
+        __syncthreads(); // (a row before this one: its last readers of shared are done)
+        const float top_p = same_in_all(a.params[row].top_p);
+        const float min_p = same_in_all(a.params[row].min_p);
+        const float uniform = same_in_all(a.uniforms[row]);
+        const uint32_t shift = same_in_all(record.shift);
+        const uint32_t window = same_in_all(record.window);
+        const uint32_t binned = same_in_all(record.binned);
+        const uint32_t head_bins = same_in_all(record.head_bins);
+        const uint32_t head_count = same_in_all(record.head_count);
+        const uint32_t listed = same_in_all(record.listed[WALK]);
+        const uint32_t limit = WALK == 0 ? window : same_in_all(record.limit[WALK - 1]);
+        const uint32_t cut_bin = WALK == 1 ? same_in_all(record.cut_bin) : kBins;
+        const float cut_term = WALK == 1 ? same_in_all(record.cut_term) : 0.0f;
+        uint32_t cut_in_tail = WALK == 1 ? same_in_all(record.cut_in_tail) : 0u;
+        const bool behind_head = limit > head_count && binned > head_count; // this launch's own sum goes on behind the head
+        float normalizer = WALK == 0 ? 1.0f : same_in_all(record.normalizer);
+        float renormalizer = WALK == 2 ? same_in_all(record.renormalizer) : 1.0f;
+        const float sum_so_far = WALK == 0 ? 0.0f : same_in_all(record.head_sum[WALK - 1]);
+        uint32_t kept = WALK == 2 ? same_in_all(record.kept) : 0u;
+        const BinStretch s = bin_stretch<LogitsVector<DTYPE>::kElementBytes>(a, row, grid.part, grid.parts);
+        const uint32_t positions = (s.end + 7u) / 8u * 8u;
+        const float* row_terms = bin_terms(a, row);
+        float* const sorted_terms_out = g.head_terms + static_cast<size_t>(row) * kBinListCap;
+        uint32_t* const sorted_tokens_out = g.head_tokens + static_cast<size_t>(row) * kBinListCap;
+
+        // ---- the list, the bins and their steps.  The head is ordered by WALK 0, read back by WALK 1, no longer needed by WALK 2.
+        constexpr uint32_t kPerThread = kBinListCap / kWalkThreads;
+        const uint32_t list_first = WALK == 0 ? 0u : head_count;
+        float own_terms[kPerThread];
+        uint32_t own_tokens[kPerThread];
+        {
+            const float* from_terms = g.list_terms[kFrom] + static_cast<size_t>(row) * kBinListCap;
+            const uint32_t* from_tokens = g.list_tokens[kFrom] + static_cast<size_t>(row) * kBinListCap;
+#pragma unroll
+            for (uint32_t k = 0; k < kPerThread; ++k)
+            {
+                const uint32_t i = list_first + k * kWalkThreads + tid;
+                own_terms[k] = i < listed ? from_terms[i] : 0.0f;
+                own_tokens[k] = i < listed ? from_tokens[i] : 0u;
+            }
+        }
+        uint4 words{0u, 0u, 0u, 0u};
+        uint32_t own_steps[4] = {0u, 0u, 0u, 0u};
+        uint32_t tie_word = 0, untold_word = 0;
+        const uint32_t tie_lane = static_cast<uint32_t>(tid) - (kWalkThreads - kWaveSize);
+        if (holds_bins)
+            words = reinterpret_cast<const uint4*>(g.packed[kFrom] + static_cast<size_t>(row) * kBins)[tid];
+        if (behind_head)
+        {
+            const size_t first_pair = slot * grid.parts;
+            if (holds_bins && bin + 3u >= head_bins)
+            {
+                const uint4* from = reinterpret_cast<const uint4*>(g.steps[kFrom] + first_pair * kBins) + tid;
+                for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
+                {
+                    uint4 of_part[kPartsAtATime];
+#pragma unroll
+                    for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                        of_part[k] = from[static_cast<size_t>(min(first + k, grid.parts - 1u)) * kBinQuads];
+#pragma unroll
+                    for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                    {
+                        const uint32_t some = first + k < grid.parts ? 0xffffffffu : 0u;
+                        own_steps[0] += of_part[k].x & some, own_steps[1] += of_part[k].y & some;
+                        own_steps[2] += of_part[k].z & some, own_steps[3] += of_part[k].w & some;
+                    }
+                }
+            }
+            // (the last waves hold no bins: they collect the words of the bins with terms half way)
+            if (tie_lane < kBinWords)
+            {
+                uint32_t other_words = 0;
+#pragma unroll
+                for (uint32_t q = 0; q < kMaxBinParts; ++q)
+                {
+                    const uint32_t* from = g.ties[kFrom] + (first_pair + min(q, grid.parts - 1u)) * 3u * kBinWords + tie_lane;
+                    tie_word |= from[0];
+                    other_words |= from[kBinWords] | from[2u * kBinWords];
+                }
+                untold_word = other_words;
+            }
+        }
+        static_assert(kBinWords <= kWaveSize && kBinQuads <= kWalkThreads - kWaveSize, "the last wave holds no bins");
+        if (holds_bins)
+            *reinterpret_cast<uint4*>(shared.packed + bin) = words;
+        if (tie_lane < kBinWords)
+        {
+            shared.ties[tie_lane] = tie_word;
+            shared.ties[kBinWords + tie_lane] = untold_word;
+        }
+        if (tid == 0)
+            shared.mask_count = 0u;
+        if (tid < 4)
+            shared.packed[kBins + tid] = (kBinBeyond << 30) | binned;
+        if constexpr (WALK == 1)
+        {
+            for (uint32_t i = tid; i < head_count; i += kWalkThreads)
+                shared.terms[i] = sorted_terms_out[i];
+        }
+        __syncthreads();
+        // ---- stops: bins that the walk looks into, and bins from which on another exponent was assumed
+        uint32_t front[5];
+        float mass[5]; // about what the sum holds in front of each bin, behind the head (in the sum's own units)
+        uint32_t stops;
+        {
+            const uint32_t packed[4] = {words.x, words.y, words.z, words.w};
+            uint32_t kind[4];
+            float own_mass[4];
+            uint32_t stop_word[4];
+            uint32_t sums[3] = {0u, 0u, 0u}; // steps added, elements listed, stops
+            float masses = 0.0f;
+            const float scale = 1.0f / (normalizer * renormalizer);
+            const uint32_t tie_bits = holds_bins ? shared.ties[bin >> 5] >> (bin & 31u) : 0u;
+            const uint32_t untold_bits = holds_bins ? shared.ties[kBinWords + (bin >> 5)] >> (bin & 31u) : 0u;
+            uint32_t masked[4];
+            uint32_t previous = holds_bins && bin > head_bins ? shared.packed[bin - 1u] : packed[0];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                front[j] = packed_front(packed[j]);
+            front[4] = holds_bins ? packed_front(shared.packed[bin + 4u]) : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const uint32_t b = bin + j;
+                const uint32_t count = front[j + 1] - front[j];
+                const bool behind = holds_bins && b >= head_bins;
+                if (b <= head_bins)
+                    previous = packed[j];
+                kind[j] = packed_kind(packed[j]);
+                if (kind[j] == kBinAdded && (tie_bits >> j & 1u) != 0u)
+                    kind[j] = kBinWanted;
+                const bool ends = behind && kind[j] == kBinBeyond && (b == head_bins || packed_kind(previous) != kBinBeyond);
+                const bool looks = behind && (kind[j] == kBinListed || kind[j] == kBinWanted);
+                const bool changes = behind && kind[j] != kBinBeyond && packed_exponent(previous) != packed_exponent(packed[j]);
+                stop_word[j] = ends || looks ? b : changes ? (b | 0x80000000u) : 0xffffffffu;
+                // a bin whose terms half way the masks tell: its masks, from every part (a value half way that two parts
+                // have seen is there twice, which a mask cannot tell)
+                masked[j] = 0u;
+                if (behind && kind[j] == kBinWanted && packed_kind(packed[j]) == kBinAdded && (untold_bits >> j & 1u) == 0u)
+                {
+                    uint32_t parities = 0, halves = 0, twice = 0;
+                    for (uint32_t q = 0; q < grid.parts; ++q)
+                    {
+                        const uint32_t* from = g.masks[kFrom] + static_cast<size_t>(slot * grid.parts + q) * 2u * kBins + b;
+                        parities ^= from[0];
+                        twice |= halves & from[kBins];
+                        halves |= from[kBins];
+                    }
+                    const uint32_t i = twice == 0u ? atomicAdd(&shared.mask_count, 1u) : kBinMasks;
+                    if (i < kBinMasks)
+                    {
+                        shared.bin_masks[2u * i] = parities;
+                        shared.bin_masks[2u * i + 1u] = halves;
+                        masked[j] = kHasMasks | i;
+                    }
+                }
+                const bool adds = behind && (kind[j] == kBinAdded || masked[j] != 0u);
+                own_steps[j] = adds ? own_steps[j] : 0u;
+                own_mass[j] = adds ? static_cast<float>(own_steps[j]) * __uint_as_float((max(packed_exponent(packed[j]), 24u) - 23u) << 23)
+                    : looks ? static_cast<float>(count) * bin_top(b, shift) * (1.0f - 0.4f / kBinsPerBinade) * scale : 0.0f;
+                sums[0] += own_steps[j];
+                sums[1] += behind && kind[j] == kBinListed ? count : 0u;
+                sums[2] += stop_word[j] != 0xffffffffu ? 1u : 0u;
+                masses += own_mass[j];
+                previous = packed[j];
+            }
+            uint32_t totals[3];
+            bin_scan<kWalkWaves>(sums, totals, masses, shared.scan, tid);
+            stops = min(totals[2], kBinStops - 1u);
+            uint32_t prefix = sums[0], place = head_count + sums[1], stop = sums[2];
+            mass[0] = masses;
+            if (holds_bins)
+            {
+                uint32_t new_packed[4];
+                uint32_t prefixes[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    const uint32_t b = bin + j;
+                    const uint32_t count = front[j + 1] - front[j];
+                    const bool behind = b >= head_bins;
+                    mass[j + 1] = mass[j] + own_mass[j];
+                    prefixes[j] = prefix;
+                    prefix += own_steps[j];
+                    if (stop_word[j] != 0xffffffffu && stop + 1u < kBinStops)
+                        shared.stop_bin[stop] = stop_word[j];
+                    stop += stop_word[j] != 0xffffffffu ? 1u : 0u;
+                    uint32_t where = behind ? place : front[j];
+                    if (behind && kind[j] == kBinListed)
+                        place += count;
+                    if (masked[j] != 0u)
+                        where = masked[j];
+                    shared.places[b] = static_cast<uint16_t>(where);
+                    new_packed[j] = (packed[j] & 0x3fffffffu) | (kind[j] << 30);
+                }
+                *reinterpret_cast<uint4*>(shared.packed + bin) = uint4{new_packed[0], new_packed[1], new_packed[2], new_packed[3]};
+                *reinterpret_cast<uint4*>(shared.prefix + bin) = uint4{prefixes[0], prefixes[1], prefixes[2], prefixes[3]};
+            }
+            else
+            {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    mass[j + 1] = mass[j];
+            }
+            if (tid == static_cast<int>(kBinQuads) - 1)
+                shared.prefix[kBins] = prefix;
+            if (tid == 0)
+            {
+                shared.stop_bin[stops] = kBins;
+                shared.status = totals[2] >= kBinStops ? 2u : 1u;
+            }
+            // ---- the listed elements in order: a bin's elements lie side by side in the list
+            __syncthreads();
+            uint32_t fine[kPerThread];
+#pragma unroll
+            for (uint32_t k = 0; k < kPerThread; ++k)
+            {
+                fine[k] = 0u;
+                if (list_first + k * kWalkThreads + tid < listed)
+                {
+                    const uint32_t b = (kOneBits - __float_as_uint(own_terms[k])) >> shift;
+                    fine[k] = shared.places[b] - list_first + fine_place(own_terms[k], shift, packed_front(shared.packed[b + 1u]) - packed_front(shared.packed[b]));
+                }
+            }
+            order_elements<kPerThread>(shared, list_first, listed - list_first, own_terms, own_tokens, fine, tid);
+        }
+        if (shared.status == 2u)
+        {
+            leave(kBinRowLeft); // (more places to look at than the walk keeps: left to the full-order kernels)
+            continue;
+        }
+        // ---- the sums.  `head_sum`: of the sum that the next launch goes on with; `next_*`: what it runs over
+        float head_sum = 0.0f;
+        uint32_t next_limit = 0, next_cut_bin = kBins;
+        float next_cut_term = 0.0f;
+        bool top_p_done = WALK == 2;
+        bool given_up = false;
+        if constexpr (WALK == 0)
+        {
+            const uint32_t head = min(window, head_count);
+            sum_chunks<kWalkWaves>(shared.head, shared.terms, head_count, tid);
+            sum_head<kWalkWaves, 0>(shared.head, shared.terms, head, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+            float sum = same_in_all(shared.head.sum);
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+                mass[j] += sum;
+            if (behind_head)
+            {
+                walk_bins<0>(shared, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+                given_up = shared.status == 2u;
+                sum = same_in_all(shared.sum);
+            }
+            if (given_up)
+            {
+                leave(kBinRowLeft);
+                continue;
+            }
+            normalizer = sum;
+            // Min-P: the survivors are a prefix; where it ends inside the head it is known at once, else the smallest
+            // term that survives is (fp32 division is monotone, and the term is within a few ulps of threshold x normaliser)
+            uint32_t candidates = window;
+            bool candidates_known = window <= head_count;
+            if (min_p > 0.0f)
+            {
+                const float threshold = (1.0f / normalizer) * min_p;
+                const float* terms = shared.terms;
+                const uint32_t first = wave_partition_point(head, [terms, normalizer, threshold](uint32_t i) { return terms[i] / normalizer >= threshold; });
+                if (first < head)
+                {
+                    candidates = first;
+                    candidates_known = true;
+                }
+                else if (window > head_count)
+                {
+                    const float about = threshold * normalizer;
+                    if (!(about > 3.1e-8f)) // (2^-25 and some ulps: below every bin)
+                        cut_in_tail = 1u;
+                    else
+                    {
+                        const uint32_t probe = __float_as_uint(about) + static_cast<uint32_t>(tid & (kWaveSize - 1)) - 32u;
+                        const uint64_t survives = __builtin_amdgcn_ballot_w64(__uint_as_float(probe) / normalizer >= threshold);
+                        const uint32_t cut_bits = __float_as_uint(about) - 32u + static_cast<uint32_t>(__builtin_ctzll(survives | 0x8000000000000000ull));
+                        next_cut_term = __uint_as_float(cut_bits);
+                        const uint32_t below = kOneBits - cut_bits;
+                        if (below < kTailDistance)
+                            next_cut_bin = min(below >> shift, kBins);
+                    }
+                }
+            }
+            if (!candidates_known && head_count == binned)
+            {
+                // every term that is in a bin is in the head, and what lies behind moves no sum: the sum runs to the
+                // window's end, or, with a Min-P cut, over what is in the bins
+                given_up = cut_in_tail != 0u;
+                candidates = min_p > 0.0f ? binned : window;
+                candidates_known = true;
+            }
+            sum_head<kWalkWaves, 1>(shared.head, shared.terms, min(candidates, head_count), kStopAtOrAbove, top_p, normalizer, 1.0f, tid);
+            head_sum = same_in_all(shared.head.sum);
+            const uint32_t stop = same_in_all(shared.head.stop);
+            if (given_up && stop == 0xffffffffu)
+            {
+                leave(kBinRowLeft);
+                continue;
+            }
+            if (stop != 0xffffffffu || candidates_known)
+            {
+                kept = stop != 0xffffffffu ? stop + 1u : candidates;
+                renormalizer = head_sum;
+                top_p_done = true;
+            }
+            else
+                next_limit = window;
+        }
+        if constexpr (WALK == 1)
+        {
+            walk_bins<1>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
+                         normalizer, 1.0f, tid);
+            const bool stopped = shared.stopped != 0u;
+            // (a sum that no stop condition ends runs to the window's end, or to the Min-P cut, which no bin may hold)
+            given_up = shared.status == 2u || (!stopped && limit > binned && cut_in_tail != 0u);
+            if (given_up)
+            {
+                leave(kBinRowLeft);
+                continue;
+            }
+            // (behind the bins nothing moves the sum: it runs to its limit unless the cut ends it)
+            kept = stopped ? shared.stop_rank + 1u : (cut_bin < kBins ? shared.taken : (limit > binned ? limit : shared.taken));
+            kept = same_in_all(kept);
+            renormalizer = same_in_all(shared.sum);
+            top_p_done = true;
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+                mass[j] += sum_so_far;
+            __syncthreads();
+        }
+        // ---- the draw, inside the head or behind it
+        if (top_p_done)
+        {
+            uint32_t at = 0, first_of_list = 0, end_of_list = head_count;
+            const uint32_t* tokens = WALK == 1 ? sorted_tokens_out : shared.tokens;
+            bool found = kept == 1u;
+            if (WALK < 2 && !found)
+            {
+                if (WALK == 1)
+                    sum_chunks<kWalkWaves>(shared.head, shared.terms, head_count, tid);
+                sum_head<kWalkWaves, 2>(shared.head, shared.terms, min(kept, head_count), kStopAbove, uniform, normalizer, renormalizer, tid);
+                head_sum = same_in_all(shared.head.sum);
+                const uint32_t stop = same_in_all(shared.head.stop);
+                found = stop != 0xffffffffu || kept <= head_count;
+                at = stop != 0xffffffffu ? stop : kept - 1u;
+                next_limit = kept;
+            }
+            if constexpr (WALK == 2)
+            {
+                walk_bins<2>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
+                             normalizer, renormalizer, tid);
+                // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
+                at = same_in_all(shared.stop_at);
+                if (shared.status != 1u || shared.stopped == 0u || at == 0xffffffffu)
+                    continue;
+                found = true;
+                first_of_list = at >= kBinExtraPlace ? kBinExtraPlace : head_count;
+                end_of_list = at >= kBinExtraPlace ? kBinExtraPlace + same_in_all(shared.extra_count) : listed;
+            }
+            if (found)
+            {
+                if (grid.part == 0u)
+                {
+                    const int32_t token = token_of_listed<DTYPE>(a, row, shared, tokens, at, first_of_list, end_of_list, tid);
+                    if (tid == 0)
+                    {
+                        const ncnn_moe_sample_params p = a.params[row];
+                        const uint32_t flags = (counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
+                            (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u);
+                        const float term = shared.terms[at];
+                        write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, static_cast<uint8_t>(flags));
+                        a.row_state[row] = kRowDone;
+                        record.served = 1u;
+                    }
+                }
+                leave(kBinRowLeft);
+                continue;
+            }
+            if (WALK == 0 || head_count == binned)
+            {
+                // (the draw passes every term in a bin: the last element kept lies in no list)
+                leave(kBinRowLeft);
+                continue;
+            }
+        }
+        if constexpr (WALK < 2)
+        {
+            // ---- the bins' steps of the next sum: the Top-P sum's behind WALK 0, the draw's behind WALK 1
+            const float scale = 1.0f / (WALK == 0 ? normalizer : renormalizer);
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+                mass[j] *= scale;
+            BinPlan plan = plan_bins(bin, front, mass, head_bins, next_limit, next_cut_bin, WALK == 0 ? top_p : uniform, kForeseenLater);
+            uint32_t to_list[1] = {holds_bins ? plan.listed : 0u};
+            {
+                uint32_t totals[1];
+                float none = 0.0f;
+                bin_scan<kWalkWaves>(to_list, totals, none, shared.scan, tid);
+            }
+            uint32_t place[4];
+            const uint32_t own_end = fit_plan(plan, front, head_count + to_list[0], place);
+            uint32_t* const entries = shared.prefix;
+            uint32_t* const steps = shared.packed;
+            uint32_t* const masks = shared.tokens;                      // (the list has been used)
+            uint32_t* const ties = shared.tokens + 2u * kBins;
+            // the sorted head is kept for the launch behind this one
+            if (WALK == 0 && grid.part == 0u)
+            {
+                for (uint32_t i = tid; i < head_count; i += kWalkThreads)
+                {
+                    sorted_terms_out[i] = shared.terms[i];
+                    sorted_tokens_out[i] = shared.tokens[i];
+                }
+            }
+            if (tid == 0)
+                shared.listed_end = 0u;
+            __syncthreads();
+            if (tid < static_cast<int>(3u * kBinWords))
+                ties[tid] = 0u;
+            if (holds_bins)
+            {
+                reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
+                reinterpret_cast<uint4*>(masks)[kBinQuads + tid] = uint4{0u, 0u, 0u, 0u};
+                uint32_t next_packed[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    next_packed[j] = (plan.kind[j] << 30) | (plan.exponent[j] << 22) | front[j];
+                    uint32_t entry = plan.kind[j] == kBinAdded ? plan.exponent[j] : 0x40000000u;
+                    if (plan.kind[j] == kBinListed)
+                        entry = 0x80000000u | (place[j] + count_in_front_parts(g, grid, slot, bin + j));
+                    entries[bin + j] = entry;
+                }
+                *reinterpret_cast<uint4*>(steps + bin) = uint4{0u, 0u, 0u, 0u};
+                if (grid.part == 0u)
+                    reinterpret_cast<uint4*>(g.packed[kTo] + static_cast<size_t>(row) * kBins)[tid] = uint4{next_packed[0], next_packed[1], next_packed[2], next_packed[3]};
+            }
+            __syncthreads();
+            if (grid.part == 0u && own_end != 0u && holds_bins)
+                atomicMax(&shared.listed_end, own_end);
+            add_bin_steps<WALK + 1, kWalkThreads>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks,
+                                                  g.list_terms[kTo] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[kTo] + static_cast<size_t>(row) * kBinListCap, tid);
+            __syncthreads();
+            const size_t pair = slot * grid.parts + grid.part;
+            if (holds_bins)
+                reinterpret_cast<uint4*>(g.steps[kTo] + pair * kBins)[tid] = *reinterpret_cast<uint4*>(steps + bin);
+            if (tid < static_cast<int>(kBinQuads))
+            {
+                reinterpret_cast<uint4*>(g.masks[kTo] + pair * 2u * kBins)[tid] = reinterpret_cast<uint4*>(masks)[tid];
+                reinterpret_cast<uint4*>(g.masks[kTo] + pair * 2u * kBins)[kBinQuads + tid] = reinterpret_cast<uint4*>(masks)[kBinQuads + tid];
+            }
+            if (tid < static_cast<int>(3u * kBinWords))
+                g.ties[kTo][pair * 3u * kBinWords + tid] = ties[tid];
+            if (grid.part == 0u && tid == 0)
+            {
+                record.normalizer = normalizer;
+                record.renormalizer = renormalizer;
+                record.kept = kept;
+                record.head_sum[WALK] = head_sum;
+                record.limit[WALK] = next_limit;
+                record.listed[WALK + 1] = max(shared.listed_end, head_count);
+                if (WALK == 0)
+                {
+                    record.cut_bin = next_cut_bin;
+                    record.cut_term = next_cut_term;
+                    record.cut_in_tail = cut_in_tail;
+                }
+                record.state[WALK + 2] = kBinRowGoesOn;
+            }
+        }
+    }
+}
+
+// Lists the rows that the first select leaves (by_options: by their options, else those that it left pending): those with
+// a window of the window kernels' widths (null: nowhere), and the others.  One workgroup.
+__global__ __launch_bounds__(kBinThreads) void later_rows_list_kernel(SamplerArgs a, uint32_t by_options, uint32_t* windows, uint32_t* others)
+{
+    __shared__ uint32_t wave_totals[2][kBinWaves];
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6;
+    uint32_t listed[2] = {0u, 0u};
+    for (uint32_t first = 0; first < a.rows; first += kBinThreads)
+    {
+        const uint32_t row = first + static_cast<uint32_t>(tid);
+        bool mine[2] = {false, false};
+        if (row < a.rows)
+        {
+            uint32_t effective_k = 0;
+            int status = NCNN_MOE_ROW_OK;
+            const int mode = resolve_row_mode(a.params[row], a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
+            const bool left = by_options != 0u ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && a.row_state[row] == kRowNeedsGeneral;
+            const bool window = windows != nullptr && effective_k <= static_cast<uint32_t>(kSelectTopK);
+            mine[0] = left && window;
+            mine[1] = left && !window;
+        }
+        uint64_t mask[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+        {
+            mask[i] = __builtin_amdgcn_ballot_w64(mine[i]);
+            if ((tid & (kWaveSize - 1)) == 0)
+                wave_totals[i][wave] = static_cast<uint32_t>(__popcll(mask[i]));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+        {
+            uint32_t before = 0, total = 0;
+#pragma unroll
+            for (int w = 0; w < kBinWaves; ++w)
+            {
+                before += w < wave ? wave_totals[i][w] : 0u;
+                total += wave_totals[i][w];
+            }
+            uint32_t* const list = i == 0 ? windows : others;
+            if (mine[i] && list != nullptr)
+                list[1u + listed[i] + before + static_cast<uint32_t>(lanes_below(mask[i]))] = row;
+            listed[i] += total;
+        }
+        __syncthreads();
+    }
+    if (tid == 0)
+    {
+        if (windows != nullptr)
+            windows[0] = listed[0];
+        if (others != nullptr)
+            others[0] = listed[1];
+    }
+}
+
+} // namespace ncnn_moe_hip
+
+#endif // NCNN_MOE_HIP_SAMPLER_BINS_H

@@ -248,21 +248,9 @@ __device__ __constant__ const uint64_t kExp2Table[32] = {NCNN_MOE_EXP2_TABLE_VAL
 // FMA build of that routine does; the polynomial rounds identically with or without fused steps.
 // table: the 32 entries of kExp2Table, in constant memory or a copy of them in LDS (a caller on a
 // latency-critical path stages it there while it waits for something else).
-__device__ __forceinline__ float expf_libm(float x, const uint64_t* table = kExp2Table)
+// expf_of_small_argument: for |x| below 88 (the range checks are the caller's).
+__device__ __forceinline__ float expf_of_small_argument(float x, const uint64_t* table)
 {
-    const uint32_t bits = __float_as_uint(x);
-    const uint32_t abstop = (bits >> 20) & 0x7ffu;
-    if (abstop >= 0x42bu) // |x| >= 88 or not finite
-    {
-        if (bits == 0xff800000u)
-            return 0.0f;
-        if (abstop >= 0x7f8u)
-            return x + x;
-        if (x > 0x1.62e42ep6f)
-            return __uint_as_float(0x7f800000u);
-        if (x < -0x1.9fe368p6f)
-            return 0.0f;
-    }
     const double inverse_ln2_scaled = 0x1.71547652b82fep+0 * 32.0;
     const double shift = 0x1.8p+52;
     const double c0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
@@ -282,6 +270,24 @@ __device__ __forceinline__ float expf_libm(float x, const uint64_t* table = kExp
     y = fma(p, r2, y);
     y = y * scale;
     return static_cast<float>(y);
+}
+
+__device__ __forceinline__ float expf_libm(float x, const uint64_t* table = kExp2Table)
+{
+    const uint32_t bits = __float_as_uint(x);
+    const uint32_t abstop = (bits >> 20) & 0x7ffu;
+    if (abstop >= 0x42bu) // |x| >= 88 or not finite
+    {
+        if (bits == 0xff800000u)
+            return 0.0f;
+        if (abstop >= 0x7f8u)
+            return x + x;
+        if (x > 0x1.62e42ep6f)
+            return __uint_as_float(0x7f800000u);
+        if (x < -0x1.9fe368p6f)
+            return 0.0f;
+    }
+    return expf_of_small_argument(x, table);
 }
 
 // Ascending sort key for the order (logit descending, index ascending under a stable sort):

@@ -6,12 +6,17 @@
 //   general_sort_kernel    (sampler_full_order.h) full stable order of a row that has no Top-K window
 //   general_replay_kernel  and the sampler's walk over it with exactly reproduced sequential sums
 //                          (sampler_exact_sum.h).
+//   bin_*_kernel           (sampler_bins.h) the same sums without the order: rows with no Top-K window, or one wider
+//                          than 1024.
+//   window_*_kernel        (sampler_windows.h) rows with a Top-K window of 65 to 1024.
 #ifndef NCNN_MOE_HIP_SAMPLER_KERNELS_H
 #define NCNN_MOE_HIP_SAMPLER_KERNELS_H
 
+#include "sampler_bins.h"
 #include "sampler_full_order.h"
 #include "sampler_select.h"
 #include "sampler_split.h"
+#include "sampler_windows.h"
 
 namespace ncnn_moe_hip {
 

@@ -1,0 +1,467 @@
+// Rows with a Top-K window of 65 to 1024 (and narrower ones that the first select hands on): candidates, then the walk.
+//
+//   window_candidates   a row's logits are streamed once, by several workgroups, each of which keeps the logits of its part
+//                       that reach a bound and hands them over.  The bound comes from a sample of the whole row (one to
+//                       four 16-byte vectors a thread, evenly spaced): with r = row length / sample size, the sample's m-th
+//                       largest value is reached by about m r logits of the row, give or take r sqrt(m), and m solves
+//                       m r - 5.5 r sqrt(m) = K.  Every workgroup of the row works the bound out for itself.
+//   window_finish       one workgroup per row puts the candidates in order (value descending, index ascending) and walks
+//                       the window's first K: the three sums with sum_head of sampler_bins.h.
+// A row whose candidates are fewer than its window (the sample misled, or few logits are finite) or more than a list
+// holds (thousands of ties) stays pending for the full-order kernels.
+//
+// Bound: the stream at many rows (the row is read once and a part in 24 a second time), the chain sample - stream - order - sums
+// at few.  The one-workgroup-per-row select it stands in for took 65 to 115 us at any number of rows.
+#ifndef NCNN_MOE_HIP_SAMPLER_WINDOWS_H
+#define NCNN_MOE_HIP_SAMPLER_WINDOWS_H
+
+#include "sampler_bins.h"
+
+namespace ncnn_moe_hip {
+
+constexpr uint32_t kWindowListCap = 4096;        // candidates of a row
+constexpr uint32_t kWindowSampleRatio = 24;      // logits of the row per logit of the sample aimed at ...
+constexpr uint32_t kWindowSampleVectors = 4;     // ... within so many vectors a thread
+constexpr uint32_t kWindowMaxVocab = 1u << 19;   // beyond it a window of 1024 may not fit the list
+constexpr uint32_t kWindowBins = 4096;           // of the sample's histogram: the upper twelve bits of a key
+
+struct WindowArgs
+{
+    SamplerArgs a;
+    const uint32_t* list;   // the rows served: [0] their number, then the rows
+    uint32_t* counts;       // [rows] candidates; zero when a launch begins (window_finish returns them to zero)
+    uint32_t* flags;        // [rows] NaN seen; the same
+    uint32_t* keys;         // [rows][kWindowListCap]
+    uint32_t* tokens;       // [rows][kWindowListCap]
+    uint32_t windows_are_selects; // as in BinArgs
+};
+
+struct WindowCandidatesShared
+{
+    alignas(16) uint32_t counts[kWindowBins];
+    uint32_t wave_totals[kBinWaves];
+    uint32_t keys[kWindowListCap];
+    uint32_t tokens[kWindowListCap];
+    uint32_t coarse, above, bound; // the bin that holds the m-th largest sample, samples above it, the bound found
+    uint32_t count, base, saw_nan;
+};
+
+// The bin of `counts` (from the top) in which the count from the top reaches `wanted`; every thread calls it.
+template <uint32_t BINS>
+__device__ __forceinline__ void find_from_top(WindowCandidatesShared& shared, uint32_t wanted, int tid)
+{
+    constexpr uint32_t kEach = BINS / kBinThreads == 0 ? 1 : BINS / kBinThreads;
+    const int wave = tid >> 6;
+    const uint32_t first = static_cast<uint32_t>(tid) * kEach; // counted from the top
+    uint32_t own[kEach];
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; ++k)
+    {
+        own[k] = first + k < BINS ? shared.counts[BINS - 1u - (first + k)] : 0u;
+        total += own[k];
+    }
+    const uint32_t through = wave_prefix_sum_u32(total);
+    if ((tid & (kWaveSize - 1)) == kWaveSize - 1)
+        shared.wave_totals[wave] = through;
+    __syncthreads();
+    uint32_t before = through - total;
+    for (int w = 0; w < wave; ++w)
+        before += shared.wave_totals[w];
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; ++k)
+    {
+        if (before < wanted && before + own[k] >= wanted)
+        {
+            shared.coarse = BINS - 1u - (first + k);
+            shared.above = before;
+        }
+        before += own[k];
+    }
+    __syncthreads();
+}
+
+template <int DTYPE>
+__device__ __forceinline__ void window_candidates(const WindowArgs& g, const BinGrid& grid, WindowCandidatesShared& shared, int tid)
+{
+    using Vector = LogitsVector<DTYPE>;
+    constexpr uint32_t kWidth = Vector::kWidth;
+    constexpr int kLoads = DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2;
+    const SamplerArgs& a = g.a;
+    const int lane = tid & (kWaveSize - 1);
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = same_in_all(g.list[1u + slot]);
+        const uint32_t top_k = same_in_all(a.params[row].top_k);
+        const uint32_t window = top_k == 0u || top_k >= a.vocab ? a.vocab : top_k;
+        const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
+        const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
+            static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
+        // ---- the sample: vectors that lie inside the row as a whole
+        const uint32_t first_whole = (s.misalignment + kWidth - 1u) / kWidth;
+        const uint32_t whole = s.end / kWidth - min(first_whole, s.end / kWidth);
+        const uint32_t per_thread = min(kWindowSampleVectors, max(1u, whole / (kWindowSampleRatio * kBinThreads)));
+        const uint32_t sampled = min(whole, per_thread * kBinThreads);
+        if (tid == 0)
+        {
+            shared.count = 0u;
+            shared.saw_nan = 0u;
+            shared.bound = 0u;
+        }
+        for (uint32_t i = tid; i < kWindowBins / 4u; i += kBinThreads)
+            reinterpret_cast<uint4*>(shared.counts)[i] = uint4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        const auto sample_vector = [&](uint32_t k, float (&x)[kWidth]) -> bool {
+            const uint32_t i = k * kBinThreads + tid;
+            if (i >= sampled)
+                return false;
+            const uint32_t v = first_whole + static_cast<uint32_t>(static_cast<uint64_t>(i) * whole / sampled);
+            Vector::unpack(*reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u), x);
+            return true;
+        };
+        for (uint32_t k = 0; k < per_thread; ++k)
+        {
+            float x[kWidth];
+            if (sample_vector(k, x))
+            {
+#pragma unroll
+                for (uint32_t c = 0; c < kWidth; ++c)
+                {
+                    // (only what can be among the largest matters: a NaN counts as nothing)
+                    if (x[c] == x[c])
+                        atomicAdd(&shared.counts[ascending_key(x[c]) >> 20], 1u);
+                }
+            }
+        }
+        __syncthreads();
+        const float ratio = static_cast<float>(a.vocab) / static_cast<float>(max(1u, sampled * kWidth));
+        const float root = 0.5f * (5.5f + sqrtf(30.25f + 4.0f * static_cast<float>(window) / ratio));
+        const uint32_t wanted = sampled == whole ? min(window, sampled * kWidth) : min(static_cast<uint32_t>(root * root) + 1u, sampled * kWidth);
+        const bool everything = sampled * kWidth < window + 2u * kWidth; // a short row: its few logits are all candidates
+        if (!everything)
+        {
+            if (tid == 0)
+                shared.coarse = 0u, shared.above = 0u;
+            __syncthreads();
+            find_from_top<kWindowBins>(shared, wanted, tid);
+            const uint32_t coarse = shared.coarse;
+            const uint32_t still = wanted - shared.above;
+            __syncthreads();
+            // the next eight bits of the samples in that bin
+            if (tid < 256)
+                shared.counts[tid] = 0u;
+            __syncthreads();
+            for (uint32_t k = 0; k < per_thread; ++k)
+            {
+                float x[kWidth];
+                if (sample_vector(k, x))
+                {
+#pragma unroll
+                    for (uint32_t c = 0; c < kWidth; ++c)
+                    {
+                        const uint32_t key = ascending_key(x[c]);
+                        if (x[c] == x[c] && key >> 20 == coarse)
+                            atomicAdd(&shared.counts[(key >> 12) & 255u], 1u);
+                    }
+                }
+            }
+            if (tid == 0)
+                shared.coarse = 0u, shared.above = 0u;
+            __syncthreads();
+            find_from_top<256>(shared, still, tid);
+            if (tid == 0)
+                shared.bound = (coarse << 20) | (shared.coarse << 12);
+            __syncthreads();
+        }
+        // (an infinite logit below everything is no candidate: the window counts finite logits)
+        const float bound = value_from_ascending_key(max(shared.bound, ascending_key(-3.402823466e38f)));
+        // ---- the part's logits at or above it
+        const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
+        bool saw_nan = false;
+        for (uint32_t at = first + tid; at < last + kBinThreads; at += kLoads * kBinThreads)
+        {
+            // (whole waves stay in the loop: its appends are theirs)
+            if (at - lane >= last)
+                break;
+            uint4 raw[kLoads];
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k)
+                raw[k] = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(min(at + k * kBinThreads, last - 1u)) * 16u);
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k)
+            {
+                const uint32_t v = at + k * kBinThreads;
+                float x[kWidth];
+                Vector::unpack(raw[k], x);
+                const uint32_t position = v * kWidth;
+                uint32_t hits = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < kWidth; ++c)
+                {
+                    const bool inside = v < last && position + c - s.misalignment < a.vocab;
+                    hits |= inside && x[c] >= bound ? 1u << c : 0u;
+                    saw_nan = saw_nan || (inside && x[c] != x[c]);
+                }
+                if (__builtin_amdgcn_ballot_w64(hits != 0u) != 0ull)
+                {
+                    const uint32_t own = static_cast<uint32_t>(__popc(hits));
+                    const uint32_t through = wave_prefix_sum_u32(own);
+                    uint32_t place = 0;
+                    if (lane == kWaveSize - 1)
+                        place = atomicAdd(&shared.count, through);
+                    place = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(place), kWaveSize - 1)) + through - own;
+#pragma unroll
+                    for (uint32_t c = 0; c < kWidth; ++c)
+                    {
+                        if ((hits >> c & 1u) != 0u)
+                        {
+                            if (place < kWindowListCap)
+                            {
+                                shared.keys[place] = ascending_key(x[c]);
+                                shared.tokens[place] = position + c - s.misalignment;
+                            }
+                            ++place;
+                        }
+                    }
+                }
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(saw_nan) != 0ull && lane == 0)
+            shared.saw_nan = 1u;
+        __syncthreads();
+        // ---- handed over: one counter per row
+        const uint32_t count = shared.count;
+        if (tid == 0)
+        {
+            shared.base = count != 0u ? atomicAdd(&g.counts[row], count) : 0u;
+            if (shared.saw_nan != 0u)
+                atomicOr(&g.flags[row], 1u);
+        }
+        __syncthreads();
+        const uint32_t place = shared.base;
+        for (uint32_t i = tid; i < min(count, kWindowListCap); i += kBinThreads)
+        {
+            if (place + i < kWindowListCap)
+            {
+                g.keys[static_cast<size_t>(row) * kWindowListCap + place + i] = shared.keys[i];
+                g.tokens[static_cast<size_t>(row) * kWindowListCap + place + i] = shared.tokens[i];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+struct WindowFinishShared
+{
+    alignas(16) uint32_t keys[kWindowListCap];
+    alignas(16) uint32_t tokens[kWindowListCap];
+    uint32_t counters[kWindowListCap];
+    alignas(16) float terms[kSelectTopK];
+    HeadScratch head;
+    BinScanScratch scan;
+    uint32_t least, most;
+    uint64_t exp2_table[32];
+};
+
+// One row's candidates to its result.  WAVES waves call it.
+template <int DTYPE, int WAVES>
+__device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row, WindowFinishShared& shared, int tid)
+{
+    constexpr uint32_t kThreads = WAVES * kWaveSize;
+    constexpr uint32_t kPerThread = kWindowListCap / kThreads;
+    const SamplerArgs& a = g.a;
+    const uint32_t count = same_in_all(g.counts[row]);
+    const bool saw_nan = same_in_all(g.flags[row]) != 0u;
+    const ncnn_moe_sample_params p = a.params[row];
+    const float uniform = same_in_all(a.uniforms[row]);
+    const uint32_t window = p.top_k == 0u || p.top_k >= a.vocab ? a.vocab : p.top_k;
+    if (tid < 32)
+        shared.exp2_table[tid] = kExp2Table[tid];
+    if (tid == 0)
+    {
+        shared.least = 0xffffffffu;
+        shared.most = 0u;
+    }
+    __syncthreads(); // (every thread has read the counters)
+    if (tid == 0)
+    {
+        g.counts[row] = 0u;
+        g.flags[row] = 0u;
+    }
+    // fewer candidates than the window, and logits below the bound: the sample misled.  (A row of few finite logits, or
+    // one shorter than its window, is left as well.)
+    if (count > kWindowListCap || count < window)
+        return;
+    uint32_t keys[kPerThread], tokens[kPerThread];
+    uint32_t least = 0xffffffffu, most = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+    {
+        const uint32_t i = k * kThreads + tid;
+        keys[k] = i < count ? g.keys[static_cast<size_t>(row) * kWindowListCap + i] : 0u;
+        tokens[k] = i < count ? g.tokens[static_cast<size_t>(row) * kWindowListCap + i] : 0u;
+        least = i < count ? min(least, keys[k]) : least;
+        most = max(most, keys[k]);
+        if (i < count)
+            shared.counters[i] = 0u;
+    }
+    most = wave_max_u32(most);
+    least = ~wave_max_u32(~least);
+    if ((tid & (kWaveSize - 1)) == 0)
+    {
+        atomicMax(&shared.most, most);
+        atomicMin(&shared.least, least);
+    }
+    __syncthreads();
+    most = same_in_all(shared.most);
+    least = same_in_all(shared.least);
+    uint8_t flags = counts_as_select(g.windows_are_selects, a.vocab, p) ? 0 : NCNN_MOE_ROW_FLAG_GENERAL_PATH;
+    if (saw_nan)
+        flags |= NCNN_MOE_ROW_FLAG_HAS_NAN;
+    const float largest = value_from_ascending_key(most);
+    const float maximum = largest / p.temperature;
+    if (!is_finite_f32(largest))
+    {
+        if (tid == 0)
+        {
+            write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags);
+            a.row_state[row] = kRowDone;
+        }
+        return;
+    }
+    if (!is_finite_f32(maximum))
+        return;
+    // ---- in order: about where a candidate belongs by its value, then against those that belong in the same place
+    const float smallest = value_from_ascending_key(least);
+    const float scale = largest > smallest ? static_cast<float>(count) / (largest - smallest) : 0.0f;
+    uint32_t fine[kPerThread], turn[kPerThread];
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+    {
+        fine[k] = turn[k] = 0u;
+        if (k * kThreads + tid < count)
+        {
+            fine[k] = min(count - 1u, static_cast<uint32_t>((largest - value_from_ascending_key(keys[k])) * scale));
+            turn[k] = atomicAdd(&shared.counters[fine[k]], 1u);
+        }
+    }
+    __syncthreads();
+    {
+        uint32_t held[kPerThread];
+        uint32_t total[1] = {0u};
+        const uint32_t first = tid * kPerThread;
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            held[k] = first + k < count ? shared.counters[first + k] : 0u;
+            total[0] += held[k];
+        }
+        uint32_t totals[1];
+        float none = 0.0f;
+        bin_scan<WAVES>(total, totals, none, shared.scan, tid);
+        uint32_t front = total[0];
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            if (first + k < count)
+                shared.counters[first + k] = front;
+            front += held[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+    {
+        if (k * kThreads + tid < count)
+        {
+            const uint32_t at = shared.counters[fine[k]] + turn[k];
+            shared.keys[at] = keys[k];
+            shared.tokens[at] = tokens[k];
+        }
+    }
+    __syncthreads();
+    uint32_t rank[kPerThread];
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+    {
+        rank[k] = 0u;
+        if (k * kThreads + tid < count)
+        {
+            const uint32_t low = shared.counters[fine[k]];
+            const uint32_t high = fine[k] + 1u < count ? shared.counters[fine[k] + 1u] : count;
+            rank[k] = low;
+            if (low < window) // (what lies behind the window need not be in order)
+            {
+                for (uint32_t j = low; j < high; ++j)
+                {
+                    const uint32_t other = shared.keys[j];
+                    rank[k] += other > keys[k] || (other == keys[k] && shared.tokens[j] < tokens[k]) ? 1u : 0u;
+                }
+            }
+            else
+                rank[k] = window;
+        }
+    }
+    __syncthreads();
+    // ---- the window: its tokens and terms
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+    {
+        if (k * kThreads + tid < count && rank[k] < window)
+        {
+            shared.tokens[rank[k]] = tokens[k];
+            shared.terms[rank[k]] = expf_libm(value_from_ascending_key(keys[k]) / p.temperature - maximum, shared.exp2_table);
+        }
+    }
+    __syncthreads();
+    sum_chunks<WAVES>(shared.head, shared.terms, window, tid);
+    sum_head<WAVES, 0>(shared.head, shared.terms, window, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+    const float normalizer = same_in_all(shared.head.sum);
+    uint32_t candidates = window;
+    if (p.min_p > 0.0f)
+    {
+        const float threshold = (1.0f / normalizer) * p.min_p;
+        const float* terms = shared.terms;
+        candidates = wave_partition_point(window, [terms, normalizer, threshold](uint32_t i) { return terms[i] / normalizer >= threshold; });
+    }
+    sum_head<WAVES, 1>(shared.head, shared.terms, candidates, kStopAtOrAbove, p.top_p, normalizer, 1.0f, tid);
+    const float renormalizer = same_in_all(shared.head.sum);
+    const uint32_t top_p_stop = same_in_all(shared.head.stop);
+    const uint32_t kept = top_p_stop != 0xffffffffu ? top_p_stop + 1u : candidates;
+    uint32_t selected = 0;
+    if (kept > 1u)
+    {
+        sum_head<WAVES, 2>(shared.head, shared.terms, kept, kStopAbove, uniform, normalizer, renormalizer, tid);
+        const uint32_t stop = same_in_all(shared.head.stop);
+        selected = stop != 0xffffffffu ? stop : kept - 1u;
+    }
+    if (tid == 0)
+    {
+        const float probability = kept == 1u ? 1.0f : (shared.terms[selected] / normalizer) / renormalizer;
+        write_token(a, row, p, static_cast<int32_t>(shared.tokens[selected]), probability, kept, kept == 1u ? 0 : 1, flags);
+        a.row_state[row] = kRowDone;
+    }
+}
+
+template <int DTYPE>
+__global__ __launch_bounds__(kBinThreads) void window_candidates_kernel(WindowArgs g)
+{
+    __shared__ WindowCandidatesShared shared;
+    window_candidates<DTYPE>(g, bin_grid(g.list, g.a.vocab), shared, threadIdx.x);
+}
+
+template <int DTYPE>
+__global__ __launch_bounds__(kWalkThreads) void window_finish_kernel(WindowArgs g)
+{
+    __shared__ WindowFinishShared shared;
+    const uint32_t rows = same_in_all(g.list[0]);
+    for (uint32_t slot = blockIdx.x; slot < rows; slot += gridDim.x)
+    {
+        window_finish<DTYPE, kWalkWaves>(g, same_in_all(g.list[1u + slot]), shared, threadIdx.x);
+        __syncthreads();
+    }
+}
+
+} // namespace ncnn_moe_hip
+
+#endif // NCNN_MOE_HIP_SAMPLER_WINDOWS_H

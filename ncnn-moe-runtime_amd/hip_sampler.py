@@ -71,6 +71,8 @@ EXPORTED_SYMBOLS = [
 TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_force_general",
     "ncnn_moe_hip_sampler_debug_scatter_segments",
+    "ncnn_moe_hip_sampler_debug_binned_sums",
+    "ncnn_moe_hip_sampler_debug_binned_rows",
     "ncnn_moe_hip_sampler_debug_spread_sort",
     "ncnn_moe_hip_sampler_debug_fused_bf16",
     "ncnn_moe_hip_sampler_debug_partial_sort",
@@ -122,6 +124,8 @@ def _bind(lib, testing):
         return lib
     lib.ncnn_moe_hip_sampler_debug_force_general.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
+    lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
+    lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_spread_sort.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_partial_sort.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_sort_lengths.argtypes = [vp, vp, ctypes.c_uint32]
@@ -335,6 +339,17 @@ class HipSampler:
     def chunk_steps(self, enabled):
         """Test hook: whole chunks of a sorted fp32 row added in one precomputed step (default) or round by round."""
         self._check(self._hooks().ncnn_moe_hip_sampler_debug_chunk_steps(self._handle, 1 if enabled else 0))
+
+    def binned_sums(self, enabled):
+        """Test hook: rows that the first select leaves are served without an order of their logits (the shipped
+        library's way; off by default in the testing build) or sorted."""
+        self._check(self._hooks().ncnn_moe_hip_sampler_debug_binned_sums(self._handle, 1 if enabled else 0))
+
+    def binned_rows(self, rows):
+        """Test hook: which of the handle's first `rows` rows the binned sums finished (1) the last time they were given them."""
+        out = np.empty(rows, dtype=np.uint32)
+        self._check(self._hooks(True).ncnn_moe_hip_sampler_debug_binned_rows(self._handle, out.ctypes.data, rows))
+        return out
 
     def spread_sort(self, enabled):
         """Test hook: the radix sort of long full-order rows on several workgroups (default) or on one."""

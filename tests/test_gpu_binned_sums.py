@@ -1,0 +1,72 @@
+"""Rows that the first select leaves, served by the window kernels and by sums over unordered bins of terms (GPU): the
+oracle's results, on rows where the sums cross many binades, end inside the sorted head or far behind it, meet terms half way between two sums,
+ties, cuts and windows, at the sizes where the parts and bins of a row begin and end."""
+import numpy as np
+import pytest
+
+import parity_util
+from ncnn_moe_runtime_amd import hip_sampler, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def _batch(rng, rows, vocab, top_k):
+    logits = (rng.standard_normal((rows, vocab)) * rng.uniform(0.3, 3.0, (rows, 1))).astype(np.float32)
+    kinds = np.arange(rows) % 8
+    logits[kinds == 1] = np.round(logits[kinds == 1] * 16) / 16          # a few hundred values: large bins of equal terms
+    logits[kinds == 2, ::97] += np.float32(9.0)                           # a peaked row
+    logits[kinds == 3, vocab // 3:] = -np.inf                             # a masked vocabulary
+    logits[kinds == 4] = logits[kinds == 4] * np.float32(0.01) + np.float32(40.0)  # narrow: every term in one binade
+    logits[kinds == 5, vocab // 2] = np.nan
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["temperature"] = rng.choice(np.array([0.2, 0.7, 1.0, 1.3, 2.5], dtype=np.float32), rows)
+    params["top_k"] = rng.choice(np.array(top_k, dtype=np.uint32), rows)
+    params["top_p"] = rng.choice(np.array([0.3, 0.8, 0.95, 0.999, 1.0], dtype=np.float32), rows)
+    params["min_p"] = rng.choice(np.array([0.0, 0.0, 1e-4, 0.02], dtype=np.float32), rows)
+    return logits, params, rng.random(rows, dtype=np.float32)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,vocab", [(1, 151936), (3, 2047), (9, 8193), (8, 100003), (40, 32771), (130, 16411), (520, 2049)])
+def test_binned_sums_match_the_oracle(dtype, rows, vocab):
+    rng = np.random.default_rng(rows * 1000003 + vocab)
+    # (bf16 rows without a window have a kernel of their own)
+    top_k = [0, 0, 65, 1000, 1025, 5000, vocab - 1] if dtype == "f32" else [65, 200, 700, 1024]
+    print("[case] binned sums, %d x %d %s" % (rows, vocab, dtype), flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, top_k)
+    data = workloads.float32_to_bf16_bits(logits) if dtype == "bf16" else logits
+    cpu = parity_util.run_oracle(data, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.upload_logits(data)
+        sorted_way = sampler.sample(params, uniforms)
+        sampler.binned_sums(True)
+        gpu = sampler.sample(params, uniforms)
+        windows = (params["top_k"] > 0) & (params["top_k"] <= 1024) | (vocab <= 1024)
+        general = (gpu["flags"] & hip_sampler.FLAG_GENERAL_PATH) != 0
+        served = np.where(windows, ~general, sampler.binned_rows(rows) == 1)
+        again = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, dtype, "binned sums")
+    for field in ("token_id", "probability", "kept_count", "status", "draw_consumed"):
+        assert gpu[field].tobytes() == sorted_way[field].tobytes(), field
+    assert gpu.tobytes() == again.tobytes()
+    # what is left to the sort is the exception: thousands of equal terms, and draws that no partial sum exceeds
+    assert served.sum() >= rows - 1 - rows // 5, (served, rows)
+
+
+def test_draws_and_cuts_at_the_ends():
+    """Draws at the ends of [0, 1), Min-P cuts at and behind the last bin, a Top-P that the first element meets."""
+    rng = np.random.default_rng(99)
+    rows, vocab = 24, 50021
+    logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 3000])
+    uniforms[0::3] = 0.0
+    uniforms[1::3] = np.float32(1.0) - np.float32(2.0 ** -24)
+    params["min_p"][2::4] = np.float32(1e-7)
+    params["min_p"][3::4] = np.float32(1e-30)
+    params["top_p"][::5] = np.float32(1e-6)
+    params["min_p"][::7] = 1.0
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, "f32", "ends")
