@@ -104,6 +104,7 @@ struct ncnn_moe_hip_sampler
     int32_t* verify_long_ids = nullptr;
     float* verify_long_probabilities = nullptr;
     float* verify_dense = nullptr;
+    VerifySumsArgs verify_sums{}; // scratch of a step over rows that the binned sums served
     // the options of the last step that needed them: the next step with the same options goes there at once
     bool verify_dense_known = false;
     ncnn_moe_sample_params verify_dense_options{};
@@ -294,7 +295,7 @@ struct SamplerPasses
 // Enqueues what follows the first select: the window kernels (sampler_windows.h) and the binned sums (sampler_bins.h) for
 // the rows that it left pending; by_options: for those that it leaves by their options.
 template <int DTYPE>
-void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool sums, bool by_options, hipStream_t stream)
+void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool sums, bool by_options, bool want_filters, hipStream_t stream)
 {
     hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, by_options ? 1u : 0u,
                        windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
@@ -311,6 +312,7 @@ void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windo
         BinArgs g = s->bins;
         g.a = a;
         g.windows_are_selects = windows ? 1u : 0u;
+        g.want_filters = want_filters ? 1u : 0u;
         hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
         hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
         hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
@@ -320,11 +322,12 @@ void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windo
     }
 }
 
-// Enqueues the sampling path for `rows` rows.
+// Enqueues the sampling path for `rows` rows.  want_filters: the rows without a window leave their filtered distributions
+// in the binned sums' records (bf16 rows too).
 int launch_sampler(
     ncnn_moe_hip_sampler* s, const void* logits, int dtype, uint32_t rows, uint32_t vocab, uint64_t row_stride,
     const ncnn_moe_sample_params* params, const float* uniforms, const int32_t* stop_ids,
-    ncnn_moe_sample_result* results, DistributionExport export_to, SamplerPasses passes, hipStream_t stream)
+    ncnn_moe_sample_result* results, DistributionExport export_to, SamplerPasses passes, hipStream_t stream, bool want_filters = false)
 {
     const bool want_distribution = export_to.count != nullptr;
     SamplerArgs a;
@@ -380,18 +383,18 @@ int launch_sampler(
     // kernel of their own); what they leave pending goes to the full-order kernels.  A call that exports distributions
     // needs the order itself.
     const bool windows = passes.wide_select && vocab <= kWindowMaxVocab;
-    const bool sums = passes.full_order && dtype == NCNN_MOE_LOGITS_F32 && vocab <= kBinMaxVocab;
+    const bool sums = passes.full_order && (dtype == NCNN_MOE_LOGITS_F32 || want_filters) && vocab <= kBinMaxVocab;
     if (s->binned_sums != 0 && passes.select && !want_distribution && (windows || sums) && windows == passes.wide_select)
     {
         if (dtype == NCNN_MOE_LOGITS_F32)
         {
             launch_select<NCNN_MOE_LOGITS_F32>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
-            launch_later_rows<NCNN_MOE_LOGITS_F32>(s, a, windows, sums, passes.side_by_side, stream);
+            launch_later_rows<NCNN_MOE_LOGITS_F32>(s, a, windows, sums, passes.side_by_side, want_filters, stream);
         }
         else
         {
             launch_select<NCNN_MOE_LOGITS_BF16>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
-            launch_later_rows<NCNN_MOE_LOGITS_BF16>(s, a, windows, false, passes.side_by_side, stream);
+            launch_later_rows<NCNN_MOE_LOGITS_BF16>(s, a, windows, sums, passes.side_by_side, want_filters, stream);
         }
         if (passes.full_order)
         {
@@ -773,6 +776,14 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
         place(&s->verify_long_ids, long_rows * max_vocab * sizeof(int32_t));
         place(&s->verify_long_probabilities, long_rows * max_vocab * sizeof(float));
         place(&s->verify_dense, 2 * static_cast<size_t>(max_vocab) * sizeof(float));
+        const size_t chunks = (static_cast<size_t>(max_vocab) + kResidualChunk - 1) / kResidualChunk;
+        place(&s->verify_sums.residual, chunks * kResidualChunk * sizeof(float));
+        place(&s->verify_sums.sub_sums, chunks * kWaveSize * sizeof(float));
+        place(&s->verify_sums.sub_steps, chunks * kWaveSize * sizeof(uint4));
+        place(&s->verify_sums.chunk_steps, chunks * sizeof(uint4));
+        place(&s->verify_sums.chunk_sums, chunks * sizeof(double));
+        place(&s->verify_sums.chunk_last, chunks * sizeof(int32_t));
+        place(&s->verify_sums.decision, 4 * sizeof(uint32_t));
     }
     place(&s->single_params, sizeof(ncnn_moe_sample_params));
     place(&s->single_uniform, sizeof(float));
@@ -1201,6 +1212,45 @@ int ncnn_moe_hip_sampler_speculative_verify(
     SamplerPasses passes;
     passes.full_order = s->force_general != 0 || row_left_pending(row_options, s->logits_vocab, kSelectTopK);
     passes.wide_select = !passes.full_order && row_left_pending(row_options, s->logits_vocab, kFastTopK);
+    // Rows without a window: the binned sums leave each row's filtered distribution as a few numbers, and the step needs
+    // no lists.  (A row that they leave to the sort has the step run again below.)
+    if (s->binned_sums != 0 && s->force_general == 0 && passes.full_order && s->logits_vocab <= kBinMaxVocab)
+    {
+        SamplerPasses every_row;
+        every_row.full_order = true;
+        const int rc = launch_sampler(
+            s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
+            s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, DistributionExport{}, every_row, s->stream, true);
+        if (rc != NCNN_MOE_SAMPLER_SUCCESS)
+            return rc;
+        VerifySumsArgs d = s->verify_sums;
+        d.a.logits = s->logits;
+        d.a.row_stride = s->logits_stride;
+        d.a.vocab = s->logits_vocab;
+        d.a.results = s->results;
+        d.records = s->bins.records;
+        d.draft_count = draft_count;
+        d.temperature = row_options.temperature;
+        d.proposed = v.proposed;
+        d.uniforms = v.uniforms;
+        d.accepted_probabilities = v.accepted_probabilities;
+        d.result = v.result;
+        const uint32_t chunks = (s->logits_vocab + kResidualChunk - 1) / kResidualChunk;
+        if (s->logits_dtype == NCNN_MOE_LOGITS_F32)
+            hipLaunchKernelGGL((verify_residual_kernel<NCNN_MOE_LOGITS_F32>), dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
+        else
+            hipLaunchKernelGGL((verify_residual_kernel<NCNN_MOE_LOGITS_BF16>), dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
+        hipLaunchKernelGGL(verify_steps_kernel, dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
+        hipLaunchKernelGGL(verify_draw_kernel, dim3(1), dim3(kResidualThreads), 0, s->stream, d, chunks);
+        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+        if (s->verify_output_host->result.status != NCNN_MOE_VERIFY_UNSUPPORTED_WINDOW)
+        {
+            *result = s->verify_output_host->result;
+            std::memcpy(accepted_probabilities, s->verify_output_host->accepted, draft_count * sizeof(float));
+            return NCNN_MOE_SAMPLER_SUCCESS;
+        }
+    }
     bool dense = s->verify_dense_known && std::memcmp(&s->verify_dense_options, &row_options, sizeof(row_options)) == 0;
     for (int attempt = 0; attempt < 2 && !dense; ++attempt)
     {

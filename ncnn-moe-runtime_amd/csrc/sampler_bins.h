@@ -101,6 +101,12 @@ struct BinRow
     float renormalizer;
     uint32_t kept;
     uint32_t served;        // the row was finished here
+    // the filtered distribution, where BinArgs::want_filters asks for it: probability((exp(logit/T - maximum) / normalizer)
+    // / renormalizer) of the elements kept, which are those up to filter_key, filter_token in the row's order
+    uint32_t filtered;
+    float maximum;
+    uint32_t filter_key;    // descending key
+    uint32_t filter_token;
 };
 
 struct BinArgs
@@ -118,6 +124,7 @@ struct BinArgs
     float* head_terms;     // [rows][kBinListCap], sorted
     uint32_t* head_tokens;
     BinRow* records;       // [rows]
+    uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
 };
 
@@ -307,6 +314,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_terms_kernel(BinArgs g)
             record.shift = shift;
             record.window = (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite;
             record.served = 0u;
+            record.filtered = 0u;
+            record.maximum = maximum;
             record.saw_nan = (flags & kScanSawNan) != 0u ? 1u : 0u;
             if (rejected)
             {
@@ -1888,6 +1897,35 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
 #pragma unroll
             for (int j = 0; j < 5; ++j)
                 mass[j] += sum_so_far;
+            __syncthreads();
+        }
+        if (WALK < 2 && g.want_filters != 0u && top_p_done && grid.part == 0u)
+        {
+            // the last element kept: in the head, where the Top-P sum stopped, or (no stop, no cut, no window) the last
+            // finite one; a row whose last element lies elsewhere gets no filter
+            const bool in_head = kept <= head_count;
+            const uint32_t last = in_head ? kept - 1u : WALK == 1 && shared.stopped != 0u ? same_in_all(shared.stop_at) : 0xffffffffu;
+            const bool everything = !in_head && kept == window && (WALK == 0 || shared.stopped == 0u) && min_p == 0.0f &&
+                (a.params[row].top_k == 0u || a.params[row].top_k >= a.vocab);
+            uint32_t filter_key = kLastFiniteKey, filter_token = a.vocab;
+            if (last != 0xffffffffu)
+            {
+                const bool extra = WALK == 1 && last >= kBinExtraPlace;
+                const uint32_t first_of_list = extra ? kBinExtraPlace : WALK == 1 && !in_head ? head_count : 0u;
+                const uint32_t end_of_list = extra ? kBinExtraPlace + same_in_all(shared.extra_count) : WALK == 1 && !in_head ? listed : head_count;
+                const int32_t token = token_of_listed<DTYPE>(a, row, shared, WALK == 1 && in_head ? sorted_tokens_out : shared.tokens, last, first_of_list, end_of_list, tid);
+                filter_token = static_cast<uint32_t>(token);
+                filter_key = descending_key(load_logit<DTYPE>(static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes, filter_token));
+            }
+            if (tid == 0 && (last != 0xffffffffu || everything))
+            {
+                record.normalizer = normalizer;
+                record.renormalizer = renormalizer;
+                record.kept = kept;
+                record.filter_key = filter_key;
+                record.filter_token = filter_token;
+                record.filtered = 1u;
+            }
             __syncthreads();
         }
         // ---- the draw, inside the head or behind it

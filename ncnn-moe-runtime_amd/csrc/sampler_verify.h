@@ -4,8 +4,7 @@
 #ifndef NCNN_MOE_HIP_SAMPLER_VERIFY_H
 #define NCNN_MOE_HIP_SAMPLER_VERIFY_H
 
-#include "sampler_common.h"
-#include "sampler_exact_sum.h"
+#include "sampler_bins.h"
 
 namespace ncnn_moe_hip {
 
@@ -443,6 +442,384 @@ __global__ __launch_bounds__(kReplayThreads) void speculative_verify_dense_kerne
             write_verify_result(v, accepted, next.token_id, next.probability, NCNN_MOE_VERIFY_OK, 0, accept_draws,
                                 next.draw_consumed, 0);
     }
+}
+
+// The same step for rows that the binned sums served (no Top-K window): each row's filtered distribution is known as its
+// three sums and its last element kept, so a token's probability needs its logit alone, and nothing is listed.  A
+// rejection's residual is a dense vector over the vocabulary, made, summed and walked by three launches, a workgroup per
+// 4,096 entries:
+//   verify_residual_kernel  the accept loop (every workgroup walks it for itself; the first writes the outcome), and on a
+//                           rejection the entries of max(0, target - draft) and their plain sums per 64
+//   verify_steps_kernel     what each 64 entries do to a running sum of the exponent that those plain sums foretell, and
+//                           what each 4,096 do
+//   verify_draw_kernel      the exact sum over the composed steps (entries are looked at only where it leaves its binade),
+//                           then the draw inside the one stretch whose partial sums pass it
+// What bounds it: launches and trips to memory (the step reads 1.3 MB of logits and 0.6 MB of residual).  With exported
+// lists, a pair sort of every row and one workgroup for the residual a step of 5 drafts over 151,936 logits took 640 us.
+constexpr uint32_t kResidualSub = kWaveSize;
+constexpr uint32_t kResidualChunk = kWaveSize * kResidualSub;
+constexpr int kResidualThreads = 512;
+constexpr uint32_t kResidualEach = kResidualChunk / kResidualThreads;
+
+struct VerifySumsArgs
+{
+    SamplerArgs a;                 // logits and options of the 2 * draft_count + 1 rows
+    const BinRow* records;         // their filters
+    uint32_t draft_count;
+    float temperature;
+    const int32_t* proposed;       // [draft_count]
+    const float* uniforms;         // [draft_count + 1]
+    float* accepted_probabilities; // [draft_count]
+    ncnn_moe_verify_result* result;
+    float* residual;               // [chunks][kResidualChunk]
+    float* sub_sums;               // [chunks][kWaveSize]
+    uint4* sub_steps;              // [chunks][kWaveSize]: exponent, step on an even mantissa, step on an odd one
+    uint4* chunk_steps;            // [chunks]
+    double* chunk_sums;            // [chunks]
+    int32_t* chunk_last;           // [chunks]: the last entry that holds mass, -1 for none
+    uint32_t* decision;            // [0] 1: rejected, the residual decides; [1] positions accepted; [2] uniforms used
+};
+
+// The probability of a token in a row's filtered distribution (0 for one that is not in it).
+template <int DTYPE>
+__device__ __forceinline__ float filtered_probability(const void* row_pointer, uint32_t token, const BinRow& filter, float temperature, const uint64_t* exp2_table)
+{
+    const float value = load_logit<DTYPE>(row_pointer, token);
+    const uint32_t key = descending_key(value);
+    if (key > filter.filter_key || (key == filter.filter_key && token > filter.filter_token))
+        return 0.0f;
+    return (expf_libm(value / temperature - filter.maximum, exp2_table) / filter.normalizer) / filter.renormalizer;
+}
+
+struct VerifyWalkShared
+{
+    float found[2 * NCNN_MOE_MAX_DRAFT_TOKENS];
+    ncnn_moe_sample_result row_results[2 * NCNN_MOE_MAX_DRAFT_TOKENS + 1];
+    BinRow filters[2 * NCNN_MOE_MAX_DRAFT_TOKENS + 1];
+    float uniforms[NCNN_MOE_MAX_DRAFT_TOKENS + 1];
+    float wave_sums[kResidualThreads / kWaveSize];
+    int32_t last;
+    uint64_t exp2_table[32];
+};
+
+template <int DTYPE>
+__global__ __launch_bounds__(kResidualThreads) void verify_residual_kernel(VerifySumsArgs v)
+{
+    __shared__ VerifyWalkShared shared;
+    const SamplerArgs& a = v.a;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWaveSize - 1);
+    const uint32_t drafts = v.draft_count;
+    const uint32_t rows = 2u * drafts + 1u;
+    const bool writes = blockIdx.x == 0u && tid == 0;
+    const auto row_pointer = [&a](uint32_t row) {
+        return static_cast<const void*>(static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes);
+    };
+    const auto outcome = [&](uint32_t accepted, int32_t token, float probability, uint32_t status, uint32_t row_status, uint32_t accept_draws, uint32_t final_draw) {
+        if (!writes)
+            return;
+        v.decision[0] = 0u;
+        ncnn_moe_verify_result r;
+        r.accepted = accepted;
+        r.next_token_id = status == NCNN_MOE_VERIFY_OK ? token : -1;
+        r.next_probability = status == NCNN_MOE_VERIFY_OK ? probability : 0.0f;
+        r.status = status;
+        r.row_status = row_status;
+        r.accept_draws = accept_draws;
+        r.final_draw_consumed = final_draw;
+        r.next_is_residual = 0;
+        *v.result = r;
+    };
+    if (static_cast<uint32_t>(tid) < rows)
+    {
+        shared.row_results[tid] = a.results[tid];
+        shared.filters[tid] = v.records[tid];
+    }
+    if (static_cast<uint32_t>(tid) <= drafts)
+        shared.uniforms[tid] = v.uniforms[tid];
+    if (tid >= kWaveSize && tid < kWaveSize + 32)
+        shared.exp2_table[tid - kWaveSize] = kExp2Table[tid - kWaveSize];
+    if (tid == 0)
+        shared.last = -1;
+    __syncthreads();
+    // candidate_probability (session.cpp:138-148) of every proposed token: the targets', then the drafts'
+    if (static_cast<uint32_t>(tid) < 2u * drafts)
+    {
+        const uint32_t i = static_cast<uint32_t>(tid) % drafts;
+        const uint32_t row = static_cast<uint32_t>(tid) < drafts ? i : drafts + 1u + i;
+        const uint32_t token = static_cast<uint32_t>(v.proposed[i]);
+        shared.found[tid] = token < a.vocab && shared.filters[row].filtered != 0u
+            ? filtered_probability<DTYPE>(row_pointer(row), token, shared.filters[row], v.temperature, shared.exp2_table) : 0.0f;
+    }
+    __syncthreads();
+    // ---- session.cpp:797-842: accept with probability min(1, target / draft)
+    uint32_t accepted = 0;
+    for (; accepted < drafts; ++accepted)
+    {
+        const ncnn_moe_sample_result target = shared.row_results[accepted];
+        const ncnn_moe_sample_result draft = shared.row_results[drafts + 1u + accepted];
+        if (target.status != NCNN_MOE_ROW_OK || draft.status != NCNN_MOE_ROW_OK)
+            return outcome(accepted, -1, 0.0f, NCNN_MOE_VERIFY_ROW_ERROR, target.status != NCNN_MOE_ROW_OK ? target.status : draft.status, accepted, 0);
+        // (a row that the sort served has no filter: the step is run again with exported lists)
+        if (shared.filters[accepted].filtered == 0u || shared.filters[drafts + 1u + accepted].filtered == 0u)
+            return outcome(accepted, -1, 0.0f, NCNN_MOE_VERIFY_UNSUPPORTED_WINDOW, 0, accepted, 0);
+        const float target_probability = shared.found[accepted];
+        const float draft_probability = shared.found[drafts + accepted];
+        if (draft_probability <= 0.0f)
+            return outcome(accepted, -1, 0.0f, NCNN_MOE_VERIFY_ZERO_DRAFT_PROBABILITY, 0, accepted, 0);
+        const float ratio = target_probability / draft_probability;
+        const float acceptance = ratio < 1.0f ? ratio : 1.0f; // std::min(1.0f, ratio)
+        if (shared.uniforms[accepted] >= acceptance)
+            break;
+        if (writes)
+            v.accepted_probabilities[accepted] = target_probability;
+    }
+    if (accepted == drafts)
+    {
+        // ---- session.cpp:871-873: the target's own sample after the last drafted token
+        const ncnn_moe_sample_result next = shared.row_results[accepted];
+        if (next.status != NCNN_MOE_ROW_OK)
+            return outcome(accepted, -1, 0.0f, NCNN_MOE_VERIFY_ROW_ERROR, next.status, accepted, 0);
+        return outcome(accepted, next.token_id, next.probability, NCNN_MOE_VERIFY_OK, 0, accepted, next.draw_consumed);
+    }
+    // ---- rejected: this workgroup's entries of max(0, target - draft) (session.cpp:150-202)
+    if (writes)
+    {
+        v.decision[0] = 1u;
+        v.decision[1] = accepted;
+        v.decision[2] = accepted + 1u;
+    }
+    const void* const target_logits = row_pointer(accepted);
+    const void* const draft_logits = row_pointer(drafts + 1u + accepted);
+    const BinRow& target_filter = shared.filters[accepted];
+    const BinRow& draft_filter = shared.filters[drafts + 1u + accepted];
+    const uint32_t first = blockIdx.x * kResidualChunk + static_cast<uint32_t>(tid) * kResidualEach;
+    float own[kResidualEach];
+    float sum = 0.0f;
+    int32_t last = -1;
+#pragma unroll
+    for (uint32_t j = 0; j < kResidualEach; ++j)
+    {
+        const uint32_t token = first + j;
+        own[j] = 0.0f;
+        if (token < a.vocab)
+        {
+            const float target = filtered_probability<DTYPE>(target_logits, token, target_filter, v.temperature, shared.exp2_table);
+            if (target > 0.0f)
+            {
+                const float difference = target - filtered_probability<DTYPE>(draft_logits, token, draft_filter, v.temperature, shared.exp2_table);
+                own[j] = 0.0f < difference ? difference : 0.0f; // std::max(0.0f, difference)
+                last = own[j] > 0.0f ? static_cast<int32_t>(token) : last;
+            }
+        }
+        sum += own[j];
+    }
+    float* const out = v.residual + static_cast<size_t>(blockIdx.x) * kResidualChunk + static_cast<uint32_t>(tid) * kResidualEach;
+#pragma unroll
+    for (uint32_t j = 0; j < kResidualEach; j += 4u)
+        *reinterpret_cast<float4*>(out + j) = float4{own[j], own[j + 1], own[j + 2], own[j + 3]};
+    // plain sums of 64 entries (eight threads') and of the chunk
+    static_assert(kResidualSub / kResidualEach == 8, "eight threads hold the entries of a plain sum");
+    sum += __shfl_xor(sum, 1, kWaveSize);
+    sum += __shfl_xor(sum, 2, kWaveSize);
+    sum += __shfl_xor(sum, 4, kWaveSize);
+    if ((tid & 7) == 0)
+        v.sub_sums[static_cast<size_t>(blockIdx.x) * kWaveSize + (tid >> 3)] = sum;
+    sum += __shfl_xor(sum, 8, kWaveSize);
+    sum += __shfl_xor(sum, 16, kWaveSize);
+    sum += __shfl_xor(sum, 32, kWaveSize);
+    if (lane == 0)
+        shared.wave_sums[tid >> 6] = sum;
+    if (last >= 0)
+        atomicMax(&shared.last, last);
+    __syncthreads();
+    if (tid == 0)
+    {
+        double total = 0.0;
+        for (int w = 0; w < kResidualThreads / kWaveSize; ++w)
+            total += shared.wave_sums[w];
+        v.chunk_sums[blockIdx.x] = total;
+        v.chunk_last[blockIdx.x] = shared.last;
+    }
+}
+
+__global__ __launch_bounds__(kResidualThreads) void verify_steps_kernel(VerifySumsArgs v)
+{
+    constexpr uint32_t kWaves = kResidualThreads / kWaveSize;
+    __shared__ uint4 steps[kWaveSize];
+    __shared__ double wave_sums[kWaves];
+    if (v.decision[0] == 0u)
+        return;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWaveSize - 1);
+    const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
+    const uint32_t chunk = blockIdx.x;
+    float own[kWaveSize / kWaves];
+#pragma unroll
+    for (uint32_t k = 0; k < kWaveSize / kWaves; ++k)
+        own[k] = v.residual[static_cast<size_t>(chunk) * kResidualChunk + (k * kWaves + wave) * kResidualSub + lane];
+    const float sub_sum = v.sub_sums[static_cast<size_t>(chunk) * kWaveSize + lane];
+    // what the chunks in front of this one add up to, about
+    double before = 0.0;
+    for (uint32_t c = tid; c < chunk; c += kResidualThreads)
+        before += v.chunk_sums[c];
+#pragma unroll
+    for (int distance = kWaveSize / 2; distance > 0; distance >>= 1)
+        before += __shfl_xor(before, distance, kWaveSize);
+    if (lane == 0)
+        wave_sums[wave] = before;
+    __syncthreads();
+    before = 0.0;
+    for (uint32_t w = 0; w < kWaves; ++w)
+        before += wave_sums[w];
+    const float front = static_cast<float>(before) + (wave_prefix_sum_f32(sub_sum) - sub_sum); // lane l: in front of the l-th 64 entries
+#pragma unroll
+    for (uint32_t k = 0; k < kWaveSize / kWaves; ++k)
+    {
+        const uint32_t sub = k * kWaves + wave;
+        const uint32_t exponent = max(same_in_all(__float_as_uint(read_lane(front, static_cast<int>(sub)))) >> 23, 1u);
+        const ParityStep through = wave_scan_steps(step_of_term(own[k], static_cast<int>(exponent)));
+        if (lane == kWaveSize - 1)
+            steps[sub] = uint4{exponent, through.even, through.odd, 0u};
+    }
+    __syncthreads();
+    if (wave == 0u)
+    {
+        // the chunk's own step, where all of it lies in one binade (else an exponent that no sum has)
+        const uint4 mine = steps[lane];
+        v.sub_steps[static_cast<size_t>(chunk) * kWaveSize + lane] = mine;
+        const ParityStep through = wave_scan_steps(ParityStep{mine.y, mine.z});
+        const uint32_t first_exponent = same_in_all(mine.x);
+        const bool one_binade = __builtin_amdgcn_ballot_w64(mine.x != first_exponent) == 0ull;
+        if (lane == kWaveSize - 1)
+            v.chunk_steps[chunk] = uint4{one_binade ? first_exponent : 0u, through.even, through.odd, 0u};
+    }
+}
+
+// Adds up to 64 composed steps, lane l's `mine` (exponent, even, odd) the l-th, from `first` on, as long as each has the
+// sum's exponent and leaves the mantissa below the goal.  Returns the first that does not; `behind` is every lane's sum.
+__device__ __forceinline__ uint32_t add_composed_steps(const uint4& mine, uint32_t first, uint32_t count, int mode, float bound, float& sum, float& behind)
+{
+    const uint32_t lane = static_cast<uint32_t>(lane_id());
+    int exponent;
+    uint32_t mantissa;
+    decode_sum(sum, exponent, mantissa);
+    const uint32_t goal = min(stop_mantissa(mode, bound, exponent), kBinadeFull);
+    const bool ahead = lane >= first && lane < count;
+    const bool usable = ahead && mine.x == static_cast<uint32_t>(exponent);
+    const ParityStep through = wave_scan_steps(ParityStep{usable ? mine.y : 0u, usable ? mine.z : 0u});
+    const uint32_t after = apply_step(mantissa, through);
+    behind = encode_sum(exponent, min(after, kBinadeFull - 1u));
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(ahead && !(usable && after < goal));
+    const uint32_t first_bad = bad != 0ull ? static_cast<uint32_t>(__builtin_ctzll(bad)) : count;
+    if (first_bad > first)
+        sum = read_lane(behind, static_cast<int>(first_bad - 1u));
+    return first_bad;
+}
+
+__global__ __launch_bounds__(kResidualThreads) void verify_draw_kernel(VerifySumsArgs v, uint32_t chunks)
+{
+    __shared__ __align__(16) float entries[kResidualSub];
+    if (v.decision[0] == 0u || threadIdx.x >= kWaveSize)
+        return;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t accepted = v.decision[1];
+    const uint32_t accept_draws = v.decision[2];
+    const float uniform = v.uniforms[accept_draws];
+    // one chunk, 64 entries at a time; true where the stop condition holds at entry `index`
+    const auto walk_chunk = [&](uint32_t chunk, int mode, float bound, float& sum, uint32_t& index) -> bool {
+        const uint4 mine = v.sub_steps[static_cast<size_t>(chunk) * kWaveSize + lane];
+        float behind;
+        for (uint32_t sub = 0; sub < kWaveSize;)
+        {
+            sub = add_composed_steps(mine, sub, kWaveSize, mode, bound, sum, behind);
+            if (sub == kWaveSize)
+                break;
+            const uint32_t first = chunk * kResidualChunk + sub * kResidualSub;
+            entries[lane] = v.residual[first + lane];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            const WaveSum result = wave_add_terms<0>(entries, kResidualSub, sum, mode, bound, 1.0f, 1.0f);
+            __builtin_amdgcn_wave_barrier();
+            sum = result.sum;
+            if (result.stopped)
+            {
+                index = first + result.index;
+                return true;
+            }
+            ++sub;
+        }
+        return false;
+    };
+    const auto finish = [&](int32_t token, float probability, uint32_t status, uint32_t final_draw) {
+        if (lane != 0u)
+            return;
+        ncnn_moe_verify_result r;
+        r.accepted = accepted;
+        r.next_token_id = status == NCNN_MOE_VERIFY_OK ? token : -1;
+        r.next_probability = status == NCNN_MOE_VERIFY_OK ? probability : 0.0f;
+        r.status = status;
+        r.row_status = 0;
+        r.accept_draws = accept_draws;
+        r.final_draw_consumed = final_draw;
+        r.next_is_residual = 1;
+        *v.result = r;
+    };
+    // ---- the sum.  Every chunk's partial sum is kept (in place of its composed step)
+    float sum = 0.0f;
+    int32_t last = -1;
+    float* const partial = reinterpret_cast<float*>(v.chunk_sums);
+    for (uint32_t base = 0; base < chunks; base += kWaveSize)
+    {
+        const uint32_t count = min(chunks - base, static_cast<uint32_t>(kWaveSize));
+        const uint4 mine = lane < count ? v.chunk_steps[base + lane] : uint4{0u, 0u, 0u, 0u};
+        last = max(last, lane < count ? v.chunk_last[base + lane] : -1);
+        float own = 0.0f; // the sum behind the lane's chunk
+        for (uint32_t c = 0; c < count;)
+        {
+            float behind;
+            const uint32_t stop = add_composed_steps(mine, c, count, kStopNever, 0.0f, sum, behind);
+            own = lane >= c && lane < stop ? behind : own;
+            c = stop;
+            if (c == count)
+                break;
+            uint32_t index = 0;
+            walk_chunk(base + c, kStopNever, 0.0f, sum, index);
+            own = lane == c ? sum : own;
+            ++c;
+        }
+        if (lane < count)
+            partial[base + lane] = own;
+    }
+    last = static_cast<int32_t>(wave_max_u32(static_cast<uint32_t>(last + 1))) - 1;
+    const float normalizer = sum;
+    if (!is_finite_f32(normalizer) || !(normalizer > 0.0f))
+        return finish(-1, 0.0f, NCNN_MOE_VERIFY_RESIDUAL_EMPTY, 0);
+    // ---- the draw: uniform_real_distribution<float>(0, normalizer) is the canonical draw times the range.  The first
+    // partial sum above it lies in the first chunk whose last one is.
+    const float sample_value = uniform * normalizer;
+    int32_t selected = last; // session.cpp:189-198: past the end, the last token that has any residual mass
+    float before = 0.0f;
+    for (uint32_t base = 0; base < chunks; base += kWaveSize)
+    {
+        const uint32_t count = min(chunks - base, static_cast<uint32_t>(kWaveSize));
+        const float own = lane < count ? partial[base + lane] : 0.0f;
+        const uint64_t passing = __builtin_amdgcn_ballot_w64(lane < count && own > sample_value);
+        if (passing != 0ull)
+        {
+            const int c = __builtin_ctzll(passing);
+            if (c > 0)
+                before = read_lane(own, c - 1);
+            uint32_t index = 0;
+            if (walk_chunk(base + static_cast<uint32_t>(c), kStopAbove, sample_value, before, index))
+                selected = static_cast<int32_t>(index);
+            break;
+        }
+        before = read_lane(own, static_cast<int>(count) - 1);
+    }
+    if (selected < 0)
+        return finish(-1, 0.0f, NCNN_MOE_VERIFY_RESIDUAL_FAILED, 1);
+    finish(selected, v.residual[selected] / normalizer, NCNN_MOE_VERIFY_OK, 1);
 }
 
 } // namespace ncnn_moe_hip
