@@ -47,21 +47,19 @@ constexpr uint32_t kOneBits = 0x3f800000u;       // the largest term
 constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms of 2^-25 or less move no sum
 constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
 constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
-constexpr uint32_t kBinHead = 3072;              // elements of the sorted head at most (unless one bin or a window takes more) ...
-constexpr uint32_t kBinHeadDense = 1024;         // ... behind this many it takes only bins of
-constexpr uint32_t kBinHeadBin = 48;             // ... this many elements at most: dense bins cost their ordering and save little
+constexpr uint32_t kBinHead = 2048;              // elements of the sorted head at most (unless one bin or a window takes more)
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
 constexpr uint32_t kBinStops = 512;
 constexpr int kMaskedDifference = 14;            // so many binades below the sum a bin's terms (within a 64th of each other) take 18 different steps at most
 constexpr uint32_t kBinRequests = 64;            // ... and how often per walk
 constexpr uint32_t kMaxBinParts = 16;
-constexpr uint32_t kPartsAtATime = 8;            // loads of the parts' numbers in flight together
+constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers in flight together
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
 constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
-constexpr float kForeseenFirst = 4e-4f;          // relative error allowed for the sums foreseen from the bins' masses
-constexpr float kForeseenLater = 4e-4f;          // ... and from the steps of the sum before
+constexpr float kForeseenFirst = 1e-4f;          // relative error allowed for the sums foreseen from the bins' masses
+constexpr float kForeseenLater = 1e-4f;          // ... and from the steps of the sum before
 static_assert(kBinQuads <= kWalkThreads && kBinListCap % kWalkThreads == 0 && kBinListCap <= 64 * kWaveSize, "the walk's thread and lane counts");
 
 // A bin as the walk sees it: kind (2 bits), biased exponent assumed for the running sum (8), elements in front of it (22).
@@ -185,7 +183,7 @@ __device__ __forceinline__ float* bin_terms(const SamplerArgs& a, uint32_t row)
 
 // ---- (1) largest and smallest finite logit, number of finite logits, NaN and +inf seen
 template <int DTYPE>
-__global__ __launch_bounds__(kBinThreads) void bin_stats_kernel(BinArgs g)
+__global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
 {
     using Vector = LogitsVector<DTYPE>;
     constexpr uint32_t kWidth = Vector::kWidth;
@@ -203,59 +201,71 @@ __global__ __launch_bounds__(kBinThreads) void bin_stats_kernel(BinArgs g)
         const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
         float largest = -INFINITY, smallest = INFINITY;
         uint32_t finite = 0, flags = 0;
-        for (uint32_t at = first + tid; at < last; at += kLoads * kBinThreads)
+        const auto take = [&](float x) {
+            const uint32_t magnitude = __float_as_uint(x) & 0x7fffffffu;
+            const bool counts = magnitude < 0x7f800000u;
+            largest = fmaxf(largest, counts ? x : -INFINITY);
+            smallest = fminf(smallest, counts ? x : INFINITY);
+            finite += counts ? 1u : 0u;
+            flags |= magnitude > 0x7f800000u ? static_cast<uint32_t>(kScanSawNan) : 0u;
+            flags |= __float_as_uint(x) == 0x7f800000u ? static_cast<uint32_t>(kScanSawPositiveInfinity) : 0u;
+        };
+        // (a vector that holds other elements too: the row's first and last)
+        const auto take_inside = [&](uint32_t v) {
+            float x[kWidth];
+            Vector::unpack(*reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u), x);
+#pragma unroll
+            for (uint32_t c = 0; c < kWidth; ++c)
+            {
+                if (v * kWidth + c - s.misalignment < a.vocab)
+                    take(x[c]);
+            }
+        };
+        const uint32_t first_whole = max(first, (s.misalignment + kWidth - 1u) / kWidth);
+        const uint32_t last_whole = min(last, s.end / kWidth);
+        if (tid == 0 && first < min(first_whole, last))
+            take_inside(first);
+        if (tid == kWaveSize && first_whole <= last_whole && last_whole < last)
+            take_inside(last_whole);
+        for (uint32_t at = first_whole + tid; at < last_whole; at += kLoads * kBinThreads)
         {
             uint4 raw[kLoads];
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
-            {
-                const uint32_t v = min(at + k * kBinThreads, last - 1u);
-                raw[k] = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u);
-            }
+                raw[k] = *reinterpret_cast<const uint4*>(base + min(at + k * kBinThreads, last_whole - 1u) * 16u); // (rows below 2^32 bytes)
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
             {
-                const uint32_t v = at + k * kBinThreads;
-                float x[kWidth];
-                Vector::unpack(raw[k], x);
-                const uint32_t position = v * kWidth;
-                const bool whole = v < last && position >= s.misalignment && position + kWidth <= s.end;
-#pragma unroll
-                for (uint32_t c = 0; c < kWidth; ++c)
+                if (at + k * kBinThreads < last_whole)
                 {
-                    const bool inside = whole || (v < last && position + c >= s.misalignment && position + c < s.end);
-                    const uint32_t magnitude = __float_as_uint(x[c]) & 0x7fffffffu;
-                    const bool counts = inside && magnitude < 0x7f800000u;
-                    largest = fmaxf(largest, counts ? x[c] : -INFINITY);
-                    smallest = fminf(smallest, counts ? x[c] : INFINITY);
-                    finite += counts ? 1u : 0u;
-                    flags |= inside && magnitude > 0x7f800000u ? static_cast<uint32_t>(kScanSawNan) : 0u;
-                    flags |= inside && __float_as_uint(x[c]) == 0x7f800000u ? static_cast<uint32_t>(kScanSawPositiveInfinity) : 0u;
+                    float x[kWidth];
+                    Vector::unpack(raw[k], x);
+#pragma unroll
+                    for (uint32_t c = 0; c < kWidth; ++c)
+                        take(x[c]);
                 }
             }
         }
-#pragma unroll
-        for (int distance = kWaveSize / 2; distance > 0; distance >>= 1)
-        {
-            largest = fmaxf(largest, __shfl_xor(largest, distance, kWaveSize));
-            smallest = fminf(smallest, __shfl_xor(smallest, distance, kWaveSize));
-            finite += __shfl_xor(finite, distance, kWaveSize);
-            flags |= __shfl_xor(flags, distance, kWaveSize);
-        }
+        const auto reduce = [&](int lanes) {
+            for (int distance = lanes / 2; distance > 0; distance >>= 1)
+            {
+                largest = fmaxf(largest, __shfl_xor(largest, distance, kWaveSize));
+                smallest = fminf(smallest, __shfl_xor(smallest, distance, kWaveSize));
+                finite += __shfl_xor(finite, distance, kWaveSize);
+                flags |= __shfl_xor(flags, distance, kWaveSize);
+            }
+        };
+        reduce(kWaveSize);
         if ((tid & (kWaveSize - 1)) == 0)
             wave_stats[tid >> 6] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
         __syncthreads();
-        if (tid == 0)
+        if (tid < kWaveSize)
         {
-            for (int w = 1; w < kBinWaves; ++w)
-            {
-                const uint4 other = wave_stats[w];
-                largest = fmaxf(largest, __uint_as_float(other.x));
-                smallest = fminf(smallest, __uint_as_float(other.y));
-                finite += other.z;
-                flags |= other.w;
-            }
-            g.stats[slot * grid.parts + grid.part] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
+            const uint4 of_wave = wave_stats[tid & (kBinWaves - 1)];
+            largest = __uint_as_float(of_wave.x), smallest = __uint_as_float(of_wave.y), finite = of_wave.z, flags = of_wave.w;
+            reduce(kBinWaves);
+            if (tid == 0)
+                g.stats[slot * grid.parts + grid.part] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
         }
         __syncthreads();
     }
@@ -263,7 +273,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_stats_kernel(BinArgs g)
 
 // ---- (2) the terms, in the row's order, and how many fall into each bin
 template <int DTYPE>
-__global__ __launch_bounds__(kBinThreads) void bin_terms_kernel(BinArgs g)
+__global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
 {
     using Vector = LogitsVector<DTYPE>;
     constexpr uint32_t kWidth = Vector::kWidth;
@@ -341,7 +351,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_terms_kernel(BinArgs g)
                 for (int k = 0; k < kLoads; ++k)
                 {
                     const uint32_t v = min(at + k * kBinThreads, last - 1u);
-                    raw[k] = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(v) * 16u);
+                    raw[k] = *reinterpret_cast<const uint4*>(base + v * 16u); // (rows below 2^32 bytes)
                 }
 #pragma unroll
                 for (int k = 0; k < kLoads; ++k)
@@ -455,7 +465,8 @@ struct BinPlan
 };
 
 __device__ __forceinline__ BinPlan plan_bins(
-    uint32_t bin, const uint32_t (&front)[5], const float (&mass)[5], uint32_t head_bins, uint32_t limit, uint32_t cut_bin, float bound, float error)
+    uint32_t bin, const uint32_t (&front)[5], const float (&mass)[5], uint32_t head_bins, uint32_t limit, uint32_t cut_bin, float bound, float error,
+    uint32_t shift, float scale)
 {
     BinPlan plan;
     plan.listed = 0;
@@ -474,7 +485,9 @@ __device__ __forceinline__ BinPlan plan_bins(
         else if (count > 0u)
         {
             const bool ends = front[j + 1] > limit || b == cut_bin;
-            const bool leaves = ((__float_as_uint(low) ^ __float_as_uint(high)) >> 23) != 0u;
+            // (terms below half an ulp of the lower of the two sums move neither)
+            const bool moves = bin_top(b, shift) * scale * 1.0001f >= __uint_as_float((max(__float_as_uint(low) >> 23, 25u) - 24u) << 23);
+            const bool leaves = moves && ((__float_as_uint(low) ^ __float_as_uint(high)) >> 23) != 0u;
             plan.ends |= ends ? 1u << j : 0u;
             if (ends || leaves || high >= bound)
             {
@@ -595,7 +608,7 @@ __device__ __forceinline__ void add_bin_steps(
 }
 
 // ---- (3) the head and the bins whose order is foreseen to matter go to the list; the others' steps of the normaliser
-__global__ __launch_bounds__(kBinThreads) void bin_sum_kernel(BinArgs g, uint32_t element_bytes)
+__global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint32_t element_bytes)
 {
     __shared__ __align__(16) uint32_t entries[kBins];
     __shared__ __align__(16) uint32_t steps[kBins];
@@ -620,38 +633,49 @@ __global__ __launch_bounds__(kBinThreads) void bin_sum_kernel(BinArgs g, uint32_
         }
         const uint32_t shift = record.shift;
         const uint32_t window = record.window;
-        // counts of the thread's bins, of the whole row and of the parts in front of this one, and their masses
+        // counts of the thread's bins, of the whole row and of the parts in front of this one, and (by other threads) where
+        // in their bins the terms lie
         uint32_t count[4] = {0u, 0u, 0u, 0u}, before[4] = {0u, 0u, 0u, 0u};
-        uint32_t places[4] = {0u, 0u, 0u, 0u};
-        if (holds_bins)
+        const bool holds_places = tid >= kBinThreads / 2 && tid < kBinThreads / 2 + static_cast<int>(kBinQuads);
+        if (holds_bins || holds_places)
         {
-            const uint4* counts = reinterpret_cast<const uint4*>(g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins) + tid;
+            const uint4* counts = reinterpret_cast<const uint4*>(g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins) +
+                (holds_bins ? static_cast<uint32_t>(tid) : kBinQuads + static_cast<uint32_t>(tid) - kBinThreads / 2);
             for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
             {
-                uint4 of_part[kPartsAtATime], place_sums[kPartsAtATime];
+                uint4 of_part[kPartsAtATime];
 #pragma unroll
                 for (uint32_t k = 0; k < kPartsAtATime; ++k)
-                {
-                    const uint4* from = counts + static_cast<size_t>(min(first + k, grid.parts - 1u)) * 2u * kBinQuads;
-                    of_part[k] = from[0];
-                    place_sums[k] = from[kBinQuads];
-                }
+                    of_part[k] = counts[static_cast<size_t>(min(first + k, grid.parts - 1u)) * 2u * kBinQuads];
 #pragma unroll
                 for (uint32_t k = 0; k < kPartsAtATime; ++k)
                 {
                     const uint32_t some = first + k < grid.parts ? 0xffffffffu : 0u;
                     const uint32_t some_before = first + k < grid.part ? 0xffffffffu : 0u;
                     const uint32_t c[4] = {of_part[k].x, of_part[k].y, of_part[k].z, of_part[k].w};
-                    const uint32_t o[4] = {place_sums[k].x, place_sums[k].y, place_sums[k].z, place_sums[k].w};
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                     {
-                        count[j] += c[j] & some;
+                        count[j] += c[j] & some; // (places: below 2^22 x 2^12; only a bin of a million terms wraps, a wrong guess)
                         before[j] += c[j] & some_before;
-                        places[j] += o[j] & some; // (a bin's places add up to less than 2^22 x 2^12: only a bin of a million terms wraps, a wrong guess)
                     }
                 }
             }
+        }
+        if (holds_places)
+            reinterpret_cast<uint4*>(steps)[tid - kBinThreads / 2] = uint4{count[0], count[1], count[2], count[3]};
+        __syncthreads();
+        uint32_t places[4] = {0u, 0u, 0u, 0u};
+        if (holds_bins)
+        {
+            const uint4 words = reinterpret_cast<const uint4*>(steps)[tid];
+            places[0] = words.x, places[1] = words.y, places[2] = words.z, places[3] = words.w;
+        }
+        else
+        {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                count[j] = before[j] = 0u;
         }
         if (tid == 0)
             head_bins_of_row = head_count_of_row = end_of_list = 0u;
@@ -722,7 +746,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_sum_kernel(BinArgs g, uint32_
             for (int j = 3; j >= 0; --j)
             {
                 const bool in_head = window_in_head ? front[j] < window
-                    : front[j + 1] <= kBinHead && (front[j + 1] <= kBinHeadDense || count[j] <= kBinHeadBin);
+                    : front[j + 1] <= kBinHead;
                 if (!in_head && bin + j != 0u)
                     first_not = bin + j;
             }
@@ -752,7 +776,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_sum_kernel(BinArgs g, uint32_
             continue;
         }
         const bool beyond = window > head_count && binned > head_count; // the sum goes on behind the head
-        BinPlan plan = plan_bins(bin, front, mass, head_bins, beyond ? window : 0u, kBins, INFINITY, kForeseenFirst);
+        BinPlan plan = plan_bins(bin, front, mass, head_bins, beyond ? window : 0u, kBins, INFINITY, kForeseenFirst, shift, 1.0f);
         uint32_t listed[1] = {holds_bins ? plan.listed : 0u};
         {
             uint32_t totals[1];
@@ -1326,6 +1350,15 @@ __device__ __forceinline__ void walk_bins(
                 shared.stop_at = place;
                 finish(1u);
             };
+            // every term of the bin, and of those behind it, is below half an ulp of the sum: none moves it
+            const auto moves_nothing = [&](uint32_t bin) {
+                float top = bin_top(bin, shift);
+                if (PHASE >= 1)
+                    top = top / divisor;
+                if (PHASE >= 2)
+                    top = top / second_divisor;
+                return top < __uint_as_float((max(__float_as_uint(sum) >> 23, 25u) - 24u) << 23);
+            };
             const auto ask_for = [&](uint32_t low, uint32_t high) {
                 shared.low = low;
                 shared.high = high;
@@ -1403,6 +1436,8 @@ __device__ __forceinline__ void walk_bins(
                         cur += good;
                         ask_for(cur, cur);
                     }
+                    else if (moves_nothing(cur))
+                        cur = stop_here;
                     else
                     {
                         // the sum has another exponent than was foreseen: as many bins as can be fetched at a time
@@ -1990,7 +2025,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
 #pragma unroll
             for (int j = 0; j < 5; ++j)
                 mass[j] *= scale;
-            BinPlan plan = plan_bins(bin, front, mass, head_bins, next_limit, next_cut_bin, WALK == 0 ? top_p : uniform, kForeseenLater);
+            BinPlan plan = plan_bins(bin, front, mass, head_bins, next_limit, next_cut_bin, WALK == 0 ? top_p : uniform, kForeseenLater, shift,
+                                     1.0f / (WALK == 0 ? normalizer : normalizer * renormalizer));
             uint32_t to_list[1] = {holds_bins ? plan.listed : 0u};
             {
                 uint32_t totals[1];

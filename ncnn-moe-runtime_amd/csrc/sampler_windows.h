@@ -444,7 +444,7 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
 }
 
 template <int DTYPE>
-__global__ __launch_bounds__(kBinThreads) void window_candidates_kernel(WindowArgs g)
+__global__ __launch_bounds__(kBinThreads, 8) void window_candidates_kernel(WindowArgs g)
 {
     __shared__ WindowCandidatesShared shared;
     window_candidates<DTYPE>(g, bin_grid(g.list, g.a.vocab), shared, threadIdx.x);
