@@ -47,7 +47,8 @@ constexpr uint32_t kOneBits = 0x3f800000u;       // the largest term
 constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms of 2^-25 or less move no sum
 constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
 constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
-constexpr uint32_t kBinHead = 2048;              // elements of the sorted head at most (unless one bin or a window takes more)
+constexpr uint32_t kBinHead = 2048;              // elements of the sorted head at most (unless a window takes more): behind
+                                                 // so many a term half way seldom has to be fetched, 40 us each
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
 constexpr uint32_t kBinStops = 512;
@@ -58,6 +59,8 @@ constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers 
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
 constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
+// (the foreseen sums were off by a few 1e-5 at most; where a sum grows by single ulps a margin of 1e-4 lists 1,700 elements
+// at most on both sides of a power of two, so that they always fit)
 constexpr float kForeseenFirst = 1e-4f;          // relative error allowed for the sums foreseen from the bins' masses
 constexpr float kForeseenLater = 1e-4f;          // ... and from the steps of the sum before
 static_assert(kBinQuads <= kWalkThreads && kBinListCap % kWalkThreads == 0 && kBinListCap <= 64 * kWaveSize, "the walk's thread and lane counts");
@@ -181,6 +184,10 @@ __device__ __forceinline__ float* bin_terms(const SamplerArgs& a, uint32_t row)
     return reinterpret_cast<float*>(a.sort_indices[0] + row * a.sort_stride);
 }
 
+// Kernels (1) to (3) are bound to 64 registers: two workgroups of 1,024 threads share a compute unit then, and the 512
+// workgroups of a launch that many rows fill run at once, not in two rounds (512 rows of 129,280 of mixed options: 17, 26
+// and 32 us before, 14, 22 and 25 us with the bound).
+//
 // ---- (1) largest and smallest finite logit, number of finite logits, NaN and +inf seen
 template <int DTYPE>
 __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
