@@ -68,16 +68,22 @@ uint32_t check_options(uint32_t token_count, const ncnn_moe_router_options& o)
 template <int SLOTS>
 void launch_select(const RouterArgs& args, hipStream_t stream)
 {
-    const unsigned blocks = (args.tokens + kRouterWavesPerBlock - 1) / kRouterWavesPerBlock;
     if (args.tokens <= static_cast<uint32_t>(kRouterChunkTokens))
     {
         // one chunk of tokens: the select kernel's last workgroup places the routes itself, and the
         // scores are computed by all threads of a workgroup of few tokens
         const unsigned staged_blocks = (args.tokens + kStagedTokensPerBlock - 1) / kStagedTokensPerBlock;
-        hipLaunchKernelGGL((router_select_kernel<SLOTS, true, true>), dim3(staged_blocks), dim3(kRouterThreads), 0, stream, args);
+        hipLaunchKernelGGL(router_select_kernel<SLOTS>, dim3(staged_blocks), dim3(kRouterThreads), 0, stream, args);
         return;
     }
-    hipLaunchKernelGGL((router_select_kernel<SLOTS, false, false>), dim3(blocks), dim3(kRouterThreads), 0, stream, args);
+    // two tokens per wave where a token is little work (128 experts at most) and there are enough of them to fill the SIMDs'
+    // waves all the same (8,192); else one, which leaves more waves to hide behind
+    const uint32_t tokens_per_wave = SLOTS <= 2 && args.tokens >= 8192u ? 2u : 1u;
+    const unsigned blocks = (args.tokens + kBatchWaves * tokens_per_wave - 1u) / (kBatchWaves * tokens_per_wave);
+    if (tokens_per_wave == 2u)
+        hipLaunchKernelGGL((router_batch_kernel<SLOTS, SLOTS <= 2 ? 2 : 1>), dim3(blocks), dim3(kBatchThreads), 0, stream, args);
+    else
+        hipLaunchKernelGGL((router_batch_kernel<SLOTS, 1>), dim3(blocks), dim3(kBatchThreads), 0, stream, args);
     const unsigned chunks = (args.tokens + kRouterChunkTokens - 1) / kRouterChunkTokens;
     hipLaunchKernelGGL(router_group_kernel, dim3(chunks), dim3(kRouterThreads), 0, stream, args);
 }
@@ -145,7 +151,7 @@ int ncnn_moe_hip_router_create(int device, uint32_t max_tokens, uint32_t max_exp
     ok = ok && hipMalloc(&r->explicit_ids, assignments * sizeof(uint32_t)) == hipSuccess;
     ok = ok && hipMalloc(&r->selected_experts, assignments * sizeof(uint32_t)) == hipSuccess;
     ok = ok && hipMalloc(&r->selected_weights, assignments * sizeof(float)) == hipSuccess;
-    const size_t chunk_counters = ((tokens + kRouterChunkTokens - 1) / kRouterChunkTokens) * max_experts;
+    const size_t chunk_counters = ((tokens + kRouterChunkTokens - 1) / kRouterChunkTokens) * chunk_count_stride(max_experts);
     ok = ok && hipMalloc(&r->chunk_counts, chunk_counters * sizeof(uint32_t)) == hipSuccess;
     ok = ok && hipMalloc(&r->scratch_words, 4 * sizeof(uint32_t)) == hipSuccess;
     // the kernels find these zeroed (no failing token: all ones) and leave them so

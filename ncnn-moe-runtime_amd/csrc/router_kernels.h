@@ -1,6 +1,7 @@
 // Expert router kernels (src/graph/expert_dispatcher.cpp:12-157 of the runtime, on the device):
-//   router_select_kernel  one wave per token: scores, Top-K routes, normalised weights
-//   router_group_kernel   one workgroup per 256 tokens: their routes to their places in the plan
+//   router_select_kernel  up to 256 tokens: scores, Top-K routes, normalised weights, and the routes to their places
+//   router_batch_kernel   more tokens: scores, Top-K routes, normalised weights
+//   router_group_kernel   ... and one workgroup per 256 tokens: their routes to their places in the plan
 #ifndef NCNN_MOE_HIP_ROUTER_KERNELS_H
 #define NCNN_MOE_HIP_ROUTER_KERNELS_H
 
@@ -16,23 +17,15 @@ constexpr int kRouterChunkTokens = 256; // tokens whose routes one workgroup of 
 // log1pf bit-identical to glibc 2.35's (sysdeps/ieee754/flt-32/s_log1pf.c) for finite x > 0, which is
 // all stable_softplus hands it (an exponential).  Plain fp32 operations in the library's order; built
 // without contraction, so every one rounds once.  Compared with libm on every positive float.
-__device__ __forceinline__ float log1pf_libm_positive(float x)
+// log1pf_libm_general: for x of 2^-29 or more and finite.  The library's range cases (x < 0.41422: no reduction; x < 2^53:
+// reduce 1 + x and keep the rounding error of the sum as a correction; above: reduce x itself; 1 + x next to a power of
+// two: a shorter series) are selects, so that lanes in different ranges, and a lane's experts, share one instruction stream.
+__device__ __forceinline__ float log1pf_libm_general(float x)
 {
     const float ln2_hi = 6.9313812256e-01f, ln2_lo = 9.0580006145e-06f;
     const float Lp1 = 6.6666668653e-01f, Lp2 = 4.0000000596e-01f, Lp3 = 2.8571429849e-01f, Lp4 = 2.2222198546e-01f,
                 Lp5 = 1.8183572590e-01f, Lp6 = 1.5313838422e-01f, Lp7 = 1.4798198640e-01f;
     const int32_t hx = static_cast<int32_t>(__float_as_uint(x));
-    if (hx < 0x31000000) // x < 2^-29
-    {
-        if (hx < 0x24800000) // x < 2^-54
-            return x;
-        return x - x * x * 0.5f;
-    }
-    if (hx >= 0x7f800000)
-        return x + x;
-    // The library's three range cases (x < 0.41422: no reduction; x < 2^53: reduce 1 + x and keep the
-    // rounding error of the sum as a correction; above: reduce x itself) as selects, so that lanes in
-    // different ranges share one instruction stream.
     const bool direct = hx < 0x3ed413d7;
     const bool huge = hx >= 0x5a000000;
     float u = huge ? x : 1.0f + x;
@@ -51,26 +44,32 @@ __device__ __forceinline__ float log1pf_libm_positive(float x)
     hu = direct ? 1 : hu;
     const float hfsq = 0.5f * f * f;
     const float kf = static_cast<float>(k);
-    if (hu == 0) // |f| < 2^-20
-    {
-        if (f == 0.0f)
-        {
-            if (k == 0)
-                return 0.0f;
-            c += kf * ln2_lo;
-            return kf * ln2_hi + c;
-        }
-        const float R = hfsq * (1.0f - 0.66666666666666666f * f);
-        if (k == 0)
-            return f - R;
-        return kf * ln2_hi - ((R - (kf * ln2_lo + c)) - f);
-    }
     const float s = f / (2.0f + f);
     const float z = s * s;
     const float R = z * (Lp1 + z * (Lp2 + z * (Lp3 + z * (Lp4 + z * (Lp5 + z * (Lp6 + z * Lp7))))));
     const float near = f - (hfsq - s * (hfsq + R));
     const float far = kf * ln2_hi - ((hfsq - (s * (hfsq + R) + (kf * ln2_lo + c))) - f);
-    return k == 0 ? near : far;
+    // |f| < 2^-20
+    const float short_R = hfsq * (1.0f - 0.66666666666666666f * f);
+    const float short_near = f == 0.0f ? 0.0f : f - short_R;
+    const float short_far = f == 0.0f ? kf * ln2_hi + (c + kf * ln2_lo) : kf * ln2_hi - ((short_R - (kf * ln2_lo + c)) - f);
+    const float of_short = k == 0 ? short_near : short_far;
+    const float of_long = k == 0 ? near : far;
+    return hu == 0 ? of_short : of_long;
+}
+
+__device__ __forceinline__ float log1pf_libm_positive(float x)
+{
+    const int32_t hx = static_cast<int32_t>(__float_as_uint(x));
+    if (hx < 0x31000000) // x < 2^-29
+    {
+        if (hx < 0x24800000) // x < 2^-54
+            return x;
+        return x - x * x * 0.5f;
+    }
+    if (hx >= 0x7f800000)
+        return x + x;
+    return log1pf_libm_general(x);
 }
 
 // Wave-wide reductions through the data-parallel primitives: four exchanges inside each row of 16
@@ -95,27 +94,26 @@ __device__ __forceinline__ float wave_max(float value)
     return fmaxf(fmaxf(read_lane(value, 0), read_lane(value, 16)), fmaxf(read_lane(value, 32), read_lane(value, 48)));
 }
 
-__device__ __forceinline__ int wave_min(int value)
+// expf_libm without its branches, for x finite or -inf: the function's two ends as selects, so that the exponentials of a
+// lane's experts overlap (one behind the other, each waits for its table entry and its chain of double operations).
+__device__ __forceinline__ float expf_selects(float x, const uint64_t* exp2_table)
 {
-    value = min(value, dpp_move<kDppSwapPairs>(value));
-    value = min(value, dpp_move<kDppSwapHalves>(value));
-    value = min(value, dpp_move<kDppHalfMirror>(value));
-    value = min(value, dpp_move<kDppMirror>(value));
-    return min(min(read_lane(value, 0), read_lane(value, 16)), min(read_lane(value, 32), read_lane(value, 48)));
+    const float y = expf_of_small_argument(fminf(fmaxf(x, -104.0f), 89.0f), exp2_table);
+    return x < -0x1.9fe368p6f ? 0.0f : x > 0x1.62e42ep6f ? __builtin_inff() : y;
 }
 
 // score_router_logit (src/graph/expert_dispatcher.cpp:24-38)
-__device__ __forceinline__ float router_score_of_logit(float logit, uint32_t score_function)
+__device__ __forceinline__ float sigmoid_score(float logit, const uint64_t* exp2_table)
 {
-    if (score_function == NCNN_MOE_ROUTER_SIGMOID)
-        return 1.0f / (1.0f + expf_libm(-logit));
-    float softplus;
-    if (logit > 20.0f)
-        softplus = logit;
-    else if (logit < -20.0f)
-        softplus = expf_libm(logit);
-    else
-        softplus = log1pf_libm_positive(expf_libm(logit));
+    return 1.0f / (1.0f + expf_selects(-logit, exp2_table));
+}
+
+__device__ __forceinline__ float sqrt_softplus_score(float logit, const uint64_t* exp2_table)
+{
+    // (the exponential of a logit in [-20, 20] is at least 2^-29 and far below 2^53: log1pf's general range)
+    const float exponential = expf_selects(logit, exp2_table);
+    const float general = log1pf_libm_general(logit >= -20.0f && logit <= 20.0f ? exponential : 1.0f);
+    const float softplus = logit > 20.0f ? logit : logit < -20.0f ? exponential : general;
     return __builtin_sqrtf(softplus); // correctly rounded: built with -fhip-fp32-correctly-rounded-divide-sqrt
 }
 
@@ -141,22 +139,362 @@ struct RouterArgs
     uint32_t* status;             // the call's ncnn_moe_router_status
 };
 
-struct RouterShared
+// The chunk counters of one chunk, in words: whole groups of four experts.
+__host__ __device__ inline uint32_t chunk_count_stride(uint32_t experts)
 {
-    float scores[kRouterWavesPerBlock][NCNN_MOE_ROUTER_MAX_EXPERTS]; // a token's scores: for the caller-named experts, or staged
-    uint32_t non_finite[kRouterWavesPerBlock];                       // staged scoring: the token holds a non-finite logit
-    float staged_maximum[kRouterWavesPerBlock];                      // staged softmax: the waves' maxima
+    return (experts + 3u) / 4u * 4u;
+}
+
+// A wave's scratch for the routes of one token.
+struct RouteScratch
+{
+    uint64_t candidates[kWaveSize + 4]; // ordered selection score (32 bits), complement of the expert id (32)
+    float scores[kWaveSize + 4];        // the candidates' scores
+    float selected[kWaveSize + 4];      // the selected scores, in rank order, then zeros
 };
 
-// Decode-sized calls (STAGED): a workgroup takes kStagedTokensPerBlock tokens instead of one per wave
-// and all its threads compute the scores, one or a few experts each, into LDS; a wave per token then
-// selects from there.  The scores of a token (exp, log1p, sqrt per expert) are two fifths of a lone
-// wave's time for it; spread over four waves they take a quarter as long.  (The softmax sum is the CPU's
-// loop, one addition at a time in expert order, and stays with the selecting wave.)
+// This wave's LDS accesses in front of it come before those behind it (a wave's LDS operations run in order: only the
+// compiler has to keep it).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The sum of a row of `padded` scores (a multiple of 16), one addition at a time in expert order, as the CPU's loop; lanes
+// may sum different rows.  The scores past the last expert are 0, which leaves the sum as it is.
+__device__ __forceinline__ float sequential_row_sums(const float* row_of_lane, uint32_t padded)
+{
+    const float4* quads = reinterpret_cast<const float4*>(row_of_lane);
+    float sum = 0.0f;
+#pragma unroll 1
+    for (uint32_t q = 0; q < padded / 4u; q += 4u)
+    {
+        float4 four[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            four[k] = quads[q + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            sum = (((sum + four[k].x) + four[k].y) + four[k].z) + four[k].w;
+    }
+    return sum;
+}
+
+// ---- select_topk_routes (src/graph/expert_dispatcher.cpp:61-77): the best top_k of a token's experts by (score + bias
+// descending, expert id ascending).  Expert e lives in slot e / 64 of lane e % 64.
+// A threshold with top_k to `most` scores at or above it is searched over the scores' order-preserving bits: from the
+// largest score down in growing steps, then by halving; a step is one comparison per slot, and the counting runs on the
+// scalar unit.  The experts above the threshold are collected in id order and ranked against each other.  Where equal
+// scores leave no such threshold, the lowest ids among the equals are collected.
+// What bounds it: instructions, some 130 per token of 256 experts and 8 routes, where choosing one route per round by
+// wave-wide maxima took some 500.
+// Returns the sum of the selected scores in rank order (src/graph/expert_dispatcher.cpp:137-143); the calling lane's
+// route is `my_expert` with `my_rank` (none: a rank of top_k or more).
+template <int SLOTS>
+__device__ __forceinline__ float select_best(const RouterArgs& r, const float (&score)[SLOTS], const float (&bias)[SLOTS], RouteScratch& scratch,
+                                             int lane, uint32_t& my_expert, uint32_t& my_rank, float& my_score)
+{
+    const uint32_t top_k = r.top_k;
+    uint32_t key[SLOTS];
+    uint32_t largest = 0u;
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s)
+    {
+        const float keyed = score[s] + bias[s];
+        const uint32_t bits = __float_as_uint(keyed); // (never -0: a score is not)
+        const uint32_t ordered = bits ^ (static_cast<uint32_t>(static_cast<int32_t>(bits) >> 31) | 0x80000000u);
+        key[s] = static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts ? 0u : keyed != keyed ? 1u : ordered;
+        largest = max(largest, key[s]);
+    }
+    largest = wave_max_u32(largest);
+    const auto count_from = [&](uint32_t least) {
+        uint32_t count = 0;
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+            count += static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(key[s] >= least)));
+        return count;
+    };
+    const uint32_t most = min(static_cast<uint32_t>(kWaveSize), top_k + top_k / 2u + 8u);
+    uint32_t low = 1u, high = largest + 1u; // as many as wanted from `low` on, too few from `high` on
+    uint32_t step = 1u << 22;               // half a binade
+    uint32_t threshold = largest > step ? largest - step : 1u;
+    uint32_t equals = 0xffffffffu;          // how many scores that equal the threshold are taken
+    for (;;)
+    {
+        const uint32_t count = count_from(threshold);
+        if (count >= top_k && count <= most)
+            break;
+        if (count < top_k)
+            high = threshold;
+        else
+        {
+            low = threshold;
+            step = 0u;
+        }
+        if (high - low <= 1u)
+        {
+            threshold = low;
+            equals = top_k - count_from(low + 1u);
+            break;
+        }
+        step = step < 0x40000000u ? step * 2u : step;
+        const bool falls = step != 0u && largest - low > step && largest - step < high;
+        threshold = falls ? largest - step : low + (high - low) / 2u;
+    }
+    uint32_t count = 0, equals_before = 0;
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s)
+    {
+        bool taken = key[s] >= threshold;
+        if (equals != 0xffffffffu)
+        {
+            const uint64_t equal = __builtin_amdgcn_ballot_w64(key[s] == threshold);
+            taken = key[s] > threshold || (key[s] == threshold && equals_before + static_cast<uint32_t>(lanes_below(equal)) < equals);
+            equals_before += static_cast<uint32_t>(__popcll(equal));
+        }
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(taken);
+        if (taken)
+        {
+            const uint32_t place = count + static_cast<uint32_t>(lanes_below(mask));
+            scratch.candidates[place] = (static_cast<uint64_t>(key[s]) << 32) | (0xffffffffu - static_cast<uint32_t>(s * kWaveSize + lane));
+            scratch.scores[place] = score[s];
+        }
+        count += static_cast<uint32_t>(__popcll(mask));
+    }
+    if (lane < 4)
+    {
+        scratch.candidates[count + static_cast<uint32_t>(lane)] = 0ull;
+        scratch.selected[top_k + static_cast<uint32_t>(lane)] = 0.0f;
+    }
+    wave_lds_fence();
+    const uint64_t mine = static_cast<uint32_t>(lane) < count ? scratch.candidates[lane] : 0ull;
+    my_score = static_cast<uint32_t>(lane) < count ? scratch.scores[lane] : 0.0f;
+    uint32_t rank = 0;
+    for (uint32_t i = 0; i < count; i += 4u)
+    {
+        const ulonglong2 two = *reinterpret_cast<const ulonglong2*>(&scratch.candidates[i]);
+        const ulonglong2 more = *reinterpret_cast<const ulonglong2*>(&scratch.candidates[i + 2u]);
+        rank += (two.x > mine ? 1u : 0u) + (two.y > mine ? 1u : 0u) + (more.x > mine ? 1u : 0u) + (more.y > mine ? 1u : 0u);
+    }
+    my_expert = 0xffffffffu - static_cast<uint32_t>(mine);
+    my_rank = static_cast<uint32_t>(lane) < count ? rank : 0xffffffffu;
+    if (my_rank < top_k)
+        scratch.selected[my_rank] = my_score;
+    wave_lds_fence();
+    float selected_sum = 0.0f;
+    for (uint32_t i = 0; i < top_k; i += 4u)
+    {
+        const float4 four = *reinterpret_cast<const float4*>(&scratch.selected[i]);
+        selected_sum = (((selected_sum + four.x) + four.y) + four.z) + four.w;
+    }
+    return selected_sum;
+}
+
+// The routes that the caller names (src/graph/expert_dispatcher.cpp:124-135), rank = position; `scores`: the token's
+// scores, `divisor`: what they still have to be divided by.  False: an id is out of range.
+__device__ __forceinline__ bool take_explicit(const RouterArgs& r, const float* scores, float divisor, uint32_t token, int lane, uint32_t& my_expert,
+                                              uint32_t& my_rank, float& my_score, float& selected_sum)
+{
+    const int top_k = static_cast<int>(r.top_k);
+    my_expert = lane < top_k ? r.explicit_ids[static_cast<size_t>(token) * r.top_k + lane] : 0u;
+    if (__builtin_amdgcn_ballot_w64(my_expert >= r.experts) != 0ull)
+    {
+        if (lane == 0)
+            atomicMin(&r.error_words[1], (token << 3) | NCNN_MOE_ROUTER_EXPERT_OUT_OF_RANGE);
+        return false;
+    }
+    my_rank = lane < top_k ? static_cast<uint32_t>(lane) : 0xffffffffu;
+    my_score = lane < top_k ? scores[my_expert] / divisor : 0.0f;
+    selected_sum = 0.0f;
+    for (int rank = 0; rank < top_k; ++rank)
+        selected_sum += read_lane(my_score, rank);
+    return true;
+}
+
+// A token's routes from its scores in LDS (not yet divided by `divisor`), by one wave.
+template <int SLOTS, bool FUSED>
+__device__ __forceinline__ void route_token(const RouterArgs& r, const float* scores, float divisor, RouteScratch& scratch, uint32_t token, int lane)
+{
+    uint32_t my_expert, my_rank;
+    float my_score, selected_sum;
+    if (r.explicit_ids != nullptr)
+    {
+        if (!take_explicit(r, scores, divisor, token, lane, my_expert, my_rank, my_score, selected_sum))
+            return;
+    }
+    else
+    {
+        float score[SLOTS], bias[SLOTS];
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+        {
+            const uint32_t e = static_cast<uint32_t>(s * kWaveSize + lane);
+            bias[s] = (e < r.experts && r.selection_bias != nullptr) ? r.selection_bias[e] : 0.0f;
+            score[s] = e < r.experts ? scores[e] : 0.0f;
+        }
+        if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+        {
+#pragma unroll
+            for (int s = 0; s < SLOTS; ++s)
+                score[s] = score[s] / divisor;
+        }
+        selected_sum = select_best<SLOTS>(r, score, bias, scratch, lane, my_expert, my_rank, my_score);
+    }
+    // ---- src/graph/expert_dispatcher.cpp:144-150
+    if (r.renormalize != 0u && selected_sum <= 0.0f)
+    {
+        if (lane == 0)
+            atomicMin(&r.error_words[1], (token << 3) | NCNN_MOE_ROUTER_NON_POSITIVE_SUM);
+        return;
+    }
+    if (my_rank < r.top_k)
+    {
+        const float weight = (r.renormalize != 0u ? my_score / selected_sum : my_score) * r.scaling;
+        uint32_t* const expert_out = &r.selected_experts[static_cast<size_t>(token) * r.top_k + my_rank];
+        float* const weight_out = &r.selected_weights[static_cast<size_t>(token) * r.top_k + my_rank];
+        if constexpr (FUSED)
+        {
+            // written through the per-XCD L2: the workgroup that groups the routes may sit on another XCD
+            store_agent(expert_out, my_expert);
+            store_agent(reinterpret_cast<uint32_t*>(weight_out), __float_as_uint(weight));
+        }
+        else
+        {
+            *expert_out = my_expert;
+            *weight_out = weight;
+            // (a call of one chunk is counted by the workgroup that groups it)
+            atomicAdd(&r.chunk_counts[static_cast<size_t>(token / kRouterChunkTokens) * chunk_count_stride(r.experts) + my_expert], 1u);
+        }
+    }
+}
+
+// Calls of more than one chunk: a wave takes TOKENS tokens from their logits to their routes, without waiting for another
+// wave.  The scores pass through LDS, so that the softmax sum, one addition at a time in expert order, is a chain of
+// additions on four scores a read (lane reads, one per addition, took half as long again), one for all of the wave's tokens.
+// What bounds it: instructions, some 680 per token of 256 experts under the softmax: 320 for the sum, 110 for the
+// exponentials, 50 for the divisions, 130 for the selection.  16,384 tokens, 8 routes of 256 experts, softmax: 44 us with
+// one wave-wide maximum per route, 20 us so.  Sums of several waves' tokens by one of them, behind barriers, take half of
+// the instructions and no less time.
+constexpr int kBatchWaves = 4;
+constexpr int kBatchThreads = kBatchWaves * kWaveSize;
+
+template <int SLOTS, int TOKENS>
+__global__ __launch_bounds__(kBatchThreads) void router_batch_kernel(RouterArgs r)
+{
+    constexpr uint32_t kRow = SLOTS * kWaveSize + 4; // (the rows' offset keeps the lanes of the sums on different banks)
+    __shared__ __align__(16) float rows[kBatchWaves * TOKENS * kRow];
+    __shared__ __align__(16) RouteScratch scratch[kBatchWaves];
+    __shared__ uint64_t exp2_table[32];
+    const int lane = threadIdx.x & (kWaveSize - 1);
+    const int wave = threadIdx.x >> 6;
+    const uint32_t first_token = (blockIdx.x * kBatchWaves + static_cast<uint32_t>(wave)) * TOKENS;
+    float* const own_rows = rows + wave * TOKENS * kRow;
+    float logit[TOKENS][SLOTS];
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t)
+    {
+        const float* logits = r.logits + static_cast<size_t>(min(first_token + t, r.tokens - 1u)) * r.experts;
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+        {
+            const uint32_t e = static_cast<uint32_t>(s * kWaveSize + lane);
+            logit[t][s] = e < r.experts ? logits[e] : -__builtin_inff();
+        }
+    }
+    if (threadIdx.x < 32)
+        exp2_table[threadIdx.x] = kExp2Table[threadIdx.x];
+    __syncthreads();
+    // lane t: the largest logit of token t
+    float maxima = 0.0f;
+    uint32_t failed = 0u; // the tokens with a logit that is not finite
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t)
+    {
+        bool finite = true;
+        float maximum = -__builtin_inff();
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+        {
+            finite = finite && (static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts || is_finite_f32(logit[t][s]));
+            maximum = fmaxf(maximum, logit[t][s]);
+            own_rows[t * kRow + s * kWaveSize + lane] = logit[t][s];
+        }
+        if (__builtin_amdgcn_ballot_w64(!finite) != 0ull)
+            failed |= 1u << t;
+        if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+        {
+            maximum = wave_max(maximum);
+            maxima = lane == t ? maximum : maxima;
+        }
+    }
+    // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
+    float sums = 1.0f;
+    const auto each_score = [&](auto score_of) {
+#pragma unroll 1
+        for (int t = 0; t < TOKENS; ++t)
+        {
+            float* const row = own_rows + t * kRow + lane;
+            const float maximum = read_lane(maxima, t);
+            // (four experts of a lane overlap; more would take registers that waves in flight need)
+            constexpr int kTogether = SLOTS < 4 ? SLOTS : 4;
+#pragma unroll 1
+            for (int first = 0; first < SLOTS; first += kTogether)
+            {
+                float score[kTogether];
+#pragma unroll
+                for (int s = 0; s < kTogether; ++s)
+                    score[s] = score_of(row[(first + s) * kWaveSize], maximum);
+#pragma unroll
+                for (int s = 0; s < kTogether; ++s)
+                    row[(first + s) * kWaveSize] = score[s];
+            }
+        }
+        wave_lds_fence();
+    };
+    wave_lds_fence();
+    if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+    {
+        // (past the last expert: exp(-inf) is 0)
+        each_score([&](float x, float maximum) { return expf_selects(x - maximum, exp2_table); });
+        sums = sequential_row_sums(own_rows + (lane % TOKENS) * kRow, SLOTS * kWaveSize);
+    }
+    else if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
+        each_score([&](float x, float) { return sigmoid_score(x, exp2_table); });
+    else
+        each_score([&](float x, float) { return sqrt_softplus_score(x, exp2_table); });
+#pragma unroll 1
+    for (int t = 0; t < TOKENS; ++t)
+    {
+        const uint32_t token = first_token + static_cast<uint32_t>(t);
+        if (token >= r.tokens)
+            break;
+        if ((failed >> t & 1u) != 0u)
+        {
+            // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
+            if (lane == 0)
+                atomicOr(&r.error_words[0], 1u);
+            continue;
+        }
+        route_token<SLOTS, false>(r, own_rows + t * kRow, read_lane(sums, t), scratch[wave], token, lane);
+        wave_lds_fence();
+    }
+}
+
+// Calls of one chunk of tokens (decode-sized): a workgroup takes kStagedTokensPerBlock tokens and all its threads compute
+// the scores, one or a few experts each, into LDS; a wave per token then selects from there.  (A token's scores are two
+// fifths of a lone wave's time for it; spread over four waves they take a quarter as long.)
 constexpr int kStagedTokensPerBlock = 2;
 constexpr int kStagedThreadsPerToken = kRouterThreads / kStagedTokensPerBlock;
 
-__device__ __forceinline__ float router_score_of_logit(float logit, uint32_t score_function);
+struct RouterShared
+{
+    float scores[kStagedTokensPerBlock][NCNN_MOE_ROUTER_MAX_EXPERTS];
+    uint32_t non_finite[kStagedTokensPerBlock];    // the token holds a non-finite logit
+    float maximum[kRouterWavesPerBlock];           // softmax: the waves' maxima
+    RouteScratch scratch[kStagedTokensPerBlock];
+    uint64_t exp2_table[32];
+};
 
 __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterShared& shared, uint32_t first_token)
 {
@@ -165,7 +503,6 @@ __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterSh
     const uint32_t token = first_token + static_cast<uint32_t>(slot);
     if (threadIdx.x < kStagedTokensPerBlock)
         shared.non_finite[threadIdx.x] = 0u;
-    __syncthreads();
     constexpr int kPerThread = NCNN_MOE_ROUTER_MAX_EXPERTS / kStagedThreadsPerToken;
     float logit[kPerThread];
     bool finite = true;
@@ -179,207 +516,44 @@ __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterSh
         finite = finite && (e >= r.experts || is_finite_f32(logit[k]));
         maximum = fmaxf(maximum, logit[k]);
     }
-    if (token < r.tokens && !finite)
-        shared.non_finite[slot] = 1u;
+    if (threadIdx.x < 32)
+        shared.exp2_table[threadIdx.x] = kExp2Table[threadIdx.x];
     if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
     {
         // the row maximum first (src/graph/expert_dispatcher.cpp:44-46); the sum stays with the selecting wave
         maximum = wave_max(maximum);
         if ((threadIdx.x & (kWaveSize - 1)) == 0)
-            shared.staged_maximum[threadIdx.x >> 6] = maximum;
-        __syncthreads();
-        constexpr int kWavesPerToken = kStagedThreadsPerToken / kWaveSize;
-        maximum = shared.staged_maximum[slot * kWavesPerToken];
-#pragma unroll
-        for (int w = 1; w < kWavesPerToken; ++w)
-            maximum = fmaxf(maximum, shared.staged_maximum[slot * kWavesPerToken + w]);
-    }
-#pragma unroll
-    for (int k = 0; k < kPerThread; ++k)
-    {
-        const uint32_t e = static_cast<uint32_t>(k * kStagedThreadsPerToken + member);
-        if (token < r.tokens && e < r.experts)
-            shared.scores[slot][e] = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? expf_libm(logit[k] - maximum)
-                                                                                : router_score_of_logit(logit[k], r.score_function);
+            shared.maximum[threadIdx.x >> 6] = maximum;
     }
     __syncthreads();
-}
-
-// One wave per token.  Expert e lives in slot e / 64 of lane e % 64, so a loop over slots, then lanes,
-// visits the experts in index order: the softmax sum is the CPU loop itself, one fp32 addition at a
-// time.  The routes are chosen one per round and stay in registers: lane r keeps the route of rank r.
-template <int SLOTS, bool COUNT_CHUNKS, bool STAGED>
-__device__ __forceinline__ void select_token_routes(const RouterArgs& r, RouterShared& shared, uint32_t token, int lane, int wave)
-{
-    const int experts = static_cast<int>(r.experts);
-    const int top_k = static_cast<int>(r.top_k);
-    const float* logits = r.logits + static_cast<size_t>(token) * r.experts;
-    const bool explicit_routes = r.explicit_ids != nullptr;
-
-    // every load of the token up front
-    float logit[SLOTS];
-    float bias[SLOTS];
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s)
-    {
-        const int e = s * kWaveSize + lane;
-        logit[s] = (e < experts && !STAGED) ? logits[e] : 0.0f;
-        bias[s] = (e < experts && r.selection_bias != nullptr && !explicit_routes) ? r.selection_bias[e] : 0.0f;
-    }
-    uint32_t my_expert = (explicit_routes && lane < top_k) ? r.explicit_ids[static_cast<size_t>(token) * r.top_k + lane] : 0u;
-
-    bool finite = true;
-    float maximum = -__builtin_inff();
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s)
-    {
-        const int e = s * kWaveSize + lane;
-        if (e < experts)
-        {
-            finite = finite && is_finite_f32(logit[s]);
-            maximum = fmaxf(maximum, logit[s]);
-        }
-    }
-    if (STAGED ? shared.non_finite[wave] != 0u : __ballot(!finite) != 0)
-    {
-        // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
-        if (lane == 0)
-            atomicOr(&r.error_words[0], 1u);
-        return;
-    }
-
-    // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
-    float score[SLOTS];
+    if (token < r.tokens && !finite)
+        shared.non_finite[slot] = 1u;
     if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
     {
-        maximum = wave_max(maximum);
+        constexpr int kWavesPerToken = kStagedThreadsPerToken / kWaveSize;
+        maximum = shared.maximum[slot * kWavesPerToken];
 #pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-        {
-            if constexpr (STAGED)
-                score[s] = (s * kWaveSize + lane) < experts ? shared.scores[wave][s * kWaveSize + lane] : 0.0f;
-            else
-                score[s] = (s * kWaveSize + lane) < experts ? expf_libm(logit[s] - maximum) : 0.0f;
-        }
-        float sum = 0.0f;
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-        {
-            // in trips of eight (a loop trip of a lone wave costs as much as a dozen additions); the
-            // lanes past the last expert hold 0, which leaves the sum as it is
-            const int slot_count = min(kWaveSize, experts - s * kWaveSize);
-            for (int trip = 0; trip * 8 < slot_count; ++trip)
-            {
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    sum += read_lane(score[s], trip * 8 + k);
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-            score[s] = score[s] / sum;
+        for (int w = 1; w < kWavesPerToken; ++w)
+            maximum = fmaxf(maximum, shared.maximum[slot * kWavesPerToken + w]);
     }
-    else if constexpr (STAGED)
-    {
+    // (the row is filled up to a multiple of 64 with zeros)
+    const uint32_t padded = (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize;
+    const auto each_score = [&](auto score_of) {
 #pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-            score[s] = (s * kWaveSize + lane) < experts ? shared.scores[wave][s * kWaveSize + lane] : 0.0f;
-    }
+        for (int k = 0; k < kPerThread; ++k)
+        {
+            const uint32_t e = static_cast<uint32_t>(k * kStagedThreadsPerToken + member);
+            if (e < padded)
+                shared.scores[slot][e] = e >= r.experts ? 0.0f : score_of(logit[k]);
+        }
+    };
+    if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+        each_score([&](float x) { return expf_selects(x - maximum, shared.exp2_table); });
+    else if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
+        each_score([&](float x) { return sigmoid_score(x, shared.exp2_table); });
     else
-    {
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-            score[s] = (s * kWaveSize + lane) < experts ? router_score_of_logit(logit[s], r.score_function) : 0.0f;
-    }
-
-    float my_score = 0.0f;
-    float selected_sum = 0.0f;
-    if (explicit_routes)
-    {
-        // src/graph/expert_dispatcher.cpp:124-135: the caller names the experts; rank = position
-        const bool in_range = lane >= top_k || my_expert < r.experts;
-        if (__ballot(!in_range) != 0)
-        {
-            if (lane == 0)
-                atomicMin(&r.error_words[1], (token << 3) | NCNN_MOE_ROUTER_EXPERT_OUT_OF_RANGE);
-            return;
-        }
-        // (staged scores are in LDS already, but a softmax row only before its division by the sum)
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-        {
-            const int e = s * kWaveSize + lane;
-            if (e < experts)
-                shared.scores[wave][e] = score[s];
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f); // this wave's LDS writes, before its lanes read them back
-        __builtin_amdgcn_wave_barrier();
-        if (lane < top_k)
-            my_score = shared.scores[wave][my_expert];
-        for (int rank = 0; rank < top_k; ++rank)
-            selected_sum += read_lane(my_score, rank);
-    }
-    else
-    {
-        // ---- select_topk_routes (src/graph/expert_dispatcher.cpp:61-77): the best top_k by
-        // (score + bias descending, expert id ascending), one per round; the selected scores are
-        // summed in rank order (src/graph/expert_dispatcher.cpp:137-143)
-        float keyed[SLOTS];
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-            keyed[s] = score[s] + bias[s];
-        uint32_t taken = 0; // this lane's slots already selected
-        for (int round = 0; round < top_k; ++round)
-        {
-            // this lane's best remaining expert: the lowest slot (lowest id) among equals
-            float lane_best = -__builtin_inff();
-            float lane_score = 0.0f;
-            int lane_expert = 0x7fffffff; // none
-#pragma unroll
-            for (int s = 0; s < SLOTS; ++s)
-            {
-                const int e = s * kWaveSize + lane;
-                const bool available = e < experts && ((taken >> s) & 1u) == 0u;
-                if (available && (lane_expert == 0x7fffffff || keyed[s] > lane_best))
-                {
-                    lane_best = keyed[s];
-                    lane_score = score[s];
-                    lane_expert = e;
-                }
-            }
-            const float best = wave_max(lane_best);
-            int winner = wave_min((lane_expert != 0x7fffffff && lane_best == best) ? lane_expert : 0x7fffffff);
-            if (winner == 0x7fffffff) // selection scores that compare unordered: any remaining expert
-                winner = wave_min(lane_expert);
-            const int winner_lane = winner & (kWaveSize - 1);
-            const float winner_score = read_lane(lane_score, winner_lane);
-            if (lane == winner_lane)
-                taken |= 1u << (winner >> 6);
-            selected_sum += winner_score;
-            if (lane == round)
-            {
-                my_expert = static_cast<uint32_t>(winner);
-                my_score = winner_score;
-            }
-        }
-    }
-
-    // ---- src/graph/expert_dispatcher.cpp:144-150
-    if (r.renormalize != 0u && selected_sum <= 0.0f)
-    {
-        if (lane == 0)
-            atomicMin(&r.error_words[1], (token << 3) | NCNN_MOE_ROUTER_NON_POSITIVE_SUM);
-        return;
-    }
-    if (lane < top_k)
-    {
-        const float weight = (r.renormalize != 0u ? my_score / selected_sum : my_score) * r.scaling;
-        // written through the per-XCD L2: the workgroup that groups the routes may sit on another XCD
-        store_agent(&r.selected_experts[static_cast<size_t>(token) * r.top_k + lane], my_expert);
-        store_agent(reinterpret_cast<uint32_t*>(&r.selected_weights[static_cast<size_t>(token) * r.top_k + lane]), __float_as_uint(weight));
-        if (COUNT_CHUNKS) // a call of one chunk is counted by the workgroup that groups it
-            atomicAdd(&r.chunk_counts[static_cast<size_t>(token / kRouterChunkTokens) * r.experts + my_expert], 1u);
-    }
+        each_score([&](float x) { return sqrt_softplus_score(x, shared.exp2_table); });
+    __syncthreads();
 }
 
 // Grouping is a stable counting sort of the flat assignment array (token-major, so already in
@@ -393,11 +567,21 @@ struct GroupShared
     uint32_t wave_base[kRouterWavesPerBlock][NCNN_MOE_ROUTER_MAX_EXPERTS];
     uint32_t wave_totals[kRouterWavesPerBlock];
     uint32_t is_last;
+    uint32_t routed[NCNN_MOE_ROUTER_MAX_EXPERTS];        // several chunks: routes of all of them
+    uint32_t routed_before[NCNN_MOE_ROUTER_MAX_EXPERTS]; // ... and of those in front of this one
 };
+
+// What another workgroup of the same launch wrote is read around the L2, what the launch before wrote is not.
+template <bool FUSED>
+__device__ __forceinline__ uint32_t load_route_word(const uint32_t* address)
+{
+    return FUSED ? load_agent(address) : *address;
+}
 
 constexpr int kGroupExpertsPerThread = NCNN_MOE_ROUTER_MAX_EXPERTS / kRouterThreads; // experts one thread owns, at most
 constexpr int kGroupBatch = 8;                                                       // loads in flight per lane
 
+template <bool FUSED>
 __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupShared& shared, uint32_t chunk, uint32_t chunks)
 {
     const int tid = threadIdx.x;
@@ -421,11 +605,11 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
     for (int k = 0; k < kGroupBatch; ++k)
     {
         const uint32_t i = static_cast<uint32_t>(k * kWaveSize + lane);
-        first_named[k] = i < count ? load_agent(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
-        first_weight[k] = i < count ? __uint_as_float(load_agent(reinterpret_cast<const uint32_t*>(&r.selected_weights[first_assignment + i]))) : 0.0f;
+        first_named[k] = i < count ? load_route_word<FUSED>(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
+        first_weight[k] = i < count ? __uint_as_float(load_route_word<FUSED>(reinterpret_cast<const uint32_t*>(&r.selected_weights[first_assignment + i]))) : 0.0f;
     }
-    const uint32_t non_finite = load_agent(&r.error_words[0]);
-    const uint32_t first_bad = load_agent(&r.error_words[1]);
+    const uint32_t non_finite = load_route_word<FUSED>(&r.error_words[0]);
+    const uint32_t first_bad = load_route_word<FUSED>(&r.error_words[1]);
     uint32_t status = NCNN_MOE_ROUTER_OK;
     if (non_finite != 0u)
         status = NCNN_MOE_ROUTER_NON_FINITE_LOGIT;
@@ -458,7 +642,7 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
                     const uint32_t i = first + static_cast<uint32_t>(k * kWaveSize + lane);
                     named[k] = first_named[k];
                     if (first != 0u)
-                        named[k] = i < count ? load_agent(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
+                        named[k] = i < count ? load_route_word<FUSED>(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
                 }
 #pragma unroll
                 for (int k = 0; k < kGroupBatch; ++k)
@@ -480,7 +664,7 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
             total[j] = 0u;
             before[j] = 0u;
         }
-        if (chunks == 1u)
+        if constexpr (FUSED)
         {
             build_histogram();
 #pragma unroll
@@ -497,16 +681,53 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
         }
         else
         {
-#pragma unroll 8
-            for (uint32_t c = 0; c < chunks; ++c)
+            // a wave adds every eighth chunk's counters, four experts a lane, the loads of eight chunks in flight together (a
+            // load per expert and chunk, a few at a time, was half of the kernel)
+            for (uint32_t e = tid; e < experts; e += kRouterThreads)
+                shared.routed[e] = shared.routed_before[e] = 0u;
+            lds_barrier();
+            const uint32_t quads = chunk_count_stride(experts) / 4u;
+            for (uint32_t first_quad = 0; first_quad < quads; first_quad += kWaveSize)
             {
-#pragma unroll
-                for (int j = 0; j < kGroupExpertsPerThread; ++j)
+                const uint32_t quad = first_quad + static_cast<uint32_t>(lane);
+                const uint4* counts = reinterpret_cast<const uint4*>(r.chunk_counts) + min(quad, quads - 1u);
+                uint4 of_all{0u, 0u, 0u, 0u}, of_earlier{0u, 0u, 0u, 0u};
+                for (uint32_t first = static_cast<uint32_t>(wave); first < chunks; first += kRouterWavesPerBlock * kGroupBatch)
                 {
-                    const uint32_t e = tid * per_thread + j;
-                    const uint32_t routed = (static_cast<uint32_t>(j) < per_thread && e < experts) ? load_agent(&r.chunk_counts[c * experts + e]) : 0u;
-                    total[j] += routed;
-                    before[j] += c < chunk ? routed : 0u;
+                    uint4 routed[kGroupBatch];
+#pragma unroll
+                    for (int k = 0; k < kGroupBatch; ++k)
+                        routed[k] = counts[static_cast<size_t>(min(first + k * kRouterWavesPerBlock, chunks - 1u)) * quads];
+#pragma unroll
+                    for (int k = 0; k < kGroupBatch; ++k)
+                    {
+                        const uint32_t c = first + k * kRouterWavesPerBlock;
+                        const uint32_t all = c < chunks ? 0xffffffffu : 0u, earlier = c < chunk ? 0xffffffffu : 0u;
+                        of_all.x += routed[k].x & all, of_all.y += routed[k].y & all, of_all.z += routed[k].z & all, of_all.w += routed[k].w & all;
+                        of_earlier.x += routed[k].x & earlier, of_earlier.y += routed[k].y & earlier;
+                        of_earlier.z += routed[k].z & earlier, of_earlier.w += routed[k].w & earlier;
+                    }
+                }
+                const uint32_t add[8] = {of_all.x, of_all.y, of_all.z, of_all.w, of_earlier.x, of_earlier.y, of_earlier.z, of_earlier.w};
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j)
+                {
+                    if (4u * quad + j < experts)
+                    {
+                        atomicAdd(&shared.routed[4u * quad + j], add[j]);
+                        atomicAdd(&shared.routed_before[4u * quad + j], add[4u + j]);
+                    }
+                }
+            }
+            lds_barrier();
+#pragma unroll
+            for (int j = 0; j < kGroupExpertsPerThread; ++j)
+            {
+                const uint32_t e = tid * per_thread + j;
+                if (static_cast<uint32_t>(j) < per_thread && e < experts)
+                {
+                    total[j] = shared.routed[e];
+                    before[j] = shared.routed_before[e];
                 }
             }
         }
@@ -523,7 +744,7 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
         }
         if (lane == kWaveSize - 1)
             shared.wave_totals[wave] = inclusive;
-        if (chunks == 1u)
+        if constexpr (FUSED)
             __syncthreads();
         else
             build_histogram();
@@ -568,8 +789,8 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
                 weight[k] = first_weight[k];
                 if (first != 0u)
                 {
-                    named[k] = i < count ? load_agent(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
-                    weight[k] = i < count ? __uint_as_float(load_agent(reinterpret_cast<const uint32_t*>(&r.selected_weights[first_assignment + i]))) : 0.0f;
+                    named[k] = i < count ? load_route_word<FUSED>(&r.selected_experts[first_assignment + i]) : 0xffffffffu;
+                    weight[k] = i < count ? __uint_as_float(load_route_word<FUSED>(reinterpret_cast<const uint32_t*>(&r.selected_weights[first_assignment + i]))) : 0.0f;
                 }
             }
 #pragma unroll
@@ -611,13 +832,13 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
     if (tid == 0)
     {
         const uint32_t finished =
-            chunks == 1u ? 0u : __hip_atomic_fetch_add(r.finished_chunks, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        shared.is_last = finished == chunks - 1u ? 1u : 0u;
+            FUSED ? 0u : __hip_atomic_fetch_add(r.finished_chunks, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        shared.is_last = FUSED || finished == chunks - 1u ? 1u : 0u;
     }
     __syncthreads();
     if (shared.is_last != 0u)
     {
-        for (uint32_t i = tid; chunks > 1u && i < chunks * experts; i += kRouterThreads)
+        for (uint32_t i = tid; !FUSED && i < chunks * chunk_count_stride(experts); i += kRouterThreads)
             r.chunk_counts[i] = 0u;
         if (tid == 0)
         {
@@ -631,45 +852,50 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
 __global__ __launch_bounds__(kRouterThreads) void router_group_kernel(RouterArgs r)
 {
     __shared__ GroupShared shared;
-    place_chunk_routes(r, shared, blockIdx.x, gridDim.x);
+    place_chunk_routes<false>(r, shared, blockIdx.x, gridDim.x);
 }
 
-// FUSED (calls of at most one chunk of tokens): the workgroup that finishes last also places the
-// routes, so the whole dispatch is one launch.
-template <int SLOTS, bool FUSED, bool STAGED>
+// Calls of at most one chunk of tokens: the workgroup that finishes last also places the routes, so the whole dispatch is
+// one launch.
+template <int SLOTS>
 __global__ __launch_bounds__(kRouterThreads) void router_select_kernel(RouterArgs r)
 {
-    static_assert(FUSED || !STAGED, "staged scoring serves the single-launch calls");
     __shared__ RouterShared shared;
+    __shared__ GroupShared group_shared;
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = threadIdx.x >> 6;
-    constexpr int kTokensPerBlock = STAGED ? kStagedTokensPerBlock : kRouterWavesPerBlock;
-    const uint32_t token = blockIdx.x * kTokensPerBlock + wave;
-    if constexpr (STAGED)
-        stage_token_scores(r, shared, blockIdx.x * kTokensPerBlock);
-    if (wave < kTokensPerBlock && token < r.tokens)
-        select_token_routes<SLOTS, !FUSED, STAGED>(r, shared, token, lane, wave);
-    if constexpr (FUSED)
+    const uint32_t token = blockIdx.x * kStagedTokensPerBlock + wave;
+    stage_token_scores(r, shared, blockIdx.x * kStagedTokensPerBlock);
+    if (wave < kStagedTokensPerBlock && token < r.tokens)
     {
-        __shared__ GroupShared group_shared;
-        // this workgroup's routes (written through), counts and error words (atomics) have landed once
-        // its waves have waited for them; then the workgroup is counted, and whoever counts last reads
-        // every other workgroup's around its own L2: no cache write-back or invalidate is needed
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (threadIdx.x == 0)
+        if (shared.non_finite[wave] != 0u)
         {
-            const uint32_t finished = __hip_atomic_fetch_add(r.finished_selects, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            group_shared.is_last = finished == gridDim.x - 1u ? 1u : 0u;
+            // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
+            if (lane == 0)
+                atomicOr(&r.error_words[0], 1u);
         }
-        __syncthreads();
-        if (group_shared.is_last == 0u)
-            return;
-        if (threadIdx.x == 0)
-            *r.finished_selects = 0u;
-        __syncthreads(); // is_last is read by all before place_chunk_routes writes it again
-        place_chunk_routes(r, group_shared, 0u, 1u);
+        else
+        {
+            const float sum = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? sequential_row_sums(shared.scores[wave], (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize) : 1.0f;
+            route_token<SLOTS, true>(r, shared.scores[wave], sum, shared.scratch[wave], token, lane);
+        }
     }
+    // this workgroup's routes (written through), counts and error words (atomics) have landed once
+    // its waves have waited for them; then the workgroup is counted, and whoever counts last reads
+    // every other workgroup's around its own L2: no cache write-back or invalidate is needed
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        const uint32_t finished = __hip_atomic_fetch_add(r.finished_selects, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        group_shared.is_last = finished == gridDim.x - 1u ? 1u : 0u;
+    }
+    __syncthreads();
+    if (group_shared.is_last == 0u)
+        return;
+    if (threadIdx.x == 0)
+        *r.finished_selects = 0u;
+    place_chunk_routes<true>(r, group_shared, 0u, 1u);
 }
 
 __global__ void log1pf_probe_kernel(const float* in, float* out, size_t n)

@@ -1,0 +1,37 @@
+"""The router on calls of several thousand tokens (GPU), where a wave takes one token or two: the oracle's plan, at
+token counts that leave waves and workgroups incomplete, with ties and thresholds that many experts share."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import oracle_lib
+from ncnn_moe_runtime_amd import hip_router
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")  # before the router library, so that both bind the same HIP runtime
+
+
+@pytest.mark.parametrize("tokens,experts,top_k", [(8191, 64, 6), (8192, 8, 8), (8195, 100, 12), (4111, 256, 8), (1003, 512, 3), (515, 1024, 64)])
+def test_batches_match_the_oracle(tokens, experts, top_k):
+    rng = np.random.default_rng(tokens * 31 + experts)
+    logits = (rng.standard_normal((tokens, experts)) * 2).astype(np.float32)
+    logits[1::5] = np.round(logits[1::5] * 4) / 4   # ties all over the row
+    logits[2::7] = np.float32(1.5)                  # every score equal
+    logits[3::11, experts // 2:] *= np.float32(60)  # scores that saturate or vanish
+    bias = (rng.standard_normal(experts) * 0.3).astype(np.float32)
+    with contextlib.closing(hip_router.HipRouter(tokens, experts, top_k)) as router:
+        for score in (hip_router.SOFTMAX, hip_router.SIGMOID, hip_router.SQRT_SOFTPLUS):
+            for options in (dict(), dict(selection_bias=bias, renormalize=False, routed_scaling_factor=2.5),
+                            dict(explicit_expert_ids=rng.integers(0, experts, (tokens, top_k)).astype(np.uint32), renormalize=False)):
+                print("[case] %d tokens, %d experts, top %d, score %d, %s" % (tokens, experts, top_k, score, sorted(options)), flush=True)
+                status, offsets, routes = router.dispatch(logits, top_k, score_function=score, **options)
+                cpu_status, cpu_offsets, cpu_routes = oracle_lib.oracle_router_dispatch(logits, top_k, score_function=score, **options)
+                assert status == cpu_status == 0
+                assert np.array_equal(offsets, cpu_offsets)
+                for field in ("token_index", "rank"):
+                    assert np.array_equal(routes[field], cpu_routes[field]), field
+                assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
+        logits[tokens - 1, experts - 1] = np.inf
+        assert router.dispatch(logits, top_k)[0] == hip_router.STATUS_NON_FINITE_LOGIT
