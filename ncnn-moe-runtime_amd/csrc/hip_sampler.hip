@@ -292,6 +292,14 @@ struct SamplerPasses
     bool side_by_side = false; // the wide select on the handle's second stream, beside the full-order kernels
 };
 
+template <int DTYPE, bool ROOMY>
+void launch_bin_walks(const BinArgs& g, hipStream_t stream)
+{
+    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 0, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 1, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+}
+
 // Enqueues what follows the first select: the window kernels (sampler_windows.h) and the binned sums (sampler_bins.h) for
 // the rows that it left pending; by_options: for those that it leaves by their options.
 template <int DTYPE>
@@ -316,9 +324,10 @@ void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windo
         hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
         hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
         hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
-        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 0>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 1>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-        hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+        if (a.rows <= kRoomyRows)
+            launch_bin_walks<DTYPE, true>(g, stream);
+        else
+            launch_bin_walks<DTYPE, false>(g, stream);
     }
 }
 

@@ -58,6 +58,11 @@ constexpr uint32_t kMaxBinParts = 16;
 constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers in flight together
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
 constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
+// The walks want 220 registers; at 128, which two of their workgroups to a compute unit leave, some 35 of them and 130
+// scalars pass through scratch and lane moves.  A call of so few rows that every part has a compute unit of its own takes
+// the walks built for 256 (8 x 151,936 without a window: 141 -> 131 us, 11 such rows of a verification step: 240 -> 223 us);
+// more rows need the second workgroup.
+constexpr uint32_t kRoomyRows = kBinGrid / 2u / kMaxBinParts;
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
 // (the foreseen sums were off by a few 1e-5 at most; where a sum grows by single ulps a margin of 1e-4 lists 1,700 elements
 // at most on both sides of a power of two, so that they always fit)
@@ -1124,9 +1129,15 @@ __device__ __forceinline__ uint32_t fine_place(float term, uint32_t shift, uint3
 
 // Fetches the elements of bins [shared.low, shared.high] (at most kBinExtraCap of them; shared.extra_count: how many there
 // are), in order, to shared.terms[kBinExtraPlace ..].
+// What bounds it: the row's terms through one compute unit with two wavefronts per SIMD in flight.  Every load waited for
+// in turn and five instructions per element took 20 us for 151,936 terms, and with many rows the call waits for the one
+// that fetches most often; with the next loads under way and one comparison per element a call of 512 mixed rows of
+// 129,280 takes 352 us instead of 366.
+template <bool ROOMY>
 __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t positions, uint32_t misalignment, uint32_t shift, BinWalkShared& shared, int tid)
 {
-    constexpr int kLoads = 8;
+    constexpr uint32_t kLoads = ROOMY ? 8 : 4; // (twice: those under way and those looked at)
+    constexpr uint32_t kStride = kLoads * kWalkThreads;
     if (tid == 0)
     {
         shared.extra_count = 0u;
@@ -1136,34 +1147,49 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     __syncthreads();
     const uint32_t top = kOneBits - (shared.low << shift);        // bits of the largest term wanted
     const uint32_t width = (shared.high + 1u - shared.low) << shift;
+    // (the bins end kTailDistance below one: neither a term below them nor a zero lies within `width` of `top`)
+    static_assert((kBins << 17) == kTailDistance && ((kTailDistance - 1u) >> 17) < kBins, "a bin is at most 2^17 wide");
     const uint32_t vectors = positions / 4u;
-    for (uint32_t at = tid; at < vectors; at += kLoads * kWalkThreads)
-    {
-        float4 raw[kLoads];
+    const auto load = [&](uint4 (&raw)[kLoads], uint32_t at) {
 #pragma unroll
-        for (int k = 0; k < kLoads; ++k)
-            raw[k] = reinterpret_cast<const float4*>(terms)[min(at + k * kWalkThreads, vectors - 1u)];
+        for (uint32_t k = 0; k < kLoads; ++k)
+            raw[k] = reinterpret_cast<const uint4*>(terms)[min(at + k * kWalkThreads, vectors - 1u)];
+    };
+    const auto take = [&](const uint4 (&raw)[kLoads], uint32_t at) {
 #pragma unroll
-        for (int k = 0; k < kLoads; ++k)
+        for (uint32_t k = 0; k < kLoads; ++k)
         {
+            const uint32_t bits[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+            const uint32_t nearest = min(min(top - bits[0], top - bits[1]), min(top - bits[2], top - bits[3]));
             const uint32_t v = at + k * kWalkThreads;
-            const float t[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
+            if (nearest >= width || v >= vectors)
+                continue;
+#pragma unroll 1
+            for (uint32_t c = 0; c < 4u; ++c)
             {
-                const uint32_t bits = __float_as_uint(t[c]);
-                if (top - bits < width && kOneBits - bits < kTailDistance && v < vectors)
+                const uint32_t of_element = c == 0u ? bits[0] : c == 1u ? bits[1] : c == 2u ? bits[2] : bits[3];
+                if (top - of_element >= width)
+                    continue;
+                const uint32_t at_place = atomicAdd(&shared.extra_count, 1u);
+                atomicMin(&shared.extra_least, of_element);
+                atomicMax(&shared.extra_most, of_element);
+                if (at_place < kBinExtraCap)
                 {
-                    const uint32_t at_place = atomicAdd(&shared.extra_count, 1u);
-                    atomicMin(&shared.extra_least, bits);
-                    atomicMax(&shared.extra_most, bits);
-                    if (at_place < kBinExtraCap)
-                    {
-                        shared.terms[kBinExtraPlace + at_place] = t[c];
-                        shared.tokens[kBinExtraPlace + at_place] = v * 4u + c - misalignment;
-                    }
+                    shared.terms[kBinExtraPlace + at_place] = __uint_as_float(of_element);
+                    shared.tokens[kBinExtraPlace + at_place] = v * 4u + c - misalignment;
                 }
             }
+        }
+    };
+    {
+        uint4 raw[kLoads], more[kLoads];
+        load(raw, tid);
+        for (uint32_t at = tid; at < vectors; at += 2u * kStride)
+        {
+            load(more, at + kStride);
+            take(raw, at);
+            load(raw, at + 2u * kStride);
+            take(more, at + kStride);
         }
     }
     __syncthreads();
@@ -1171,6 +1197,7 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     if (count <= kBinExtraCap)
     {
         constexpr uint32_t kPerThread = (kBinExtraCap + kWalkThreads - 1) / kWalkThreads;
+        const float places_per_bit = static_cast<float>(count) / static_cast<float>(width);
         float own[kPerThread];
         uint32_t token[kPerThread], fine[kPerThread];
 #pragma unroll
@@ -1183,7 +1210,8 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
             {
                 own[k] = shared.terms[kBinExtraPlace + i];
                 token[k] = shared.tokens[kBinExtraPlace + i];
-                fine[k] = static_cast<uint32_t>((static_cast<uint64_t>(top - __float_as_uint(own[k])) * count) / width);
+                // (rounded, but never falling where the term falls)
+                fine[k] = min(static_cast<uint32_t>(static_cast<float>(top - __float_as_uint(own[k])) * places_per_bit), count - 1u);
             }
         }
         __syncthreads();
@@ -1316,7 +1344,7 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
 // fetches what it asks for.  Ends with shared.status 1 (ended: sum, stopped, ...) or 2 (given up).
 //   limit     elements that the sum runs over at most; cut_bin, cut_term: it ends at the first term below cut_term,
 //             which lies in that bin (kBins: nowhere)
-template <int PHASE>
+template <int PHASE, bool ROOMY>
 __device__ __forceinline__ void walk_bins(
     BinWalkShared& shared, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins,
     uint32_t limit, uint32_t cut_bin, float cut_term, float start_sum, int mode, float bound, float divisor, float second_divisor, int tid)
@@ -1527,7 +1555,7 @@ __device__ __forceinline__ void walk_bins(
         __syncthreads();
         if (shared.status != 0u)
             return;
-        fetch_bins(row_terms, positions, misalignment, shift, shared, tid);
+        fetch_bins<ROOMY>(row_terms, positions, misalignment, shift, shared, tid);
         fetched = true;
     }
 }
@@ -1579,8 +1607,9 @@ __device__ __forceinline__ int32_t token_of_listed(
 // ---- (4), (5), (6): WALK 0 walks the normaliser and, inside the head, the Top-P sum and the draw, WALK 1 the Top-P sum
 // behind the head (and the draw inside it), WALK 2 the draw behind the head.  Each then has the bins' steps of the next
 // sum added for the calling part of the row, unless the row is finished.  Every part of a row walks for itself.
-template <int DTYPE, int WALK>
-__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void bin_walk_kernel(BinArgs g)
+// ROOMY: at most kRoomyRows rows, one workgroup to a compute unit.
+template <int DTYPE, int WALK, bool ROOMY>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(ROOMY ? 2 : 4, ROOMY ? 2 : 4))) void bin_walk_kernel(BinArgs g)
 {
     __shared__ BinWalkShared shared;
     constexpr int kFrom = WALK & 1;      // which of the alternating buffers this launch reads
@@ -1658,14 +1687,15 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
             if (holds_bins && bin + 3u >= head_bins)
             {
                 const uint4* from = reinterpret_cast<const uint4*>(g.steps[kFrom] + first_pair * kBins) + tid;
-                for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
+                constexpr uint32_t kTogether = ROOMY ? kMaxBinParts : kPartsAtATime;
+                for (uint32_t first = 0; first < grid.parts; first += kTogether)
                 {
-                    uint4 of_part[kPartsAtATime];
+                    uint4 of_part[kTogether];
 #pragma unroll
-                    for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                    for (uint32_t k = 0; k < kTogether; ++k)
                         of_part[k] = from[static_cast<size_t>(min(first + k, grid.parts - 1u)) * kBinQuads];
 #pragma unroll
-                    for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                    for (uint32_t k = 0; k < kTogether; ++k)
                     {
                         const uint32_t some = first + k < grid.parts ? 0xffffffffu : 0u;
                         own_steps[0] += of_part[k].x & some, own_steps[1] += of_part[k].y & some;
@@ -1853,7 +1883,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
                 mass[j] += sum;
             if (behind_head)
             {
-                walk_bins<0>(shared, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+                walk_bins<0, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
                 given_up = shared.status == 2u;
                 sum = same_in_all(shared.sum);
             }
@@ -1921,7 +1951,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
         }
         if constexpr (WALK == 1)
         {
-            walk_bins<1>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
+            walk_bins<1, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
                          normalizer, 1.0f, tid);
             const bool stopped = shared.stopped != 0u;
             // (a sum that no stop condition ends runs to the window's end, or to the Min-P cut, which no bin may hold)
@@ -1989,7 +2019,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4,
             }
             if constexpr (WALK == 2)
             {
-                walk_bins<2>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
+                walk_bins<2, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
                              normalizer, renormalizer, tid);
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);

@@ -70,3 +70,23 @@ def test_draws_and_cuts_at_the_ends():
         sampler.upload_logits(logits)
         gpu = sampler.sample(params, uniforms)
     parity_util.assert_results_match(gpu, cpu, "f32", "ends")
+
+
+@pytest.mark.parametrize("rows", [16, 17])
+def test_walks_with_and_without_a_compute_unit_of_their_own(rows):
+    """The last number of rows whose walks have a compute unit each, and the first that share; many ties half way between two
+    sums, which the walks fetch."""
+    rng = np.random.default_rng(rows)
+    vocab = 65537
+    print("[case] walks, %d rows" % rows, flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 5000])
+    logits[::2] = rng.integers(-400, 400, (len(logits[::2]), vocab)).astype(np.float32) / 128
+    params["temperature"][::2] = 1.0
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+        again = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, "f32", "walks")
+    assert gpu.tobytes() == again.tobytes()
