@@ -300,35 +300,73 @@ void launch_bin_walks(const BinArgs& g, hipStream_t stream)
     hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
 }
 
-// Enqueues what follows the first select: the window kernels (sampler_windows.h) and the binned sums (sampler_bins.h) for
-// the rows that it left pending; by_options: for those that it leaves by their options.
+// The window kernels (sampler_windows.h) over the rows in the handle's window list.
 template <int DTYPE>
-void launch_later_rows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool sums, bool by_options, bool want_filters, hipStream_t stream)
+void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, hipStream_t stream)
 {
-    hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, by_options ? 1u : 0u,
-                       windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
+    WindowArgs w = s->windows;
+    w.a = a;
+    w.windows_are_selects = 1u;
+    hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
+    hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
+}
+
+// The binned sums (sampler_bins.h) over the rows in the handle's bin list; the walks, which finish rows, wait for
+// `before_walks` (null: for nothing).
+template <int DTYPE>
+hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool want_filters, hipEvent_t before_walks, hipStream_t stream)
+{
+    BinArgs g = s->bins;
+    g.a = a;
+    g.windows_are_selects = windows ? 1u : 0u;
+    g.want_filters = want_filters ? 1u : 0u;
+    hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
+    hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
+    hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
+    const hipError_t waits = before_walks != nullptr ? hipStreamWaitEvent(stream, before_walks, 0) : hipSuccess;
+    if (a.rows <= kRoomyRows)
+        launch_bin_walks<DTYPE, true>(g, stream);
+    else
+        launch_bin_walks<DTYPE, false>(g, stream);
+    return waits;
+}
+
+// Enqueues the first select and what follows it for the rows that it leaves pending: the window kernels and the binned
+// sums.  side_by_side: those rows are known by their options, and the chain of the sums (the longest, its walks a few
+// dependent steps a row) runs on the caller's stream while the select and the window kernels (bound by the stream of
+// logits) run on the handle's second one.  A walk marks its row as done, which the select marks as pending, so the walks
+// wait for the select; it has ended long before.  512 rows of 129,280, mixed options: 351 us one behind the
+// other, 321 us so.
+template <int DTYPE>
+hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
+                            bool want_filters, hipStream_t stream)
+{
+    const auto list_rows = [&]() {
+        hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, side_by_side ? 1u : 0u,
+                           windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
+    };
+    const auto select = [&](hipStream_t on) { launch_select<DTYPE>(geometry, a.rows, on, a, 0, s->scatter_segments != 0); };
+    if (side_by_side && windows && sums && s->side_stream != nullptr)
+    {
+        list_rows();
+        hipError_t result = hipEventRecord(s->side_fork, stream);
+        if (result == hipSuccess)
+            result = hipStreamWaitEvent(s->side_stream, s->side_fork, 0);
+        if (result != hipSuccess)
+            return result;
+        select(s->side_stream);
+        result = hipEventRecord(s->cut_done, s->side_stream);
+        launch_windows<DTYPE>(s, a, s->side_stream);
+        const hipError_t joins = hipEventRecord(s->side_join, s->side_stream);
+        const hipError_t waits = launch_bin_sums<DTYPE>(s, a, windows, want_filters, s->cut_done, stream);
+        const hipError_t joined = hipStreamWaitEvent(stream, s->side_join, 0);
+        return result != hipSuccess ? result : joins != hipSuccess ? joins : waits != hipSuccess ? waits : joined;
+    }
+    select(stream);
+    list_rows();
     if (windows)
-    {
-        WindowArgs w = s->windows;
-        w.a = a;
-        w.windows_are_selects = 1u;
-        hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
-        hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
-    }
-    if (sums)
-    {
-        BinArgs g = s->bins;
-        g.a = a;
-        g.windows_are_selects = windows ? 1u : 0u;
-        g.want_filters = want_filters ? 1u : 0u;
-        hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
-        hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
-        hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
-        if (a.rows <= kRoomyRows)
-            launch_bin_walks<DTYPE, true>(g, stream);
-        else
-            launch_bin_walks<DTYPE, false>(g, stream);
-    }
+        launch_windows<DTYPE>(s, a, stream);
+    return sums ? launch_bin_sums<DTYPE>(s, a, windows, want_filters, nullptr, stream) : hipSuccess;
 }
 
 // Enqueues the sampling path for `rows` rows.  want_filters: the rows without a window leave their filtered distributions
@@ -395,16 +433,9 @@ int launch_sampler(
     const bool sums = passes.full_order && (dtype == NCNN_MOE_LOGITS_F32 || want_filters) && vocab <= kBinMaxVocab;
     if (s->binned_sums != 0 && passes.select && !want_distribution && (windows || sums) && windows == passes.wide_select)
     {
-        if (dtype == NCNN_MOE_LOGITS_F32)
-        {
-            launch_select<NCNN_MOE_LOGITS_F32>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
-            launch_later_rows<NCNN_MOE_LOGITS_F32>(s, a, windows, sums, passes.side_by_side, want_filters, stream);
-        }
-        else
-        {
-            launch_select<NCNN_MOE_LOGITS_BF16>(batch_geometry, rows, stream, a, 0, s->scatter_segments != 0);
-            launch_later_rows<NCNN_MOE_LOGITS_BF16>(s, a, windows, sums, passes.side_by_side, want_filters, stream);
-        }
+        SAMPLER_HIP_CHECK(s, dtype == NCNN_MOE_LOGITS_F32
+                                 ? launch_unordered<NCNN_MOE_LOGITS_F32>(s, a, batch_geometry, windows, sums, passes.side_by_side, want_filters, stream)
+                                 : launch_unordered<NCNN_MOE_LOGITS_BF16>(s, a, batch_geometry, windows, sums, passes.side_by_side, want_filters, stream));
         if (passes.full_order)
         {
             if (dtype == NCNN_MOE_LOGITS_F32)
