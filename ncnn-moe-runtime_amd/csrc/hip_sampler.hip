@@ -439,7 +439,10 @@ int launch_sampler(
         if (passes.full_order)
         {
             if (dtype == NCNN_MOE_LOGITS_F32)
-                hipLaunchKernelGGL(sort_and_replay_kernel, dim3(rows), dim3(kSortThreads), 0, stream, a);
+            {
+                hipLaunchKernelGGL((general_sort_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kSortThreads), 0, stream, a);
+                hipLaunchKernelGGL((general_replay_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kReplayThreads), 0, stream, a);
+            }
             else
                 hipLaunchKernelGGL(bf16_counting_replay_kernel, dim3(rows), dim3(kSortThreads), 0, stream, a);
         }

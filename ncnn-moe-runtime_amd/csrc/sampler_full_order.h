@@ -314,10 +314,14 @@ __device__ __forceinline__ float load_logit<NCNN_MOE_LOGITS_BF16>(const void* ro
 // sort_indices[1] (needed only when the whole filtered distribution is exported); sampling sorts the
 // keys alone and recovers the one index it needs from the logits afterwards.
 template <int DTYPE, bool PAIRS>
-__device__ __forceinline__ void sort_whole_row(const SamplerArgs& a, uint32_t row, int tid)
+__global__ __launch_bounds__(kSortThreads) void general_sort_kernel(SamplerArgs a)
 {
     constexpr int kPasses = DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2;
     constexpr int kFirstDigit = DTYPE == NCNN_MOE_LOGITS_F32 ? 0 : 2;
+    const uint32_t row = blockIdx.x;
+    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
+        return;
+    const int tid = threadIdx.x;
     const int lane = tid & (kWaveSize - 1);
     const int wave = tid >> 6;
     const uint32_t n = a.vocab;
@@ -533,15 +537,6 @@ __device__ __forceinline__ void sort_whole_row(const SamplerArgs& a, uint32_t ro
         __threadfence_block();
         __syncthreads();
     }
-}
-
-template <int DTYPE, bool PAIRS>
-__global__ __launch_bounds__(kSortThreads) void general_sort_kernel(SamplerArgs a)
-{
-    const uint32_t row = blockIdx.x;
-    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
-        return;
-    sort_whole_row<DTYPE, PAIRS>(a, row, threadIdx.x);
 }
 
 // ---- the same sort with a row spread over several workgroups.  A batch rarely holds more full-order
@@ -1591,8 +1586,12 @@ __device__ __forceinline__ void replay_row(
 }
 
 template <int DTYPE, bool RUNS>
-__device__ __forceinline__ void replay_sorted_row(const SamplerArgs& a, uint32_t row, int tid)
+__global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerArgs a)
 {
+    const uint32_t row = blockIdx.x;
+    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
+        return;
+    const int tid = threadIdx.x;
     NCNN_MOE_STAMP(blockIdx.x, 15, 0);
     const ncnn_moe_sample_params p = a.params[row];
     const uint32_t* keys = a.sort_keys[1] + row * a.sort_stride;
@@ -1664,29 +1663,6 @@ __device__ __forceinline__ void replay_sorted_row(const SamplerArgs& a, uint32_t
         terms0 = terms;
     }
     replay_row<DTYPE, RUNS>(a, row, p, keys, run_ends, run_total_of_row, terms0, tid);
-}
-
-template <int DTYPE, bool RUNS>
-__global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerArgs a)
-{
-    const uint32_t row = blockIdx.x;
-    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
-        return;
-    replay_sorted_row<DTYPE, RUNS>(a, row, threadIdx.x);
-}
-
-// Sort and replay of an fp32 row that the window kernels and the binned sums have left, in ONE kernel: hardly any row is
-// left, and a launch that finds none costs some 2 us all the same (33 x 100,003, windows of 200: 53.1 us with two kernels,
-// 51.5 us so; 8 x 151,936 without a window 130.5 and 128.2 us).
-__global__ __launch_bounds__(kSortThreads) void sort_and_replay_kernel(SamplerArgs a)
-{
-    static_assert(kSortThreads == kReplayThreads, "the sort and the walk share a workgroup");
-    const uint32_t row = blockIdx.x;
-    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
-        return;
-    sort_whole_row<NCNN_MOE_LOGITS_F32, false>(a, row, threadIdx.x);
-    __syncthreads(); // (the sorted keys are in device memory, written by this workgroup)
-    replay_sorted_row<NCNN_MOE_LOGITS_F32, false>(a, row, threadIdx.x);
 }
 
 // bf16 full-order rows in ONE kernel: bf16_counting_sort_kernel and general_replay_kernel<BF16, runs> back to
