@@ -64,16 +64,20 @@ constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: t
 // more rows need the second workgroup.
 constexpr uint32_t kRoomyRows = kBinGrid / 2u / kMaxBinParts;
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
-// (the foreseen sums were off by a few 1e-5 at most; where a sum grows by single ulps a margin of 1e-4 lists 1,700 elements
-// at most on both sides of a power of two, so that they always fit)
+// Foreseen sums decide what is prepared, never what a sum is: a walk that finds its exact sum elsewhere fetches what it needs.
+// They are off by a few 1e-5 on most rows and by 4e-4 (normal logits) to 2e-3 (logits rounded to eighths) on some: a bin
+// that was listed or fetched enters the next forecast with a guess of its terms, and the next sum's terms round differently.
+// The margin for listing stays at 1e-4 all the same: where a sum grows by single ulps it lists 1,700 elements at most on
+// both sides of a power of two, so that they always fit, and a miss costs the one row a fetch.
 constexpr float kForeseenFirst = 1e-4f;          // relative error allowed for the sums foreseen from the bins' masses
 constexpr float kForeseenLater = 1e-4f;          // ... and from the steps of the sum before
+constexpr float kForeseenEnd = 4e-3f;            // ... before a bin is taken to lie behind the end of the sum and gets no steps
 static_assert(kBinQuads <= kWalkThreads && kBinListCap % kWalkThreads == 0 && kBinListCap <= 64 * kWaveSize, "the walk's thread and lane counts");
 
 // A bin as the walk sees it: kind (2 bits), biased exponent assumed for the running sum (8), elements in front of it (22).
 constexpr uint32_t kBinAdded = 0u;  // its elements' steps are added as one integer
 constexpr uint32_t kBinListed = 1u; // its elements are in the list
-constexpr uint32_t kBinBeyond = 2u; // behind the end of the sum
+constexpr uint32_t kBinBeyond = 2u; // behind the end of the sum, as far as that can be foreseen
 constexpr uint32_t kBinWanted = 3u; // its elements are needed and not in the list: fetched on demand
 
 __device__ __forceinline__ uint32_t packed_kind(uint32_t packed) { return packed >> 30; }
@@ -467,7 +471,7 @@ __device__ __forceinline__ float bin_top(uint32_t bin, uint32_t shift)
 //   front          elements in front of each bin; front[4] behind the last
 //   mass           about what the sum holds in front of each bin
 //   limit          elements that the sum runs over; cut_bin: no bin behind it takes part, and the sum may end inside it
-//   bound          the sum may end once it reaches this; error: relative error of the masses
+//   bound          the sum may end once it reaches this; error: relative error of the masses that lists bins
 struct BinPlan
 {
     uint32_t kind[4];
@@ -492,7 +496,7 @@ __device__ __forceinline__ BinPlan plan_bins(
         const float high = mass[j + 1] * (1.0f + error);
         plan.exponent[j] = (__float_as_uint(mass[j]) >> 23) & 0xffu;
         uint32_t kind = kBinAdded;
-        if (b < head_bins || front[j] >= limit || b > cut_bin || low > bound)
+        if (b < head_bins || front[j] >= limit || b > cut_bin || mass[j] * (1.0f - kForeseenEnd) > bound)
             kind = kBinBeyond;
         else if (count > 0u)
         {
@@ -501,7 +505,7 @@ __device__ __forceinline__ BinPlan plan_bins(
             const bool moves = bin_top(b, shift) * scale * 1.0001f >= __uint_as_float((max(__float_as_uint(low) >> 23, 25u) - 24u) << 23);
             const bool leaves = moves && ((__float_as_uint(low) ^ __float_as_uint(high)) >> 23) != 0u;
             plan.ends |= ends ? 1u << j : 0u;
-            if (ends || leaves || high >= bound)
+            if (ends || leaves || (high >= bound && low <= bound))
             {
                 kind = kBinListed;
                 plan.listed += count;
@@ -1354,6 +1358,7 @@ __device__ __forceinline__ void walk_bins(
     uint32_t stop = 0;
     float sum = start_sum;
     bool fetched = false;
+    bool unforeseen = false; // the sum goes on behind the end that was foreseen: every bin from here on is fetched
     const auto front_of = [&shared](uint32_t bin) { return packed_front(shared.packed[bin]); };
     for (uint32_t requests = 0;; ++requests)
     {
@@ -1400,6 +1405,14 @@ __device__ __forceinline__ void walk_bins(
                 shared.high = high;
                 finish(requests < kBinRequests ? 0u : 2u);
             };
+            // as many bins in front of `end` as can be fetched at a time
+            const auto ask_for_most = [&](uint32_t low, uint32_t end) {
+                const uint32_t front = front_of(low);
+                const uint32_t more = wave_partition_point(end - low, [&shared, low, front](uint32_t i) {
+                    return packed_front(shared.packed[low + i + 1u]) - front <= kBinExtraCap;
+                });
+                ask_for(low, low + max(more, 1u) - 1u);
+            };
             if (fetched)
             {
                 const uint32_t low = shared.low, high = shared.high, count = shared.extra_count;
@@ -1436,6 +1449,19 @@ __device__ __forceinline__ void walk_bins(
             }
             while (status == 3u)
             {
+                if (unforeseen)
+                {
+                    const uint32_t front = front_of(cur);
+                    if (cur > cut_bin || front >= limit || front == front_of(kBins))
+                        end_at(min(limit, front));
+                    else if (!moves_nothing(cur))
+                        ask_for_most(cur, min(cut_bin + 1u, kBins));
+                    else if (cut_bin < kBins && front_of(cut_bin) < limit)
+                        ask_for(cut_bin, cut_bin); // (the elements behind this one move nothing, but are counted up to the cut)
+                    else
+                        end_at(min(limit, front_of(kBins)));
+                    continue;
+                }
                 const uint32_t stop_word = shared.stop_bin[stop];
                 const uint32_t stop_here = stop_word & 0x7fffffffu;
                 if (cur < stop_here)
@@ -1476,18 +1502,14 @@ __device__ __forceinline__ void walk_bins(
                         cur = stop_here;
                     else
                     {
-                        // the sum has another exponent than was foreseen: as many bins as can be fetched at a time
-                        const uint32_t first = cur;
-                        const uint32_t more = wave_partition_point(stop_here - cur, [&shared, first, front](uint32_t i) {
-                            return packed_front(shared.packed[first + i + 1u]) - front <= kBinExtraCap;
-                        });
-                        ask_for(cur, cur + max(more, 1u) - 1u);
+                        // the sum has another exponent than was foreseen
+                        ask_for_most(cur, stop_here);
                     }
                 }
                 else if ((stop_word & 0x80000000u) != 0u)
                     ++stop; // (a new exponent from this bin on)
                 else if (stop_here == kBins || packed_kind(shared.packed[stop_here]) == kBinBeyond)
-                    end_at(min(limit, front_of(stop_here)));
+                    unforeseen = true; // (the end, unless there is more to run over and the exact sum has not met its stop condition)
                 else if (packed_kind(shared.packed[stop_here]) != kBinListed)
                 {
                     // terms half way: their roundings follow from the masks, unless the sum has another exponent than was

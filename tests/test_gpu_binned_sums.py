@@ -90,3 +90,39 @@ def test_walks_with_and_without_a_compute_unit_of_their_own(rows):
         again = sampler.sample(params, uniforms)
     parity_util.assert_results_match(gpu, cpu, "f32", "walks")
     assert gpu.tobytes() == again.tobytes()
+
+
+def _bf16_values(row):
+    return workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(row))
+
+
+# (scale of the normal logits, what they are rounded to, Top-P, seeds): rows on which the sums foreseen from the bins are off
+# by 1e-4 and more where the Top-P sum ends
+FORESEEN_ENDS = [
+    (2.5, "bf16", 0.98, (20,)),
+    (2.5, "", 0.9999, (0, 17, 19, 21, 28)),
+    (2.0, "eighths", 0.999, (0, 3, 9, 11)),
+    (2.0, "eighths", 1.0, (3, 6, 20, 22)),
+]
+
+
+@pytest.mark.parametrize("scale,rounded,top_p,seeds", FORESEEN_ENDS)
+def test_the_exact_sum_decides_where_the_top_p_sum_ends(scale, rounded, top_p, seeds):
+    """A sum that the bins' masses foresee as ended goes on as long as the exact one has not reached its bound."""
+    vocab = 151936
+    logits = np.stack([(np.random.default_rng(seed).standard_normal(vocab) * scale).astype(np.float32) for seed in seeds])
+    if rounded == "bf16":
+        logits = _bf16_values(logits)
+    elif rounded == "eighths":
+        logits = np.round(logits * 8) / 8
+    logits = np.ascontiguousarray(np.repeat(logits, 3, axis=0), dtype=np.float32)
+    rows = len(logits)
+    print("[case] foreseen ends, %g %s top_p %g" % (scale, rounded, top_p), flush=True)
+    params = hip_sampler.make_params(rows, 1.0, 0, top_p, 0.0)
+    uniforms = np.tile(np.array([0.25, 0.9, 1.0 - 2.0 ** -24], dtype=np.float32), len(seeds))
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+    assert gpu["kept_count"].tolist() == cpu["kept_count"].tolist()
+    parity_util.assert_results_match(gpu, cpu, "f32", "foreseen ends")
