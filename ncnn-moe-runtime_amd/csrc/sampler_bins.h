@@ -52,6 +52,12 @@ constexpr uint32_t kBinHead = 2048;              // elements of the sorted head 
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
 constexpr uint32_t kBinStops = 512;
+// Steps are added modulo 2^32, and a sum of them counts while it is below 2^24.  A bin whose terms may take 2^25 steps and
+// more is therefore not added but fetched, and a row whose bins together may take 2^32 is left to the full-order kernels.
+constexpr float kBinMostSteps = 33554432.0f;
+constexpr uint32_t kBinStepUnit = 16;            // log2 of the unit in which a row's steps are added up once more
+constexpr uint32_t kBinStopBits = 11;            // ... above the row's number of stops, in one word
+static_assert(kBins < 1u << kBinStopBits && (kBins << (26 - kBinStepUnit)) < 1u << (32 - kBinStopBits), "the steps of 2^25 and a little a bin fit beside the stops");
 constexpr int kMaskedDifference = 14;            // so many binades below the sum a bin's terms (within a 64th of each other) take 18 different steps at most
 constexpr uint32_t kBinRequests = 64;            // ... and how often per walk
 constexpr uint32_t kMaxBinParts = 16;
@@ -476,7 +482,7 @@ struct BinPlan
 {
     uint32_t kind[4];
     uint32_t exponent[4];
-    uint32_t ends;   // bit j: the sum ends inside bin j
+    uint32_t fetched; // bit j: bin j is fetched where it does not fit the list: the sum ends inside it, or its steps are too many to add
     uint32_t listed; // elements of the four bins that should be in the list
 };
 
@@ -486,7 +492,7 @@ __device__ __forceinline__ BinPlan plan_bins(
 {
     BinPlan plan;
     plan.listed = 0;
-    plan.ends = 0;
+    plan.fetched = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
     {
@@ -504,12 +510,18 @@ __device__ __forceinline__ BinPlan plan_bins(
             // (terms below half an ulp of the lower of the two sums move neither)
             const bool moves = bin_top(b, shift) * scale * 1.0001f >= __uint_as_float((max(__float_as_uint(low) >> 23, 25u) - 24u) << 23);
             const bool leaves = moves && ((__float_as_uint(low) ^ __float_as_uint(high)) >> 23) != 0u;
-            plan.ends |= ends ? 1u << j : 0u;
+            // (a step is a term in ulps of the sum, rounded; the quotient below is a few roundings off)
+            const float ulps_per_one = __uint_as_float((277u - min(max(plan.exponent[j], 24u), 250u)) << 23);
+            const float most_steps = static_cast<float>(count) * (bin_top(b, shift) * scale * 1.0001f * ulps_per_one + 1.0f);
+            const bool too_many = most_steps >= kBinMostSteps;
+            plan.fetched |= ends || too_many ? 1u << j : 0u;
             if (ends || leaves || (high >= bound && low <= bound))
             {
                 kind = kBinListed;
                 plan.listed += count;
             }
+            else if (too_many)
+                kind = kBinWanted;
         }
         plan.kind[j] = kind;
     }
@@ -529,7 +541,7 @@ __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&fro
         {
             position += front[j + 1] - front[j];
             if (position > kBinListCap)
-                plan.kind[j] = (plan.ends >> j & 1u) != 0u ? kBinWanted : kBinAdded;
+                plan.kind[j] = (plan.fetched >> j & 1u) != 0u ? kBinWanted : kBinAdded;
             else
                 end_of_list = position;
         }
@@ -1767,7 +1779,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             uint32_t kind[4];
             float own_mass[4];
             uint32_t stop_word[4];
-            uint32_t sums[3] = {0u, 0u, 0u}; // steps added, elements listed, stops
+            uint32_t sums[3] = {0u, 0u, 0u}; // steps added, elements listed, stops and (above them) steps in coarse units
             float masses = 0.0f;
             const float scale = 1.0f / (normalizer * renormalizer);
             const uint32_t tie_bits = holds_bins ? shared.ties[bin >> 5] >> (bin & 31u) : 0u;
@@ -1850,14 +1862,16 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                     : looks ? static_cast<float>(count) * bin_top(b, shift) * (1.0f - 0.4f / kBinsPerBinade) * scale : 0.0f;
                 sums[0] += own_steps[j];
                 sums[1] += behind && kind[j] == kBinListed ? count : 0u;
-                sums[2] += stop_word[j] != 0xffffffffu ? 1u : 0u;
+                sums[2] += (stop_word[j] != 0xffffffffu ? 1u : 0u) + (own_steps[j] >> kBinStepUnit << kBinStopBits);
                 masses += own_mass[j];
                 previous = packed[j];
             }
             uint32_t totals[3];
             bin_scan<kWalkWaves>(sums, totals, masses, shared.scan, tid);
-            stops = min(totals[2], kBinStops - 1u);
-            uint32_t prefix = sums[0], place = head_count + sums[1], stop = sums[2];
+            const uint32_t all_stops = totals[2] & ((1u << kBinStopBits) - 1u);
+            const bool overflows = kBinStops <= all_stops || (totals[2] >> kBinStopBits) + kBins >= 1u << (32 - kBinStepUnit);
+            stops = min(all_stops, kBinStops - 1u);
+            uint32_t prefix = sums[0], place = head_count + sums[1], stop = sums[2] & ((1u << kBinStopBits) - 1u);
             mass[0] = masses;
             if (holds_bins)
             {
@@ -1897,7 +1911,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             if (tid == 0)
             {
                 shared.stop_bin[stops] = kBins;
-                shared.status = totals[2] >= kBinStops ? 2u : 1u;
+                shared.status = overflows ? 2u : 1u;
             }
             // ---- the listed elements in order: a bin's elements lie side by side in the list
             __syncthreads();
@@ -1916,7 +1930,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         }
         if (shared.status == 2u)
         {
-            leave(kBinRowLeft); // (more places to look at than the walk keeps: left to the full-order kernels)
+            leave(kBinRowLeft); // (more places to look at, or more steps, than the walk holds: left to the full-order kernels)
             continue;
         }
         // ---- the sums.  `head_sum`: of the sum that the next launch goes on with; `next_*`: what it runs over

@@ -126,3 +126,25 @@ def test_the_exact_sum_decides_where_the_top_p_sum_ends(scale, rounded, top_p, s
         gpu = sampler.sample(params, uniforms)
     assert gpu["kept_count"].tolist() == cpu["kept_count"].tolist()
     parity_util.assert_results_match(gpu, cpu, "f32", "foreseen ends")
+
+
+@pytest.mark.parametrize("equal", [4097, 8192, 70000])
+def test_a_bin_of_more_than_two_to_the_32_steps(equal):
+    """A few tokens above thousands of equal ones: the equal ones' steps at the exponent of the sum in front of them add up to
+    2^32 and more, which must not be taken for the small number that is left of them modulo 2^32."""
+    heights = [np.float32(0.6931472), np.float32(0.0078125), np.float32(2.0), np.float32(8.0), np.float32(16.0)]
+    rows, vocab = 2 * len(heights), equal + 3
+    print("[case] flat rows of %d with spikes" % equal, flush=True)
+    logits = np.zeros((rows, vocab), dtype=np.float32)
+    for i, height in enumerate(heights):
+        logits[2 * i, vocab // 2] = height
+        logits[2 * i + 1, :3] = height
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["top_p"][1::4] = np.float32(0.7)
+    uniforms = np.linspace(0.05, 0.95, rows).astype(np.float32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+    assert gpu["kept_count"].tolist() == cpu["kept_count"].tolist()
+    parity_util.assert_results_match(gpu, cpu, "f32", "flat rows")
