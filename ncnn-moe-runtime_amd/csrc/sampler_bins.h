@@ -93,7 +93,8 @@ __device__ __forceinline__ uint32_t packed_front(uint32_t packed) { return packe
 enum BinRowState : uint32_t
 {
     kBinRowLeft = 0,  // not (or no longer) served here: finished, or left to the full-order kernels
-    kBinRowGoesOn = 1 // the next launch goes on with it
+    kBinRowGoesOn = 1, // the next launch goes on with it
+    kBinRowRejected = 2 // no finite logit, or +inf among them: the first walk reports it
 };
 
 // What the launches of a call keep of a row.  A launch reads what earlier ones wrote and writes other words (its own
@@ -342,22 +343,15 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
         if (grid.part == 0u && tid == 0)
         {
             BinRow& record = g.records[row];
-            record.state[0] = served ? kBinRowGoesOn : kBinRowLeft;
+            // A row is rejected (as the CPU sampler does) by the first walk and not here: beside the first launches the
+            // first select may still be marking the same row as pending, and the walks wait for it.
+            record.state[0] = served ? kBinRowGoesOn : rejected ? kBinRowRejected : kBinRowLeft;
             record.shift = shift;
             record.window = (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite;
             record.served = 0u;
             record.filtered = 0u;
             record.maximum = maximum;
             record.saw_nan = (flags & kScanSawNan) != 0u ? 1u : 0u;
-            if (rejected)
-            {
-                // no finite logit, or +inf among them: the CPU sampler rejects the row
-                uint32_t row_flags = counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH);
-                if ((flags & kScanSawNan) != 0u)
-                    row_flags |= NCNN_MOE_ROW_FLAG_HAS_NAN;
-                write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, static_cast<uint8_t>(row_flags));
-                a.row_state[row] = kRowDone;
-            }
         }
         if (served)
         {
@@ -656,7 +650,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         if (record.state[0] != kBinRowGoesOn)
         {
             if (grid.part == 0u && tid == 0)
-                record.state[1] = kBinRowLeft;
+                record.state[1] = record.state[0];
             continue;
         }
         const uint32_t shift = record.shift;
@@ -1664,8 +1658,18 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             if (WALK < 2 && grid.part == 0u && tid == 0)
                 record.state[WALK + 2] = state;
         };
-        if (same_in_all(record.state[WALK + 1]) != kBinRowGoesOn)
+        const auto result_flags = [&](const ncnn_moe_sample_params& p) {
+            return static_cast<uint8_t>((counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
+                                        (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u));
+        };
+        const uint32_t state = same_in_all(record.state[WALK + 1]);
+        if (state != kBinRowGoesOn)
         {
+            if (WALK == 0 && state == kBinRowRejected && grid.part == 0u && tid == 0)
+            {
+                write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, result_flags(a.params[row]));
+                a.row_state[row] = kRowDone;
+            }
             leave(kBinRowLeft);
             continue;
         }
@@ -2104,10 +2108,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                     if (tid == 0)
                     {
                         const ncnn_moe_sample_params p = a.params[row];
-                        const uint32_t flags = (counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
-                            (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u);
                         const float term = shared.terms[at];
-                        write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, static_cast<uint8_t>(flags));
+                        write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, result_flags(p));
                         a.row_state[row] = kRowDone;
                         record.served = 1u;
                     }

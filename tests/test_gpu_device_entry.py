@@ -149,3 +149,26 @@ def test_no_wide_windows_flag(dtype):
         broken_promise = _run(sampler, data, params, uniforms, flags | hip_sampler.PASSES_SIDE_BY_SIDE, stream)
         parity_util.assert_results_match(broken_promise, cpu, dtype, "wide windows without the wide select")
         assert (broken_promise["flags"][3::6] & hip_sampler.FLAG_GENERAL_PATH != 0).all()
+
+
+def test_rejected_rows_side_by_side():
+    """Rows without a finite logit, or with +inf, among the rows that the first select marks as pending on the second stream
+    while their sums begin on the caller's: rejected in every call, none left pending."""
+    print("[case] rejected rows side by side", flush=True)
+    rng = np.random.default_rng(78)
+    rows, vocab = 192, 20011
+    logits = (rng.standard_normal((rows, vocab)) * 2.0).astype(np.float32)
+    logits[0::6] = -np.inf
+    logits[1::6, vocab - 1] = np.inf
+    logits[2::12] = np.nan
+    params = hip_sampler.make_params(rows, 0.9, 0, 0.9, 0.0)
+    params["top_k"] = np.array([(0, 0, 0, 700, 300, 0, 0)[i % 7] for i in range(rows)], dtype=np.uint32)
+    uniforms = rng.random(rows).astype(np.float32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    stream = torch.cuda.Stream(device="cuda:0")
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        for _ in range(4):
+            beside = _run(sampler, logits, params, uniforms, hip_sampler.PASSES_FULL_ORDER | hip_sampler.PASSES_SIDE_BY_SIDE, stream)
+            parity_util.assert_results_match(beside, cpu, "f32", "rejected rows, device entry")
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "rejected rows, host entry")
