@@ -1166,6 +1166,9 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
         for (uint32_t k = 0; k < kLoads; ++k)
             raw[k] = reinterpret_cast<const uint4*>(terms)[min(at + k * kWalkThreads, vectors - 1u)];
     };
+    // (a wave makes room for its elements with one addition: one addition, minimum and maximum an element, all of them to
+    // the same three words, took 40 ns each, 60 us where the bins hold 1,500)
+    uint32_t least = 0xffffffffu, most = 0u;
     const auto take = [&](const uint4 (&raw)[kLoads], uint32_t at) {
 #pragma unroll
         for (uint32_t k = 0; k < kLoads; ++k)
@@ -1173,21 +1176,31 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
             const uint32_t bits[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
             const uint32_t nearest = min(min(top - bits[0], top - bits[1]), min(top - bits[2], top - bits[3]));
             const uint32_t v = at + k * kWalkThreads;
-            if (nearest >= width || v >= vectors)
+            const bool some = nearest < width && v < vectors;
+            if (__builtin_amdgcn_ballot_w64(some) == 0ull)
                 continue;
-#pragma unroll 1
+            uint32_t own = 0;
+#pragma unroll
+            for (uint32_t c = 0; c < 4u; ++c)
+                own += some && top - bits[c] < width ? 1u : 0u;
+            const uint32_t through = wave_prefix_sum_u32(own);
+            uint32_t place = 0;
+            if (lane_id() == kWaveSize - 1)
+                place = atomicAdd(&shared.extra_count, through);
+            place = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(place), kWaveSize - 1)) + through - own;
+#pragma unroll
             for (uint32_t c = 0; c < 4u; ++c)
             {
-                const uint32_t of_element = c == 0u ? bits[0] : c == 1u ? bits[1] : c == 2u ? bits[2] : bits[3];
-                if (top - of_element >= width)
-                    continue;
-                const uint32_t at_place = atomicAdd(&shared.extra_count, 1u);
-                atomicMin(&shared.extra_least, of_element);
-                atomicMax(&shared.extra_most, of_element);
-                if (at_place < kBinExtraCap)
+                if (some && top - bits[c] < width)
                 {
-                    shared.terms[kBinExtraPlace + at_place] = __uint_as_float(of_element);
-                    shared.tokens[kBinExtraPlace + at_place] = v * 4u + c - misalignment;
+                    least = min(least, bits[c]);
+                    most = max(most, bits[c]);
+                    if (place < kBinExtraCap)
+                    {
+                        shared.terms[kBinExtraPlace + place] = __uint_as_float(bits[c]);
+                        shared.tokens[kBinExtraPlace + place] = v * 4u + c - misalignment;
+                    }
+                    ++place;
                 }
             }
         }
@@ -1195,13 +1208,20 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     {
         uint4 raw[kLoads], more[kLoads];
         load(raw, tid);
-        for (uint32_t at = tid; at < vectors; at += 2u * kStride)
+        for (uint32_t at = tid; same_in_all(at) < vectors; at += 2u * kStride) // (whole waves stay in the loop)
         {
             load(more, at + kStride);
             take(raw, at);
             load(raw, at + 2u * kStride);
             take(more, at + kStride);
         }
+    }
+    least = ~wave_max_u32(~least);
+    most = wave_max_u32(most);
+    if (lane_id() == 0 && most != 0u)
+    {
+        atomicMin(&shared.extra_least, least);
+        atomicMax(&shared.extra_most, most);
     }
     __syncthreads();
     const uint32_t count = shared.extra_count;
