@@ -999,6 +999,9 @@ struct HeadScratch
 
 constexpr uint32_t kBinMasks = 128;      // bins with terms half way whose masks the walk keeps
 constexpr uint32_t kHasMasks = 0x8000u;
+constexpr uint32_t kStopExponent = 0x80000000u; // a stop: nothing but a new exponent from this bin on
+constexpr uint32_t kStopRun = 0x40000000u;      // ... the next bins are listed as well
+constexpr uint32_t kStopBin = 0x3fffffffu;
 
 struct BinWalkShared
 {
@@ -1006,11 +1009,11 @@ struct BinWalkShared
     alignas(16) uint32_t prefix[kBins + 4]; // steps added in front of each bin (modulo 2^32)
     alignas(16) float terms[kBinListCap + kBinExtraCap];
     alignas(16) uint32_t tokens[kBinListCap + kBinExtraCap];
-    uint16_t places[kBins];                 // where a listed bin's elements begin; kHasMasks + i: the bin's masks are the i-th
+    uint16_t places[kBins + 2];             // where a listed bin's elements begin (as many are listed in front of the others); kHasMasks + i: the bin's masks are the i-th
     uint32_t bin_masks[2 * kBinMasks];      // of bins with terms half way
     uint16_t mask_bin[kBinMasks];
     uint32_t mask_count;
-    uint32_t stop_bin[kBinStops];           // bins at which the walk looks closer, in order; bit 31: nothing but a new exponent
+    uint32_t stop_bin[kBinStops];           // bins at which the walk looks closer, in order (kStopBin, kStopExponent, kStopRun)
     uint32_t ties[2 * kBinWords];           // bins with terms half way; those of them that the masks do not tell
     BinScanScratch scan;
     HeadScratch head;
@@ -1377,7 +1380,7 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
 //             which lies in that bin (kBins: nowhere)
 template <int PHASE, bool ROOMY>
 __device__ __forceinline__ void walk_bins(
-    BinWalkShared& shared, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins,
+    BinWalkShared& shared, uint32_t stops, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins,
     uint32_t limit, uint32_t cut_bin, float cut_term, float start_sum, int mode, float bound, float divisor, float second_divisor, int tid)
 {
     uint32_t cur = head_bins;
@@ -1469,7 +1472,7 @@ __device__ __forceinline__ void walk_bins(
                     else if (take < count)
                         end_at(front + take);
                     cur = high + 1u;
-                    while ((shared.stop_bin[stop] & 0x7fffffffu) <= high)
+                    while ((shared.stop_bin[stop] & kStopBin) <= high)
                         ++stop;
                 }
             }
@@ -1489,7 +1492,7 @@ __device__ __forceinline__ void walk_bins(
                     continue;
                 }
                 const uint32_t stop_word = shared.stop_bin[stop];
-                const uint32_t stop_here = stop_word & 0x7fffffffu;
+                const uint32_t stop_here = stop_word & kStopBin;
                 if (cur < stop_here)
                 {
                     // bins that are one integer each
@@ -1532,7 +1535,7 @@ __device__ __forceinline__ void walk_bins(
                         ask_for_most(cur, stop_here);
                     }
                 }
-                else if ((stop_word & 0x80000000u) != 0u)
+                else if ((stop_word & kStopExponent) != 0u)
                     ++stop; // (a new exponent from this bin on)
                 else if (stop_here == kBins || packed_kind(shared.packed[stop_here]) == kBinBeyond)
                     unforeseen = true; // (the end, unless there is more to run over and the exact sum has not met its stop condition)
@@ -1588,16 +1591,29 @@ __device__ __forceinline__ void walk_bins(
                 {
                     const uint32_t place = shared.places[stop_here];
                     const uint32_t front = front_of(stop_here);
-                    const uint32_t count = front_of(stop_here + 1u) - front;
-                    const uint32_t take = share_of_sum(stop_here, stop_here, place, count);
+                    // Listed bins one behind the other lie side by side in the list and are added together: in the last binades
+                    // of a sum, and in short rows, 100 bins and more of a few elements each are listed, at 1 us a bin (64 rows
+                    // of 4,096 without a window: 261 us so, 72 us together).  They end where elements are not in the list.
+                    uint32_t behind = stop_here + 1u;
+                    if ((stop_word & kStopRun) != 0u)
+                    {
+                        const uint32_t first = behind + 1u;
+                        behind += wave_partition_point(kBins - behind, [&shared, first, place, front](uint32_t i) {
+                            return shared.places[first + i] - place == packed_front(shared.packed[first + i]) - front;
+                        });
+                    }
+                    const uint32_t count = front_of(behind) - front;
+                    const uint32_t take = share_of_sum(stop_here, behind - 1u, place, count);
                     const WaveSum result = wave_add_terms<PHASE>(shared.terms + place, take, sum, mode, bound, divisor, second_divisor);
                     sum = result.sum;
                     if (result.stopped)
                         stopped_at(front + result.index, place + result.index);
                     else if (take < count)
                         end_at(front + take);
-                    cur = stop_here + 1u;
+                    cur = behind;
                     ++stop;
+                    if ((stop_word & kStopRun) != 0u)
+                        stop += wave_partition_point(stops - stop, [&shared, stop, behind](uint32_t i) { return (shared.stop_bin[stop + i] & kStopBin) < behind; });
                 }
             }
         }
@@ -1863,7 +1879,13 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 front[j] = packed_front(packed[j]);
-            front[4] = holds_bins ? packed_front(shared.packed[bin + 4u]) : 0u;
+            uint4 next{0u, 0u, 0u, 0u};
+            if (holds_bins)
+                next = *reinterpret_cast<const uint4*>(shared.packed + bin + 4u);
+            front[4] = packed_front(next.x);
+            // (which of this thread's bins and the three behind them are listed)
+            const uint32_t kinds[7] = {packed_kind(words.x), packed_kind(words.y), packed_kind(words.z), packed_kind(words.w),
+                                       packed_kind(next.x), packed_kind(next.y), packed_kind(next.z)};
 #pragma unroll
             for (int j = 0; j < 4; ++j)
             {
@@ -1878,7 +1900,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 const bool ends = behind && kind[j] == kBinBeyond && (b == head_bins || packed_kind(previous) != kBinBeyond);
                 const bool looks = behind && (kind[j] == kBinListed || kind[j] == kBinWanted);
                 const bool changes = behind && kind[j] != kBinBeyond && packed_exponent(previous) != packed_exponent(packed[j]);
-                stop_word[j] = ends || looks ? b : changes ? (b | 0x80000000u) : 0xffffffffu;
+                const bool run = kinds[j] == kBinListed && kinds[j + 1] == kBinListed && kinds[j + 2] == kBinListed && kinds[j + 3] == kBinListed;
+                stop_word[j] = ends || looks ? (run ? b | kStopRun : b) : changes ? (b | kStopExponent) : 0xffffffffu;
                 masked[j] = masks_of(j, b, kind[j], packed[j], behind);
                 const bool adds = behind && (kind[j] == kBinAdded || masked[j] != 0u);
                 own_steps[j] = adds ? own_steps[j] : 0u;
@@ -1931,7 +1954,10 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                     mass[j + 1] = mass[j];
             }
             if (tid == static_cast<int>(kBinQuads) - 1)
+            {
                 shared.prefix[kBins] = prefix;
+                shared.places[kBins] = static_cast<uint16_t>(place);
+            }
             if (tid == 0)
             {
                 shared.stop_bin[stops] = kBins;
@@ -1974,7 +2000,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 mass[j] += sum;
             if (behind_head)
             {
-                walk_bins<0, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+                walk_bins<0, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
                 given_up = shared.status == 2u;
                 sum = same_in_all(shared.sum);
             }
@@ -2042,7 +2068,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         }
         if constexpr (WALK == 1)
         {
-            walk_bins<1, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
+            walk_bins<1, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
                          normalizer, 1.0f, tid);
             const bool stopped = shared.stopped != 0u;
             // (a sum that no stop condition ends runs to the window's end, or to the Min-P cut, which no bin may hold)
@@ -2110,7 +2136,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             }
             if constexpr (WALK == 2)
             {
-                walk_bins<2, ROOMY>(shared, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
+                walk_bins<2, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
                              normalizer, renormalizer, tid);
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);

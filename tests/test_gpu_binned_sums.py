@@ -148,3 +148,21 @@ def test_a_bin_of_more_than_two_to_the_32_steps(equal):
         gpu = sampler.sample(params, uniforms)
     assert gpu["kept_count"].tolist() == cpu["kept_count"].tolist()
     parity_util.assert_results_match(gpu, cpu, "f32", "flat rows")
+
+
+@pytest.mark.parametrize("rows,vocab,finite", [(64, 4096, 4096), (7, 16384, 16384), (5, 100003, 20000)])
+def test_runs_of_listed_bins(rows, vocab, finite):
+    """Short rows, and rows whose last binades are listed, have long runs of listed bins: the sums end behind them, and at
+    stops, windows and cuts inside them."""
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] runs of listed bins, %d x %d" % (rows, vocab), flush=True)
+    logits = np.full((rows, vocab), -np.inf, dtype=np.float32)
+    for row in logits:
+        row[rng.choice(vocab, finite, replace=False)] = rng.standard_normal(finite) * 2.5
+    uniforms = rng.random(rows, dtype=np.float32)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        for top_p, min_p, top_k in ((1.0, 0.0, 0), (0.9999, 0.0, 0), (0.95, 0.0, 0), (1.0, 2e-5, 0), (1.0, 3e-4, 0), (1.0, 0.0, finite // 2), (0.999, 1e-4, finite - 1)):
+            params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "top_p %g min_p %g top_k %d" % (top_p, min_p, top_k))
