@@ -60,6 +60,7 @@ constexpr uint32_t kBinStopBits = 11;            // ... above the row's number o
 static_assert(kBins < 1u << kBinStopBits && (kBins << (26 - kBinStepUnit)) < 1u << (32 - kBinStopBits), "the steps of 2^25 and a little a bin fit beside the stops");
 constexpr int kMaskedDifference = 14;            // so many binades below the sum a bin's terms (within a 64th of each other) take 18 different steps at most
 constexpr uint32_t kBinRequests = 64;            // ... and how often per walk
+constexpr uint32_t kBinComparedTies = 256;       // equal terms of a list that are told apart by comparing each with each
 constexpr uint32_t kMaxBinParts = 16;
 constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers in flight together
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
@@ -780,7 +781,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                 atomicMax(&head_bins_of_row, most);
         }
         __syncthreads();
-        const uint32_t head_bins = kBins - head_bins_of_row;
+        uint32_t head_bins = kBins - head_bins_of_row;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
@@ -788,15 +789,9 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                 head_count_of_row = front[j + 1];
         }
         __syncthreads();
-        const uint32_t head_count = head_count_of_row;
-        if (head_count == 0u || head_count > kBinListCap)
-        {
-            // thousands of equal terms at the row's top: left to the full-order kernels
-            if (grid.part == 0u && tid == 0)
-                record.state[1] = kBinRowLeft;
-            __syncthreads();
-            continue;
-        }
+        uint32_t head_count = head_count_of_row;
+        if (head_count > kBinListCap)
+            head_bins = head_count = 0u; // (thousands of equal terms at the row's top: no head, the walks begin by fetching them)
         const bool beyond = window > head_count && binned > head_count; // the sum goes on behind the head
         BinPlan plan = plan_bins(bin, front, mass, head_bins, beyond ? window : 0u, kBins, INFINITY, kForeseenFirst, shift, 1.0f);
         uint32_t listed[1] = {holds_bins ? plan.listed : 0u};
@@ -1028,6 +1023,7 @@ struct BinWalkShared
     uint32_t taken;      // elements added when the sum ran to its end
     uint32_t listed_end;
     int32_t token;
+    uint32_t least_key, most_key, matches; // see token_of_equal
 };
 
 constexpr uint32_t kBinExtraPlace = kBinListCap;
@@ -1625,11 +1621,153 @@ __device__ __forceinline__ void walk_bins(
     }
 }
 
-// The token of the element at terms[at] of a list [list_first, list_end) in order: elements of equal term are in no
-// particular order, and are told apart by their logits and indices.
+// The token of the rank-th (from 0) of the row's elements whose term is `term`, in the row's order: for a stretch of thousands
+// of equal terms, which no list holds.  Their logits are equal too, or a few neighbouring values: the logit is found by
+// bisection of the keys, then its rank-th index, each by a pass over the row's terms (8 us of one compute unit for 151,936).
+template <int DTYPE>
+__device__ __forceinline__ int32_t token_of_equal(
+    const SamplerArgs& a, uint32_t row, BinWalkShared& shared, const float* terms, uint32_t positions, uint32_t misalignment, float term, uint32_t rank, int tid)
+{
+    const char* pointer = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes;
+    const uint32_t wanted = __float_as_uint(term);
+    const uint32_t vectors = positions / 4u;
+    const int lane = tid & (kWaveSize - 1);
+    const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
+    const auto key_of = [&](uint32_t v, uint32_t c) { return descending_key(load_logit<DTYPE>(pointer, v * 4u + c - misalignment)); };
+    // which of a vector's four elements match: the term, and the key where [least, most] is given
+    const auto matching = [&](uint32_t v, bool by_key, uint32_t least, uint32_t most) {
+        const uint4 raw = reinterpret_cast<const uint4*>(terms)[v];
+        uint32_t hits = (raw.x == wanted ? 1u : 0u) | (raw.y == wanted ? 2u : 0u) | (raw.z == wanted ? 4u : 0u) | (raw.w == wanted ? 8u : 0u);
+        if (by_key)
+        {
+            for (uint32_t c = 0; c < 4u; ++c)
+            {
+                if ((hits >> c & 1u) != 0u)
+                {
+                    const uint32_t key = key_of(v, c);
+                    hits &= ~(key < least || key > most ? 1u << c : 0u);
+                }
+            }
+        }
+        return hits;
+    };
+    __syncthreads();
+    if (tid == 0)
+    {
+        shared.least_key = 0xffffffffu;
+        shared.most_key = 0u;
+    }
+    __syncthreads();
+    {
+        uint32_t least = 0xffffffffu, most = 0u;
+        for (uint32_t v = tid; v < vectors; v += kWalkThreads)
+        {
+            const uint32_t hits = matching(v, false, 0u, 0u);
+            for (uint32_t c = 0; c < 4u; ++c)
+            {
+                if ((hits >> c & 1u) != 0u)
+                {
+                    const uint32_t key = key_of(v, c);
+                    least = min(least, key);
+                    most = max(most, key);
+                }
+            }
+        }
+        least = ~wave_max_u32(~least);
+        most = wave_max_u32(most);
+        if (lane == 0)
+        {
+            atomicMin(&shared.least_key, least);
+            atomicMax(&shared.most_key, most);
+        }
+    }
+    __syncthreads();
+    uint32_t low = same_in_all(shared.least_key), high = same_in_all(shared.most_key);
+    const uint32_t first_key = low;
+    const bool by_key = low != high;
+    while (low < high)
+    {
+        const uint32_t middle = low + (high - low) / 2u;
+        __syncthreads();
+        if (tid == 0)
+            shared.matches = 0u;
+        __syncthreads();
+        uint32_t own = 0;
+        for (uint32_t v = tid; v < vectors; v += kWalkThreads)
+            own += static_cast<uint32_t>(__popc(matching(v, true, first_key, middle)));
+        const uint32_t of_wave = wave_prefix_sum_u32(own);
+        if (lane == kWaveSize - 1)
+            atomicAdd(&shared.matches, of_wave);
+        __syncthreads();
+        const uint32_t through = same_in_all(shared.matches);
+        if (through > rank)
+            high = middle;
+        else
+            low = middle + 1u;
+    }
+    // ---- the elements of that key by index: those of smaller keys are counted off with them
+    const uint32_t of_wave = ((vectors + kWalkWaves - 1u) / kWalkWaves + kWaveSize - 1u) / kWaveSize * kWaveSize;
+    const uint32_t first = min(vectors, wave * of_wave), last = min(vectors, first + of_wave);
+    uint32_t smaller = 0, own = 0;
+    for (uint32_t v = first + lane; v < last; v += kWaveSize)
+    {
+        own += static_cast<uint32_t>(__popc(matching(v, by_key, low, low)));
+        if (low != first_key)
+            smaller += static_cast<uint32_t>(__popc(matching(v, true, first_key, low - 1u)));
+    }
+    const uint32_t own_of_wave = wave_prefix_sum_u32(own), smaller_of_wave = wave_prefix_sum_u32(smaller);
+    __syncthreads();
+    if (lane == kWaveSize - 1)
+    {
+        shared.scan.u[0][wave] = own_of_wave;
+        shared.scan.u[1][wave] = smaller_of_wave;
+    }
+    __syncthreads();
+    uint32_t before = 0, below = 0;
+    for (uint32_t w = 0; w < static_cast<uint32_t>(kWalkWaves); ++w)
+    {
+        before += w < wave ? shared.scan.u[0][w] : 0u;
+        below += shared.scan.u[1][w];
+    }
+    const uint32_t index = rank - below;
+    const uint32_t in_wave = shared.scan.u[0][wave];
+    if (index >= before && index - before < in_wave)
+    {
+        uint32_t count = before;
+        for (uint32_t base = first; base < last; base += kWaveSize)
+        {
+            const uint32_t v = base + lane;
+            const uint32_t hits = v < last ? matching(v, by_key, low, low) : 0u;
+            const uint32_t held = static_cast<uint32_t>(__popc(hits));
+            const uint32_t through = wave_prefix_sum_u32(held);
+            uint32_t at = count + through - held;
+            for (uint32_t c = 0; c < 4u; ++c)
+            {
+                if ((hits >> c & 1u) != 0u)
+                {
+                    if (at == index)
+                        shared.token = static_cast<int32_t>(v * 4u + c - misalignment);
+                    ++at;
+                }
+            }
+            count += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), kWaveSize - 1));
+            if (count > index)
+                break;
+        }
+    }
+    __syncthreads();
+    const int32_t token = same_in_all(static_cast<uint32_t>(shared.token));
+    __syncthreads();
+    return token;
+}
+
+// The token of the element at terms[at] of a list [list_first, list_end) in order, which holds all elements of its term: those
+// are in no particular order, and are told apart by their logits and indices, each against each while they are few (2,000
+// of them took 500 us so).
 template <int DTYPE>
 __device__ __forceinline__ int32_t token_of_listed(
-    const SamplerArgs& a, uint32_t row, BinWalkShared& shared, const uint32_t* tokens, uint32_t at, uint32_t list_first, uint32_t list_end, int tid)
+    const SamplerArgs& a, uint32_t row, BinWalkShared& shared, const float* row_terms, uint32_t positions, uint32_t misalignment, const uint32_t* tokens,
+    uint32_t at, uint32_t list_first, uint32_t list_end, int tid)
 {
     const float term = shared.terms[at];
     const float* terms = shared.terms;
@@ -1637,27 +1775,23 @@ __device__ __forceinline__ int32_t token_of_listed(
     const uint32_t high = at + 1u + wave_partition_point(list_end - at - 1u, [terms, at, term](uint32_t i) { return terms[at + 1u + i] >= term; });
     if (high - low == 1u)
         return static_cast<int32_t>(tokens[at]);
+    if (high - low > kBinComparedTies)
+        return token_of_equal<DTYPE>(a, row, shared, row_terms, positions, misalignment, same_in_all(term), same_in_all(at - low), tid);
     const char* pointer = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes;
-    // their keys, where the bins' words were
-    uint32_t* const keys = shared.packed;
-    const bool keys_fit = high - low <= 2u * kBins;
-    static_assert(offsetof(BinWalkShared, prefix) == sizeof(uint32_t) * (kBins + 4), "packed and prefix lie one behind the other");
-    const auto key_of = [&](uint32_t i) { return descending_key(load_logit<DTYPE>(pointer, tokens[i])); };
+    uint32_t* const keys = shared.packed; // (where the bins' words were)
+    static_assert(kBinComparedTies <= kBins, "the keys fit");
     __syncthreads();
-    if (keys_fit)
-    {
-        for (uint32_t i = low + tid; i < high; i += kWalkThreads)
-            keys[i - low] = key_of(i);
-    }
+    for (uint32_t i = low + tid; i < high; i += kWalkThreads)
+        keys[i - low] = descending_key(load_logit<DTYPE>(pointer, tokens[i]));
     __syncthreads();
     for (uint32_t i = low + tid; i < high; i += kWalkThreads)
     {
         const uint32_t token = tokens[i];
-        const uint32_t key = keys_fit ? keys[i - low] : key_of(i);
+        const uint32_t key = keys[i - low];
         uint32_t rank = 0;
         for (uint32_t j = low; j < high; ++j)
         {
-            const uint32_t other = keys_fit ? keys[j - low] : key_of(j);
+            const uint32_t other = keys[j - low];
             rank += other < key || (other == key && tokens[j] < token) ? 1u : 0u;
         }
         if (rank == at - low)
@@ -2093,20 +2227,27 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             // the last element kept: in the head, where the Top-P sum stopped, or (no stop, no cut, no window) the last
             // finite one; a row whose last element lies elsewhere gets no filter
             const bool in_head = kept <= head_count;
-            const uint32_t last = in_head ? kept - 1u : WALK == 1 && shared.stopped != 0u ? same_in_all(shared.stop_at) : 0xffffffffu;
+            const bool stopped_behind = !in_head && WALK == 1 && shared.stopped != 0u;
+            const uint32_t last = in_head ? kept - 1u : stopped_behind ? same_in_all(shared.stop_at) : 0xffffffffu;
+            const bool in_equal = stopped_behind && last == 0xffffffffu; // ... among thousands of equal terms
             const bool everything = !in_head && kept == window && (WALK == 0 || shared.stopped == 0u) && min_p == 0.0f &&
                 (a.params[row].top_k == 0u || a.params[row].top_k >= a.vocab);
             uint32_t filter_key = kLastFiniteKey, filter_token = a.vocab;
-            if (last != 0xffffffffu)
+            if (last != 0xffffffffu || in_equal)
             {
                 const bool extra = WALK == 1 && last >= kBinExtraPlace;
                 const uint32_t first_of_list = extra ? kBinExtraPlace : WALK == 1 && !in_head ? head_count : 0u;
                 const uint32_t end_of_list = extra ? kBinExtraPlace + same_in_all(shared.extra_count) : WALK == 1 && !in_head ? listed : head_count;
-                const int32_t token = token_of_listed<DTYPE>(a, row, shared, WALK == 1 && in_head ? sorted_tokens_out : shared.tokens, last, first_of_list, end_of_list, tid);
+                int32_t token;
+                if (WALK == 1 && in_equal)
+                    token = token_of_equal<DTYPE>(a, row, shared, row_terms, positions, s.misalignment, __uint_as_float(same_in_all(shared.extra_least)),
+                                                  kept - 1u - packed_front(same_in_all(shared.packed[shared.low])), tid);
+                else
+                    token = token_of_listed<DTYPE>(a, row, shared, row_terms, positions, s.misalignment, WALK == 1 && in_head ? sorted_tokens_out : shared.tokens, last, first_of_list, end_of_list, tid);
                 filter_token = static_cast<uint32_t>(token);
                 filter_key = descending_key(load_logit<DTYPE>(static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes, filter_token));
             }
-            if (tid == 0 && (last != 0xffffffffu || everything))
+            if (tid == 0 && (last != 0xffffffffu || in_equal || everything))
             {
                 record.normalizer = normalizer;
                 record.renormalizer = renormalizer;
@@ -2122,7 +2263,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         {
             uint32_t at = 0, first_of_list = 0, end_of_list = head_count;
             const uint32_t* tokens = WALK == 1 ? sorted_tokens_out : shared.tokens;
-            bool found = kept == 1u;
+            bool found = kept == 1u && head_count != 0u;
             if (WALK < 2 && !found)
             {
                 if (WALK == 1)
@@ -2140,7 +2281,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                              normalizer, renormalizer, tid);
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);
-                if (shared.status != 1u || shared.stopped == 0u || at == 0xffffffffu)
+                if (shared.status != 1u || shared.stopped == 0u)
                     continue;
                 found = true;
                 first_of_list = at >= kBinExtraPlace ? kBinExtraPlace : head_count;
@@ -2150,11 +2291,22 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             {
                 if (grid.part == 0u)
                 {
-                    const int32_t token = token_of_listed<DTYPE>(a, row, shared, tokens, at, first_of_list, end_of_list, tid);
+                    int32_t token;
+                    float term;
+                    if (WALK == 2 && at == 0xffffffffu) // (among thousands of equal terms)
+                    {
+                        term = __uint_as_float(same_in_all(shared.extra_least));
+                        token = token_of_equal<DTYPE>(a, row, shared, row_terms, positions, s.misalignment, term,
+                                                      same_in_all(shared.stop_rank) - packed_front(same_in_all(shared.packed[shared.low])), tid);
+                    }
+                    else
+                    {
+                        token = token_of_listed<DTYPE>(a, row, shared, row_terms, positions, s.misalignment, tokens, at, first_of_list, end_of_list, tid);
+                        term = shared.terms[at];
+                    }
                     if (tid == 0)
                     {
                         const ncnn_moe_sample_params p = a.params[row];
-                        const float term = shared.terms[at];
                         write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, result_flags(p));
                         a.row_state[row] = kRowDone;
                         record.served = 1u;

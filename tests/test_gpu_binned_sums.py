@@ -166,3 +166,25 @@ def test_runs_of_listed_bins(rows, vocab, finite):
             params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
             cpu = parity_util.run_oracle(logits, params, uniforms)
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "top_p %g min_p %g top_k %d" % (top_p, min_p, top_k))
+
+
+@pytest.mark.parametrize("vocab", [4200, 40003, 151936])
+@pytest.mark.parametrize("kind", ["halves", "eighths", "equal", "two values", "equal terms of several logits"])
+def test_thousands_of_equal_terms(kind, vocab):
+    """Draws, Top-P ends, windows and cuts among thousands of equal terms, at the top of the row and behind it: the token is the
+    one of that rank in the row's order, and no row is left to the sort."""
+    rng = np.random.default_rng(vocab)
+    rows = 10
+    print("[case] equal terms, %s x %d" % (kind, vocab), flush=True)
+    base = rng.standard_normal((rows, vocab))
+    logits = {"halves": np.round(base * 4) / 2, "eighths": np.round(base * 16) / 8, "equal": np.full((rows, vocab), 0.5),
+              "two values": (base > 0.5) * 1.5, "equal terms of several logits": rng.integers(0, 6, (rows, vocab)) * 1e-9 + (base > 1.0)}[kind].astype(np.float32)
+    uniforms = np.linspace(0.0, 0.97, rows).astype(np.float32)  # (a draw that no partial sum exceeds is the sort's)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        for top_p, min_p, top_k in ((0.95, 0.0, 0), (1.0, 0.0, 0), (1.0, 0.01, 0), (0.5, 0.0, vocab // 2), (1e-6, 0.0, 0)):
+            params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "%s top_p %g min_p %g top_k %d" % (kind, top_p, min_p, top_k))
+            assert sampler.binned_rows(rows).tolist() == [1] * rows, (top_p, min_p, top_k)
