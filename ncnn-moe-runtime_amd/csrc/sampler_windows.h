@@ -7,8 +7,9 @@
 //                       m r - 5.5 r sqrt(m) = K.  Every workgroup of the row works the bound out for itself.
 //   window_finish       one workgroup per row puts the candidates in order (value descending, index ascending) and walks
 //                       the window's first K: the three sums with sum_head of sampler_bins.h.
-// A row whose candidates are fewer than its window (the sample misled, or few logits are finite) or more than a list
-// holds (thousands of ties) stays pending for the full-order kernels.
+// A row of fewer finite logits than its window has all of them as candidates and ends there.  A row whose candidates are fewer
+// than its window because the sample misled, or more than a list holds (thousands of ties), stays pending for the
+// full-order kernels.
 //
 // Bound: the stream at many rows (the row is read once and a part in 24 a second time), the chain sample - stream - order - sums
 // at few.  The one-workgroup-per-row select it stands in for took 65 to 115 us at any number of rows.
@@ -23,6 +24,8 @@ constexpr uint32_t kWindowListCap = 4096;        // candidates of a row
 constexpr uint32_t kWindowSampleRatio = 24;      // logits of the row per logit of the sample aimed at ...
 constexpr uint32_t kWindowSampleVectors = 4;     // ... within so many vectors a thread
 constexpr uint32_t kWindowMaxVocab = 1u << 19;   // beyond it a window of 1024 may not fit the list
+constexpr uint32_t kWindowSawNan = 1u;
+constexpr uint32_t kWindowHasAll = 2u;           // every finite logit is a candidate
 constexpr uint32_t kWindowBins = 4096;           // of the sample's histogram: the upper twelve bits of a key
 
 struct WindowArgs
@@ -30,7 +33,7 @@ struct WindowArgs
     SamplerArgs a;
     const uint32_t* list;   // the rows served: [0] their number, then the rows
     uint32_t* counts;       // [rows] candidates; zero when a launch begins (window_finish returns them to zero)
-    uint32_t* flags;        // [rows] NaN seen; the same
+    uint32_t* flags;        // [rows] kWindowSawNan, kWindowHasAll; the same
     uint32_t* keys;         // [rows][kWindowListCap]
     uint32_t* tokens;       // [rows][kWindowListCap]
     uint32_t windows_are_selects; // as in BinArgs
@@ -174,7 +177,9 @@ __device__ __forceinline__ void window_candidates(const WindowArgs& g, const Bin
             __syncthreads();
         }
         // (an infinite logit below everything is no candidate: the window counts finite logits)
-        const float bound = value_from_ascending_key(max(shared.bound, ascending_key(-3.402823466e38f)));
+        const uint32_t lowest = ascending_key(-3.402823466e38f);
+        const bool has_all = shared.bound <= lowest;
+        const float bound = value_from_ascending_key(max(shared.bound, lowest));
         // ---- the part's logits at or above it
         const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
         bool saw_nan = false;
@@ -234,8 +239,9 @@ __device__ __forceinline__ void window_candidates(const WindowArgs& g, const Bin
         if (tid == 0)
         {
             shared.base = count != 0u ? atomicAdd(&g.counts[row], count) : 0u;
-            if (shared.saw_nan != 0u)
-                atomicOr(&g.flags[row], 1u);
+            const uint32_t seen = (shared.saw_nan != 0u ? kWindowSawNan : 0u) | (has_all && grid.part == 0u ? kWindowHasAll : 0u);
+            if (seen != 0u)
+                atomicOr(&g.flags[row], seen);
         }
         __syncthreads();
         const uint32_t place = shared.base;
@@ -271,10 +277,10 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
     constexpr uint32_t kPerThread = kWindowListCap / kThreads;
     const SamplerArgs& a = g.a;
     const uint32_t count = same_in_all(g.counts[row]);
-    const bool saw_nan = same_in_all(g.flags[row]) != 0u;
+    const uint32_t seen = same_in_all(g.flags[row]);
     const ncnn_moe_sample_params p = a.params[row];
     const float uniform = same_in_all(a.uniforms[row]);
-    const uint32_t window = p.top_k == 0u || p.top_k >= a.vocab ? a.vocab : p.top_k;
+    const uint32_t wanted = p.top_k == 0u || p.top_k >= a.vocab ? a.vocab : p.top_k;
     if (tid < 32)
         shared.exp2_table[tid] = kExp2Table[tid];
     if (tid == 0)
@@ -288,10 +294,22 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
         g.counts[row] = 0u;
         g.flags[row] = 0u;
     }
-    // fewer candidates than the window, and logits below the bound: the sample misled.  (A row of few finite logits, or
-    // one shorter than its window, is left as well.)
-    if (count > kWindowListCap || count < window)
+    // (fewer candidates than the window, and logits below the bound: the sample misled)
+    if (count > kWindowListCap || (count < wanted && (seen & kWindowHasAll) == 0u))
         return;
+    uint8_t flags = counts_as_select(g.windows_are_selects, a.vocab, p) ? 0 : NCNN_MOE_ROW_FLAG_GENERAL_PATH;
+    if ((seen & kWindowSawNan) != 0u)
+        flags |= NCNN_MOE_ROW_FLAG_HAS_NAN;
+    const auto reject = [&]() {
+        if (tid == 0)
+        {
+            write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags);
+            a.row_state[row] = kRowDone;
+        }
+    };
+    if (count == 0u)
+        return reject();
+    const uint32_t window = min(wanted, count);
     uint32_t keys[kPerThread], tokens[kPerThread];
     uint32_t least = 0xffffffffu, most = 0u;
 #pragma unroll
@@ -315,20 +333,10 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
     __syncthreads();
     most = same_in_all(shared.most);
     least = same_in_all(shared.least);
-    uint8_t flags = counts_as_select(g.windows_are_selects, a.vocab, p) ? 0 : NCNN_MOE_ROW_FLAG_GENERAL_PATH;
-    if (saw_nan)
-        flags |= NCNN_MOE_ROW_FLAG_HAS_NAN;
     const float largest = value_from_ascending_key(most);
     const float maximum = largest / p.temperature;
     if (!is_finite_f32(largest))
-    {
-        if (tid == 0)
-        {
-            write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags);
-            a.row_state[row] = kRowDone;
-        }
-        return;
-    }
+        return reject();
     if (!is_finite_f32(maximum))
         return;
     // ---- in order: about where a candidate belongs by its value, then against those that belong in the same place
