@@ -33,6 +33,8 @@ int ncnn_moe_hip_sampler_debug_chunk_steps(ncnn_moe_hip_sampler* sampler, int en
  * first `rows` rows, 1 for a row that was finished that way the last time it was given to it. */
 int ncnn_moe_hip_sampler_debug_binned_sums(ncnn_moe_hip_sampler* sampler, int enabled);
 int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32_t* served, uint32_t rows);
+/* Which of the handle's first `rows` rows the binned sums left the filtered distribution of in the last verification step. */
+int ncnn_moe_hip_sampler_debug_filtered_rows(ncnn_moe_hip_sampler* sampler, uint32_t* filtered, uint32_t rows);
 /* spread_sort (on by default): the radix sort of a long full-order row runs on several workgroups; off,
  * every row is sorted by one workgroup. */
 int ncnn_moe_hip_sampler_debug_spread_sort(ncnn_moe_hip_sampler* sampler, int enabled);

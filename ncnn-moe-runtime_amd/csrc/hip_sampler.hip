@@ -1414,6 +1414,20 @@ int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* s, uint32_t* se
     return NCNN_MOE_SAMPLER_SUCCESS;
 }
 
+// Which of the handle's first `rows` rows the binned sums left the filtered distribution of in the last verification step.
+int ncnn_moe_hip_sampler_debug_filtered_rows(ncnn_moe_hip_sampler* s, uint32_t* filtered, uint32_t rows)
+{
+    if (s == nullptr || filtered == nullptr || rows > s->max_rows)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
+    SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+    std::vector<BinRow> records(rows);
+    SAMPLER_HIP_CHECK(s, hipMemcpy(records.data(), s->bins.records, rows * sizeof(BinRow), hipMemcpyDeviceToHost));
+    for (uint32_t row = 0; row < rows; ++row)
+        filtered[row] = records[row].filtered;
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
 int ncnn_moe_hip_sampler_debug_spread_sort(ncnn_moe_hip_sampler* s, int enabled)
 {
     if (s == nullptr)

@@ -120,11 +120,13 @@ struct BinRow
     uint32_t kept;
     uint32_t served;        // the row was finished here
     // the filtered distribution, where BinArgs::want_filters asks for it: probability((exp(logit/T - maximum) / normalizer)
-    // / renormalizer) of the elements kept, which are those up to filter_key, filter_token in the row's order
+    // / renormalizer) of the elements kept, which are those up to filter_key, filter_token in the row's order whose term is
+    // least_term or more
     uint32_t filtered;
     float maximum;
     uint32_t filter_key;    // descending key
     uint32_t filter_token;
+    float least_term;
 };
 
 struct BinArgs
@@ -2224,14 +2226,16 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         }
         if (WALK < 2 && g.want_filters != 0u && top_p_done && grid.part == 0u)
         {
-            // the last element kept: in the head, where the Top-P sum stopped, or (no stop, no cut, no window) the last
-            // finite one; a row whose last element lies elsewhere gets no filter
+            // the last element kept: in the head, where the Top-P sum stopped, or (no stop, no window) the last finite one, or
+            // the last whose term the Min-P cut keeps; a row whose last element lies elsewhere gets no filter
             const bool in_head = kept <= head_count;
             const bool stopped_behind = !in_head && WALK == 1 && shared.stopped != 0u;
             const uint32_t last = in_head ? kept - 1u : stopped_behind ? same_in_all(shared.stop_at) : 0xffffffffu;
             const bool in_equal = stopped_behind && last == 0xffffffffu; // ... among thousands of equal terms
-            const bool everything = !in_head && kept == window && (WALK == 0 || shared.stopped == 0u) && min_p == 0.0f &&
-                (a.params[row].top_k == 0u || a.params[row].top_k >= a.vocab);
+            const bool unlimited = a.params[row].top_k == 0u || a.params[row].top_k >= a.vocab;
+            const bool runs_on = !in_head && !stopped_behind;
+            const bool by_cut = runs_on && WALK == 1 && cut_bin < kBins && (unlimited || kept < limit);
+            const bool everything = by_cut || (runs_on && kept == window && min_p == 0.0f && unlimited);
             uint32_t filter_key = kLastFiniteKey, filter_token = a.vocab;
             if (last != 0xffffffffu || in_equal)
             {
@@ -2254,6 +2258,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 record.kept = kept;
                 record.filter_key = filter_key;
                 record.filter_token = filter_token;
+                record.least_term = by_cut ? cut_term : 0.0f;
                 record.filtered = 1u;
             }
             __syncthreads();

@@ -488,7 +488,8 @@ __device__ __forceinline__ float filtered_probability(const void* row_pointer, u
     const uint32_t key = descending_key(value);
     if (key > filter.filter_key || (key == filter.filter_key && token > filter.filter_token))
         return 0.0f;
-    return (expf_libm(value / temperature - filter.maximum, exp2_table) / filter.normalizer) / filter.renormalizer;
+    const float term = expf_libm(value / temperature - filter.maximum, exp2_table);
+    return term < filter.least_term ? 0.0f : (term / filter.normalizer) / filter.renormalizer;
 }
 
 struct VerifyWalkShared

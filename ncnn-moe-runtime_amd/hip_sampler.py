@@ -73,6 +73,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_scatter_segments",
     "ncnn_moe_hip_sampler_debug_binned_sums",
     "ncnn_moe_hip_sampler_debug_binned_rows",
+    "ncnn_moe_hip_sampler_debug_filtered_rows",
     "ncnn_moe_hip_sampler_debug_spread_sort",
     "ncnn_moe_hip_sampler_debug_fused_bf16",
     "ncnn_moe_hip_sampler_debug_partial_sort",
@@ -126,6 +127,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_filtered_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_spread_sort.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_partial_sort.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_sort_lengths.argtypes = [vp, vp, ctypes.c_uint32]
@@ -349,6 +351,13 @@ class HipSampler:
         """Test hook: which of the handle's first `rows` rows the binned sums finished (1) the last time they were given them."""
         out = np.empty(rows, dtype=np.uint32)
         self._check(self._hooks(True).ncnn_moe_hip_sampler_debug_binned_rows(self._handle, out.ctypes.data, rows))
+        return out
+
+    def filtered_rows(self, rows):
+        """Test hook: which of the handle's first `rows` rows the binned sums left the filtered distribution of (1) in the last
+        verification step."""
+        out = np.empty(rows, dtype=np.uint32)
+        self._check(self._hooks(True).ncnn_moe_hip_sampler_debug_filtered_rows(self._handle, out.ctypes.data, rows))
         return out
 
     def spread_sort(self, enabled):

@@ -29,3 +29,23 @@ def test_steps_without_a_window_match_the_oracle(vocab, drafts, bf16):
             if trial == 5:
                 uniforms[1:] = np.float32(1.0) - np.float32(2.0 ** -24)
             speculative._compare(sampler, target, draft, proposed, uniforms, "%d drafts over %d, trial %d" % (drafts, vocab, trial), bf16=bf16, **options)
+
+
+@pytest.mark.parametrize("vocab,top_k,min_p", [(40961, 0, 0.02), (151936, 0, 0.001), (151936, 0, 2e-5), (40961, 30000, 0.02), (9000, 0, 1e-3)])
+def test_steps_whose_min_p_cut_lies_behind_the_head(vocab, top_k, min_p):
+    """The filtered distribution that a Min-P cut ends thousands of tokens down is known by the smallest term that it keeps: the
+    step is not run a second time with exported lists."""
+    rng = np.random.default_rng(vocab + top_k)
+    drafts = 3
+    with hip_sampler.HipSampler(2 * drafts + 1, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        for trial in range(4):
+            options = dict(temperature=1.0, top_p=1.0 if trial % 2 else 0.9999, min_p=min_p, top_k=top_k)
+            target = (rng.standard_normal((drafts + 1, vocab)) * 1.2).astype(np.float32)
+            draft = (target[:drafts] + (0.1 if trial < 3 else 2.0) * rng.standard_normal((drafts, vocab))).astype(np.float32)
+            proposed = speculative._propose(rng, draft, options)
+            uniforms = rng.random(drafts + 1, dtype=np.float32)
+            if trial >= 2:
+                uniforms[1] = np.float32(1.0) - np.float32(2.0 ** -24)
+            speculative._compare(sampler, target, draft, proposed, uniforms, "cut at %g over %d, trial %d" % (min_p, vocab, trial), **options)
+            assert sampler.filtered_rows(2 * drafts + 1).tolist() == [1] * (2 * drafts + 1)
