@@ -189,8 +189,13 @@ __device__ __forceinline__ float sequential_row_sums(const float* row_of_lane, u
 // scores leave no such threshold, the lowest ids among the equals are collected.
 // What bounds it: instructions, some 130 per token of 256 experts and 8 routes, where choosing one route per round by
 // wave-wide maxima took some 500.
+// Up to kRankedExperts experts are ranked against each other at once, by lane reads: the threshold and the trips through LDS
+// cost more there (one token of 8 experts and 2 routes: 6.2 to 6.6 us so, 5.9 to 6.2 ranked; 16 experts are ranked in
+// 6.4 us, 6.0 so).
 // Returns the sum of the selected scores in rank order (src/graph/expert_dispatcher.cpp:137-143); the calling lane's
 // route is `my_expert` with `my_rank` (none: a rank of top_k or more).
+constexpr uint32_t kRankedExperts = 8;
+
 template <int SLOTS>
 __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&score)[SLOTS], const float (&bias)[SLOTS], RouteScratch& scratch,
                                              int lane, uint32_t& my_expert, uint32_t& my_rank, float& my_score)
@@ -206,6 +211,23 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
         const uint32_t ordered = bits ^ (static_cast<uint32_t>(static_cast<int32_t>(bits) >> 31) | 0x80000000u);
         key[s] = static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts ? 0u : keyed != keyed ? 1u : ordered;
         largest = max(largest, key[s]);
+    }
+    if (SLOTS == 1 && r.experts <= kRankedExperts)
+    {
+        uint32_t rank = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < kRankedExperts; ++e) // (past the last expert: keys of 0, in front of none)
+        {
+            const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key[0]), static_cast<int>(e)));
+            rank += other > key[0] || (other == key[0] && e < static_cast<uint32_t>(lane)) ? 1u : 0u;
+        }
+        my_expert = static_cast<uint32_t>(lane);
+        my_rank = my_expert < r.experts ? rank : 0xffffffffu;
+        my_score = score[0];
+        float selected_sum = 0.0f;
+        for (uint32_t i = 0; i < top_k; ++i)
+            selected_sum += read_lane(my_score, __builtin_ctzll(__builtin_amdgcn_ballot_w64(my_rank == i)));
+        return selected_sum;
     }
     largest = wave_max_u32(largest);
     const auto count_from = [&](uint32_t least) {
@@ -536,7 +558,7 @@ __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterSh
         for (int w = 1; w < kWavesPerToken; ++w)
             maximum = fmaxf(maximum, shared.maximum[slot * kWavesPerToken + w]);
     }
-    // (the row is filled up to a multiple of 64 with zeros)
+    // (the row is filled up to a multiple of 64 with zeros; its sum takes it up to a multiple of 16)
     const uint32_t padded = (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize;
     const auto each_score = [&](auto score_of) {
 #pragma unroll
@@ -876,7 +898,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_select_kernel(RouterArg
         }
         else
         {
-            const float sum = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? sequential_row_sums(shared.scores[wave], (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize) : 1.0f;
+            const float sum = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? sequential_row_sums(shared.scores[wave], (r.experts + 15u) / 16u * 16u) : 1.0f;
             route_token<SLOTS, true>(r, shared.scores[wave], sum, shared.scratch[wave], token, lane);
         }
     }

@@ -35,3 +35,26 @@ def test_batches_match_the_oracle(tokens, experts, top_k):
                 assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
         logits[tokens - 1, experts - 1] = np.inf
         assert router.dispatch(logits, top_k)[0] == hip_router.STATUS_NON_FINITE_LOGIT
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 257, 4095, 4096])
+@pytest.mark.parametrize("experts,top_k", [(1, 1), (2, 1), (7, 3), (8, 2), (8, 8), (9, 9)])
+def test_few_experts_match_the_oracle(tokens, experts, top_k):
+    """Up to eight experts are ranked against each other, more go through a threshold: ties, equal rows, scores that vanish."""
+    rng = np.random.default_rng(tokens * 31 + experts)
+    logits = (rng.standard_normal((tokens, experts)) * 2).astype(np.float32)
+    logits[1::5] = np.round(logits[1::5])
+    logits[2::7] = np.float32(1.5)
+    logits[3::11, (experts + 1) // 2:] *= np.float32(6)
+    bias = (rng.standard_normal(experts) * 0.3).astype(np.float32)
+    print("[case] %d tokens, %d experts, top %d" % (tokens, experts, top_k), flush=True)
+    with contextlib.closing(hip_router.HipRouter(tokens, experts, top_k)) as router:
+        for score in (hip_router.SOFTMAX, hip_router.SIGMOID, hip_router.SQRT_SOFTPLUS):
+            for options in (dict(), dict(selection_bias=bias, routed_scaling_factor=2.5)):
+                status, offsets, routes = router.dispatch(logits, top_k, score_function=score, **options)
+                cpu_status, cpu_offsets, cpu_routes = oracle_lib.oracle_router_dispatch(logits, top_k, score_function=score, **options)
+                assert status == cpu_status == 0
+                assert np.array_equal(offsets, cpu_offsets)
+                for field in ("token_index", "rank"):
+                    assert np.array_equal(routes[field], cpu_routes[field]), field
+                assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
