@@ -13,9 +13,11 @@ pytestmark = pytest.mark.gpu
 MAX_ROWS, MAX_VOCAB = 300, 70000
 
 
-@pytest.fixture(scope="module")
-def sampler():
+@pytest.fixture(scope="module", params=["sorted", "as shipped"])
+def sampler(request):
+    """The testing build sorts the rows that the first select leaves; the shipped library serves them by windows and sums."""
     handle = hip_sampler.HipSampler(MAX_ROWS, MAX_VOCAB, testing=True)
+    handle.binned_sums(request.param == "as shipped")
     yield handle
     handle.close()
 
@@ -69,3 +71,48 @@ def test_random_batches(sampler, seed):
         sampler.scatter_segments(False)
     cpu = parity_util.run_oracle(logits, params, uniforms, stop_ids)
     parity_util.assert_results_match(gpu, cpu, "bf16" if bf16 else "f32", "fuzz seed %d" % seed)
+
+
+def _long_row(rng, vocab):
+    """Rows as a serving loop has them without a window: fp32, fp32 of bf16 values, coarser ones, masked ones, narrow ones."""
+    row = (rng.standard_normal(vocab) * rng.uniform(1.0, 4.0)).astype(np.float32)
+    kind = int(rng.integers(0, 9))
+    if kind in (1, 2):
+        row = workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(row))
+    elif kind == 3:
+        row = np.round(row * 8) / 8
+    elif kind == 4:
+        row = np.round(row * 2) / 2
+    elif kind == 5:
+        row[rng.random(vocab) < rng.choice([0.1, 0.9, 0.999])] = -np.inf
+    elif kind == 6:
+        row = row * np.float32(0.01) + np.float32(20.0)
+    elif kind == 7:
+        row[:] = np.float32(0.25)
+        row[rng.integers(0, vocab, 5)] = rng.choice(np.array([0.25, 0.9431472, 2.0, 12.0], dtype=np.float32))
+    elif kind == 8:
+        row[rng.integers(0, vocab, 20)] += np.float32(15.0)
+    return np.ascontiguousarray(row, dtype=np.float32)
+
+
+@pytest.mark.parametrize("seed", range(20))
+def test_random_batches_of_long_rows(seed):
+    rng = np.random.default_rng(70000 + seed)
+    rows = int(rng.choice([5, 16, 17, 40, 70]))
+    vocab = int(rng.choice([4099, 16385, 32000, 50257, 100003, 151936]))
+    bf16 = seed % 5 == 4
+    print("[case] long rows, seed %d: %d x %d %s" % (seed, rows, vocab, "bf16" if bf16 else "f32"), flush=True)
+    logits = np.stack([_long_row(rng, vocab) for _ in range(rows)])
+    params = hip_sampler.make_params(rows)
+    params["temperature"] = rng.choice(np.array([0.5, 1.0, 1.0, 1.3], dtype=np.float32), size=rows)
+    params["top_k"] = rng.choice(np.array([0, 0, 0, 0, 100, 1000, 1025, 30000], dtype=np.uint32), size=rows)
+    params["top_p"] = rng.choice(np.array([1.0, 1.0, 0.9999, 0.999, 0.98, 0.95, 0.5], dtype=np.float32), size=rows)
+    params["min_p"] = rng.choice(np.array([0.0, 0.0, 1e-5, 1e-3, 0.05], dtype=np.float32), size=rows)
+    uniforms = rng.choice([rng.random(rows), np.full(rows, 1.0 - 2.0 ** -24)], p=[0.9, 0.1]).astype(np.float32)
+    if bf16:
+        logits = workloads.float32_to_bf16_bits(logits)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, "bf16" if bf16 else "f32", "long rows, seed %d" % seed)

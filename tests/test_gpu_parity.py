@@ -14,9 +14,11 @@ def _announce(text):
     print("[case] " + text, flush=True)
 
 
-@pytest.fixture(scope="module")
-def small_sampler():
+@pytest.fixture(scope="module", params=["sorted", "as shipped"])
+def small_sampler(request):
+    """The testing build sorts the rows that the first select leaves; the shipped library serves them by windows and sums."""
     sampler = hip_sampler.HipSampler(64, 40000, testing=True)
+    sampler.binned_sums(request.param == "as shipped")
     yield sampler
     sampler.close()
 
