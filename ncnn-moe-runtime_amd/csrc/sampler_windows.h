@@ -24,6 +24,7 @@ constexpr uint32_t kWindowListCap = 4096;        // candidates of a row
 constexpr uint32_t kWindowSampleRatio = 24;      // logits of the row per logit of the sample aimed at ...
 constexpr uint32_t kWindowSampleVectors = 4;     // ... within so many vectors a thread
 constexpr uint32_t kWindowMaxVocab = 1u << 19;   // beyond it a window of 1024 may not fit the list
+constexpr uint32_t kWindowRankedTies = 256;      // neighbours in value that are ranked against each other; more are sorted
 constexpr uint32_t kWindowSawNan = 1u;
 constexpr uint32_t kWindowHasAll = 2u;           // every finite logit is a candidate
 constexpr uint32_t kWindowBins = 4096;           // of the sample's histogram: the upper twelve bits of a key
@@ -259,15 +260,49 @@ __device__ __forceinline__ void window_candidates(const WindowArgs& g, const Bin
 
 struct WindowFinishShared
 {
-    alignas(16) uint32_t keys[kWindowListCap];
+    alignas(16) uint32_t keys[kWindowListCap]; // (keys and tokens together: the pairs that sort_candidates sorts)
     alignas(16) uint32_t tokens[kWindowListCap];
     uint32_t counters[kWindowListCap];
     alignas(16) float terms[kSelectTopK];
     HeadScratch head;
     BinScanScratch scan;
-    uint32_t least, most;
+    uint32_t least, most, neighbours;
     uint64_t exp2_table[32];
 };
+
+// Puts `count` pairs (key in the upper 32 bits, complement of the token below) in descending order: bitonic, in LDS.  Rows of few
+// distinct values, or with one value far above the others, have thousands of candidates next to each other, and ranking those
+// against each other takes as the square of their number (33 x 100,003 logits in halves, a window of 200: 143 us so, 73 us
+// sorted; where they are few the ranks are faster, 52 against some 90 us).
+template <int WAVES>
+__device__ __forceinline__ void sort_candidates(uint64_t* pairs, uint32_t count, int tid)
+{
+    constexpr uint32_t kThreads = WAVES * kWaveSize;
+    uint32_t size = 1u;
+    while (size < count)
+        size *= 2u;
+    for (uint32_t i = count + tid; i < size; i += kThreads)
+        pairs[i] = 0u;
+    __syncthreads();
+    for (uint32_t length = 2u; length <= size; length *= 2u)
+    {
+        for (uint32_t distance = length / 2u; distance > 0u; distance /= 2u)
+        {
+            for (uint32_t i = tid; i < size / 2u; i += kThreads)
+            {
+                const uint32_t first = 2u * i - (i & (distance - 1u));
+                const uint32_t second = first + distance;
+                const uint64_t a = pairs[first], b = pairs[second];
+                if ((a < b) == ((first & length) == 0u) && a != b)
+                {
+                    pairs[first] = b;
+                    pairs[second] = a;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
 
 // One row's candidates to its result.  WAVES waves call it.
 template <int DTYPE, int WAVES>
@@ -287,6 +322,7 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
     {
         shared.least = 0xffffffffu;
         shared.most = 0u;
+        shared.neighbours = 0u;
     }
     __syncthreads(); // (every thread has read the counters)
     if (tid == 0)
@@ -353,7 +389,38 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
             turn[k] = atomicAdd(&shared.counters[fine[k]], 1u);
         }
     }
+    uint32_t neighbours = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPerThread; ++k)
+        neighbours = max(neighbours, turn[k]);
+    neighbours = wave_max_u32(neighbours);
+    if ((tid & (kWaveSize - 1)) == 0 && neighbours >= kWindowRankedTies)
+        atomicMax(&shared.neighbours, neighbours);
     __syncthreads();
+    const bool sorts = shared.neighbours != 0u;
+    if (sorts)
+    {
+        static_assert(offsetof(WindowFinishShared, tokens) == kWindowListCap * sizeof(uint32_t), "keys and tokens lie one behind the other");
+        uint64_t* const pairs = reinterpret_cast<uint64_t*>(shared.keys);
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            const uint32_t i = k * kThreads + tid;
+            if (i < count)
+                pairs[i] = (static_cast<uint64_t>(keys[k]) << 32) | (0xffffffffu - tokens[k]);
+        }
+        sort_candidates<WAVES>(pairs, count, tid);
+        // (from here on as after ranking: the thread holds some of the window's elements and their ranks)
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            const uint64_t pair = pairs[k * kThreads + tid];
+            keys[k] = static_cast<uint32_t>(pair >> 32);
+            tokens[k] = 0xffffffffu - static_cast<uint32_t>(pair);
+        }
+        __syncthreads();
+    }
+    else
     {
         uint32_t held[kPerThread];
         uint32_t total[1] = {0u};
@@ -380,7 +447,7 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
 #pragma unroll
     for (uint32_t k = 0; k < kPerThread; ++k)
     {
-        if (k * kThreads + tid < count)
+        if (!sorts && k * kThreads + tid < count)
         {
             const uint32_t at = shared.counters[fine[k]] + turn[k];
             shared.keys[at] = keys[k];
@@ -392,8 +459,8 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
 #pragma unroll
     for (uint32_t k = 0; k < kPerThread; ++k)
     {
-        rank[k] = 0u;
-        if (k * kThreads + tid < count)
+        rank[k] = k * kThreads + tid;
+        if (!sorts && k * kThreads + tid < count)
         {
             const uint32_t low = shared.counters[fine[k]];
             const uint32_t high = fine[k] + 1u < count ? shared.counters[fine[k] + 1u] : count;

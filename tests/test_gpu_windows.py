@@ -35,3 +35,26 @@ def test_windows_over_few_finite_logits(dtype, vocab):
     parity_util.assert_results_match(gpu, cpu, dtype, "few finite logits")
     assert gpu.tobytes() == again.tobytes()
     assert (gpu["flags"] & hip_sampler.FLAG_GENERAL_PATH == 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["halves", "sixteenths", "one far above", "all equal"])
+def test_windows_over_many_neighbours(kind, dtype):
+    """Hundreds and thousands of candidates of one value, or next to each other because another lies far above them."""
+    rng = np.random.default_rng(7)
+    rows, vocab = 12, 50021
+    print("[case] many neighbours, %s %s" % (kind, dtype), flush=True)
+    base = rng.standard_normal((rows, vocab)) * 2.5
+    logits = {"halves": np.round(base * 2) / 2, "sixteenths": np.round(base * 16) / 16, "one far above": base, "all equal": np.full((rows, vocab), 1.5)}[kind].astype(np.float32)
+    if kind == "one far above":
+        logits[np.arange(rows), rng.integers(0, vocab, rows)] = 1e5
+    if kind == "all equal":
+        logits[:, rng.choice(vocab, vocab - 3000, replace=False)] = -np.inf  # (more than 4,096 candidates go to the sort)
+    uniforms = rng.random(rows, dtype=np.float32)
+    data = workloads.float32_to_bf16_bits(logits) if dtype == "bf16" else logits
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(data)
+        for top_k, top_p in ((65, 1.0), (200, 0.95), (1000, 1.0), (1024, 0.9)):
+            params = hip_sampler.make_params(rows, 1.0, top_k, top_p, 0.0)
+            cpu = parity_util.run_oracle(data, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, dtype, "%s top_k %d" % (kind, top_k))
