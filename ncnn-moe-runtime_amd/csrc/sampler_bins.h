@@ -1627,7 +1627,7 @@ __device__ __forceinline__ void walk_bins(
 // of equal terms, which no list holds.  Their logits are equal too, or a few neighbouring values: the logit is found by
 // bisection of the keys, then its rank-th index, each by a pass over the row's terms (8 us of one compute unit for 151,936).
 template <int DTYPE>
-__device__ __forceinline__ int32_t token_of_equal(
+__device__ __noinline__ int32_t token_of_equal(
     const SamplerArgs& a, uint32_t row, BinWalkShared& shared, const float* terms, uint32_t positions, uint32_t misalignment, float term, uint32_t rank, int tid)
 {
     const char* pointer = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * LogitsVector<DTYPE>::kElementBytes;
