@@ -216,7 +216,7 @@ def bench_speculative_verify(args, hip_sampler):
                    "entry_point": "ncnn_moe_hip_sampler_speculative_verify (host operands, synchronous)"},
         "roofline": {"bound": "hbm", "achieved": bytes_per_step / seconds_per_step / 1e9, "peak": HBM_PEAK_BYTES_PER_S / 1e9,
                      "unit": "GB/s", "frac": bytes_per_step / seconds_per_step / HBM_PEAK_BYTES_PER_S, "traffic": None,
-                     "kernel": ("full-order kernels with exported distributions + speculative_verify_dense_kernel" if args.dense_verify
+                     "kernel": ("binned sums of every row + verify_residual, verify_steps and verify_draw kernels" if args.dense_verify
                                 else "scan_select_kernel + speculative_verify_kernel") + ", wall clock of the synchronous call",
                      "algorithmic_bytes_per_launch": bytes_per_step},
         "parity": {"steps_checked": 16, "step_mismatches": mismatches, "mean_accepted": accepted_total / 16.0},
@@ -303,7 +303,7 @@ def bench_router_dispatch(args):
                    "entry_point": "ncnn_moe_hip_router_dispatch_device (no host synchronisation inside the timed region)"},
         "roofline": {"bound": "hbm", "achieved": bytes_per_step / device_seconds_per_step / 1e9, "peak": HBM_PEAK_BYTES_PER_S / 1e9,
                      "unit": "GB/s", "frac": bytes_per_step / device_seconds_per_step / HBM_PEAK_BYTES_PER_S, "traffic": None,
-                     "kernel": "router_clear_kernel + router_select_kernel + router_group_kernel, device time per dispatch "
+                     "kernel": "router_select_kernel, or router_batch_kernel + router_group_kernel, device time per dispatch "
                                "between two events on the launch stream",
                      "algorithmic_bytes_per_launch": bytes_per_step, "device_us_per_step": device_seconds_per_step * 1e6},
         "parity": {"dispatches_checked": buffers, "dispatch_mismatches": mismatches},
@@ -872,7 +872,7 @@ def main():
               hip_sampler.GEOMETRY_SPLIT_ONE_CHUNK: "split_select_kernel (%d one-chunk workgroups per row)" % segments,
               hip_sampler.GEOMETRY_SPLIT_LOOPED: "scan_select_kernel (%d workgroups per row, %d chunks each)" % (segments, chunks)}[variant]
     if may_need_full_order:
-        kernel += " + the later passes for rows without a Top-K window of at most 64 (wide select, sort, replay)"
+        kernel += " + the later passes for rows without a Top-K window of at most 64 (window kernels, binned sums, sort, replay)"
     metric = METRICS.get(workload["name"], "sampled rows/sec + HBM GB/s (% peak), " + workload["name"])
     if not own_shape:
         metric += " [shape overridden: %d x %d %s]" % (rows, vocab, workload["dtype"])

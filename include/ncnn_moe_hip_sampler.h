@@ -131,17 +131,17 @@ int ncnn_moe_hip_sampler_sample(
  * returns at once.  device_logits may be any device matrix (row_stride in elements), not only the
  * handle's buffer.  This is the entry the decode step calls in its own stream.
  * may_need_full_order: pass 0 when the caller knows from its host-side SamplingOptions that every
- * row is greedy or has 1 <= top_k <= 64 (then one kernel is enqueued); pass 1 otherwise (a select
- * kernel for Top-K windows up to 1024 and the full-order kernels are enqueued as well and pick up
- * the rows that need them); pass 3 (1 | NCNN_MOE_PASSES_SIDE_BY_SIDE) when the caller knows that the
- * batch holds both rows with 64 < top_k <= 1024 and rows with a wider or no window: the two later
- * passes, each of which keeps one workgroup per row busy, then run side by side, one of them on a
- * second stream of the handle that forks from and joins `stream` (worth its two stream hand-overs,
- * some 30 us, from about a hundred rows of each kind; a row with top_k <= 64 whose ties overflow the
- * first kernel's lists is then finished by the full-order kernels rather than by the select kernel for
- * wider windows: same result, NCNN_MOE_ROW_FLAG_GENERAL_PATH set); add NCNN_MOE_PASSES_NO_WIDE_WINDOWS when the
- * caller knows that no row has 64 < top_k <= 1024: the select kernel for such windows is then not
- * enqueued (a row that has one after all is served by the full-order kernels: slower, same result).
+ * row is greedy or has 1 <= top_k <= 64 (then one kernel is enqueued); pass 1 otherwise (the kernels
+ * for Top-K windows up to 1024, for rows without a window and for what those leave are enqueued as
+ * well and pick up the rows that need them); pass 3 (1 | NCNN_MOE_PASSES_SIDE_BY_SIDE) when the
+ * caller knows that the batch holds both rows with 64 < top_k <= 1024 and rows with a wider or no
+ * window: the first kernel and those for wide windows then run beside those for rows without one, on
+ * a second stream of the handle that forks from and joins `stream` (worth its stream hand-overs from
+ * some dozens of rows of each kind; a row with top_k <= 64 whose ties overflow the first kernel's
+ * lists is then finished by the full-order kernels: same result, NCNN_MOE_ROW_FLAG_GENERAL_PATH
+ * set); add NCNN_MOE_PASSES_NO_WIDE_WINDOWS when the caller knows that no row has
+ * 64 < top_k <= 1024: the kernels for such windows are then not enqueued (a row that has one after
+ * all is served like one without a window: slower, same result).
  * Calls on one handle share its scratch memory and must not overlap. */
 #define NCNN_MOE_PASSES_FULL_ORDER 1
 #define NCNN_MOE_PASSES_SIDE_BY_SIDE 2

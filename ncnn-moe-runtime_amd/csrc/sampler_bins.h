@@ -48,7 +48,7 @@ constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms
 constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
 constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
 constexpr uint32_t kBinHead = 2048;              // elements of the sorted head at most (unless a window takes more): behind
-                                                 // so many a term half way seldom has to be fetched, 40 us each
+                                                 // so many a term half way seldom has to be fetched, 9 us and more each
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
 constexpr uint32_t kBinStops = 512;
@@ -68,7 +68,9 @@ constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: t
 // The walks want 220 registers; at 128, which two of their workgroups to a compute unit leave, some 35 of them and 130
 // scalars pass through scratch and lane moves.  A call of so few rows that every part has a compute unit of its own takes
 // the walks built for 256 (8 x 151,936 without a window: 141 -> 131 us, 11 such rows of a verification step: 240 -> 223 us);
-// more rows need the second workgroup.
+// more rows need the second workgroup.  The rule looks at the call's rows, because how many of them have no window is known to
+// the device only; with few of them the two kinds are close (16 and 17 rows of 151,936, of which 1, 4 or 8 have no window:
+// 111, 112 and 113 us with 256 registers, 104, 114 and 125 us with 128).
 constexpr uint32_t kRoomyRows = kBinGrid / 2u / kMaxBinParts;
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
 // Foreseen sums decide what is prepared, never what a sum is: a walk that finds its exact sum elsewhere fetches what it needs.
@@ -1141,10 +1143,11 @@ __device__ __forceinline__ uint32_t fine_place(float term, uint32_t shift, uint3
 
 // Fetches the elements of bins [shared.low, shared.high] (at most kBinExtraCap of them; shared.extra_count: how many there
 // are), in order, to shared.terms[kBinExtraPlace ..].
-// What bounds it: the row's terms through one compute unit with two wavefronts per SIMD in flight.  Every load waited for
-// in turn and five instructions per element took 20 us for 151,936 terms, and with many rows the call waits for the one
-// that fetches most often; with the next loads under way and one comparison per element a call of 512 mixed rows of
-// 129,280 takes 352 us instead of 366.
+// What bounds it: the row's terms through one compute unit with two wavefronts per SIMD in flight (8 to 9 us for 151,936),
+// then the elements found (1,500 of them some 20 us more: a place each, then order).  Every load waited for in turn and five
+// instructions per element took 20 us before any was found, and with many rows the call waits for the one that fetches most
+// often; with the next loads under way and one comparison per element a call of 512 mixed rows of 129,280 took 352 us
+// instead of 366.
 template <bool ROOMY>
 __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t positions, uint32_t misalignment, uint32_t shift, BinWalkShared& shared, int tid)
 {
