@@ -397,28 +397,34 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
     if ((tid & (kWaveSize - 1)) == 0 && neighbours >= kWindowRankedTies)
         atomicMax(&shared.neighbours, neighbours);
     __syncthreads();
-    const bool sorts = shared.neighbours != 0u;
-    if (sorts)
+    const auto take = [&](uint32_t rank, uint32_t key, uint32_t token) {
+        shared.tokens[rank] = token;
+        shared.terms[rank] = expf_libm(value_from_ascending_key(key) / p.temperature - maximum, shared.exp2_table);
+    };
+    if (same_in_all(shared.neighbours) != 0u)
     {
         static_assert(offsetof(WindowFinishShared, tokens) == kWindowListCap * sizeof(uint32_t), "keys and tokens lie one behind the other");
+        constexpr uint32_t kWindowEach = kSelectTopK / kThreads;
+        static_assert(kWindowEach * kThreads == kSelectTopK, "the threads hold the widest window");
         uint64_t* const pairs = reinterpret_cast<uint64_t*>(shared.keys);
-#pragma unroll
         for (uint32_t k = 0; k < kPerThread; ++k)
         {
             const uint32_t i = k * kThreads + tid;
             if (i < count)
-                pairs[i] = (static_cast<uint64_t>(keys[k]) << 32) | (0xffffffffu - tokens[k]);
+                pairs[i] = (static_cast<uint64_t>(g.keys[static_cast<size_t>(row) * kWindowListCap + i]) << 32) | (0xffffffffu - g.tokens[static_cast<size_t>(row) * kWindowListCap + i]);
         }
         sort_candidates<WAVES>(pairs, count, tid);
-        // (from here on as after ranking: the thread holds some of the window's elements and their ranks)
+        uint64_t own[kWindowEach];
 #pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k)
-        {
-            const uint64_t pair = pairs[k * kThreads + tid];
-            keys[k] = static_cast<uint32_t>(pair >> 32);
-            tokens[k] = 0xffffffffu - static_cast<uint32_t>(pair);
-        }
+        for (uint32_t k = 0; k < kWindowEach; ++k)
+            own[k] = pairs[k * kThreads + tid];
         __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kWindowEach; ++k)
+        {
+            if (k * kThreads + tid < window)
+                take(k * kThreads + tid, static_cast<uint32_t>(own[k] >> 32), 0xffffffffu - static_cast<uint32_t>(own[k]));
+        }
     }
     else
     {
@@ -442,50 +448,47 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
                 shared.counters[first + k] = front;
             front += held[k];
         }
-    }
-    __syncthreads();
+        __syncthreads();
 #pragma unroll
-    for (uint32_t k = 0; k < kPerThread; ++k)
-    {
-        if (!sorts && k * kThreads + tid < count)
+        for (uint32_t k = 0; k < kPerThread; ++k)
         {
-            const uint32_t at = shared.counters[fine[k]] + turn[k];
-            shared.keys[at] = keys[k];
-            shared.tokens[at] = tokens[k];
-        }
-    }
-    __syncthreads();
-    uint32_t rank[kPerThread];
-#pragma unroll
-    for (uint32_t k = 0; k < kPerThread; ++k)
-    {
-        rank[k] = k * kThreads + tid;
-        if (!sorts && k * kThreads + tid < count)
-        {
-            const uint32_t low = shared.counters[fine[k]];
-            const uint32_t high = fine[k] + 1u < count ? shared.counters[fine[k] + 1u] : count;
-            rank[k] = low;
-            if (low < window) // (what lies behind the window need not be in order)
+            if (k * kThreads + tid < count)
             {
-                for (uint32_t j = low; j < high; ++j)
-                {
-                    const uint32_t other = shared.keys[j];
-                    rank[k] += other > keys[k] || (other == keys[k] && shared.tokens[j] < tokens[k]) ? 1u : 0u;
-                }
+                const uint32_t at = shared.counters[fine[k]] + turn[k];
+                shared.keys[at] = keys[k];
+                shared.tokens[at] = tokens[k];
             }
-            else
-                rank[k] = window;
         }
-    }
-    __syncthreads();
-    // ---- the window: its tokens and terms
+        __syncthreads();
+        uint32_t rank[kPerThread];
 #pragma unroll
-    for (uint32_t k = 0; k < kPerThread; ++k)
-    {
-        if (k * kThreads + tid < count && rank[k] < window)
+        for (uint32_t k = 0; k < kPerThread; ++k)
         {
-            shared.tokens[rank[k]] = tokens[k];
-            shared.terms[rank[k]] = expf_libm(value_from_ascending_key(keys[k]) / p.temperature - maximum, shared.exp2_table);
+            rank[k] = 0u;
+            if (k * kThreads + tid < count)
+            {
+                const uint32_t low = shared.counters[fine[k]];
+                const uint32_t high = fine[k] + 1u < count ? shared.counters[fine[k] + 1u] : count;
+                rank[k] = low;
+                if (low < window) // (what lies behind the window need not be in order)
+                {
+                    for (uint32_t j = low; j < high; ++j)
+                    {
+                        const uint32_t other = shared.keys[j];
+                        rank[k] += other > keys[k] || (other == keys[k] && shared.tokens[j] < tokens[k]) ? 1u : 0u;
+                    }
+                }
+                else
+                    rank[k] = window;
+            }
+        }
+        __syncthreads();
+        // ---- the window: its tokens and terms
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+        {
+            if (k * kThreads + tid < count && rank[k] < window)
+                take(rank[k], keys[k], tokens[k]);
         }
     }
     __syncthreads();
