@@ -1479,6 +1479,8 @@ __device__ __forceinline__ void walk_bins(
             }
             while (status == 3u)
             {
+                // (the end, unless there is more to run over and the exact sum has not met its stop condition)
+                unforeseen = unforeseen || packed_kind(shared.packed[cur]) == kBinBeyond;
                 if (unforeseen)
                 {
                     const uint32_t front = front_of(cur);
@@ -1538,8 +1540,6 @@ __device__ __forceinline__ void walk_bins(
                 }
                 else if ((stop_word & kStopExponent) != 0u)
                     ++stop; // (a new exponent from this bin on)
-                else if (stop_here == kBins || packed_kind(shared.packed[stop_here]) == kBinBeyond)
-                    unforeseen = true; // (the end, unless there is more to run over and the exact sum has not met its stop condition)
                 else if (packed_kind(shared.packed[stop_here]) != kBinListed)
                 {
                     // terms half way: their roundings follow from the masks, unless the sum has another exponent than was

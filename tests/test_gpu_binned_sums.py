@@ -188,3 +188,19 @@ def test_thousands_of_equal_terms(kind, vocab):
             cpu = parity_util.run_oracle(logits, params, uniforms)
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "%s top_p %g min_p %g top_k %d" % (kind, top_p, min_p, top_k))
             assert sampler.binned_rows(rows).tolist() == [1] * rows, (top_p, min_p, top_k)
+
+
+@pytest.mark.parametrize("vocab", [4099, 16384])
+def test_runs_of_listed_bins_that_end_with_the_sum(vocab):
+    """A Min-P cut or a window ends the sum behind a run of listed bins, and the next bins hold nothing: the end is not run past."""
+    rng = np.random.default_rng(vocab + 1)
+    rows = 64
+    print("[case] runs that end with the sum, %d x %d" % (rows, vocab), flush=True)
+    logits = _bf16_values((rng.standard_normal((rows, vocab)) * rng.uniform(1.5, 4.0, (rows, 1))).astype(np.float32))
+    uniforms = rng.random(rows, dtype=np.float32)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        for top_p, min_p, top_k in ((1.0, 1e-6, 0), (1.0, 3e-6, 0), (1.0, 3e-5, 0), (0.9999, 1e-6, 0), (1.0, 0.0, vocab - 20), (1.0, 1e-6, vocab - 20)):
+            params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "top_p %g min_p %g top_k %d" % (top_p, min_p, top_k))
