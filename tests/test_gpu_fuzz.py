@@ -74,9 +74,10 @@ def test_random_batches(sampler, seed):
 
 
 def _long_row(rng, vocab):
-    """Rows as a serving loop has them without a window: fp32, fp32 of bf16 values, coarser ones, masked ones, narrow ones."""
+    """Rows as a serving loop has them without a window (fp32, fp32 of bf16 values, coarser ones, masked ones, narrow ones), and rows
+    of few levels or of terms that end half way between two sums."""
     row = (rng.standard_normal(vocab) * rng.uniform(1.0, 4.0)).astype(np.float32)
-    kind = int(rng.integers(0, 9))
+    kind = int(rng.integers(0, 12))
     if kind in (1, 2):
         row = workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(row))
     elif kind == 3:
@@ -92,10 +93,16 @@ def _long_row(rng, vocab):
         row[rng.integers(0, vocab, 5)] = rng.choice(np.array([0.25, 0.9431472, 2.0, 12.0], dtype=np.float32))
     elif kind == 8:
         row[rng.integers(0, vocab, 20)] += np.float32(15.0)
+    elif kind == 9:
+        row = rng.choice(np.sort(rng.uniform(-12.0, 0.0, int(rng.integers(2, 30)))), vocab)  # a few levels
+    elif kind == 10:
+        row = np.log(2.0) * -rng.integers(0, 24, vocab)  # terms that are powers of two: many half way values
+    elif kind == 11:
+        row = rng.permutation(-np.arange(vocab) * rng.uniform(1e-5, 1e-2))
     return np.ascontiguousarray(row, dtype=np.float32)
 
 
-@pytest.mark.parametrize("seed", range(20))
+@pytest.mark.parametrize("seed", range(60))
 def test_random_batches_of_long_rows(seed):
     rng = np.random.default_rng(70000 + seed)
     rows = int(rng.choice([5, 16, 17, 40, 70]))
