@@ -47,7 +47,7 @@ constexpr uint32_t kOneBits = 0x3f800000u;       // the largest term
 constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms of 2^-25 or less move no sum
 constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
 constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
-constexpr uint32_t kBinHead = 2048;              // elements of the sorted head at most (unless a window takes more): behind
+constexpr uint32_t kBinHead = 1920;              // elements of the sorted head at most (unless a window takes more), 30 chunks of sum_head: behind
                                                  // so many a term half way seldom has to be fetched, 9 us and more each
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
@@ -852,7 +852,6 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
     }
 }
 
-// The terms at terms[0 .. count) (LDS, in descending order) added to `sum` by one wave, two consecutive ones a lane.
 struct WaveSum
 {
     float sum;
@@ -860,85 +859,42 @@ struct WaveSum
     bool stopped;
 };
 
+// The terms at terms[0 .. count) (LDS, in descending order) added to `sum` by one wave, one addition behind the other, 64 of them in some
+// 530 cycles (`scratch`: see wave_sequential_total).  Scans of the terms' steps, two terms a lane and one scan more for each
+// binade that the sum leaves, took 2,000 to 2,300 cycles for up to 128 terms.
 template <int PHASE>
-__device__ __forceinline__ WaveSum wave_add_terms(
-    const float* terms, uint32_t count, float sum, int mode, float bound, float divisor, float second_divisor)
+__device__ __forceinline__ WaveSum wave_add_in_order(
+    const float* terms, uint32_t count, float sum, int mode, float bound, float divisor, float second_divisor, float* scratch)
 {
-    constexpr uint32_t kPerLane = 2;
     const uint32_t lane = static_cast<uint32_t>(lane_id());
-    for (uint32_t base = 0; base < count; base += kPerLane * kWaveSize)
+    for (uint32_t first = 0; first < count; first += kWaveSize)
     {
-        const uint32_t own = base + lane * kPerLane;
-        float v[kPerLane];
-#pragma unroll
-        for (uint32_t j = 0; j < kPerLane; ++j)
+        const uint32_t here = min(count - first, static_cast<uint32_t>(kWaveSize));
+        float own = lane < here ? terms[first + lane] : 0.0f;
+        if (PHASE >= 1)
+            own = own / divisor;
+        if (PHASE >= 2)
+            own = own / second_divisor;
+        scratch[lane] = own;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (uint32_t part = 0; part < here; part += kTotalled)
         {
-            v[j] = own + j < count ? terms[own + j] : 0.0f;
-            if (PHASE >= 1)
-                v[j] = v[j] / divisor;
-            if (PHASE >= 2)
-                v[j] = v[j] / second_divisor;
+            const float behind = wave_sequential_total(scratch, static_cast<int>(part), sum);
+            if ((mode == kStopAtOrAbove && behind >= bound) || (mode == kStopAbove && behind > bound))
+            {
+                // (the sums never fall: one of these is the first)
+                own = lane < kTotalled ? scratch[part + lane] : 0.0f;
+                own = lane == 0u ? sum + own : own;
+                const float sums = wave_sequential_sums_of_first<16>(own, kTotalled);
+                const bool stops = (mode == kStopAtOrAbove && sums >= bound) || (mode == kStopAbove && sums > bound);
+                const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < kTotalled && stops));
+                return WaveSum{read_lane(sums, at), first + part + static_cast<uint32_t>(at), true};
+            }
+            sum = behind;
         }
-        uint32_t start = base;
-        while (true)
-        {
-            int exponent;
-            uint32_t mantissa;
-            decode_sum(sum, exponent, mantissa);
-            const uint32_t stop_at = stop_mantissa(mode, bound, exponent);
-            const uint32_t limit = min(stop_at, kBinadeFull);
-            ParityStep steps[kPerLane];
-            ParityStep total{0u, 0u};
-#pragma unroll
-            for (uint32_t j = 0; j < kPerLane; ++j)
-            {
-                const ParityStep step = step_of_term(v[j], exponent);
-                const bool active = own + j >= start;
-                steps[j] = ParityStep{active ? step.even : 0u, active ? step.odd : 0u};
-                total = compose_steps(total, steps[j]);
-            }
-            const ParityStep through = wave_scan_steps(total);
-            ParityStep in_front{__shfl_up(through.even, 1, kWaveSize), __shfl_up(through.odd, 1, kWaveSize)};
-            if (lane == 0u)
-                in_front = ParityStep{0u, 0u};
-            uint32_t current = apply_step(mantissa, in_front);
-            const uint32_t behind = apply_step(mantissa, through);
-            const uint64_t reaching = __builtin_amdgcn_ballot_w64(behind >= limit);
-            if (reaching == 0ull)
-            {
-                sum = encode_sum(exponent, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(behind), kWaveSize - 1)));
-                break;
-            }
-            const int first = __builtin_ctzll(reaching);
-            // the first term of that lane that takes the mantissa to the limit
-            uint32_t at = 0, before = 0, after = 0;
-            float term = 0.0f;
-            bool hit = false;
-#pragma unroll
-            for (uint32_t j = 0; j < kPerLane; ++j)
-            {
-                const uint32_t next = apply_step(current, steps[j]);
-                const bool here = !hit && own + j >= start && next >= limit;
-                at = here ? own + j : at;
-                before = here ? current : before;
-                after = here ? next : after;
-                term = here ? v[j] : term;
-                hit = hit || here;
-                current = next;
-            }
-            at = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), first));
-            before = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(before), first));
-            after = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(after), first));
-            term = read_lane(term, first);
-            if (after < kBinadeFull)
-                return WaveSum{encode_sum(exponent, after), at, true};
-            sum = encode_sum(exponent, before) + term;
-            if ((mode == kStopAtOrAbove && sum >= bound) || (mode == kStopAbove && sum > bound))
-                return WaveSum{sum, at, true};
-            start = at + 1u;
-            if (start >= count)
-                break;
-        }
+        __builtin_amdgcn_wave_barrier();
     }
     return WaveSum{sum, 0u, false};
 }
@@ -986,11 +942,12 @@ __device__ __forceinline__ WaveSum wave_add_repeated(
     return WaveSum{sum, 0u, false};
 }
 
-// Of the sums over a sorted stretch of terms in LDS (sum_chunks, sum_head): per 64 terms the sum in front of them (about),
+// Of the sums over a sorted stretch of terms in LDS (sum_chunks, sum_head): per 64 terms their plain sum,
 // and what they do to a sum of that exponent.
 struct HeadScratch
 {
-    float chunk_front[kWaveSize];
+    alignas(16) float in_order[kWaveSize]; // (see wave_sequential_total)
+    float chunk_sum[kWaveSize];
     uint32_t chunk_exponent[kWaveSize], chunk_even[kWaveSize], chunk_odd[kWaveSize];
     float sum;
     uint32_t stop; // 0xffffffff: no element met the stop condition
@@ -1254,36 +1211,84 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     }
 }
 
-// The plain sums of the terms in front of each 64 of `count` (4096 at most).
+// The inclusive sums over each row of 16 lanes.
+__device__ __forceinline__ uint32_t row16_prefix_sum_u32(uint32_t value)
+{
+    value += dpp_source<0x111, 0xf>(value); // row_shr:1
+    value += dpp_source<0x112, 0xf>(value); // row_shr:2
+    value += dpp_source<0x114, 0xf>(value); // row_shr:4
+    value += dpp_source<0x118, 0xf>(value); // row_shr:8
+    return value;
+}
+
+// The plain sum of each 64 of `count` terms (4096 at most): a row of 16 lanes holds 64 terms, a lane four of them.
 template <int WAVES>
 __device__ __forceinline__ void sum_chunks(HeadScratch& scratch, const float* terms, uint32_t count, int tid)
 {
-    const int lane = tid & (kWaveSize - 1);
-    const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
-    const uint32_t chunks = (count + kWaveSize - 1u) / kWaveSize;
-    for (uint32_t c = wave; c < chunks; c += WAVES)
+    for (uint32_t i = 4u * static_cast<uint32_t>(tid); same_in_all(i) < count; i += 4u * WAVES * kWaveSize)
     {
-        const uint32_t i = c * kWaveSize + lane;
-        const float sum = wave_prefix_sum_f32(i < count ? terms[i] : 0.0f);
-        if (lane == kWaveSize - 1)
-            scratch.chunk_front[c] = sum;
+        const float4 own = *reinterpret_cast<const float4*>(terms + i);
+        float sum = ((i < count ? own.x : 0.0f) + (i + 1u < count ? own.y : 0.0f)) + ((i + 2u < count ? own.z : 0.0f) + (i + 3u < count ? own.w : 0.0f));
+#define NCNN_MOE_ADD_STAGE(CONTROL) sum += __uint_as_float(dpp_source<CONTROL, 0xf>(__float_as_uint(sum)));
+        NCNN_MOE_ADD_STAGE(0x111)
+        NCNN_MOE_ADD_STAGE(0x112)
+        NCNN_MOE_ADD_STAGE(0x114)
+        NCNN_MOE_ADD_STAGE(0x118)
+#undef NCNN_MOE_ADD_STAGE
+        if ((tid & 15) == 15)
+            scratch.chunk_sum[i / kWaveSize] = sum;
     }
     __syncthreads();
-    const float own = static_cast<uint32_t>(lane) < chunks ? scratch.chunk_front[lane] : 0.0f;
-    const float through = wave_prefix_sum_f32(own);
-    __syncthreads();
-    if (wave == 0u)
-        scratch.chunk_front[lane] = through - own;
-    __syncthreads();
+}
+
+// What four terms a lane, 64 a row of 16 lanes, do to a sum of that exponent: the row's last lane has the whole of it.
+__device__ __forceinline__ ParityStep row16_steps(const float (&terms)[4], int exponent)
+{
+    uint32_t sum = 0;
+    bool differ = false; // a term half way between two sums
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+    {
+        // (as step_of_term, for zero and normal numbers: zero comes out as a step of zero)
+        const uint32_t bits = __float_as_uint(terms[c]);
+        const uint32_t mantissa = (bits & 0x7fffffu) | 0x800000u;
+        const int difference = exponent - static_cast<int>(bits >> 23);
+        const uint32_t shift = static_cast<uint32_t>(min(max(difference, 1), 25));
+        const uint32_t half = 1u << (shift - 1u);
+        differ = differ || ((mantissa & (2u * half - 1u)) == half && difference > 0);
+        sum += difference > 0 ? (mantissa + half) >> shift : kBinadeFull;
+    }
+    if (__builtin_amdgcn_ballot_w64(differ) == 0ull)
+    {
+        // (64 steps of 2^24 at most)
+        const uint32_t through = min(row16_prefix_sum_u32(sum), kStepCap);
+        return ParityStep{through, through};
+    }
+    ParityStep steps[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        steps[c] = step_of_term(terms[c], exponent);
+    ParityStep through = compose_steps(compose_steps(steps[0], steps[1]), compose_steps(steps[2], steps[3]));
+#define NCNN_MOE_SCAN_STAGE(CONTROL) through = compose_steps(ParityStep{dpp_source<CONTROL, 0xf>(through.even), dpp_source<CONTROL, 0xf>(through.odd)}, through);
+    NCNN_MOE_SCAN_STAGE(0x111)
+    NCNN_MOE_SCAN_STAGE(0x112)
+    NCNN_MOE_SCAN_STAGE(0x114)
+    NCNN_MOE_SCAN_STAGE(0x118)
+#undef NCNN_MOE_SCAN_STAGE
+    return through;
 }
 
 // The sum of `count` terms in descending order (scratch.sum, scratch.stop), exactly as a sequential loop makes it; every thread calls it.  The waves work
 // out what each 64 terms do to a sum of the exponent that it should have there (from sum_chunks), while the first wave adds the first
-// terms in order; it then takes the chunks whose exponent was right in one scan and looks into the others.
+// terms in order; it then takes the chunks whose exponent was right in one scan and adds the terms of the others in order.
+// What bounds it: dependent instructions of the first wave, some 530 cycles for 64 terms in order, 300 for each scan.  2,044 terms on 8
+// waves, sums that leave one to three binades behind the first 64 terms: the normaliser's 2,500 to 5,300 cycles, the Top-P sum's 3,200 to
+// 5,800, the draw's 3,500 to 5,200; with the first 256 terms in order at 12 cycles each, a chunk at a time a wave and scans of the terms'
+// steps for a chunk in which the sum leaves its binade 7,000 to 10,400, 5,200 to 11,800 and 4,800 to 8,400.
 template <int WAVES, int PHASE>
 __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* terms, uint32_t count, int mode, float bound, float divisor, float second_divisor, int tid)
 {
-    constexpr uint32_t kInOrder = 4; // chunks added in order
+    constexpr uint32_t kInOrder = 2; // chunks added in order (four of them where there are no more: 3,000 to 3,800 cycles instead of 2,300 to 3,400)
     const int lane = tid & (kWaveSize - 1);
     const uint32_t wave = same_in_all(static_cast<uint32_t>(tid) >> 6);
     const uint32_t chunks = (count + kWaveSize - 1u) / kWaveSize;
@@ -1294,40 +1299,33 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
             t = t / second_divisor;
         return t;
     };
-    const float scale = PHASE == 0 ? 1.0f : PHASE == 1 ? 1.0f / divisor : 1.0f / (divisor * second_divisor);
-    for (uint32_t c = wave == 0u ? WAVES : wave; c < chunks; c += WAVES)
-    {
-        if (c < kInOrder)
-            continue;
-        const uint32_t i = c * kWaveSize + lane;
-        const uint32_t exponent = same_in_all(__float_as_uint(scratch.chunk_front[c] * scale) >> 23);
-        const ParityStep through = wave_scan_steps(step_of_term(scaled(i < count ? terms[i] : 0.0f), static_cast<int>(exponent)));
-        if (lane == kWaveSize - 1)
-        {
-            scratch.chunk_exponent[c] = exponent;
-            scratch.chunk_even[c] = through.even;
-            scratch.chunk_odd[c] = through.odd;
-        }
-    }
     float sum = 0.0f;
     uint32_t stop = 0xffffffffu;
     if (wave == 0u)
     {
-        const uint32_t in_order = min(count, kInOrder * kWaveSize);
-        for (uint32_t first = 0; first < in_order && stop == 0xffffffffu; first += kWaveSize)
+        // (its share would be the terms among which those half way are frequent)
+        const WaveSum result = wave_add_in_order<PHASE>(terms, min(count, kInOrder * kWaveSize), sum, mode, bound, divisor, second_divisor, scratch.in_order);
+        sum = result.sum;
+        if (result.stopped)
+            stop = result.index;
+    }
+    else
+    {
+        const float scale = PHASE == 0 ? 1.0f : PHASE == 1 ? 1.0f / divisor : 1.0f / (divisor * second_divisor);
+        const float chunk_sum = static_cast<uint32_t>(lane) < chunks ? scratch.chunk_sum[lane] : 0.0f;
+        const float chunk_front = wave_prefix_sum_f32(chunk_sum) - chunk_sum;
+        for (uint32_t i = kInOrder * kWaveSize + 4u * static_cast<uint32_t>(tid - kWaveSize); same_in_all(i) < count; i += 4u * (WAVES - 1) * kWaveSize)
         {
-            const uint32_t i = first + lane;
-            float own = i < count ? scaled(terms[i]) : 0.0f;
-            own = lane == 0 ? sum + own : own;
-            const float sums = wave_sequential_sums(own);
-            const bool stops = i < count && ((mode == kStopAtOrAbove && sums >= bound) || (mode == kStopAbove && sums > bound));
-            const uint64_t stopping = __builtin_amdgcn_ballot_w64(stops);
-            sum = read_lane(sums, kWaveSize - 1);
-            if (stopping != 0ull)
+            const float4 raw = *reinterpret_cast<const float4*>(terms + i);
+            const float own[4] = {i < count ? scaled(raw.x) : 0.0f, i + 1u < count ? scaled(raw.y) : 0.0f, i + 2u < count ? scaled(raw.z) : 0.0f,
+                                  i + 3u < count ? scaled(raw.w) : 0.0f};
+            const uint32_t exponent = __float_as_uint(__shfl(chunk_front, static_cast<int>(i / kWaveSize), kWaveSize) * scale) >> 23;
+            const ParityStep through = row16_steps(own, static_cast<int>(exponent));
+            if ((tid & 15) == 15)
             {
-                const int at = __builtin_ctzll(stopping);
-                sum = read_lane(sums, at);
-                stop = first + static_cast<uint32_t>(at);
+                scratch.chunk_exponent[i / kWaveSize] = exponent;
+                scratch.chunk_even[i / kWaveSize] = through.even;
+                scratch.chunk_odd[i / kWaveSize] = through.odd;
             }
         }
     }
@@ -1336,34 +1334,44 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
     {
         uint32_t c = kInOrder;
         uint32_t own_exponent = 0, own_even = 0, own_odd = 0;
-        if (static_cast<uint32_t>(lane) < chunks && static_cast<uint32_t>(lane) >= kInOrder)
+        if (stop == 0xffffffffu && static_cast<uint32_t>(lane) < chunks && static_cast<uint32_t>(lane) >= kInOrder)
         {
             own_exponent = scratch.chunk_exponent[lane];
             own_even = scratch.chunk_even[lane];
             own_odd = scratch.chunk_odd[lane];
         }
+        // (the chunks from c on that the sum runs through are consecutive: the steps up to each are one difference.  64 numbers of
+        // 2^25 at most: what is past the binade is only compared against it)
+        const uint32_t through = wave_prefix_sum_u32(min(own_even, 2u * kBinadeFull));
         while (c < chunks && stop == 0xffffffffu)
         {
             int exponent;
             uint32_t mantissa;
             decode_sum(sum, exponent, mantissa);
             const uint32_t goal = min(stop_mantissa(mode, bound, exponent), kBinadeFull);
+            const uint32_t in_front = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), static_cast<int>(c - 1u)));
             const bool ahead = static_cast<uint32_t>(lane) >= c && static_cast<uint32_t>(lane) < chunks;
-            const bool usable = ahead && own_exponent == static_cast<uint32_t>(exponent);
-            const ParityStep through = wave_scan_steps(ParityStep{usable ? own_even : 0u, usable ? own_odd : 0u});
-            const uint32_t behind = apply_step(mantissa, through);
-            const uint64_t bad = __builtin_amdgcn_ballot_w64(ahead && !(usable && behind < goal));
-            const uint32_t first_bad = bad != 0ull ? static_cast<uint32_t>(__builtin_ctzll(bad)) : chunks;
-            if (first_bad > c)
-                sum = encode_sum(exponent, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(behind), static_cast<int>(first_bad - 1u))));
-            c = first_bad;
+            const uint32_t behind = mantissa + (through - in_front);
+            const uint64_t special = __builtin_amdgcn_ballot_w64(ahead && (own_exponent != static_cast<uint32_t>(exponent) || own_even != own_odd || behind >= goal));
+            const uint32_t first_special = special != 0ull ? static_cast<uint32_t>(__builtin_ctzll(special)) : chunks;
+            if (first_special > c)
+                mantissa = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(behind), static_cast<int>(first_special - 1u)));
+            c = first_special;
+            sum = encode_sum(exponent, mantissa);
             if (c >= chunks)
                 break;
-            const uint32_t first = c * kWaveSize;
-            const WaveSum result = wave_add_terms<PHASE>(terms + first, min(count - first, static_cast<uint32_t>(kWaveSize)), sum, mode, bound, divisor, second_divisor);
-            sum = result.sum;
-            if (result.stopped)
-                stop = first + result.index;
+            const uint32_t of_chunk = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>((mantissa & 1u) != 0u ? own_odd : own_even), static_cast<int>(c)));
+            if (static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(own_exponent), static_cast<int>(c))) == static_cast<uint32_t>(exponent) &&
+                mantissa + of_chunk < goal)
+                sum = encode_sum(exponent, mantissa + of_chunk); // (a term half way between two sums among its terms)
+            else
+            {
+                const uint32_t first = c * kWaveSize;
+                const WaveSum result = wave_add_in_order<PHASE>(terms + first, min(count - first, static_cast<uint32_t>(kWaveSize)), sum, mode, bound, divisor, second_divisor, scratch.in_order);
+                sum = result.sum;
+                if (result.stopped)
+                    stop = first + result.index;
+            }
             ++c;
         }
         if (lane == 0)
@@ -1465,7 +1473,7 @@ __device__ __forceinline__ void walk_bins(
                     else
                     {
                         take = share_of_sum(low, high, kBinExtraPlace, count);
-                        result = wave_add_terms<PHASE>(shared.terms + kBinExtraPlace, take, sum, mode, bound, divisor, second_divisor);
+                        result = wave_add_in_order<PHASE>(shared.terms + kBinExtraPlace, take, sum, mode, bound, divisor, second_divisor, shared.head.in_order);
                     }
                     sum = result.sum;
                     if (result.stopped)
@@ -1605,7 +1613,7 @@ __device__ __forceinline__ void walk_bins(
                     }
                     const uint32_t count = front_of(behind) - front;
                     const uint32_t take = share_of_sum(stop_here, behind - 1u, place, count);
-                    const WaveSum result = wave_add_terms<PHASE>(shared.terms + place, take, sum, mode, bound, divisor, second_divisor);
+                    const WaveSum result = wave_add_in_order<PHASE>(shared.terms + place, take, sum, mode, bound, divisor, second_divisor, shared.head.in_order);
                     sum = result.sum;
                     if (result.stopped)
                         stopped_at(front + result.index, place + result.index);

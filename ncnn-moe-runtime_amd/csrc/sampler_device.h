@@ -441,21 +441,39 @@ __device__ __forceinline__ float wave_sequential_sums(float term)
 }
 
 // The same for the wave's first `count` lanes (count: the same in every lane): count - 1 turns, rounded up to
-// whole trips of four (a turn too many changes nothing: a lane whose lower neighbour is final computes its own
-// final value again).  The lanes from `count` on return no sum of anything.
+// whole trips of TURNS (a turn too many changes nothing: a lane whose lower neighbour is final computes its own
+// final value again; a turn is 12 cycles, a trip some 30 more).  The lanes from `count` on return no sum of anything.
+template <int TURNS = 4>
 __device__ __forceinline__ float wave_sequential_sums_of_first(float term, int count)
 {
     float sums = term;
-    for (int turn = 1; turn < count; turn += 4)
+    for (int turn = 1; turn < count; turn += TURNS)
     {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < TURNS; ++k)
         {
             const float below = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sums), 0x138, 0xf, 0xf, true));
             sums = below + term;
         }
     }
     return sums;
+}
+
+// `sum` plus the kTotalled terms of the wave's lanes from `first` on (non-negative; `scratch`, 16-byte aligned, holds one per lane), added in
+// lane order: the last of the sums above alone.  Every lane reads the terms back and adds them all: 6 cycles a term against the 12
+// of an addition across lanes.
+constexpr int kTotalled = 32;
+
+__device__ __forceinline__ float wave_sequential_total(const float* scratch, int first, float sum)
+{
+    float4 terms[kTotalled / 4];
+#pragma unroll
+    for (int k = 0; k < kTotalled / 4; ++k)
+        terms[k] = reinterpret_cast<const float4*>(scratch + first)[k];
+#pragma unroll
+    for (int k = 0; k < kTotalled / 4; ++k)
+        sum = (((sum + terms[k].x) + terms[k].y) + terms[k].z) + terms[k].w;
+    return sum;
 }
 
 // Reduction over each row of 16 lanes (every lane receives its row's result), by four DPP exchanges:

@@ -92,8 +92,16 @@ __device__ __forceinline__ ParityStep repeat_steps(const ParityStep s, uint32_t 
 // Inclusive scan of the lanes' steps in lane order (lane i: the composition of lanes 0 .. i), by DPP shifts
 // inside rows of 16 lanes and two broadcasts across rows; a lane without a source composes with the
 // identity (a step of zero).
+// A stage of compositions is some 13 dependent instructions, 470 cycles for the six of them; where no lane's two steps differ
+// (no term half way between two sums: most waves) the steps are plain numbers and their sums take 130.
 __device__ __forceinline__ ParityStep wave_scan_steps(ParityStep v)
 {
+    if (__builtin_amdgcn_ballot_w64(v.even != v.odd) == 0ull)
+    {
+        // (64 numbers of 2^25 at most: what is past the binade is only compared against it)
+        const uint32_t through = min(wave_prefix_sum_u32(min(v.even, 2u * kBinadeFull)), kStepCap);
+        return ParityStep{through, through};
+    }
 #define NCNN_MOE_SCAN_STAGE(CONTROL, ROW_MASK)                                                              \
     {                                                                                                        \
         const ParityStep earlier{dpp_source<CONTROL, ROW_MASK>(v.even), dpp_source<CONTROL, ROW_MASK>(v.odd)}; \

@@ -721,6 +721,7 @@ __device__ __forceinline__ uint32_t add_composed_steps(const uint4& mine, uint32
 __global__ __launch_bounds__(kResidualThreads) void verify_draw_kernel(VerifySumsArgs v, uint32_t chunks)
 {
     __shared__ __align__(16) float entries[kResidualSub];
+    __shared__ __align__(16) float in_order[kWaveSize];
     if (v.decision[0] == 0u || threadIdx.x >= kWaveSize)
         return;
     const uint32_t lane = threadIdx.x;
@@ -740,7 +741,7 @@ __global__ __launch_bounds__(kResidualThreads) void verify_draw_kernel(VerifySum
             entries[lane] = v.residual[first + lane];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
             __builtin_amdgcn_wave_barrier();
-            const WaveSum result = wave_add_terms<0>(entries, kResidualSub, sum, mode, bound, 1.0f, 1.0f);
+            const WaveSum result = wave_add_in_order<0>(entries, kResidualSub, sum, mode, bound, 1.0f, 1.0f, in_order);
             __builtin_amdgcn_wave_barrier();
             sum = result.sum;
             if (result.stopped)

@@ -58,3 +58,27 @@ def test_windows_over_many_neighbours(kind, dtype):
             params = hip_sampler.make_params(rows, 1.0, top_k, top_p, 0.0)
             cpu = parity_util.run_oracle(data, params, uniforms)
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, dtype, "%s top_k %d" % (kind, top_k))
+
+
+@pytest.mark.parametrize("spread,rounded", [(0.0, 0), (0.05, 0), (1.0, 0), (2.5, 0), (2.5, 16), (8.0, 0)])
+def test_sums_over_the_edges_of_their_chunks(spread, rounded):
+    """Windows that end at and next to the chunks of 64 terms, the 32 terms added at a time and the four terms of a lane, the draw and the Top-P
+    stop anywhere among them.  (spread 0.05: the sums leave a binade inside most chunks; 8: most terms are below half an ulp.)"""
+    rng = np.random.default_rng(int(spread * 100) + rounded)
+    windows = [65, 66, 95, 96, 97, 127, 128, 129, 130, 131, 132, 133, 191, 192, 193, 255, 256, 257, 320, 511, 512, 513, 575, 576, 577, 641, 1000, 1023, 1024]
+    rows, vocab = 4 * len(windows), 5003
+    print("[case] chunk edges, spread %g" % spread, flush=True)
+    logits = rng.standard_normal((rows, vocab)) * spread
+    if rounded:
+        logits = np.round(logits * rounded) / rounded
+    logits = (logits + np.linspace(0, 0.5, vocab) * (spread == 0.0)).astype(np.float32)
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["top_k"] = np.repeat(np.array(windows, dtype=np.uint32), 4)
+    params["top_p"] = rng.choice(np.array([1.0, 0.9999, 0.97, 0.6, 0.1], dtype=np.float32), rows)
+    params["min_p"][::5] = np.float32(0.02)
+    uniforms = rng.random(rows, dtype=np.float32)
+    uniforms[::7] = np.float32(1.0 - 2.0 ** -24)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "chunk edges, spread %g" % spread)
