@@ -420,21 +420,35 @@ struct BinScanScratch
     float f[kBinWaves];
 };
 
-__device__ __forceinline__ float wave_prefix_sum_f32(float value)
+// The inclusive sums over each row of 16 lanes, and over the wave.
+__device__ __forceinline__ uint32_t row16_prefix_sum_u32(uint32_t value)
 {
-#define NCNN_MOE_ADD_STAGE(CONTROL, ROW_MASK) value += __uint_as_float(dpp_source<CONTROL, ROW_MASK>(__float_as_uint(value)));
-    NCNN_MOE_ADD_STAGE(0x111, 0xf)
-    NCNN_MOE_ADD_STAGE(0x112, 0xf)
-    NCNN_MOE_ADD_STAGE(0x114, 0xf)
-    NCNN_MOE_ADD_STAGE(0x118, 0xf)
-    NCNN_MOE_ADD_STAGE(0x142, 0xa)
-    NCNN_MOE_ADD_STAGE(0x143, 0xc)
-#undef NCNN_MOE_ADD_STAGE
+    value += dpp_source<0x111, 0xf>(value); // row_shr:1
+    value += dpp_source<0x112, 0xf>(value); // row_shr:2
+    value += dpp_source<0x114, 0xf>(value); // row_shr:4
+    value += dpp_source<0x118, 0xf>(value); // row_shr:8
     return value;
 }
 
-template <int WAVES, int COUNT>
-__device__ __forceinline__ void bin_scan(uint32_t (&u)[COUNT], uint32_t (&totals)[COUNT], float& f, BinScanScratch& scratch, int tid)
+__device__ __forceinline__ float row16_prefix_sum_f32(float value)
+{
+    value += __uint_as_float(dpp_source<0x111, 0xf>(__float_as_uint(value)));
+    value += __uint_as_float(dpp_source<0x112, 0xf>(__float_as_uint(value)));
+    value += __uint_as_float(dpp_source<0x114, 0xf>(__float_as_uint(value)));
+    value += __uint_as_float(dpp_source<0x118, 0xf>(__float_as_uint(value)));
+    return value;
+}
+
+__device__ __forceinline__ float wave_prefix_sum_f32(float value)
+{
+    value = row16_prefix_sum_f32(value);
+    value += __uint_as_float(dpp_source<0x142, 0xa>(__float_as_uint(value)));
+    value += __uint_as_float(dpp_source<0x143, 0xc>(__float_as_uint(value)));
+    return value;
+}
+
+template <int WAVES, bool WITH_FLOAT, int COUNT>
+__device__ __forceinline__ void bin_scan_of(uint32_t (&u)[COUNT], uint32_t (&totals)[COUNT], float& f, BinScanScratch& scratch, int tid)
 {
     const int lane = tid & (kWaveSize - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -448,22 +462,39 @@ __device__ __forceinline__ void bin_scan(uint32_t (&u)[COUNT], uint32_t (&totals
         if (lane == kWaveSize - 1)
             scratch.u[i][wave] = inclusive[i];
     }
-    const float inclusive_f = wave_prefix_sum_f32(f);
-    if (lane == kWaveSize - 1)
+    const float inclusive_f = WITH_FLOAT ? wave_prefix_sum_f32(f) : 0.0f;
+    if (WITH_FLOAT && lane == kWaveSize - 1)
         scratch.f[wave] = inclusive_f;
     __syncthreads();
+    static_assert(WAVES <= 16, "the waves' sums lie in one row of lanes");
 #pragma unroll
     for (int i = 0; i < COUNT; ++i)
     {
-        const uint32_t through = wave_prefix_sum_u32(lane < WAVES ? scratch.u[i][lane] : 0u);
+        const uint32_t through = row16_prefix_sum_u32(lane < WAVES ? scratch.u[i][lane] : 0u);
         totals[i] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), WAVES - 1));
         const uint32_t before = wave > 0 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(through), wave - 1)) : 0u;
         u[i] = before + inclusive[i] - own[i];
     }
-    const float through = wave_prefix_sum_f32(lane < WAVES ? scratch.f[lane] : 0.0f);
-    const float before = wave > 0 ? read_lane(through, wave - 1) : 0.0f;
-    f = before + (inclusive_f - f);
+    if (WITH_FLOAT)
+    {
+        const float through = row16_prefix_sum_f32(lane < WAVES ? scratch.f[lane] : 0.0f);
+        const float before = wave > 0 ? read_lane(through, wave - 1) : 0.0f;
+        f = before + (inclusive_f - f);
+    }
     __syncthreads();
+}
+
+template <int WAVES, int COUNT>
+__device__ __forceinline__ void bin_scan(uint32_t (&u)[COUNT], uint32_t (&totals)[COUNT], float& f, BinScanScratch& scratch, int tid)
+{
+    bin_scan_of<WAVES, true>(u, totals, f, scratch, tid);
+}
+
+template <int WAVES, int COUNT>
+__device__ __forceinline__ void bin_scan(uint32_t (&u)[COUNT], uint32_t (&totals)[COUNT], BinScanScratch& scratch, int tid)
+{
+    float none = 0.0f;
+    bin_scan_of<WAVES, false>(u, totals, none, scratch, tid);
 }
 
 // The largest term that a bin can hold (the lower end of a bin is the upper end of the next).
@@ -772,8 +803,10 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
 #pragma unroll
             for (int j = 3; j >= 0; --j)
             {
+                // (where a bin's terms are kMaskedDifference binades below the sum, its masks tell how those half way are rounded, and
+                // few are: a sorted head would save the walk nothing)
                 const bool in_head = window_in_head ? front[j] < window
-                    : front[j + 1] <= kBinHead;
+                    : front[j + 1] <= kBinHead && bin_top(bin + j, shift) * static_cast<float>(1 << kMaskedDifference) >= mass[j];
                 if (!in_head && bin + j != 0u)
                     first_not = bin + j;
             }
@@ -801,8 +834,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         uint32_t listed[1] = {holds_bins ? plan.listed : 0u};
         {
             uint32_t totals[1];
-            float none = 0.0f;
-            bin_scan<kBinWaves>(listed, totals, none, scan, tid);
+            bin_scan<kBinWaves>(listed, totals, scan, tid);
         }
         uint32_t place[4];
         const uint32_t own_end = fit_plan(plan, front, head_count + listed[0], place);
@@ -985,6 +1017,7 @@ struct BinWalkShared
     uint32_t listed_end;
     int32_t token;
     uint32_t least_key, most_key, matches; // see token_of_equal
+    uint32_t many;                          // see order_elements
 };
 
 constexpr uint32_t kBinExtraPlace = kBinListCap;
@@ -999,95 +1032,148 @@ __device__ __forceinline__ float same_in_all(float value)
     return __uint_as_float(same_in_all(__float_as_uint(value)));
 }
 
+// How many places for each of `count` elements order_elements tells apart: two where the counters fit.
+__device__ __forceinline__ uint32_t fineness_of(uint32_t place, uint32_t count)
+{
+    return count <= 4u * kWalkThreads && (place & ~3u) + 2u * count + 8u <= kBinListCap + kBinExtraCap ? 2u : 1u;
+}
+
 // Puts `count` elements (thread i % kWalkThreads holds element i, its term and token in registers) in descending order of
-// their terms at terms[place ..], tokens[place ..].  `fine` is about where each belongs (0 .. count - 1, falling with the
+// their terms at terms[place ..], tokens[place ..].  `fine` is about where each belongs (0 .. fineness * count - 1, falling with the
 // term): elements of one `fine` are neighbours, few of them unless they are equal, and are ranked against each other.
-// The place where the tokens go counts the elements of each `fine` first.  Every thread calls it.
+// The place where the tokens go (and some behind it) counts the elements of each `fine` first.  Every thread calls it.
+// What bounds it: trips to LDS one behind the other (zero, count, front, place, rank, write).  A thread's elements make them
+// together, four at a time, and are told apart twice as finely as there are elements: one element behind the other, with as many
+// places as elements, 1,910 of them took 10,400 cycles, 5,200 in the ranking; so 6,300 and 2,400.
 template <uint32_t PER_THREAD>
 __device__ __forceinline__ void order_elements(
-    BinWalkShared& shared, uint32_t place, uint32_t count, const float (&own)[PER_THREAD], const uint32_t (&token)[PER_THREAD],
+    BinWalkShared& shared, uint32_t place, uint32_t count, uint32_t fineness, const float (&own)[PER_THREAD], const uint32_t (&token)[PER_THREAD],
     const uint32_t (&fine)[PER_THREAD], int tid)
 {
     constexpr uint32_t kMixed = 0x80000000u; // the elements of this `fine` are not all equal
-    uint32_t* const counters = shared.tokens + place;
+    constexpr uint32_t kMany = 16;           // ... which is looked at where so many have one `fine`
+    constexpr uint32_t kTogether = PER_THREAD < 4u ? PER_THREAD : 4u;
+    static_assert(PER_THREAD % kTogether == 0u, "a thread's elements are whole groups");
+    uint32_t* const counters = shared.tokens + (place & ~3u); // (16-byte aligned)
+    uint32_t* const tokens = shared.tokens + place;
     float* const terms = shared.terms + place;
-    uint32_t turn[PER_THREAD];
-    for (uint32_t i = tid; i < count; i += kWalkThreads)
-        counters[i] = 0u;
-    __syncthreads();
+    const uint32_t places = fineness * count;
+    uint32_t at[PER_THREAD], turn[PER_THREAD];
+    // calls f(k, whether the thread has a k-th element) for each k, those of four k behind each other without a branch between
+    const auto each_element = [&](auto f) {
 #pragma unroll
-    for (uint32_t k = 0; k < PER_THREAD; ++k)
-    {
-        if (k * kWalkThreads + tid < count)
+        for (uint32_t first = 0; first < PER_THREAD; first += kTogether)
+        {
+            if (first * kWalkThreads < count)
+            {
+#pragma unroll
+                for (uint32_t k = first; k < first + kTogether; ++k)
+                    f(k, k * kWalkThreads + tid < count);
+            }
+        }
+    };
+    for (uint32_t i = 4u * static_cast<uint32_t>(tid); i < places; i += 4u * kWalkThreads)
+        *reinterpret_cast<uint4*>(counters + i) = uint4{0u, 0u, 0u, 0u};
+    if (tid == 0)
+        shared.many = 0u;
+    __syncthreads();
+    each_element([&](uint32_t k, bool mine) {
+        turn[k] = 0u;
+        if (mine)
             turn[k] = atomicAdd(&counters[fine[k]], 1u);
+    });
+    {
+        uint32_t most = 0;
+        each_element([&](uint32_t k, bool) { most = max(most, turn[k]); });
+        if (most + 1u >= kMany)
+            shared.many = 1u;
     }
     __syncthreads();
+    const bool many = same_in_all(shared.many) != 0u;
     {
-        const uint32_t each = (count + kWalkThreads - 1u) / kWalkThreads;
-        const uint32_t first = tid * each;
-        uint32_t held[PER_THREAD];
-        uint32_t total[1] = {0u};
-#pragma unroll
-        for (uint32_t k = 0; k < PER_THREAD; ++k)
-        {
-            held[k] = k < each && first + k < count ? counters[first + k] : 0u;
-            total[0] += held[k];
-        }
+        // (four counters a thread, eight where that is not enough)
+        const uint32_t groups = places <= 4u * kWalkThreads ? 1u : 2u;
+        static_assert(PER_THREAD <= 8u, "two groups of four counters a thread");
+        const uint32_t first = 4u * groups * static_cast<uint32_t>(tid);
+        uint4 held[2] = {uint4{0u, 0u, 0u, 0u}, uint4{0u, 0u, 0u, 0u}};
+        if (first < places)
+            held[0] = *reinterpret_cast<const uint4*>(counters + first);
+        if (groups == 2u && first + 4u < places)
+            held[1] = *reinterpret_cast<const uint4*>(counters + first + 4u);
+        const uint32_t of_first = held[0].x + held[0].y + held[0].z + held[0].w;
+        uint32_t total[1] = {of_first + held[1].x + held[1].y + held[1].z + held[1].w};
         uint32_t totals[1];
-        float none = 0.0f;
-        bin_scan<kWalkWaves>(total, totals, none, shared.scan, tid);
-        uint32_t front = total[0];
-#pragma unroll
-        for (uint32_t k = 0; k < PER_THREAD; ++k)
-        {
-            if (k < each && first + k < count)
-                counters[first + k] = front;
-            front += held[k];
-        }
+        bin_scan<kWalkWaves>(total, totals, shared.scan, tid);
+        const auto fronts_of = [](uint32_t front, const uint4& v) { return uint4{front, front + v.x, front + v.x + v.y, front + v.x + v.y + v.z}; };
+        if (first < places)
+            *reinterpret_cast<uint4*>(counters + first) = fronts_of(total[0], held[0]);
+        if (groups == 2u && first + 4u < places)
+            *reinterpret_cast<uint4*>(counters + first + 4u) = fronts_of(total[0] + of_first, held[1]);
     }
     __syncthreads();
-    uint32_t at[PER_THREAD];
-#pragma unroll
-    for (uint32_t k = 0; k < PER_THREAD; ++k)
-    {
-        at[k] = 0u;
-        if (k * kWalkThreads + tid < count)
-        {
-            at[k] = counters[fine[k]] + turn[k];
+    uint32_t low[PER_THREAD], length[PER_THREAD];
+    each_element([&](uint32_t k, bool) {
+        low[k] = counters[fine[k]];
+        length[k] = counters[min(fine[k] + 1u, places - 1u)];
+    });
+    each_element([&](uint32_t k, bool mine) {
+        length[k] = mine ? (fine[k] + 1u < places ? length[k] : count) - low[k] : 0u;
+        at[k] = low[k] + turn[k];
+        if (mine)
             terms[at[k]] = own[k];
-        }
-    }
+    });
     __syncthreads();
-#pragma unroll
-    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    if (many)
     {
-        if (k * kWalkThreads + tid < count && terms[at[k] - turn[k]] != own[k])
-            atomicOr(&counters[fine[k]], kMixed);
+        // (thousands of equal elements are not ranked against each other)
+        each_element([&](uint32_t k, bool mine) {
+            if (mine && terms[low[k]] != own[k])
+                atomicOr(&counters[fine[k]], kMixed);
+        });
+        __syncthreads();
+        each_element([&](uint32_t k, bool mine) { length[k] = mine && (counters[fine[k]] & kMixed) != 0u ? length[k] : 0u; });
     }
-    __syncthreads();
 #pragma unroll
-    for (uint32_t k = 0; k < PER_THREAD; ++k)
+    for (uint32_t first = 0; first < PER_THREAD; first += kTogether)
     {
-        if (k * kWalkThreads + tid < count && (counters[fine[k]] & kMixed) != 0u)
+        if (first * kWalkThreads >= count)
+            break;
+        uint32_t longest = 0;
+#pragma unroll
+        for (uint32_t k = first; k < first + kTogether; ++k)
         {
-            const uint32_t low = at[k] - turn[k];
-            const uint32_t high = fine[k] + 1u < count ? counters[fine[k] + 1u] & ~kMixed : count;
-            uint32_t rank = low;
-            for (uint32_t j = low; j < high; ++j)
-                rank += terms[j] > own[k] || (terms[j] == own[k] && j < at[k]) ? 1u : 0u;
-            at[k] = rank;
+            length[k] = length[k] > 1u ? length[k] : 0u;
+            at[k] = length[k] != 0u ? low[k] : at[k];
+            longest = max(longest, length[k]);
+        }
+        for (uint32_t t = 0; __builtin_amdgcn_ballot_w64(t < longest) != 0ull; t += 2u)
+        {
+            float other[2][kTogether];
+#pragma unroll
+            for (uint32_t i = 0; i < kTogether; ++i)
+            {
+                // (behind the group's last element: any, which is left out below)
+                other[0][i] = terms[t < length[first + i] ? low[first + i] + t : 0u];
+                other[1][i] = terms[t + 1u < length[first + i] ? low[first + i] + t + 1u : 0u];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kTogether; ++i)
+            {
+                const uint32_t k = first + i;
+                // (as numbers the terms are ordered like their bits, and an equal one counts where its turn is the earlier)
+                at[k] += t < length[k] && __float_as_uint(other[0][i]) >= __float_as_uint(own[k]) + (t < turn[k] ? 0u : 1u) ? 1u : 0u;
+                at[k] += t + 1u < length[k] && __float_as_uint(other[1][i]) >= __float_as_uint(own[k]) + (t + 1u < turn[k] ? 0u : 1u) ? 1u : 0u;
+            }
         }
     }
     __syncthreads();
-#pragma unroll
-    for (uint32_t k = 0; k < PER_THREAD; ++k)
-    {
-        if (k * kWalkThreads + tid < count)
+    each_element([&](uint32_t k, bool mine) {
+        if (mine)
         {
             terms[at[k]] = own[k];
-            counters[at[k]] = token[k];
+            tokens[at[k]] = token[k];
         }
-    }
+    });
     __syncthreads();
 }
 
@@ -1189,7 +1275,8 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     if (count <= kBinExtraCap)
     {
         constexpr uint32_t kPerThread = (kBinExtraCap + kWalkThreads - 1) / kWalkThreads;
-        const float places_per_bit = static_cast<float>(count) / static_cast<float>(width);
+        const uint32_t fineness = fineness_of(kBinExtraPlace, count);
+        const float places_per_bit = static_cast<float>(fineness * count) / static_cast<float>(width);
         float own[kPerThread];
         uint32_t token[kPerThread], fine[kPerThread];
 #pragma unroll
@@ -1203,22 +1290,12 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
                 own[k] = shared.terms[kBinExtraPlace + i];
                 token[k] = shared.tokens[kBinExtraPlace + i];
                 // (rounded, but never falling where the term falls)
-                fine[k] = min(static_cast<uint32_t>(static_cast<float>(top - __float_as_uint(own[k])) * places_per_bit), count - 1u);
+                fine[k] = min(static_cast<uint32_t>(static_cast<float>(top - __float_as_uint(own[k])) * places_per_bit), fineness * count - 1u);
             }
         }
         __syncthreads();
-        order_elements<kPerThread>(shared, kBinExtraPlace, count, own, token, fine, tid);
+        order_elements<kPerThread>(shared, kBinExtraPlace, count, fineness, own, token, fine, tid);
     }
-}
-
-// The inclusive sums over each row of 16 lanes.
-__device__ __forceinline__ uint32_t row16_prefix_sum_u32(uint32_t value)
-{
-    value += dpp_source<0x111, 0xf>(value); // row_shr:1
-    value += dpp_source<0x112, 0xf>(value); // row_shr:2
-    value += dpp_source<0x114, 0xf>(value); // row_shr:4
-    value += dpp_source<0x118, 0xf>(value); // row_shr:8
-    return value;
 }
 
 // The plain sum of each 64 of `count` terms (4096 at most): a row of 16 lanes holds 64 terms, a lane four of them.
@@ -1228,13 +1305,7 @@ __device__ __forceinline__ void sum_chunks(HeadScratch& scratch, const float* te
     for (uint32_t i = 4u * static_cast<uint32_t>(tid); same_in_all(i) < count; i += 4u * WAVES * kWaveSize)
     {
         const float4 own = *reinterpret_cast<const float4*>(terms + i);
-        float sum = ((i < count ? own.x : 0.0f) + (i + 1u < count ? own.y : 0.0f)) + ((i + 2u < count ? own.z : 0.0f) + (i + 3u < count ? own.w : 0.0f));
-#define NCNN_MOE_ADD_STAGE(CONTROL) sum += __uint_as_float(dpp_source<CONTROL, 0xf>(__float_as_uint(sum)));
-        NCNN_MOE_ADD_STAGE(0x111)
-        NCNN_MOE_ADD_STAGE(0x112)
-        NCNN_MOE_ADD_STAGE(0x114)
-        NCNN_MOE_ADD_STAGE(0x118)
-#undef NCNN_MOE_ADD_STAGE
+        const float sum = row16_prefix_sum_f32(((i < count ? own.x : 0.0f) + (i + 1u < count ? own.y : 0.0f)) + ((i + 2u < count ? own.z : 0.0f) + (i + 3u < count ? own.w : 0.0f)));
         if ((tid & 15) == 15)
             scratch.chunk_sum[i / kWaveSize] = sum;
     }
@@ -2112,6 +2183,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             }
             // ---- the listed elements in order: a bin's elements lie side by side in the list
             __syncthreads();
+            const uint32_t fineness = fineness_of(list_first, listed - list_first);
             uint32_t fine[kPerThread];
 #pragma unroll
             for (uint32_t k = 0; k < kPerThread; ++k)
@@ -2120,10 +2192,18 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 if (list_first + k * kWalkThreads + tid < listed)
                 {
                     const uint32_t b = (kOneBits - __float_as_uint(own_terms[k])) >> shift;
-                    fine[k] = shared.places[b] - list_first + fine_place(own_terms[k], shift, packed_front(shared.packed[b + 1u]) - packed_front(shared.packed[b]));
+                    fine[k] = fineness * (shared.places[b] - list_first) +
+                        fine_place(own_terms[k], shift, fineness * (packed_front(shared.packed[b + 1u]) - packed_front(shared.packed[b])));
                 }
             }
-            order_elements<kPerThread>(shared, list_first, listed - list_first, own_terms, own_tokens, fine, tid);
+            if (WALK > 0 && listed - list_first <= kWalkThreads)
+            {
+                const float first_term[1] = {own_terms[0]};
+                const uint32_t first_token[1] = {own_tokens[0]}, first_fine[1] = {fine[0]};
+                order_elements<1>(shared, list_first, listed - list_first, fineness, first_term, first_token, first_fine, tid);
+            }
+            else
+                order_elements<kPerThread>(shared, list_first, listed - list_first, fineness, own_terms, own_tokens, fine, tid);
         }
         if (shared.status == 2u)
         {
@@ -2350,8 +2430,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             uint32_t to_list[1] = {holds_bins ? plan.listed : 0u};
             {
                 uint32_t totals[1];
-                float none = 0.0f;
-                bin_scan<kWalkWaves>(to_list, totals, none, shared.scan, tid);
+                bin_scan<kWalkWaves>(to_list, totals, shared.scan, tid);
             }
             uint32_t place[4];
             const uint32_t own_end = fit_plan(plan, front, head_count + to_list[0], place);

@@ -438,8 +438,7 @@ __device__ __forceinline__ void window_finish(const WindowArgs& g, uint32_t row,
             total[0] += held[k];
         }
         uint32_t totals[1];
-        float none = 0.0f;
-        bin_scan<WAVES>(total, totals, none, shared.scan, tid);
+        bin_scan<WAVES>(total, totals, shared.scan, tid);
         uint32_t front = total[0];
 #pragma unroll
         for (uint32_t k = 0; k < kPerThread; ++k)
