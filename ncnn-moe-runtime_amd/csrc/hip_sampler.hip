@@ -441,10 +441,7 @@ int launch_sampler(
         if (passes.full_order)
         {
             if (dtype == NCNN_MOE_LOGITS_F32)
-            {
-                hipLaunchKernelGGL((general_sort_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kSortThreads), 0, stream, a);
-                hipLaunchKernelGGL((general_replay_kernel<NCNN_MOE_LOGITS_F32, false>), dim3(rows), dim3(kReplayThreads), 0, stream, a);
-            }
+                launch_sort_and_replay(a, stream);
             else
                 hipLaunchKernelGGL(bf16_counting_replay_kernel, dim3(rows), dim3(kSortThreads), 0, stream, a);
         }

@@ -66,7 +66,7 @@ constexpr int kReplayChunk = kSumThreads * kReplayPerThread;
 #ifdef NCNN_MOE_TIMELINE
 constexpr int kTimelineRows = 64;
 constexpr int kTimelineSlots = 16;
-__device__ unsigned long long g_timeline[kTimelineRows * kMaxSegments * kTimelineSlots];
+static __device__ unsigned long long g_timeline[kTimelineRows * kMaxSegments * kTimelineSlots];
 #define NCNN_MOE_STAMP(row, segment, slot)                                                                   \
     do                                                                                                       \
     {                                                                                                        \
@@ -80,7 +80,7 @@ __device__ unsigned long long g_timeline[kTimelineRows * kMaxSegments * kTimelin
             g_timeline[((row) * kMaxSegments + (segment)) * kTimelineSlots + (slot)] = (value);              \
     } while (0)
 // stamps of the row's last workgroup, from code that does not know its segment; the calling lane is that wave's first
-__device__ unsigned long long g_timeline_rows[kTimelineRows * kTimelineSlots];
+static __device__ unsigned long long g_timeline_rows[kTimelineRows * kTimelineSlots];
 #define NCNN_MOE_STAMP_ROW(row, slot)                                                                        \
     do                                                                                                       \
     {                                                                                                        \

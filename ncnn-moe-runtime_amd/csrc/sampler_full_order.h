@@ -90,7 +90,7 @@ __device__ __forceinline__ void list_full_order_rows(const SamplerArgs& a, uint3
         list[0] = listed;
 }
 
-__global__ __launch_bounds__(kSortThreads) void full_order_row_list_kernel(SamplerArgs a, uint32_t rows, uint32_t* list)
+[[maybe_unused]] static __global__ __launch_bounds__(kSortThreads) void full_order_row_list_kernel(SamplerArgs a, uint32_t rows, uint32_t* list)
 {
     list_full_order_rows(a, rows, list);
 }
@@ -116,7 +116,7 @@ constexpr int kCutStride = kCutBuckets + 1;     // (the copies of a counter lie 
 constexpr uint32_t kCutSample = 4096;           // 16-byte groups of the row that are looked at
 constexpr float kCutMinimum = 4096.0f;          // rows are not cut shorter than about this
 
-__global__ __launch_bounds__(kSortThreads) void full_order_cut_kernel(SamplerArgs a)
+[[maybe_unused]] static __global__ __launch_bounds__(kSortThreads) void full_order_cut_kernel(SamplerArgs a)
 {
     static_assert(kCutSample == 4u * kSortThreads && kCutBuckets == 4 * kSortThreads, "four loads and four buckets a thread");
     const uint32_t row = blockIdx.x;
@@ -314,14 +314,10 @@ __device__ __forceinline__ float load_logit<NCNN_MOE_LOGITS_BF16>(const void* ro
 // sort_indices[1] (needed only when the whole filtered distribution is exported); sampling sorts the
 // keys alone and recovers the one index it needs from the logits afterwards.
 template <int DTYPE, bool PAIRS>
-__global__ __launch_bounds__(kSortThreads) void general_sort_kernel(SamplerArgs a)
+__device__ __forceinline__ void sort_whole_row(const SamplerArgs& a, uint32_t row, int tid)
 {
     constexpr int kPasses = DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2;
     constexpr int kFirstDigit = DTYPE == NCNN_MOE_LOGITS_F32 ? 0 : 2;
-    const uint32_t row = blockIdx.x;
-    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
-        return;
-    const int tid = threadIdx.x;
     const int lane = tid & (kWaveSize - 1);
     const int wave = tid >> 6;
     const uint32_t n = a.vocab;
@@ -537,6 +533,15 @@ __global__ __launch_bounds__(kSortThreads) void general_sort_kernel(SamplerArgs 
         __threadfence_block();
         __syncthreads();
     }
+}
+
+template <int DTYPE, bool PAIRS>
+__global__ __launch_bounds__(kSortThreads) void general_sort_kernel(SamplerArgs a)
+{
+    const uint32_t row = blockIdx.x;
+    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
+        return;
+    sort_whole_row<DTYPE, PAIRS>(a, row, threadIdx.x);
 }
 
 // ---- the same sort with a row spread over several workgroups.  A batch rarely holds more full-order
@@ -1203,7 +1208,7 @@ __device__ __forceinline__ bool write_runs_of_counts(
     return true;
 }
 
-__global__ __launch_bounds__(kSortThreads) void bf16_counting_sort_kernel(SamplerArgs a)
+[[maybe_unused]] static __global__ __launch_bounds__(kSortThreads) void bf16_counting_sort_kernel(SamplerArgs a)
 {
     const uint32_t row = blockIdx.x;
     if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
@@ -1586,12 +1591,8 @@ __device__ __forceinline__ void replay_row(
 }
 
 template <int DTYPE, bool RUNS>
-__global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerArgs a)
+__device__ __forceinline__ void replay_sorted_row(const SamplerArgs& a, uint32_t row, int tid)
 {
-    const uint32_t row = blockIdx.x;
-    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
-        return;
-    const int tid = threadIdx.x;
     NCNN_MOE_STAMP(blockIdx.x, 15, 0);
     const ncnn_moe_sample_params p = a.params[row];
     const uint32_t* keys = a.sort_keys[1] + row * a.sort_stride;
@@ -1665,6 +1666,15 @@ __global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerA
     replay_row<DTYPE, RUNS>(a, row, p, keys, run_ends, run_total_of_row, terms0, tid);
 }
 
+template <int DTYPE, bool RUNS>
+__global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerArgs a)
+{
+    const uint32_t row = blockIdx.x;
+    if (a.row_state[row] != kRowNeedsGeneral || left_to_the_wide_select(a, row))
+        return;
+    replay_sorted_row<DTYPE, RUNS>(a, row, threadIdx.x);
+}
+
 // bf16 full-order rows in ONE kernel: bf16_counting_sort_kernel and general_replay_kernel<BF16, runs> back to
 // back in one workgroup per row, which both are.  The runs never leave the compute unit: once every counter
 // sits in a register they are written over the counters themselves (keys, ends and, behind them, the terms: a
@@ -1673,7 +1683,7 @@ __global__ __launch_bounds__(kReplayThreads) void general_replay_kernel(SamplerA
 // kernels do, and walks them from there.
 constexpr uint32_t kRunsInPlace = (kCountWords / 3) & ~3u; // 10,920 runs with their ends and terms in the counters' LDS (each array on a 16-byte boundary)
 
-__global__ __launch_bounds__(kSortThreads) void bf16_counting_replay_kernel(SamplerArgs a)
+[[maybe_unused]] static __global__ __launch_bounds__(kSortThreads) void bf16_counting_replay_kernel(SamplerArgs a)
 {
     static_assert(kSortThreads == kReplayThreads, "the count and the walk share a workgroup");
     const uint32_t row = blockIdx.x;
@@ -1865,7 +1875,7 @@ __device__ __forceinline__ uint32_t touched_up_place_of_long_group(const uint32_
     return i - belong_behind + belong_in_front;
 }
 
-__global__ __launch_bounds__(kTermsThreads) void full_order_terms_kernel(SamplerArgs a)
+[[maybe_unused]] static __global__ __launch_bounds__(kTermsThreads) void full_order_terms_kernel(SamplerArgs a)
 {
     uint32_t row;
     if (!spread_grid_row(a, row))
@@ -2015,7 +2025,7 @@ __global__ __launch_bounds__(kTermsThreads) void full_order_terms_kernel(Sampler
 constexpr int kChunkStepThreads = 256;
 constexpr int kChunkStepPerThread = kReplayChunk / kChunkStepThreads;
 
-__global__ __launch_bounds__(kChunkStepThreads) void full_order_chunk_steps_kernel(SamplerArgs a)
+[[maybe_unused]] static __global__ __launch_bounds__(kChunkStepThreads) void full_order_chunk_steps_kernel(SamplerArgs a)
 {
     static_assert(kChunkStepPerThread * kChunkStepThreads == kReplayChunk && kChunkStepPerThread % 4 == 0, "float4 loads over a whole chunk");
     static_assert(kReplayChunk % (kTermsThreads * kTermsPerThread) == 0, "a chunk is a whole number of the terms kernel's blocks");

@@ -20,6 +20,9 @@
 
 namespace ncnn_moe_hip {
 
+// hip_leftover_rows.hip: fp32 rows that the windows' and sums' kernels have left pending, sorted and replayed
+void launch_sort_and_replay(const SamplerArgs& a, hipStream_t stream);
+
 #ifdef NCNN_MOE_TESTING
 // Evaluates expf_libm on n values (test hook; in the testing build of the library only).
 __global__ void expf_probe_kernel(const float* in, float* out, size_t n)
