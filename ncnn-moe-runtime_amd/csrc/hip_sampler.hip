@@ -300,13 +300,15 @@ void launch_bin_walks(const BinArgs& g, hipStream_t stream)
     hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
 }
 
-// The window kernels (sampler_windows.h) over the rows in the handle's window list.
+// The window kernels (sampler_windows.h) over the rows in the handle's window list (`other_list`: see list_rows_in_place).
 template <int DTYPE>
-void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, hipStream_t stream)
+void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, uint32_t* other_list, hipStream_t stream)
 {
     WindowArgs w = s->windows;
     w.a = a;
     w.windows_are_selects = 1u;
+    w.listing = listing;
+    w.other_list = other_list;
     hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
     hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
 }
@@ -314,12 +316,13 @@ void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, hipStream_t s
 // The binned sums (sampler_bins.h) over the rows in the handle's bin list; the walks, which finish rows, wait for
 // `before_walks` (null: for nothing).
 template <int DTYPE>
-hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, bool windows, bool want_filters, hipEvent_t before_walks, hipStream_t stream)
+hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t before_walks, hipStream_t stream)
 {
     BinArgs g = s->bins;
     g.a = a;
     g.windows_are_selects = windows ? 1u : 0u;
     g.want_filters = want_filters ? 1u : 0u;
+    g.listing = listing;
     hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
     hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
     hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
@@ -341,9 +344,12 @@ template <int DTYPE>
 hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
                             bool want_filters, hipStream_t stream)
 {
+    const bool in_place = a.rows <= kRowsListedInPlace;
+    const RowListing listing = !in_place ? kRowsListed : side_by_side ? kRowsByOptions : kRowsByState;
     const auto list_rows = [&]() {
-        hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, side_by_side ? 1u : 0u,
-                           windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
+        if (!in_place)
+            hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, side_by_side ? 1u : 0u,
+                               windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
     };
     const auto select = [&](hipStream_t on) { launch_select<DTYPE>(geometry, a.rows, on, a, 0, s->scatter_segments != 0); };
     if (side_by_side && windows && sums && s->side_stream != nullptr)
@@ -356,17 +362,17 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
             return result;
         select(s->side_stream);
         result = hipEventRecord(s->cut_done, s->side_stream);
-        launch_windows<DTYPE>(s, a, s->side_stream);
+        launch_windows<DTYPE>(s, a, listing, nullptr, s->side_stream);
         const hipError_t joins = hipEventRecord(s->side_join, s->side_stream);
-        const hipError_t waits = launch_bin_sums<DTYPE>(s, a, windows, want_filters, s->cut_done, stream);
+        const hipError_t waits = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, s->cut_done, stream);
         const hipError_t joined = hipStreamWaitEvent(stream, s->side_join, 0);
         return result != hipSuccess ? result : joins != hipSuccess ? joins : waits != hipSuccess ? waits : joined;
     }
     select(stream);
     list_rows();
     if (windows)
-        launch_windows<DTYPE>(s, a, stream);
-    return sums ? launch_bin_sums<DTYPE>(s, a, windows, want_filters, nullptr, stream) : hipSuccess;
+        launch_windows<DTYPE>(s, a, listing, sums ? s->bin_list : nullptr, stream);
+    return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, windows, want_filters, nullptr, stream) : hipSuccess;
 }
 
 // Enqueues the sampling path for `rows` rows.  want_filters: the rows without a window leave their filtered distributions

@@ -134,7 +134,7 @@ struct BinRow
 struct BinArgs
 {
     SamplerArgs a;
-    const uint32_t* list;  // the rows served: [0] their number, then the rows
+    uint32_t* list;        // the rows served: [0] their number, then the rows
     uint4* stats;          // [pairs] (row, part): largest and smallest finite logit, finite logits, flags
     uint32_t* counts;      // [pairs][2][kBins]: terms in each bin, and the sum of their places in it (kOffsetBits)
     uint32_t* steps[2];    // [pairs][kBins], of alternate launches
@@ -148,7 +148,106 @@ struct BinArgs
     BinRow* records;       // [rows]
     uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
+    uint32_t listing;      // RowListing: how the first launch finds its rows
 };
+
+__device__ __forceinline__ uint32_t same_in_all(uint32_t value)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(value)));
+}
+
+__device__ __forceinline__ float same_in_all(float value)
+{
+    return __uint_as_float(same_in_all(__float_as_uint(value)));
+}
+
+// The rows that the first select leaves, those with a window of the window kernels' widths apart from the others.
+enum RowListing : uint32_t
+{
+    kRowsListed = 0,    // a launch of its own has listed them
+    kRowsByState = 1,   // the first select has run: the rows that it left pending
+    kRowsByOptions = 2  // ... runs beside: the rows whose options say so
+};
+
+__device__ __forceinline__ bool row_is_left(const SamplerArgs& a, uint32_t row, bool by_options, bool windows_apart, bool& window)
+{
+    uint32_t effective_k = 0;
+    int status = NCNN_MOE_ROW_OK;
+    const int mode = resolve_row_mode(a.params[row], a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
+    window = windows_apart && effective_k <= static_cast<uint32_t>(kSelectTopK);
+    return by_options ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && a.row_state[row] == kRowNeedsGeneral;
+}
+
+// A call of no more rows than a workgroup has threads needs no launch that lists them: every workgroup of the first launch that
+// wants the list works it out for itself (1.6 us more than reading it, where the launch took 3.0 us with the gap in front of it),
+// and one writes it down for the launches behind.
+constexpr uint32_t kRowsListedInPlace = kBinThreads;
+
+struct RowList
+{
+    uint32_t wave_totals[kBinWaves];
+    uint16_t rows[kRowsListedInPlace];
+};
+
+// How many rows there are; they are list[1 ..] where listing is kRowsListed, else shared.rows.  `others` (null: nowhere): the rows of
+// the other kind are listed there for a later launch.
+__device__ __forceinline__ uint32_t list_rows_in_place(
+    const SamplerArgs& a, uint32_t listing, bool windows_apart, bool want_windows, uint32_t* list, uint32_t* others, RowList& shared, int tid)
+{
+    if (listing == kRowsListed)
+        return list[0];
+    const int wave = tid >> 6;
+    const uint32_t row = static_cast<uint32_t>(tid);
+    bool left = false, window = false;
+    if (row < a.rows)
+        left = row_is_left(a, row, listing == kRowsByOptions, windows_apart, window);
+    // where a row stands among those for which `mine` holds, and their number
+    const auto place_of = [&](bool mine, uint32_t& total) {
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(mine);
+        if ((tid & (kWaveSize - 1)) == 0)
+            shared.wave_totals[wave] = static_cast<uint32_t>(__popcll(mask));
+        __syncthreads();
+        uint32_t before = 0;
+        total = 0;
+#pragma unroll
+        for (int w = 0; w < kBinWaves; ++w)
+        {
+            before += w < wave ? shared.wave_totals[w] : 0u;
+            total += shared.wave_totals[w];
+        }
+        return before + static_cast<uint32_t>(lanes_below(mask));
+    };
+    uint32_t rows = 0;
+    const bool mine = left && window == want_windows;
+    const uint32_t place = place_of(mine, rows);
+    if (mine)
+        shared.rows[place] = static_cast<uint16_t>(row);
+    if (blockIdx.x == 0u)
+    {
+        if (mine)
+            list[1u + place] = row;
+        if (tid == 0)
+            list[0] = rows;
+        if (others != nullptr)
+        {
+            __syncthreads();
+            uint32_t other_rows = 0;
+            const bool other = left && window != want_windows;
+            const uint32_t other_place = place_of(other, other_rows);
+            if (other)
+                others[1u + other_place] = row;
+            if (tid == 0)
+                others[0] = other_rows;
+        }
+    }
+    __syncthreads();
+    return rows;
+}
+
+__device__ __forceinline__ uint32_t row_of_slot(uint32_t listing, const uint32_t* list, const RowList& shared, uint32_t slot)
+{
+    return listing == kRowsListed ? list[1u + slot] : shared.rows[slot];
+}
 
 // How a launch's workgroups cover the listed rows: all parts of a row on one XCD (workgroups are dealt out to the XCDs
 // in turn), so that what one launch leaves of a row is found in that XCD's L2 by the next.
@@ -157,10 +256,10 @@ struct BinGrid
     uint32_t rows, parts, first_slot, slot_step, part;
 };
 
-__device__ __forceinline__ BinGrid bin_grid(const uint32_t* list, uint32_t vocab)
+__device__ __forceinline__ BinGrid bin_grid(uint32_t rows, uint32_t vocab)
 {
     BinGrid r;
-    r.rows = list[0];
+    r.rows = rows;
     const uint32_t per_xcd = kBinGrid / 8u;
     const uint32_t slots_per_xcd = max(1u, (r.rows + 7u) / 8u);
     const uint32_t most = min(kMaxBinParts, (vocab + kBinPartElements - 1u) / kBinPartElements);
@@ -218,11 +317,13 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
     constexpr int kLoads = 4;
     __shared__ uint4 wave_stats[kBinWaves];
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    __shared__ RowList listed_rows;
     const int tid = threadIdx.x;
+    const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, nullptr, listed_rows, tid);
+    const BinGrid grid = bin_grid(rows, a.vocab);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
-        const uint32_t row = g.list[1u + slot];
+        const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
         const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
         const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
             static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
@@ -310,7 +411,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
     __shared__ uint4 part_stats[kMaxBinParts];
     __shared__ uint64_t exp2_table[32];
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
     const int tid = threadIdx.x;
     if (tid < 32)
         exp2_table[tid] = kExp2Table[tid];
@@ -675,7 +776,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
     __shared__ BinScanScratch scan;
     __shared__ uint32_t head_bins_of_row, head_count_of_row, end_of_list;
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
     const int tid = threadIdx.x;
     const uint32_t bin = 4u * static_cast<uint32_t>(tid);
     const bool holds_bins = tid < static_cast<int>(kBinQuads);
@@ -1021,16 +1122,6 @@ struct BinWalkShared
 };
 
 constexpr uint32_t kBinExtraPlace = kBinListCap;
-
-__device__ __forceinline__ uint32_t same_in_all(uint32_t value)
-{
-    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(value)));
-}
-
-__device__ __forceinline__ float same_in_all(float value)
-{
-    return __uint_as_float(same_in_all(__float_as_uint(value)));
-}
 
 // How many places for each of `count` elements order_elements tells apart: two where the counters fit.
 __device__ __forceinline__ uint32_t fineness_of(uint32_t place, uint32_t count)
@@ -1898,7 +1989,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
     constexpr int kFrom = WALK & 1;      // which of the alternating buffers this launch reads
     constexpr int kTo = kFrom ^ 1;
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list, g.a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
     const int tid = threadIdx.x;
     const uint32_t bin = 4u * static_cast<uint32_t>(tid);
     const bool holds_bins = tid < static_cast<int>(kBinQuads);
@@ -2506,8 +2597,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
     }
 }
 
-// Lists the rows that the first select leaves (by_options: by their options, else those that it left pending): those with
-// a window of the window kernels' widths (null: nowhere), and the others.  One workgroup.
+// Lists the rows that the first select leaves, those with a window (null: nowhere) and the others, for a call of more rows than
+// kRowsListedInPlace.  One workgroup.
 __global__ __launch_bounds__(kBinThreads) void later_rows_list_kernel(SamplerArgs a, uint32_t by_options, uint32_t* windows, uint32_t* others)
 {
     __shared__ uint32_t wave_totals[2][kBinWaves];
@@ -2520,11 +2611,8 @@ __global__ __launch_bounds__(kBinThreads) void later_rows_list_kernel(SamplerArg
         bool mine[2] = {false, false};
         if (row < a.rows)
         {
-            uint32_t effective_k = 0;
-            int status = NCNN_MOE_ROW_OK;
-            const int mode = resolve_row_mode(a.params[row], a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
-            const bool left = by_options != 0u ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && a.row_state[row] == kRowNeedsGeneral;
-            const bool window = windows != nullptr && effective_k <= static_cast<uint32_t>(kSelectTopK);
+            bool window = false;
+            const bool left = row_is_left(a, row, by_options != 0u, windows != nullptr, window);
             mine[0] = left && window;
             mine[1] = left && !window;
         }

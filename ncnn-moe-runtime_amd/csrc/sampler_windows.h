@@ -32,12 +32,14 @@ constexpr uint32_t kWindowBins = 4096;           // of the sample's histogram: t
 struct WindowArgs
 {
     SamplerArgs a;
-    const uint32_t* list;   // the rows served: [0] their number, then the rows
+    uint32_t* list;         // the rows served: [0] their number, then the rows
     uint32_t* counts;       // [rows] candidates; zero when a launch begins (window_finish returns them to zero)
     uint32_t* flags;        // [rows] kWindowSawNan, kWindowHasAll; the same
     uint32_t* keys;         // [rows][kWindowListCap]
     uint32_t* tokens;       // [rows][kWindowListCap]
     uint32_t windows_are_selects; // as in BinArgs
+    uint32_t listing;
+    uint32_t* other_list;   // where the sums' rows are listed as well (null: nowhere)
 };
 
 struct WindowCandidatesShared
@@ -86,7 +88,7 @@ __device__ __forceinline__ void find_from_top(WindowCandidatesShared& shared, ui
 }
 
 template <int DTYPE>
-__device__ __forceinline__ void window_candidates(const WindowArgs& g, const BinGrid& grid, WindowCandidatesShared& shared, int tid)
+__device__ __forceinline__ void window_candidates(const WindowArgs& g, const BinGrid& grid, const RowList& listed_rows, WindowCandidatesShared& shared, int tid)
 {
     using Vector = LogitsVector<DTYPE>;
     constexpr uint32_t kWidth = Vector::kWidth;
@@ -95,7 +97,7 @@ __device__ __forceinline__ void window_candidates(const WindowArgs& g, const Bin
     const int lane = tid & (kWaveSize - 1);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
-        const uint32_t row = same_in_all(g.list[1u + slot]);
+        const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
         const uint32_t top_k = same_in_all(a.params[row].top_k);
         const uint32_t window = top_k == 0u || top_k >= a.vocab ? a.vocab : top_k;
         const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
@@ -525,7 +527,9 @@ template <int DTYPE>
 __global__ __launch_bounds__(kBinThreads, 8) void window_candidates_kernel(WindowArgs g)
 {
     __shared__ WindowCandidatesShared shared;
-    window_candidates<DTYPE>(g, bin_grid(g.list, g.a.vocab), shared, threadIdx.x);
+    __shared__ RowList listed_rows;
+    const uint32_t rows = list_rows_in_place(g.a, g.listing, true, true, g.list, g.other_list, listed_rows, threadIdx.x);
+    window_candidates<DTYPE>(g, bin_grid(rows, g.a.vocab), listed_rows, shared, threadIdx.x);
 }
 
 template <int DTYPE>

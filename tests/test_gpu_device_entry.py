@@ -172,3 +172,26 @@ def test_rejected_rows_side_by_side():
             beside = _run(sampler, logits, params, uniforms, hip_sampler.PASSES_FULL_ORDER | hip_sampler.PASSES_SIDE_BY_SIDE, stream)
             parity_util.assert_results_match(beside, cpu, "f32", "rejected rows, device entry")
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "rejected rows, host entry")
+
+
+@pytest.mark.parametrize("rows", [1, 63, 65, 1023, 1024, 1025, 2050])
+def test_rows_listed_by_the_first_launch_or_by_one_of_their_own(rows):
+    """Up to 1,024 rows the launches that want a list of rows make it themselves: of each kind, alone, together and side by side."""
+    rng = np.random.default_rng(rows)
+    vocab = 1211
+    print("[case] %d rows listed" % rows, flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * 2.0).astype(np.float32)
+    uniforms = rng.random(rows).astype(np.float32)
+    stream = torch.cuda.Stream(device="cuda:0")
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        for kinds in ((20, 0, 200, 1000), (0,), (200,), (20,)):
+            params = hip_sampler.make_params(rows, 0.9, 0, 0.93, 0.0)
+            params["top_k"] = rng.choice(np.array(kinds, dtype=np.uint32), rows)
+            params["temperature"][::9] = 0.0
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            flags = [hip_sampler.PASSES_FULL_ORDER, hip_sampler.PASSES_FULL_ORDER | hip_sampler.PASSES_SIDE_BY_SIDE]
+            if 200 not in kinds:
+                flags.append(hip_sampler.PASSES_FULL_ORDER | hip_sampler.PASSES_NO_WIDE_WINDOWS)
+            for passes in flags:
+                gpu = _run(sampler, logits, params, uniforms, passes, stream)
+                parity_util.assert_results_match(gpu, cpu, "f32", "%d rows of %s, passes %d" % (rows, kinds, passes))
