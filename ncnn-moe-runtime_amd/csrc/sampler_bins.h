@@ -2019,6 +2019,9 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             continue;
         }
         __syncthreads(); // (a row before this one: its last readers of shared are done)
+        if (tid < static_cast<int>(2u * kBinWords))
+            shared.ties[tid] = 0u;
+        __syncthreads();
         const float top_p = same_in_all(a.params[row].top_p);
         const float min_p = same_in_all(a.params[row].min_p);
         const float uniform = same_in_all(a.uniforms[row]);
@@ -2062,7 +2065,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         uint4 words{0u, 0u, 0u, 0u};
         uint32_t own_steps[4] = {0u, 0u, 0u, 0u};
         uint32_t tie_word = 0, untold_word = 0;
-        const uint32_t tie_lane = static_cast<uint32_t>(tid) - (kWalkThreads - kWaveSize);
+        const uint32_t tie_lane = static_cast<uint32_t>(tid) & (kWaveSize - 1);
         if (holds_bins)
             words = reinterpret_cast<const uint4*>(g.packed[kFrom] + static_cast<size_t>(row) * kBins)[tid];
         if (behind_head)
@@ -2087,28 +2090,28 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                     }
                 }
             }
-            // (the last waves hold no bins: they collect the words of the bins with terms half way)
+            // (every wave collects the words of some parts' bins with terms half way: by one wave, a part behind the other, they
+            // arrived 2 us after everything else)
             if (tie_lane < kBinWords)
             {
-                uint32_t other_words = 0;
+                static_assert(kMaxBinParts % kWalkWaves == 0, "as many parts for each wave");
 #pragma unroll
-                for (uint32_t q = 0; q < kMaxBinParts; ++q)
+                for (uint32_t k = 0; k < kMaxBinParts / kWalkWaves; ++k)
                 {
+                    const uint32_t q = static_cast<uint32_t>(tid) / kWaveSize + k * kWalkWaves;
                     const uint32_t* from = g.ties[kFrom] + (first_pair + min(q, grid.parts - 1u)) * 3u * kBinWords + tie_lane;
                     tie_word |= from[0];
-                    other_words |= from[kBinWords] | from[2u * kBinWords];
+                    untold_word |= from[kBinWords] | from[2u * kBinWords];
                 }
-                untold_word = other_words;
             }
         }
-        static_assert(kBinWords <= kWaveSize && kBinQuads <= kWalkThreads - kWaveSize, "the last wave holds no bins");
+        static_assert(kBinWords <= kWaveSize, "a word a lane");
         if (holds_bins)
             *reinterpret_cast<uint4*>(shared.packed + bin) = words;
-        if (tie_lane < kBinWords)
-        {
-            shared.ties[tie_lane] = tie_word;
-            shared.ties[kBinWords + tie_lane] = untold_word;
-        }
+        if (tie_word != 0u)
+            atomicOr(&shared.ties[tie_lane], tie_word);
+        if (untold_word != 0u)
+            atomicOr(&shared.ties[kBinWords + tie_lane], untold_word);
         if (tid == 0)
             shared.mask_count = 0u;
         if (tid < 4)
