@@ -839,6 +839,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->bins.records, rows * sizeof(BinRow));
     place(&s->bins.stats, pairs * sizeof(uint4));
     place(&s->bins.counts, pairs * 2 * kBins * sizeof(uint32_t));
+    place(&s->bins.before, pairs * kBins * sizeof(uint32_t));
     place(&s->bins.head_terms, rows * kBinListCap * sizeof(float));
     place(&s->bins.head_tokens, rows * kBinListCap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i)

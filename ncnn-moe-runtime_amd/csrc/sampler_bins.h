@@ -137,6 +137,7 @@ struct BinArgs
     uint32_t* list;        // the rows served: [0] their number, then the rows
     uint4* stats;          // [pairs] (row, part): largest and smallest finite logit, finite logits, flags
     uint32_t* counts;      // [pairs][2][kBins]: terms in each bin, and the sum of their places in it (kOffsetBits)
+    uint32_t* before;      // [pairs][kBins]: elements of each bin in the parts in front
     uint32_t* steps[2];    // [pairs][kBins], of alternate launches
     uint32_t* ties[2];     // [pairs][3][kBinWords]: bins with terms half way, with two of one value, and with some that their masks cannot hold
     uint32_t* masks[2];    // [pairs][2][kBins]: parities of the odd steps, and the values half way, by step (see add_bin_steps)
@@ -680,18 +681,22 @@ __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&fro
     return end_of_list;
 }
 
-// Elements of a bin in the parts in front of the calling one.
-__device__ __forceinline__ uint32_t count_in_front_parts(const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t bin)
+// Correctly rounded quotients by one divisor: two corrections of dividend x reciprocal, each with its exact remainder (P. Markstein,
+// Computation of elementary functions on the IBM RISC System/6000 processor, 1990: a quotient less than an ulp off, corrected with
+// the remainder times the correctly rounded reciprocal, is the correctly rounded one).  Five instructions instead of the ten and a
+// reciprocal of a division; for numbers whose quotient and remainder are far from the denormal ones, as the bins' terms are (compared
+// with the division for 4,000 divisors and every mantissa of the dividend).
+struct Divisor
 {
-    uint32_t before = 0;
-#pragma unroll
-    for (uint32_t q = 0; q + 1u < kMaxBinParts; ++q)
+    float value, reciprocal;
+    __device__ __forceinline__ explicit Divisor(float divisor) : value(divisor), reciprocal(1.0f / divisor) {}
+    __device__ __forceinline__ float divide(float dividend) const
     {
-        if (q < grid.part)
-            before += g.counts[static_cast<size_t>(slot * grid.parts + q) * 2u * kBins + bin];
+        const float about = dividend * reciprocal;
+        const float near = __builtin_fmaf(__builtin_fmaf(-about, value, dividend), reciprocal, about);
+        return __builtin_fmaf(__builtin_fmaf(-near, value, dividend), reciprocal, near);
     }
-    return before;
-}
+};
 
 // Adds the steps of a part's terms to the bins' integers, and puts the terms of listed bins into the list.
 //   entries   per bin: bit 31 the bin is listed and the rest is the next place of this part in the list; bit 30 it takes
@@ -707,6 +712,7 @@ __device__ __forceinline__ void add_bin_steps(
 {
     constexpr int kLoads = 4;
     const uint32_t first = s.first * 2u, last = s.last * 2u;
+    const Divisor by(divisor), by_second(second_divisor);
     for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
     {
         float4 raw[kLoads];
@@ -732,9 +738,9 @@ __device__ __forceinline__ void add_bin_steps(
                 {
                     float term = t[c];
                     if (PHASE >= 1)
-                        term = term / divisor;
+                        term = by.divide(term);
                     if (PHASE >= 2)
-                        term = term / second_divisor;
+                        term = by_second.divide(term);
                     const uint32_t bits = __float_as_uint(term);
                     const uint32_t mantissa = (bits & 0x7fffffu) | 0x800000u;
                     const int difference = static_cast<int>(entry) - static_cast<int>(bits >> 23);
@@ -752,7 +758,7 @@ __device__ __forceinline__ void add_bin_steps(
                         else if ((atomicOr(&masks[kBins + bin], 1u << ((step - 1u) & 31u)) >> ((step - 1u) & 31u) & 1u) != 0u)
                             atomicOr(&ties[kBinWords + (bin >> 5)], bit);
                     }
-                    else if ((step & 1u) != 0u)
+                    else if ((step & 1u) != 0u && difference >= kMaskedDifference) // (masks of nearer terms are not looked at)
                         atomicXor(&masks[bin], 1u << ((step >> 1) & 31u));
                 }
                 else if ((entry & 0x80000000u) != 0u)
@@ -971,6 +977,11 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks,
                                       g.list_terms[0] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[0] + static_cast<size_t>(row) * kBinListCap, tid);
         __syncthreads();
+        {
+            const size_t pair = slot * grid.parts + grid.part;
+            if (holds_bins)
+                reinterpret_cast<uint4*>(g.before + pair * kBins)[tid] = uint4{before[0], before[1], before[2], before[3]};
+        }
         if (beyond)
         {
             const size_t pair = slot * grid.parts + grid.part;
@@ -1101,7 +1112,7 @@ struct BinWalkShared
     uint16_t places[kBins + 2];             // where a listed bin's elements begin (as many are listed in front of the others); kHasMasks + i: the bin's masks are the i-th
     uint32_t bin_masks[2 * kBinMasks];      // of bins with terms half way
     uint16_t mask_bin[kBinMasks];
-    uint32_t mask_count;
+    uint32_t mask_count, any_ties;
     uint32_t stop_bin[kBinStops];           // bins at which the walk looks closer, in order (kStopBin, kStopExponent, kStopRun)
     uint32_t ties[2 * kBinWords];           // bins with terms half way; those of them that the masks do not tell
     BinScanScratch scan;
@@ -2021,6 +2032,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         __syncthreads(); // (a row before this one: its last readers of shared are done)
         if (tid < static_cast<int>(2u * kBinWords))
             shared.ties[tid] = 0u;
+        if (tid == 0)
+            shared.any_ties = 0u;
         __syncthreads();
         const float top_p = same_in_all(a.params[row].top_p);
         const float min_p = same_in_all(a.params[row].min_p);
@@ -2066,8 +2079,13 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         uint32_t own_steps[4] = {0u, 0u, 0u, 0u};
         uint32_t tie_word = 0, untold_word = 0;
         const uint32_t tie_lane = static_cast<uint32_t>(tid) & (kWaveSize - 1);
+        uint4 before{0u, 0u, 0u, 0u}; // elements of the thread's bins in the parts in front (where the next list takes this part's)
         if (holds_bins)
+        {
             words = reinterpret_cast<const uint4*>(g.packed[kFrom] + static_cast<size_t>(row) * kBins)[tid];
+            if (WALK < 2)
+                before = reinterpret_cast<const uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid];
+        }
         if (behind_head)
         {
             const size_t first_pair = slot * grid.parts;
@@ -2109,7 +2127,10 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         if (holds_bins)
             *reinterpret_cast<uint4*>(shared.packed + bin) = words;
         if (tie_word != 0u)
+        {
             atomicOr(&shared.ties[tie_lane], tie_word);
+            shared.any_ties = 1u;
+        }
         if (untold_word != 0u)
             atomicOr(&shared.ties[kBinWords + tie_lane], untold_word);
         if (tid == 0)
@@ -2139,7 +2160,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             // The bins whose terms half way the masks tell: their masks, from every part.  They lie anywhere among the bins, so
             // they are listed first and 16 lanes take the parts of each (a thread that went through its bins' parts one after
             // the other took 3 us a bin; 8 x 151,936 without a window: 148 us then, 135 us so).
-            if (behind_head)
+            if (behind_head && same_in_all(shared.any_ties) != 0u)
             {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
@@ -2551,13 +2572,14 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
                 reinterpret_cast<uint4*>(masks)[kBinQuads + tid] = uint4{0u, 0u, 0u, 0u};
                 uint32_t next_packed[4];
+                const uint32_t in_front[4] = {before.x, before.y, before.z, before.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
                     next_packed[j] = (plan.kind[j] << 30) | (plan.exponent[j] << 22) | front[j];
                     uint32_t entry = plan.kind[j] == kBinAdded ? plan.exponent[j] : 0x40000000u;
                     if (plan.kind[j] == kBinListed)
-                        entry = 0x80000000u | (place[j] + count_in_front_parts(g, grid, slot, bin + j));
+                        entry = 0x80000000u | (place[j] + in_front[j]);
                     entries[bin + j] = entry;
                 }
                 *reinterpret_cast<uint4*>(steps + bin) = uint4{0u, 0u, 0u, 0u};
