@@ -846,7 +846,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     {
         place(&s->bins.steps[i], pairs * kBins * sizeof(uint32_t));
         place(&s->bins.ties[i], pairs * 3 * kBinWords * sizeof(uint32_t));
-        place(&s->bins.masks[i], pairs * 2 * kBins * sizeof(uint32_t));
+        place(&s->bins.masks[i], pairs * kMaskWords * sizeof(uint32_t));
         place(&s->bins.packed[i], rows * kBins * sizeof(uint32_t));
         place(&s->bins.list_terms[i], rows * kBinListCap * sizeof(float));
         place(&s->bins.list_tokens[i], rows * kBinListCap * sizeof(uint32_t));

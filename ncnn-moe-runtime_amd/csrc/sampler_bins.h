@@ -59,6 +59,15 @@ constexpr uint32_t kBinStepUnit = 16;            // log2 of the unit in which a 
 constexpr uint32_t kBinStopBits = 11;            // ... above the row's number of stops, in one word
 static_assert(kBins < 1u << kBinStopBits && (kBins << (26 - kBinStepUnit)) < 1u << (32 - kBinStopBits), "the steps of 2^25 and a little a bin fit beside the stops");
 constexpr int kMaskedDifference = 14;            // so many binades below the sum a bin's terms (within a 64th of each other) take 18 different steps at most
+// ... and so many below it 66: the first bins of that distance have masks of four times the width.  A term half way that no mask
+// tells costs its row a fetch, and nearly all of those were 12 or 13 binades below the sum (of 94 rows in a batch of mixed options
+// some 13 % had one in each sum, and the batch waits for its slowest row).
+constexpr int kWideDifference = 12;
+constexpr uint32_t kWideBins = 128;
+constexpr uint32_t kWideParities = 2, kWideHalves = 4; // words a bin
+constexpr uint32_t kWideWords = kWideParities + kWideHalves;
+constexpr uint32_t kMaskWords = 2u * kBins + kWideBins * kWideWords; // of a part: two words a bin, then the wide ones
+static_assert(kMaskWords % 4u == 0u && kBins % 4u == 0u, "masks are moved in vectors of four words");
 constexpr uint32_t kBinRequests = 64;            // ... and how often per walk
 constexpr uint32_t kBinComparedTies = 256;       // equal terms of a list that are told apart by comparing each with each
 constexpr uint32_t kMaxBinParts = 16;
@@ -111,6 +120,7 @@ struct BinRow
     uint32_t saw_nan;
     uint32_t head_bins;     // bins [0, head_bins) are the head, head_count elements
     uint32_t head_count;
+    uint32_t wide_first[3]; // of each walk's sum: the first of the kWideBins bins with wide masks
     uint32_t listed[3];     // elements in the list of each walk (the first walk's holds the head, the others' places behind it)
     float normalizer;
     float head_sum[2];      // the Top-P sum and the draw's behind the head
@@ -140,7 +150,7 @@ struct BinArgs
     uint32_t* before;      // [pairs][kBins]: elements of each bin in the parts in front
     uint32_t* steps[2];    // [pairs][kBins], of alternate launches
     uint32_t* ties[2];     // [pairs][3][kBinWords]: bins with terms half way, with two of one value, and with some that their masks cannot hold
-    uint32_t* masks[2];    // [pairs][2][kBins]: parities of the odd steps, and the values half way, by step (see add_bin_steps)
+    uint32_t* masks[2];    // [pairs][kMaskWords]: parities of the odd steps, and the values half way, by step (see add_bin_steps)
     uint32_t* packed[2];   // [rows][kBins]
     float* list_terms[2];  // [rows][kBinListCap]
     uint32_t* list_tokens[2];
@@ -660,6 +670,27 @@ __device__ __forceinline__ BinPlan plan_bins(
     return plan;
 }
 
+// Whether the calling lane is the first of its wave (of those that call) for which `holds`: the one of them that speaks for the wave.
+__device__ __forceinline__ bool leads_wave(bool holds)
+{
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(holds);
+    return mask != 0ull && lane_id() == __builtin_ctzll(mask);
+}
+
+// The first of the thread's bins whose terms are kWideDifference binades and more below the sum (kBins: none).
+__device__ __forceinline__ uint32_t first_wide_bin(const BinPlan& plan, uint32_t bin, uint32_t shift, float scale)
+{
+    uint32_t first = kBins;
+#pragma unroll
+    for (int j = 3; j >= 0; --j)
+    {
+        const uint32_t top_exponent = __float_as_uint(bin_top(bin + j, shift) * scale) >> 23;
+        if (plan.kind[j] == kBinAdded && plan.exponent[j] >= top_exponent + kWideDifference)
+            first = bin + j;
+    }
+    return first;
+}
+
 // Where the thread's listed bins lie in the list (base: the position of the first); a bin that does not fit is not listed.
 __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&front)[5], uint32_t base, uint32_t (&place)[4])
 {
@@ -704,11 +735,12 @@ struct Divisor
 //   ties      bins with a term half way between two sums (its step is counted rounded up), with a second one of the same
 //             value, and with one that the masks cannot tell (the bin's terms take more than 32 steps)
 //   masks     per bin, for terms kMaskedDifference binades and more below the sum: bit (step / 2) % 32 the parity of the
-//             odd steps of that value; then bit step % 32 for a term half way between `step` and the next
+//             odd steps of that value; then bit step % 32 for a term half way between `step` and the next.  The kWideBins bins
+//             from wide_first on have the same with 64 and 128 bits
 template <int PHASE, int THREADS>
 __device__ __forceinline__ void add_bin_steps(
     const float* terms, const BinStretch& s, uint32_t shift, uint32_t first_bin, uint32_t bin_count, float divisor, float second_divisor,
-    uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, float* list_terms, uint32_t* list_tokens, int tid)
+    uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, uint32_t wide_first, float* list_terms, uint32_t* list_tokens, int tid)
 {
     constexpr int kLoads = 4;
     const uint32_t first = s.first * 2u, last = s.last * 2u;
@@ -749,17 +781,21 @@ __device__ __forceinline__ void add_bin_steps(
                     const uint32_t rest = mantissa & (2u * half - 1u);
                     const uint32_t step = (mantissa + half) >> down;
                     atomicAdd(&steps[bin], step);
+                    const uint32_t place_wide = bin - wide_first;
+                    const bool wide = place_wide < kWideBins;
+                    uint32_t* const wide_masks = masks + 2u * kBins + place_wide * kWideWords;
                     if ((rest == half) || difference < 1)
                     {
                         const uint32_t bit = 1u << (bin & 31u);
+                        const uint32_t half_way = step - 1u;
                         atomicOr(&ties[bin >> 5], bit);
-                        if (difference < kMaskedDifference)
+                        if (!wide && difference < kMaskedDifference)
                             atomicOr(&ties[2u * kBinWords + (bin >> 5)], bit);
-                        else if ((atomicOr(&masks[kBins + bin], 1u << ((step - 1u) & 31u)) >> ((step - 1u) & 31u) & 1u) != 0u)
+                        else if ((atomicOr(wide ? &wide_masks[kWideParities + (half_way >> 5) % kWideHalves] : &masks[kBins + bin], 1u << (half_way & 31u)) >> (half_way & 31u) & 1u) != 0u)
                             atomicOr(&ties[kBinWords + (bin >> 5)], bit);
                     }
-                    else if ((step & 1u) != 0u && difference >= kMaskedDifference) // (masks of nearer terms are not looked at)
-                        atomicXor(&masks[bin], 1u << ((step >> 1) & 31u));
+                    else if ((step & 1u) != 0u && (wide || difference >= kMaskedDifference)) // (masks of nearer terms are not looked at)
+                        atomicXor(wide ? &wide_masks[(step >> 6) % kWideParities] : &masks[bin], 1u << ((step >> 1) & 31u));
                 }
                 else if ((entry & 0x80000000u) != 0u)
                 {
@@ -777,10 +813,10 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
 {
     __shared__ __align__(16) uint32_t entries[kBins];
     __shared__ __align__(16) uint32_t steps[kBins];
-    __shared__ __align__(16) uint32_t masks[2 * kBins];
+    __shared__ __align__(16) uint32_t masks[kMaskWords];
     __shared__ uint32_t ties[3 * kBinWords];
     __shared__ BinScanScratch scan;
-    __shared__ uint32_t head_bins_of_row, head_count_of_row, end_of_list;
+    __shared__ uint32_t head_bins_of_row, head_count_of_row, end_of_list, wide_first_of_row;
     const SamplerArgs& a = g.a;
     const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
     const int tid = threadIdx.x;
@@ -843,10 +879,14 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                 count[j] = before[j] = 0u;
         }
         if (tid == 0)
+        {
             head_bins_of_row = head_count_of_row = end_of_list = 0u;
+            wide_first_of_row = kBins;
+        }
         if (holds_bins)
             reinterpret_cast<uint4*>(steps)[tid] = uint4{0u, 0u, 0u, 0u};
-        if (tid < static_cast<int>(2u * kBinQuads))
+        static_assert(kMaskWords / 4u <= kBinThreads, "a vector of the masks a thread");
+        if (tid < static_cast<int>(kMaskWords / 4u))
             reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
         if (tid < static_cast<int>(3u * kBinWords))
             ties[tid] = 0u;
@@ -910,10 +950,10 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
 #pragma unroll
             for (int j = 3; j >= 0; --j)
             {
-                // (where a bin's terms are kMaskedDifference binades below the sum, its masks tell how those half way are rounded, and
-                // few are: a sorted head would save the walk nothing)
+                // (where a bin's terms are kWideDifference binades below the sum, its masks tell how those half way are rounded: a
+                // sorted head would save the walk nothing.  Two binades further: verification without a window 168 us instead of 163)
                 const bool in_head = window_in_head ? front[j] < window
-                    : front[j + 1] <= kBinHead && bin_top(bin + j, shift) * static_cast<float>(1 << kMaskedDifference) >= mass[j];
+                    : front[j + 1] <= kBinHead && bin_top(bin + j, shift) * static_cast<float>(1 << kWideDifference) >= mass[j];
                 if (!in_head && bin + j != 0u)
                     first_not = bin + j;
             }
@@ -947,6 +987,9 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         const uint32_t own_end = fit_plan(plan, front, head_count + listed[0], place);
         if (holds_bins)
         {
+            const uint32_t wide_first = first_wide_bin(plan, bin, shift, 1.0f);
+            if (leads_wave(wide_first < kBins))
+                atomicMin(&wide_first_of_row, wide_first);
             uint32_t packed[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -972,9 +1015,10 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
             record.head_bins = head_bins;
             record.head_count = head_count;
             record.listed[0] = max(end_of_list, head_count);
+            record.wide_first[0] = wide_first_of_row;
         }
         const BinStretch s = element_bytes == 4u ? bin_stretch<4>(a, row, grid.part, grid.parts) : bin_stretch<2>(a, row, grid.part, grid.parts);
-        add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks,
+        add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks, wide_first_of_row,
                                       g.list_terms[0] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[0] + static_cast<size_t>(row) * kBinListCap, tid);
         __syncthreads();
         {
@@ -987,8 +1031,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
             const size_t pair = slot * grid.parts + grid.part;
             if (holds_bins)
                 reinterpret_cast<uint4*>(g.steps[0] + pair * kBins)[tid] = reinterpret_cast<uint4*>(steps)[tid];
-            if (tid < static_cast<int>(2u * kBinQuads))
-                reinterpret_cast<uint4*>(g.masks[0] + pair * 2u * kBins)[tid] = reinterpret_cast<uint4*>(masks)[tid];
+            if (tid < static_cast<int>(kMaskWords / 4u))
+                reinterpret_cast<uint4*>(g.masks[0] + pair * kMaskWords)[tid] = reinterpret_cast<uint4*>(masks)[tid];
             if (tid < static_cast<int>(3u * kBinWords))
                 g.ties[0][pair * 3u * kBinWords + tid] = ties[tid];
         }
@@ -1110,7 +1154,7 @@ struct BinWalkShared
     alignas(16) float terms[kBinListCap + kBinExtraCap];
     alignas(16) uint32_t tokens[kBinListCap + kBinExtraCap];
     uint16_t places[kBins + 2];             // where a listed bin's elements begin (as many are listed in front of the others); kHasMasks + i: the bin's masks are the i-th
-    uint32_t bin_masks[2 * kBinMasks];      // of bins with terms half way
+    uint32_t bin_masks[kWideWords * kBinMasks]; // of bins with terms half way: parities, then the values half way (one word each unless the bin is a wide one)
     uint16_t mask_bin[kBinMasks];
     uint32_t mask_count, any_ties;
     uint32_t stop_bin[kBinStops];           // bins at which the walk looks closer, in order (kStopBin, kStopExponent, kStopRun)
@@ -1126,7 +1170,7 @@ struct BinWalkShared
     uint32_t stop_rank;  // rank in the sorted row, and place in terms[], of the element the sum stopped at
     uint32_t stop_at;
     uint32_t taken;      // elements added when the sum ran to its end
-    uint32_t listed_end;
+    uint32_t listed_end, wide_first;
     int32_t token;
     uint32_t least_key, most_key, matches; // see token_of_equal
     uint32_t many;                          // see order_elements
@@ -1562,7 +1606,7 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
 //             which lies in that bin (kBins: nowhere)
 template <int PHASE, bool ROOMY>
 __device__ __forceinline__ void walk_bins(
-    BinWalkShared& shared, uint32_t stops, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins,
+    BinWalkShared& shared, uint32_t stops, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins, uint32_t wide_first,
     uint32_t limit, uint32_t cut_bin, float cut_term, float start_sum, int mode, float bound, float divisor, float second_divisor, int tid)
 {
     uint32_t cur = head_bins;
@@ -1734,29 +1778,39 @@ __device__ __forceinline__ void walk_bins(
                     if (known)
                     {
                         const uint32_t total = shared.prefix[stop_here + 1u] - shared.prefix[stop_here];
-                        const uint32_t parities = shared.bin_masks[2u * (place & ~kHasMasks)], halves = shared.bin_masks[2u * (place & ~kHasMasks) + 1u];
+                        const uint32_t* const masks = shared.bin_masks + kWideWords * (place & ~kHasMasks);
+                        const bool wide = stop_here - wide_first < kWideBins;
                         float top = bin_top(stop_here, shift);
                         if (PHASE >= 1)
                             top = top / divisor;
                         if (PHASE >= 2)
                             top = top / second_divisor;
+                        known = exponent - static_cast<int>(__float_as_uint(top) >> 23) >= (wide ? kWideDifference : kMaskedDifference);
+                        const uint32_t highest = step_of_term(top, exponent).odd + 1u;
+                        uint32_t parity = mantissa, less = 0, odd_in_front = 0;
                         // lane l: the terms of step highest - l, and the value half way between that step and the one below
-                        known = exponent - static_cast<int>(__float_as_uint(top) >> 23) >= kMaskedDifference;
-                        const uint32_t step = step_of_term(top, exponent).odd + 1u - static_cast<uint32_t>(lane_id());
-                        const bool in_range = lane_id() < 32;
-                        const uint64_t odd_steps = __builtin_amdgcn_ballot_w64(in_range && (step & 1u) != 0u && (parities >> ((step >> 1) & 31u) & 1u) != 0u);
-                        uint64_t half_way = __builtin_amdgcn_ballot_w64(in_range && (halves >> ((step - 1u) & 31u) & 1u) != 0u);
-                        const uint32_t highest = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(step), 0));
-                        uint32_t parity = mantissa, less = 0;
-                        while (half_way != 0ull)
+                        // (a wide bin's: 64 steps, then those behind them)
+                        constexpr uint32_t kSteps = 24, kWideSteps = 80;
+                        for (uint32_t first = 0; first < (wide ? kWideSteps : kSteps); first += kWaveSize)
                         {
-                            const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(half_way));
-                            half_way &= half_way - 1ull;
-                            const uint32_t below = highest - l - 1u; // the value lies half way between this step and the next
-                            const uint32_t in_front = static_cast<uint32_t>(__popcll(odd_steps & ((2ull << l) - 1ull)));
-                            const uint32_t up = (parity + in_front + below) & 1u; // to the even neighbour
-                            parity += below + up;
-                            less += 1u - up;
+                            const uint32_t number = first + static_cast<uint32_t>(lane_id());
+                            const uint32_t step = highest - number, half = step - 1u;
+                            const bool in_range = number < (wide ? kWideSteps : kSteps);
+                            const uint32_t parities = masks[wide ? (step >> 6) % kWideParities : 0u];
+                            const uint32_t halves = masks[kWideParities + (wide ? (half >> 5) % kWideHalves : 0u)];
+                            const uint64_t odd_steps = __builtin_amdgcn_ballot_w64(in_range && (step & 1u) != 0u && (parities >> ((step >> 1) & 31u) & 1u) != 0u);
+                            uint64_t half_way = __builtin_amdgcn_ballot_w64(in_range && (halves >> (half & 31u) & 1u) != 0u);
+                            while (half_way != 0ull)
+                            {
+                                const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(half_way));
+                                half_way &= half_way - 1ull;
+                                const uint32_t below = highest - first - l - 1u; // the value lies half way between this step and the next
+                                const uint32_t in_front = odd_in_front + static_cast<uint32_t>(__popcll(odd_steps & ((2ull << l) - 1ull)));
+                                const uint32_t up = (parity + in_front + below) & 1u; // to the even neighbour
+                                parity += below + up;
+                                less += 1u - up;
+                            }
+                            odd_in_front += static_cast<uint32_t>(__popcll(odd_steps));
                         }
                         known = known && total < kBinadeFull && mantissa + total < goal;
                         if (known)
@@ -2044,6 +2098,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         const uint32_t head_bins = same_in_all(record.head_bins);
         const uint32_t head_count = same_in_all(record.head_count);
         const uint32_t listed = same_in_all(record.listed[WALK]);
+        const uint32_t wide_first = same_in_all(record.wide_first[WALK]);
         const uint32_t limit = WALK == 0 ? window : same_in_all(record.limit[WALK - 1]);
         const uint32_t cut_bin = WALK == 1 ? same_in_all(record.cut_bin) : kBins;
         const float cut_term = WALK == 1 ? same_in_all(record.cut_term) : 0.0f;
@@ -2182,21 +2237,39 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 const uint32_t mask_count = min(shared.mask_count, kBinMasks);
                 for (uint32_t i = static_cast<uint32_t>(tid) / kMaxBinParts; i < mask_count; i += kWalkThreads / kMaxBinParts)
                 {
-                    const uint32_t* from = g.masks[kFrom] + static_cast<size_t>(slot * grid.parts + min(part, grid.parts - 1u)) * 2u * kBins + shared.mask_bin[i];
-                    uint32_t parities = part < grid.parts ? from[0] : 0u, halves = part < grid.parts ? from[kBins] : 0u, twice = 0u;
+                    const uint32_t* const of_part = g.masks[kFrom] + static_cast<size_t>(slot * grid.parts + min(part, grid.parts - 1u)) * kMaskWords;
+                    const uint32_t mask_bin = shared.mask_bin[i];
+                    const bool wide = mask_bin - wide_first < kWideBins;
+                    const uint32_t* const wide_masks = of_part + 2u * kBins + (wide ? mask_bin - wide_first : 0u) * kWideWords;
+                    uint32_t words_of_bin[kWideWords];
+#pragma unroll
+                    for (uint32_t w = 0; w < kWideWords; ++w)
+                    {
+                        const uint32_t word = wide ? wide_masks[w] : w == 0u ? of_part[mask_bin] : w == kWideParities ? of_part[kBins + mask_bin] : 0u;
+                        words_of_bin[w] = part < grid.parts ? word : 0u;
+                    }
+                    uint32_t twice = 0u;
 #pragma unroll
                     for (int distance = 1; distance < static_cast<int>(kMaxBinParts); distance *= 2)
                     {
-                        const uint32_t others = __shfl_xor(halves, distance, kMaxBinParts);
-                        parities ^= __shfl_xor(parities, distance, kMaxBinParts);
-                        twice |= __shfl_xor(twice, distance, kMaxBinParts) | (halves & others);
-                        halves |= others;
+                        twice |= __shfl_xor(twice, distance, kMaxBinParts);
+#pragma unroll
+                        for (uint32_t w = 0; w < kWideWords; ++w)
+                        {
+                            const uint32_t others = __shfl_xor(words_of_bin[w], distance, kMaxBinParts);
+                            if (w >= kWideParities)
+                                twice |= words_of_bin[w] & others;
+                            words_of_bin[w] = w < kWideParities ? words_of_bin[w] ^ others : words_of_bin[w] | others;
+                        }
                     }
                     if (part == 0u)
                     {
-                        shared.bin_masks[2u * i] = parities;
                         // (a value half way that two parts have seen is there twice, which a mask cannot tell)
-                        shared.bin_masks[2u * i + 1u] = twice == 0u ? halves : 0u;
+                        if (twice != 0u)
+                            shared.mask_bin[i] = static_cast<uint16_t>(kBins);
+#pragma unroll
+                        for (uint32_t w = 0; w < kWideWords; ++w)
+                            shared.bin_masks[kWideWords * i + w] = words_of_bin[w];
                     }
                 }
                 __syncthreads();
@@ -2205,7 +2278,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 if (!(behind && kind_here == kBinWanted && packed_kind(packed_here) == kBinAdded && (untold_bits >> j & 1u) == 0u))
                     return 0u;
                 const uint32_t i = shared.places[b];
-                return i < kBinMasks && shared.bin_masks[2u * i + 1u] != 0u ? kHasMasks | i : 0u;
+                return i < kBinMasks && shared.mask_bin[i] == b ? kHasMasks | i : 0u;
             };
             uint32_t masked[4];
             uint32_t previous = holds_bins && bin > head_bins ? shared.packed[bin - 1u] : packed[0];
@@ -2342,7 +2415,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 mass[j] += sum;
             if (behind_head)
             {
-                walk_bins<0, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+                walk_bins<0, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
                 given_up = shared.status == 2u;
                 sum = same_in_all(shared.sum);
             }
@@ -2410,7 +2483,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         }
         if constexpr (WALK == 1)
         {
-            walk_bins<1, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
+            walk_bins<1, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
                          normalizer, 1.0f, tid);
             const bool stopped = shared.stopped != 0u;
             // (a sum that no stop condition ends runs to the window's end, or to the Min-P cut, which no bin may hold)
@@ -2488,7 +2561,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             }
             if constexpr (WALK == 2)
             {
-                walk_bins<2, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
+                walk_bins<2, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
                              normalizer, renormalizer, tid);
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);
@@ -2552,7 +2625,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             uint32_t* const entries = shared.prefix;
             uint32_t* const steps = shared.packed;
             uint32_t* const masks = shared.tokens;                      // (the list has been used)
-            uint32_t* const ties = shared.tokens + 2u * kBins;
+            uint32_t* const ties = shared.tokens + kMaskWords;
+            static_assert(kMaskWords + 3u * kBinWords <= kBinListCap + kBinExtraCap, "masks and words fit where the list was");
             // the sorted head is kept for the launch behind this one
             if (WALK == 0 && grid.part == 0u)
             {
@@ -2563,14 +2637,20 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 }
             }
             if (tid == 0)
+            {
                 shared.listed_end = 0u;
+                shared.wide_first = kBins;
+            }
             __syncthreads();
             if (tid < static_cast<int>(3u * kBinWords))
                 ties[tid] = 0u;
+            for (uint32_t i = tid; i < kMaskWords / 4u; i += kWalkThreads)
+                reinterpret_cast<uint4*>(masks)[i] = uint4{0u, 0u, 0u, 0u};
             if (holds_bins)
             {
-                reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
-                reinterpret_cast<uint4*>(masks)[kBinQuads + tid] = uint4{0u, 0u, 0u, 0u};
+                const uint32_t next_wide = first_wide_bin(plan, bin, shift, 1.0f / (WALK == 0 ? normalizer : normalizer * renormalizer));
+                if (leads_wave(next_wide < kBins))
+                    atomicMin(&shared.wide_first, next_wide);
                 uint32_t next_packed[4];
                 const uint32_t in_front[4] = {before.x, before.y, before.z, before.w};
 #pragma unroll
@@ -2589,17 +2669,14 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             __syncthreads();
             if (grid.part == 0u && own_end != 0u && holds_bins)
                 atomicMax(&shared.listed_end, own_end);
-            add_bin_steps<WALK + 1, kWalkThreads>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks,
+            add_bin_steps<WALK + 1, kWalkThreads>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks, shared.wide_first,
                                                   g.list_terms[kTo] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[kTo] + static_cast<size_t>(row) * kBinListCap, tid);
             __syncthreads();
             const size_t pair = slot * grid.parts + grid.part;
             if (holds_bins)
                 reinterpret_cast<uint4*>(g.steps[kTo] + pair * kBins)[tid] = *reinterpret_cast<uint4*>(steps + bin);
-            if (tid < static_cast<int>(kBinQuads))
-            {
-                reinterpret_cast<uint4*>(g.masks[kTo] + pair * 2u * kBins)[tid] = reinterpret_cast<uint4*>(masks)[tid];
-                reinterpret_cast<uint4*>(g.masks[kTo] + pair * 2u * kBins)[kBinQuads + tid] = reinterpret_cast<uint4*>(masks)[kBinQuads + tid];
-            }
+            for (uint32_t i = tid; i < kMaskWords / 4u; i += kWalkThreads)
+                reinterpret_cast<uint4*>(g.masks[kTo] + pair * kMaskWords)[i] = reinterpret_cast<uint4*>(masks)[i];
             if (tid < static_cast<int>(3u * kBinWords))
                 g.ties[kTo][pair * 3u * kBinWords + tid] = ties[tid];
             if (grid.part == 0u && tid == 0)
@@ -2610,6 +2687,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 record.head_sum[WALK] = head_sum;
                 record.limit[WALK] = next_limit;
                 record.listed[WALK + 1] = max(shared.listed_end, head_count);
+                record.wide_first[WALK + 1] = shared.wide_first;
                 if (WALK == 0)
                 {
                     record.cut_bin = next_cut_bin;

@@ -204,3 +204,23 @@ def test_runs_of_listed_bins_that_end_with_the_sum(vocab):
             params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
             cpu = parity_util.run_oracle(logits, params, uniforms)
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "top_p %g min_p %g top_k %d" % (top_p, min_p, top_k))
+
+
+@pytest.mark.parametrize("vocab", [20011, 100003, 151936])
+@pytest.mark.parametrize("spread", [0.3, 1.0, 1.33, 1.8, 2.5])
+def test_terms_half_way_at_every_distance(spread, vocab):
+    """Rows whose sums meet terms that lie half way between two sums 10 to 20 binades below them: those that no mask, a narrow one and a
+    wide one tells, in the normaliser, the Top-P sum and the draw.  (Rounded to 1/4096 the rows hold many of them twice.)"""
+    rng = np.random.default_rng(int(spread * 100) + vocab)
+    rows = 40
+    print("[case] terms half way, %d of spread %g" % (vocab, spread), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * spread).astype(np.float32)
+    logits[::3] = (np.round(logits[::3] * 4096.0) / 4096.0).astype(np.float32)
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["temperature"] = rng.choice(np.array([1.0, 0.8, 1.3], dtype=np.float32), rows)
+    params["top_p"] = rng.choice(np.array([1.0, 0.9999, 0.99, 0.9, 0.7], dtype=np.float32), rows)
+    uniforms = rng.random(rows, dtype=np.float32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "terms half way, %d of spread %g" % (vocab, spread))
