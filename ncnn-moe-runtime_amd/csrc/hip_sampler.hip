@@ -313,10 +313,10 @@ void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing li
     hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
 }
 
-// The binned sums (sampler_bins.h) over the rows in the handle's bin list; the walks, which finish rows, wait for
-// `before_walks` (null: for nothing).
+// The binned sums (sampler_bins.h) over the rows in the handle's bin list.  `behind_sum` (null: none): an event behind the last
+// launch that reads a row as a stream.
 template <int DTYPE>
-hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t before_walks, hipStream_t stream)
+hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t behind_sum, hipStream_t stream)
 {
     BinArgs g = s->bins;
     g.a = a;
@@ -325,21 +325,35 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
     g.listing = listing;
     hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
     hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
-    hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
-    const hipError_t waits = before_walks != nullptr ? hipStreamWaitEvent(stream, before_walks, 0) : hipSuccess;
+    constexpr uint32_t kElementBytes = DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u;
+    // (the event rides on the kernel's own completion signal where the stream is not being captured: a record of its own is
+    // one more packet for the walks to wait behind)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (behind_sum != nullptr)
+        (void)hipStreamIsCapturing(stream, &capturing);
+    hipError_t result = hipSuccess;
+    if (behind_sum != nullptr && capturing == hipStreamCaptureStatusNone)
+        hipExtLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, nullptr, behind_sum, 0, g, kElementBytes);
+    else
+    {
+        hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, kElementBytes);
+        if (behind_sum != nullptr)
+            result = hipEventRecord(behind_sum, stream);
+    }
     if (a.rows <= kRoomyRows)
         launch_bin_walks<DTYPE, true>(g, stream);
     else
         launch_bin_walks<DTYPE, false>(g, stream);
-    return waits;
+    return result;
 }
 
 // Enqueues the first select and what follows it for the rows that it leaves pending: the window kernels and the binned
 // sums.  side_by_side: those rows are known by their options, and the chain of the sums (the longest, its walks a few
-// dependent steps a row) runs on the caller's stream while the select and the window kernels (bound by the stream of
-// logits) run on the handle's second one.  A walk marks its row as done, which the select marks as pending, so the walks
-// wait for the select; it has ended long before.  512 rows of 129,280, mixed options: 351 us one behind the
-// other, 321 us so.
+// dependent steps a row) runs on the caller's stream beside the select and the window kernels (bound by the stream of
+// logits) on the handle's second one.  The sums read their rows first: beside a select that has the memory to itself for 55 us
+// their three passes took 110 us, alone 35, and the walks behind them hardly use it.  So the select starts behind those passes;
+// it leaves the sums' rows alone, since a walk may have finished one by then.  512 rows of 129,280, mixed options: 351 us one
+// behind the other, 256 us with the select in front, 227 us so.
 template <int DTYPE>
 hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
                             bool want_filters, hipStream_t stream)
@@ -351,24 +365,24 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
             hipLaunchKernelGGL(later_rows_list_kernel, dim3(1), dim3(kBinThreads), 0, stream, a, side_by_side ? 1u : 0u,
                                windows ? s->window_list : nullptr, sums ? s->bin_list : nullptr);
     };
-    const auto select = [&](hipStream_t on) { launch_select<DTYPE>(geometry, a.rows, on, a, 0, s->scatter_segments != 0); };
+    const auto select = [&](const SamplerArgs& args, hipStream_t on) { launch_select<DTYPE>(geometry, a.rows, on, args, 0, s->scatter_segments != 0); };
     if (side_by_side && windows && sums && s->side_stream != nullptr)
     {
         list_rows();
-        hipError_t result = hipEventRecord(s->side_fork, stream);
+        hipError_t result = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, s->side_fork, stream);
         if (result == hipSuccess)
             result = hipStreamWaitEvent(s->side_stream, s->side_fork, 0);
         if (result != hipSuccess)
             return result;
-        select(s->side_stream);
-        result = hipEventRecord(s->cut_done, s->side_stream);
+        SamplerArgs others = a;
+        others.leave_sums_rows = 1;
+        select(others, s->side_stream);
         launch_windows<DTYPE>(s, a, listing, nullptr, s->side_stream);
-        const hipError_t joins = hipEventRecord(s->side_join, s->side_stream);
-        const hipError_t waits = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, s->cut_done, stream);
+        result = hipEventRecord(s->side_join, s->side_stream);
         const hipError_t joined = hipStreamWaitEvent(stream, s->side_join, 0);
-        return result != hipSuccess ? result : joins != hipSuccess ? joins : waits != hipSuccess ? waits : joined;
+        return result != hipSuccess ? result : joined;
     }
-    select(stream);
+    select(a, stream);
     list_rows();
     if (windows)
         launch_windows<DTYPE>(s, a, listing, sums ? s->bin_list : nullptr, stream);

@@ -460,8 +460,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
         if (grid.part == 0u && tid == 0)
         {
             BinRow& record = g.records[row];
-            // A row is rejected (as the CPU sampler does) by the first walk and not here: beside the first launches the
-            // first select may still be marking the same row as pending, and the walks wait for it.
+            // (pending until a walk has finished it: a first select that runs beside leaves these rows alone)
+            a.row_state[row] = kRowNeedsGeneral;
             record.state[0] = served ? kBinRowGoesOn : rejected ? kBinRowRejected : kBinRowLeft;
             record.shift = shift;
             record.window = (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite;

@@ -495,7 +495,8 @@ __global__ __launch_bounds__(kScanThreads, (!LOOPED && DTYPE == NCNN_MOE_LOGITS_
         // one; and the first select leaves the wide select's rows alone when told that one runs beside it.
         const bool not_mine = a.only_pending == 2 || (a.only_pending == 1 && mode == kModeGeneral) ||
             (!WIDE && a.leave_wide_rows != 0 && mode == kModeGeneral && a.force_general == 0 &&
-             effective_k <= static_cast<uint32_t>(kSelectTopK));
+             effective_k <= static_cast<uint32_t>(kSelectTopK)) ||
+            (!WIDE && a.leave_sums_rows != 0 && mode == kModeGeneral && effective_k > static_cast<uint32_t>(kSelectTopK));
         if (segment == 0 && tid == 0 && !not_mine)
         {
             if (mode == kModeInvalid)
