@@ -349,11 +349,12 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
 
 // Enqueues the first select and what follows it for the rows that it leaves pending: the window kernels and the binned
 // sums.  side_by_side: those rows are known by their options, and the chain of the sums (the longest, its walks a few
-// dependent steps a row) runs on the caller's stream beside the select and the window kernels (bound by the stream of
+// dependent steps a row) runs on the caller's stream beside the window kernels and the select (bound by the stream of
 // logits) on the handle's second one.  The sums read their rows first: beside a select that has the memory to itself for 55 us
-// their three passes took 110 us, alone 35, and the walks behind them hardly use it.  So the select starts behind those passes;
-// it leaves the sums' rows alone, since a walk may have finished one by then.  512 rows of 129,280, mixed options: 351 us one
-// behind the other, 256 us with the select in front, 227 us so.
+// their three passes took 110 us, alone 70, and the walks behind them hardly use it.  So the second stream starts behind those
+// passes, with the windows, whose second kernel is a chain as well, in front of the select; the select leaves the rows of both
+// alone, since one of them may be finished by then.  512 rows of 129,280, mixed options: 351 us one behind the other, 256 us
+// with select and windows beside the passes, 227 us with them behind, select first, and 223 us so.
 template <int DTYPE>
 hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
                             bool want_filters, hipStream_t stream)
@@ -374,10 +375,10 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
             result = hipStreamWaitEvent(s->side_stream, s->side_fork, 0);
         if (result != hipSuccess)
             return result;
-        SamplerArgs others = a;
-        others.leave_sums_rows = 1;
-        select(others, s->side_stream);
         launch_windows<DTYPE>(s, a, listing, nullptr, s->side_stream);
+        SamplerArgs others = a;
+        others.leave_later_rows = 1;
+        select(others, s->side_stream);
         result = hipEventRecord(s->side_join, s->side_stream);
         const hipError_t joined = hipStreamWaitEvent(stream, s->side_join, 0);
         return result != hipSuccess ? result : joined;

@@ -20,7 +20,7 @@ struct SamplerArgs
     int only_pending;            // wide select: 1 = serve the rows an earlier launch of the call left pending; 2 = serve the rows
                                  // whose options ask for a window of 65 to 1024, whatever their state (it runs beside the first select)
     int leave_wide_rows;         // first select and full-order kernels: rows that the wide select serves are another stream's
-    int leave_sums_rows;         // first select: rows without a window of the window kernels' widths are another stream's, which has marked them pending
+    int leave_later_rows;        // first select: rows that it does not serve are those of earlier launches, which have marked them pending
 
     const ncnn_moe_sample_params* params;
     const float* uniforms;

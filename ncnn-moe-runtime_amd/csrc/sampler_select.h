@@ -496,7 +496,7 @@ __global__ __launch_bounds__(kScanThreads, (!LOOPED && DTYPE == NCNN_MOE_LOGITS_
         const bool not_mine = a.only_pending == 2 || (a.only_pending == 1 && mode == kModeGeneral) ||
             (!WIDE && a.leave_wide_rows != 0 && mode == kModeGeneral && a.force_general == 0 &&
              effective_k <= static_cast<uint32_t>(kSelectTopK)) ||
-            (!WIDE && a.leave_sums_rows != 0 && mode == kModeGeneral && effective_k > static_cast<uint32_t>(kSelectTopK));
+            (!WIDE && a.leave_later_rows != 0 && mode == kModeGeneral);
         if (segment == 0 && tid == 0 && !not_mine)
         {
             if (mode == kModeInvalid)

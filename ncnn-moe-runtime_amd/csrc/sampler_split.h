@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kScanThreads, DTYPE == NCNN_MOE_LOGITS_F32 ? 8 : 4)
         // (a row with a window of 65 to 1024 is left alone when a wide select runs beside this kernel)
         const bool not_mine = (a.leave_wide_rows != 0 && mode == kModeGeneral && a.force_general == 0 &&
                                effective_k <= static_cast<uint32_t>(kSelectTopK)) ||
-            (a.leave_sums_rows != 0 && mode == kModeGeneral && effective_k > static_cast<uint32_t>(kSelectTopK));
+            (a.leave_later_rows != 0 && mode == kModeGeneral);
         if (segment == 0 && tid == 0 && !not_mine)
         {
             if (mode == kModeInvalid)

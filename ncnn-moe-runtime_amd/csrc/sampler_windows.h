@@ -113,6 +113,9 @@ __device__ __forceinline__ void window_candidates(const WindowArgs& g, const Bin
             shared.count = 0u;
             shared.saw_nan = 0u;
             shared.bound = 0u;
+            // (pending until window_finish has finished it: a first select that comes later leaves these rows alone)
+            if (grid.part == 0u)
+                a.row_state[row] = kRowNeedsGeneral;
         }
         for (uint32_t i = tid; i < kWindowBins / 4u; i += kBinThreads)
             reinterpret_cast<uint4*>(shared.counts)[i] = uint4{0u, 0u, 0u, 0u};
