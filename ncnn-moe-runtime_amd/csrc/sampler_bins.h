@@ -63,6 +63,7 @@ constexpr int kMaskedDifference = 14;            // so many binades below the su
 // tells costs its row a fetch, and nearly all of those were 12 or 13 binades below the sum (of 94 rows in a batch of mixed options
 // some 13 % had one in each sum, and the batch waits for its slowest row).
 constexpr int kWideDifference = 12;
+constexpr float kNearlyTopP = 0.85f;                // of the Top-P, in the longest head: see the head of bin_sum_kernel
 constexpr uint32_t kWideBins = 128;
 constexpr uint32_t kWideParities = 2, kWideHalves = 4; // words a bin
 constexpr uint32_t kWideWords = kWideParities + kWideHalves;
@@ -948,7 +949,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         // bin's terms are kWideDifference binades below the sum, its masks tell how those half way are rounded, and a sorted head
         // would save the walk nothing: it ends there (two binades further: verification without a window 168 us instead of 163)
         // unless the longest head holds the row's Top-P as well, and with it the ends of the second and third walk (64 x 4,096,
-        // Top-P 0.95: 81.8 us with the head that ends early, 58.8 us so).
+        // Top-P 0.95: 81.8 us with the head that ends early, 58.8 us so), or nearly: most draws end in it then (100 x 8,192, Top-P
+        // 0.9: 114.1 us where it has to hold all of it, 104.4 us so; 32 x 32,000 and 8 x 151,936, whose heads hold less, as before).
         const bool window_in_head = window <= kBinHead;
         {
             // (the bins of a head are the first ones: one that is not of it ends it)
@@ -988,7 +990,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                 heads_hold[1] = front[j + 1];
         }
         __syncthreads();
-        const uint32_t taken = longest_holds >= top_p * row_holds ? 0u : 1u;
+        const uint32_t taken = longest_holds >= kNearlyTopP * top_p * row_holds ? 0u : 1u;
         uint32_t head_bins = taken == 0u ? longest_bins : early_bins;
         uint32_t head_count = heads_hold[taken];
         if (head_count > kBinListCap)

@@ -224,3 +224,22 @@ def test_terms_half_way_at_every_distance(spread, vocab):
     with hip_sampler.HipSampler(rows, vocab) as sampler:
         sampler.upload_logits(logits)
         parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "terms half way, %d of spread %g" % (vocab, spread))
+
+
+@pytest.mark.parametrize("vocab", [1921, 4096, 8192])
+@pytest.mark.parametrize("spread", [1.0, 2.0, 2.5])
+def test_heads_that_hold_the_top_p_and_heads_that_end_before_it(spread, vocab):
+    """Rows short enough for the longest sorted head to hold the whole Top-P, nearly all of it or less, and draws on both sides of
+    the head's end: the head ends early or late by the row's own Top-P, and the token, the filters and the draw stay the same."""
+    rng = np.random.default_rng(int(spread * 100) + vocab)
+    rows = 48
+    print("[case] heads, %d of spread %g" % (vocab, spread), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * spread).astype(np.float32)
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["top_p"] = np.linspace(0.3, 1.0, rows, dtype=np.float32)
+    uniforms = rng.random(rows, dtype=np.float32)
+    uniforms[::4] = np.float32(1.0) - np.float32(2.0) ** -24
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "heads, %d of spread %g" % (vocab, spread))
