@@ -7,7 +7,7 @@
 // leaves its binade nor meets such a term may be added in any order, as integers.  The rows served here (no Top-K
 // window, or one wider than the first select's) are therefore not sorted:
 //   * the terms fall into kBins bins by their bit pattern (0.4 to 0.8 % of a term wide; bins follow the sorted order);
-//   * the head of the row (the bins of its first few thousand elements) is sorted in LDS and added exactly as the
+//   * the head of the row (the bins of its first 1,920 elements at most) is sorted in LDS and added exactly as the
 //     CPU does, which takes the sum through most of its binades;
 //   * every other bin is one integer: the sum of its terms' steps at the exponent that the running sum will have there;
 //   * the few bins in which the order matters - the sum leaves its binade, a stop condition is met, the window or the
@@ -24,9 +24,9 @@
 // and bin counts, (3) head fetched, steps of the normaliser's sum, (4) normaliser walked, steps of the Top-P sum,
 // (5) Top-P walked, steps of the draw's sum, (6) draw walked.  A row whose walks end inside its head is finished by (4).
 //
-// What bounds it: at few rows the chain of launches and, inside (4) to (6), the walk (some 5 to 10 us each, LDS and
-// dependent instructions); at a hundred rows and more the instructions per logit (some 40 for the exponential and its
-// bin, 25 to 40 for a step).
+// What bounds it: at few rows the chain of launches and, inside (3) to (6), dependent instructions and trips to LDS and
+// memory (8 rows of 151,936: 6, 8, 16, 29, 26 and 14 us; of a walk some 5.5 us add the next sum's steps, bound by LDS
+// atomics); at a hundred rows and more the reads of the rows and their terms, and the slowest row's walk.
 #ifndef NCNN_MOE_HIP_SAMPLER_BINS_H
 #define NCNN_MOE_HIP_SAMPLER_BINS_H
 
