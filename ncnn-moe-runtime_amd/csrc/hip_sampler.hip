@@ -302,44 +302,59 @@ void launch_bin_walks(const BinArgs& g, hipStream_t stream)
 
 // The window kernels (sampler_windows.h) over the rows in the handle's window list (`other_list`: see list_rows_in_place).
 template <int DTYPE>
-void launch_windows(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, uint32_t* other_list, hipStream_t stream)
+void launch_window_candidates(const WindowArgs& w, hipStream_t stream)
+{
+    hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
+}
+
+template <int DTYPE>
+void launch_window_finish(const WindowArgs& w, hipStream_t stream)
+{
+    hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(w.a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
+}
+
+WindowArgs window_args(const ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, uint32_t* other_list)
 {
     WindowArgs w = s->windows;
     w.a = a;
     w.windows_are_selects = 1u;
     w.listing = listing;
     w.other_list = other_list;
-    hipLaunchKernelGGL((window_candidates_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, w);
-    hipLaunchKernelGGL((window_finish_kernel<DTYPE>), dim3(std::min<uint32_t>(a.rows, kBinGrid)), dim3(kWalkThreads), 0, stream, w);
+    w.turn = kWindowsOnce;
+    w.sums_list = s->bin_list;
+    return w;
 }
 
-// The binned sums (sampler_bins.h) over the rows in the handle's bin list.  `behind_sum` (null: none): an event behind the last
-// launch that reads a row as a stream.
+// The binned sums (sampler_bins.h) over the rows in the handle's bin list.  `behind_terms`, `behind_sum` (null: none): events
+// behind the launch that writes the rows' terms and behind the last one that reads a row as a stream.
 template <int DTYPE>
-hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t behind_sum, hipStream_t stream)
+hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t behind_terms,
+                           hipEvent_t behind_sum, hipStream_t stream)
 {
     BinArgs g = s->bins;
     g.a = a;
     g.windows_are_selects = windows ? 1u : 0u;
     g.want_filters = want_filters ? 1u : 0u;
     g.listing = listing;
-    hipLaunchKernelGGL((bin_stats_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
-    hipLaunchKernelGGL((bin_terms_kernel<DTYPE>), dim3(kBinGrid), dim3(kBinThreads), 0, stream, g);
-    constexpr uint32_t kElementBytes = DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u;
-    // (the event rides on the kernel's own completion signal where the stream is not being captured: a record of its own is
-    // one more packet for the walks to wait behind)
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (behind_sum != nullptr)
-        (void)hipStreamIsCapturing(stream, &capturing);
     hipError_t result = hipSuccess;
-    if (behind_sum != nullptr && capturing == hipStreamCaptureStatusNone)
-        hipExtLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, nullptr, behind_sum, 0, g, kElementBytes);
-    else
-    {
-        hipLaunchKernelGGL(bin_sum_kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, g, kElementBytes);
-        if (behind_sum != nullptr)
-            result = hipEventRecord(behind_sum, stream);
-    }
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (behind_terms != nullptr || behind_sum != nullptr)
+        (void)hipStreamIsCapturing(stream, &capturing);
+    // (an event rides on the kernel's own completion signal where the stream is not being captured: a record of its own is
+    // one more packet for the launches behind it to wait for)
+    const auto launch = [&](hipEvent_t behind, auto kernel, auto... arguments) {
+        if (behind != nullptr && capturing == hipStreamCaptureStatusNone)
+            hipExtLaunchKernelGGL(kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, nullptr, behind, 0, arguments...);
+        else
+        {
+            hipLaunchKernelGGL(kernel, dim3(kBinGrid), dim3(kBinThreads), 0, stream, arguments...);
+            if (behind != nullptr && result == hipSuccess)
+                result = hipEventRecord(behind, stream);
+        }
+    };
+    launch(nullptr, bin_stats_kernel<DTYPE>, g);
+    launch(behind_terms, bin_terms_kernel<DTYPE>, g);
+    launch(behind_sum, bin_sum_kernel, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
     if (a.rows <= kRoomyRows)
         launch_bin_walks<DTYPE, true>(g, stream);
     else
@@ -354,7 +369,8 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
 // their three passes took 110 us, alone 70, and the walks behind them hardly use it.  So the second stream starts behind those
 // passes, with the windows, whose second kernel is a chain as well, in front of the select; the select leaves the rows of both
 // alone, since one of them may be finished by then.  512 rows of 129,280, mixed options: 351 us one behind the other, 256 us
-// with select and windows beside the passes, 227 us with them behind, select first, and 223 us so.
+// with select and windows beside the passes, 227 us with them behind, select first, and 223 us so.  Where the windows are far
+// more than the sums (windows_go_ahead) their candidates start behind the terms already.
 template <int DTYPE>
 hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
                             bool want_filters, hipStream_t stream)
@@ -370,12 +386,26 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
     if (side_by_side && windows && sums && s->side_stream != nullptr)
     {
         list_rows();
-        hipError_t result = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, s->side_fork, stream);
+        WindowArgs w = window_args(s, a, listing, nullptr);
+        // (a call of fewer logits than the rule asks for has no launch for it)
+        const bool may_go_ahead = static_cast<uint64_t>(a.rows) * a.vocab >= kWindowsAheadLogits;
+        hipError_t result = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, may_go_ahead ? s->cut_done : nullptr, s->side_fork, stream);
+        if (may_go_ahead)
+        {
+            if (result == hipSuccess)
+                result = hipStreamWaitEvent(s->side_stream, s->cut_done, 0);
+            if (result != hipSuccess)
+                return result;
+            w.turn = kWindowsAhead;
+            launch_window_candidates<DTYPE>(w, s->side_stream);
+            w.turn = kWindowsBehind;
+        }
         if (result == hipSuccess)
             result = hipStreamWaitEvent(s->side_stream, s->side_fork, 0);
         if (result != hipSuccess)
             return result;
-        launch_windows<DTYPE>(s, a, listing, nullptr, s->side_stream);
+        launch_window_candidates<DTYPE>(w, s->side_stream);
+        launch_window_finish<DTYPE>(w, s->side_stream);
         SamplerArgs others = a;
         others.leave_later_rows = 1;
         select(others, s->side_stream);
@@ -386,8 +416,12 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
     select(a, stream);
     list_rows();
     if (windows)
-        launch_windows<DTYPE>(s, a, listing, sums ? s->bin_list : nullptr, stream);
-    return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, windows, want_filters, nullptr, stream) : hipSuccess;
+    {
+        const WindowArgs w = window_args(s, a, listing, sums ? s->bin_list : nullptr);
+        launch_window_candidates<DTYPE>(w, stream);
+        launch_window_finish<DTYPE>(w, stream);
+    }
+    return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, windows, want_filters, nullptr, nullptr, stream) : hipSuccess;
 }
 
 // Enqueues the sampling path for `rows` rows.  want_filters: the rows without a window leave their filtered distributions

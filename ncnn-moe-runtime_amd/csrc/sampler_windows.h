@@ -40,7 +40,34 @@ struct WindowArgs
     uint32_t windows_are_selects; // as in BinArgs
     uint32_t listing;
     uint32_t* other_list;   // where the sums' rows are listed as well (null: nowhere)
+    uint32_t turn;          // WindowTurn
+    const uint32_t* sums_list; // of the two turns: the sums' rows, listed by an earlier launch
 };
+
+// Beside the binned sums the candidates are collected by one of two launches, and the other leaves at once: the number of rows
+// of each kind is known to the device only.
+enum WindowTurn : uint32_t
+{
+    kWindowsOnce = 0,
+    kWindowsAhead = 1,  // behind the launch that writes the sums' terms: where the windows are the longer piece of work
+    kWindowsBehind = 2  // behind the last launch that reads the sums' rows as a stream: everywhere else
+};
+
+// Are the windows so much more than the sums that what streams them should not wait for the sums' passes?  The passes over a few
+// dozen rows are chains that leave the memory idle, some 45 us, and the walks behind them hide no more than the stream of some 500
+// rows of 129,280.  Rows with windows and rows without one, us ahead / behind (Top-K 300, normal logits of spread 2 and 3): 900 and 32
+// of 1,024 of 129,280 306 / 352 and 286 / 347, 640 and 32 298 / 306 and 274 / 303, 1,900 and 64 of 2,048 462 / 562 and 446 / 557,
+// 2,200 and 64 of 4,096 of 32,000 358 / 401 and 348 / 397, 500 and 64 of 600 of 262,144 390 / 389 and 343 / 380.  With more rows to
+// sum behind is faster (640 and 100 of 1,024 335 / 313 and 301 / 301, 1,024 and 500 of 2,048 730 / 676 and 638 / 634), and with fewer
+// windows it depends on how long the walks are (400 and 32 of 512, spread 1.5 270 / 247, 2 232 / 250, 3 211 / 241; 230 and 32 of 256 of
+// 151,936 198 / 170; 92 and 92 of 512 252 / 226).
+constexpr uint32_t kWindowsAheadRatio = 7;
+constexpr uint64_t kWindowsAheadLogits = 1ull << 26;
+
+__device__ __forceinline__ bool windows_go_ahead(uint32_t windows, uint32_t sums, uint32_t vocab)
+{
+    return windows >= kWindowsAheadRatio * sums && static_cast<uint64_t>(windows) * vocab >= kWindowsAheadLogits;
+}
 
 struct WindowCandidatesShared
 {
@@ -532,6 +559,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void window_candidates_kernel(Windo
     __shared__ WindowCandidatesShared shared;
     __shared__ RowList listed_rows;
     const uint32_t rows = list_rows_in_place(g.a, g.listing, true, true, g.list, g.other_list, listed_rows, threadIdx.x);
+    if (g.turn != kWindowsOnce && windows_go_ahead(rows, g.sums_list[0], g.a.vocab) != (g.turn == kWindowsAhead))
+        return;
     window_candidates<DTYPE>(g, bin_grid(rows, g.a.vocab), listed_rows, shared, threadIdx.x);
 }
 

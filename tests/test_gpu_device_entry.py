@@ -195,3 +195,50 @@ def test_rows_listed_by_the_first_launch_or_by_one_of_their_own(rows):
             for passes in flags:
                 gpu = _run(sampler, logits, params, uniforms, passes, stream)
                 parity_util.assert_results_match(gpu, cpu, "f32", "%d rows of %s, passes %d" % (rows, kinds, passes))
+
+
+@pytest.mark.parametrize("rows,vocab,windows,sums", [(320, 262147, 256, 36), (320, 262147, 256, 37), (320, 262143, 256, 36), (257, 262147, 256, 0), (1100, 65537, 1024, 40)])
+def test_windows_that_go_ahead_of_the_sums(rows, vocab, windows, sums):
+    """Side by side, windows of 2^26 logits and more and of seven rows and more for each row without one start before the sums'
+    passes have ended: on both sides of both limits, with the rows listed in place and by a launch, eager and captured, the rows'
+    results are those of the passes one behind the other, and the oracle's."""
+    print("[case] windows ahead, %d x %d, %d windows, %d sums" % (rows, vocab, windows, sums), flush=True)
+    rng = np.random.default_rng(windows + sums)
+    generator = torch.Generator(device="cuda:0").manual_seed(vocab)
+    d_logits = torch.randn(rows, vocab, device="cuda:0", generator=generator).mul_(2.0)
+    params = hip_sampler.make_params(rows, 0.9, 20, 0.93, 0.0)
+    kinds = rng.permutation(rows)
+    params["top_k"][kinds[:windows]] = rng.choice(np.array([65, 300, 1024], dtype=np.uint32), windows)
+    params["top_k"][kinds[windows:windows + sums]] = 0
+    uniforms = rng.random(rows, dtype=np.float32)
+    d_params, d_uniforms = _device(params.view(np.uint8)), _device(uniforms)
+    d_results = torch.zeros(rows * 16, dtype=torch.uint8, device="cuda:0")
+    stream = torch.cuda.Stream(device="cuda:0")
+    torch.cuda.synchronize()
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        def enqueue(passes):
+            sampler.sample_device(d_logits.data_ptr(), hip_sampler.LOGITS_F32, rows, vocab, vocab, d_params.data_ptr(), d_uniforms.data_ptr(),
+                                  None, d_results.data_ptr(), passes, stream.cuda_stream)
+
+        def results():
+            torch.cuda.synchronize()
+            out = d_results.cpu().numpy().view(hip_sampler.RESULT_DTYPE).reshape(rows)
+            d_results.zero_()
+            torch.cuda.synchronize()
+            return out
+
+        enqueue(hip_sampler.PASSES_FULL_ORDER)
+        in_turn = results()
+        beside_flags = hip_sampler.PASSES_FULL_ORDER | hip_sampler.PASSES_SIDE_BY_SIDE
+        for _ in range(2):
+            enqueue(beside_flags)
+            assert results().tobytes() == in_turn.tobytes()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            enqueue(beside_flags)
+        for _ in range(3):
+            graph.replay()
+            assert results().tobytes() == in_turn.tobytes()
+    checked = np.concatenate([kinds[:8], kinds[windows:windows + min(sums, 8)], kinds[-4:]])
+    cpu = parity_util.run_oracle(d_logits[torch.from_numpy(checked).to("cuda:0")].cpu().numpy(), params[checked], uniforms[checked])
+    parity_util.assert_results_match(in_turn[checked], cpu, "f32", "windows ahead")
