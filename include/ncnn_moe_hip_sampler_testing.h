@@ -64,6 +64,9 @@ int ncnn_moe_hip_sampler_debug_wide_sampled_bound(ncnn_moe_hip_sampler* sampler,
  * few launches in front of the point where the epochs start over. */
 int ncnn_moe_hip_sampler_debug_set_row_epochs(ncnn_moe_hip_sampler* sampler, int device, uint32_t epoch);
 int ncnn_moe_hip_sampler_debug_expf(ncnn_moe_hip_sampler* sampler, const float* in, float* out, size_t n);
+/* quotients[i] = dividends[i] / divisors[i] as the binned sums divide a bin's terms (Divisor of sampler_bins.h). */
+int ncnn_moe_hip_sampler_debug_quotients(
+    ncnn_moe_hip_sampler* sampler, const float* dividends, const float* divisors, float* quotients, size_t n);
 void ncnn_moe_hip_sampler_debug_exp2_table(uint64_t out[32]);
 
 /* How the first select kernel covers a batch of this shape (rows aligned to 16 bytes): workgroups per

@@ -9,6 +9,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -760,6 +761,43 @@ __global__ void static_scratch_clear_kernel(StaticScratchLayout* layout)
             layout->split_records[static_cast<size_t>(i) * kSplitRecordSlots + entry] = 0ull; // epoch 0 tags nothing
     }
 }
+
+#ifdef NCNN_MOE_TESTING
+// `launch` on n values of each of `inputs`, copied to the device and its n results copied back.
+template <size_t INPUTS, typename Launch>
+int probe_values(ncnn_moe_hip_sampler* s, const std::array<const float*, INPUTS>& inputs, float* out, size_t n, const char* what, Launch launch)
+{
+    if (s == nullptr || out == nullptr)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    for (const float* input : inputs)
+    {
+        if (input == nullptr)
+            return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    }
+    if (n == 0)
+        return NCNN_MOE_SAMPLER_SUCCESS;
+    SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
+    float* device = nullptr;
+    SAMPLER_HIP_CHECK(s, hipMalloc(&device, (INPUTS + 1) * n * sizeof(float)));
+    hipError_t error = hipSuccess;
+    for (size_t i = 0; i < INPUTS && error == hipSuccess; ++i)
+        error = hipMemcpy(device + i * n, inputs[i], n * sizeof(float), hipMemcpyHostToDevice);
+    if (error == hipSuccess)
+    {
+        launch(device, device + INPUTS * n, static_cast<unsigned>((n + 255) / 256));
+        error = hipGetLastError();
+    }
+    if (error == hipSuccess)
+        error = hipStreamSynchronize(s->stream);
+    if (error == hipSuccess)
+        error = hipMemcpy(out, device + INPUTS * n, n * sizeof(float), hipMemcpyDeviceToHost);
+    (void)hipFree(device);
+    if (error != hipSuccess)
+        return hip_fail(s, error, what);
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+#endif
 
 } // namespace
 
@@ -1649,33 +1687,16 @@ int ncnn_moe_hip_sampler_debug_stream_only(
 
 int ncnn_moe_hip_sampler_debug_expf(ncnn_moe_hip_sampler* s, const float* in, float* out, size_t n)
 {
-    if (s == nullptr || in == nullptr || out == nullptr)
-        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
-    if (n == 0)
-        return NCNN_MOE_SAMPLER_SUCCESS;
-    SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
-    float* device_in = nullptr;
-    float* device_out = nullptr;
-    SAMPLER_HIP_CHECK(s, hipMalloc(&device_in, n * sizeof(float)));
-    hipError_t error = hipMalloc(&device_out, n * sizeof(float));
-    if (error == hipSuccess)
-        error = hipMemcpy(device_in, in, n * sizeof(float), hipMemcpyHostToDevice);
-    if (error == hipSuccess)
-    {
-        const unsigned blocks = static_cast<unsigned>((n + 255) / 256);
-        hipLaunchKernelGGL(expf_probe_kernel, dim3(blocks), dim3(256), 0, s->stream, device_in, device_out, n);
-        error = hipGetLastError();
-    }
-    if (error == hipSuccess)
-        error = hipStreamSynchronize(s->stream);
-    if (error == hipSuccess)
-        error = hipMemcpy(out, device_out, n * sizeof(float), hipMemcpyDeviceToHost);
-    (void)hipFree(device_in);
-    if (device_out != nullptr)
-        (void)hipFree(device_out);
-    if (error != hipSuccess)
-        return hip_fail(s, error, "debug_expf");
-    return NCNN_MOE_SAMPLER_SUCCESS;
+    return probe_values<1>(s, {in}, out, n, "debug_expf", [=](const float* values, float* results, unsigned blocks) {
+        hipLaunchKernelGGL(expf_probe_kernel, dim3(blocks), dim3(256), 0, s->stream, values, results, n);
+    });
+}
+
+int ncnn_moe_hip_sampler_debug_quotients(ncnn_moe_hip_sampler* s, const float* dividends, const float* divisors, float* quotients, size_t n)
+{
+    return probe_values<2>(s, {dividends, divisors}, quotients, n, "debug_quotients", [=](const float* values, float* results, unsigned blocks) {
+        hipLaunchKernelGGL(quotient_probe_kernel, dim3(blocks), dim3(256), 0, s->stream, values, values + n, results, n);
+    });
 }
 
 #ifdef NCNN_MOE_TIMELINE

@@ -716,8 +716,8 @@ __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&fro
 // Correctly rounded quotients by one divisor: two corrections of dividend x reciprocal, each with its exact remainder (P. Markstein,
 // Computation of elementary functions on the IBM RISC System/6000 processor, 1990: a quotient less than an ulp off, corrected with
 // the remainder times the correctly rounded reciprocal, is the correctly rounded one).  Five instructions instead of the ten and a
-// reciprocal of a division; for numbers whose quotient and remainder are far from the denormal ones, as the bins' terms are (compared
-// with the division for 4,000 divisors and every mantissa of the dividend).
+// reciprocal of a division; for numbers whose quotient and remainder are far from the denormal ones, as the bins' terms are: they are
+// 2^-25 to 1, a normaliser is 1 to 2^22, the divisor behind it no less than the first term over the normaliser, 2^-22.
 struct Divisor
 {
     float value, reciprocal;

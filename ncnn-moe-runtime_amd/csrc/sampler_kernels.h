@@ -31,6 +31,14 @@ __global__ void expf_probe_kernel(const float* in, float* out, size_t n)
     if (i < n)
         out[i] = expf_libm(in[i]);
 }
+
+// Divisor (sampler_bins.h) on n pairs of values (test hook, as above).
+__global__ void quotient_probe_kernel(const float* dividends, const float* divisors, float* quotients, size_t n)
+{
+    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n)
+        quotients[i] = Divisor(divisors[i]).divide(dividends[i]);
+}
 #endif
 
 } // namespace ncnn_moe_hip

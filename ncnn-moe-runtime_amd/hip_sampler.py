@@ -85,6 +85,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_stream_only",
     "ncnn_moe_hip_sampler_debug_set_row_epochs",
     "ncnn_moe_hip_sampler_debug_expf",
+    "ncnn_moe_hip_sampler_debug_quotients",
     "ncnn_moe_hip_sampler_debug_exp2_table",
     "ncnn_moe_hip_sampler_debug_select_geometry",
 ]
@@ -139,6 +140,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_stream_only.argtypes = [vp, vp, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, vp]
     lib.ncnn_moe_hip_sampler_debug_set_row_epochs.argtypes = [vp, ctypes.c_int, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_expf.argtypes = [vp, vp, vp, ctypes.c_size_t]
+    lib.ncnn_moe_hip_sampler_debug_quotients.argtypes = [vp, vp, vp, vp, ctypes.c_size_t]
     lib.ncnn_moe_hip_sampler_debug_exp2_table.argtypes = [vp]
     lib.ncnn_moe_hip_sampler_debug_exp2_table.restype = None
     lib.ncnn_moe_hip_sampler_debug_select_geometry.argtypes = [
@@ -403,6 +405,16 @@ class HipSampler:
         values = np.ascontiguousarray(values, dtype=np.float32)
         out = np.empty_like(values)
         self._check(self._hooks().ncnn_moe_hip_sampler_debug_expf(self._handle, values.ctypes.data, out.ctypes.data, values.size))
+        return out
+
+    def quotients(self, dividends, divisors):
+        """Test hook: dividends / divisors as the binned sums divide."""
+        dividends = np.ascontiguousarray(dividends, dtype=np.float32)
+        divisors = np.ascontiguousarray(divisors, dtype=np.float32)
+        assert dividends.shape == divisors.shape
+        out = np.empty_like(dividends)
+        self._check(self._hooks().ncnn_moe_hip_sampler_debug_quotients(
+            self._handle, dividends.ctypes.data, divisors.ctypes.data, out.ctypes.data, dividends.size))
         return out
 
 

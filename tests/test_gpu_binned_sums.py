@@ -243,3 +243,32 @@ def test_heads_that_hold_the_top_p_and_heads_that_end_before_it(spread, vocab):
     with hip_sampler.HipSampler(rows, vocab) as sampler:
         sampler.upload_logits(logits)
         parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "heads, %d of spread %g" % (vocab, spread))
+
+
+@pytest.mark.parametrize("exponent", [-22, -1, 0, 1, 21])
+def test_quotients_of_terms_are_correctly_rounded(exponent):
+    """The quotients that the sums add up as whole steps, against numpy's division (correctly rounded): every mantissa of the
+    dividend by divisors of the kinds at which a corrected quotient can go wrong (at and next to a power of two, 2/3 and 4/3, sqrt 2,
+    the last mantissas) and random ones, then random pairs, over the terms' and divisors' whole range."""
+    rng = np.random.default_rng(exponent + 100)
+    print("[case] quotients, divisors of 2^%d" % exponent, flush=True)
+    mantissas = np.concatenate([np.array([0, 1, 2, 3, 0x7fffff, 0x7ffffe, 0x7ffffd, 0x555555, 0x2aaaab, 0x3504f3, 0x400000], dtype=np.uint32),
+                                rng.integers(0, 1 << 23, 5).astype(np.uint32)])
+    divisors = ((np.uint32(127 + exponent) << 23) | mantissas).astype(np.uint32).view(np.float32)
+    every = np.arange(1 << 23, dtype=np.uint32)
+    with hip_sampler.HipSampler(1, 64, testing=True) as sampler:
+        for i, divisor in enumerate(divisors):
+            term_exponent = -25 + (7 * i) % 25
+            dividends = ((np.uint32(127 + term_exponent) << 23) | every).view(np.float32)
+            quotients = sampler.quotients(dividends, np.full_like(dividends, divisor))
+            wrong = np.nonzero(quotients.view(np.uint32) != (dividends / divisor).view(np.uint32))[0]
+            assert wrong.size == 0, "%r / %r" % (dividends[wrong[0]], divisor)
+        some = 1 << 23
+        dividends = (((127 - rng.integers(0, 26, some)) << 23) | rng.integers(0, 1 << 23, some)).astype(np.uint32).view(np.float32)
+        divisors = ((np.uint32(127 + exponent) << 23) | rng.integers(0, 1 << 23, some).astype(np.uint32)).view(np.float32)
+        quotients = sampler.quotients(dividends, divisors)
+        assert np.array_equal(quotients.view(np.uint32), (dividends / divisors).view(np.uint32))
+        # ... and a quotient divided again, as the draw's terms are
+        again = (((127 - rng.integers(1, 23, some)) << 23) | rng.integers(0, 1 << 23, some)).astype(np.uint32).view(np.float32)
+        if exponent >= 0:
+            assert np.array_equal(sampler.quotients(quotients, again).view(np.uint32), (quotients / again).view(np.uint32))
