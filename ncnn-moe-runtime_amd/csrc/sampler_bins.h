@@ -1552,12 +1552,13 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
         const float chunk_front = wave_prefix_sum_f32(chunk_sum) - chunk_sum;
         for (uint32_t i = kInOrder * kWaveSize + 4u * static_cast<uint32_t>(tid - kWaveSize); same_in_all(i) < count; i += 4u * (WAVES - 1) * kWaveSize)
         {
-            const float4 raw = *reinterpret_cast<const float4*>(terms + i);
+            // (the last wave's lanes may lie behind the last chunk: those have no terms, and no place in the scratch)
+            const float4 raw = *reinterpret_cast<const float4*>(terms + (i < count ? i : 0u));
             const float own[4] = {i < count ? scaled(raw.x) : 0.0f, i + 1u < count ? scaled(raw.y) : 0.0f, i + 2u < count ? scaled(raw.z) : 0.0f,
                                   i + 3u < count ? scaled(raw.w) : 0.0f};
             const uint32_t exponent = __float_as_uint(__shfl(chunk_front, static_cast<int>(i / kWaveSize), kWaveSize) * scale) >> 23;
             const ParityStep through = row16_steps(own, static_cast<int>(exponent));
-            if ((tid & 15) == 15)
+            if ((tid & 15) == 15 && i / kWaveSize < chunks)
             {
                 scratch.chunk_exponent[i / kWaveSize] = exponent;
                 scratch.chunk_even[i / kWaveSize] = through.even;

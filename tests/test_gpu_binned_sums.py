@@ -245,6 +245,30 @@ def test_heads_that_hold_the_top_p_and_heads_that_end_before_it(spread, vocab):
         parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "heads, %d of spread %g" % (vocab, spread))
 
 
+@pytest.mark.parametrize("first_bin", [3967, 3968, 3969, 4032, 4033, 4095, 4096, 4097])
+@pytest.mark.parametrize("behind", [0, 900])
+def test_heads_of_one_bin_up_to_the_whole_list(first_bin, behind):
+    """A first bin is in the head whatever it holds, up to the list's 4,096 elements: heads that end in the last 64 of them, of
+    equal and of unequal terms, with and without elements behind, ended by the row, by Top-P, by Min-P and by the draw."""
+    rng = np.random.default_rng(first_bin + behind)
+    rows, vocab = 12, first_bin + behind
+    print("[case] one bin of %d, %d behind" % (first_bin, behind), flush=True)
+    logits = np.full((rows, vocab), 0.5, dtype=np.float32)
+    logits[1::2, :first_bin] += rng.random((rows // 2, first_bin), dtype=np.float32) * np.float32(0.003)
+    logits[:, first_bin:] -= rng.random((rows, behind), dtype=np.float32) * np.float32(6.0) + np.float32(0.02)
+    logits = np.ascontiguousarray(rng.permuted(logits, axis=1))
+    uniforms = np.linspace(0.0, 0.97, rows).astype(np.float32)  # (a draw that no partial sum exceeds is the sort's)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        for top_p, min_p in ((1.0, 0.0), (0.97, 0.0), (0.5, 0.0), (1.0, 0.99), (1e-6, 0.0)):
+            params = hip_sampler.make_params(rows, 1.0, 0, top_p, min_p)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "one bin of %d, top_p %g min_p %g" % (first_bin, top_p, min_p))
+            if first_bin <= 4096:
+                assert sampler.binned_rows(rows).tolist() == [1] * rows, (top_p, min_p)
+
+
 @pytest.mark.parametrize("exponent", [-22, -1, 0, 1, 21])
 def test_quotients_of_terms_are_correctly_rounded(exponent):
     """The quotients that the sums add up as whole steps, against numpy's division (correctly rounded): every mantissa of the
