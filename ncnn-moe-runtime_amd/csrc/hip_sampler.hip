@@ -326,17 +326,18 @@ WindowArgs window_args(const ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowL
     return w;
 }
 
-// The binned sums (sampler_bins.h) over the rows in the handle's bin list.  `behind_terms`, `behind_sum` (null: none): events
-// behind the launch that writes the rows' terms and behind the last one that reads a row as a stream.
+// The binned sums (sampler_bins.h) over the rows in the handle's bin list (`window_list`: see BinArgs).  `behind_terms`, `behind_sum`
+// (null: none): events behind the launch that writes the rows' terms and behind the last one that reads a row as a stream.
 template <int DTYPE>
-hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, bool windows, bool want_filters, hipEvent_t behind_terms,
-                           hipEvent_t behind_sum, hipStream_t stream)
+hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowListing listing, uint32_t* window_list, bool windows, bool want_filters,
+                           hipEvent_t behind_terms, hipEvent_t behind_sum, hipStream_t stream)
 {
     BinArgs g = s->bins;
     g.a = a;
     g.windows_are_selects = windows ? 1u : 0u;
     g.want_filters = want_filters ? 1u : 0u;
     g.listing = listing;
+    g.window_list = window_list;
     hipError_t result = hipSuccess;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (behind_terms != nullptr || behind_sum != nullptr)
@@ -387,10 +388,12 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
     if (side_by_side && windows && sums && s->side_stream != nullptr)
     {
         list_rows();
-        WindowArgs w = window_args(s, a, listing, nullptr);
+        // (the sums' first launch lists the windows' rows too.  A launch of candidates that leaves at once costs nothing that shows then,
+        // and 6 of 262 us where each of its workgroups lists them beside the sums' last pass: 1,024 x 129,280, 100 windows and 32 rows to sum)
+        WindowArgs w = window_args(s, a, kRowsListed, nullptr);
         // (a call of fewer logits than the rule asks for has no launch for it)
         const bool may_go_ahead = static_cast<uint64_t>(a.rows) * a.vocab >= kWindowsAheadLogits;
-        hipError_t result = launch_bin_sums<DTYPE>(s, a, listing, windows, want_filters, may_go_ahead ? s->cut_done : nullptr, s->side_fork, stream);
+        hipError_t result = launch_bin_sums<DTYPE>(s, a, listing, s->window_list, windows, want_filters, may_go_ahead ? s->cut_done : nullptr, s->side_fork, stream);
         if (may_go_ahead)
         {
             if (result == hipSuccess)
@@ -422,7 +425,7 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
         launch_window_candidates<DTYPE>(w, stream);
         launch_window_finish<DTYPE>(w, stream);
     }
-    return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, windows, want_filters, nullptr, nullptr, stream) : hipSuccess;
+    return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, nullptr, windows, want_filters, nullptr, nullptr, stream) : hipSuccess;
 }
 
 // Enqueues the sampling path for `rows` rows.  want_filters: the rows without a window leave their filtered distributions

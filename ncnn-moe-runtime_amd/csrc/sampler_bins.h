@@ -161,6 +161,7 @@ struct BinArgs
     uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
     uint32_t listing;      // RowListing: how the first launch finds its rows
+    uint32_t* window_list; // where it lists those with a window as well (null: nowhere; see list_rows_in_place)
 };
 
 __device__ __forceinline__ uint32_t same_in_all(uint32_t value)
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
     const SamplerArgs& a = g.a;
     __shared__ RowList listed_rows;
     const int tid = threadIdx.x;
-    const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, nullptr, listed_rows, tid);
+    const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
     const BinGrid grid = bin_grid(rows, a.vocab);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
