@@ -3,6 +3,9 @@
 #include "ncnn_moe_hip_sampler_testing.h"
 
 #include "sampler_kernels.h"
+#ifdef NCNN_MOE_TIMELINE
+#include "hip_leftover_rows.hip" // (one unit, so that its stamps go to the array that is read)
+#endif
 #include "sampler_verify.h"
 
 #include <hip/hip_runtime.h>
