@@ -135,11 +135,14 @@ int ncnn_moe_hip_sampler_sample(
  * for Top-K windows up to 1024, for rows without a window and for what those leave are enqueued as
  * well and pick up the rows that need them); pass 3 (1 | NCNN_MOE_PASSES_SIDE_BY_SIDE) when the
  * caller knows that the batch holds both rows with 64 < top_k <= 1024 and rows with a wider or no
- * window: the first kernel and those for wide windows then run beside those for rows without one, on
- * a second stream of the handle that forks from and joins `stream` (worth its stream hand-overs from
- * some dozens of rows of each kind; a row with top_k <= 64 whose ties overflow the first kernel's
- * lists is then finished by the full-order kernels: same result, NCNN_MOE_ROW_FLAG_GENERAL_PATH
- * set); add NCNN_MOE_PASSES_NO_WIDE_WINDOWS when the caller knows that no row has
+ * window: of fp32 logits the first kernel and those for wide windows are then enqueued on a second
+ * stream of the handle that forks from and joins `stream`: behind the kernels that read the rows without
+ * a window, beside those that finish them (where wide windows are far more, their first kernel starts
+ * earlier, behind the one that writes the other rows' terms); rows of more than 2^19 logits of either
+ * type have the kernels for wide windows beside all of those for rows without one, shorter bf16 rows
+ * gain nothing (worth its stream hand-overs from some dozens of rows of each kind; a row with
+ * top_k <= 64 whose ties overflow the first kernel's lists is then finished by the full-order kernels:
+ * same result, NCNN_MOE_ROW_FLAG_GENERAL_PATH set); add NCNN_MOE_PASSES_NO_WIDE_WINDOWS when the caller knows that no row has
  * 64 < top_k <= 1024: the kernels for such windows are then not enqueued (a row that has one after
  * all is served like one without a window: slower, same result).
  * Calls on one handle share its scratch memory and must not overlap. */

@@ -9,8 +9,8 @@
 namespace ncnn_moe_hip {
 
 // Sort and replay in ONE kernel: hardly any row is left, and a launch that finds none costs 2.3 us all the same, most of it the gap
-// between two launches (33 x 100,003, windows of 200: 52.3 us with two kernels, 50.0 us so; 8 x 151,936 without a window 119.1
-// and 116.6 us).
+// between two launches (33 x 100,003, windows of 200: 52.4 us with two kernels, 51.0 us so; 8 x 151,936 without a window 119.1
+// and 117.8 us).
 static __global__ __launch_bounds__(kSortThreads) void sort_and_replay_kernel(SamplerArgs a)
 {
     static_assert(kSortThreads == kReplayThreads, "the sort and the walk share a workgroup");

@@ -374,8 +374,13 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
 // their three passes took 110 us, alone 70, and the walks behind them hardly use it.  So the second stream starts behind those
 // passes, with the windows, whose second kernel is a chain as well, in front of the select; the select leaves the rows of both
 // alone, since one of them may be finished by then.  512 rows of 129,280, mixed options: 351 us one behind the other, 256 us
-// with select and windows beside the passes, 227 us with them behind, select first, and 223 us so.  Where the windows are far
-// more than the sums (windows_go_ahead) their candidates start behind the terms already.
+// with select and windows beside the passes, 227 us with them behind, select first, and 223 us so.  Elsewhere, select and windows
+// beside the passes / so (Top-K 300 and 20, rows with a window and without, normal logits of spread 2): 1,024 rows of 129,280 with 64
+// and 64 319 / 276 us, 32 and 32 290 / 261, 200 and 200 402 / 373, 500 and 200 455 / 387, 512 with 64 and 32 228 / 210, 2,048 with 64
+// and 64 389 / 351, 512 of 32,000 with 40 and 40 179 / 163, 256 of 8,000 with 100 and 100 140 / 134; where the select is nearly all
+// of the call or there is none, 4,096 of 129,280 with 64 and 64 511 / 518, of 32,000 271 / 272 (spread 3: 241 / 250), 64 of 129,280
+// with 32 and 32 196 / 201.  Where the windows are far more than the sums (windows_go_ahead) their candidates start behind the
+// terms already.
 template <int DTYPE>
 hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const SelectGeometry& geometry, bool windows, bool sums, bool side_by_side,
                             bool want_filters, hipStream_t stream)

@@ -952,6 +952,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         // unless the longest head holds the row's Top-P as well, and with it the ends of the second and third walk (64 x 4,096,
         // Top-P 0.95: 81.8 us with the head that ends early, 58.8 us so), or nearly: most draws end in it then (100 x 8,192, Top-P
         // 0.9: 114.1 us where it has to hold all of it, 104.4 us so; 32 x 32,000 and 8 x 151,936, whose heads hold less, as before).
+        // What counts as nearly matters little: over 100 x 4,096, 8,192 and 16,384, 32 x 16,384 and 32,000 and 8 x 151,936, Top-P 0.8 to
+        // 0.99 and spreads of 2 to 3, the mean of 72 such calls is 96.0 us at 0.5, 95.9 at 0.7 to 0.85, 96.2 at 0.9 and 97.9 at 1.
         const bool window_in_head = window <= kBinHead;
         {
             // (the bins of a head are the first ones: one that is not of it ends it)
