@@ -47,8 +47,9 @@ constexpr uint32_t kOneBits = 0x3f800000u;       // the largest term
 constexpr uint32_t kTailDistance = kBinBinades << 23; // in bits below it: terms of 2^-25 or less move no sum
 constexpr float kTailArgument = -17.4f;          // exp of anything less is below 2^-25 (2^-25 = exp(-17.33))
 constexpr uint32_t kOffsetBits = 12;             // where in its bin a term lies, summed per bin
-constexpr uint32_t kBinHead = 1920;              // elements of the sorted head at most (unless a window takes more), 30 chunks of sum_head: behind
-                                                 // so many a term half way seldom has to be fetched, 9 us and more each
+constexpr uint32_t kBinHead = 1920;              // elements of the sorted head at most, 30 chunks of sum_head: behind so many a term half
+                                                 // way seldom has to be fetched, 9 us and more each
+constexpr uint32_t kBinWholeRow = 2048;          // ... unless these are all that the sums run over
 constexpr uint32_t kBinListCap = 4096;           // head and foreseen bins, elements
 constexpr uint32_t kBinExtraCap = 1536;          // elements fetched on demand at a time
 constexpr uint32_t kBinStops = 512;
@@ -946,7 +947,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
             for (int j = 0; j < 4; ++j)
                 mass[j + 1] = mass[j] + own[j];
         }
-        // The head: as many bins as hold kBinHead elements at most, or those that hold the whole of a window that narrow.  Where a
+        // The head: as many bins as hold kBinHead elements at most, or those that hold the whole of a narrow window.  Where a
         // bin's terms are kWideDifference binades below the sum, its masks tell how those half way are rounded, and a sorted head
         // would save the walk nothing: it ends there (two binades further: verification without a window 168 us instead of 163)
         // unless the longest head holds the row's Top-P as well, and with it the ends of the second and third walk (64 x 4,096,
@@ -954,14 +955,17 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         // 0.9: 114.1 us where it has to hold all of it, 104.4 us so; 32 x 32,000 and 8 x 151,936, whose heads hold less, as before).
         // What counts as nearly matters little: over 100 x 4,096, 8,192 and 16,384, 32 x 16,384 and 32,000 and 8 x 151,936, Top-P 0.8 to
         // 0.99 and spreads of 2 to 3, the mean of 72 such calls is 96.0 us at 0.5, 95.9 at 0.7 to 0.85, 96.2 at 0.9 and 97.9 at 1.
-        const bool window_in_head = window <= kBinHead;
+        // A row or a window of kBinWholeRow elements at most is all head, and its first walk its last: 300 x 2,000, Top-P 1, 158 us with
+        // heads of 1,920 at most, 85 us so.
+        const bool window_in_head = window <= kBinWholeRow;
+        const uint32_t most_in_head = binned <= kBinWholeRow ? kBinWholeRow : kBinHead;
         {
             // (the bins of a head are the first ones: one that is not of it ends it)
             uint32_t first_not[2] = {kBins, kBins};
 #pragma unroll
             for (int j = 3; j >= 0; --j)
             {
-                const bool in_longest = window_in_head ? front[j] < window : front[j + 1] <= kBinHead;
+                const bool in_longest = window_in_head ? front[j] < window : front[j + 1] <= most_in_head;
                 const bool told_by_masks = !window_in_head && bin_top(bin + j, shift) * static_cast<float>(1 << kWideDifference) < mass[j];
                 if (!in_longest && bin + j != 0u)
                     first_not[0] = bin + j;

@@ -245,6 +245,27 @@ def test_heads_that_hold_the_top_p_and_heads_that_end_before_it(spread, vocab):
         parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "heads, %d of spread %g" % (vocab, spread))
 
 
+@pytest.mark.parametrize("vocab", [1920, 1921, 2047, 2048, 2049, 5000])
+def test_rows_and_windows_that_are_all_head(vocab):
+    """Rows, finite prefixes and windows of 1,920 to 2,049 elements, which the sorted head holds whole or just does not, with sums
+    that run to their ends."""
+    rng = np.random.default_rng(vocab + 7)
+    rows = 24
+    print("[case] all head, %d" % vocab, flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * rng.uniform(0.3, 4.0, (rows, 1))).astype(np.float32)
+    logits[1::4] = np.round(logits[1::4] * 8) / 8
+    logits[2::4] -= np.where(rng.random((rows // 4, vocab)) < 0.1, np.float32(40.0), np.float32(0.0))  # terms that move no sum
+    if vocab == 5000:
+        logits[3::4, rng.permutation(vocab)[:vocab - 2048]] = -np.inf
+    uniforms = rng.random(rows, dtype=np.float32)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        for top_p, min_p, top_k in ((1.0, 0.0, 0), (0.9999, 0.0, 0), (0.9, 0.0, 0), (1.0, 1e-4, 0), (1.0, 0.0, 1921), (1.0, 0.0, 2048), (0.999, 0.0, 2049)):
+            params = hip_sampler.make_params(rows, 1.0, top_k, top_p, min_p)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "all head, %d top_p %g min_p %g top_k %d" % (vocab, top_p, min_p, top_k))
+
+
 @pytest.mark.parametrize("first_bin", [3967, 3968, 3969, 4032, 4033, 4095, 4096, 4097])
 @pytest.mark.parametrize("behind", [0, 900])
 def test_heads_of_one_bin_up_to_the_whole_list(first_bin, behind):
