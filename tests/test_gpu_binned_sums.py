@@ -266,6 +266,26 @@ def test_rows_and_windows_that_are_all_head(vocab):
             parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "all head, %d top_p %g min_p %g top_k %d" % (vocab, top_p, min_p, top_k))
 
 
+@pytest.mark.parametrize("vocab", [4096, 16384, 32003])
+@pytest.mark.parametrize("spread", [1.5, 2.5])
+def test_min_p_cuts_around_the_ends_of_heads(spread, vocab):
+    """Min-P cuts in front of the head that ends early, between it and the end of the longest one, and behind both."""
+    rng = np.random.default_rng(int(spread * 10) + vocab)
+    rows = 48
+    print("[case] cuts around heads, %d of spread %g" % (vocab, spread), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * spread).astype(np.float32)
+    logits[::6] = np.round(logits[::6] * 16) / 16
+    params = hip_sampler.make_params(rows, 1.0, 0, 1.0, 0.0)
+    params["min_p"] = np.geomspace(3e-4, 0.2, rows).astype(np.float32)
+    params["top_p"][1::3] = np.float32(0.9)
+    params["top_p"][2::3] = np.float32(0.999)
+    uniforms = rng.random(rows, dtype=np.float32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "cuts around heads, %d of spread %g" % (vocab, spread))
+
+
 @pytest.mark.parametrize("first_bin", [3967, 3968, 3969, 4032, 4033, 4095, 4096, 4097])
 @pytest.mark.parametrize("behind", [0, 900])
 def test_heads_of_one_bin_up_to_the_whole_list(first_bin, behind):
