@@ -33,6 +33,9 @@ int ncnn_moe_hip_sampler_debug_chunk_steps(ncnn_moe_hip_sampler* sampler, int en
  * first `rows` rows, 1 for a row that was finished that way the last time it was given to it. */
 int ncnn_moe_hip_sampler_debug_binned_sums(ncnn_moe_hip_sampler* sampler, int enabled);
 int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32_t* served, uint32_t rows);
+/* most_looks: how often a part of a row looks for the row's other parts before it gives the row up, which is then sorted (0:
+ * a part that has to wait gives up at once).  Same results either way. */
+int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* sampler, uint32_t looks);
 /* Which of the handle's first `rows` rows the binned sums left the filtered distribution of in the last verification step. */
 int ncnn_moe_hip_sampler_debug_filtered_rows(ncnn_moe_hip_sampler* sampler, uint32_t* filtered, uint32_t rows);
 /* spread_sort (on by default): the radix sort of a long full-order row runs on several workgroups; off,

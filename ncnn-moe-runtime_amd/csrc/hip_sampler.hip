@@ -296,14 +296,6 @@ struct SamplerPasses
     bool side_by_side = false; // the wide select on the handle's second stream, beside the full-order kernels
 };
 
-template <int DTYPE, bool ROOMY>
-void launch_bin_walks(const BinArgs& g, hipStream_t stream)
-{
-    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 0, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 1, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-    hipLaunchKernelGGL((bin_walk_kernel<DTYPE, 2, ROOMY>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-}
-
 // The window kernels (sampler_windows.h) over the rows in the handle's window list (`other_list`: see list_rows_in_place).
 template <int DTYPE>
 void launch_window_candidates(const WindowArgs& w, hipStream_t stream)
@@ -361,9 +353,9 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
     launch(behind_terms, bin_terms_kernel<DTYPE>, g);
     launch(behind_sum, bin_sum_kernel, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
     if (a.rows <= kRoomyRows)
-        launch_bin_walks<DTYPE, true>(g, stream);
+        hipLaunchKernelGGL((bin_walks_kernel<DTYPE, true>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
     else
-        launch_bin_walks<DTYPE, false>(g, stream);
+        hipLaunchKernelGGL((bin_walks_kernel<DTYPE, false>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
     return result;
 }
 
@@ -884,6 +876,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->row_state, rows * sizeof(uint32_t));
     place(&s->windows.counts, rows * sizeof(uint32_t));
     place(&s->windows.flags, rows * sizeof(uint32_t));
+    place(&s->bins.arrivals, rows * kArrivalWords * sizeof(uint32_t));
     const size_t cleared = bytes;
     place(&s->row_epoch, rows * sizeof(uint32_t));
     place(&s->logits, rows * s->logits_stride_f32 * sizeof(float));
@@ -938,14 +931,13 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->bins.stats, pairs * sizeof(uint4));
     place(&s->bins.counts, pairs * 2 * kBins * sizeof(uint32_t));
     place(&s->bins.before, pairs * kBins * sizeof(uint32_t));
-    place(&s->bins.head_terms, rows * kBinListCap * sizeof(float));
+    place(&s->bins.packed, rows * kBins * sizeof(uint32_t));
     place(&s->bins.head_tokens, rows * kBinListCap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i)
     {
         place(&s->bins.steps[i], pairs * kBins * sizeof(uint32_t));
         place(&s->bins.ties[i], pairs * 3 * kBinWords * sizeof(uint32_t));
         place(&s->bins.masks[i], pairs * kMaskWords * sizeof(uint32_t));
-        place(&s->bins.packed[i], rows * kBins * sizeof(uint32_t));
         place(&s->bins.list_terms[i], rows * kBinListCap * sizeof(float));
         place(&s->bins.list_tokens[i], rows * kBinListCap * sizeof(uint32_t));
     }
@@ -956,6 +948,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     for (const auto& [pointer, offset] : buffers)
         *pointer = static_cast<uint8_t*>(s->device_memory) + offset;
     s->bins.list = s->bin_list;
+    s->bins.most_looks = kMostLooks;
     s->windows.list = s->window_list;
     CREATE_CHECK(hipMemsetAsync(s->device_memory, 0, cleared, s->stream));
     CREATE_CHECK(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(s->row_epoch), 1, rows, s->stream));
@@ -1501,6 +1494,15 @@ int ncnn_moe_hip_sampler_debug_binned_sums(ncnn_moe_hip_sampler* s, int enabled)
     if (s == nullptr)
         return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
     s->binned_sums = enabled ? 1 : 0;
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+// How often a part of a row looks for the others before it gives up (0: a part that has to wait gives up at once).
+int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* s, uint32_t looks)
+{
+    if (s == nullptr)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    s->bins.most_looks = looks;
     return NCNN_MOE_SAMPLER_SUCCESS;
 }
 

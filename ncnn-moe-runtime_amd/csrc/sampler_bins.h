@@ -20,13 +20,17 @@
 // at least 2^-24; the other two sums start at the first term divided by the same numbers as every other): such terms
 // are in no bin.  A foreseen exponent is checked against the exact sum before a bin's integer is used.
 //
-// Five or six launches serve every row of a call, each workgroup a part of one row: (1) maximum and counts, (2) terms
-// and bin counts, (3) head fetched, steps of the normaliser's sum, (4) normaliser walked, steps of the Top-P sum,
-// (5) Top-P walked, steps of the draw's sum, (6) draw walked.  A row whose walks end inside its head is finished by (4).
+// Four launches serve every row of a call, each workgroup a part of one row: (1) maximum and counts, (2) terms
+// and bin counts, (3) head fetched, steps of the normaliser's sum, (4) normaliser walked, steps of the Top-P sum, Top-P walked,
+// steps of the draw's sum, draw walked.  A row's three walks are one launch, in which its parts meet (parts_meet) where they hand
+// steps to each other: two microseconds with the loads of what was handed over, where another launch cost a gap of 2.6, 1.5
+// before it knew its row and some 2 for loads that found nothing in the L2 (8 rows of 151,936 without a window 105.3 -> 99.2 us,
+// 5 such drafts verified 170.3 -> 163.1; 33 windows of 200 among 100,003, for which the launches find no row, 51.3 -> 47.1; 512 rows
+// of 129,280 with mixed options 222.1 -> 218.2).
 //
-// What bounds it: at few rows the chain of launches and, inside (3) to (6), dependent instructions and trips to LDS and
-// memory (8 rows of 151,936: 6, 8, 16, 29, 26 and 14 us; of a walk some 5.5 us add the next sum's steps, bound by LDS
-// atomics); at a hundred rows and more the reads of the rows and their terms, and the slowest row's walk.
+// What bounds it: instructions, of which each SIMD has those of two wavefronts to issue, and trips to LDS and memory one behind the
+// other (8 rows of 151,936: 5, 5, 14, and 60 for the walks; of a walk some 5 us add the next sum's steps); at a hundred rows and
+// more the reads of the rows and their terms, and the slowest row's walk.
 #ifndef NCNN_MOE_HIP_SAMPLER_BINS_H
 #define NCNN_MOE_HIP_SAMPLER_BINS_H
 
@@ -75,6 +79,7 @@ constexpr uint32_t kBinComparedTies = 256;       // equal terms of a list that a
 constexpr uint32_t kMaxBinParts = 16;
 constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers in flight together
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
+constexpr uint32_t kArrivalWords = 32;           // of a row (see parts_meet): a cache line
 constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
 // The walks want 220 registers; at 128, which two of their workgroups to a compute unit leave, some 35 of them and 130
 // scalars pass through scratch and lane moves.  A call of so few rows that every part has a compute unit of its own takes
@@ -115,28 +120,22 @@ enum BinRowState : uint32_t
 // workgroups read the row's record at different times).
 struct BinRow
 {
-    uint32_t state[4];      // after launches (2), (3), (4), (5)
+    uint32_t state[2];      // after launches (2), (3)
     uint32_t shift;         // a term's bin: (kOneBits - bits) >> shift
     uint32_t window;        // elements of the Top-K window (finite logits at most)
     uint32_t binned;        // elements in bins
     uint32_t saw_nan;
     uint32_t head_bins;     // bins [0, head_bins) are the head, head_count elements
     uint32_t head_count;
-    uint32_t wide_first[3]; // of each walk's sum: the first of the kWideBins bins with wide masks
-    uint32_t listed[3];     // elements in the list of each walk (the first walk's holds the head, the others' places behind it)
-    float normalizer;
-    float head_sum[2];      // the Top-P sum and the draw's behind the head
-    uint32_t limit[2];      // elements that those sums run over at most
-    uint32_t cut_bin;       // Min-P: the bin that holds the smallest term kept (kBins: no cut inside the bins), and that term
-    float cut_term;
-    uint32_t cut_in_tail;   // ... or it lies in no bin
-    float renormalizer;
-    uint32_t kept;
+    uint32_t wide_first;    // of the normaliser's sum: the first of the kWideBins bins with wide masks
+    uint32_t listed;        // elements in the first list, the head among them
     uint32_t served;        // the row was finished here
     // the filtered distribution, where BinArgs::want_filters asks for it: probability((exp(logit/T - maximum) / normalizer)
     // / renormalizer) of the elements kept, which are those up to filter_key, filter_token in the row's order whose term is
     // least_term or more
     uint32_t filtered;
+    float normalizer, renormalizer;
+    uint32_t kept;
     float maximum;
     uint32_t filter_key;    // descending key
     uint32_t filter_token;
@@ -153,12 +152,13 @@ struct BinArgs
     uint32_t* steps[2];    // [pairs][kBins], of alternate launches
     uint32_t* ties[2];     // [pairs][3][kBinWords]: bins with terms half way, with two of one value, and with some that their masks cannot hold
     uint32_t* masks[2];    // [pairs][kMaskWords]: parities of the odd steps, and the values half way, by step (see add_bin_steps)
-    uint32_t* packed[2];   // [rows][kBins]
+    uint32_t* packed;      // [rows][kBins]
     float* list_terms[2];  // [rows][kBinListCap]
     uint32_t* list_tokens[2];
-    float* head_terms;     // [rows][kBinListCap], sorted
-    uint32_t* head_tokens;
+    uint32_t* head_tokens; // [rows][kBinListCap], sorted
     BinRow* records;       // [rows]
+    uint32_t* arrivals;    // [rows][kArrivalWords], zero between launches: see parts_meet
+    uint32_t most_looks;   // ... kMostLooks
     uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
     uint32_t listing;      // RowListing: how the first launch finds its rows
@@ -732,6 +732,49 @@ struct Divisor
     }
 };
 
+// What the parts of a row hand to each other inside one launch passes around their compute units' L1 caches and, where the parts should
+// not share an XCD, its L2: agent scope.  (A quarter of a microsecond until such stores have arrived, as far as the XCD's L2 alone
+// would take; the loads take as long as plain ones.)
+template <bool ACROSS>
+__device__ __forceinline__ void hand_over(uint32_t* to, uint32_t value)
+{
+    if (ACROSS)
+        __hip_atomic_store(to, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *to = value;
+}
+
+template <bool ACROSS>
+__device__ __forceinline__ uint32_t taken_over(const uint32_t* from)
+{
+    return ACROSS ? __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *from;
+}
+
+// ... vectors of four words: vector `index` of the `bytes` from `base` on (both the same in all lanes of a wave)
+typedef uint32_t BinVector __attribute__((ext_vector_type(4)));
+constexpr int kAgentScope = 16; // SC1 of a buffer instruction
+constexpr uint32_t kBufferFormat = 0x00027000u;
+
+template <bool ACROSS>
+__device__ __forceinline__ void hand_over_vector(uint32_t* base, uint32_t bytes, uint32_t index, const uint4& value)
+{
+    if (ACROSS)
+        __builtin_amdgcn_raw_buffer_store_b128(BinVector{value.x, value.y, value.z, value.w},
+                                               __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), kBufferFormat), static_cast<int>(index * 16u), 0, kAgentScope);
+    else
+        reinterpret_cast<uint4*>(base)[index] = value;
+}
+
+template <bool ACROSS>
+__device__ __forceinline__ uint4 taken_over_vector(uint32_t* base, uint32_t bytes, uint32_t index)
+{
+    if (!ACROSS)
+        return reinterpret_cast<const uint4*>(base)[index];
+    const BinVector v = __builtin_bit_cast(BinVector, __builtin_amdgcn_raw_buffer_load_b128(
+        __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), kBufferFormat), static_cast<int>(index * 16u), 0, kAgentScope));
+    return uint4{v.x, v.y, v.z, v.w};
+}
+
 // Adds the steps of a part's terms to the bins' integers, and puts the terms of listed bins into the list.
 //   entries   per bin: bit 31 the bin is listed and the rest is the next place of this part in the list; bit 30 it takes
 //             no part in the sum; else the exponent assumed for the sum
@@ -803,8 +846,8 @@ __device__ __forceinline__ void add_bin_steps(
                 else if ((entry & 0x80000000u) != 0u)
                 {
                     const uint32_t place = atomicAdd(&entries[bin], 1u) & 0x7fffffffu;
-                    list_terms[place] = t[c];
-                    list_tokens[place] = v * 4u + c - s.misalignment;
+                    hand_over<(PHASE >= 1)>(reinterpret_cast<uint32_t*>(list_terms) + place, __float_as_uint(t[c]));
+                    hand_over<(PHASE >= 1)>(list_tokens + place, v * 4u + c - s.misalignment);
                 }
             }
         }
@@ -1033,7 +1076,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
             }
             if (grid.part == 0u)
             {
-                reinterpret_cast<uint4*>(g.packed[0] + static_cast<size_t>(row) * kBins)[tid] = uint4{packed[0], packed[1], packed[2], packed[3]};
+                reinterpret_cast<uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid] = uint4{packed[0], packed[1], packed[2], packed[3]};
                 if (own_end != 0u)
                     atomicMax(&end_of_list, own_end);
             }
@@ -1045,8 +1088,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
             record.binned = binned;
             record.head_bins = head_bins;
             record.head_count = head_count;
-            record.listed[0] = max(end_of_list, head_count);
-            record.wide_first[0] = wide_first_of_row;
+            record.listed = max(end_of_list, head_count);
+            record.wide_first = wide_first_of_row;
         }
         const BinStretch s = element_bytes == 4u ? bin_stretch<4>(a, row, grid.part, grid.parts) : bin_stretch<2>(a, row, grid.part, grid.parts);
         add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks, wide_first_of_row,
@@ -1205,6 +1248,7 @@ struct BinWalkShared
     int32_t token;
     uint32_t least_key, most_key, matches; // see token_of_equal
     uint32_t many;                          // see order_elements
+    uint32_t met;                           // see parts_meet
 };
 
 constexpr uint32_t kBinExtraPlace = kBinListCap;
@@ -2075,45 +2119,60 @@ __device__ __forceinline__ int32_t token_of_listed(
     return token;
 }
 
-// ---- (4), (5), (6): WALK 0 walks the normaliser and, inside the head, the Top-P sum and the draw, WALK 1 the Top-P sum
-// behind the head (and the draw inside it), WALK 2 the draw behind the head.  Each then has the bins' steps of the next
+// ---- (4): walk 0 walks the normaliser and, inside the head, the Top-P sum and the draw, walk 1 the Top-P sum
+// behind the head (and the draw inside it), walk 2 the draw behind the head.  Walks 0 and 1 then have the bins' steps of the next
 // sum added for the calling part of the row, unless the row is finished.  Every part of a row walks for itself.
 // ROOMY: at most kRoomyRows rows, one workgroup to a compute unit.
-template <int DTYPE, int WALK, bool ROOMY>
-__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(ROOMY ? 2 : 4, ROOMY ? 2 : 4))) void bin_walk_kernel(BinArgs g)
+
+// What a row's walks hand to each other: the same in each of its parts, which all do the same.
+struct BinWalkRow
 {
-    __shared__ BinWalkShared shared;
-    constexpr int kFrom = WALK & 1;      // which of the alternating buffers this launch reads
+    float normalizer, renormalizer;
+    float head_sum;         // the next walk's sum behind the head
+    uint32_t limit;         // elements that it runs over at most
+    uint32_t kept;
+    uint32_t cut_bin;       // Min-P: the bin that holds the smallest term kept (kBins: no cut inside the bins), and that term
+    float cut_term;
+    uint32_t cut_in_tail;   // ... or it lies in no bin
+    uint32_t listed;        // elements in the list of the next walk (the first walk's holds the head, the others' places behind it)
+    uint32_t wide_first;    // of its sum: the first of the kWideBins bins with wide masks
+    uint4 words;            // the calling thread's four bins
+    uint4 before;           // their elements in the parts in front (where the next list takes this part's)
+};
+
+enum BinWalkOutcome : uint32_t
+{
+    kBinWalkEnds = 0,  // the row is finished, or left to the full-order kernels
+    kBinWalkGoesOn = 1 // the next walk goes on with it
+};
+
+template <int DTYPE, int WALK, bool ROOMY>
+__device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t row, BinWalkShared& shared, BinWalkRow& carried, int tid)
+{
+    constexpr int kFrom = WALK & 1;      // which of the alternating buffers this walk reads
     constexpr int kTo = kFrom ^ 1;
+    constexpr bool kAcross = WALK > 0;   // ... and whether this launch has written it
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
-    const int tid = threadIdx.x;
     const uint32_t bin = 4u * static_cast<uint32_t>(tid);
     const bool holds_bins = tid < static_cast<int>(kBinQuads);
-    if (WALK == 2 && grid.part != 0u)
-        return;
-    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    BinRow& record = g.records[row];
+    const auto result_flags = [&](const ncnn_moe_sample_params& p) {
+        return static_cast<uint8_t>((counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
+                                    (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u));
+    };
     {
-        const uint32_t row = same_in_all(g.list[1u + slot]);
-        BinRow& record = g.records[row];
-        const auto leave = [&](uint32_t state) {
-            if (WALK < 2 && grid.part == 0u && tid == 0)
-                record.state[WALK + 2] = state;
-        };
-        const auto result_flags = [&](const ncnn_moe_sample_params& p) {
-            return static_cast<uint8_t>((counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
-                                        (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u));
-        };
-        const uint32_t state = same_in_all(record.state[WALK + 1]);
-        if (state != kBinRowGoesOn)
+        if (WALK == 0)
         {
-            if (WALK == 0 && state == kBinRowRejected && grid.part == 0u && tid == 0)
+            const uint32_t state = same_in_all(record.state[1]);
+            if (state != kBinRowGoesOn)
             {
-                write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, result_flags(a.params[row]));
-                a.row_state[row] = kRowDone;
+                if (state == kBinRowRejected && grid.part == 0u && tid == 0)
+                {
+                    write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, result_flags(a.params[row]));
+                    a.row_state[row] = kRowDone;
+                }
+                return kBinWalkEnds;
             }
-            leave(kBinRowLeft);
-            continue;
         }
         __syncthreads(); // (a row before this one: its last readers of shared are done)
         if (tid < static_cast<int>(2u * kBinWords))
@@ -2129,24 +2188,25 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         const uint32_t binned = same_in_all(record.binned);
         const uint32_t head_bins = same_in_all(record.head_bins);
         const uint32_t head_count = same_in_all(record.head_count);
-        const uint32_t listed = same_in_all(record.listed[WALK]);
-        const uint32_t wide_first = same_in_all(record.wide_first[WALK]);
-        const uint32_t limit = WALK == 0 ? window : same_in_all(record.limit[WALK - 1]);
-        const uint32_t cut_bin = WALK == 1 ? same_in_all(record.cut_bin) : kBins;
-        const float cut_term = WALK == 1 ? same_in_all(record.cut_term) : 0.0f;
-        uint32_t cut_in_tail = WALK == 1 ? same_in_all(record.cut_in_tail) : 0u;
+        const uint32_t listed = WALK == 0 ? same_in_all(record.listed) : carried.listed;
+        const uint32_t wide_first = WALK == 0 ? same_in_all(record.wide_first) : carried.wide_first;
+        const uint32_t limit = WALK == 0 ? window : carried.limit;
+        const uint32_t cut_bin = WALK == 1 ? carried.cut_bin : kBins;
+        const float cut_term = WALK == 1 ? carried.cut_term : 0.0f;
+        uint32_t cut_in_tail = WALK == 1 ? carried.cut_in_tail : 0u;
         const bool behind_head = limit > head_count && binned > head_count; // this launch's own sum goes on behind the head
-        float normalizer = WALK == 0 ? 1.0f : same_in_all(record.normalizer);
-        float renormalizer = WALK == 2 ? same_in_all(record.renormalizer) : 1.0f;
-        const float sum_so_far = WALK == 0 ? 0.0f : same_in_all(record.head_sum[WALK - 1]);
-        uint32_t kept = WALK == 2 ? same_in_all(record.kept) : 0u;
+        float normalizer = WALK == 0 ? 1.0f : carried.normalizer;
+        float renormalizer = WALK == 2 ? carried.renormalizer : 1.0f;
+        const float sum_so_far = WALK == 0 ? 0.0f : carried.head_sum;
+        uint32_t kept = WALK == 2 ? carried.kept : 0u;
         const BinStretch s = bin_stretch<LogitsVector<DTYPE>::kElementBytes>(a, row, grid.part, grid.parts);
         const uint32_t positions = (s.end + 7u) / 8u * 8u;
         const float* row_terms = bin_terms(a, row);
-        float* const sorted_terms_out = g.head_terms + static_cast<size_t>(row) * kBinListCap;
+        // (the sorted head's terms stay in LDS; its tokens make room there for the steps of the next sum, and the first part alone
+        // looks at them again)
         uint32_t* const sorted_tokens_out = g.head_tokens + static_cast<size_t>(row) * kBinListCap;
 
-        // ---- the list, the bins and their steps.  The head is ordered by WALK 0, read back by WALK 1, no longer needed by WALK 2.
+        // ---- the list, the bins and their steps.  The head is ordered by walk 0, and no longer needed by walk 2.
         constexpr uint32_t kPerThread = kBinListCap / kWalkThreads;
         const uint32_t list_first = WALK == 0 ? 0u : head_count;
         float own_terms[kPerThread];
@@ -2158,34 +2218,33 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             for (uint32_t k = 0; k < kPerThread; ++k)
             {
                 const uint32_t i = list_first + k * kWalkThreads + tid;
-                own_terms[k] = i < listed ? from_terms[i] : 0.0f;
-                own_tokens[k] = i < listed ? from_tokens[i] : 0u;
+                own_terms[k] = i < listed ? __uint_as_float(taken_over<kAcross>(reinterpret_cast<const uint32_t*>(from_terms) + i)) : 0.0f;
+                own_tokens[k] = i < listed ? taken_over<kAcross>(from_tokens + i) : 0u;
             }
         }
-        uint4 words{0u, 0u, 0u, 0u};
+        uint4 words = WALK == 0 ? uint4{0u, 0u, 0u, 0u} : carried.words;
         uint32_t own_steps[4] = {0u, 0u, 0u, 0u};
         uint32_t tie_word = 0, untold_word = 0;
         const uint32_t tie_lane = static_cast<uint32_t>(tid) & (kWaveSize - 1);
-        uint4 before{0u, 0u, 0u, 0u}; // elements of the thread's bins in the parts in front (where the next list takes this part's)
-        if (holds_bins)
+        if (WALK == 0 && holds_bins)
         {
-            words = reinterpret_cast<const uint4*>(g.packed[kFrom] + static_cast<size_t>(row) * kBins)[tid];
-            if (WALK < 2)
-                before = reinterpret_cast<const uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid];
+            words = reinterpret_cast<const uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid];
+            carried.before = reinterpret_cast<const uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid];
         }
         if (behind_head)
         {
             const size_t first_pair = slot * grid.parts;
             if (holds_bins && bin + 3u >= head_bins)
             {
-                const uint4* from = reinterpret_cast<const uint4*>(g.steps[kFrom] + first_pair * kBins) + tid;
+                uint32_t* const from = g.steps[kFrom] + first_pair * kBins;
+                const uint32_t bytes = grid.parts * kBins * 4u;
                 constexpr uint32_t kTogether = ROOMY ? kMaxBinParts : kPartsAtATime;
                 for (uint32_t first = 0; first < grid.parts; first += kTogether)
                 {
                     uint4 of_part[kTogether];
 #pragma unroll
                     for (uint32_t k = 0; k < kTogether; ++k)
-                        of_part[k] = from[static_cast<size_t>(min(first + k, grid.parts - 1u)) * kBinQuads];
+                        of_part[k] = taken_over_vector<kAcross>(from, bytes, min(first + k, grid.parts - 1u) * kBinQuads + static_cast<uint32_t>(tid));
 #pragma unroll
                     for (uint32_t k = 0; k < kTogether; ++k)
                     {
@@ -2205,8 +2264,8 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 {
                     const uint32_t q = static_cast<uint32_t>(tid) / kWaveSize + k * kWalkWaves;
                     const uint32_t* from = g.ties[kFrom] + (first_pair + min(q, grid.parts - 1u)) * 3u * kBinWords + tie_lane;
-                    tie_word |= from[0];
-                    untold_word |= from[kBinWords] | from[2u * kBinWords];
+                    tie_word |= taken_over<kAcross>(from);
+                    untold_word |= taken_over<kAcross>(from + kBinWords) | taken_over<kAcross>(from + 2u * kBinWords);
                 }
             }
         }
@@ -2224,11 +2283,6 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             shared.mask_count = 0u;
         if (tid < 4)
             shared.packed[kBins + tid] = (kBinBeyond << 30) | binned;
-        if constexpr (WALK == 1)
-        {
-            for (uint32_t i = tid; i < head_count; i += kWalkThreads)
-                shared.terms[i] = sorted_terms_out[i];
-        }
         __syncthreads();
         // ---- stops: bins that the walk looks into, and bins from which on another exponent was assumed
         uint32_t front[5];
@@ -2277,7 +2331,9 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
 #pragma unroll
                     for (uint32_t w = 0; w < kWideWords; ++w)
                     {
-                        const uint32_t word = wide ? wide_masks[w] : w == 0u ? of_part[mask_bin] : w == kWideParities ? of_part[kBins + mask_bin] : 0u;
+                        const uint32_t word = wide ? taken_over<kAcross>(wide_masks + w)
+                            : w == 0u ? taken_over<kAcross>(of_part + mask_bin)
+                            : w == kWideParities ? taken_over<kAcross>(of_part + kBins + mask_bin) : 0u;
                         words_of_bin[w] = part < grid.parts ? word : 0u;
                     }
                     uint32_t twice = 0u;
@@ -2427,8 +2483,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
         }
         if (shared.status == 2u)
         {
-            leave(kBinRowLeft); // (more places to look at, or more steps, than the walk holds: left to the full-order kernels)
-            continue;
+            return kBinWalkEnds; // (more places to look at, or more steps, than the walk holds: left to the full-order kernels)
         }
         // ---- the sums.  `head_sum`: of the sum that the next launch goes on with; `next_*`: what it runs over
         float head_sum = 0.0f;
@@ -2453,8 +2508,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             }
             if (given_up)
             {
-                leave(kBinRowLeft);
-                continue;
+                return kBinWalkEnds;
             }
             normalizer = sum;
             // Min-P: the survivors are a prefix; where it ends inside the head it is known at once, else the smallest
@@ -2501,8 +2555,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             const uint32_t stop = same_in_all(shared.head.stop);
             if (given_up && stop == 0xffffffffu)
             {
-                leave(kBinRowLeft);
-                continue;
+                return kBinWalkEnds;
             }
             if (stop != 0xffffffffu || candidates_known)
             {
@@ -2522,8 +2575,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             given_up = shared.status == 2u || (!stopped && limit > binned && cut_in_tail != 0u);
             if (given_up)
             {
-                leave(kBinRowLeft);
-                continue;
+                return kBinWalkEnds;
             }
             // (behind the bins nothing moves the sum: it runs to its limit unless the cut ends it)
             kept = stopped ? shared.stop_rank + 1u : (cut_bin < kBins ? shared.taken : (limit > binned ? limit : shared.taken));
@@ -2598,7 +2650,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);
                 if (shared.status != 1u || shared.stopped == 0u)
-                    continue;
+                    return kBinWalkEnds;
                 found = true;
                 first_of_list = at >= kBinExtraPlace ? kBinExtraPlace : head_count;
                 end_of_list = at >= kBinExtraPlace ? kBinExtraPlace + same_in_all(shared.extra_count) : listed;
@@ -2628,14 +2680,12 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                         record.served = 1u;
                     }
                 }
-                leave(kBinRowLeft);
-                continue;
+                return kBinWalkEnds;
             }
             if (WALK == 0 || head_count == binned)
             {
                 // (the draw passes every term in a bin: the last element kept lies in no list)
-                leave(kBinRowLeft);
-                continue;
+                return kBinWalkEnds;
             }
         }
         if constexpr (WALK < 2)
@@ -2659,14 +2709,11 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
             uint32_t* const masks = shared.tokens;                      // (the list has been used)
             uint32_t* const ties = shared.tokens + kMaskWords;
             static_assert(kMaskWords + 3u * kBinWords <= kBinListCap + kBinExtraCap, "masks and words fit where the list was");
-            // the sorted head is kept for the launch behind this one
+            // the sorted head's tokens are kept for the next walk
             if (WALK == 0 && grid.part == 0u)
             {
                 for (uint32_t i = tid; i < head_count; i += kWalkThreads)
-                {
-                    sorted_terms_out[i] = shared.terms[i];
                     sorted_tokens_out[i] = shared.tokens[i];
-                }
             }
             if (tid == 0)
             {
@@ -2684,7 +2731,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                 if (leads_wave(next_wide < kBins))
                     atomicMin(&shared.wide_first, next_wide);
                 uint32_t next_packed[4];
-                const uint32_t in_front[4] = {before.x, before.y, before.z, before.w};
+                const uint32_t in_front[4] = {carried.before.x, carried.before.y, carried.before.z, carried.before.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
@@ -2695,40 +2742,118 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
                     entries[bin + j] = entry;
                 }
                 *reinterpret_cast<uint4*>(steps + bin) = uint4{0u, 0u, 0u, 0u};
-                if (grid.part == 0u)
-                    reinterpret_cast<uint4*>(g.packed[kTo] + static_cast<size_t>(row) * kBins)[tid] = uint4{next_packed[0], next_packed[1], next_packed[2], next_packed[3]};
+                carried.words = uint4{next_packed[0], next_packed[1], next_packed[2], next_packed[3]};
             }
             __syncthreads();
-            if (grid.part == 0u && own_end != 0u && holds_bins)
+            if (own_end != 0u && holds_bins)
                 atomicMax(&shared.listed_end, own_end);
             add_bin_steps<WALK + 1, kWalkThreads>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks, shared.wide_first,
                                                   g.list_terms[kTo] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[kTo] + static_cast<size_t>(row) * kBinListCap, tid);
             __syncthreads();
             const size_t pair = slot * grid.parts + grid.part;
             if (holds_bins)
-                reinterpret_cast<uint4*>(g.steps[kTo] + pair * kBins)[tid] = *reinterpret_cast<uint4*>(steps + bin);
+                hand_over_vector<true>(g.steps[kTo] + pair * kBins, kBins * 4u, static_cast<uint32_t>(tid), *reinterpret_cast<uint4*>(steps + bin));
             for (uint32_t i = tid; i < kMaskWords / 4u; i += kWalkThreads)
-                reinterpret_cast<uint4*>(g.masks[kTo] + pair * kMaskWords)[i] = reinterpret_cast<uint4*>(masks)[i];
+                hand_over_vector<true>(g.masks[kTo] + pair * kMaskWords, kMaskWords * 4u, i, reinterpret_cast<uint4*>(masks)[i]);
             if (tid < static_cast<int>(3u * kBinWords))
-                g.ties[kTo][pair * 3u * kBinWords + tid] = ties[tid];
-            if (grid.part == 0u && tid == 0)
+                hand_over<true>(g.ties[kTo] + pair * 3u * kBinWords + tid, ties[tid]);
+            carried.normalizer = normalizer;
+            carried.renormalizer = renormalizer;
+            carried.kept = kept;
+            carried.head_sum = head_sum;
+            carried.limit = same_in_all(next_limit);
+            carried.listed = same_in_all(max(shared.listed_end, head_count));
+            carried.wide_first = same_in_all(shared.wide_first);
+            if (WALK == 0)
             {
-                record.normalizer = normalizer;
-                record.renormalizer = renormalizer;
-                record.kept = kept;
-                record.head_sum[WALK] = head_sum;
-                record.limit[WALK] = next_limit;
-                record.listed[WALK + 1] = max(shared.listed_end, head_count);
-                record.wide_first[WALK + 1] = shared.wide_first;
-                if (WALK == 0)
-                {
-                    record.cut_bin = next_cut_bin;
-                    record.cut_term = next_cut_term;
-                    record.cut_in_tail = cut_in_tail;
-                }
-                record.state[WALK + 2] = kBinRowGoesOn;
+                carried.cut_bin = next_cut_bin;
+                carried.cut_term = next_cut_term;
+                carried.cut_in_tail = cut_in_tail;
             }
         }
+    }
+    return WALK < 2 ? kBinWalkGoesOn : kBinWalkEnds;
+}
+
+// The parts of a row meet: what each has handed over before is there for all behind it.  False: given up, because a part did not come.
+// Every thread calls it; `meeting` counts from 1, `wait`: whether the caller takes anything over.
+//
+// All parts of a row are workgroups of one launch that follow each other on an XCD (bin_grid), so the wait ends: workgroups start in
+// order, no part waits before it has come itself, and the parts that are missing start at the latest where a row whose parts
+// have all started is finished.  Workgroups of other launches may hold the places for a while; a part that has looked kMostLooks times
+// (some 20 ms) gives up for the whole row, which is then left to the full-order kernels, as are the rows of a GPU on which
+// fewer workgroups run at a time than a row has parts.
+//
+// arrivals[0] counts the parts that have come to the row's meetings, arrivals[1] those that are done with the row: the last of them
+// returns both to zero.
+constexpr uint32_t kMostLooks = 40000;
+constexpr uint32_t kRowGivenUp = 0x80000000u;
+
+__device__ __forceinline__ bool parts_meet(uint32_t* arrivals, uint32_t parts, uint32_t meeting, bool wait, uint32_t most_looks, BinWalkShared& shared, int tid)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (stores of agent scope: they have arrived when they are counted)
+    __syncthreads();
+    if (parts == 1u)
+        return true;
+    if (tid == 0)
+    {
+        uint32_t seen = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        const uint32_t goal = meeting * parts;
+        for (uint32_t looks = 0; wait && (seen & ~kRowGivenUp) < goal; ++looks)
+        {
+            if ((seen & kRowGivenUp) != 0u)
+                break;
+            if (looks == most_looks)
+            {
+                __hip_atomic_fetch_or(arrivals, kRowGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        shared.met = wait && (seen & ~kRowGivenUp) >= goal ? 1u : 0u;
+    }
+    __syncthreads();
+    return same_in_all(shared.met) != 0u;
+}
+
+__device__ __forceinline__ void part_leaves(uint32_t* arrivals, uint32_t parts, int tid)
+{
+    if (parts > 1u && tid == 0 && __hip_atomic_fetch_add(arrivals + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == parts)
+    {
+        __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(arrivals + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// The launch's arguments (its only ones, BinArgs) read once more: what is read at a kernel's start is kept to its end otherwise, here in
+// some hundred scalar registers that there are not.
+__device__ __forceinline__ const BinArgs& arguments_read_anew()
+{
+    using ConstantBytes = const __attribute__((address_space(4))) uint8_t;
+    ConstantBytes* p = (ConstantBytes*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const BinArgs*)p;
+}
+
+template <int DTYPE, bool ROOMY>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(ROOMY ? 2 : 4, ROOMY ? 2 : 4))) void bin_walks_kernel(BinArgs g)
+{
+    __shared__ BinWalkShared shared;
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
+    const int tid = threadIdx.x;
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = same_in_all(g.list[1u + slot]);
+        uint32_t* const arrivals = g.arrivals + static_cast<size_t>(row) * kArrivalWords;
+        BinWalkRow carried;
+        // (behind the second meeting the first part goes on alone)
+        if (bin_walk<DTYPE, 0, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid) == kBinWalkGoesOn &&
+            parts_meet(arrivals, grid.parts, 1u, true, g.most_looks, shared, tid) &&
+            bin_walk<DTYPE, 1, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid) == kBinWalkGoesOn &&
+            parts_meet(arrivals, grid.parts, 2u, grid.part == 0u, g.most_looks, shared, tid) && grid.part == 0u)
+            bin_walk<DTYPE, 2, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid);
+        part_leaves(arrivals, grid.parts, tid);
     }
 }
 

@@ -72,6 +72,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_force_general",
     "ncnn_moe_hip_sampler_debug_scatter_segments",
     "ncnn_moe_hip_sampler_debug_binned_sums",
+    "ncnn_moe_hip_sampler_debug_most_looks",
     "ncnn_moe_hip_sampler_debug_binned_rows",
     "ncnn_moe_hip_sampler_debug_filtered_rows",
     "ncnn_moe_hip_sampler_debug_spread_sort",
@@ -127,6 +128,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_force_general.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
+    lib.ncnn_moe_hip_sampler_debug_most_looks.argtypes = [vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_filtered_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_spread_sort.argtypes = [vp, ctypes.c_int]
@@ -348,6 +350,10 @@ class HipSampler:
         """Test hook: rows that the first select leaves are served without an order of their logits (the shipped
         library's way; off by default in the testing build) or sorted."""
         self._check(self._hooks().ncnn_moe_hip_sampler_debug_binned_sums(self._handle, 1 if enabled else 0))
+
+    def most_looks(self, looks):
+        """Test hook: how often a part of a row looks for the row's other parts before it gives the row up."""
+        self._check(self._hooks().ncnn_moe_hip_sampler_debug_most_looks(self._handle, looks))
 
     def binned_rows(self, rows):
         """Test hook: which of the handle's first `rows` rows the binned sums finished (1) the last time they were given them."""

@@ -92,6 +92,31 @@ def test_walks_with_and_without_a_compute_unit_of_their_own(rows):
     assert gpu.tobytes() == again.tobytes()
 
 
+@pytest.mark.parametrize("rows,vocab", [(8, 151936), (16, 40009), (40, 20011)])
+def test_rows_whose_parts_do_not_wait_for_each_other(rows, vocab):
+    """A part that finds the others missing gives its row up: the row is sorted, and the launches behind find everything as a
+    finished row leaves it."""
+    rng = np.random.default_rng(rows)
+    print("[case] parts that do not wait, %d x %d" % (rows, vocab), flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 5000])
+    params["top_p"] = 1.0
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        first = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows).sum()
+        sampler.most_looks(0)
+        for _ in range(3):
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "parts that do not wait")
+        assert sampler.binned_rows(rows).sum() < served
+        sampler.most_looks(40000)
+        again = sampler.sample(params, uniforms)
+        assert sampler.binned_rows(rows).sum() == served
+    parity_util.assert_results_match(first, cpu, "f32", "parts that wait")
+    assert first.tobytes() == again.tobytes()
+
+
 def _bf16_values(row):
     return workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(row))
 
