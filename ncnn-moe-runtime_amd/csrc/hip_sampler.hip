@@ -321,6 +321,13 @@ WindowArgs window_args(const ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowL
     return w;
 }
 
+// Whether the binned sums are one launch (see kChainPartElements).
+bool goes_as_chain(uint32_t rows, uint32_t vocab, bool windows)
+{
+    const uint32_t parts = std::max(1u, std::min(kMaxBinParts, kChainGrid / 8u / ((rows + 7u) / 8u)));
+    return rows <= kChainRows && vocab / parts <= (windows ? kChainPartElementsWithWindows : kChainPartElements);
+}
+
 // The binned sums (sampler_bins.h) over the rows in the handle's bin list (`window_list`: see BinArgs).  `behind_terms`, `behind_sum`
 // (null: none): events behind the launch that writes the rows' terms and behind the last one that reads a row as a stream.
 template <int DTYPE>
@@ -349,13 +356,15 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
                 result = hipEventRecord(behind, stream);
         }
     };
+    if (behind_sum == nullptr && goes_as_chain(a.rows, a.vocab, windows))
+    {
+        hipLaunchKernelGGL(bin_chain_kernel<DTYPE>, dim3(kChainGrid), dim3(kWalkThreads), 0, stream, g);
+        return result;
+    }
     launch(nullptr, bin_stats_kernel<DTYPE>, g);
     launch(behind_terms, bin_terms_kernel<DTYPE>, g);
     launch(behind_sum, bin_sum_kernel, g, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u);
-    if (a.rows <= kRoomyRows)
-        hipLaunchKernelGGL((bin_walks_kernel<DTYPE, true>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
-    else
-        hipLaunchKernelGGL((bin_walks_kernel<DTYPE, false>), dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
+    hipLaunchKernelGGL(bin_walks_kernel<DTYPE>, dim3(kBinGrid), dim3(kWalkThreads), 0, stream, g);
     return result;
 }
 
@@ -876,7 +885,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->row_state, rows * sizeof(uint32_t));
     place(&s->windows.counts, rows * sizeof(uint32_t));
     place(&s->windows.flags, rows * sizeof(uint32_t));
-    place(&s->bins.arrivals, rows * kArrivalWords * sizeof(uint32_t));
+    place(&s->bins.arrivals, rows * kArrivalWords * sizeof(unsigned long long));
     const size_t cleared = bytes;
     place(&s->row_epoch, rows * sizeof(uint32_t));
     place(&s->logits, rows * s->logits_stride_f32 * sizeof(float));

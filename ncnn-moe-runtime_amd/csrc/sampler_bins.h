@@ -20,16 +20,17 @@
 // at least 2^-24; the other two sums start at the first term divided by the same numbers as every other): such terms
 // are in no bin.  A foreseen exponent is checked against the exact sum before a bin's integer is used.
 //
-// Four launches serve every row of a call, each workgroup a part of one row: (1) maximum and counts, (2) terms
-// and bin counts, (3) head fetched, steps of the normaliser's sum, (4) normaliser walked, steps of the Top-P sum, Top-P walked,
-// steps of the draw's sum, draw walked.  A row's three walks are one launch, in which its parts meet (parts_meet) where they hand
-// steps to each other: two microseconds with the loads of what was handed over, where another launch cost a gap of 2.6, 1.5
-// before it knew its row and some 2 for loads that found nothing in the L2 (8 rows of 151,936 without a window 105.3 -> 99.2 us,
-// 5 such drafts verified 170.3 -> 163.1; 33 windows of 200 among 100,003, for which the launches find no row, 51.3 -> 47.1; 512 rows
-// of 129,280 with mixed options 222.1 -> 218.2).
+// Each workgroup takes a part of one row: (1) maximum and counts, (2) terms and bin counts, (3) head fetched, steps of the
+// normaliser's sum, (4) normaliser walked, steps of the Top-P sum, Top-P walked, steps of the draw's sum, draw walked.  Calls of few
+// elements do all of it in one launch (bin_chain_kernel), larger ones (1) to (3) in a launch each and the walks in a fourth
+// (bin_walks_kernel).  Inside a launch a row's parts meet where they hand something to each other (parts_meet): 1 us and the loads of what was
+// handed over, where another launch costs a gap of 2 to 3, 1.5 before it knows its row and loads that find nothing in the L2.
+// One launch for the three walks: 8 rows of 151,936 without a window 105.3 -> 99.2 us, 512 of 129,280 with mixed options 222.1 -> 218.2;
+// one for all: 8 rows 99.2 -> 93.4, 33 x 100,003 with windows of 200, for which the launches find no row, 47.1 -> 39.4, a verification
+// step of 5 drafts without a window 163.1 -> 146.
 //
 // What bounds it: instructions, of which each SIMD has those of two wavefronts to issue, and trips to LDS and memory one behind the
-// other (8 rows of 151,936: 5, 5, 14, and 60 for the walks; of a walk some 5 us add the next sum's steps); at a hundred rows and
+// other (8 rows of 151,936: 6, 6, 13 and 55 to 60 for the walks; of a walk some 5 us add the next sum's steps); at a hundred rows and
 // more the reads of the rows and their terms, and the slowest row's walk.
 #ifndef NCNN_MOE_HIP_SAMPLER_BINS_H
 #define NCNN_MOE_HIP_SAMPLER_BINS_H
@@ -79,15 +80,22 @@ constexpr uint32_t kBinComparedTies = 256;       // equal terms of a list that a
 constexpr uint32_t kMaxBinParts = 16;
 constexpr uint32_t kPartsAtATime = 4;            // loads of the parts' numbers in flight together
 constexpr uint32_t kBinPartElements = 2048;      // a part is not made smaller
-constexpr uint32_t kArrivalWords = 32;           // of a row (see parts_meet): a cache line
+constexpr uint32_t kArrivalWords = 16;           // of a row (see parts_meet): a cache line
 constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: two per compute unit
-// The walks want 220 registers; at 128, which two of their workgroups to a compute unit leave, some 35 of them and 130
-// scalars pass through scratch and lane moves.  A call of so few rows that every part has a compute unit of its own takes
-// the walks built for 256 (8 x 151,936 without a window: 141 -> 131 us, 11 such rows of a verification step: 240 -> 223 us);
-// more rows need the second workgroup.  The rule looks at the call's rows, because how many of them have no window is known to
-// the device only; with few of them the two kinds are close (16 and 17 rows of 151,936, of which 1, 4 or 8 have no window:
-// 111, 112 and 113 us with 256 registers, 104, 114 and 125 us with 128).
-constexpr uint32_t kRoomyRows = kBinGrid / 2u / kMaxBinParts;
+// (1) to (4) are one launch, bin_chain_kernel, where a part holds so few elements that what a launch costs by itself outweighs what it is
+// good for: kernels (1) to (3) of 1,024 threads, two workgroups to a compute unit, get through many elements faster.  us a call without a
+// window, by one launch and by four, with the elements of a part of the chain: 17 rows of 151,936 (15,200) 107 and 122, 40 of 32,000 (5,300) 82 and
+// 103, of 100,003 (16,700) 116 and 125, of 129,280 (21,500) 131 and 130; 64 of 2,000 35 and 44, of 64,000 (16,000) 111 and 117, of 100,003
+// (25,000) 135 and 132; 100 of 16,384 (8,200) 82 and 93, of 50,257 (25,100) 128 and 123; 256 of 16,384 101 and 109; 4 of 1,000,000 (62,500)
+// 242 and 228, 16 of 400,000 (25,000) 147 and 144.  Where rows have windows as well, most of the call's rows are not these, and the launches that find
+// none cost 2 us each: mixed options, 40 rows of 129,280 132 and 139, 100 143 and 155; windows of 300, 33 of 100,003 38 and 44, 100 of 129,280
+// (64,600) 50 and 57, 256 of 50,257 46 and 52.  A chain has a compute unit to itself: its walks want 220 registers, and at 128, which two
+// workgroups to a compute unit leave, some of them and 200 scalars pass through scratch and lane moves (17 rows of 151,936 131 us so).  More rows
+// than compute units would take turns (300 of 16,384 168 and 124).
+constexpr uint32_t kChainGrid = kBinGrid / 2u;
+constexpr uint32_t kChainRows = kChainGrid;
+constexpr uint32_t kChainPartElements = 20000;
+constexpr uint32_t kChainPartElementsWithWindows = 80000;
 constexpr uint32_t kBinMaxVocab = (1u << 22) - 16u; // a rank fits 22 bits
 // Foreseen sums decide what is prepared, never what a sum is: a walk that finds its exact sum elsewhere fetches what it needs.
 // They are off by a few 1e-5 on most rows and by 4e-4 (normal logits) to 2e-3 (logits rounded to eighths) on some: a bin
@@ -157,7 +165,7 @@ struct BinArgs
     uint32_t* list_tokens[2];
     uint32_t* head_tokens; // [rows][kBinListCap], sorted
     BinRow* records;       // [rows]
-    uint32_t* arrivals;    // [rows][kArrivalWords], zero between launches: see parts_meet
+    unsigned long long* arrivals; // [rows][kArrivalWords], zero between launches: see parts_meet
     uint32_t most_looks;   // ... kMostLooks
     uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
@@ -175,6 +183,28 @@ __device__ __forceinline__ float same_in_all(float value)
     return __uint_as_float(same_in_all(__float_as_uint(value)));
 }
 
+// A row's options, and its uniform behind them: the first threads read a word each, once a launch (they may lie in host memory).
+constexpr uint32_t kParamsWords = sizeof(ncnn_moe_sample_params) / 4u;
+constexpr uint32_t kRowOptionWords = kParamsWords + 1u;
+static_assert(sizeof(ncnn_moe_sample_params) % 4u == 0u, "the options are whole words");
+
+__device__ __forceinline__ uint32_t read_option(const SamplerArgs& a, uint32_t row, int tid)
+{
+    uint32_t word = 0;
+    if (tid < static_cast<int>(kParamsWords))
+        word = reinterpret_cast<const uint32_t*>(a.params + row)[tid];
+    else if (tid == static_cast<int>(kParamsWords))
+        word = __float_as_uint(a.uniforms[row]);
+    return word;
+}
+
+__device__ __forceinline__ ncnn_moe_sample_params params_of(const uint32_t (&options)[kRowOptionWords])
+{
+    ncnn_moe_sample_params p;
+    __builtin_memcpy(&p, options, sizeof(p));
+    return p;
+}
+
 // The rows that the first select leaves, those with a window of the window kernels' widths apart from the others.
 enum RowListing : uint32_t
 {
@@ -187,9 +217,21 @@ __device__ __forceinline__ bool row_is_left(const SamplerArgs& a, uint32_t row, 
 {
     uint32_t effective_k = 0;
     int status = NCNN_MOE_ROW_OK;
-    const int mode = resolve_row_mode(a.params[row], a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
+    // (all of it is asked for at once)
+    uint32_t words[kParamsWords];
+#pragma unroll
+    for (uint32_t i = 0; i < kParamsWords; ++i)
+        words[i] = reinterpret_cast<const uint32_t*>(a.params + row)[i];
+    uint32_t state = by_options ? 0u : a.row_state[row];
+#pragma unroll
+    for (uint32_t i = 0; i < kParamsWords; ++i)
+        asm volatile("" : "+v"(words[i]));
+    asm volatile("" : "+v"(state));
+    ncnn_moe_sample_params p;
+    __builtin_memcpy(&p, words, sizeof(p));
+    const int mode = resolve_row_mode(p, a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
     window = windows_apart && effective_k <= static_cast<uint32_t>(kSelectTopK);
-    return by_options ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && a.row_state[row] == kRowNeedsGeneral;
+    return by_options ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && state == kRowNeedsGeneral;
 }
 
 // A call of no more rows than a workgroup has threads needs no launch that lists them: every workgroup of the first launch that
@@ -203,13 +245,15 @@ struct RowList
     uint16_t rows[kRowsListedInPlace];
 };
 
+// (For a workgroup of WAVES waves, and calls of no more rows than it has threads.)
 // How many rows there are; they are list[1 ..] where listing is kRowsListed, else shared.rows.  `others` (null: nowhere): the rows of
 // the other kind are listed there for a later launch.
+template <int WAVES = kBinWaves>
 __device__ __forceinline__ uint32_t list_rows_in_place(
     const SamplerArgs& a, uint32_t listing, bool windows_apart, bool want_windows, uint32_t* list, uint32_t* others, RowList& shared, int tid)
 {
     if (listing == kRowsListed)
-        return list[0];
+        return same_in_all(list[0]);
     const int wave = tid >> 6;
     const uint32_t row = static_cast<uint32_t>(tid);
     bool left = false, window = false;
@@ -224,7 +268,7 @@ __device__ __forceinline__ uint32_t list_rows_in_place(
         uint32_t before = 0;
         total = 0;
 #pragma unroll
-        for (int w = 0; w < kBinWaves; ++w)
+        for (int w = 0; w < WAVES; ++w)
         {
             before += w < wave ? shared.wave_totals[w] : 0u;
             total += shared.wave_totals[w];
@@ -255,7 +299,7 @@ __device__ __forceinline__ uint32_t list_rows_in_place(
         }
     }
     __syncthreads();
-    return rows;
+    return same_in_all(rows);
 }
 
 __device__ __forceinline__ uint32_t row_of_slot(uint32_t listing, const uint32_t* list, const RowList& shared, uint32_t slot)
@@ -270,11 +314,11 @@ struct BinGrid
     uint32_t rows, parts, first_slot, slot_step, part;
 };
 
-__device__ __forceinline__ BinGrid bin_grid(uint32_t rows, uint32_t vocab)
+__device__ __forceinline__ BinGrid bin_grid(uint32_t rows, uint32_t vocab, uint32_t workgroups = kBinGrid)
 {
     BinGrid r;
     r.rows = rows;
-    const uint32_t per_xcd = kBinGrid / 8u;
+    const uint32_t per_xcd = workgroups / 8u;
     const uint32_t slots_per_xcd = max(1u, (r.rows + 7u) / 8u);
     const uint32_t most = min(kMaxBinParts, (vocab + kBinPartElements - 1u) / kBinPartElements);
     r.parts = max(1u, min(most, per_xcd / slots_per_xcd));
@@ -318,26 +362,64 @@ __device__ __forceinline__ float* bin_terms(const SamplerArgs& a, uint32_t row)
     return reinterpret_cast<float*>(a.sort_indices[0] + row * a.sort_stride);
 }
 
+// What the parts of a row hand to each other inside one launch (ACROSS).  Loads pass around the compute units' L1 caches (agent scope), and
+// so do stores where the parts are not all on one XCD (`near`, see parts_meet).  Where they are, and bin_grid sees to it, they meet in
+// that XCD's L2: a store of agent scope goes to memory and leaves no line there, and every load behind it is a trip to
+// memory (16 vectors a thread, 102 KB a row: 3.4 us instead of 1.5; 8 rows of 151,936 without a window, which hand over four
+// times, 93 us instead of 85).  As buffer instructions, not as atomics: the compiler orders those, and waits for each before it issues the
+// next.  `base`, `bytes`: the same in all lanes of a wave; what lies behind them is not written, and reads as zero.
+typedef uint32_t BinVector __attribute__((ext_vector_type(4)));
+constexpr int kAgentScope = 16; // SC1 of a buffer instruction
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* base, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00027000);
+}
+
+__device__ __forceinline__ void hand_over(bool near, void* base, uint32_t bytes, uint32_t index, uint32_t value)
+{
+    if (near)
+        __builtin_amdgcn_raw_buffer_store_b32(value, buffer_of(base, bytes), static_cast<int>(index * 4u), 0, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b32(value, buffer_of(base, bytes), static_cast<int>(index * 4u), 0, kAgentScope);
+}
+
+template <bool ACROSS>
+__device__ __forceinline__ uint32_t taken_over(const void* base, uint32_t bytes, uint32_t index)
+{
+    return __builtin_amdgcn_raw_buffer_load_b32(buffer_of(base, bytes), static_cast<int>(index * 4u), 0, ACROSS ? kAgentScope : 0);
+}
+
+// ... vectors of four words, `index` of them behind `base`
+__device__ __forceinline__ void hand_over_vector(bool near, void* base, uint32_t bytes, uint32_t index, const uint4& value)
+{
+    const BinVector v{value.x, value.y, value.z, value.w};
+    if (near)
+        __builtin_amdgcn_raw_buffer_store_b128(v, buffer_of(base, bytes), static_cast<int>(index * 16u), 0, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b128(v, buffer_of(base, bytes), static_cast<int>(index * 16u), 0, kAgentScope);
+}
+
+template <bool ACROSS>
+__device__ __forceinline__ uint4 taken_over_vector(const void* base, uint32_t bytes, uint32_t index)
+{
+    const BinVector v = __builtin_bit_cast(BinVector, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(base, bytes), static_cast<int>(index * 16u), 0, ACROSS ? kAgentScope : 0));
+    return uint4{v.x, v.y, v.z, v.w};
+}
+
 // Kernels (1) to (3) are bound to 64 registers: two workgroups of 1,024 threads share a compute unit then, and the 512
 // workgroups of a launch that many rows fill run at once, not in two rounds (512 rows of 129,280 of mixed options: 17, 26
 // and 32 us before, 14, 22 and 25 us with the bound).
 //
 // ---- (1) largest and smallest finite logit, number of finite logits, NaN and +inf seen
-template <int DTYPE>
-__global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
+// `wave_stats`: one for each of the workgroup's waves.  The first wave returns those of the part.
+template <int DTYPE, int THREADS>
+__device__ __forceinline__ uint4 stats_of_part(const SamplerArgs& a, const BinGrid& grid, uint32_t row, uint4* wave_stats, int tid)
 {
     using Vector = LogitsVector<DTYPE>;
     constexpr uint32_t kWidth = Vector::kWidth;
-    constexpr int kLoads = 4;
-    __shared__ uint4 wave_stats[kBinWaves];
-    const SamplerArgs& a = g.a;
-    __shared__ RowList listed_rows;
-    const int tid = threadIdx.x;
-    const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
-    const BinGrid grid = bin_grid(rows, a.vocab);
-    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    constexpr int kLoads = 4 * kBinThreads / THREADS;
     {
-        const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
         const BinStretch s = bin_stretch<Vector::kElementBytes>(a, row, grid.part, grid.parts);
         const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
             static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
@@ -370,16 +452,16 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
             take_inside(first);
         if (tid == kWaveSize && first_whole <= last_whole && last_whole < last)
             take_inside(last_whole);
-        for (uint32_t at = first_whole + tid; at < last_whole; at += kLoads * kBinThreads)
+        for (uint32_t at = first_whole + tid; at < last_whole; at += kLoads * THREADS)
         {
             uint4 raw[kLoads];
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
-                raw[k] = *reinterpret_cast<const uint4*>(base + min(at + k * kBinThreads, last_whole - 1u) * 16u); // (rows below 2^32 bytes)
+                raw[k] = *reinterpret_cast<const uint4*>(base + min(at + k * THREADS, last_whole - 1u) * 16u); // (rows below 2^32 bytes)
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
             {
-                if (at + k * kBinThreads < last_whole)
+                if (at + k * THREADS < last_whole)
                 {
                     float x[kWidth];
                     Vector::unpack(raw[k], x);
@@ -404,39 +486,56 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
         __syncthreads();
         if (tid < kWaveSize)
         {
-            const uint4 of_wave = wave_stats[tid & (kBinWaves - 1)];
+            constexpr int kWaves = THREADS / kWaveSize;
+            const uint4 of_wave = wave_stats[tid & (kWaves - 1)];
             largest = __uint_as_float(of_wave.x), smallest = __uint_as_float(of_wave.y), finite = of_wave.z, flags = of_wave.w;
-            reduce(kBinWaves);
-            if (tid == 0)
-                g.stats[slot * grid.parts + grid.part] = uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
+            reduce(kWaves);
         }
+        return uint4{__float_as_uint(largest), __float_as_uint(smallest), finite, flags};
+    }
+}
+
+template <int DTYPE>
+__global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
+{
+    __shared__ uint4 wave_stats[kBinWaves];
+    __shared__ RowList listed_rows;
+    const SamplerArgs& a = g.a;
+    const int tid = threadIdx.x;
+    const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
+    const BinGrid grid = bin_grid(rows, a.vocab);
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
+        const uint4 of_part = stats_of_part<DTYPE, kBinThreads>(a, grid, row, wave_stats, tid);
+        if (tid == 0)
+            g.stats[slot * grid.parts + grid.part] = of_part;
         __syncthreads();
     }
 }
 
 // ---- (2) the terms, in the row's order, and how many fall into each bin
-template <int DTYPE>
-__global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
+// What is known of a row before its sums: the same in each of its parts.
+struct BinRowStart
+{
+    uint32_t state, shift, window, saw_nan;
+};
+
+// `bins`: 2 x kBins words of LDS.  ACROSS: the launch itself has written the parts' statistics, and the counts are for itself.
+template <int DTYPE, int THREADS, bool ACROSS>
+__device__ __forceinline__ BinRowStart terms_of_part(
+    const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t row, const ncnn_moe_sample_params& p, bool near, uint32_t* bins, uint4* part_stats,
+    const uint64_t* exp2_table, int tid)
 {
     using Vector = LogitsVector<DTYPE>;
     constexpr uint32_t kWidth = Vector::kWidth;
-    constexpr int kLoads = DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2;
-    __shared__ __align__(16) uint32_t bins[2 * kBins];
-    __shared__ uint4 part_stats[kMaxBinParts];
-    __shared__ uint64_t exp2_table[32];
+    constexpr int kLoads = (DTYPE == NCNN_MOE_LOGITS_F32 ? 4 : 2) * kBinThreads / THREADS;
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
-    const int tid = threadIdx.x;
-    if (tid < 32)
-        exp2_table[tid] = kExp2Table[tid];
-    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
-        const uint32_t row = g.list[1u + slot];
-        const ncnn_moe_sample_params p = a.params[row];
         if (tid < static_cast<int>(grid.parts))
-            part_stats[tid] = g.stats[slot * grid.parts + tid];
-        if (tid < static_cast<int>(2u * kBinQuads))
-            reinterpret_cast<uint4*>(bins)[tid] = uint4{0u, 0u, 0u, 0u};
+            part_stats[tid] = taken_over_vector<ACROSS>(g.stats + slot * grid.parts, grid.parts * 16u, static_cast<uint32_t>(tid));
+        for (uint32_t i = tid; i < 2u * kBinQuads; i += THREADS)
+            reinterpret_cast<uint4*>(bins)[i] = uint4{0u, 0u, 0u, 0u};
         __syncthreads();
         float largest = -INFINITY, smallest = INFINITY;
         uint32_t finite = 0, flags = 0;
@@ -460,18 +559,20 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
             ++shift;
         const uint32_t place_mask = (1u << shift) - 1u;
         const uint32_t place_shift = shift > kOffsetBits ? shift - kOffsetBits : 0u;
+        const BinRowStart start{served ? kBinRowGoesOn : rejected ? kBinRowRejected : kBinRowLeft, shift,
+                                (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite, (flags & kScanSawNan) != 0u ? 1u : 0u};
         if (grid.part == 0u && tid == 0)
         {
             BinRow& record = g.records[row];
             // (pending until a walk has finished it: a first select that runs beside leaves these rows alone)
             a.row_state[row] = kRowNeedsGeneral;
-            record.state[0] = served ? kBinRowGoesOn : rejected ? kBinRowRejected : kBinRowLeft;
+            record.state[0] = start.state;
             record.shift = shift;
-            record.window = (p.top_k > 0u && p.top_k < a.vocab && finite > p.top_k) ? p.top_k : finite;
+            record.window = start.window;
             record.served = 0u;
             record.filtered = 0u;
             record.maximum = maximum;
-            record.saw_nan = (flags & kScanSawNan) != 0u ? 1u : 0u;
+            record.saw_nan = start.saw_nan;
         }
         if (served)
         {
@@ -479,20 +580,21 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
             const char* base = static_cast<const char*>(a.logits) + static_cast<size_t>(row) * a.row_stride * Vector::kElementBytes -
                 static_cast<size_t>(s.misalignment) * Vector::kElementBytes;
             float* terms = bin_terms(a, row);
+            const uint32_t terms_bytes = (s.end + 7u) / 8u * 32u;
             const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
-            for (uint32_t at = first + tid; at < last; at += kLoads * kBinThreads)
+            for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
             {
                 uint4 raw[kLoads];
 #pragma unroll
                 for (int k = 0; k < kLoads; ++k)
                 {
-                    const uint32_t v = min(at + k * kBinThreads, last - 1u);
+                    const uint32_t v = min(at + k * THREADS, last - 1u);
                     raw[k] = *reinterpret_cast<const uint4*>(base + v * 16u); // (rows below 2^32 bytes)
                 }
 #pragma unroll
                 for (int k = 0; k < kLoads; ++k)
                 {
-                    const uint32_t v = at + k * kBinThreads;
+                    const uint32_t v = at + k * THREADS;
                     if (v >= last)
                         break;
                     float x[kWidth], t[kWidth];
@@ -514,16 +616,35 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
                     }
 #pragma unroll
                     for (uint32_t c = 0; c < kWidth; c += 4u)
-                        *reinterpret_cast<float4*>(terms + position + c) = float4{t[c], t[c + 1], t[c + 2], t[c + 3]};
+                        hand_over_vector(near, terms, terms_bytes, (position + c) / 4u,
+                                                 uint4{__float_as_uint(t[c]), __float_as_uint(t[c + 1]), __float_as_uint(t[c + 2]), __float_as_uint(t[c + 3])});
                 }
             }
             // (the last group of eight positions of the row may reach a vector further than the row does)
             if (kWidth == 4u && tid == 0 && s.last * 2u > last && last > first)
-                *reinterpret_cast<float4*>(terms + last * 4u) = float4{0.0f, 0.0f, 0.0f, 0.0f};
+                hand_over_vector(near, terms, terms_bytes, last, uint4{0u, 0u, 0u, 0u});
             __syncthreads();
-            if (tid < static_cast<int>(2u * kBinQuads))
-                reinterpret_cast<uint4*>(g.counts + static_cast<size_t>(slot * grid.parts + grid.part) * 2u * kBins)[tid] = reinterpret_cast<uint4*>(bins)[tid];
+            for (uint32_t i = tid; i < 2u * kBinQuads; i += THREADS)
+                hand_over_vector(near, g.counts + static_cast<size_t>(slot * grid.parts + grid.part) * 2u * kBins, 2u * kBins * 4u, i, reinterpret_cast<uint4*>(bins)[i]);
         }
+        return start;
+    }
+}
+
+template <int DTYPE>
+__global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
+{
+    __shared__ __align__(16) uint32_t bins[2 * kBins];
+    __shared__ uint4 part_stats[kMaxBinParts];
+    __shared__ uint64_t exp2_table[32];
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
+    const int tid = threadIdx.x;
+    if (tid < 32)
+        exp2_table[tid] = kExp2Table[tid];
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = g.list[1u + slot];
+        terms_of_part<DTYPE, kBinThreads, false>(g, grid, slot, row, g.a.params[row], true, bins, part_stats, exp2_table, tid);
         __syncthreads();
     }
 }
@@ -732,49 +853,6 @@ struct Divisor
     }
 };
 
-// What the parts of a row hand to each other inside one launch passes around their compute units' L1 caches and, where the parts should
-// not share an XCD, its L2: agent scope.  (A quarter of a microsecond until such stores have arrived, as far as the XCD's L2 alone
-// would take; the loads take as long as plain ones.)
-template <bool ACROSS>
-__device__ __forceinline__ void hand_over(uint32_t* to, uint32_t value)
-{
-    if (ACROSS)
-        __hip_atomic_store(to, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else
-        *to = value;
-}
-
-template <bool ACROSS>
-__device__ __forceinline__ uint32_t taken_over(const uint32_t* from)
-{
-    return ACROSS ? __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *from;
-}
-
-// ... vectors of four words: vector `index` of the `bytes` from `base` on (both the same in all lanes of a wave)
-typedef uint32_t BinVector __attribute__((ext_vector_type(4)));
-constexpr int kAgentScope = 16; // SC1 of a buffer instruction
-constexpr uint32_t kBufferFormat = 0x00027000u;
-
-template <bool ACROSS>
-__device__ __forceinline__ void hand_over_vector(uint32_t* base, uint32_t bytes, uint32_t index, const uint4& value)
-{
-    if (ACROSS)
-        __builtin_amdgcn_raw_buffer_store_b128(BinVector{value.x, value.y, value.z, value.w},
-                                               __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), kBufferFormat), static_cast<int>(index * 16u), 0, kAgentScope);
-    else
-        reinterpret_cast<uint4*>(base)[index] = value;
-}
-
-template <bool ACROSS>
-__device__ __forceinline__ uint4 taken_over_vector(uint32_t* base, uint32_t bytes, uint32_t index)
-{
-    if (!ACROSS)
-        return reinterpret_cast<const uint4*>(base)[index];
-    const BinVector v = __builtin_bit_cast(BinVector, __builtin_amdgcn_raw_buffer_load_b128(
-        __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), kBufferFormat), static_cast<int>(index * 16u), 0, kAgentScope));
-    return uint4{v.x, v.y, v.z, v.w};
-}
-
 // Adds the steps of a part's terms to the bins' integers, and puts the terms of listed bins into the list.
 //   entries   per bin: bit 31 the bin is listed and the rest is the next place of this part in the list; bit 30 it takes
 //             no part in the sum; else the exponent assumed for the sum
@@ -783,27 +861,28 @@ __device__ __forceinline__ uint4 taken_over_vector(uint32_t* base, uint32_t byte
 //   masks     per bin, for terms kMaskedDifference binades and more below the sum: bit (step / 2) % 32 the parity of the
 //             odd steps of that value; then bit step % 32 for a term half way between `step` and the next.  The kWideBins bins
 //             from wide_first on have the same with 64 and 128 bits
-template <int PHASE, int THREADS>
+template <int PHASE, int THREADS, bool ACROSS>
 __device__ __forceinline__ void add_bin_steps(
     const float* terms, const BinStretch& s, uint32_t shift, uint32_t first_bin, uint32_t bin_count, float divisor, float second_divisor,
-    uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, uint32_t wide_first, float* list_terms, uint32_t* list_tokens, int tid)
+    uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, uint32_t wide_first, float* list_terms, uint32_t* list_tokens, bool near, int tid)
 {
     constexpr int kLoads = 4;
+    const uint32_t bytes = (s.end + 7u) / 8u * 32u;
     const uint32_t first = s.first * 2u, last = s.last * 2u;
     const Divisor by(divisor), by_second(second_divisor);
     for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
     {
-        float4 raw[kLoads];
+        uint4 raw[kLoads];
 #pragma unroll
         for (int k = 0; k < kLoads; ++k)
-            raw[k] = reinterpret_cast<const float4*>(terms)[min(at + k * THREADS, last - 1u)];
+            raw[k] = taken_over_vector<ACROSS>(terms, bytes, min(at + k * THREADS, last - 1u));
 #pragma unroll
         for (int k = 0; k < kLoads; ++k)
         {
             const uint32_t v = at + k * THREADS;
             if (v >= last)
                 break;
-            const float t[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+            const float t[4] = {__uint_as_float(raw[k].x), __uint_as_float(raw[k].y), __uint_as_float(raw[k].z), __uint_as_float(raw[k].w)};
 #pragma unroll
             for (int c = 0; c < 4; ++c)
             {
@@ -846,57 +925,74 @@ __device__ __forceinline__ void add_bin_steps(
                 else if ((entry & 0x80000000u) != 0u)
                 {
                     const uint32_t place = atomicAdd(&entries[bin], 1u) & 0x7fffffffu;
-                    hand_over<(PHASE >= 1)>(reinterpret_cast<uint32_t*>(list_terms) + place, __float_as_uint(t[c]));
-                    hand_over<(PHASE >= 1)>(list_tokens + place, v * 4u + c - s.misalignment);
+                    hand_over(near, list_terms, kBinListCap * 4u, place, __float_as_uint(t[c]));
+                    hand_over(near, list_tokens, kBinListCap * 4u, place, v * 4u + c - s.misalignment);
                 }
             }
         }
     }
 }
 
-// ---- (3) the head and the bins whose order is foreseen to matter go to the list; the others' steps of the normaliser
-__global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint32_t element_bytes)
+// What a row's sums hand to each other, in LDS: the same in each of its parts, which all do the same.
+struct BinWalkRow
 {
-    __shared__ __align__(16) uint32_t entries[kBins];
-    __shared__ __align__(16) uint32_t steps[kBins];
-    __shared__ __align__(16) uint32_t masks[kMaskWords];
-    __shared__ uint32_t ties[3 * kBinWords];
-    __shared__ BinScanScratch scan;
-    __shared__ uint32_t bins_behind_heads[2], heads_hold[2], end_of_list, wide_first_of_row;
-    __shared__ float longest_holds, row_holds;
+    uint32_t shift;         // a term's bin: (kOneBits - bits) >> shift
+    uint32_t window;        // elements of the Top-K window (finite logits at most)
+    uint32_t saw_nan;
+    uint32_t options[kRowOptionWords]; // ncnn_moe_sample_params, then the uniform
+    uint32_t binned;        // elements in bins
+    uint32_t head_bins;     // bins [0, head_bins) are the head, head_count elements
+    uint32_t head_count;
+    float normalizer, renormalizer;
+    float head_sum;         // the next walk's sum behind the head
+    uint32_t limit;         // elements that it runs over at most
+    uint32_t kept;
+    uint32_t cut_bin;       // Min-P: the bin that holds the smallest term kept (kBins: no cut inside the bins), and that term
+    float cut_term;
+    uint32_t cut_in_tail;   // ... or it lies in no bin
+    uint32_t listed;        // elements in the list of the next walk (the first walk's holds the head, the others' places behind it)
+    uint32_t wide_first;    // of its sum: the first of the kWideBins bins with wide masks
+};
+
+// ---- (3) the head and the bins whose order is foreseen to matter go to the list; the others' steps of the normaliser
+struct BinSumShared
+{
+    uint32_t bins_behind_heads[2], heads_hold[2], end_of_list, wide_first_of_row;
+    float longest_holds, row_holds;
+};
+
+// `entries`, `steps`: kBins words of LDS, `masks`: kMaskWords, `ties`: 3 x kBinWords.  ACROSS: the launch itself has written the parts'
+// counts, and the steps are for itself.  Fills in `carried` for the first walk, and returns the calling thread's four bins.
+template <int THREADS, bool ACROSS>
+__device__ __forceinline__ uint4 sum_of_part(
+    const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t row, float top_p, float min_p, bool near, const BinStretch& s, uint32_t* entries, uint32_t* steps, uint32_t* masks, uint32_t* ties,
+    BinScanScratch& scan, BinSumShared& shared, BinWalkRow& carried, int tid)
+{
+    constexpr int kWaves = THREADS / kWaveSize;
+    constexpr bool kPlacesApart = THREADS / 2 >= static_cast<int>(kBinQuads); // other threads load where in their bins the terms lie
+    uint32_t (&bins_behind_heads)[2] = shared.bins_behind_heads;
+    uint32_t (&heads_hold)[2] = shared.heads_hold;
+    uint32_t &end_of_list = shared.end_of_list, &wide_first_of_row = shared.wide_first_of_row;
+    float &longest_holds = shared.longest_holds, &row_holds = shared.row_holds;
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
-    const int tid = threadIdx.x;
     const uint32_t bin = 4u * static_cast<uint32_t>(tid);
     const bool holds_bins = tid < static_cast<int>(kBinQuads);
-    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
-        const uint32_t row = g.list[1u + slot];
-        BinRow& record = g.records[row];
-        if (record.state[0] != kBinRowGoesOn)
-        {
-            if (grid.part == 0u && tid == 0)
-                record.state[1] = record.state[0];
-            continue;
-        }
-        const uint32_t shift = record.shift;
-        const uint32_t window = record.window;
-        const float top_p = same_in_all(a.params[row].top_p);
-        const float min_p = same_in_all(a.params[row].min_p);
-        // counts of the thread's bins, of the whole row and of the parts in front of this one, and (by other threads) where
-        // in their bins the terms lie
+        const uint32_t shift = same_in_all(carried.shift);
+        const uint32_t window = same_in_all(carried.window);
+        uint4 words{0u, 0u, 0u, 0u};
+        // counts of the thread's bins, of the whole row and of the parts in front of this one, and where in their bins the terms lie
         uint32_t count[4] = {0u, 0u, 0u, 0u}, before[4] = {0u, 0u, 0u, 0u};
-        const bool holds_places = tid >= kBinThreads / 2 && tid < kBinThreads / 2 + static_cast<int>(kBinQuads);
-        if (holds_bins || holds_places)
-        {
-            const uint4* counts = reinterpret_cast<const uint4*>(g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins) +
-                (holds_bins ? static_cast<uint32_t>(tid) : kBinQuads + static_cast<uint32_t>(tid) - kBinThreads / 2);
+        // (counted in vectors of four bins, `first_vector` of each part's; `before`: of the parts in front)
+        const auto collect = [&](uint32_t first_vector, uint32_t (&all)[4], uint32_t (&in_front)[4]) {
+            uint32_t* const counts = g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins;
+            const uint32_t bytes = grid.parts * 2u * kBins * 4u;
             for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
             {
                 uint4 of_part[kPartsAtATime];
 #pragma unroll
                 for (uint32_t k = 0; k < kPartsAtATime; ++k)
-                    of_part[k] = counts[static_cast<size_t>(min(first + k, grid.parts - 1u)) * 2u * kBinQuads];
+                    of_part[k] = taken_over_vector<ACROSS>(counts, bytes, min(first + k, grid.parts - 1u) * 2u * kBinQuads + first_vector);
 #pragma unroll
                 for (uint32_t k = 0; k < kPartsAtATime; ++k)
                 {
@@ -906,26 +1002,38 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                     {
-                        count[j] += c[j] & some; // (places: below 2^22 x 2^12; only a bin of a million terms wraps, a wrong guess)
-                        before[j] += c[j] & some_before;
+                        all[j] += c[j] & some; // (places: below 2^22 x 2^12; only a bin of a million terms wraps, a wrong guess)
+                        in_front[j] += c[j] & some_before;
                     }
                 }
             }
-        }
-        if (holds_places)
-            reinterpret_cast<uint4*>(steps)[tid - kBinThreads / 2] = uint4{count[0], count[1], count[2], count[3]};
-        __syncthreads();
+        };
         uint32_t places[4] = {0u, 0u, 0u, 0u};
-        if (holds_bins)
+        if constexpr (kPlacesApart)
         {
-            const uint4 words = reinterpret_cast<const uint4*>(steps)[tid];
-            places[0] = words.x, places[1] = words.y, places[2] = words.z, places[3] = words.w;
-        }
-        else
-        {
+            const bool holds_places = tid >= THREADS / 2 && tid < THREADS / 2 + static_cast<int>(kBinQuads);
+            if (holds_bins || holds_places)
+                collect(holds_bins ? static_cast<uint32_t>(tid) : kBinQuads + static_cast<uint32_t>(tid) - THREADS / 2, count, before);
+            if (holds_places)
+                reinterpret_cast<uint4*>(steps)[tid - THREADS / 2] = uint4{count[0], count[1], count[2], count[3]};
+            __syncthreads();
+            if (holds_bins)
+            {
+                const uint4 words = reinterpret_cast<const uint4*>(steps)[tid];
+                places[0] = words.x, places[1] = words.y, places[2] = words.z, places[3] = words.w;
+            }
+            else
+            {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                count[j] = before[j] = 0u;
+                for (int j = 0; j < 4; ++j)
+                    count[j] = before[j] = 0u;
+            }
+        }
+        else if (holds_bins)
+        {
+            uint32_t none[4] = {0u, 0u, 0u, 0u};
+            collect(static_cast<uint32_t>(tid), count, before);
+            collect(kBinQuads + static_cast<uint32_t>(tid), places, none);
         }
         if (tid == 0)
         {
@@ -934,9 +1042,8 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         }
         if (holds_bins)
             reinterpret_cast<uint4*>(steps)[tid] = uint4{0u, 0u, 0u, 0u};
-        static_assert(kMaskWords / 4u <= kBinThreads, "a vector of the masks a thread");
-        if (tid < static_cast<int>(kMaskWords / 4u))
-            reinterpret_cast<uint4*>(masks)[tid] = uint4{0u, 0u, 0u, 0u};
+        for (uint32_t i = tid; i < kMaskWords / 4u; i += THREADS)
+            reinterpret_cast<uint4*>(masks)[i] = uint4{0u, 0u, 0u, 0u};
         if (tid < static_cast<int>(3u * kBinWords))
             ties[tid] = 0u;
         // elements and mass in front of the thread's bins: first the plain masses, then what the sum makes of them (a term
@@ -958,7 +1065,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                     : static_cast<float>(count[j]) * top - width * static_cast<float>(places[j]) * (shift > kOffsetBits ? 1.0f / (1u << kOffsetBits) : 1.0f / static_cast<float>(1u << shift));
                 masses += own[j];
             }
-            bin_scan<kBinWaves>(total, totals, masses, scan, tid);
+            bin_scan<kWaves>(total, totals, masses, scan, tid);
             binned = totals[0];
             front[0] = total[0];
             mass[0] = masses;
@@ -985,7 +1092,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                 rounded += own[j];
             }
             uint32_t none[1] = {0u};
-            bin_scan<kBinWaves>(none, totals, rounded, scan, tid);
+            bin_scan<kWaves>(none, totals, rounded, scan, tid);
             mass[0] = rounded;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -1055,7 +1162,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
         uint32_t listed[1] = {holds_bins ? plan.listed : 0u};
         {
             uint32_t totals[1];
-            bin_scan<kBinWaves>(listed, totals, scan, tid);
+            bin_scan<kWaves>(listed, totals, scan, tid);
         }
         uint32_t place[4];
         const uint32_t own_end = fit_plan(plan, front, head_count + listed[0], place);
@@ -1074,41 +1181,77 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
                     : plan.kind[j] == kBinListed ? (0x80000000u | (place[j] + before[j]))
                     : plan.kind[j] == kBinAdded ? plan.exponent[j] : 0x40000000u;
             }
-            if (grid.part == 0u)
-            {
-                reinterpret_cast<uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid] = uint4{packed[0], packed[1], packed[2], packed[3]};
-                if (own_end != 0u)
-                    atomicMax(&end_of_list, own_end);
-            }
+            words = uint4{packed[0], packed[1], packed[2], packed[3]};
+            reinterpret_cast<uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid] = uint4{before[0], before[1], before[2], before[3]};
+            if (own_end != 0u)
+                atomicMax(&end_of_list, own_end);
         }
         __syncthreads();
-        if (grid.part == 0u && tid == 0)
+        if (tid == 0)
         {
-            record.state[1] = kBinRowGoesOn;
-            record.binned = binned;
-            record.head_bins = head_bins;
-            record.head_count = head_count;
-            record.listed = max(end_of_list, head_count);
-            record.wide_first = wide_first_of_row;
+            carried.binned = binned;
+            carried.head_bins = head_bins;
+            carried.head_count = head_count;
+            carried.listed = max(end_of_list, head_count);
+            carried.wide_first = wide_first_of_row;
         }
-        const BinStretch s = element_bytes == 4u ? bin_stretch<4>(a, row, grid.part, grid.parts) : bin_stretch<2>(a, row, grid.part, grid.parts);
-        add_bin_steps<0, kBinThreads>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks, wide_first_of_row,
-                                      g.list_terms[0] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[0] + static_cast<size_t>(row) * kBinListCap, tid);
+        add_bin_steps<0, THREADS, ACROSS>(bin_terms(a, row), s, shift, 0u, beyond ? kBins : head_bins, 1.0f, 1.0f, entries, steps, ties, masks, wide_first_of_row,
+                                      g.list_terms[0] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[0] + static_cast<size_t>(row) * kBinListCap, near, tid);
         __syncthreads();
-        {
-            const size_t pair = slot * grid.parts + grid.part;
-            if (holds_bins)
-                reinterpret_cast<uint4*>(g.before + pair * kBins)[tid] = uint4{before[0], before[1], before[2], before[3]};
-        }
         if (beyond)
         {
             const size_t pair = slot * grid.parts + grid.part;
             if (holds_bins)
-                reinterpret_cast<uint4*>(g.steps[0] + pair * kBins)[tid] = reinterpret_cast<uint4*>(steps)[tid];
-            if (tid < static_cast<int>(kMaskWords / 4u))
-                reinterpret_cast<uint4*>(g.masks[0] + pair * kMaskWords)[tid] = reinterpret_cast<uint4*>(masks)[tid];
+                hand_over_vector(near, g.steps[0] + pair * kBins, kBins * 4u, static_cast<uint32_t>(tid), reinterpret_cast<uint4*>(steps)[tid]);
+            for (uint32_t i = tid; i < kMaskWords / 4u; i += THREADS)
+                hand_over_vector(near, g.masks[0] + pair * kMaskWords, kMaskWords * 4u, i, reinterpret_cast<uint4*>(masks)[i]);
             if (tid < static_cast<int>(3u * kBinWords))
-                g.ties[0][pair * 3u * kBinWords + tid] = ties[tid];
+                hand_over(near, g.ties[0] + pair * 3u * kBinWords, 3u * kBinWords * 4u, static_cast<uint32_t>(tid), ties[tid]);
+        }
+        return words;
+    }
+}
+
+__global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint32_t element_bytes)
+{
+    __shared__ __align__(16) uint32_t entries[kBins];
+    __shared__ __align__(16) uint32_t steps[kBins];
+    __shared__ __align__(16) uint32_t masks[kMaskWords];
+    __shared__ uint32_t ties[3 * kBinWords];
+    __shared__ BinScanScratch scan;
+    __shared__ BinSumShared shared;
+    __shared__ BinWalkRow carried;
+    const SamplerArgs& a = g.a;
+    const BinGrid grid = bin_grid(g.list[0], a.vocab);
+    const int tid = threadIdx.x;
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = g.list[1u + slot];
+        BinRow& record = g.records[row];
+        if (record.state[0] != kBinRowGoesOn)
+        {
+            if (grid.part == 0u && tid == 0)
+                record.state[1] = record.state[0];
+            continue;
+        }
+        if (tid == 0)
+        {
+            carried.shift = record.shift;
+            carried.window = record.window;
+        }
+        __syncthreads();
+        const BinStretch s = element_bytes == 4u ? bin_stretch<4>(a, row, grid.part, grid.parts) : bin_stretch<2>(a, row, grid.part, grid.parts);
+        const uint4 words = sum_of_part<kBinThreads, false>(g, grid, slot, row, same_in_all(a.params[row].top_p), same_in_all(a.params[row].min_p), true, s, entries, steps, masks, ties, scan, shared, carried, tid);
+        if (grid.part == 0u && tid < static_cast<int>(kBinQuads))
+            reinterpret_cast<uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid] = words;
+        if (grid.part == 0u && tid == 0)
+        {
+            record.state[1] = kBinRowGoesOn;
+            record.binned = carried.binned;
+            record.head_bins = carried.head_bins;
+            record.head_count = carried.head_count;
+            record.listed = carried.listed;
+            record.wide_first = carried.wide_first;
         }
         __syncthreads();
     }
@@ -1248,7 +1391,8 @@ struct BinWalkShared
     int32_t token;
     uint32_t least_key, most_key, matches; // see token_of_equal
     uint32_t many;                          // see order_elements
-    uint32_t met;                           // see parts_meet
+    uint32_t met, near;                     // see parts_meet
+    BinWalkRow row;
 };
 
 constexpr uint32_t kBinExtraPlace = kBinListCap;
@@ -1412,10 +1556,10 @@ __device__ __forceinline__ uint32_t fine_place(float term, uint32_t shift, uint3
 // instructions per element took 20 us before any was found, and with many rows the call waits for the one that fetches most
 // often; with the next loads under way and one comparison per element a call of 512 mixed rows of 129,280 took 352 us
 // instead of 366.
-template <bool ROOMY>
+template <bool CHAINED>
 __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t positions, uint32_t misalignment, uint32_t shift, BinWalkShared& shared, int tid)
 {
-    constexpr uint32_t kLoads = ROOMY ? 8 : 4; // (twice: those under way and those looked at)
+    constexpr uint32_t kLoads = CHAINED ? 8 : 4; // (twice: those under way and those looked at)
     constexpr uint32_t kStride = kLoads * kWalkThreads;
     if (tid == 0)
     {
@@ -1432,7 +1576,7 @@ __device__ __forceinline__ void fetch_bins(const float* terms, uint32_t position
     const auto load = [&](uint4 (&raw)[kLoads], uint32_t at) {
 #pragma unroll
         for (uint32_t k = 0; k < kLoads; ++k)
-            raw[k] = reinterpret_cast<const uint4*>(terms)[min(at + k * kWalkThreads, vectors - 1u)];
+            raw[k] = taken_over_vector<CHAINED>(terms, positions * 4u, min(at + k * kWalkThreads, vectors - 1u));
     };
     // (a wave makes room for its elements with one addition: one addition, minimum and maximum an element, all of them to
     // the same three words, took 40 ns each, 60 us where the bins hold 1,500)
@@ -1680,7 +1824,7 @@ __device__ __forceinline__ void sum_head(HeadScratch& scratch, const float* term
 // fetches what it asks for.  Ends with shared.status 1 (ended: sum, stopped, ...) or 2 (given up).
 //   limit     elements that the sum runs over at most; cut_bin, cut_term: it ends at the first term below cut_term,
 //             which lies in that bin (kBins: nowhere)
-template <int PHASE, bool ROOMY>
+template <int PHASE, bool CHAINED>
 __device__ __forceinline__ void walk_bins(
     BinWalkShared& shared, uint32_t stops, const float* row_terms, uint32_t positions, uint32_t misalignment, uint32_t shift, uint32_t head_bins, uint32_t wide_first,
     uint32_t limit, uint32_t cut_bin, float cut_term, float start_sum, int mode, float bound, float divisor, float second_divisor, int tid)
@@ -1932,7 +2076,7 @@ __device__ __forceinline__ void walk_bins(
         __syncthreads();
         if (shared.status != 0u)
             return;
-        fetch_bins<ROOMY>(row_terms, positions, misalignment, shift, shared, tid);
+        fetch_bins<CHAINED>(row_terms, positions, misalignment, shift, shared, tid);
         fetched = true;
     }
 }
@@ -1952,7 +2096,7 @@ __device__ __noinline__ int32_t token_of_equal(
     const auto key_of = [&](uint32_t v, uint32_t c) { return descending_key(load_logit<DTYPE>(pointer, v * 4u + c - misalignment)); };
     // which of a vector's four elements match: the term, and the key where [least, most] is given
     const auto matching = [&](uint32_t v, bool by_key, uint32_t least, uint32_t most) {
-        const uint4 raw = reinterpret_cast<const uint4*>(terms)[v];
+        const uint4 raw = taken_over_vector<true>(terms, positions * 4u, v);
         uint32_t hits = (raw.x == wanted ? 1u : 0u) | (raw.y == wanted ? 2u : 0u) | (raw.z == wanted ? 4u : 0u) | (raw.w == wanted ? 8u : 0u);
         if (by_key)
         {
@@ -2122,23 +2266,23 @@ __device__ __forceinline__ int32_t token_of_listed(
 // ---- (4): walk 0 walks the normaliser and, inside the head, the Top-P sum and the draw, walk 1 the Top-P sum
 // behind the head (and the draw inside it), walk 2 the draw behind the head.  Walks 0 and 1 then have the bins' steps of the next
 // sum added for the calling part of the row, unless the row is finished.  Every part of a row walks for itself.
-// ROOMY: at most kRoomyRows rows, one workgroup to a compute unit.
+// CHAINED: a walk of bin_chain_kernel, which has written what the first one reads and has a compute unit to itself.
 
-// What a row's walks hand to each other: the same in each of its parts, which all do the same.
-struct BinWalkRow
+__device__ __forceinline__ uint8_t flags_of_row(const BinArgs& g, const ncnn_moe_sample_params& p, uint32_t saw_nan)
 {
-    float normalizer, renormalizer;
-    float head_sum;         // the next walk's sum behind the head
-    uint32_t limit;         // elements that it runs over at most
-    uint32_t kept;
-    uint32_t cut_bin;       // Min-P: the bin that holds the smallest term kept (kBins: no cut inside the bins), and that term
-    float cut_term;
-    uint32_t cut_in_tail;   // ... or it lies in no bin
-    uint32_t listed;        // elements in the list of the next walk (the first walk's holds the head, the others' places behind it)
-    uint32_t wide_first;    // of its sum: the first of the kWideBins bins with wide masks
-    uint4 words;            // the calling thread's four bins
-    uint4 before;           // their elements in the parts in front (where the next list takes this part's)
-};
+    return static_cast<uint8_t>((counts_as_select(g.windows_are_selects, g.a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
+                                (saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u));
+}
+
+// A row that is finished, or not served, before its first walk.
+__device__ __forceinline__ void end_early(const BinArgs& g, uint32_t part, uint32_t row, const ncnn_moe_sample_params& p, uint32_t state, uint32_t saw_nan, int tid)
+{
+    if (state == kBinRowRejected && part == 0u && tid == 0)
+    {
+        write_error(g.a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags_of_row(g, p, saw_nan));
+        g.a.row_state[row] = kRowDone;
+    }
+}
 
 enum BinWalkOutcome : uint32_t
 {
@@ -2146,59 +2290,44 @@ enum BinWalkOutcome : uint32_t
     kBinWalkGoesOn = 1 // the next walk goes on with it
 };
 
-template <int DTYPE, int WALK, bool ROOMY>
-__device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t row, BinWalkShared& shared, BinWalkRow& carried, int tid)
+template <int DTYPE, int WALK, bool CHAINED>
+__device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGrid& grid, uint32_t slot, uint32_t row, bool near, BinWalkShared& shared, uint4& words_of_thread, int tid)
 {
     constexpr int kFrom = WALK & 1;      // which of the alternating buffers this walk reads
     constexpr int kTo = kFrom ^ 1;
-    constexpr bool kAcross = WALK > 0;   // ... and whether this launch has written it
+    constexpr bool kAcross = WALK > 0 || CHAINED; // ... and whether this launch has written it
     const SamplerArgs& a = g.a;
     const uint32_t bin = 4u * static_cast<uint32_t>(tid);
     const bool holds_bins = tid < static_cast<int>(kBinQuads);
     BinRow& record = g.records[row];
-    const auto result_flags = [&](const ncnn_moe_sample_params& p) {
-        return static_cast<uint8_t>((counts_as_select(g.windows_are_selects, a.vocab, p) ? 0u : static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_GENERAL_PATH)) |
-                                    (record.saw_nan != 0u ? static_cast<uint32_t>(NCNN_MOE_ROW_FLAG_HAS_NAN) : 0u));
-    };
+    BinWalkRow& carried = shared.row;
+    const auto result_flags = [&](const ncnn_moe_sample_params& p) { return flags_of_row(g, p, carried.saw_nan); };
     {
-        if (WALK == 0)
-        {
-            const uint32_t state = same_in_all(record.state[1]);
-            if (state != kBinRowGoesOn)
-            {
-                if (state == kBinRowRejected && grid.part == 0u && tid == 0)
-                {
-                    write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, result_flags(a.params[row]));
-                    a.row_state[row] = kRowDone;
-                }
-                return kBinWalkEnds;
-            }
-        }
         __syncthreads(); // (a row before this one: its last readers of shared are done)
         if (tid < static_cast<int>(2u * kBinWords))
             shared.ties[tid] = 0u;
         if (tid == 0)
             shared.any_ties = 0u;
         __syncthreads();
-        const float top_p = same_in_all(a.params[row].top_p);
-        const float min_p = same_in_all(a.params[row].min_p);
-        const float uniform = same_in_all(a.uniforms[row]);
-        const uint32_t shift = same_in_all(record.shift);
-        const uint32_t window = same_in_all(record.window);
-        const uint32_t binned = same_in_all(record.binned);
-        const uint32_t head_bins = same_in_all(record.head_bins);
-        const uint32_t head_count = same_in_all(record.head_count);
-        const uint32_t listed = WALK == 0 ? same_in_all(record.listed) : carried.listed;
-        const uint32_t wide_first = WALK == 0 ? same_in_all(record.wide_first) : carried.wide_first;
-        const uint32_t limit = WALK == 0 ? window : carried.limit;
-        const uint32_t cut_bin = WALK == 1 ? carried.cut_bin : kBins;
-        const float cut_term = WALK == 1 ? carried.cut_term : 0.0f;
-        uint32_t cut_in_tail = WALK == 1 ? carried.cut_in_tail : 0u;
+        const float top_p = same_in_all(params_of(carried.options).top_p);
+        const float min_p = same_in_all(params_of(carried.options).min_p);
+        const float uniform = __uint_as_float(same_in_all(carried.options[kParamsWords]));
+        const uint32_t shift = same_in_all(carried.shift);
+        const uint32_t window = same_in_all(carried.window);
+        const uint32_t binned = same_in_all(carried.binned);
+        const uint32_t head_bins = same_in_all(carried.head_bins);
+        const uint32_t head_count = same_in_all(carried.head_count);
+        const uint32_t listed = same_in_all(carried.listed);
+        const uint32_t wide_first = same_in_all(carried.wide_first);
+        const uint32_t limit = WALK == 0 ? window : same_in_all(carried.limit);
+        const uint32_t cut_bin = WALK == 1 ? same_in_all(carried.cut_bin) : kBins;
+        const float cut_term = WALK == 1 ? same_in_all(carried.cut_term) : 0.0f;
+        uint32_t cut_in_tail = WALK == 1 ? same_in_all(carried.cut_in_tail) : 0u;
         const bool behind_head = limit > head_count && binned > head_count; // this launch's own sum goes on behind the head
-        float normalizer = WALK == 0 ? 1.0f : carried.normalizer;
-        float renormalizer = WALK == 2 ? carried.renormalizer : 1.0f;
-        const float sum_so_far = WALK == 0 ? 0.0f : carried.head_sum;
-        uint32_t kept = WALK == 2 ? carried.kept : 0u;
+        float normalizer = WALK == 0 ? 1.0f : same_in_all(carried.normalizer);
+        float renormalizer = WALK == 2 ? same_in_all(carried.renormalizer) : 1.0f;
+        const float sum_so_far = WALK == 0 ? 0.0f : same_in_all(carried.head_sum);
+        uint32_t kept = WALK == 2 ? same_in_all(carried.kept) : 0u;
         const BinStretch s = bin_stretch<LogitsVector<DTYPE>::kElementBytes>(a, row, grid.part, grid.parts);
         const uint32_t positions = (s.end + 7u) / 8u * 8u;
         const float* row_terms = bin_terms(a, row);
@@ -2218,27 +2347,40 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
             for (uint32_t k = 0; k < kPerThread; ++k)
             {
                 const uint32_t i = list_first + k * kWalkThreads + tid;
-                own_terms[k] = i < listed ? __uint_as_float(taken_over<kAcross>(reinterpret_cast<const uint32_t*>(from_terms) + i)) : 0.0f;
-                own_tokens[k] = i < listed ? taken_over<kAcross>(from_tokens + i) : 0u;
+                own_terms[k] = 0.0f;
+                own_tokens[k] = 0u;
+                if (list_first + k * kWalkThreads < listed)
+                {
+                    own_terms[k] = __uint_as_float(taken_over<kAcross>(from_terms, listed * 4u, i));
+                    own_tokens[k] = taken_over<kAcross>(from_tokens, listed * 4u, i);
+                }
             }
         }
-        uint4 words = WALK == 0 ? uint4{0u, 0u, 0u, 0u} : carried.words;
+        const uint4 words = words_of_thread;
         uint32_t own_steps[4] = {0u, 0u, 0u, 0u};
         uint32_t tie_word = 0, untold_word = 0;
         const uint32_t tie_lane = static_cast<uint32_t>(tid) & (kWaveSize - 1);
-        if (WALK == 0 && holds_bins)
-        {
-            words = reinterpret_cast<const uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid];
-            carried.before = reinterpret_cast<const uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid];
-        }
         if (behind_head)
         {
             const size_t first_pair = slot * grid.parts;
+            // (every wave collects the words of some parts' bins with terms half way: by one wave, a part behind the other, they
+            // arrived 2 us after everything else.  Asked for in front of the steps, whose loads are waited for one by one)
+            constexpr uint32_t kEach = kMaxBinParts / kWalkWaves;
+            static_assert(kMaxBinParts % kWalkWaves == 0, "as many parts for each wave");
+            uint32_t words_of_part[kEach][3];
+#pragma unroll
+            for (uint32_t k = 0; k < kEach; ++k)
+            {
+                const uint32_t q = same_in_all(static_cast<uint32_t>(tid) / kWaveSize) + k * kWalkWaves;
+#pragma unroll
+                for (uint32_t w = 0; w < 3u; ++w)
+                    words_of_part[k][w] = taken_over<kAcross>(g.ties[kFrom] + first_pair * 3u * kBinWords, grid.parts * 3u * kBinWords * 4u, (q * 3u + w) * kBinWords + tie_lane);
+            }
             if (holds_bins && bin + 3u >= head_bins)
             {
                 uint32_t* const from = g.steps[kFrom] + first_pair * kBins;
                 const uint32_t bytes = grid.parts * kBins * 4u;
-                constexpr uint32_t kTogether = ROOMY ? kMaxBinParts : kPartsAtATime;
+                constexpr uint32_t kTogether = CHAINED ? kMaxBinParts : kPartsAtATime;
                 for (uint32_t first = 0; first < grid.parts; first += kTogether)
                 {
                     uint4 of_part[kTogether];
@@ -2254,18 +2396,13 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                     }
                 }
             }
-            // (every wave collects the words of some parts' bins with terms half way: by one wave, a part behind the other, they
-            // arrived 2 us after everything else)
             if (tie_lane < kBinWords)
             {
-                static_assert(kMaxBinParts % kWalkWaves == 0, "as many parts for each wave");
 #pragma unroll
-                for (uint32_t k = 0; k < kMaxBinParts / kWalkWaves; ++k)
+                for (uint32_t k = 0; k < kEach; ++k)
                 {
-                    const uint32_t q = static_cast<uint32_t>(tid) / kWaveSize + k * kWalkWaves;
-                    const uint32_t* from = g.ties[kFrom] + (first_pair + min(q, grid.parts - 1u)) * 3u * kBinWords + tie_lane;
-                    tie_word |= taken_over<kAcross>(from);
-                    untold_word |= taken_over<kAcross>(from + kBinWords) | taken_over<kAcross>(from + 2u * kBinWords);
+                    tie_word |= words_of_part[k][0];
+                    untold_word |= words_of_part[k][1] | words_of_part[k][2];
                 }
             }
         }
@@ -2323,18 +2460,16 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                 const uint32_t mask_count = min(shared.mask_count, kBinMasks);
                 for (uint32_t i = static_cast<uint32_t>(tid) / kMaxBinParts; i < mask_count; i += kWalkThreads / kMaxBinParts)
                 {
-                    const uint32_t* const of_part = g.masks[kFrom] + static_cast<size_t>(slot * grid.parts + min(part, grid.parts - 1u)) * kMaskWords;
+                    const uint32_t* const of_parts = g.masks[kFrom] + static_cast<size_t>(slot * grid.parts) * kMaskWords;
+                    const uint32_t bytes = grid.parts * kMaskWords * 4u; // (a part that there is not, and a word that there is not: zero)
                     const uint32_t mask_bin = shared.mask_bin[i];
                     const bool wide = mask_bin - wide_first < kWideBins;
-                    const uint32_t* const wide_masks = of_part + 2u * kBins + (wide ? mask_bin - wide_first : 0u) * kWideWords;
                     uint32_t words_of_bin[kWideWords];
 #pragma unroll
                     for (uint32_t w = 0; w < kWideWords; ++w)
                     {
-                        const uint32_t word = wide ? taken_over<kAcross>(wide_masks + w)
-                            : w == 0u ? taken_over<kAcross>(of_part + mask_bin)
-                            : w == kWideParities ? taken_over<kAcross>(of_part + kBins + mask_bin) : 0u;
-                        words_of_bin[w] = part < grid.parts ? word : 0u;
+                        const uint32_t narrow = w == 0u ? mask_bin : w == kWideParities ? kBins + mask_bin : bytes;
+                        words_of_bin[w] = taken_over<kAcross>(of_parts, bytes, part * kMaskWords + (wide ? 2u * kBins + (mask_bin - wide_first) * kWideWords + w : narrow));
                     }
                     uint32_t twice = 0u;
 #pragma unroll
@@ -2502,7 +2637,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                 mass[j] += sum;
             if (behind_head)
             {
-                walk_bins<0, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
+                walk_bins<0, CHAINED>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, window, kBins, 0.0f, sum, kStopNever, 0.0f, 1.0f, 1.0f, tid);
                 given_up = shared.status == 2u;
                 sum = same_in_all(shared.sum);
             }
@@ -2568,7 +2703,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
         }
         if constexpr (WALK == 1)
         {
-            walk_bins<1, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
+            walk_bins<1, CHAINED>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, cut_bin, cut_term, sum_so_far, kStopAtOrAbove, top_p,
                          normalizer, 1.0f, tid);
             const bool stopped = shared.stopped != 0u;
             // (a sum that no stop condition ends runs to the window's end, or to the Min-P cut, which no bin may hold)
@@ -2595,7 +2730,8 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
             const bool stopped_behind = !in_head && WALK == 1 && shared.stopped != 0u;
             const uint32_t last = in_head ? kept - 1u : stopped_behind ? same_in_all(shared.stop_at) : 0xffffffffu;
             const bool in_equal = stopped_behind && last == 0xffffffffu; // ... among thousands of equal terms
-            const bool unlimited = a.params[row].top_k == 0u || a.params[row].top_k >= a.vocab;
+            const uint32_t top_k = same_in_all(params_of(carried.options).top_k);
+            const bool unlimited = top_k == 0u || top_k >= a.vocab;
             const bool runs_on = !in_head && !stopped_behind;
             const bool by_cut = runs_on && WALK == 1 && cut_bin < kBins && (unlimited || kept < limit);
             const bool everything = by_cut || (runs_on && kept == window && min_p == 0.0f && unlimited);
@@ -2645,7 +2781,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
             }
             if constexpr (WALK == 2)
             {
-                walk_bins<2, ROOMY>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
+                walk_bins<2, CHAINED>(shared, stops, row_terms, positions, s.misalignment, shift, head_bins, wide_first, limit, kBins, 0.0f, sum_so_far, kStopAbove, uniform,
                              normalizer, renormalizer, tid);
                 // (no partial sum exceeds the draw: the last element kept, which may lie anywhere: left to the full-order kernels)
                 at = same_in_all(shared.stop_at);
@@ -2674,7 +2810,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                     }
                     if (tid == 0)
                     {
-                        const ncnn_moe_sample_params p = a.params[row];
+                        const ncnn_moe_sample_params p = params_of(carried.options);
                         write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, result_flags(p));
                         a.row_state[row] = kRowDone;
                         record.served = 1u;
@@ -2695,6 +2831,9 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
 #pragma unroll
             for (int j = 0; j < 5; ++j)
                 mass[j] *= scale;
+            uint4 before{0u, 0u, 0u, 0u}; // elements of the thread's bins in the parts in front (where the next list takes this part's)
+            if (holds_bins)
+                before = reinterpret_cast<const uint4*>(g.before + static_cast<size_t>(slot * grid.parts + grid.part) * kBins)[tid];
             BinPlan plan = plan_bins(bin, front, mass, head_bins, next_limit, next_cut_bin, WALK == 0 ? top_p : uniform, kForeseenLater, shift,
                                      1.0f / (WALK == 0 ? normalizer : normalizer * renormalizer));
             uint32_t to_list[1] = {holds_bins ? plan.listed : 0u};
@@ -2731,7 +2870,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                 if (leads_wave(next_wide < kBins))
                     atomicMin(&shared.wide_first, next_wide);
                 uint32_t next_packed[4];
-                const uint32_t in_front[4] = {carried.before.x, carried.before.y, carried.before.z, carried.before.w};
+                const uint32_t in_front[4] = {before.x, before.y, before.z, before.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
@@ -2742,33 +2881,36 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                     entries[bin + j] = entry;
                 }
                 *reinterpret_cast<uint4*>(steps + bin) = uint4{0u, 0u, 0u, 0u};
-                carried.words = uint4{next_packed[0], next_packed[1], next_packed[2], next_packed[3]};
+                words_of_thread = uint4{next_packed[0], next_packed[1], next_packed[2], next_packed[3]};
             }
             __syncthreads();
             if (own_end != 0u && holds_bins)
                 atomicMax(&shared.listed_end, own_end);
-            add_bin_steps<WALK + 1, kWalkThreads>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks, shared.wide_first,
-                                                  g.list_terms[kTo] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[kTo] + static_cast<size_t>(row) * kBinListCap, tid);
+            add_bin_steps<WALK + 1, kWalkThreads, CHAINED>(row_terms, s, shift, head_bins, kBins - head_bins, normalizer, renormalizer, entries, steps, ties, masks, shared.wide_first,
+                                                  g.list_terms[kTo] + static_cast<size_t>(row) * kBinListCap, g.list_tokens[kTo] + static_cast<size_t>(row) * kBinListCap, near, tid);
             __syncthreads();
             const size_t pair = slot * grid.parts + grid.part;
             if (holds_bins)
-                hand_over_vector<true>(g.steps[kTo] + pair * kBins, kBins * 4u, static_cast<uint32_t>(tid), *reinterpret_cast<uint4*>(steps + bin));
+                hand_over_vector(near, g.steps[kTo] + pair * kBins, kBins * 4u, static_cast<uint32_t>(tid), *reinterpret_cast<uint4*>(steps + bin));
             for (uint32_t i = tid; i < kMaskWords / 4u; i += kWalkThreads)
-                hand_over_vector<true>(g.masks[kTo] + pair * kMaskWords, kMaskWords * 4u, i, reinterpret_cast<uint4*>(masks)[i]);
+                hand_over_vector(near, g.masks[kTo] + pair * kMaskWords, kMaskWords * 4u, i, reinterpret_cast<uint4*>(masks)[i]);
             if (tid < static_cast<int>(3u * kBinWords))
-                hand_over<true>(g.ties[kTo] + pair * 3u * kBinWords + tid, ties[tid]);
-            carried.normalizer = normalizer;
-            carried.renormalizer = renormalizer;
-            carried.kept = kept;
-            carried.head_sum = head_sum;
-            carried.limit = same_in_all(next_limit);
-            carried.listed = same_in_all(max(shared.listed_end, head_count));
-            carried.wide_first = same_in_all(shared.wide_first);
-            if (WALK == 0)
+                hand_over(near, g.ties[kTo] + pair * 3u * kBinWords, 3u * kBinWords * 4u, static_cast<uint32_t>(tid), ties[tid]);
+            if (tid == 0)
             {
-                carried.cut_bin = next_cut_bin;
-                carried.cut_term = next_cut_term;
-                carried.cut_in_tail = cut_in_tail;
+                carried.normalizer = normalizer;
+                carried.renormalizer = renormalizer;
+                carried.kept = kept;
+                carried.head_sum = head_sum;
+                carried.limit = next_limit;
+                carried.listed = max(shared.listed_end, head_count);
+                carried.wide_first = shared.wide_first;
+                if (WALK == 0)
+                {
+                    carried.cut_bin = next_cut_bin;
+                    carried.cut_term = next_cut_term;
+                    carried.cut_in_tail = cut_in_tail;
+                }
             }
         }
     }
@@ -2784,25 +2926,39 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
 // (some 20 ms) gives up for the whole row, which is then left to the full-order kernels, as are the rows of a GPU on which
 // fewer workgroups run at a time than a row has parts.
 //
-// arrivals[0] counts the parts that have come to the row's meetings, arrivals[1] those that are done with the row: the last of them
-// returns both to zero.
+// arrivals[0] counts the parts that have come to the row's meetings and, above, how many came to the first from each XCD: from then on
+// shared.near tells whether all are on one.  arrivals[1] counts those that are done with the row: the last of them returns both to zero.
 constexpr uint32_t kMostLooks = 40000;
-constexpr uint32_t kRowGivenUp = 0x80000000u;
+constexpr unsigned long long kArrivalsOnly = 0xffffull;
+constexpr unsigned long long kRowGivenUp = 1ull << 63;
+constexpr uint32_t kXcdShift = 16, kXcdBits = 5;
+static_assert(kMaxBinParts < 1u << kXcdBits, "the parts that come from one XCD are counted in kXcdBits");
 
-__device__ __forceinline__ bool parts_meet(uint32_t* arrivals, uint32_t parts, uint32_t meeting, bool wait, uint32_t most_looks, BinWalkShared& shared, int tid)
+__device__ __forceinline__ uint32_t own_xcd()
 {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (stores of agent scope: they have arrived when they are counted)
-    __syncthreads();
+    return __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u; // HW_REG_XCC_ID
+}
+
+__device__ __forceinline__ bool parts_meet(unsigned long long* arrivals, uint32_t parts, uint32_t meeting, bool wait, uint32_t most_looks, BinWalkShared& shared, int tid)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (stores have arrived in the L2, or in memory, when they are counted)
     if (parts == 1u)
+    {
+        if (tid == 0)
+            shared.near = 1u;
+        __syncthreads();
         return true;
+    }
+    __syncthreads();
     if (tid == 0)
     {
-        uint32_t seen = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        const unsigned long long own_place = 1ull << (kXcdShift + kXcdBits * own_xcd());
+        const unsigned long long one = meeting == 1u ? 1ull + own_place : 1ull;
+        unsigned long long seen = __hip_atomic_fetch_add(arrivals, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + one;
         const uint32_t goal = meeting * parts;
-        for (uint32_t looks = 0; wait && (seen & ~kRowGivenUp) < goal; ++looks)
+        const auto come = [&]() { return static_cast<uint32_t>(seen & kArrivalsOnly) >= goal; };
+        for (uint32_t looks = 0; wait && !come() && (seen & kRowGivenUp) == 0ull; ++looks)
         {
-            if ((seen & kRowGivenUp) != 0u)
-                break;
             if (looks == most_looks)
             {
                 __hip_atomic_fetch_or(arrivals, kRowGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2811,18 +2967,20 @@ __device__ __forceinline__ bool parts_meet(uint32_t* arrivals, uint32_t parts, u
             __builtin_amdgcn_s_sleep(1);
             seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        shared.met = wait && (seen & ~kRowGivenUp) >= goal ? 1u : 0u;
+        shared.met = wait && come() ? 1u : 0u;
+        if (meeting == 1u)
+            shared.near = (seen & ~kRowGivenUp) >> kXcdShift == parts * (own_place >> kXcdShift) ? 1u : 0u;
     }
     __syncthreads();
     return same_in_all(shared.met) != 0u;
 }
 
-__device__ __forceinline__ void part_leaves(uint32_t* arrivals, uint32_t parts, int tid)
+__device__ __forceinline__ void part_leaves(unsigned long long* arrivals, uint32_t parts, int tid)
 {
-    if (parts > 1u && tid == 0 && __hip_atomic_fetch_add(arrivals + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == parts)
+    if (parts > 1u && tid == 0 && __hip_atomic_fetch_add(arrivals + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ull == parts)
     {
-        __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(arrivals + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(arrivals + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -2836,8 +2994,23 @@ __device__ __forceinline__ const BinArgs& arguments_read_anew()
     return *(const BinArgs*)p;
 }
 
-template <int DTYPE, bool ROOMY>
-__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(ROOMY ? 2 : 4, ROOMY ? 2 : 4))) void bin_walks_kernel(BinArgs g)
+// The walks of a row, from where its parts have met `met` times (not at all: whether they are on one XCD is not known before the first
+// walk has handed over).
+template <int DTYPE, bool CHAINED>
+__device__ __forceinline__ void walk_row(
+    const BinGrid& grid, uint32_t slot, uint32_t row, unsigned long long* arrivals, uint32_t met, uint32_t most_looks, BinWalkShared& shared, uint4 words, int tid)
+{
+    const auto near = [&]() { return same_in_all(shared.near) != 0u; };
+    // (behind the second meeting the first part goes on alone)
+    if (bin_walk<DTYPE, 0, CHAINED>(arguments_read_anew(), grid, slot, row, CHAINED ? near() : grid.parts == 1u, shared, words, tid) == kBinWalkGoesOn &&
+        parts_meet(arrivals, grid.parts, met + 1u, true, most_looks, shared, tid) &&
+        bin_walk<DTYPE, 1, CHAINED>(arguments_read_anew(), grid, slot, row, near(), shared, words, tid) == kBinWalkGoesOn &&
+        parts_meet(arrivals, grid.parts, met + 2u, grid.part == 0u, most_looks, shared, tid) && grid.part == 0u)
+        bin_walk<DTYPE, 2, CHAINED>(arguments_read_anew(), grid, slot, row, true, shared, words, tid);
+}
+
+template <int DTYPE>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void bin_walks_kernel(BinArgs g)
 {
     __shared__ BinWalkShared shared;
     const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
@@ -2845,15 +3018,90 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RO
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
         const uint32_t row = same_in_all(g.list[1u + slot]);
-        uint32_t* const arrivals = g.arrivals + static_cast<size_t>(row) * kArrivalWords;
-        BinWalkRow carried;
-        // (behind the second meeting the first part goes on alone)
-        if (bin_walk<DTYPE, 0, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid) == kBinWalkGoesOn &&
-            parts_meet(arrivals, grid.parts, 1u, true, g.most_looks, shared, tid) &&
-            bin_walk<DTYPE, 1, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid) == kBinWalkGoesOn &&
-            parts_meet(arrivals, grid.parts, 2u, grid.part == 0u, g.most_looks, shared, tid) && grid.part == 0u)
-            bin_walk<DTYPE, 2, ROOMY>(arguments_read_anew(), grid, slot, row, shared, carried, tid);
+        unsigned long long* const arrivals = g.arrivals + static_cast<size_t>(row) * kArrivalWords;
+        const BinRow& record = g.records[row];
+        const uint32_t state = same_in_all(record.state[1]);
+        if (tid == 0)
+        {
+            shared.row.shift = record.shift;
+            shared.row.window = record.window;
+            shared.row.saw_nan = record.saw_nan;
+            shared.row.binned = record.binned;
+            shared.row.head_bins = record.head_bins;
+            shared.row.head_count = record.head_count;
+            shared.row.listed = record.listed;
+            shared.row.wide_first = record.wide_first;
+        }
+        const uint32_t option = read_option(g.a, row, tid);
+        uint4 words{0u, 0u, 0u, 0u};
+        if (tid < static_cast<int>(kBinQuads))
+            words = reinterpret_cast<const uint4*>(g.packed + static_cast<size_t>(row) * kBins)[tid];
+        if (tid < static_cast<int>(kRowOptionWords))
+            shared.row.options[tid] = option;
+        __syncthreads();
+        if (state == kBinRowGoesOn)
+            walk_row<DTYPE, false>(grid, slot, row, arrivals, 0u, g.most_looks, shared, words, tid);
+        else
+            end_early(g, grid.part, row, params_of(shared.row.options), state, record.saw_nan, tid);
         part_leaves(arrivals, grid.parts, tid);
+        __syncthreads();
+    }
+}
+
+// (1) to (4) in one launch.
+template <int DTYPE>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void bin_chain_kernel(BinArgs g)
+{
+    __shared__ BinWalkShared shared;
+    __shared__ BinSumShared of_sum;
+    __shared__ RowList listed_rows;
+    __shared__ uint4 stats[kMaxBinParts];
+    __shared__ uint64_t exp2_table[32];
+    static_assert(kWalkWaves <= static_cast<int>(kMaxBinParts), "the waves' statistics and the parts' take turns");
+    const int tid = threadIdx.x;
+    if (tid < 32)
+        exp2_table[tid] = kExp2Table[tid];
+    const uint32_t rows = list_rows_in_place<kWalkWaves>(g.a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
+    const BinGrid grid = bin_grid(rows, g.a.vocab, kChainGrid);
+    for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
+    {
+        const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
+        unsigned long long* const arrivals = g.arrivals + static_cast<size_t>(row) * kArrivalWords;
+        const BinStretch s = bin_stretch<LogitsVector<DTYPE>::kElementBytes>(g.a, row, grid.part, grid.parts);
+        const uint32_t option = read_option(g.a, row, tid);
+        if (grid.part == 0u && tid == 0)
+        {
+            // (whatever becomes of the row: an earlier call's do not count)
+            g.records[row].served = 0u;
+            g.records[row].filtered = 0u;
+        }
+        const uint4 of_part = stats_of_part<DTYPE, kWalkThreads>(g.a, grid, row, stats, tid);
+        if (tid < static_cast<int>(kRowOptionWords))
+            shared.row.options[tid] = option;
+        if (tid == 0)
+            hand_over_vector(grid.parts == 1u, g.stats + slot * grid.parts, grid.parts * 16u, grid.part, of_part);
+        if (parts_meet(arrivals, grid.parts, 1u, true, g.most_looks, shared, tid))
+        {
+            const bool near = same_in_all(shared.near) != 0u;
+            const BinRowStart start = terms_of_part<DTYPE, kWalkThreads, true>(arguments_read_anew(), grid, slot, row, params_of(shared.row.options), near, shared.tokens, stats, exp2_table, tid);
+            if (tid == 0)
+            {
+                shared.row.shift = start.shift;
+                shared.row.window = start.window;
+                shared.row.saw_nan = start.saw_nan;
+            }
+            if (same_in_all(start.state) != kBinRowGoesOn)
+                end_early(g, grid.part, row, params_of(shared.row.options), start.state, start.saw_nan, tid);
+            else if (parts_meet(arrivals, grid.parts, 2u, true, g.most_looks, shared, tid))
+            {
+                const uint4 words = sum_of_part<kWalkThreads, true>(arguments_read_anew(), grid, slot, row, same_in_all(params_of(shared.row.options).top_p),
+                    same_in_all(params_of(shared.row.options).min_p), near, s, shared.prefix, shared.packed, shared.tokens, shared.tokens + kMaskWords, shared.scan, of_sum, shared.row, tid);
+                if (parts_meet(arrivals, grid.parts, 3u, true, g.most_looks, shared, tid))
+                    walk_row<DTYPE, true>(grid, slot, row, arrivals, 3u, g.most_looks, shared, words, tid);
+            }
+        }
+        part_leaves(arrivals, grid.parts, tid);
+        __syncthreads();
     }
 }
 
