@@ -76,16 +76,7 @@ void launch_select(const RouterArgs& args, hipStream_t stream)
         hipLaunchKernelGGL(router_select_kernel<SLOTS>, dim3(staged_blocks), dim3(kRouterThreads), 0, stream, args);
         return;
     }
-    // Two tokens per wave where a token is little work (128 experts at most) and there are enough of them to fill the SIMDs'
-    // waves all the same; else one, which leaves more waves to hide behind.  One against two, us, softmax: 1,024 tokens of
-    // 128 experts and 8 routes 13.9 / 14.3, 2,048 14.8 / 14.8, 4,096 15.9 / 15.6, 16,384 25.7 / 22.7; of 8 experts and 2 routes
-    // 13.9 / 14.1, 18.2 / 18.2, 18.6 / 18.3, 28.3 / 21.6.
-    const uint32_t tokens_per_wave = SLOTS <= 2 && args.tokens >= 4096u ? 2u : 1u;
-    const unsigned blocks = (args.tokens + kBatchWaves * tokens_per_wave - 1u) / (kBatchWaves * tokens_per_wave);
-    if (tokens_per_wave == 2u)
-        hipLaunchKernelGGL((router_batch_kernel<SLOTS, SLOTS <= 2 ? 2 : 1>), dim3(blocks), dim3(kBatchThreads), 0, stream, args);
-    else
-        hipLaunchKernelGGL((router_batch_kernel<SLOTS, 1>), dim3(blocks), dim3(kBatchThreads), 0, stream, args);
+    hipLaunchKernelGGL(router_batch_kernel<SLOTS>, dim3((args.tokens + kBatchWaves - 1u) / kBatchWaves), dim3(kBatchThreads), 0, stream, args);
     const unsigned chunks = (args.tokens + kRouterChunkTokens - 1) / kRouterChunkTokens;
     hipLaunchKernelGGL(router_group_kernel, dim3(chunks), dim3(kRouterThreads), 0, stream, args);
 }

@@ -181,6 +181,31 @@ __device__ __forceinline__ float sequential_row_sums(const float* row_of_lane, u
     return sum;
 }
 
+// The same by 16 lanes: each holds four consecutive scores and adds them to the sum that its lower neighbour holds, 16 times over
+// for 64 scores; after turn k the lanes up to k are final.  The wave's four rows of lanes do the same; every lane returns the sum.  256
+// scores: 280 instructions and four reads of LDS, where a chain on broadcast reads takes 320 and 64, 512 cycles of the compute unit's LDS
+// (300 tokens of 512 experts 17.2 -> 16.1 us, 16,384 of 256 28.7 -> 28.1).
+__device__ __forceinline__ float sequential_sum_by_lanes(const float* row, uint32_t padded, int lane)
+{
+    const int place = lane & 15;
+    float sum = 0.0f;
+#pragma unroll 1
+    for (uint32_t first = 0; first < padded; first += kWaveSize)
+    {
+        float4 own = *reinterpret_cast<const float4*>(row + first + 4u * static_cast<uint32_t>(place));
+        const float carried = __uint_as_float(dpp_source<0x121, 0xf>(__float_as_uint(sum))); // row_ror:1: the first lane reads the last
+        own.x = place == 0 ? carried + own.x : own.x;
+        sum = 0.0f;
+#pragma unroll
+        for (int turn = 0; turn < 16; ++turn)
+        {
+            // (row_shr:1; the first lane reads 0, which leaves its sum as it is)
+            sum = (((__uint_as_float(dpp_source<0x111, 0xf>(__float_as_uint(sum))) + own.x) + own.y) + own.z) + own.w;
+        }
+    }
+    return read_lane(sum, 15);
+}
+
 // ---- select_topk_routes (src/graph/expert_dispatcher.cpp:61-77): the best top_k of a token's experts by (score + bias
 // descending, expert id ascending).  Expert e lives in slot e / 64 of lane e % 64.
 // A threshold with top_k to `most` scores at or above it is searched over the scores' order-preserving bits: from the
@@ -334,9 +359,11 @@ __device__ __forceinline__ bool take_explicit(const RouterArgs& r, const float* 
     return true;
 }
 
-// A token's routes from its scores in LDS (not yet divided by `divisor`), by one wave.
+// A token's routes from its scores in LDS (not yet divided by `divisor`), by one wave.  Not FUSED: `held` has them as well, expert e in slot
+// e / 64 of lane e % 64 (zeros past the last expert), and `counts`, in LDS, counts the routes to each expert.
 template <int SLOTS, bool FUSED>
-__device__ __forceinline__ void route_token(const RouterArgs& r, const float* scores, float divisor, RouteScratch& scratch, uint32_t token, int lane)
+__device__ __forceinline__ void route_token(
+    const RouterArgs& r, const float* scores, const float (&held)[SLOTS], float divisor, RouteScratch& scratch, uint32_t* counts, uint32_t token, int lane)
 {
     uint32_t my_expert, my_rank;
     float my_score, selected_sum;
@@ -353,7 +380,7 @@ __device__ __forceinline__ void route_token(const RouterArgs& r, const float* sc
         {
             const uint32_t e = static_cast<uint32_t>(s * kWaveSize + lane);
             bias[s] = (e < r.experts && r.selection_bias != nullptr) ? r.selection_bias[e] : 0.0f;
-            score[s] = e < r.experts ? scores[e] : 0.0f;
+            score[s] = FUSED ? (e < r.experts ? scores[e] : 0.0f) : held[s];
         }
         if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
         {
@@ -386,120 +413,97 @@ __device__ __forceinline__ void route_token(const RouterArgs& r, const float* sc
             *expert_out = my_expert;
             *weight_out = weight;
             // (a call of one chunk is counted by the workgroup that groups it)
-            atomicAdd(&r.chunk_counts[static_cast<size_t>(token / kRouterChunkTokens) * chunk_count_stride(r.experts) + my_expert], 1u);
+            atomicAdd(&counts[my_expert], 1u);
         }
     }
 }
 
-// Calls of more than one chunk: a wave takes TOKENS tokens from their logits to their routes, without waiting for another
-// wave.  The scores pass through LDS, so that the softmax sum, one addition at a time in expert order, is a chain of
-// additions on four scores a read (lane reads, one per addition, took half as long again), one for all of the wave's tokens.
-// What bounds it: instructions, some 680 per token of 256 experts under the softmax: 320 for the sum, 110 for the
-// exponentials, 50 for the divisions, 130 for the selection.  16,384 tokens, 8 routes of 256 experts, softmax: 44 us with
-// one wave-wide maximum per route, 20 us so.  Sums of several waves' tokens by one of them, behind barriers, take half of
-// the instructions and no less time.
-constexpr int kBatchWaves = 4;
+// Calls of more than one chunk: a wave takes a token from its logits to its routes, without waiting for another wave.  Under the softmax
+// the scores pass through LDS, so that their sum, one addition at a time in expert order, is a chain of additions on few reads.
+// The workgroup's routes are counted in LDS and added to the chunk's counters a line at a time: an atomic a route cost as much as all
+// the rest where experts are few (8 experts and 2 routes, 2,048 tokens 18.2 -> 9.7 us, 16,384 26.8 -> 14.8; 64 and 6, 1,024 tokens
+// 13.2 -> 10.5, 16,384 22.1 -> 18.9; 256 and 8, 16,384 28.7 -> 27.2).  Eight waves rather than four: fewer such additions (16,384 of 8
+// experts 14.8 and 16.4 us); two or four tokens a wave: 0 to 15 % slower from 64 experts on.
+// What bounds it: instructions, some 640 per token of 256 experts under the softmax: 280 for the sum, 110 for the exponentials, 50 for
+// the divisions, 130 for the selection.
+constexpr int kBatchWaves = 8;
 constexpr int kBatchThreads = kBatchWaves * kWaveSize;
+static_assert(kRouterChunkTokens % kBatchWaves == 0, "a workgroup's tokens are of one chunk");
 
-template <int SLOTS, int TOKENS>
+template <int SLOTS>
 __global__ __launch_bounds__(kBatchThreads) void router_batch_kernel(RouterArgs r)
 {
-    constexpr uint32_t kRow = SLOTS * kWaveSize + 4; // (the rows' offset keeps the lanes of the sums on different banks)
-    __shared__ __align__(16) float rows[kBatchWaves * TOKENS * kRow];
+    __shared__ __align__(16) float rows[kBatchWaves][SLOTS * kWaveSize];
     __shared__ __align__(16) RouteScratch scratch[kBatchWaves];
+    __shared__ uint32_t counts[SLOTS * kWaveSize]; // the workgroup's routes to each expert
     __shared__ uint64_t exp2_table[32];
     const int lane = threadIdx.x & (kWaveSize - 1);
-    const int wave = threadIdx.x >> 6;
-    const uint32_t first_token = (blockIdx.x * kBatchWaves + static_cast<uint32_t>(wave)) * TOKENS;
-    float* const own_rows = rows + wave * TOKENS * kRow;
-    float logit[TOKENS][SLOTS];
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint32_t token = blockIdx.x * kBatchWaves + static_cast<uint32_t>(wave);
+    const float* const logits = r.logits + static_cast<size_t>(min(token, r.tokens - 1u)) * r.experts;
+    float score[SLOTS];
 #pragma unroll
-    for (int t = 0; t < TOKENS; ++t)
+    for (int s = 0; s < SLOTS; ++s)
     {
-        const float* logits = r.logits + static_cast<size_t>(min(first_token + t, r.tokens - 1u)) * r.experts;
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-        {
-            const uint32_t e = static_cast<uint32_t>(s * kWaveSize + lane);
-            logit[t][s] = e < r.experts ? logits[e] : -__builtin_inff();
-        }
+        const uint32_t e = static_cast<uint32_t>(s * kWaveSize + lane);
+        score[s] = e < r.experts ? logits[e] : -__builtin_inff();
     }
     if (threadIdx.x < 32)
         exp2_table[threadIdx.x] = kExp2Table[threadIdx.x];
+    for (uint32_t e = threadIdx.x; e < SLOTS * kWaveSize; e += kBatchThreads)
+        counts[e] = 0u;
     __syncthreads();
-    // lane t: the largest logit of token t
-    float maxima = 0.0f;
-    uint32_t failed = 0u; // the tokens with a logit that is not finite
+    bool finite = true;
+    float maximum = -__builtin_inff();
 #pragma unroll
-    for (int t = 0; t < TOKENS; ++t)
+    for (int s = 0; s < SLOTS; ++s)
     {
-        bool finite = true;
-        float maximum = -__builtin_inff();
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-        {
-            finite = finite && (static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts || is_finite_f32(logit[t][s]));
-            maximum = fmaxf(maximum, logit[t][s]);
-            own_rows[t * kRow + s * kWaveSize + lane] = logit[t][s];
-        }
+        finite = finite && (static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts || is_finite_f32(score[s]));
+        maximum = fmaxf(maximum, score[s]);
+    }
+    if (token < r.tokens)
+    {
         if (__builtin_amdgcn_ballot_w64(!finite) != 0ull)
-            failed |= 1u << t;
-        if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
-        {
-            maximum = wave_max(maximum);
-            maxima = lane == t ? maximum : maxima;
-        }
-    }
-    // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
-    float sums = 1.0f;
-    const auto each_score = [&](auto score_of) {
-#pragma unroll 1
-        for (int t = 0; t < TOKENS; ++t)
-        {
-            float* const row = own_rows + t * kRow + lane;
-            const float maximum = read_lane(maxima, t);
-            // (four experts of a lane overlap; more would take registers that waves in flight need)
-            constexpr int kTogether = SLOTS < 4 ? SLOTS : 4;
-#pragma unroll 1
-            for (int first = 0; first < SLOTS; first += kTogether)
-            {
-                float score[kTogether];
-#pragma unroll
-                for (int s = 0; s < kTogether; ++s)
-                    score[s] = score_of(row[(first + s) * kWaveSize], maximum);
-#pragma unroll
-                for (int s = 0; s < kTogether; ++s)
-                    row[(first + s) * kWaveSize] = score[s];
-            }
-        }
-        wave_lds_fence();
-    };
-    wave_lds_fence();
-    if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
-    {
-        // (past the last expert: exp(-inf) is 0)
-        each_score([&](float x, float maximum) { return expf_selects(x - maximum, exp2_table); });
-        sums = sequential_row_sums(own_rows + (lane % TOKENS) * kRow, SLOTS * kWaveSize);
-    }
-    else if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
-        each_score([&](float x, float) { return sigmoid_score(x, exp2_table); });
-    else
-        each_score([&](float x, float) { return sqrt_softplus_score(x, exp2_table); });
-#pragma unroll 1
-    for (int t = 0; t < TOKENS; ++t)
-    {
-        const uint32_t token = first_token + static_cast<uint32_t>(t);
-        if (token >= r.tokens)
-            break;
-        if ((failed >> t & 1u) != 0u)
         {
             // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
             if (lane == 0)
                 atomicOr(&r.error_words[0], 1u);
-            continue;
         }
-        route_token<SLOTS, false>(r, own_rows + t * kRow, read_lane(sums, t), scratch[wave], token, lane);
-        wave_lds_fence();
+        else
+        {
+            // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
+            float sum = 1.0f;
+            // (past the last expert: 0)
+            const auto each_score = [&](auto score_of) {
+#pragma unroll
+                for (int s = 0; s < SLOTS; ++s)
+                {
+                    const float of_expert = score_of(score[s]);
+                    score[s] = static_cast<uint32_t>(s * kWaveSize + lane) < r.experts ? of_expert : 0.0f;
+                    rows[wave][s * kWaveSize + lane] = score[s];
+                }
+                wave_lds_fence();
+            };
+            if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+            {
+                maximum = wave_max(maximum);
+                each_score([&](float x) { return expf_selects(x - maximum, exp2_table); });
+                sum = sequential_sum_by_lanes(rows[wave], (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize, lane);
+            }
+            else if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
+                each_score([&](float x) { return sigmoid_score(x, exp2_table); });
+            else
+                each_score([&](float x) { return sqrt_softplus_score(x, exp2_table); });
+            route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], counts, token, lane);
+        }
+    }
+    __syncthreads();
+    const uint32_t chunk = blockIdx.x * kBatchWaves / kRouterChunkTokens;
+    for (uint32_t e = threadIdx.x; e < r.experts; e += kBatchThreads)
+    {
+        const uint32_t count = counts[e];
+        if (count != 0u)
+            atomicAdd(&r.chunk_counts[static_cast<size_t>(chunk) * chunk_count_stride(r.experts) + e], count);
     }
 }
 
@@ -899,7 +903,8 @@ __global__ __launch_bounds__(kRouterThreads) void router_select_kernel(RouterArg
         else
         {
             const float sum = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? sequential_row_sums(shared.scores[wave], (r.experts + 15u) / 16u * 16u) : 1.0f;
-            route_token<SLOTS, true>(r, shared.scores[wave], sum, shared.scratch[wave], token, lane);
+            const float none[SLOTS] = {};
+            route_token<SLOTS, true>(r, shared.scores[wave], none, sum, shared.scratch[wave], nullptr, token, lane);
         }
     }
     // this workgroup's routes (written through), counts and error words (atomics) have landed once

@@ -62,6 +62,22 @@ def test_random_dispatch_matches_oracle(router, experts, top_k, score):
         assert status == 0
 
 
+@pytest.mark.parametrize("tokens", [257, 263, 264, 265, 511, 513, 2055])
+def test_last_workgroups_of_a_call_count_their_routes(router, tokens):
+    """Calls whose last workgroup holds one to eight tokens, with all routes at few experts and with a token that fails: the
+    counts of routes are added up by workgroup, and a call behind a failing one finds them at zero."""
+    rng = np.random.default_rng(tokens)
+    for experts, top_k in ((2, 1), (63, 5), (257, 9)):
+        logits = _logits(rng, tokens, experts, 1.0)
+        logits[:, experts - 1] += np.float32(50.0)
+        options = dict(score_function=hip_router.SOFTMAX, renormalize=True, routed_scaling_factor=1.0)
+        assert _compare(router, logits, top_k, "last workgroup, T=%d E=%d" % (tokens, experts), **options) == 0
+        failing = logits.copy()
+        failing[tokens - 1, 0] = np.inf
+        assert _compare(router, failing, top_k, "... which fails", **options) != 0
+        assert _compare(router, logits, top_k, "... and again", **options) == 0
+
+
 def test_ties_resolve_to_the_lower_expert_id(router):
     rng = np.random.default_rng(3)
     for experts, top_k in [(16, 4), (128, 8), (300, 17)]:
