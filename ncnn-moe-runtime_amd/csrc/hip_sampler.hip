@@ -13,6 +13,8 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -284,6 +286,43 @@ struct DistributionExport
     uint32_t* count = nullptr;
     uint32_t cap = 0;
 };
+
+// What kernels write into pinned host memory is seen there 3.5 us before hipStreamSynchronize returns (one launch and its outcome: 6.0
+// us, with the stream waited for 9.5).  So a synchronous call fills the records with words that no outcome holds, and waits until they are all
+// overwritten: each word by itself, so nothing depends on how a record arrives.  A kernel writes a row's record when all that the
+// row was made from has been read, so the logits and the operands may be overwritten when the call returns.  Whatever does not come in time
+// (a fault, a GPU that others hold) is waited for by hipStreamSynchronize, which reports errors.
+constexpr uint32_t kNoOutcome = 0xfffffffeu; // no token id or count; as a probability a NaN; its lowest byte is no row status
+constexpr int64_t kMostMicrosecondsWatched = 2000;
+
+void clear_outcome(void* records, size_t words)
+{
+    std::fill_n(static_cast<uint32_t*>(records), words, kNoOutcome);
+    std::atomic_thread_fence(std::memory_order_release);
+}
+
+// Whether all words have been overwritten before `deadline`.
+bool watch_outcome(const void* records, size_t words, std::chrono::steady_clock::time_point deadline)
+{
+    const volatile uint32_t* const word = static_cast<const volatile uint32_t*>(records);
+    for (size_t i = 0; i < words; ++i)
+    {
+        for (uint32_t looks = 0; word[i] == kNoOutcome; ++looks)
+        {
+            __builtin_ia32_pause();
+            if (looks % 64u == 63u && std::chrono::steady_clock::now() > deadline)
+                return false;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+}
+
+hipError_t wait_for_outcome(const void* records, size_t words, hipStream_t stream)
+{
+    const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched);
+    return watch_outcome(records, words, deadline) ? hipSuccess : hipStreamSynchronize(stream);
+}
 
 constexpr uint32_t kSideBySideRows = 32; // rows of each kind from which sample() runs the two later passes side by side
 
@@ -1117,12 +1156,17 @@ int ncnn_moe_hip_sampler_sample(
     // enough rows of each kind for the two passes to be worth the hand-over between two streams
     passes.side_by_side = wide_rows >= kSideBySideRows && full_order_rows >= kSideBySideRows;
     const bool full_order = passes.full_order;
+    // (one launch writes each record once; behind it, pending rows' records are written again)
+    const bool one_launch = !passes.full_order && !passes.wide_select;
+    const size_t result_words = static_cast<size_t>(rows) * sizeof(ncnn_moe_sample_result) / sizeof(uint32_t);
+    if (one_launch)
+        clear_outcome(s->results_host, result_words);
     int rc = launch_sampler(
         s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
         device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, passes, s->stream);
     if (rc != NCNN_MOE_SAMPLER_SUCCESS)
         return rc;
-    SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+    SAMPLER_HIP_CHECK(s, one_launch ? wait_for_outcome(s->results_host, result_words, s->stream) : hipStreamSynchronize(s->stream));
     if (!full_order)
     {
         // a row whose ties overflowed the select buffers is finished by the full-order kernels
@@ -1353,6 +1397,22 @@ int ncnn_moe_hip_sampler_speculative_verify(
     v.uniforms = s->verify_input_mapped->uniforms;
     v.accepted_probabilities = s->verify_output_mapped->accepted;
     v.result = &s->verify_output_mapped->result;
+    // The outcome, and behind it the probabilities of the tokens that it accepts.
+    const auto expect_outcome = [s]() { clear_outcome(s->verify_output_host, sizeof(*s->verify_output_host) / sizeof(uint32_t)); };
+    const auto await_outcome = [s, draft_count]() {
+        const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched);
+        const auto& out = *s->verify_output_host;
+        const bool seen = watch_outcome(&out.result, sizeof(out.result) / sizeof(uint32_t), deadline) &&
+            watch_outcome(out.accepted, std::min(out.result.accepted, draft_count), deadline);
+        return seen ? hipSuccess : hipStreamSynchronize(s->stream);
+    };
+    const auto take_outcome = [s, draft_count, accepted_probabilities, result]() {
+        *result = s->verify_output_host->result;
+        const uint32_t accepted = std::min(result->accepted, draft_count);
+        std::copy_n(s->verify_output_host->accepted, accepted, accepted_probabilities);
+        std::fill_n(accepted_probabilities + accepted, draft_count - accepted, 0.0f);
+        return NCNN_MOE_SAMPLER_SUCCESS;
+    };
     // the host sees the options: the later passes are enqueued only if the rows can need them; a row whose
     // ties overflow the select lists reports that, and the step is run again with the full-order kernels
     SamplerPasses passes;
@@ -1382,6 +1442,7 @@ int ncnn_moe_hip_sampler_speculative_verify(
         d.accepted_probabilities = v.accepted_probabilities;
         d.result = v.result;
         const uint32_t chunks = (s->logits_vocab + kResidualChunk - 1) / kResidualChunk;
+        expect_outcome();
         if (s->logits_dtype == NCNN_MOE_LOGITS_F32)
             hipLaunchKernelGGL((verify_residual_kernel<NCNN_MOE_LOGITS_F32>), dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
         else
@@ -1389,13 +1450,9 @@ int ncnn_moe_hip_sampler_speculative_verify(
         hipLaunchKernelGGL(verify_steps_kernel, dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
         hipLaunchKernelGGL(verify_draw_kernel, dim3(1), dim3(kResidualThreads), 0, s->stream, d, chunks);
         SAMPLER_HIP_CHECK(s, hipGetLastError());
-        SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+        SAMPLER_HIP_CHECK(s, await_outcome());
         if (s->verify_output_host->result.status != NCNN_MOE_VERIFY_UNSUPPORTED_WINDOW)
-        {
-            *result = s->verify_output_host->result;
-            std::memcpy(accepted_probabilities, s->verify_output_host->accepted, draft_count * sizeof(float));
-            return NCNN_MOE_SAMPLER_SUCCESS;
-        }
+            return take_outcome();
     }
     bool dense = s->verify_dense_known && std::memcmp(&s->verify_dense_options, &row_options, sizeof(row_options)) == 0;
     for (int attempt = 0; attempt < 2 && !dense; ++attempt)
@@ -1405,9 +1462,10 @@ int ncnn_moe_hip_sampler_speculative_verify(
             s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, export_to, passes, s->stream);
         if (rc != NCNN_MOE_SAMPLER_SUCCESS)
             return rc;
+        expect_outcome();
         hipLaunchKernelGGL(speculative_verify_kernel, dim3(1), dim3(kVerifyThreads), 0, s->stream, v);
         SAMPLER_HIP_CHECK(s, hipGetLastError());
-        SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+        SAMPLER_HIP_CHECK(s, await_outcome());
         const ncnn_moe_verify_result& outcome = s->verify_output_host->result;
         const bool row_pending = outcome.status == NCNN_MOE_VERIFY_ROW_ERROR && outcome.row_status == NCNN_MOE_ROW_NEEDS_FULL_ORDER;
         if (!row_pending || passes.full_order)
@@ -1445,13 +1503,12 @@ int ncnn_moe_hip_sampler_speculative_verify(
             s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, export_to, every_pass, s->stream);
         if (rc != NCNN_MOE_SAMPLER_SUCCESS)
             return rc;
+        expect_outcome();
         hipLaunchKernelGGL(speculative_verify_dense_kernel, dim3(1), dim3(kReplayThreads), 0, s->stream, d);
         SAMPLER_HIP_CHECK(s, hipGetLastError());
-        SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+        SAMPLER_HIP_CHECK(s, await_outcome());
     }
-    *result = s->verify_output_host->result;
-    std::memcpy(accepted_probabilities, s->verify_output_host->accepted, draft_count * sizeof(float));
-    return NCNN_MOE_SAMPLER_SUCCESS;
+    return take_outcome();
 }
 
 const char* ncnn_moe_hip_sampler_verify_status_message(int verify_status)
