@@ -470,8 +470,13 @@ hipError_t launch_unordered(ncnn_moe_hip_sampler* s, const SamplerArgs& a, const
     if (windows)
     {
         const WindowArgs w = window_args(s, a, listing, sums ? s->bin_list : nullptr);
-        launch_window_candidates<DTYPE>(w, stream);
-        launch_window_finish<DTYPE>(w, stream);
+        if (a.rows <= kChainRows) // (faster at every length, see window_chain_kernel; more rows than compute units would take turns)
+            hipLaunchKernelGGL(window_chain_kernel<DTYPE>, dim3(kChainGrid), dim3(kWalkThreads), 0, stream, w);
+        else
+        {
+            launch_window_candidates<DTYPE>(w, stream);
+            launch_window_finish<DTYPE>(w, stream);
+        }
     }
     return sums ? launch_bin_sums<DTYPE>(s, a, windows ? kRowsListed : listing, nullptr, windows, want_filters, nullptr, nullptr, stream) : hipSuccess;
 }
@@ -998,6 +1003,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     s->bins.list = s->bin_list;
     s->bins.most_looks = kMostLooks;
     s->windows.list = s->window_list;
+    s->windows.arrivals = s->bins.arrivals;
     CREATE_CHECK(hipMemsetAsync(s->device_memory, 0, cleared, s->stream));
     CREATE_CHECK(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(s->row_epoch), 1, rows, s->stream));
     s->input_uniforms_offset = rows * sizeof(ncnn_moe_sample_params);

@@ -82,3 +82,36 @@ def test_sums_over_the_edges_of_their_chunks(spread, rounded):
     with hip_sampler.HipSampler(rows, vocab) as sampler:
         sampler.upload_logits(logits)
         parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "chunk edges, spread %g" % spread)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,vocab", [(1, 131), (7, 2051), (3, 100003), (130, 33001), (130, 65537), (256, 4099), (257, 4099)])
+def test_windows_over_the_edges_of_parts(rows, vocab, dtype):
+    """Rows side by side in memory, so that they begin at every alignment: one part a row and sixteen, a part of one batch of loads and of
+    more, calls of one launch and of two; tokens and NaNs at the rows' ends, where a vector holds a neighbour's."""
+    import torch
+
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] edges of parts, %d x %d %s" % (rows, vocab, dtype), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+    logits[0::3, 0] = 9.0
+    logits[1::3, vocab - 1] = 9.5
+    logits[2::5, vocab - 1] = np.nan
+    logits[3::5, 0] = np.nan
+    logits[4::7, 1:-1] = np.sort(logits[4::7, 1:-1])
+    params = hip_sampler.make_params(rows, 0.9, 0, 0.97, 0.0)
+    params["top_k"] = rng.choice([65, 100, 300, 1000], rows)
+    params["min_p"][5::7] = np.float32(0.01)
+    uniforms = rng.random(rows, dtype=np.float32)
+    data = workloads.float32_to_bf16_bits(logits) if dtype == "bf16" else logits
+    cpu = parity_util.run_oracle(data, params, uniforms)
+    device = [torch.from_numpy(x).cuda() for x in (data.view(np.int16) if dtype == "bf16" else data, params.view(np.uint8), uniforms)]
+    results = torch.zeros(rows * 16, dtype=torch.uint8, device="cuda")
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        for _ in range(2):
+            sampler.sample_device(device[0].data_ptr(), hip_sampler.LOGITS_BF16 if dtype == "bf16" else hip_sampler.LOGITS_F32, rows, vocab, vocab,
+                                  device[1].data_ptr(), device[2].data_ptr(), None, results.data_ptr(), hip_sampler.PASSES_FULL_ORDER,
+                                  torch.cuda.current_stream().cuda_stream)
+            gpu = results.cpu().numpy().view(hip_sampler.RESULT_DTYPE)
+            parity_util.assert_results_match(gpu, cpu, dtype, "edges of parts")
+            results.zero_()
