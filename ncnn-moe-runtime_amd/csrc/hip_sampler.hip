@@ -1403,7 +1403,8 @@ int ncnn_moe_hip_sampler_speculative_verify(
     v.uniforms = s->verify_input_mapped->uniforms;
     v.accepted_probabilities = s->verify_output_mapped->accepted;
     v.result = &s->verify_output_mapped->result;
-    // The outcome, and behind it the probabilities of the tokens that it accepts.
+    // The outcome, and behind it the probabilities of the tokens that it accepts.  (Where verify_residual_kernel writes it, other workgroups may
+    // read a later call's operands: they leave nothing but the scratch that the later call's own launch writes behind them.)
     const auto expect_outcome = [s]() { clear_outcome(s->verify_output_host, sizeof(*s->verify_output_host) / sizeof(uint32_t)); };
     const auto await_outcome = [s, draft_count]() {
         const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched);

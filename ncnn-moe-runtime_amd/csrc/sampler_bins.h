@@ -205,7 +205,7 @@ __device__ __forceinline__ ncnn_moe_sample_params params_of(const uint32_t (&opt
     return p;
 }
 
-// The rows that the first select leaves, those with a window of the window kernels' widths apart from the others.
+// The rows that the first select left when it ended, those with a window of the window kernels' widths apart from the others.
 enum RowListing : uint32_t
 {
     kRowsListed = 0,    // a launch of its own has listed them
@@ -213,6 +213,8 @@ enum RowListing : uint32_t
     kRowsByOptions = 2  // ... runs beside: the rows whose options say so
 };
 
+// (Those that this launch has finished since are still among them: a launch that lists its rows in place may finish some before its
+// last workgroups start, where other launches hold their places, and these have to come to the same list.)
 __device__ __forceinline__ bool row_is_left(const SamplerArgs& a, uint32_t row, bool by_options, bool windows_apart, bool& window)
 {
     uint32_t effective_k = 0;
@@ -231,7 +233,7 @@ __device__ __forceinline__ bool row_is_left(const SamplerArgs& a, uint32_t row, 
     __builtin_memcpy(&p, words, sizeof(p));
     const int mode = resolve_row_mode(p, a.vocab, static_cast<uint32_t>(kFastTopK), a.force_general, effective_k, status);
     window = windows_apart && effective_k <= static_cast<uint32_t>(kSelectTopK);
-    return by_options ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && state == kRowNeedsGeneral;
+    return by_options ? mode == kModeGeneral : (mode == kModeGeneral || mode == kModeTopK) && state != kRowDone;
 }
 
 // A call of no more rows than a workgroup has threads needs no launch that lists them: every workgroup of the first launch that
@@ -2280,7 +2282,7 @@ __device__ __forceinline__ void end_early(const BinArgs& g, uint32_t part, uint3
     if (state == kBinRowRejected && part == 0u && tid == 0)
     {
         write_error(g.a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags_of_row(g, p, saw_nan));
-        g.a.row_state[row] = kRowDone;
+        g.a.row_state[row] = kRowDoneLater;
     }
 }
 
@@ -2812,7 +2814,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
                     {
                         const ncnn_moe_sample_params p = params_of(carried.options);
                         write_token(a, row, p, token, kept == 1u ? 1.0f : (term / normalizer) / renormalizer, kept, kept == 1u ? 0 : 1, result_flags(p));
-                        a.row_state[row] = kRowDone;
+                        a.row_state[row] = kRowDoneLater;
                         record.served = 1u;
                     }
                 }

@@ -165,7 +165,8 @@ enum RowMode : int
 enum RowState : uint32_t
 {
     kRowDone = 0,
-    kRowNeedsGeneral = 1
+    kRowNeedsGeneral = 1,
+    kRowDoneLater = 2 // left pending by the first select and finished by the window kernels or the binned sums: see row_is_left
 };
 
 // Bits accumulated per row while its segments are scanned.

@@ -388,7 +388,7 @@ __device__ __forceinline__ void window_finish(
         if (tid == 0)
         {
             write_error(a, row, NCNN_MOE_ROW_NO_FINITE_LOGIT, flags);
-            a.row_state[row] = kRowDone;
+            a.row_state[row] = kRowDoneLater;
         }
     };
     if (count == 0u)
@@ -588,7 +588,7 @@ __device__ __forceinline__ void window_finish(
     {
         const float probability = kept == 1u ? 1.0f : (shared.terms[selected] / normalizer) / renormalizer;
         write_token(a, row, p, static_cast<int32_t>(shared.tokens[selected]), probability, kept, kept == 1u ? 0 : 1, flags);
-        a.row_state[row] = kRowDone;
+        a.row_state[row] = kRowDoneLater;
     }
 }
 

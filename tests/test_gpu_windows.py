@@ -115,3 +115,34 @@ def test_windows_over_the_edges_of_parts(rows, vocab, dtype):
             gpu = results.cpu().numpy().view(hip_sampler.RESULT_DTYPE)
             parity_util.assert_results_match(gpu, cpu, dtype, "edges of parts")
             results.zero_()
+
+
+@pytest.mark.parametrize("rows,vocab,top_ks", [(200, 8191, [300, 1000]), (96, 16411, [0, 300]), (40, 20011, [0])])
+def test_calls_that_hold_each_other_s_places(rows, vocab, top_ks):
+    """Three handles on three streams: workgroups of one call start when others of it have finished their rows, the soonest those
+    that have no finite logit, and come to the same list of rows all the same."""
+    import torch
+
+    print("[case] three streams, %d x %d, top_k %s" % (rows, vocab, top_ks), flush=True)
+    calls = []
+    for seed in range(3):
+        rng = np.random.default_rng(rows + seed)
+        logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+        logits[seed::7] = -np.inf
+        params = hip_sampler.make_params(rows, 0.9, 0, 0.95, 0.0)
+        params["top_k"] = rng.choice(top_ks, rows)
+        uniforms = rng.random(rows, dtype=np.float32)
+        device = [torch.from_numpy(x).cuda() for x in (logits, params.view(np.uint8), uniforms)]
+        results = torch.zeros(8, rows * 16, dtype=torch.uint8, device="cuda")
+        calls.append((hip_sampler.HipSampler(rows, vocab), torch.cuda.Stream(), device, results, parity_util.run_oracle(logits, params, uniforms)))
+    torch.cuda.synchronize()
+    for i in range(8):
+        for sampler, stream, device, results, _ in calls:
+            sampler.sample_device(device[0].data_ptr(), hip_sampler.LOGITS_F32, rows, vocab, vocab, device[1].data_ptr(), device[2].data_ptr(), None,
+                                  results[i].data_ptr(), hip_sampler.PASSES_FULL_ORDER, stream.cuda_stream)
+    torch.cuda.synchronize()
+    for sampler, _, _, results, cpu in calls:
+        for i in range(8):
+            gpu = results[i].cpu().numpy().view(hip_sampler.RESULT_DTYPE)
+            parity_util.assert_results_match(gpu, cpu, "f32", "call %d beside others" % i)
+        sampler.close()
