@@ -2,6 +2,7 @@
 results, from the window kernels and not from the sort."""
 import numpy as np
 import pytest
+import torch  # in front of the sampler's library: both then share the HIP runtime that torch brings along
 
 import parity_util
 from ncnn_moe_runtime_amd import hip_sampler, workloads
@@ -89,8 +90,6 @@ def test_sums_over_the_edges_of_their_chunks(spread, rounded):
 def test_windows_over_the_edges_of_parts(rows, vocab, dtype):
     """Rows side by side in memory, so that they begin at every alignment: one part a row and sixteen, a part of one batch of loads and of
     more, calls of one launch and of two; tokens and NaNs at the rows' ends, where a vector holds a neighbour's."""
-    import torch
-
     rng = np.random.default_rng(rows + vocab)
     print("[case] edges of parts, %d x %d %s" % (rows, vocab, dtype), flush=True)
     logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
@@ -121,8 +120,6 @@ def test_windows_over_the_edges_of_parts(rows, vocab, dtype):
 def test_calls_that_hold_each_other_s_places(rows, vocab, top_ks):
     """Three handles on three streams: workgroups of one call start when others of it have finished their rows, the soonest those
     that have no finite logit, and come to the same list of rows all the same."""
-    import torch
-
     print("[case] three streams, %d x %d, top_k %s" % (rows, vocab, top_ks), flush=True)
     calls = []
     for seed in range(3):
