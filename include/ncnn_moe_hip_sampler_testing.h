@@ -36,6 +36,9 @@ int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32
 /* most_looks: how often a part of a row looks for the row's other parts before it gives the row up, which is then sorted (0:
  * a part that has to wait gives up at once).  Same results either way. */
 int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* sampler, uint32_t looks);
+/* 1 if ncnn_moe_hip_sampler_sample watches for its records in pinned memory with these options, 0 if it waits for the stream.
+ * No GPU needed. */
+int ncnn_moe_hip_sampler_debug_outcome_watched(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab);
 /* Which of the handle's first `rows` rows the binned sums left the filtered distribution of in the last verification step. */
 int ncnn_moe_hip_sampler_debug_filtered_rows(ncnn_moe_hip_sampler* sampler, uint32_t* filtered, uint32_t rows);
 /* spread_sort (on by default): the radix sort of a long full-order row runs on several workgroups; off,

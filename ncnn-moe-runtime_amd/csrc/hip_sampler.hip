@@ -289,9 +289,10 @@ struct DistributionExport
 
 // What kernels write into pinned host memory is seen there 3.5 us before hipStreamSynchronize returns (one launch and its outcome: 6.0
 // us, with the stream waited for 9.5).  So a synchronous call fills the records with words that no outcome holds, and waits until they are all
-// overwritten: each word by itself, so nothing depends on how a record arrives.  A kernel writes a row's record when all that the
-// row was made from has been read, so the logits and the operands may be overwritten when the call returns.  Whatever does not come in time
-// (a fault, a GPU that others hold) is waited for by hipStreamSynchronize, which reports errors.
+// overwritten: each word by itself, so nothing depends on how a record arrives.  A kernel writes the record of a row with valid options when
+// all that the row was made from has been read, so the logits and the operands may be overwritten when the call returns.  (A rejected row's is
+// written by the first of its workgroups to read the options, and the others read them when they start: see outcome_tells_all.)  Whatever
+// does not come in time (a fault, a GPU that others hold) is waited for by hipStreamSynchronize, which reports errors.
 constexpr uint32_t kNoOutcome = 0xfffffffeu; // no token id or count; as a probability a NaN; its lowest byte is no row status
 constexpr int64_t kMostMicrosecondsWatched = 2000;
 
@@ -754,6 +755,36 @@ bool row_left_pending(const ncnn_moe_sample_params& p, uint32_t vocab, uint32_t 
     return resolve_row_mode(p, vocab, max_top_k, 0, effective_k, status) == kModeGeneral;
 }
 
+// Whether the records of a sample() that enqueues `passes` tell when all of its launches have read their operands.  Not behind one
+// launch: pending rows' records are written again.  Nor with a row whose options are rejected: a workgroup of that row that starts late, when
+// the next call's options lie where it reads its own, would serve the row and count itself among that call's workgroups.
+bool outcome_tells_all(const SamplerPasses& passes, const ncnn_moe_sample_params* params, uint32_t rows)
+{
+    return !passes.full_order && !passes.wide_select &&
+        std::all_of(params, params + rows, [](const ncnn_moe_sample_params& p) { return validate_params(p) == NCNN_MOE_ROW_OK; });
+}
+
+// The passes that a batch needs: the host sees the options, so the later ones are enqueued only if some row needs them.
+SamplerPasses passes_of(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab, bool force_general)
+{
+    SamplerPasses passes;
+    passes.full_order = force_general;
+    uint32_t wide_rows = 0;
+    uint32_t full_order_rows = 0;
+    for (uint32_t row = 0; row < rows; ++row)
+    {
+        const bool beyond_select = row_left_pending(params[row], vocab, kSelectTopK);
+        const bool beyond_fast = !beyond_select && row_left_pending(params[row], vocab, kFastTopK);
+        passes.wide_select = passes.wide_select || beyond_fast;
+        passes.full_order = passes.full_order || beyond_select;
+        wide_rows += beyond_fast ? 1u : 0u;
+        full_order_rows += beyond_select ? 1u : 0u;
+    }
+    // enough rows of each kind for the two passes to be worth the hand-over between two streams
+    passes.side_by_side = wide_rows >= kSideBySideRows && full_order_rows >= kSideBySideRows;
+    return passes;
+}
+
 int check_shape(ncnn_moe_hip_sampler* s, int dtype, uint32_t rows, uint32_t vocab)
 {
     if (dtype != NCNN_MOE_LOGITS_F32 && dtype != NCNN_MOE_LOGITS_BF16)
@@ -1145,34 +1176,18 @@ int ncnn_moe_hip_sampler_sample(
     }
     else if (stop_id_count > 0)
         return fail(s, NCNN_MOE_SAMPLER_INVALID_ARGUMENT, "more stop ids than the handle holds (max(64 * max_rows, max_vocab))");
-    // the host sees the options: the later passes are enqueued only if some row needs them
-    SamplerPasses passes;
-    passes.full_order = s->force_general != 0;
-    uint32_t wide_rows = 0;
-    uint32_t full_order_rows = 0;
-    for (uint32_t row = 0; row < rows; ++row)
-    {
-        const bool beyond_select = row_left_pending(params[row], s->logits_vocab, kSelectTopK);
-        const bool beyond_fast = !beyond_select && row_left_pending(params[row], s->logits_vocab, kFastTopK);
-        passes.wide_select = passes.wide_select || beyond_fast;
-        passes.full_order = passes.full_order || beyond_select;
-        wide_rows += beyond_fast ? 1u : 0u;
-        full_order_rows += beyond_select ? 1u : 0u;
-    }
-    // enough rows of each kind for the two passes to be worth the hand-over between two streams
-    passes.side_by_side = wide_rows >= kSideBySideRows && full_order_rows >= kSideBySideRows;
+    const SamplerPasses passes = passes_of(params, rows, s->logits_vocab, s->force_general != 0);
     const bool full_order = passes.full_order;
-    // (one launch writes each record once; behind it, pending rows' records are written again)
-    const bool one_launch = !passes.full_order && !passes.wide_select;
+    const bool watched = outcome_tells_all(passes, params, rows);
     const size_t result_words = static_cast<size_t>(rows) * sizeof(ncnn_moe_sample_result) / sizeof(uint32_t);
-    if (one_launch)
+    if (watched)
         clear_outcome(s->results_host, result_words);
     int rc = launch_sampler(
         s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
         device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, passes, s->stream);
     if (rc != NCNN_MOE_SAMPLER_SUCCESS)
         return rc;
-    SAMPLER_HIP_CHECK(s, one_launch ? wait_for_outcome(s->results_host, result_words, s->stream) : hipStreamSynchronize(s->stream));
+    SAMPLER_HIP_CHECK(s, watched ? wait_for_outcome(s->results_host, result_words, s->stream) : hipStreamSynchronize(s->stream));
     if (!full_order)
     {
         // a row whose ties overflowed the select buffers is finished by the full-order kernels
@@ -1577,6 +1592,14 @@ int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* s, uint32_t look
         return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
     s->bins.most_looks = looks;
     return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+// Whether sample() watches for its records with these options (else it waits for the stream).
+int ncnn_moe_hip_sampler_debug_outcome_watched(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab)
+{
+    if (params == nullptr || rows == 0 || vocab == 0)
+        return 0;
+    return outcome_tells_all(passes_of(params, rows, vocab, false), params, rows) ? 1 : 0;
 }
 
 // Which of the handle's first `rows` rows the binned sums finished the last time that they were given them.

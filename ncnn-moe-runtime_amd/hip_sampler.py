@@ -73,6 +73,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_scatter_segments",
     "ncnn_moe_hip_sampler_debug_binned_sums",
     "ncnn_moe_hip_sampler_debug_most_looks",
+    "ncnn_moe_hip_sampler_debug_outcome_watched",
     "ncnn_moe_hip_sampler_debug_binned_rows",
     "ncnn_moe_hip_sampler_debug_filtered_rows",
     "ncnn_moe_hip_sampler_debug_spread_sort",
@@ -129,6 +130,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_most_looks.argtypes = [vp, ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_outcome_watched.argtypes = [vp, ctypes.c_uint32, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_filtered_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_spread_sort.argtypes = [vp, ctypes.c_int]
@@ -198,6 +200,12 @@ def select_geometry(dtype, rows, vocab):
     if rc != RC_SUCCESS:
         raise SamplerError("select_geometry: rc=%d" % rc)
     return segments.value, chunks.value, variant.value
+
+
+def outcome_watched(params, vocab):
+    """Test hook: whether sample() watches for its records with these options (else it waits for the stream)."""
+    params = np.ascontiguousarray(params, dtype=PARAMS_DTYPE)
+    return load_testing_library().ncnn_moe_hip_sampler_debug_outcome_watched(params.ctypes.data, len(params), vocab) == 1
 
 
 def exp2_table():

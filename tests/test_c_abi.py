@@ -5,6 +5,7 @@ import os
 import re
 import subprocess
 
+import numpy as np
 import pytest
 
 from ncnn_moe_runtime_amd import hip_router, hip_sampler
@@ -62,6 +63,28 @@ def test_select_geometry_of_the_benchmark_shapes():
             assert variant == hip_sampler.GEOMETRY_SPLIT_LOOPED and chunks > 1 and 1 < segments <= 16
         segments, chunks, variant = hip_sampler.select_geometry(f32, rows, 340000)
         assert variant == hip_sampler.GEOMETRY_SPLIT_LOOPED and chunks > 1 and 1 < segments <= 16
+
+
+@pytest.mark.parametrize("field,value", [("temperature", -1.0), ("temperature", np.nan), ("top_p", 0.0), ("top_p", 1.5), ("min_p", -0.1), ("min_p", 1.5)])
+def test_calls_with_a_rejected_row_wait_for_the_stream(field, value):
+    """A rejected row's record comes before all of its workgroups have read the options: a call that returned with it could be
+    followed by one whose options those workgroups read."""
+    for rows in (1, 7):
+        params = hip_sampler.make_params(rows, 0.8, 20, 0.9, 0.0)
+        params["temperature"][0] = 0.0
+        assert hip_sampler.outcome_watched(params, 151936)
+        params[field][rows - 1] = value
+        assert not hip_sampler.outcome_watched(params, 151936)
+
+
+@pytest.mark.parametrize("top_k", [0, 65, 1024, 1025])
+def test_calls_of_several_launches_wait_for_the_stream(top_k):
+    params = hip_sampler.make_params(3, 0.8, 20, 0.9, 0.0)
+    params["top_k"][1] = top_k
+    assert not hip_sampler.outcome_watched(params, 151936)
+    assert hip_sampler.outcome_watched(params, 64)
+    params["temperature"][1] = 0.0
+    assert hip_sampler.outcome_watched(params, 151936)
 
 
 def test_router_header_and_binding_agree():

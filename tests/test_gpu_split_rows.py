@@ -137,6 +137,23 @@ def test_many_launches_on_one_handle():
         sampler.scatter_segments(False)
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 151936), (9, 262144), (300, 8192)])
+def test_rejected_calls_and_valid_ones_in_turn(rows, vocab):
+    """Calls with rejected rows, each followed at once by one with valid options on the same logits: the options that the first one's
+    workgroups read are not overwritten while any of them has still to start."""
+    print("[case] rejected and valid calls in turn, %d x %d" % (rows, vocab), flush=True)
+    logits, valid, uniforms = _batch(rows + vocab, rows, vocab)
+    rejected = valid.copy()
+    rejected["top_p"][::2] = 1.5
+    rejected["temperature"][1::3] = np.nan
+    cpu = [parity_util.run_oracle(logits, params, uniforms) for params in (rejected, valid)]
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        sampler.upload_logits(logits)
+        for turn in range(40):
+            for params, expected in zip((rejected, valid), cpu):
+                parity_util.assert_results_match(sampler.sample(params, uniforms), expected, "f32", "turn %d" % turn)
+
+
 def test_launch_numbers_start_over():
     """The per-row launch numbers (epochs) that tag the hand-over records run 1 .. 8191 and start over; a
     serving loop gets there within minutes.  A handle that has records of its first launches in place is
