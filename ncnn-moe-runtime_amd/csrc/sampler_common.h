@@ -5,6 +5,8 @@
 
 #include "sampler_device.h"
 
+#include <stddef.h>
+
 namespace ncnn_moe_hip {
 
 struct SamplerArgs
@@ -129,17 +131,24 @@ __device__ __forceinline__ uint8_t stop_flag(const SamplerArgs& a, const ncnn_mo
     return 0;
 }
 
+// A row's record, by one store of whole words: a host that watches for a record in pinned memory takes a word that has changed for
+// complete, which a store of its four bytes each by itself would not make it.
+__device__ __forceinline__ void store_record(
+    const SamplerArgs& a, uint32_t row, int32_t token, float probability, uint32_t kept, uint32_t status, uint32_t is_stop, uint32_t draw_consumed, uint32_t flags)
+{
+    typedef uint32_t Record __attribute__((ext_vector_type(4), aligned(4), may_alias));
+    static_assert(sizeof(Record) == sizeof(ncnn_moe_sample_result) && offsetof(ncnn_moe_sample_result, probability) == 4 &&
+                      offsetof(ncnn_moe_sample_result, kept_count) == 8 && offsetof(ncnn_moe_sample_result, status) == 12 &&
+                      offsetof(ncnn_moe_sample_result, is_stop) == 13 && offsetof(ncnn_moe_sample_result, draw_consumed) == 14 &&
+                      offsetof(ncnn_moe_sample_result, flags) == 15,
+                  "the record's fields lie in these words");
+    *reinterpret_cast<Record*>(a.results + row) =
+        Record{static_cast<uint32_t>(token), __float_as_uint(probability), kept, status | is_stop << 8 | draw_consumed << 16 | flags << 24};
+}
+
 __device__ __forceinline__ void write_error(const SamplerArgs& a, uint32_t row, int status, uint8_t flags)
 {
-    ncnn_moe_sample_result r;
-    r.token_id = -1;
-    r.probability = 0.0f;
-    r.kept_count = 0;
-    r.status = static_cast<uint8_t>(status);
-    r.is_stop = 0;
-    r.draw_consumed = 0;
-    r.flags = flags;
-    a.results[row] = r;
+    store_record(a, row, -1, 0.0f, 0u, static_cast<uint32_t>(status), 0u, 0u, flags);
     if (a.distribution_count != nullptr)
         a.distribution_count[row] = 0;
 }
@@ -147,30 +156,14 @@ __device__ __forceinline__ void write_error(const SamplerArgs& a, uint32_t row, 
 // Marks a row that still has to go through the full-order kernels.
 __device__ __forceinline__ void write_pending(const SamplerArgs& a, uint32_t row)
 {
-    ncnn_moe_sample_result r;
-    r.token_id = -1;
-    r.probability = 0.0f;
-    r.kept_count = 0;
-    r.status = NCNN_MOE_ROW_NEEDS_FULL_ORDER;
-    r.is_stop = 0;
-    r.draw_consumed = 0;
-    r.flags = 0;
-    a.results[row] = r;
+    store_record(a, row, -1, 0.0f, 0u, NCNN_MOE_ROW_NEEDS_FULL_ORDER, 0u, 0u, 0u);
 }
 
 __device__ __forceinline__ void write_token(
     const SamplerArgs& a, uint32_t row, const ncnn_moe_sample_params& p,
     int32_t token, float probability, uint32_t kept, uint8_t draw_consumed, uint8_t flags)
 {
-    ncnn_moe_sample_result r;
-    r.token_id = token;
-    r.probability = probability;
-    r.kept_count = kept;
-    r.status = NCNN_MOE_ROW_OK;
-    r.is_stop = stop_flag(a, p, token);
-    r.draw_consumed = draw_consumed;
-    r.flags = flags;
-    a.results[row] = r;
+    store_record(a, row, token, probability, kept, NCNN_MOE_ROW_OK, stop_flag(a, p, token), draw_consumed, flags);
 }
 
 // The CPU sampler from the sorted Top-K window onwards (src/engine/session.cpp:89-134, :429-442),
