@@ -36,6 +36,12 @@ int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32
 /* most_looks: how often a part of a row looks for the row's other parts before it gives the row up, which is then sorted (0:
  * a part that has to wait gives up at once).  Same results either way. */
 int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* sampler, uint32_t looks);
+/* compute_units: the handle's rows are cut into no more parts than a device of so many compute units would have them in (refused where
+ * that is more than the handle has).  Same results either way.  most_parts is that number of parts, first_looks how often a part
+ * looks at the row's first meeting; no GPU needed for these two. */
+int ncnn_moe_hip_sampler_debug_compute_units(ncnn_moe_hip_sampler* sampler, uint32_t compute_units);
+uint32_t ncnn_moe_hip_sampler_debug_most_parts(uint32_t compute_units);
+uint32_t ncnn_moe_hip_sampler_debug_first_looks(uint32_t rows, uint32_t vocab, int dtype, int side_by_side);
 /* 1 if ncnn_moe_hip_sampler_sample watches for its records in pinned memory with these options, 0 if it waits for the stream.
  * No GPU needed. */
 int ncnn_moe_hip_sampler_debug_outcome_watched(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab);

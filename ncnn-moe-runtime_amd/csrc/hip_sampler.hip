@@ -361,10 +361,12 @@ WindowArgs window_args(const ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowL
     return w;
 }
 
+constexpr uint32_t kLooksByLength = 0xffffffffu; // most_looks of a handle that no test has set it for
+
 // Whether the binned sums are one launch (see kChainPartElements).
-bool goes_as_chain(uint32_t rows, uint32_t vocab, bool windows)
+bool goes_as_chain(uint32_t rows, uint32_t vocab, uint32_t most_parts, bool windows)
 {
-    const uint32_t parts = std::max(1u, std::min(kMaxBinParts, kChainGrid / 8u / ((rows + 7u) / 8u)));
+    const uint32_t parts = std::max(1u, std::min(most_parts, kChainGrid / 8u / ((rows + 7u) / 8u)));
     return rows <= kChainRows && vocab / parts <= (windows ? kChainPartElementsWithWindows : kChainPartElements);
 }
 
@@ -380,6 +382,8 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
     g.want_filters = want_filters ? 1u : 0u;
     g.listing = listing;
     g.window_list = window_list;
+    if (g.most_looks == kLooksByLength)
+        g.most_looks = most_looks_of(a.rows, a.vocab, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u, behind_sum != nullptr);
     hipError_t result = hipSuccess;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (behind_terms != nullptr || behind_sum != nullptr)
@@ -396,7 +400,7 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
                 result = hipEventRecord(behind, stream);
         }
     };
-    if (behind_sum == nullptr && goes_as_chain(a.rows, a.vocab, windows))
+    if (behind_sum == nullptr && goes_as_chain(a.rows, a.vocab, g.most_parts, windows))
     {
         hipLaunchKernelGGL(bin_chain_kernel<DTYPE>, dim3(kChainGrid), dim3(kWalkThreads), 0, stream, g);
         return result;
@@ -1028,11 +1032,14 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->window_list, (rows + 1) * sizeof(uint32_t));
     place(&s->windows.keys, rows * kWindowListCap * sizeof(uint32_t));
     place(&s->windows.tokens, rows * kWindowListCap * sizeof(uint32_t));
+    int compute_units = 0;
+    CREATE_CHECK(hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, device));
     CREATE_CHECK(hipMalloc(&s->device_memory, bytes));
     for (const auto& [pointer, offset] : buffers)
         *pointer = static_cast<uint8_t*>(s->device_memory) + offset;
     s->bins.list = s->bin_list;
-    s->bins.most_looks = kMostLooks;
+    s->bins.most_looks = kLooksByLength;
+    s->bins.most_parts = most_parts_of(static_cast<uint32_t>(std::max(0, compute_units)));
     s->windows.list = s->window_list;
     s->windows.arrivals = s->bins.arrivals;
     CREATE_CHECK(hipMemsetAsync(s->device_memory, 0, cleared, s->stream));
@@ -1592,6 +1599,25 @@ int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* s, uint32_t look
         return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
     s->bins.most_looks = looks;
     return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+// Parts of a row at most, as on a device of `compute_units` (1 .. the device's own).
+int ncnn_moe_hip_sampler_debug_compute_units(ncnn_moe_hip_sampler* s, uint32_t compute_units)
+{
+    if (s == nullptr || most_parts_of(compute_units) > s->bins.most_parts)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    s->bins.most_parts = most_parts_of(compute_units);
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+uint32_t ncnn_moe_hip_sampler_debug_most_parts(uint32_t compute_units)
+{
+    return most_parts_of(compute_units);
+}
+
+uint32_t ncnn_moe_hip_sampler_debug_first_looks(uint32_t rows, uint32_t vocab, int dtype, int side_by_side)
+{
+    return most_looks_of(rows, vocab, dtype == NCNN_MOE_LOGITS_F32 ? 4u : 2u, side_by_side != 0);
 }
 
 // Whether sample() watches for its records with these options (else it waits for the stream).

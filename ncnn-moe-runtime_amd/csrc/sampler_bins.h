@@ -166,7 +166,8 @@ struct BinArgs
     uint32_t* head_tokens; // [rows][kBinListCap], sorted
     BinRow* records;       // [rows]
     unsigned long long* arrivals; // [rows][kArrivalWords], zero between launches: see parts_meet
-    uint32_t most_looks;   // ... kMostLooks
+    uint32_t most_looks;   // ... at the first meeting, see most_looks_of
+    uint32_t most_parts;   // of a row: see most_parts_of
     uint32_t want_filters;
     uint32_t windows_are_selects; // rows with a window of the wide select's widths do not count as full-order rows
     uint32_t listing;      // RowListing: how the first launch finds its rows
@@ -316,13 +317,13 @@ struct BinGrid
     uint32_t rows, parts, first_slot, slot_step, part;
 };
 
-__device__ __forceinline__ BinGrid bin_grid(uint32_t rows, uint32_t vocab, uint32_t workgroups = kBinGrid)
+__device__ __forceinline__ BinGrid bin_grid(uint32_t rows, uint32_t vocab, uint32_t most_parts = kMaxBinParts, uint32_t workgroups = kBinGrid)
 {
     BinGrid r;
     r.rows = rows;
     const uint32_t per_xcd = workgroups / 8u;
     const uint32_t slots_per_xcd = max(1u, (r.rows + 7u) / 8u);
-    const uint32_t most = min(kMaxBinParts, (vocab + kBinPartElements - 1u) / kBinPartElements);
+    const uint32_t most = min(most_parts, (vocab + kBinPartElements - 1u) / kBinPartElements);
     r.parts = max(1u, min(most, per_xcd / slots_per_xcd));
     const uint32_t lanes = per_xcd / r.parts; // slots in flight on an XCD
     const uint32_t within = blockIdx.x >> 3;
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
     const SamplerArgs& a = g.a;
     const int tid = threadIdx.x;
     const uint32_t rows = list_rows_in_place(a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
-    const BinGrid grid = bin_grid(rows, a.vocab);
+    const BinGrid grid = bin_grid(rows, a.vocab, g.most_parts);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
         const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));
@@ -639,7 +640,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_terms_kernel(BinArgs g)
     __shared__ __align__(16) uint32_t bins[2 * kBins];
     __shared__ uint4 part_stats[kMaxBinParts];
     __shared__ uint64_t exp2_table[32];
-    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab, g.most_parts);
     const int tid = threadIdx.x;
     if (tid < 32)
         exp2_table[tid] = kExp2Table[tid];
@@ -1224,7 +1225,7 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_sum_kernel(BinArgs g, uint
     __shared__ BinSumShared shared;
     __shared__ BinWalkRow carried;
     const SamplerArgs& a = g.a;
-    const BinGrid grid = bin_grid(g.list[0], a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], a.vocab, g.most_parts);
     const int tid = threadIdx.x;
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
@@ -2922,19 +2923,41 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
 // The parts of a row meet: what each has handed over before is there for all behind it.  False: given up, because a part did not come.
 // Every thread calls it; `meeting` counts from 1, `wait`: whether the caller takes anything over.
 //
-// All parts of a row are workgroups of one launch that follow each other on an XCD (bin_grid), so the wait ends: workgroups start in
-// order, no part waits before it has come itself, and the parts that are missing start at the latest where a row whose parts
-// have all started is finished.  Workgroups of other launches may hold the places for a while; a part that has looked kMostLooks times
-// (some 20 ms) gives up for the whole row, which is then left to the full-order kernels, as are the rows of a GPU on which
-// fewer workgroups run at a time than a row has parts.
+// A row's P parts are every eighth of 8 P workgroups that follow each other (bin_grid), and a workgroup has parts of one row only where rows
+// have several.  Workgroups start in order, and a part comes before it waits, so the wait ends on a device that holds 8 P workgroups at a time:
+// most_parts_of sees to that.  Workgroups of other launches may hold the places, for a while, or, where they wait for parts of their own rows
+// that find no place either, for good: three calls of 8 rows that share a device can each hold 10 of a row's 16 places.  So a part that has
+// looked most_looks times at the first meeting gives the row up, which is then left to the full-order kernels.  Behind the first meeting all
+// parts have started, and are waited for kLaterLooks times as long.
 //
 // arrivals[0] counts the parts that have come to the row's meetings and, above, how many came to the first from each XCD: from then on
 // shared.near tells whether all are on one.  arrivals[1] counts those that are done with the row: the last of them returns both to zero.
-constexpr uint32_t kMostLooks = 40000;
+constexpr uint32_t kLaterLooks = 16;
 constexpr unsigned long long kArrivalsOnly = 0xffffull;
 constexpr unsigned long long kRowGivenUp = 1ull << 63;
 constexpr uint32_t kXcdShift = 16, kXcdBits = 5;
 static_assert(kMaxBinParts < 1u << kXcdBits, "the parts that come from one XCD are counted in kXcdBits");
+
+// How often a part looks at the first meeting, half a microsecond a look: about as long as sorting the row takes instead (8 rows of 310,000
+// without a bin that serves them 0.5 ms, 1 of 1,000,000 5.5 ms, of 4,000,000 21 ms), so that waiting in vain costs no more than giving up too
+// early.  Side by side the call's own select and window kernels hold places while they stream: a look for each MB, 2 TB/s.
+constexpr uint32_t kFewestLooks = 1000;
+constexpr uint32_t kLogitsALook = 100;
+
+inline uint32_t most_looks_of(uint32_t rows, uint32_t vocab, uint32_t element_bytes, bool side_by_side)
+{
+    const uint64_t beside = side_by_side ? static_cast<uint64_t>(rows) * vocab * element_bytes >> 20 : 0u;
+    const uint64_t looks = (vocab / kLogitsALook > kFewestLooks ? vocab / kLogitsALook : kFewestLooks) + beside;
+    return static_cast<uint32_t>(looks < 0xffffffffu / kLaterLooks ? looks : 0xffffffffu / kLaterLooks);
+}
+
+// The parts of a row whose 8 P workgroups a device of `compute_units` holds at a time, one to a compute unit at least: 16 from half a
+// card on, 8 and 4 on partitions of two XCDs and of one, where a row of 16 parts would wait for workgroups that cannot start.
+inline uint32_t most_parts_of(uint32_t compute_units)
+{
+    const uint32_t parts = compute_units / 8u;
+    return parts < 1u ? 1u : parts < kMaxBinParts ? parts : kMaxBinParts;
+}
 
 __device__ __forceinline__ uint32_t own_xcd()
 {
@@ -2958,10 +2981,11 @@ __device__ __forceinline__ bool parts_meet(unsigned long long* arrivals, uint32_
         const unsigned long long one = meeting == 1u ? 1ull + own_place : 1ull;
         unsigned long long seen = __hip_atomic_fetch_add(arrivals, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + one;
         const uint32_t goal = meeting * parts;
+        const uint32_t most = meeting == 1u ? most_looks : most_looks * kLaterLooks;
         const auto come = [&]() { return static_cast<uint32_t>(seen & kArrivalsOnly) >= goal; };
         for (uint32_t looks = 0; wait && !come() && (seen & kRowGivenUp) == 0ull; ++looks)
         {
-            if (looks == most_looks)
+            if (looks == most)
             {
                 __hip_atomic_fetch_or(arrivals, kRowGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
@@ -3015,7 +3039,7 @@ template <int DTYPE>
 __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void bin_walks_kernel(BinArgs g)
 {
     __shared__ BinWalkShared shared;
-    const BinGrid grid = bin_grid(g.list[0], g.a.vocab);
+    const BinGrid grid = bin_grid(g.list[0], g.a.vocab, g.most_parts);
     const int tid = threadIdx.x;
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
@@ -3064,7 +3088,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2,
     if (tid < 32)
         exp2_table[tid] = kExp2Table[tid];
     const uint32_t rows = list_rows_in_place<kWalkWaves>(g.a, g.listing, g.windows_are_selects != 0u, false, g.list, g.window_list, listed_rows, tid);
-    const BinGrid grid = bin_grid(rows, g.a.vocab, kChainGrid);
+    const BinGrid grid = bin_grid(rows, g.a.vocab, g.most_parts, kChainGrid);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
         const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));

@@ -666,7 +666,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2,
     const int lane = tid & (kWaveSize - 1);
     clear_sample_counts<kWalkThreads>(shared, tid);
     const uint32_t rows = list_rows_in_place<kWalkWaves>(a, g.listing, true, true, g.list, g.other_list, listed_rows, tid);
-    const BinGrid grid = bin_grid(rows, a.vocab, kChainGrid);
+    const BinGrid grid = bin_grid(rows, a.vocab, kMaxBinParts, kChainGrid);
     for (uint32_t slot = grid.first_slot; slot < grid.rows; slot += grid.slot_step)
     {
         const uint32_t row = same_in_all(row_of_slot(g.listing, g.list, listed_rows, slot));

@@ -73,6 +73,9 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_scatter_segments",
     "ncnn_moe_hip_sampler_debug_binned_sums",
     "ncnn_moe_hip_sampler_debug_most_looks",
+    "ncnn_moe_hip_sampler_debug_compute_units",
+    "ncnn_moe_hip_sampler_debug_most_parts",
+    "ncnn_moe_hip_sampler_debug_first_looks",
     "ncnn_moe_hip_sampler_debug_outcome_watched",
     "ncnn_moe_hip_sampler_debug_binned_rows",
     "ncnn_moe_hip_sampler_debug_filtered_rows",
@@ -130,6 +133,11 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_most_looks.argtypes = [vp, ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_compute_units.argtypes = [vp, ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_most_parts.argtypes = [ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_most_parts.restype = ctypes.c_uint32
+    lib.ncnn_moe_hip_sampler_debug_first_looks.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
+    lib.ncnn_moe_hip_sampler_debug_first_looks.restype = ctypes.c_uint32
     lib.ncnn_moe_hip_sampler_debug_outcome_watched.argtypes = [vp, ctypes.c_uint32, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_filtered_rows.argtypes = [vp, vp, ctypes.c_uint32]
@@ -362,6 +370,10 @@ class HipSampler:
     def most_looks(self, looks):
         """Test hook: how often a part of a row looks for the row's other parts before it gives the row up."""
         self._check(self._hooks().ncnn_moe_hip_sampler_debug_most_looks(self._handle, looks))
+
+    def compute_units(self, count):
+        """Test hook: rows are cut into no more parts than on a device of so many compute units."""
+        self._check(self._hooks().ncnn_moe_hip_sampler_debug_compute_units(self._handle, count))
 
     def binned_rows(self, rows):
         """Test hook: which of the handle's first `rows` rows the binned sums finished (1) the last time they were given them."""

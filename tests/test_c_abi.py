@@ -77,6 +77,29 @@ def test_calls_with_a_rejected_row_wait_for_the_stream(field, value):
         assert not hip_sampler.outcome_watched(params, 151936)
 
 
+def test_parts_that_wait_for_each_other_fit_the_device():
+    """The parts of eight rows are workgroups that follow each other: a device holds them all at a time, one to a compute unit, so
+    that parts that wait wait for workgroups that have started."""
+    library = hip_sampler.load_testing_library()
+    for compute_units in range(0, 305):
+        parts = library.ncnn_moe_hip_sampler_debug_most_parts(compute_units)
+        assert 1 <= parts <= 16 and (parts == 1 or 8 * parts <= compute_units)
+    assert [library.ncnn_moe_hip_sampler_debug_most_parts(n) for n in (32, 64, 128, 256, 304)] == [4, 8, 16, 16, 16]
+
+
+def test_waits_are_no_longer_than_what_a_row_given_up_costs():
+    """Looks at a first meeting (half a microsecond each): half a millisecond at least, and a twentieth of a second at most where no
+    select runs beside; never so many that sixteen times as many overflow."""
+    library = hip_sampler.load_testing_library()
+    f32, bf16 = hip_sampler.LOGITS_F32, hip_sampler.LOGITS_BF16
+    looks = library.ncnn_moe_hip_sampler_debug_first_looks
+    assert looks(1, 100, f32, 0) == looks(256, 100000, f32, 0) == 1000
+    assert looks(8, 151936, f32, 0) == looks(300, 151936, bf16, 0) == 1519
+    assert looks(1, (1 << 22) - 16, f32, 0) == 41942
+    assert looks(512, 129280, f32, 1) == 1292 + (512 * 129280 * 4 >> 20)
+    assert looks(65535, (1 << 32) - 1, f32, 1) == 0xffffffff // 16
+
+
 @pytest.mark.parametrize("top_k", [0, 65, 1024, 1025])
 def test_calls_of_several_launches_wait_for_the_stream(top_k):
     params = hip_sampler.make_params(3, 0.8, 20, 0.9, 0.0)

@@ -117,6 +117,56 @@ def test_rows_whose_parts_do_not_wait_for_each_other(rows, vocab):
     assert first.tobytes() == again.tobytes()
 
 
+@pytest.mark.parametrize("rows,vocab,top_ks", [(40, 151936, [0]), (300, 4099, [0]), (80, 33001, [0, 300])])
+def test_rows_of_four_launches_whose_parts_do_not_wait_for_each_other(rows, vocab, top_ks):
+    """The same where the walks are a launch of their own: six parts a row that meet first behind the first walk, one part a row, which
+    meets nobody, and twelve beside the windows and the select."""
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] four launches, parts that do not wait, %d x %d" % (rows, vocab), flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, [0])
+    params["top_k"] = np.resize(np.array(top_ks, dtype=np.uint32), rows)
+    params["top_p"] = 1.0
+    sums = params["top_k"] == 0
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        first = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows)[sums]
+        sampler.most_looks(0)
+        for _ in range(3):
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "parts that do not wait")
+        given_up = served.sum() - sampler.binned_rows(rows)[sums].sum()
+        assert given_up == 0 if rows == 300 else given_up > 0
+        sampler.most_looks(40000)
+        again = sampler.sample(params, uniforms)
+        assert np.array_equal(sampler.binned_rows(rows)[sums], served)
+    parity_util.assert_results_match(first, cpu, "f32", "parts that wait")
+    assert first.tobytes() == again.tobytes()
+
+
+@pytest.mark.parametrize("rows,vocab", [(8, 151936), (40, 151936), (5, 20011)])
+def test_rows_cut_as_on_smaller_devices(rows, vocab):
+    """Rows of eight parts, four and one, as on a device of 64 compute units, 32 and 8: the same results, from the sums."""
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] smaller devices, %d x %d" % (rows, vocab), flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 5000])
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        first = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows).sum()
+        for compute_units in (64, 32, 8):
+            sampler.compute_units(compute_units)
+            gpu = sampler.sample(params, uniforms)
+            assert gpu.tobytes() == first.tobytes(), "as on %d compute units" % compute_units
+            assert sampler.binned_rows(rows).sum() == served
+        with pytest.raises(hip_sampler.SamplerError):
+            sampler.compute_units(64)
+    parity_util.assert_results_match(first, cpu, "f32", "all parts")
+
+
 def _bf16_values(row):
     return workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(row))
 

@@ -119,7 +119,8 @@ def test_windows_over_the_edges_of_parts(rows, vocab, dtype):
 @pytest.mark.parametrize("rows,vocab,top_ks", [(200, 8191, [300, 1000]), (96, 16411, [0, 300]), (40, 20011, [0])])
 def test_calls_that_hold_each_other_s_places(rows, vocab, top_ks):
     """Three handles on three streams: workgroups of one call start when others of it have finished their rows, the soonest those
-    that have no finite logit, and come to the same list of rows all the same."""
+    that have no finite logit, and come to the same list of rows all the same.  Parts that hold places each other's rows need give their rows up;
+    a call by itself then serves all that it served before."""
     print("[case] three streams, %d x %d, top_k %s" % (rows, vocab, top_ks), flush=True)
     calls = []
     for seed in range(3):
@@ -131,8 +132,24 @@ def test_calls_that_hold_each_other_s_places(rows, vocab, top_ks):
         uniforms = rng.random(rows, dtype=np.float32)
         device = [torch.from_numpy(x).cuda() for x in (logits, params.view(np.uint8), uniforms)]
         results = torch.zeros(8, rows * 16, dtype=torch.uint8, device="cuda")
-        calls.append((hip_sampler.HipSampler(rows, vocab), torch.cuda.Stream(), device, results, parity_util.run_oracle(logits, params, uniforms)))
+        sampler = hip_sampler.HipSampler(rows, vocab, testing=True)
+        sampler.binned_sums(True)
+        calls.append((sampler, torch.cuda.Stream(), device, results, parity_util.run_oracle(logits, params, uniforms)))
     torch.cuda.synchronize()
+
+    def last_served(call):
+        top_k = call[2][1].cpu().numpy().view(hip_sampler.PARAMS_DTYPE)["top_k"]
+        return int(call[0].binned_rows(rows)[top_k == 0].sum())
+
+    def served(call):
+        sampler, stream, device, results, _ = call
+        sampler.sample_device(device[0].data_ptr(), hip_sampler.LOGITS_F32, rows, vocab, vocab, device[1].data_ptr(), device[2].data_ptr(), None,
+                              results[0].data_ptr(), hip_sampler.PASSES_FULL_ORDER, stream.cuda_stream)
+        torch.cuda.synchronize()
+        return last_served(call)
+
+    alone = [served(call) for call in calls]
+    assert 0 not in top_ks or min(alone) > 0
     for i in range(8):
         for sampler, stream, device, results, _ in calls:
             sampler.sample_device(device[0].data_ptr(), hip_sampler.LOGITS_F32, rows, vocab, vocab, device[1].data_ptr(), device[2].data_ptr(), None,
@@ -142,4 +159,8 @@ def test_calls_that_hold_each_other_s_places(rows, vocab, top_ks):
         for i in range(8):
             gpu = results[i].cpu().numpy().view(hip_sampler.RESULT_DTYPE)
             parity_util.assert_results_match(gpu, cpu, "f32", "call %d beside others" % i)
+    print("[served] alone %s, the last of the calls beside others %s" % (
+        alone, [last_served(call) for call in calls]), flush=True)
+    assert [served(call) for call in calls] == alone
+    for sampler, *_ in calls:
         sampler.close()
