@@ -145,7 +145,9 @@ int ncnn_moe_hip_sampler_sample(
  * same result, NCNN_MOE_ROW_FLAG_GENERAL_PATH set); add NCNN_MOE_PASSES_NO_WIDE_WINDOWS when the caller knows that no row has
  * 64 < top_k <= 1024: the kernels for such windows are then not enqueued (a row that has one after
  * all is served like one without a window: slower, same result).
- * Calls on one handle share its scratch memory and must not overlap. */
+ * Calls on one handle share its scratch memory and must not overlap.  A synchronous call returns when its results are known, which
+ * may be a few microseconds before its kernels have ended on the handle's own stream; this call waits for those.  (Once a
+ * call has been captured into a graph, whose replays the handle does not see, its synchronous calls return when their kernels have ended.) */
 #define NCNN_MOE_PASSES_FULL_ORDER 1
 #define NCNN_MOE_PASSES_SIDE_BY_SIDE 2
 #define NCNN_MOE_PASSES_NO_WIDE_WINDOWS 4

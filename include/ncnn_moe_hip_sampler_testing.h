@@ -42,6 +42,8 @@ int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* sampler, uint32_
 int ncnn_moe_hip_sampler_debug_compute_units(ncnn_moe_hip_sampler* sampler, uint32_t compute_units);
 uint32_t ncnn_moe_hip_sampler_debug_most_parts(uint32_t compute_units);
 uint32_t ncnn_moe_hip_sampler_debug_first_looks(uint32_t rows, uint32_t vocab, int dtype, int side_by_side);
+/* 1 if the last synchronous call on the handle returned with its outcome and nothing has waited for the handle's stream since. */
+int ncnn_moe_hip_sampler_debug_stream_may_run(const ncnn_moe_hip_sampler* sampler);
 /* 1 if ncnn_moe_hip_sampler_sample watches for its records in pinned memory with these options, 0 if it waits for the stream.
  * No GPU needed. */
 int ncnn_moe_hip_sampler_debug_outcome_watched(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab);

@@ -43,6 +43,8 @@ struct ncnn_moe_hip_sampler
     hipEvent_t side_join = nullptr;
     hipEvent_t cut_done = nullptr;
     hipStream_t stream = nullptr;
+    bool stream_may_run = false; // a synchronous call has returned with its outcome: its launches may still be ending there
+    bool captured = false;       // a sample_device call has been captured: its replays are ordered behind nothing here
 
     void* device_memory = nullptr; // every device buffer below
     void* logits = nullptr;
@@ -319,10 +321,36 @@ bool watch_outcome(const void* records, size_t words, std::chrono::steady_clock:
     return true;
 }
 
-hipError_t wait_for_outcome(const void* records, size_t words, hipStream_t stream)
+hipError_t synchronize(ncnn_moe_hip_sampler* s)
 {
-    const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched);
-    return watch_outcome(records, words, deadline) ? hipSuccess : hipStreamSynchronize(stream);
+    const hipError_t error = hipStreamSynchronize(s->stream);
+    s->stream_may_run = s->stream_may_run && error != hipSuccess;
+    return error;
+}
+
+// `outcome_seen(deadline)` watches for what the call returns.  The launches behind it share the handle's scratch with calls on other streams:
+// sample_device waits for them (see settle).  It cannot where its launches are replays of a graph, so a handle that has
+// been captured waits for its stream here.
+template <typename OutcomeSeen>
+hipError_t wait_for_outcome(ncnn_moe_hip_sampler* s, OutcomeSeen outcome_seen)
+{
+    if (s->captured)
+        return synchronize(s);
+    s->stream_may_run = true;
+    return outcome_seen(std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched)) ? hipSuccess : synchronize(s);
+}
+
+// Waits for what a synchronous call has left on the handle's stream, in front of launches on another one (which may be
+// captured: a wait for a stream that is not is allowed in the relaxed mode only).
+hipError_t settle(ncnn_moe_hip_sampler* s)
+{
+    if (!s->stream_may_run)
+        return hipSuccess;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t error = synchronize(s);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return error;
 }
 
 constexpr uint32_t kSideBySideRows = 32; // rows of each kind from which sample() runs the two later passes side by side
@@ -1136,7 +1164,7 @@ int ncnn_moe_hip_sampler_upload_logits(
     SAMPLER_HIP_CHECK(s, hipMemcpy2DAsync(
         device_logits, device_stride * element, host_logits, row_stride * element,
         static_cast<size_t>(vocab) * element, rows, hipMemcpyHostToDevice, s->stream));
-    SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+    SAMPLER_HIP_CHECK(s, synchronize(s));
     return NCNN_MOE_SAMPLER_SUCCESS;
 }
 
@@ -1194,7 +1222,8 @@ int ncnn_moe_hip_sampler_sample(
         device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, passes, s->stream);
     if (rc != NCNN_MOE_SAMPLER_SUCCESS)
         return rc;
-    SAMPLER_HIP_CHECK(s, watched ? wait_for_outcome(s->results_host, result_words, s->stream) : hipStreamSynchronize(s->stream));
+    const auto seen = [s, result_words](auto deadline) { return watch_outcome(s->results_host, result_words, deadline); };
+    SAMPLER_HIP_CHECK(s, watched ? wait_for_outcome(s, seen) : synchronize(s));
     if (!full_order)
     {
         // a row whose ties overflowed the select buffers is finished by the full-order kernels
@@ -1211,7 +1240,7 @@ int ncnn_moe_hip_sampler_sample(
                 device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, retry, s->stream);
             if (rc != NCNN_MOE_SAMPLER_SUCCESS)
                 return rc;
-            SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+            SAMPLER_HIP_CHECK(s, synchronize(s));
         }
     }
     std::memcpy(results, s->results_host, rows * sizeof(ncnn_moe_sample_result));
@@ -1236,6 +1265,13 @@ int ncnn_moe_hip_sampler_sample_device(
     if (row_stride < vocab)
         return fail(s, NCNN_MOE_SAMPLER_INVALID_ARGUMENT, "row_stride is smaller than vocab");
     SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
+    SAMPLER_HIP_CHECK(s, settle(s));
+    if (stream != nullptr && !s->captured) // (the default stream is not captured)
+    {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        (void)hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capturing);
+        s->captured = capturing != hipStreamCaptureStatusNone;
+    }
     SamplerPasses passes;
     passes.wide_select = may_need_full_order != 0 && (may_need_full_order & NCNN_MOE_PASSES_NO_WIDE_WINDOWS) == 0;
     passes.full_order = may_need_full_order != 0 || s->force_general != 0;
@@ -1361,7 +1397,7 @@ int ncnn_moe_hip_sampler_distribution(
     uint32_t kept = 0;
     SAMPLER_HIP_CHECK(s, hipMemcpyAsync(&result, s->single_result, sizeof(result), hipMemcpyDeviceToHost, s->stream));
     SAMPLER_HIP_CHECK(s, hipMemcpyAsync(&kept, s->distribution_count, sizeof(kept), hipMemcpyDeviceToHost, s->stream));
-    SAMPLER_HIP_CHECK(s, hipStreamSynchronize(s->stream));
+    SAMPLER_HIP_CHECK(s, synchronize(s));
     *status = result.status;
     *count = kept;
     const uint32_t n = kept < cap ? kept : cap;
@@ -1429,11 +1465,11 @@ int ncnn_moe_hip_sampler_speculative_verify(
     // read a later call's operands: they leave nothing but the scratch that the later call's own launch writes behind them.)
     const auto expect_outcome = [s]() { clear_outcome(s->verify_output_host, sizeof(*s->verify_output_host) / sizeof(uint32_t)); };
     const auto await_outcome = [s, draft_count]() {
-        const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched);
-        const auto& out = *s->verify_output_host;
-        const bool seen = watch_outcome(&out.result, sizeof(out.result) / sizeof(uint32_t), deadline) &&
-            watch_outcome(out.accepted, std::min(out.result.accepted, draft_count), deadline);
-        return seen ? hipSuccess : hipStreamSynchronize(s->stream);
+        return wait_for_outcome(s, [s, draft_count](auto deadline) {
+            const auto& out = *s->verify_output_host;
+            return watch_outcome(&out.result, sizeof(out.result) / sizeof(uint32_t), deadline) &&
+                watch_outcome(out.accepted, std::min(out.result.accepted, draft_count), deadline);
+        });
     };
     const auto take_outcome = [s, draft_count, accepted_probabilities, result]() {
         *result = s->verify_output_host->result;
@@ -1618,6 +1654,12 @@ uint32_t ncnn_moe_hip_sampler_debug_most_parts(uint32_t compute_units)
 uint32_t ncnn_moe_hip_sampler_debug_first_looks(uint32_t rows, uint32_t vocab, int dtype, int side_by_side)
 {
     return most_looks_of(rows, vocab, dtype == NCNN_MOE_LOGITS_F32 ? 4u : 2u, side_by_side != 0);
+}
+
+// Whether the last synchronous call returned with its outcome, and nothing has waited for the handle's stream since.
+int ncnn_moe_hip_sampler_debug_stream_may_run(const ncnn_moe_hip_sampler* s)
+{
+    return s != nullptr && s->stream_may_run ? 1 : 0;
 }
 
 // Whether sample() watches for its records with these options (else it waits for the stream).

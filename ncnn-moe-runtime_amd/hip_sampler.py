@@ -76,6 +76,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_compute_units",
     "ncnn_moe_hip_sampler_debug_most_parts",
     "ncnn_moe_hip_sampler_debug_first_looks",
+    "ncnn_moe_hip_sampler_debug_stream_may_run",
     "ncnn_moe_hip_sampler_debug_outcome_watched",
     "ncnn_moe_hip_sampler_debug_binned_rows",
     "ncnn_moe_hip_sampler_debug_filtered_rows",
@@ -138,6 +139,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_most_parts.restype = ctypes.c_uint32
     lib.ncnn_moe_hip_sampler_debug_first_looks.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_first_looks.restype = ctypes.c_uint32
+    lib.ncnn_moe_hip_sampler_debug_stream_may_run.argtypes = [vp]
     lib.ncnn_moe_hip_sampler_debug_outcome_watched.argtypes = [vp, ctypes.c_uint32, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_binned_rows.argtypes = [vp, vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_filtered_rows.argtypes = [vp, vp, ctypes.c_uint32]
@@ -370,6 +372,10 @@ class HipSampler:
     def most_looks(self, looks):
         """Test hook: how often a part of a row looks for the row's other parts before it gives the row up."""
         self._check(self._hooks().ncnn_moe_hip_sampler_debug_most_looks(self._handle, looks))
+
+    def stream_may_run(self):
+        """Test hook: whether the last synchronous call returned with its outcome, and nothing has waited for the handle's stream since."""
+        return self._hooks().ncnn_moe_hip_sampler_debug_stream_may_run(self._handle) == 1
 
     def compute_units(self, count):
         """Test hook: rows are cut into no more parts than on a device of so many compute units."""

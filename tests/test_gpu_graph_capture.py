@@ -61,6 +61,67 @@ def test_sampler_step_in_a_graph(passes):
             parity_util.assert_results_match(gpu, cpu, "f32", "graph replay %d" % replay)
 
 
+def test_launches_on_a_caller_stream_behind_synchronous_calls():
+    """A synchronous call may return before its kernels have ended: a sample_device call behind it waits for them, captured or
+    not, and a handle that has been captured, whose replays it does not see, has none left."""
+    print("[case] sample_device and its replays behind synchronous calls", flush=True)
+    rng = np.random.default_rng(5)
+    drafts, vocab = 2, 40013
+    rows = 2 * drafts + 1
+    logits = (rng.standard_normal((rows, vocab)) * 2.5).astype(np.float32)
+    params = hip_sampler.make_params(rows, 0.8, 0, 0.9, 0.0)
+    params["top_k"][::2] = 20
+    select = hip_sampler.make_params(rows, 0.8, 50, 0.9, 0.0)
+    uniforms = rng.random(rows).astype(np.float32)
+    proposed = np.argmax(logits[drafts + 1:], axis=1).astype(np.int32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    cpu_select = parity_util.run_oracle(logits, select, uniforms)
+    device = torch.device("cuda:0")
+    d_logits, d_params, d_uniforms = torch.from_numpy(logits).to(device), _bytes(params).to(device), torch.from_numpy(uniforms).to(device)
+    d_results = torch.zeros(rows * 16, dtype=torch.uint8, device=device)
+    stream = torch.cuda.Stream(device=device)
+    torch.cuda.synchronize()
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+
+        def enqueue():
+            sampler.sample_device(d_logits.data_ptr(), hip_sampler.LOGITS_F32, rows, vocab, vocab, d_params.data_ptr(),
+                                  d_uniforms.data_ptr(), None, d_results.data_ptr(), hip_sampler.PASSES_FULL_ORDER, stream.cuda_stream)
+
+        def check(context):
+            torch.cuda.synchronize()
+            parity_util.assert_results_match(d_results.cpu().numpy().view(hip_sampler.RESULT_DTYPE), cpu, "f32", context)
+            d_results.zero_()
+            torch.cuda.synchronize()
+
+        synchronous = [
+            lambda: parity_util.assert_results_match(sampler.sample(select, uniforms), cpu_select, "f32", "synchronous"),
+            lambda: sampler.speculative_verify(proposed, uniforms[:drafts + 1], temperature=0.8, top_k=0, top_p=0.9, min_p=0.0),
+            lambda: sampler.speculative_verify(proposed, uniforms[:drafts + 1], temperature=0.8, top_k=50, top_p=0.9, min_p=0.0)]
+        for call in synchronous:
+            left = 0
+            for _ in range(10):
+                call()
+                left += sampler.stream_may_run()
+                enqueue()
+                assert not sampler.stream_may_run()
+                check("behind a synchronous call")
+            assert left > 0
+        sampler.sample(select, uniforms)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            enqueue()
+        assert not sampler.stream_may_run()
+        for replay in range(3):
+            for call in synchronous:
+                call()
+                assert not sampler.stream_may_run()
+                with torch.cuda.stream(stream):
+                    graph.replay()
+                check("replay %d behind a synchronous call" % replay)
+
+
 def test_router_dispatch_in_a_graph():
     print("[case] router dispatch_device captured in a HIP graph, 4 replays", flush=True)
     rng = np.random.default_rng(32)
