@@ -10,6 +10,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 
 using namespace ncnn_moe_hip;
 
@@ -76,7 +77,24 @@ void launch_select(const RouterArgs& args, hipStream_t stream)
         hipLaunchKernelGGL(router_select_kernel<SLOTS>, dim3(staged_blocks), dim3(kRouterThreads), 0, stream, args);
         return;
     }
-    hipLaunchKernelGGL(router_batch_kernel<SLOTS>, dim3((args.tokens + kBatchWaves - 1u) / kBatchWaves), dim3(kBatchThreads), 0, stream, args);
+    const auto batch = [&](auto waves) {
+        constexpr int kWaves = decltype(waves)::value;
+        hipLaunchKernelGGL((router_batch_kernel<SLOTS, kWaves>), dim3((args.tokens + kWaves - 1u) / kWaves), dim3(kWaves * kWaveSize), 0, stream, args);
+    };
+    // (see kBatchWaves)
+    bool few_waves = SLOTS > 8;
+    if constexpr (SLOTS == 8)
+        few_waves = args.tokens <= kFewBatchTokens;
+    if constexpr (SLOTS >= 8)
+    {
+        if (few_waves)
+            batch(std::integral_constant<int, kFewBatchWaves>{});
+    }
+    if constexpr (SLOTS <= 8)
+    {
+        if (!few_waves)
+            batch(std::integral_constant<int, kBatchWaves>{});
+    }
     const unsigned chunks = (args.tokens + kRouterChunkTokens - 1) / kRouterChunkTokens;
     hipLaunchKernelGGL(router_group_kernel, dim3(chunks), dim3(kRouterThreads), 0, stream, args);
 }

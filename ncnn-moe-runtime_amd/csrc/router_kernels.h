@@ -360,7 +360,7 @@ __device__ __forceinline__ bool take_explicit(const RouterArgs& r, const float* 
 }
 
 // A token's routes from its scores in LDS (not yet divided by `divisor`), by one wave.  Not FUSED: `held` has them as well, expert e in slot
-// e / 64 of lane e % 64 (zeros past the last expert), and `counts`, in LDS, counts the routes to each expert.
+// e / 64 of lane e % 64 (zeros past the last expert), and `counts` counts the routes to each expert.
 template <int SLOTS, bool FUSED>
 __device__ __forceinline__ void route_token(
     const RouterArgs& r, const float* scores, const float (&held)[SLOTS], float divisor, RouteScratch& scratch, uint32_t* counts, uint32_t token, int lane)
@@ -420,26 +420,36 @@ __device__ __forceinline__ void route_token(
 
 // Calls of more than one chunk: a wave takes a token from its logits to its routes, without waiting for another wave.  Under the softmax
 // the scores pass through LDS, so that their sum, one addition at a time in expert order, is a chain of additions on few reads.
-// The workgroup's routes are counted in LDS and added to the chunk's counters a line at a time: an atomic a route cost as much as all
-// the rest where experts are few (8 experts and 2 routes, 2,048 tokens 18.2 -> 9.7 us, 16,384 26.8 -> 14.8; 64 and 6, 1,024 tokens
-// 13.2 -> 10.5, 16,384 22.1 -> 18.9; 256 and 8, 16,384 28.7 -> 27.2).  Eight waves rather than four: fewer such additions (16,384 of 8
-// experts 14.8 and 16.4 us); two or four tokens a wave: 0 to 15 % slower from 64 experts on.
+// Up to 512 experts the workgroup's routes are counted in LDS and added to the chunk's counters a line at a time: an atomic a route cost as
+// much as all the rest where experts are few (8 experts and 2 routes, 2,048 tokens 18.2 -> 9.7 us, 16,384 26.8 -> 14.8; 64 and 6, 1,024 tokens
+// 13.2 -> 10.5, 16,384 22.1 -> 18.9; 256 and 8, 16,384 28.7 -> 27.2).  More experts hardly share routes, and the counters' way through LDS costs
+// more than it saves (1,024 experts, 257 tokens 22.7 and 22.4, 16,384 76.1 and 75.2 without).
+// Two or four tokens a wave: 0 to 15 % slower from 64 experts on.
 // What bounds it: instructions, some 640 per token of 256 experts under the softmax: 280 for the sum, 110 for the exponentials, 50 for
 // the divisions, 130 for the selection.
+//
+// Waves of a workgroup: eight, which add their counts up together (16,384 tokens of 8 experts 14.8 us, with four 16.4).  But four
+// from 257 experts on where that gives every compute unit one at most (1,024 tokens): a token is then so much work that waves two to a SIMD
+// wait for each other (512 experts, sqrt softplus, 257 tokens 16.6 and 16.0, 1,024 17.3 and 16.4; 1,536 17.5 and 17.7), and from 513 on always
+// (1,024 experts, softmax, 257 tokens 22.8 and 21.3, 16,384 64.8 and 63.6).
 constexpr int kBatchWaves = 8;
-constexpr int kBatchThreads = kBatchWaves * kWaveSize;
-static_assert(kRouterChunkTokens % kBatchWaves == 0, "a workgroup's tokens are of one chunk");
+constexpr int kFewBatchWaves = 4;
+constexpr uint32_t kFewBatchTokens = 256u * kFewBatchWaves;
 
-template <int SLOTS>
-__global__ __launch_bounds__(kBatchThreads) void router_batch_kernel(RouterArgs r)
+template <int SLOTS, int WAVES>
+__global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterArgs r)
 {
-    __shared__ __align__(16) float rows[kBatchWaves][SLOTS * kWaveSize];
-    __shared__ __align__(16) RouteScratch scratch[kBatchWaves];
-    __shared__ uint32_t counts[SLOTS * kWaveSize]; // the workgroup's routes to each expert
+    constexpr int kThreads = WAVES * kWaveSize;
+    constexpr bool kCountsInLds = SLOTS <= 8;
+    static_assert(kRouterChunkTokens % WAVES == 0, "a workgroup's tokens are of one chunk");
+    __shared__ __align__(16) float rows[WAVES][SLOTS * kWaveSize];
+    __shared__ __align__(16) RouteScratch scratch[WAVES];
+    __shared__ uint32_t workgroup_counts[kCountsInLds ? SLOTS * kWaveSize : 1]; // the workgroup's routes to each expert
     __shared__ uint64_t exp2_table[32];
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const uint32_t token = blockIdx.x * kBatchWaves + static_cast<uint32_t>(wave);
+    const uint32_t token = blockIdx.x * WAVES + static_cast<uint32_t>(wave);
+    uint32_t* const chunk_counts = r.chunk_counts + static_cast<size_t>(blockIdx.x * WAVES / kRouterChunkTokens) * chunk_count_stride(r.experts);
     const float* const logits = r.logits + static_cast<size_t>(min(token, r.tokens - 1u)) * r.experts;
     float score[SLOTS];
 #pragma unroll
@@ -450,8 +460,11 @@ __global__ __launch_bounds__(kBatchThreads) void router_batch_kernel(RouterArgs 
     }
     if (threadIdx.x < 32)
         exp2_table[threadIdx.x] = kExp2Table[threadIdx.x];
-    for (uint32_t e = threadIdx.x; e < SLOTS * kWaveSize; e += kBatchThreads)
-        counts[e] = 0u;
+    if constexpr (kCountsInLds)
+    {
+        for (uint32_t e = threadIdx.x; e < SLOTS * kWaveSize; e += kThreads)
+            workgroup_counts[e] = 0u;
+    }
     __syncthreads();
     bool finite = true;
     float maximum = -__builtin_inff();
@@ -494,16 +507,18 @@ __global__ __launch_bounds__(kBatchThreads) void router_batch_kernel(RouterArgs 
                 each_score([&](float x) { return sigmoid_score(x, exp2_table); });
             else
                 each_score([&](float x) { return sqrt_softplus_score(x, exp2_table); });
-            route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], counts, token, lane);
+            route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], kCountsInLds ? workgroup_counts : chunk_counts, token, lane);
         }
     }
-    __syncthreads();
-    const uint32_t chunk = blockIdx.x * kBatchWaves / kRouterChunkTokens;
-    for (uint32_t e = threadIdx.x; e < r.experts; e += kBatchThreads)
+    if constexpr (kCountsInLds)
     {
-        const uint32_t count = counts[e];
-        if (count != 0u)
-            atomicAdd(&r.chunk_counts[static_cast<size_t>(chunk) * chunk_count_stride(r.experts) + e], count);
+        __syncthreads();
+        for (uint32_t e = threadIdx.x; e < r.experts; e += kThreads)
+        {
+            const uint32_t count = workgroup_counts[e];
+            if (count != 0u)
+                atomicAdd(&chunk_counts[e], count);
+        }
     }
 }
 

@@ -78,6 +78,21 @@ def test_last_workgroups_of_a_call_count_their_routes(router, tokens):
         assert _compare(router, logits, top_k, "... and again", **options) == 0
 
 
+@pytest.mark.parametrize("tokens", [257, 1023, 1024, 1025])
+@pytest.mark.parametrize("experts", [256, 257, 512, 513, 1024])
+def test_workgroups_of_four_waves_and_of_eight(router, experts, tokens):
+    """Both sides of the token and expert counts at which a workgroup's waves and its count of routes change."""
+    rng = np.random.default_rng(experts * 10000 + tokens)
+    logits = _logits(rng, tokens, experts, 2.0)
+    for score in (hip_router.SOFTMAX, hip_router.SIGMOID, hip_router.SQRT_SOFTPLUS):
+        options = dict(score_function=score, renormalize=True, routed_scaling_factor=2.5)
+        assert _compare(router, logits, 8, "waves, T=%d E=%d score %d" % (tokens, experts, score), **options) == 0
+        failing = logits.copy()
+        failing[tokens - 1, experts - 1] = np.nan
+        assert _compare(router, failing, 8, "... which fails", **options) != 0
+        assert _compare(router, logits, 8, "... and again", **options) == 0
+
+
 def test_ties_resolve_to_the_lower_expert_id(router):
     rng = np.random.default_rng(3)
     for experts, top_k in [(16, 4), (128, 8), (300, 17)]:
