@@ -36,6 +36,8 @@ int ncnn_moe_hip_sampler_debug_binned_rows(ncnn_moe_hip_sampler* sampler, uint32
 /* most_looks: how often a part of a row looks for the row's other parts before it gives the row up, which is then sorted (0:
  * a part that has to wait gives up at once).  Same results either way. */
 int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* sampler, uint32_t looks);
+/* parts_apart: a row's parts hand over to each other as they would on several XCDs (by stores of agent scope).  Same results either way. */
+int ncnn_moe_hip_sampler_debug_parts_apart(ncnn_moe_hip_sampler* sampler, int enabled);
 /* compute_units: the handle's rows are cut into no more parts than a device of so many compute units would have them in (refused where
  * that is more than the handle has).  Same results either way.  most_parts is that number of parts, first_looks how often a part
  * looks at the row's first meeting; no GPU needed for these two. */

@@ -96,6 +96,7 @@ struct ncnn_moe_hip_sampler
     uint32_t* window_list = nullptr;
 #ifdef NCNN_MOE_TESTING
     int binned_sums = 0;        // (the tests of the sort reach it first)
+    bool parts_apart = false;   // parts of a row hand over as if they were on several XCDs
 #else
     int binned_sums = 1;        // rows that the first select leaves go to the binned sums first
 #endif
@@ -412,6 +413,10 @@ hipError_t launch_bin_sums(ncnn_moe_hip_sampler* s, const SamplerArgs& a, RowLis
     g.window_list = window_list;
     if (g.most_looks == kLooksByLength)
         g.most_looks = most_looks_of(a.rows, a.vocab, DTYPE == NCNN_MOE_LOGITS_F32 ? 4u : 2u, behind_sum != nullptr);
+#ifdef NCNN_MOE_TESTING
+    if (s->parts_apart)
+        g.most_looks |= kPartsApart;
+#endif
     hipError_t result = hipSuccess;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (behind_terms != nullptr || behind_sum != nullptr)
@@ -1633,7 +1638,16 @@ int ncnn_moe_hip_sampler_debug_most_looks(ncnn_moe_hip_sampler* s, uint32_t look
 {
     if (s == nullptr)
         return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
-    s->bins.most_looks = looks;
+    s->bins.most_looks = std::min(looks, 0xffffffffu / kLaterLooks);
+    return NCNN_MOE_SAMPLER_SUCCESS;
+}
+
+// Parts of a row hand over as if they were on several XCDs.
+int ncnn_moe_hip_sampler_debug_parts_apart(ncnn_moe_hip_sampler* s, int enabled)
+{
+    if (s == nullptr)
+        return NCNN_MOE_SAMPLER_INVALID_ARGUMENT;
+    s->parts_apart = enabled != 0;
     return NCNN_MOE_SAMPLER_SUCCESS;
 }
 

@@ -2933,6 +2933,7 @@ __device__ __forceinline__ BinWalkOutcome bin_walk(const BinArgs& g, const BinGr
 // arrivals[0] counts the parts that have come to the row's meetings and, above, how many came to the first from each XCD: from then on
 // shared.near tells whether all are on one.  arrivals[1] counts those that are done with the row: the last of them returns both to zero.
 constexpr uint32_t kLaterLooks = 16;
+constexpr uint32_t kPartsApart = 1u << 31; // in most_looks: the parts hand over as if they were on several XCDs (tests)
 constexpr unsigned long long kArrivalsOnly = 0xffffull;
 constexpr unsigned long long kRowGivenUp = 1ull << 63;
 constexpr uint32_t kXcdShift = 16, kXcdBits = 5;
@@ -2981,7 +2982,8 @@ __device__ __forceinline__ bool parts_meet(unsigned long long* arrivals, uint32_
         const unsigned long long one = meeting == 1u ? 1ull + own_place : 1ull;
         unsigned long long seen = __hip_atomic_fetch_add(arrivals, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + one;
         const uint32_t goal = meeting * parts;
-        const uint32_t most = meeting == 1u ? most_looks : most_looks * kLaterLooks;
+        const uint32_t first_looks = most_looks & ~kPartsApart;
+        const uint32_t most = meeting == 1u ? first_looks : first_looks * kLaterLooks;
         const auto come = [&]() { return static_cast<uint32_t>(seen & kArrivalsOnly) >= goal; };
         for (uint32_t looks = 0; wait && !come() && (seen & kRowGivenUp) == 0ull; ++looks)
         {
@@ -2995,7 +2997,7 @@ __device__ __forceinline__ bool parts_meet(unsigned long long* arrivals, uint32_
         }
         shared.met = wait && come() ? 1u : 0u;
         if (meeting == 1u)
-            shared.near = (seen & ~kRowGivenUp) >> kXcdShift == parts * (own_place >> kXcdShift) ? 1u : 0u;
+            shared.near = (seen & ~kRowGivenUp) >> kXcdShift == parts * (own_place >> kXcdShift) && (most_looks & kPartsApart) == 0u ? 1u : 0u;
     }
     __syncthreads();
     return same_in_all(shared.met) != 0u;

@@ -73,6 +73,7 @@ TESTING_SYMBOLS = [
     "ncnn_moe_hip_sampler_debug_scatter_segments",
     "ncnn_moe_hip_sampler_debug_binned_sums",
     "ncnn_moe_hip_sampler_debug_most_looks",
+    "ncnn_moe_hip_sampler_debug_parts_apart",
     "ncnn_moe_hip_sampler_debug_compute_units",
     "ncnn_moe_hip_sampler_debug_most_parts",
     "ncnn_moe_hip_sampler_debug_first_looks",
@@ -134,6 +135,7 @@ def _bind(lib, testing):
     lib.ncnn_moe_hip_sampler_debug_scatter_segments.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_binned_sums.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_most_looks.argtypes = [vp, ctypes.c_uint32]
+    lib.ncnn_moe_hip_sampler_debug_parts_apart.argtypes = [vp, ctypes.c_int]
     lib.ncnn_moe_hip_sampler_debug_compute_units.argtypes = [vp, ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_most_parts.argtypes = [ctypes.c_uint32]
     lib.ncnn_moe_hip_sampler_debug_most_parts.restype = ctypes.c_uint32
@@ -376,6 +378,10 @@ class HipSampler:
     def stream_may_run(self):
         """Test hook: whether the last synchronous call returned with its outcome, and nothing has waited for the handle's stream since."""
         return self._hooks().ncnn_moe_hip_sampler_debug_stream_may_run(self._handle) == 1
+
+    def parts_apart(self, enabled):
+        """Test hook: a row's parts hand over to each other as if they were on several XCDs."""
+        self._check(self._hooks().ncnn_moe_hip_sampler_debug_parts_apart(self._handle, 1 if enabled else 0))
 
     def compute_units(self, count):
         """Test hook: rows are cut into no more parts than on a device of so many compute units."""

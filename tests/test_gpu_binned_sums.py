@@ -72,24 +72,30 @@ def test_draws_and_cuts_at_the_ends():
     parity_util.assert_results_match(gpu, cpu, "f32", "ends")
 
 
-@pytest.mark.parametrize("rows", [16, 17])
-def test_walks_with_and_without_a_compute_unit_of_their_own(rows):
-    """The last number of rows whose walks have a compute unit each, and the first that share; many ties half way between two
-    sums, which the walks fetch."""
+# Both sides of what decides whether the sums are one launch: elements a part (16 parts of 20,000 logits, and 6 of 80,000 where the call has
+# windows), and as many rows as compute units.
+@pytest.mark.parametrize("rows,vocab,windows", [(16, 65537, 0), (17, 65537, 0), (3, 320015, 0), (3, 320016, 0), (256, 4099, 0), (257, 4099, 0),
+                                                (40, 480005, 3), (40, 480006, 3), (256, 4099, 20), (257, 4099, 20)])
+@pytest.mark.parametrize("apart", [False, True])
+def test_sums_of_one_launch_and_of_four(rows, vocab, windows, apart):
+    """Many ties half way between two sums, which the walks fetch; with parts that hand over inside an XCD, and as if between them."""
     rng = np.random.default_rng(rows)
-    vocab = 65537
-    print("[case] walks, %d rows" % rows, flush=True)
+    print("[case] one launch and four, %d x %d, %d windows, apart %d" % (rows, vocab, windows, apart), flush=True)
     logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 5000])
     logits[::2] = rng.integers(-400, 400, (len(logits[::2]), vocab)).astype(np.float32) / 128
     params["temperature"][::2] = 1.0
+    params["top_k"][rows - windows:] = 300
     cpu = parity_util.run_oracle(logits, params, uniforms)
     with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
         sampler.binned_sums(True)
+        sampler.parts_apart(apart)
         sampler.upload_logits(logits)
         gpu = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows)[params["top_k"] != 300].sum()
         again = sampler.sample(params, uniforms)
-    parity_util.assert_results_match(gpu, cpu, "f32", "walks")
+    parity_util.assert_results_match(gpu, cpu, "f32", "one launch and four")
     assert gpu.tobytes() == again.tobytes()
+    assert served > 0
 
 
 @pytest.mark.parametrize("rows,vocab", [(8, 151936), (16, 40009), (40, 20011)])
@@ -143,6 +149,27 @@ def test_rows_of_four_launches_whose_parts_do_not_wait_for_each_other(rows, voca
         assert np.array_equal(sampler.binned_rows(rows)[sums], served)
     parity_util.assert_results_match(first, cpu, "f32", "parts that wait")
     assert first.tobytes() == again.tobytes()
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 151936), (8, 151936), (40, 20011), (40, 151936), (130, 16411)])
+def test_parts_that_hand_over_between_xcds(rows, vocab):
+    """All that parts hand to each other in the launches of the sums, stored with agent scope, as where they are on several XCDs: the same
+    results, from the sums."""
+    rng = np.random.default_rng(rows * 7 + vocab)
+    print("[case] parts apart, %d x %d" % (rows, vocab), flush=True)
+    logits, params, uniforms = _batch(rng, rows, vocab, [0, 0, 5000])
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        near = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows)
+        sampler.parts_apart(True)
+        for _ in range(3):
+            apart = sampler.sample(params, uniforms)
+            assert apart.tobytes() == near.tobytes()
+            assert np.array_equal(sampler.binned_rows(rows), served)
+    parity_util.assert_results_match(near, cpu, "f32", "parts apart")
 
 
 @pytest.mark.parametrize("rows,vocab", [(8, 151936), (40, 151936), (5, 20011)])
