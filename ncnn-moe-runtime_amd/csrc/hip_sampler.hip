@@ -294,7 +294,7 @@ struct DistributionExport
 // us, with the stream waited for 9.5).  So a synchronous call fills the records with words that no outcome holds, and waits until they are all
 // overwritten: each word by itself, so nothing depends on how a record arrives.  A kernel writes the record of a row with valid options when
 // all that the row was made from has been read, so the logits and the operands may be overwritten when the call returns.  (A rejected row's is
-// written by the first of its workgroups to read the options, and the others read them when they start: see outcome_tells_all.)  Whatever
+// written by the first of its workgroups to read the options, and the others read them when they start: see needs_of.)  Whatever
 // does not come in time (a fault, a GPU that others hold) is waited for by hipStreamSynchronize, which reports errors.
 constexpr uint32_t kNoOutcome = 0xfffffffeu; // no token id or count; as a probability a NaN; its lowest byte is no row status
 constexpr int64_t kMostMicrosecondsWatched = 2000;
@@ -792,34 +792,39 @@ bool row_left_pending(const ncnn_moe_sample_params& p, uint32_t vocab, uint32_t 
     return resolve_row_mode(p, vocab, max_top_k, 0, effective_k, status) == kModeGeneral;
 }
 
-// Whether the records of a sample() that enqueues `passes` tell when all of its launches have read their operands.  Not behind one
-// launch: pending rows' records are written again.  Nor with a row whose options are rejected: a workgroup of that row that starts late, when
-// the next call's options lie where it reads its own, would serve the row and count itself among that call's workgroups.
-bool outcome_tells_all(const SamplerPasses& passes, const ncnn_moe_sample_params* params, uint32_t rows)
-{
-    return !passes.full_order && !passes.wide_select &&
-        std::all_of(params, params + rows, [](const ncnn_moe_sample_params& p) { return validate_params(p) == NCNN_MOE_ROW_OK; });
-}
-
-// The passes that a batch needs: the host sees the options, so the later ones are enqueued only if some row needs them.
-SamplerPasses passes_of(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab, bool force_general)
+// What a batch needs, from its options: the host sees them, so the later passes are enqueued only if some row needs them.
+struct BatchNeeds
 {
     SamplerPasses passes;
-    passes.full_order = force_general;
+    bool outcome_tells_all = false;
+};
+
+// outcome_tells_all: the rows' records tell when all launches have read their operands.  Not behind one launch: pending rows' records are
+// written again.  Nor with a row whose options are rejected: a workgroup of that row that starts late, when the next call's options lie
+// where it reads its own, would serve the row and count itself among that call's workgroups.
+// (One look a row: 1,024 rows take 5 us with a second one.)
+BatchNeeds needs_of(const ncnn_moe_sample_params* params, uint32_t rows, uint32_t vocab, bool force_general)
+{
     uint32_t wide_rows = 0;
     uint32_t full_order_rows = 0;
+    bool rejected = false;
     for (uint32_t row = 0; row < rows; ++row)
     {
-        const bool beyond_select = row_left_pending(params[row], vocab, kSelectTopK);
-        const bool beyond_fast = !beyond_select && row_left_pending(params[row], vocab, kFastTopK);
-        passes.wide_select = passes.wide_select || beyond_fast;
-        passes.full_order = passes.full_order || beyond_select;
-        wide_rows += beyond_fast ? 1u : 0u;
+        uint32_t effective_k = 0;
+        int status = NCNN_MOE_ROW_OK;
+        const bool beyond_fast = resolve_row_mode(params[row], vocab, kFastTopK, 0, effective_k, status) == kModeGeneral;
+        const bool beyond_select = beyond_fast && effective_k > static_cast<uint32_t>(kSelectTopK);
+        rejected = rejected || status != NCNN_MOE_ROW_OK;
+        wide_rows += beyond_fast && !beyond_select ? 1u : 0u;
         full_order_rows += beyond_select ? 1u : 0u;
     }
+    BatchNeeds needs;
+    needs.passes.full_order = force_general || full_order_rows != 0u;
+    needs.passes.wide_select = wide_rows != 0u;
     // enough rows of each kind for the two passes to be worth the hand-over between two streams
-    passes.side_by_side = wide_rows >= kSideBySideRows && full_order_rows >= kSideBySideRows;
-    return passes;
+    needs.passes.side_by_side = wide_rows >= kSideBySideRows && full_order_rows >= kSideBySideRows;
+    needs.outcome_tells_all = !needs.passes.full_order && !needs.passes.wide_select && !rejected;
+    return needs;
 }
 
 int check_shape(ncnn_moe_hip_sampler* s, int dtype, uint32_t rows, uint32_t vocab)
@@ -1216,9 +1221,10 @@ int ncnn_moe_hip_sampler_sample(
     }
     else if (stop_id_count > 0)
         return fail(s, NCNN_MOE_SAMPLER_INVALID_ARGUMENT, "more stop ids than the handle holds (max(64 * max_rows, max_vocab))");
-    const SamplerPasses passes = passes_of(params, rows, s->logits_vocab, s->force_general != 0);
+    const BatchNeeds needs = needs_of(params, rows, s->logits_vocab, s->force_general != 0);
+    const SamplerPasses& passes = needs.passes;
     const bool full_order = passes.full_order;
-    const bool watched = outcome_tells_all(passes, params, rows);
+    const bool watched = needs.outcome_tells_all;
     const size_t result_words = static_cast<size_t>(rows) * sizeof(ncnn_moe_sample_result) / sizeof(uint32_t);
     if (watched)
         clear_outcome(s->results_host, result_words);
@@ -1681,7 +1687,7 @@ int ncnn_moe_hip_sampler_debug_outcome_watched(const ncnn_moe_sample_params* par
 {
     if (params == nullptr || rows == 0 || vocab == 0)
         return 0;
-    return outcome_tells_all(passes_of(params, rows, vocab, false), params, rows) ? 1 : 0;
+    return needs_of(params, rows, vocab, false).outcome_tells_all ? 1 : 0;
 }
 
 // Which of the handle's first `rows` rows the binned sums finished the last time that they were given them.
