@@ -90,7 +90,9 @@ constexpr uint32_t kBinGrid = 512;               // workgroups of each launch: t
 // 242 and 228, 16 of 400,000 (25,000) 147 and 144.  Where rows have windows as well, most of the call's rows are not these, and the launches that find
 // none cost 2 us each: mixed options, 40 rows of 129,280 132 and 139, 100 143 and 155; windows of 300, 33 of 100,003 38 and 44, 100 of 129,280
 // (64,600) 50 and 57, 256 of 50,257 46 and 52.  A chain has a compute unit to itself: its walks want 220 registers, and at 128, which two
-// workgroups to a compute unit leave, some of them and 200 scalars pass through scratch and lane moves (17 rows of 151,936 131 us so).  More rows
+// workgroups to a compute unit leave, some of them and 200 scalars pass through scratch and lane moves (17 rows of 151,936 131 us so).  Few rows too
+// long for it lose nothing by that: 1 to 16 rows of 330,000 to 4,000,000 in four launches take 0.81 to 1.01 of the time that three walks with 220
+// registers each took (16 x 330,000 176 and 151, 4 x 600,000 231 and 197, 1 x 600,000 175.5 and 176.7).  More rows
 // than compute units would take turns (300 of 16,384 168 and 124).
 constexpr uint32_t kChainGrid = kBinGrid / 2u;
 constexpr uint32_t kChainRows = kChainGrid;
