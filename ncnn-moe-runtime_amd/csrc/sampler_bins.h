@@ -412,6 +412,21 @@ __device__ __forceinline__ uint4 taken_over_vector(const void* base, uint32_t by
     return uint4{v.x, v.y, v.z, v.w};
 }
 
+// (of numbers; the compiler's own make sure first that none of them is a signalling NaN, an instruction each)
+__device__ __forceinline__ float largest_of_three(float a, float b, float c)
+{
+    float result;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(result) : "v"(a), "v"(b), "v"(c));
+    return result;
+}
+
+__device__ __forceinline__ float smallest_of_three(float a, float b, float c)
+{
+    float result;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(result) : "v"(a), "v"(b), "v"(c));
+    return result;
+}
+
 // Kernels (1) to (3) are bound to 64 registers: two workgroups of 1,024 threads share a compute unit then, and the 512
 // workgroups of a launch that many rows fill run at once, not in two rounds (512 rows of 129,280 of mixed options: 17, 26
 // and 32 us before, 14, 22 and 25 us with the bound).
@@ -463,16 +478,42 @@ __device__ __forceinline__ uint4 stats_of_part(const SamplerArgs& a, const BinGr
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
                 raw[k] = *reinterpret_cast<const uint4*>(base + min(at + k * THREADS, last_whole - 1u) * 16u); // (rows below 2^32 bytes)
+            // (as if all were finite, a quarter of the instructions: 512 rows of mixed options 17.4 -> 16.3 us, then the stream of their
+            // 49 MB; a vector behind the last is that one again)
+            float largest_here = largest, smallest_here = smallest;
+            uint32_t twice = 0; // the largest of the bits without their signs, times two
 #pragma unroll
             for (int k = 0; k < kLoads; ++k)
             {
-                if (at + k * THREADS < last_whole)
-                {
-                    float x[kWidth];
-                    Vector::unpack(raw[k], x);
+                float x[kWidth];
+                Vector::unpack(raw[k], x);
 #pragma unroll
-                    for (uint32_t c = 0; c < kWidth; ++c)
-                        take(x[c]);
+                for (uint32_t c = 0; c < kWidth; c += 2u)
+                {
+                    largest_here = largest_of_three(largest_here, x[c], x[c + 1]);
+                    smallest_here = smallest_of_three(smallest_here, x[c], x[c + 1]);
+                    twice = max(max(twice, __float_as_uint(x[c]) << 1), __float_as_uint(x[c + 1]) << 1);
+                }
+            }
+            if (twice < 0xff000000u)
+            {
+                largest = largest_here;
+                smallest = smallest_here;
+                finite += kWidth * min(static_cast<uint32_t>(kLoads), (last_whole - at + THREADS - 1u) / THREADS);
+            }
+            else
+            {
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k)
+                {
+                    if (at + k * THREADS < last_whole)
+                    {
+                        float x[kWidth];
+                        Vector::unpack(raw[k], x);
+#pragma unroll
+                        for (uint32_t c = 0; c < kWidth; ++c)
+                            take(x[c]);
+                    }
                 }
             }
         }
@@ -518,6 +559,23 @@ __global__ __launch_bounds__(kBinThreads, 8) void bin_stats_kernel(BinArgs g)
         __syncthreads();
     }
 }
+
+// Correctly rounded quotients by one divisor: two corrections of dividend x reciprocal, each with its exact remainder (P. Markstein,
+// Computation of elementary functions on the IBM RISC System/6000 processor, 1990: a quotient less than an ulp off, corrected with
+// the remainder times the correctly rounded reciprocal, is the correctly rounded one).  Five instructions instead of the ten and a
+// reciprocal of a division; for numbers whose quotient and remainder are far from the denormal ones, as the bins' terms are: they are
+// 2^-25 to 1, a normaliser is 1 to 2^22, the divisor behind it no less than the first term over the normaliser, 2^-22.
+struct Divisor
+{
+    float value, reciprocal;
+    __device__ __forceinline__ explicit Divisor(float divisor) : value(divisor), reciprocal(1.0f / divisor) {}
+    __device__ __forceinline__ float divide(float dividend) const
+    {
+        const float about = dividend * reciprocal;
+        const float near = __builtin_fmaf(__builtin_fmaf(-about, value, dividend), reciprocal, about);
+        return __builtin_fmaf(__builtin_fmaf(-near, value, dividend), reciprocal, near);
+    }
+};
 
 // ---- (2) the terms, in the row's order, and how many fall into each bin
 // What is known of a row before its sums: the same in each of its parts.
@@ -587,44 +645,61 @@ __device__ __forceinline__ BinRowStart terms_of_part(
             float* terms = bin_terms(a, row);
             const uint32_t terms_bytes = (s.end + 7u) / 8u * 32u;
             const uint32_t first = s.first * 8u / kWidth, last = min(s.last * 8u / kWidth, (s.end + kWidth - 1u) / kWidth);
-            for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
-            {
-                uint4 raw[kLoads];
-#pragma unroll
-                for (int k = 0; k < kLoads; ++k)
+            // Divided by the temperature with corrections (see Divisor) where that is exact: a quotient neither overflows nor, unless it is so small that
+            // the maximum swallows it, comes near the denormal numbers.  (A logit of -inf becomes a NaN on the way: zero as well.)  What bounds the terms is
+            // instructions, 42 an element with divisions and a look at each element's place in the row, 35 so: 12.2 million logits 26.0 -> 23.4 us.
+            const Divisor by(p.temperature);
+            const float outermost = fmaxf(fabsf(largest), fabsf(smallest));
+            const bool corrected = p.temperature >= 0x1p-20f && p.temperature <= 0x1p20f && outermost <= 0x1p60f && fabsf(maximum) >= 0x1p-20f;
+            const auto terms_of = [&](auto quotient) {
+                for (uint32_t at = first + tid; at < last; at += kLoads * THREADS)
                 {
-                    const uint32_t v = min(at + k * THREADS, last - 1u);
-                    raw[k] = *reinterpret_cast<const uint4*>(base + v * 16u); // (rows below 2^32 bytes)
-                }
+                    uint4 raw[kLoads];
 #pragma unroll
-                for (int k = 0; k < kLoads; ++k)
-                {
-                    const uint32_t v = at + k * THREADS;
-                    if (v >= last)
-                        break;
-                    float x[kWidth], t[kWidth];
-                    Vector::unpack(raw[k], x);
-                    const uint32_t position = v * kWidth;
-#pragma unroll
-                    for (uint32_t c = 0; c < kWidth; ++c)
+                    for (int k = 0; k < kLoads; ++k)
                     {
-                        const float argument = x[c] / p.temperature - maximum;
-                        // (a comparison that NaN fails as well)
-                        const bool matters = argument >= kTailArgument && position + c >= s.misalignment && position + c < s.end;
-                        t[c] = matters ? expf_of_small_argument(argument, exp2_table) : 0.0f;
-                        const uint32_t below = kOneBits - __float_as_uint(t[c]);
-                        if (below < kTailDistance)
-                        {
-                            atomicAdd(&bins[below >> shift], 1u);
-                            atomicAdd(&bins[kBins + (below >> shift)], (below & place_mask) >> place_shift);
-                        }
+                        const uint32_t v = min(at + k * THREADS, last - 1u);
+                        raw[k] = *reinterpret_cast<const uint4*>(base + v * 16u); // (rows below 2^32 bytes)
                     }
 #pragma unroll
-                    for (uint32_t c = 0; c < kWidth; c += 4u)
-                        hand_over_vector(near, terms, terms_bytes, (position + c) / 4u,
-                                                 uint4{__float_as_uint(t[c]), __float_as_uint(t[c + 1]), __float_as_uint(t[c + 2]), __float_as_uint(t[c + 3])});
+                    for (int k = 0; k < kLoads; ++k)
+                    {
+                        const uint32_t v = at + k * THREADS;
+                        if (v >= last)
+                            break;
+                        float x[kWidth], t[kWidth];
+                        Vector::unpack(raw[k], x);
+                        const uint32_t position = v * kWidth;
+                        if (position < s.misalignment || position + kWidth > s.end) // (the row's first vector or its last)
+                        {
+#pragma unroll
+                            for (uint32_t c = 0; c < kWidth; ++c)
+                                x[c] = position + c >= s.misalignment && position + c < s.end ? x[c] : -INFINITY;
+                        }
+#pragma unroll
+                        for (uint32_t c = 0; c < kWidth; ++c)
+                        {
+                            const float argument = quotient(x[c]) - maximum;
+                            // (a comparison that NaN fails as well)
+                            t[c] = argument >= kTailArgument ? expf_of_small_argument(argument, exp2_table) : 0.0f;
+                            const uint32_t below = kOneBits - __float_as_uint(t[c]);
+                            if (below < kTailDistance)
+                            {
+                                atomicAdd(&bins[below >> shift], 1u);
+                                atomicAdd(&bins[kBins + (below >> shift)], (below & place_mask) >> place_shift);
+                            }
+                        }
+#pragma unroll
+                        for (uint32_t c = 0; c < kWidth; c += 4u)
+                            hand_over_vector(near, terms, terms_bytes, (position + c) / 4u,
+                                             uint4{__float_as_uint(t[c]), __float_as_uint(t[c + 1]), __float_as_uint(t[c + 2]), __float_as_uint(t[c + 3])});
+                    }
                 }
-            }
+            };
+            if (corrected)
+                terms_of([&](float x) { return by.divide(x); });
+            else
+                terms_of([&](float x) { return x / p.temperature; });
             // (the last group of eight positions of the row may reach a vector further than the row does)
             if (kWidth == 4u && tid == 0 && s.last * 2u > last && last > first)
                 hand_over_vector(near, terms, terms_bytes, last, uint4{0u, 0u, 0u, 0u});
@@ -840,23 +915,6 @@ __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&fro
     }
     return end_of_list;
 }
-
-// Correctly rounded quotients by one divisor: two corrections of dividend x reciprocal, each with its exact remainder (P. Markstein,
-// Computation of elementary functions on the IBM RISC System/6000 processor, 1990: a quotient less than an ulp off, corrected with
-// the remainder times the correctly rounded reciprocal, is the correctly rounded one).  Five instructions instead of the ten and a
-// reciprocal of a division; for numbers whose quotient and remainder are far from the denormal ones, as the bins' terms are: they are
-// 2^-25 to 1, a normaliser is 1 to 2^22, the divisor behind it no less than the first term over the normaliser, 2^-22.
-struct Divisor
-{
-    float value, reciprocal;
-    __device__ __forceinline__ explicit Divisor(float divisor) : value(divisor), reciprocal(1.0f / divisor) {}
-    __device__ __forceinline__ float divide(float dividend) const
-    {
-        const float about = dividend * reciprocal;
-        const float near = __builtin_fmaf(__builtin_fmaf(-about, value, dividend), reciprocal, about);
-        return __builtin_fmaf(__builtin_fmaf(-near, value, dividend), reciprocal, near);
-    }
-};
 
 // Adds the steps of a part's terms to the bins' integers, and puts the terms of listed bins into the list.
 //   entries   per bin: bit 31 the bin is listed and the rest is the next place of this part in the list; bit 30 it takes

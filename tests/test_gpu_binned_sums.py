@@ -72,6 +72,40 @@ def test_draws_and_cuts_at_the_ends():
     parity_util.assert_results_match(gpu, cpu, "f32", "ends")
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,vocab", [(12, 2049), (12, 16411), (300, 4099)])
+def test_quotients_and_finite_counts_at_the_ends_of_their_ranges(dtype, rows, vocab):
+    """Temperatures and logits on both sides of those whose quotients are made with corrections, a maximum next to zero among tiny logits,
+    and rows with NaN, -inf and the largest numbers at their ends and inside, in one launch and in four, in windows and without one."""
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] ends of quotients, %d x %d %s" % (rows, vocab, dtype), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+    params = hip_sampler.make_params(rows, 1.0, 0, 0.95, 0.0)
+    scales = 2.0 ** np.array([0, 0, -19.5, -20.5, 19.5, 20.5, -90, 59, 61, 0, 0, 0], dtype=np.float64)
+    kinds = np.arange(rows) % 12
+    params["temperature"] = np.clip(scales, 2.0 ** -21, 2.0 ** 21)[kinds].astype(np.float32)
+    logits = (logits * scales[kinds][:, None]).astype(np.float32)
+    logits[kinds == 1] -= logits[kinds == 1].max(axis=1, keepdims=True)      # a maximum of zero
+    logits[kinds == 9] = logits[kinds == 9] - logits[kinds == 9].max(axis=1, keepdims=True) + np.float32(2.0 ** -21)
+    logits[kinds == 9, ::5] = np.float32(-1e-39)
+    logits[kinds == 10, ::3] = -np.inf
+    for at in (0, vocab // 2, vocab - 1):
+        logits[kinds == 10, at] = np.nan
+    logits[kinds == 11, 0] = logits[kinds == 11, vocab - 1] = np.float32(-3.0e38)
+    if dtype == "bf16":
+        params["top_k"] = 100
+    else:
+        params["top_k"][rows // 2::2] = 100
+    uniforms = rng.random(rows, dtype=np.float32)
+    data = workloads.float32_to_bf16_bits(logits) if dtype == "bf16" else logits
+    cpu = parity_util.run_oracle(data, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(data)
+        gpu = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, dtype, "ends of quotients")
+
+
 # Both sides of what decides whether the sums are one launch: elements a part (16 parts of 20,000 logits, and 6 of 80,000 where the call has
 # windows), and as many rows as compute units.
 @pytest.mark.parametrize("rows,vocab,windows", [(16, 65537, 0), (17, 65537, 0), (3, 320015, 0), (3, 320016, 0), (256, 4099, 0), (257, 4099, 0),
