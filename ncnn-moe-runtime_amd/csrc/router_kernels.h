@@ -145,12 +145,15 @@ __host__ __device__ inline uint32_t chunk_count_stride(uint32_t experts)
     return (experts + 3u) / 4u * 4u;
 }
 
+constexpr uint32_t kRankedQuads = kWaveSize / 4; // see select_best
+
 // A wave's scratch for the routes of one token.
 struct RouteScratch
 {
     uint64_t candidates[kWaveSize + 4]; // ordered selection score (32 bits), complement of the expert id (32)
     float scores[kWaveSize + 4];        // the candidates' scores
     float selected[kWaveSize + 4];      // the selected scores, in rank order, then zeros
+    uint32_t quads[kRankedQuads];       // the largest key of each four lanes
 };
 
 // This wave's LDS accesses in front of it come before those behind it (a wave's LDS operations run in order: only the
@@ -206,13 +209,43 @@ __device__ __forceinline__ float sequential_sum_by_lanes(const float* row, uint3
     return read_lane(sum, 15);
 }
 
+// The same for calls of many tokens: a lane's row in a chain of its own beside those of other lanes, the next 16 scores on their way while these are added.
+__device__ __forceinline__ float sequential_row_sums_ahead(const float* row_of_lane, uint32_t padded)
+{
+    const float4* quads = reinterpret_cast<const float4*>(row_of_lane);
+    float4 now[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        now[k] = quads[k];
+    float sum = 0.0f;
+#pragma unroll 2
+    for (uint32_t q = 4; q <= padded / 4u; q += 4u)
+    {
+        float4 next[4];
+        const uint32_t ahead = min(q, padded / 4u - 4u);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            next[k] = quads[ahead + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            sum = (((sum + now[k].x) + now[k].y) + now[k].z) + now[k].w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            now[k] = next[k];
+    }
+    return sum;
+}
+
 // ---- select_topk_routes (src/graph/expert_dispatcher.cpp:61-77): the best top_k of a token's experts by (score + bias
 // descending, expert id ascending).  Expert e lives in slot e / 64 of lane e % 64.
-// A threshold with top_k to `most` scores at or above it is searched over the scores' order-preserving bits: from the
-// largest score down in growing steps, then by halving; a step is one comparison per slot, and the counting runs on the
-// scalar unit.  The experts above the threshold are collected in id order and ranked against each other.  Where equal
-// scores leave no such threshold, the lowest ids among the equals are collected.
-// What bounds it: instructions, some 130 per token of 256 experts and 8 routes, where choosing one route per round by
+// A threshold with top_k to `most` scores at or above it: the top_k-th largest of the sixteen numbers that are the largest of four lanes
+// each (a ranking of 16 words by way of LDS); some 11 of 256 scores are at or above that for 8 routes, and top_k are for certain.  With more
+// routes than quads, or too many scores above it (a few experts of one quad hold the best), it is searched over the scores'
+// order-preserving bits: from the largest score down in growing steps, then by halving, where a step is one comparison per slot, and the
+// counting runs on the scalar unit.  The search alone took four steps and more for most tokens (16,384 tokens of 256 experts and 8 routes,
+// softmax, selection 8 us of 27.4; so 4.5 of 23.7).  The experts above the threshold are collected in id order and ranked against each
+// other.  Where equal scores leave no such threshold, the lowest ids among the equals are collected.
+// What bounds it: instructions, some 100 per token of 256 experts and 8 routes, where choosing one route per round by
 // wave-wide maxima took some 500.
 // Up to kRankedExperts experts are ranked against each other at once, by lane reads: the threshold and the trips through LDS
 // cost more there (one token of 8 experts and 2 routes: 6.2 to 6.6 us so, 5.9 to 6.2 ranked; 16 experts are ranked in
@@ -254,7 +287,6 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
             selected_sum += read_lane(my_score, __builtin_ctzll(__builtin_amdgcn_ballot_w64(my_rank == i)));
         return selected_sum;
     }
-    largest = wave_max_u32(largest);
     const auto count_from = [&](uint32_t least) {
         uint32_t count = 0;
 #pragma unroll
@@ -263,31 +295,51 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
         return count;
     };
     const uint32_t most = min(static_cast<uint32_t>(kWaveSize), top_k + top_k / 2u + 8u);
-    uint32_t low = 1u, high = largest + 1u; // as many as wanted from `low` on, too few from `high` on
-    uint32_t step = 1u << 22;               // half a binade
-    uint32_t threshold = largest > step ? largest - step : 1u;
-    uint32_t equals = 0xffffffffu;          // how many scores that equal the threshold are taken
-    for (;;)
+    uint32_t threshold = 0u;
+    uint32_t equals = 0xffffffffu; // how many scores that equal the threshold are taken
+    if (top_k <= kRankedQuads)
     {
-        const uint32_t count = count_from(threshold);
-        if (count >= top_k && count <= most)
-            break;
-        if (count < top_k)
-            high = threshold;
-        else
+        uint32_t of_quad = largest;
+        of_quad = max(of_quad, static_cast<uint32_t>(dpp_move<kDppSwapPairs>(static_cast<int>(of_quad))));
+        of_quad = max(of_quad, static_cast<uint32_t>(dpp_move<kDppSwapHalves>(static_cast<int>(of_quad))));
+        scratch.quads[lane >> 2] = of_quad; // (four lanes, the same number)
+        wave_lds_fence();
+        const uint4 others = *reinterpret_cast<const uint4*>(&scratch.quads[4 * (lane & 3)]);
+        int above = (others.x > of_quad ? 1 : 0) + (others.y > of_quad ? 1 : 0) + (others.z > of_quad ? 1 : 0) + (others.w > of_quad ? 1 : 0);
+        above += dpp_move<kDppSwapPairs>(above);
+        above += dpp_move<kDppSwapHalves>(above);
+        const uint64_t kth = __builtin_amdgcn_ballot_w64(above == static_cast<int>(top_k) - 1);
+        if (kth != 0ull) // (else two quads' largest are the same)
+            threshold = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(of_quad), __builtin_ctzll(kth)));
+    }
+    if (threshold == 0u || count_from(threshold) > most)
+    {
+        largest = wave_max_u32(largest);
+        uint32_t low = max(threshold, 1u), high = largest + 1u; // as many as wanted from `low` on, too few from `high` on
+        uint32_t step = 1u << 22;                               // half a binade
+        threshold = largest - low > step ? largest - step : low + (high - low) / 2u;
+        for (;;)
         {
-            low = threshold;
-            step = 0u;
+            const uint32_t count = count_from(threshold);
+            if (count >= top_k && count <= most)
+                break;
+            if (count < top_k)
+                high = threshold;
+            else
+            {
+                low = threshold;
+                step = 0u;
+            }
+            if (high - low <= 1u)
+            {
+                threshold = low;
+                equals = top_k - count_from(low + 1u);
+                break;
+            }
+            step = step < 0x40000000u ? step * 2u : step;
+            const bool falls = step != 0u && largest - low > step && largest - step < high;
+            threshold = falls ? largest - step : low + (high - low) / 2u;
         }
-        if (high - low <= 1u)
-        {
-            threshold = low;
-            equals = top_k - count_from(low + 1u);
-            break;
-        }
-        step = step < 0x40000000u ? step * 2u : step;
-        const bool falls = step != 0u && largest - low > step && largest - step < high;
-        threshold = falls ? largest - step : low + (high - low) / 2u;
     }
     uint32_t count = 0, equals_before = 0;
 #pragma unroll
@@ -425,8 +477,13 @@ __device__ __forceinline__ void route_token(
 // 13.2 -> 10.5, 16,384 22.1 -> 18.9; 256 and 8, 16,384 28.7 -> 27.2).  More experts hardly share routes, and the counters' way through LDS costs
 // more than it saves (1,024 experts, 257 tokens 22.7 and 22.4, 16,384 76.1 and 75.2 without).
 // Two or four tokens a wave: 0 to 15 % slower from 64 experts on.
-// What bounds it: instructions, some 640 per token of 256 experts under the softmax: 280 for the sum, 110 for the exponentials, 50 for
-// the divisions, 130 for the selection.
+// The softmax's sums are chains of additions in expert order.  Where a compute unit has more than eight tokens (kChainsApart), those of
+// a workgroup's tokens go side by side in the lanes of one wave: 256 additions and 64 reads of LDS for eight tokens, where a token's
+// own wave takes 280 instructions.  With fewer there are instructions to spare, and the wave that all wait for is the slowest part (the kernel
+// alone, 256 experts, a wave each and side by side: 512 tokens 5.4 and 5.7 us, 2,048 5.7 and 6.0, 4,096 7.2 and 6.8, 8,192 10.5 and 9.2,
+// 16,384 17.5 and 15.8).
+// What bounds it: instructions, some 400 per token of 256 experts under the softmax: 110 for the exponentials, 50 for
+// the divisions, 100 for the selection, 40 for its share of the sums.
 //
 // Waves of a workgroup: eight, which add their counts up together (16,384 tokens of 8 experts 14.8 us, with four 16.4).  But four
 // from 257 experts on where that gives every compute unit one at most (1,024 tokens): a token is then so much work that waves two to a SIMD
@@ -435,6 +492,7 @@ __device__ __forceinline__ void route_token(
 constexpr int kBatchWaves = 8;
 constexpr int kFewBatchWaves = 4;
 constexpr uint32_t kFewBatchTokens = 256u * kFewBatchWaves;
+constexpr uint32_t kChainsApart = 256u * kBatchWaves; // tokens
 
 template <int SLOTS, int WAVES>
 __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterArgs r)
@@ -442,7 +500,8 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterA
     constexpr int kThreads = WAVES * kWaveSize;
     constexpr bool kCountsInLds = SLOTS <= 8;
     static_assert(kRouterChunkTokens % WAVES == 0, "a workgroup's tokens are of one chunk");
-    __shared__ __align__(16) float rows[WAVES][SLOTS * kWaveSize];
+    __shared__ __align__(16) float rows[WAVES][SLOTS * kWaveSize + 4]; // (four more: the rows' chains read other banks)
+    __shared__ float sums[WAVES];
     __shared__ __align__(16) RouteScratch scratch[WAVES];
     __shared__ uint32_t workgroup_counts[kCountsInLds ? SLOTS * kWaveSize : 1]; // the workgroup's routes to each expert
     __shared__ uint64_t exp2_table[32];
@@ -474,42 +533,54 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterA
         finite = finite && (static_cast<uint32_t>(s * kWaveSize + lane) >= r.experts || is_finite_f32(score[s]));
         maximum = fmaxf(maximum, score[s]);
     }
-    if (token < r.tokens)
-    {
-        if (__builtin_amdgcn_ballot_w64(!finite) != 0ull)
-        {
-            // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
-            if (lane == 0)
-                atomicOr(&r.error_words[0], 1u);
-        }
-        else
-        {
-            // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
-            float sum = 1.0f;
-            // (past the last expert: 0)
-            const auto each_score = [&](auto score_of) {
+    const bool routed = token < r.tokens && __builtin_amdgcn_ballot_w64(!finite) == 0ull; // (the same in all lanes)
+    // src/graph/expert_dispatcher.cpp:98-102: any non-finite logit of the call fails it
+    if (token < r.tokens && !routed && lane == 0)
+        atomicOr(&r.error_words[0], 1u);
+    // ---- router_scores (src/graph/expert_dispatcher.cpp:40-59)
+    float sum = 1.0f;
+    // (past the last expert: 0)
+    const auto each_score = [&](auto score_of) {
 #pragma unroll
-                for (int s = 0; s < SLOTS; ++s)
-                {
-                    const float of_expert = score_of(score[s]);
-                    score[s] = static_cast<uint32_t>(s * kWaveSize + lane) < r.experts ? of_expert : 0.0f;
-                    rows[wave][s * kWaveSize + lane] = score[s];
-                }
-                wave_lds_fence();
-            };
-            if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
-            {
-                maximum = wave_max(maximum);
-                each_score([&](float x) { return expf_selects(x - maximum, exp2_table); });
-                sum = sequential_sum_by_lanes(rows[wave], (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize, lane);
-            }
-            else if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
-                each_score([&](float x) { return sigmoid_score(x, exp2_table); });
-            else
-                each_score([&](float x) { return sqrt_softplus_score(x, exp2_table); });
-            route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], kCountsInLds ? workgroup_counts : chunk_counts, token, lane);
+        for (int s = 0; s < SLOTS; ++s)
+        {
+            const float of_expert = score_of(score[s]);
+            score[s] = static_cast<uint32_t>(s * kWaveSize + lane) < r.experts ? of_expert : 0.0f;
+            rows[wave][s * kWaveSize + lane] = score[s];
+        }
+    };
+    if (r.score_function == NCNN_MOE_ROUTER_SOFTMAX)
+    {
+        if (routed)
+        {
+            maximum = wave_max(maximum);
+            each_score([&](float x) { return expf_selects(x - maximum, exp2_table); });
+        }
+        if (r.tokens > kChainsApart)
+        {
+            __syncthreads();
+            // (the waves take turns, so that the SIMDs share the chains; a row without routes sums what lies there)
+            if (wave == static_cast<int>((blockIdx.x ^ (blockIdx.x >> 3) ^ (blockIdx.x >> 8)) % WAVES) && lane < WAVES)
+                sums[lane] = sequential_row_sums_ahead(rows[lane], (r.experts + 15u) / 16u * 16u);
+            __syncthreads();
+            sum = sums[wave];
+        }
+        else if (routed)
+        {
+            wave_lds_fence();
+            sum = sequential_sum_by_lanes(rows[wave], (r.experts + kWaveSize - 1u) / kWaveSize * kWaveSize, lane);
         }
     }
+    else if (routed)
+    {
+        if (r.score_function == NCNN_MOE_ROUTER_SIGMOID)
+            each_score([&](float x) { return sigmoid_score(x, exp2_table); });
+        else
+            each_score([&](float x) { return sqrt_softplus_score(x, exp2_table); });
+        wave_lds_fence();
+    }
+    if (routed)
+        route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], kCountsInLds ? workgroup_counts : chunk_counts, token, lane);
     if constexpr (kCountsInLds)
     {
         __syncthreads();
@@ -659,8 +730,19 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
     if (chunk == 0 && tid == 0)
         *r.status = status;
 
+    // Several chunks: a workgroup that has read the counters and the error words counts itself, and places its routes while that is under way.
+    uint32_t finished = 0u;
+    const auto arrive = [&]() {
+        if (tid == 0)
+            finished = __hip_atomic_fetch_add(r.finished_chunks, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     if (status != NCNN_MOE_ROUTER_OK)
     {
+        if constexpr (!FUSED)
+        {
+            __syncthreads();
+            arrive();
+        }
         if (chunk == 0)
         {
             for (uint32_t e = tid; e <= experts; e += kRouterThreads)
@@ -761,6 +843,7 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
                 }
             }
             lds_barrier();
+            arrive();
 #pragma unroll
             for (int j = 0; j < kGroupExpertsPerThread; ++j)
             {
@@ -868,19 +951,14 @@ __device__ __forceinline__ void place_chunk_routes(const RouterArgs& r, GroupSha
         }
     }
 
-    // ---- the last workgroup to get here clears the counters for the next call
-    __syncthreads();
+    // ---- the last workgroup to have read the counters and the error words clears them for the next call
     if (tid == 0)
-    {
-        const uint32_t finished =
-            FUSED ? 0u : __hip_atomic_fetch_add(r.finished_chunks, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         shared.is_last = FUSED || finished == chunks - 1u ? 1u : 0u;
-    }
     __syncthreads();
     if (shared.is_last != 0u)
     {
-        for (uint32_t i = tid; !FUSED && i < chunks * chunk_count_stride(experts); i += kRouterThreads)
-            r.chunk_counts[i] = 0u;
+        for (uint32_t i = tid; !FUSED && i < chunks * (chunk_count_stride(experts) / 4u); i += kRouterThreads)
+            reinterpret_cast<uint4*>(r.chunk_counts)[i] = uint4{0u, 0u, 0u, 0u};
         if (tid == 0)
         {
             r.error_words[0] = 0u;

@@ -58,3 +58,35 @@ def test_few_experts_match_the_oracle(tokens, experts, top_k):
                 for field in ("token_index", "rank"):
                     assert np.array_equal(routes[field], cpu_routes[field]), field
                 assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
+
+
+@pytest.mark.parametrize("tokens", [5, 263, 1030])
+@pytest.mark.parametrize("experts,top_k", [(17, 16), (64, 15), (130, 16), (256, 17), (512, 1), (1024, 16)])
+def test_thresholds_of_quads_match_the_oracle(tokens, experts, top_k):
+    """The threshold is the top_k-th of the sixteen quads' largest (up to sixteen routes) or searched for: the best experts spread over the quads,
+    all in one quad, equal in two of them, and too many above the threshold; then a call with rejected rows, and one more."""
+    rng = np.random.default_rng(tokens * 31 + experts)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    lanes = np.arange(experts) % 64
+    for row in range(tokens):
+        quad = rng.integers(0, 16)
+        if row % 4 == 1:
+            logits[row, lanes // 4 == quad] += np.float32(8)      # one quad holds the best
+        elif row % 4 == 2:
+            logits[row, lanes // 4 != quad] += np.float32(8)      # ... or all but the best
+        elif row % 4 == 3:
+            logits[row] = np.round(logits[row] * 2) / 2           # quads with the same largest
+    print("[case] quads, %d tokens, %d experts, top %d" % (tokens, experts, top_k), flush=True)
+    bad = logits.copy()
+    bad[tokens // 2, experts // 2] = np.nan
+    with contextlib.closing(hip_router.HipRouter(tokens, experts, top_k)) as router:
+        for score in (hip_router.SOFTMAX, hip_router.SIGMOID):
+            cpu_status, cpu_offsets, cpu_routes = oracle_lib.oracle_router_dispatch(logits, top_k, score_function=score)
+            for _ in range(2):
+                status, offsets, routes = router.dispatch(logits, top_k, score_function=score)
+                assert status == cpu_status == 0
+                assert np.array_equal(offsets, cpu_offsets)
+                for field in ("token_index", "rank"):
+                    assert np.array_equal(routes[field], cpu_routes[field]), field
+                assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
+                assert router.dispatch(bad, top_k, score_function=score)[0] == hip_router.STATUS_NON_FINITE_LOGIT
