@@ -7,6 +7,7 @@
 #include "hip_leftover_rows.hip" // (one unit, so that its stamps go to the array that is read)
 #endif
 #include "sampler_verify.h"
+#include "sampler_upload.h"
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
@@ -63,6 +64,13 @@ struct ncnn_moe_hip_sampler
     size_t input_uniforms_offset = 0;
     size_t input_stops_offset = 0;
     uint32_t input_stop_capacity = 0;
+    // uploads of kUploadStaging at most pass through here (sampler_upload.h)
+    uint8_t* upload_host = nullptr; // pinned
+    uint8_t* upload_mapped = nullptr; // the same memory as the device addresses it
+    size_t upload_capacity = 0;
+    uint32_t* upload_done_host = nullptr; // pinned
+    uint32_t* upload_done_mapped = nullptr;
+    uint32_t* upload_arrived = nullptr;
     ncnn_moe_sample_result* results_host = nullptr;   // pinned
     ncnn_moe_sample_result* results_host_device = nullptr; // the same memory as the device addresses it
 
@@ -319,6 +327,16 @@ bool watch_outcome(const void* records, size_t words, std::chrono::steady_clock:
         }
     }
     std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+}
+
+// Whether the runtime does not know the memory: it copies from pinned memory faster than that could be staged (608 KB 19 us).
+bool is_pageable(const void* pointer)
+{
+    hipPointerAttribute_t attributes;
+    if (hipPointerGetAttributes(&attributes, pointer) == hipSuccess)
+        return attributes.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
     return true;
 }
 
@@ -1003,6 +1021,7 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     place(&s->windows.counts, rows * sizeof(uint32_t));
     place(&s->windows.flags, rows * sizeof(uint32_t));
     place(&s->bins.arrivals, rows * kArrivalWords * sizeof(unsigned long long));
+    place(&s->upload_arrived, sizeof(uint32_t));
     const size_t cleared = bytes;
     place(&s->row_epoch, rows * sizeof(uint32_t));
     place(&s->logits, rows * s->logits_stride_f32 * sizeof(float));
@@ -1089,6 +1108,11 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     const size_t input_bytes = s->input_stops_offset + static_cast<size_t>(s->input_stop_capacity) * sizeof(int32_t);
     CREATE_CHECK(hipHostMalloc(&s->input_block_host, input_bytes, hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->input_block_mapped), s->input_block_host, 0));
+    s->upload_capacity = std::min<size_t>(rows * s->logits_stride_f32 * sizeof(float), kUploadStaging);
+    CREATE_CHECK(hipHostMalloc(&s->upload_host, s->upload_capacity, hipHostMallocDefault));
+    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->upload_mapped), s->upload_host, 0));
+    CREATE_CHECK(hipHostMalloc(&s->upload_done_host, sizeof(uint32_t), hipHostMallocDefault));
+    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->upload_done_mapped), s->upload_done_host, 0));
     CREATE_CHECK(hipHostMalloc(&s->results_host, rows * sizeof(ncnn_moe_sample_result), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->results_host_device), s->results_host, 0));
     CREATE_CHECK(hipHostMalloc(&s->verify_input_host, sizeof(ncnn_moe_hip_sampler::VerifyInput), hipHostMallocDefault));
@@ -1126,6 +1150,10 @@ void ncnn_moe_hip_sampler_destroy(ncnn_moe_hip_sampler* s)
         (void)hipFree(s->device_memory);
     if (s->input_block_host != nullptr)
         (void)hipHostFree(s->input_block_host);
+    if (s->upload_host != nullptr)
+        (void)hipHostFree(s->upload_host);
+    if (s->upload_done_host != nullptr)
+        (void)hipHostFree(s->upload_done_host);
     if (s->results_host != nullptr)
         (void)hipHostFree(s->results_host);
     if (s->verify_input_host != nullptr)
@@ -1171,6 +1199,35 @@ int ncnn_moe_hip_sampler_upload_logits(
         return NCNN_MOE_SAMPLER_SUCCESS;
     const size_t element = dtype == NCNN_MOE_LOGITS_F32 ? 4 : 2;
     SAMPLER_HIP_CHECK(s, hipSetDevice(s->device));
+    const size_t row_bytes = static_cast<size_t>(vocab) * element, from_stride = row_stride * element, to_stride = device_stride * element;
+    const size_t bytes = rows * to_stride; // (rows are a multiple of 16 bytes apart there)
+    if (bytes != 0 && bytes <= s->upload_capacity && is_pageable(host_logits))
+    {
+        const size_t pieces = std::min(kUploadPieces, (bytes + kUploadPiece - 1) / kUploadPiece);
+        const size_t each = (bytes / 16 + pieces - 1) / pieces * 16;
+        clear_outcome(s->upload_done_host, 1);
+        for (size_t first = 0; first < bytes; first += each)
+        {
+            const size_t last = std::min(bytes, first + each);
+            for (size_t row = first / to_stride; row * to_stride < last; ++row)
+            {
+                const size_t from = std::max(first, row * to_stride), to = std::min(last, row * to_stride + row_bytes);
+                if (from < to)
+                    std::memcpy(s->upload_host + from, static_cast<const uint8_t*>(host_logits) + row * from_stride + (from - row * to_stride), to - from);
+            }
+            const uint32_t vectors = static_cast<uint32_t>((last - first) / 16);
+            hipLaunchKernelGGL(upload_kernel, dim3((vectors + kUploadThreads * kUploadLoads - 1) / (kUploadThreads * kUploadLoads)), dim3(kUploadThreads), 0, s->stream,
+                               reinterpret_cast<const uint4*>(s->upload_mapped + first), static_cast<uint8_t*>(device_logits) + first, vectors, s->upload_arrived,
+                               last == bytes ? s->upload_done_mapped : nullptr);
+        }
+        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        // (what the stream held in front of the copy has ended when the copy has)
+        if (watch_outcome(s->upload_done_host, 1, std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched)))
+            s->stream_may_run = false;
+        else
+            SAMPLER_HIP_CHECK(s, synchronize(s));
+        return NCNN_MOE_SAMPLER_SUCCESS;
+    }
     SAMPLER_HIP_CHECK(s, hipMemcpy2DAsync(
         device_logits, device_stride * element, host_logits, row_stride * element,
         static_cast<size_t>(vocab) * element, rows, hipMemcpyHostToDevice, s->stream));

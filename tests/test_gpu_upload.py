@@ -1,0 +1,73 @@
+"""ncnn_moe_hip_sampler_upload_logits: what arrives in the handle's buffer is what the host held, word for word, for uploads that are
+one piece and several, end on both sides of a piece and of what the pinned staging holds, and come from rows that are further apart."""
+import numpy as np
+import pytest
+
+import parity_util
+from ncnn_moe_runtime_amd import hip_sampler
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+PIECE = 320 << 10
+STAGING = 4 << 20
+
+
+class _DeviceWords:
+    def __init__(self, pointer, count):
+        self.__cuda_array_interface__ = {"shape": (count,), "typestr": "<i2", "data": (pointer, False), "version": 2}
+
+
+def _in_device(sampler, dtype, rows, vocab, halves):
+    """[rows, vocab] as 16-bit words of the handle's buffer."""
+    pointer, stride = sampler.logits_buffer(dtype, rows, vocab)
+    words = torch.as_tensor(_DeviceWords(pointer, rows * stride * halves), device="cuda:0").cpu().numpy()
+    return words.reshape(rows, stride * halves)[:, :vocab * halves]
+
+
+SHAPES = [(1, 1), (1, 7), (3, 5), (1, PIECE // 4), (1, PIECE // 4 + 1), (2, PIECE // 2 + 3), (5, PIECE // 4 - 1), (16, STAGING // 64), (16, STAGING // 64 + 1), (7, 100003)]
+
+
+@pytest.mark.parametrize("rows,vocab", SHAPES)
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_uploads_arrive_whole(rows, vocab, bf16, pinned):
+    print("[case] upload %d x %d, bf16 %s, pinned %s" % (rows, vocab, bf16, pinned), flush=True)
+    rng = np.random.default_rng(rows * 131 + vocab)
+    dtype = hip_sampler.LOGITS_BF16 if bf16 else hip_sampler.LOGITS_F32
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        for apart in (0, 3):
+            for _ in range(2):
+                held = torch.from_numpy(rng.integers(0, 1 << 15, (rows, (vocab + apart) * (1 if bf16 else 2)), dtype=np.int16))
+                held = held.pin_memory() if pinned else held
+                logits = held.numpy().view(np.uint16 if bf16 else np.float32)
+                sampler.upload_logits(logits, vocab)
+                halves = 1 if bf16 else 2
+                assert np.array_equal(_in_device(sampler, dtype, rows, vocab, halves), held.numpy()[:, :vocab * halves])
+
+
+def test_uploads_and_calls_on_other_streams_in_turn():
+    """Upload, sample on the handle's stream, upload again and sample_device on another one from the handle's buffer."""
+    rows, vocab = 3, 50257
+    rng = np.random.default_rng(5)
+    params = hip_sampler.make_params(rows, 0.8, 20, 0.9, 0.0)
+    uniforms = rng.random(rows, dtype=np.float32)
+    on_device = [torch.from_numpy(x.view(np.uint8).copy()).cuda() for x in (params, uniforms)]
+    results = torch.zeros(rows * 16, dtype=torch.uint8, device="cuda:0")
+    stream = torch.cuda.Stream()
+    with hip_sampler.HipSampler(rows, vocab) as sampler:
+        for turn in range(6):
+            print("[case] uploads in turn, %d" % turn, flush=True)
+            logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            sampler.upload_logits(logits)
+            if turn % 2 == 0:
+                gpu = sampler.sample(params, uniforms)
+            else:
+                pointer, stride = sampler.logits_buffer(hip_sampler.LOGITS_F32, rows, vocab)
+                sampler.sample_device(pointer, hip_sampler.LOGITS_F32, rows, vocab, stride, on_device[0].data_ptr(), on_device[1].data_ptr(), None,
+                                      results.data_ptr(), 0, stream.cuda_stream)
+                stream.synchronize()
+                gpu = results.cpu().numpy().view(hip_sampler.RESULT_DTYPE).reshape(rows)
+            parity_util.assert_results_match(gpu, cpu, "f32", "turn %d" % turn)
