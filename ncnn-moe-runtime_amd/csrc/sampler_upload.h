@@ -3,8 +3,8 @@
 // What bounds it: the host's copy (130 GB/s from its caches, 47 from memory), the link (57 GB/s), and 8 us that a launch and its outcome take.
 // The runtime's own copy of pageable memory stages and pins in an order of its own, us with it and so: 8 KB 14 and 8, 32 KB 24 and 8.7,
 // 128 KB 15 to 61 and 11, 608 KB (a row of 151,936) 29 and 25, out of the host's caches 41 and 29, 2.4 MB 87 and 73, 118 and 86.  An upload and the
-call that samples from it: 1 row of 2,000 40 and 27, of 32,000 41 and 30, of 151,936 55 and 46, 6 of 151,936 154 and 130, 16 of 2,000 176 and 32,
-16 of 32,000 216 and 87.
+// call that samples from it: 1 row of 2,000 40 and 27, of 32,000 41 and 30, of 151,936 55 and 46, 6 of 151,936 154 and 130, 16 of 2,000 176 and 32,
+// 16 of 32,000 216 and 87.
 #ifndef NCNN_MOE_HIP_SAMPLER_UPLOAD_H
 #define NCNN_MOE_HIP_SAMPLER_UPLOAD_H
 
