@@ -68,7 +68,7 @@ struct ncnn_moe_hip_sampler
     uint8_t* upload_host = nullptr; // pinned
     uint8_t* upload_mapped = nullptr; // the same memory as the device addresses it
     size_t upload_capacity = 0;
-    uint32_t* upload_done_host = nullptr; // pinned
+    uint32_t* upload_done_host = nullptr; // behind it
     uint32_t* upload_done_mapped = nullptr;
     uint32_t* upload_arrived = nullptr;
     ncnn_moe_sample_result* results_host = nullptr;   // pinned
@@ -1109,10 +1109,10 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     CREATE_CHECK(hipHostMalloc(&s->input_block_host, input_bytes, hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->input_block_mapped), s->input_block_host, 0));
     s->upload_capacity = std::min<size_t>(rows * s->logits_stride_f32 * sizeof(float), kUploadStaging);
-    CREATE_CHECK(hipHostMalloc(&s->upload_host, s->upload_capacity, hipHostMallocDefault));
+    CREATE_CHECK(hipHostMalloc(&s->upload_host, s->upload_capacity + sizeof(uint32_t), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->upload_mapped), s->upload_host, 0));
-    CREATE_CHECK(hipHostMalloc(&s->upload_done_host, sizeof(uint32_t), hipHostMallocDefault));
-    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->upload_done_mapped), s->upload_done_host, 0));
+    s->upload_done_host = reinterpret_cast<uint32_t*>(s->upload_host + s->upload_capacity); // (rows are whole vectors)
+    s->upload_done_mapped = reinterpret_cast<uint32_t*>(s->upload_mapped + s->upload_capacity);
     CREATE_CHECK(hipHostMalloc(&s->results_host, rows * sizeof(ncnn_moe_sample_result), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->results_host_device), s->results_host, 0));
     CREATE_CHECK(hipHostMalloc(&s->verify_input_host, sizeof(ncnn_moe_hip_sampler::VerifyInput), hipHostMallocDefault));
@@ -1152,8 +1152,6 @@ void ncnn_moe_hip_sampler_destroy(ncnn_moe_hip_sampler* s)
         (void)hipHostFree(s->input_block_host);
     if (s->upload_host != nullptr)
         (void)hipHostFree(s->upload_host);
-    if (s->upload_done_host != nullptr)
-        (void)hipHostFree(s->upload_done_host);
     if (s->results_host != nullptr)
         (void)hipHostFree(s->results_host);
     if (s->verify_input_host != nullptr)
