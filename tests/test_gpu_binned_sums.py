@@ -473,3 +473,23 @@ def test_quotients_of_terms_are_correctly_rounded(exponent):
         again = (((127 - rng.integers(1, 23, some)) << 23) | rng.integers(0, 1 << 23, some)).astype(np.uint32).view(np.float32)
         if exponent >= 0:
             assert np.array_equal(sampler.quotients(quotients, again).view(np.uint32), (quotients / again).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,vocab", [(2, 163839), (2, 163848), (2, 10239), (1, 10249), (260, 4100)])
+def test_steps_at_the_ends_of_their_trips(rows, vocab):
+    """Parts that take one trip of their terms' loads and one element more, in one launch and in four: logits of eighths, whose equal terms and terms
+    half way between two sums reach every kind of bin, beside plain ones."""
+    rng = np.random.default_rng(rows * 7 + vocab)
+    print("[case] trips of steps, %d x %d" % (rows, vocab), flush=True)
+    logits = (rng.standard_normal((rows, vocab)) * 2.5).astype(np.float32)
+    logits[::2] = np.round(logits[::2] * 8) / 8
+    params = hip_sampler.make_params(rows, 1.0, 0, 0.999, 0.0)
+    params["top_p"][1::2] = 1.0
+    uniforms = rng.random(rows, dtype=np.float32)
+    uniforms[-1] = np.float32(0.9999)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+    parity_util.assert_results_match(gpu, cpu, "f32", "trips of steps")
