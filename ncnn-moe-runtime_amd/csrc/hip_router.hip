@@ -233,6 +233,7 @@ int ncnn_moe_hip_router_dispatch_device(
     args.score_function = options->score_function;
     args.renormalize = options->renormalize;
     args.scaling = options->routed_scaling_factor;
+    args.rank_quads = ranks_quads(options->expert_count, options->top_k);
     args.selected_experts = r->selected_experts;
     args.selected_weights = r->selected_weights;
     args.chunk_counts = r->chunk_counts;

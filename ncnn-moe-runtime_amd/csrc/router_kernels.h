@@ -128,6 +128,7 @@ struct RouterArgs
     uint32_t score_function;
     uint32_t renormalize;
     float scaling;
+    uint32_t rank_quads;          // see ranks_quads
     uint32_t* selected_experts;   // [tokens][top_k], rank order
     float* selected_weights;      // [tokens][top_k]
     uint32_t* chunk_counts;       // [chunks][experts] assignments per chunk of 256 tokens and expert, zero at launch
@@ -146,6 +147,15 @@ __host__ __device__ inline uint32_t chunk_count_stride(uint32_t experts)
 }
 
 constexpr uint32_t kRankedQuads = kWaveSize / 4; // see select_best
+
+// Whether the threshold of a token's selection comes from its quads: up to three quarters as many routes as there are quads with experts.  12 routes of 64 experts
+// and more find it there mostly (16,384 tokens of 128 experts, softmax, 24.1 -> 21.3 us, of 16 and 3 routes 16.9 -> 14.4); where nearly every quad has to have its
+// share above it (10 routes of 20 experts, 16 of 64), most rows are searched as well (20.5 -> 21.1).
+__host__ __device__ inline uint32_t ranks_quads(uint32_t experts, uint32_t top_k)
+{
+    const uint32_t quads = experts < 4u * kRankedQuads ? (experts + 3u) / 4u : kRankedQuads;
+    return 4u * top_k <= 3u * quads ? 1u : 0u;
+}
 
 // A wave's scratch for the routes of one token.
 struct RouteScratch
@@ -239,8 +249,8 @@ __device__ __forceinline__ float sequential_row_sums_ahead(const float* row_of_l
 // ---- select_topk_routes (src/graph/expert_dispatcher.cpp:61-77): the best top_k of a token's experts by (score + bias
 // descending, expert id ascending).  Expert e lives in slot e / 64 of lane e % 64.
 // A threshold with top_k to `most` scores at or above it: the top_k-th largest of the sixteen numbers that are the largest of four lanes
-// each (a ranking of 16 words by way of LDS); some 11 of 256 scores are at or above that for 8 routes, and top_k are for certain.  With more
-// routes than quads, or too many scores above it (a few experts of one quad hold the best), it is searched over the scores'
+// each (a ranking of 16 words by way of LDS); some 11 of 256 scores are at or above that for 8 routes, 21 for 12, and top_k are for certain.  With more
+// routes than three quarters of the quads, or too many scores above it (a few experts of one quad hold the best), it is searched over the scores'
 // order-preserving bits: from the largest score down in growing steps, then by halving, where a step is one comparison per slot, and the
 // counting runs on the scalar unit.  The search alone took four steps and more for most tokens (16,384 tokens of 256 experts and 8 routes,
 // softmax, selection 8 us of 27.4; so 4.5 of 23.7).  The experts above the threshold are collected in id order and ranked against each
@@ -295,9 +305,10 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
         return count;
     };
     const uint32_t most = min(static_cast<uint32_t>(kWaveSize), top_k + top_k / 2u + 8u);
-    uint32_t threshold = 0u;
+    uint32_t threshold;
     uint32_t equals = 0xffffffffu; // how many scores that equal the threshold are taken
-    if (top_k <= kRankedQuads)
+    bool search = r.rank_quads == 0u;
+    if (!search)
     {
         uint32_t of_quad = largest;
         of_quad = max(of_quad, static_cast<uint32_t>(dpp_move<kDppSwapPairs>(static_cast<int>(of_quad))));
@@ -309,15 +320,19 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
         above += dpp_move<kDppSwapPairs>(above);
         above += dpp_move<kDppSwapHalves>(above);
         const uint64_t kth = __builtin_amdgcn_ballot_w64(above == static_cast<int>(top_k) - 1);
-        if (kth != 0ull) // (else two quads' largest are the same)
+        search = kth == 0ull; // (two quads' largest are the same)
+        if (!search)
+        {
             threshold = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(of_quad), __builtin_ctzll(kth)));
+            search = count_from(threshold) > most;
+        }
     }
-    if (threshold == 0u || count_from(threshold) > most)
+    if (search)
     {
         largest = wave_max_u32(largest);
-        uint32_t low = max(threshold, 1u), high = largest + 1u; // as many as wanted from `low` on, too few from `high` on
-        uint32_t step = 1u << 22;                               // half a binade
-        threshold = largest - low > step ? largest - step : low + (high - low) / 2u;
+        uint32_t low = 1u, high = largest + 1u; // as many as wanted from `low` on, too few from `high` on
+        uint32_t step = 1u << 22;               // half a binade
+        threshold = largest > step ? largest - step : 1u;
         for (;;)
         {
             const uint32_t count = count_from(threshold);
@@ -481,7 +496,8 @@ __device__ __forceinline__ void route_token(
 // a workgroup's tokens go side by side in the lanes of one wave: 256 additions and 64 reads of LDS for eight tokens, where a token's
 // own wave takes 280 instructions.  With fewer there are instructions to spare, and the wave that all wait for is the slowest part (the kernel
 // alone, 256 experts, a wave each and side by side: 512 tokens 5.4 and 5.7 us, 2,048 5.7 and 6.0, 4,096 7.2 and 6.8, 8,192 10.5 and 9.2,
-// 16,384 17.5 and 15.8).
+// 16,384 17.5 and 15.8).  Up to 64 experts a token's own wave takes 80 instructions, and the choice alone costs its searched rows 1 to 2 % (16,384
+// tokens of 20 experts and 10 routes 20.5, 20.8 and 21.1, of 33 and 12 21.7, 21.9 and 22.4: before the quads, a wave each, side by side).
 // What bounds it: instructions, some 400 per token of 256 experts under the softmax: 110 for the exponentials, 50 for
 // the divisions, 100 for the selection, 40 for its share of the sums.
 //
@@ -556,7 +572,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterA
             maximum = wave_max(maximum);
             each_score([&](float x) { return expf_selects(x - maximum, exp2_table); });
         }
-        if (r.tokens > kChainsApart)
+        if (SLOTS > 1 && r.tokens > kChainsApart)
         {
             __syncthreads();
             // (the waves take turns, so that the SIMDs share the chains; a row without routes sums what lies there)
