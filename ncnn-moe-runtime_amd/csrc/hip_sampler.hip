@@ -1204,7 +1204,10 @@ int ncnn_moe_hip_sampler_upload_logits(
         const size_t pieces = std::min(kUploadPieces, (bytes + kUploadPiece - 1) / kUploadPiece);
         const size_t each = (bytes / 16 + pieces - 1) / pieces * 16;
         clear_outcome(s->upload_done_host, 1);
-        for (size_t first = 0; first < bytes; first += each)
+        (void)hipGetLastError(); // (what an earlier call of this thread left is no error of this one)
+        hipError_t launched = hipSuccess;
+        s->stream_may_run = true; // (until all pieces are known to have ended)
+        for (size_t first = 0; first < bytes && launched == hipSuccess; first += each)
         {
             const size_t last = std::min(bytes, first + each);
             for (size_t row = first / to_stride; row * to_stride < last; ++row)
@@ -1217,8 +1220,14 @@ int ncnn_moe_hip_sampler_upload_logits(
             hipLaunchKernelGGL(upload_kernel, dim3((vectors + kUploadThreads * kUploadLoads - 1) / (kUploadThreads * kUploadLoads)), dim3(kUploadThreads), 0, s->stream,
                                reinterpret_cast<const uint4*>(s->upload_mapped + first), static_cast<uint8_t*>(device_logits) + first, vectors, s->upload_arrived,
                                last == bytes ? s->upload_done_mapped : nullptr);
+            launched = hipGetLastError();
         }
-        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        if (launched != hipSuccess)
+        {
+            // (the pieces in front read the staging memory, which the next upload overwrites)
+            (void)synchronize(s);
+            return hip_fail(s, launched, "upload_kernel");
+        }
         // (what the stream held in front of the copy has ended when the copy has)
         if (watch_outcome(s->upload_done_host, 1, std::chrono::steady_clock::now() + std::chrono::microseconds(kMostMicrosecondsWatched)))
             s->stream_may_run = false;

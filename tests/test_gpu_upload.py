@@ -1,5 +1,6 @@
 """ncnn_moe_hip_sampler_upload_logits: what arrives in the handle's buffer is what the host held, word for word, for uploads that are
-one piece and several, end on both sides of a piece and of what the pinned staging holds, and come from rows that are further apart."""
+one piece and several, end on both sides of a piece and of what the pinned staging holds, and come from rows that are further apart; also
+behind an error that an earlier call left."""
 import numpy as np
 import pytest
 
@@ -71,3 +72,20 @@ def test_uploads_and_calls_on_other_streams_in_turn():
                 stream.synchronize()
                 gpu = results.cpu().numpy().view(hip_sampler.RESULT_DTYPE).reshape(rows)
             parity_util.assert_results_match(gpu, cpu, "f32", "turn %d" % turn)
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 7), (4, PIECE // 4)])
+def test_an_error_that_an_earlier_call_left_is_not_the_uploads(rows, vocab):
+    """A device that there is not leaves an error on the thread; the uploads behind it succeed, and the calls behind them read all rows."""
+    print("[case] upload %d x %d behind an error" % (rows, vocab), flush=True)
+    rng = np.random.default_rng(rows + vocab)
+    params = hip_sampler.make_params(rows, 0.8, min(20, vocab), 0.9, 0.0)
+    uniforms = rng.random(rows, dtype=np.float32)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        for _ in range(3):
+            logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+            assert sampler._lib.hipSetDevice(1 << 20) != 0
+            sampler.upload_logits(logits)
+            assert not sampler.stream_may_run()
+            cpu = parity_util.run_oracle(logits, params, uniforms)
+            parity_util.assert_results_match(sampler.sample(params, uniforms), cpu, "f32", "behind an error")
