@@ -372,6 +372,30 @@ hipError_t settle(ncnn_moe_hip_sampler* s)
     return error;
 }
 
+// A synchronous call that fails behind launches of its own: they read their operands in the handle's pinned memory, which the next call
+// overwrites, so they end first.
+int give_up(ncnn_moe_hip_sampler* s, int rc)
+{
+    if (s->side_stream != nullptr)
+        (void)hipStreamSynchronize(s->side_stream);
+    s->stream_may_run = true; // (until it is known to have ended)
+    (void)synchronize(s);
+    return rc;
+}
+
+// What the launches since the last drop_earlier_errors() came to.
+int check_launches(ncnn_moe_hip_sampler* s)
+{
+    const hipError_t error = hipGetLastError();
+    return error == hipSuccess ? NCNN_MOE_SAMPLER_SUCCESS : hip_fail(s, error, "a kernel launch");
+}
+
+// What an earlier call of this thread left is no error of the launches that follow.
+void drop_earlier_errors()
+{
+    (void)hipGetLastError();
+}
+
 constexpr uint32_t kSideBySideRows = 32; // rows of each kind from which sample() runs the two later passes side by side
 
 // Which kernels a call enqueues.  Rows a pass cannot serve are marked pending and taken by the next.
@@ -544,6 +568,7 @@ int launch_sampler(
     const ncnn_moe_sample_params* params, const float* uniforms, const int32_t* stop_ids,
     ncnn_moe_sample_result* results, DistributionExport export_to, SamplerPasses passes, hipStream_t stream, bool want_filters = false)
 {
+    drop_earlier_errors();
     const bool want_distribution = export_to.count != nullptr;
     SamplerArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -613,8 +638,7 @@ int launch_sampler(
             else
                 hipLaunchKernelGGL(bf16_counting_replay_kernel, dim3(rows), dim3(kSortThreads), 0, stream, a);
         }
-        SAMPLER_HIP_CHECK(s, hipGetLastError());
-        return NCNN_MOE_SAMPLER_SUCCESS;
+        return check_launches(s);
     }
     // fp32 rows whose sort is spread over the GPU are sorted only as far as their terms can move a sum
     // (full_order_cut_kernel); a row whose replay finds that guess too short stays pending, and a second launch of
@@ -798,8 +822,7 @@ int launch_sampler(
         if (partial_sort)
             launch_full_order(a, true);
     }
-    SAMPLER_HIP_CHECK(s, hipGetLastError());
-    return NCNN_MOE_SAMPLER_SUCCESS;
+    return check_launches(s);
 }
 
 // Would a select kernel serving windows up to max_top_k leave the row to a later pass?
@@ -1204,7 +1227,7 @@ int ncnn_moe_hip_sampler_upload_logits(
         const size_t pieces = std::min(kUploadPieces, (bytes + kUploadPiece - 1) / kUploadPiece);
         const size_t each = (bytes / 16 + pieces - 1) / pieces * 16;
         clear_outcome(s->upload_done_host, 1);
-        (void)hipGetLastError(); // (what an earlier call of this thread left is no error of this one)
+        drop_earlier_errors();
         hipError_t launched = hipSuccess;
         s->stream_may_run = true; // (until all pieces are known to have ended)
         for (size_t first = 0; first < bytes && launched == hipSuccess; first += each)
@@ -1296,7 +1319,7 @@ int ncnn_moe_hip_sampler_sample(
         s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
         device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, passes, s->stream);
     if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-        return rc;
+        return give_up(s, rc);
     const auto seen = [s, result_words](auto deadline) { return watch_outcome(s->results_host, result_words, deadline); };
     SAMPLER_HIP_CHECK(s, watched ? wait_for_outcome(s, seen) : synchronize(s));
     if (!full_order)
@@ -1314,7 +1337,7 @@ int ncnn_moe_hip_sampler_sample(
                 s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
                 device_params, device_uniforms, device_stops, s->results_host_device, DistributionExport{}, retry, s->stream);
             if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-                return rc;
+                return give_up(s, rc);
             SAMPLER_HIP_CHECK(s, synchronize(s));
         }
     }
@@ -1379,6 +1402,7 @@ int ncnn_moe_hip_sampler_sample_device_static(
     hipError_t error = hipSetDevice(device);
     if (error != hipSuccess)
         return static_fail(NCNN_MOE_SAMPLER_HIP_ERROR, "hipSetDevice", hipGetErrorString(error));
+    drop_earlier_errors();
     const hipStream_t on = static_cast<hipStream_t>(stream);
     StaticScratchLayout* layout = nullptr;
     {
@@ -1467,7 +1491,7 @@ int ncnn_moe_hip_sampler_distribution(
         s, row_logits, s->logits_dtype, 1, s->logits_vocab, s->logits_stride,
         s->single_params, s->single_uniform, nullptr, s->single_result, single_row_export, distribution_passes, s->stream);
     if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-        return rc;
+        return give_up(s, rc);
     ncnn_moe_sample_result result;
     uint32_t kept = 0;
     SAMPLER_HIP_CHECK(s, hipMemcpyAsync(&result, s->single_result, sizeof(result), hipMemcpyDeviceToHost, s->stream));
@@ -1568,7 +1592,7 @@ int ncnn_moe_hip_sampler_speculative_verify(
             s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
             s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, DistributionExport{}, every_row, s->stream, true);
         if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-            return rc;
+            return give_up(s, rc);
         VerifySumsArgs d = s->verify_sums;
         d.a.logits = s->logits;
         d.a.row_stride = s->logits_stride;
@@ -1589,7 +1613,8 @@ int ncnn_moe_hip_sampler_speculative_verify(
             hipLaunchKernelGGL((verify_residual_kernel<NCNN_MOE_LOGITS_BF16>), dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
         hipLaunchKernelGGL(verify_steps_kernel, dim3(chunks), dim3(kResidualThreads), 0, s->stream, d);
         hipLaunchKernelGGL(verify_draw_kernel, dim3(1), dim3(kResidualThreads), 0, s->stream, d, chunks);
-        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        if (const int launched = check_launches(s); launched != NCNN_MOE_SAMPLER_SUCCESS)
+            return give_up(s, launched);
         SAMPLER_HIP_CHECK(s, await_outcome());
         if (s->verify_output_host->result.status != NCNN_MOE_VERIFY_UNSUPPORTED_WINDOW)
             return take_outcome();
@@ -1601,10 +1626,11 @@ int ncnn_moe_hip_sampler_speculative_verify(
             s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
             s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, export_to, passes, s->stream);
         if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-            return rc;
+            return give_up(s, rc);
         expect_outcome();
         hipLaunchKernelGGL(speculative_verify_kernel, dim3(1), dim3(kVerifyThreads), 0, s->stream, v);
-        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        if (const int launched = check_launches(s); launched != NCNN_MOE_SAMPLER_SUCCESS)
+            return give_up(s, launched);
         SAMPLER_HIP_CHECK(s, await_outcome());
         const ncnn_moe_verify_result& outcome = s->verify_output_host->result;
         const bool row_pending = outcome.status == NCNN_MOE_VERIFY_ROW_ERROR && outcome.row_status == NCNN_MOE_ROW_NEEDS_FULL_ORDER;
@@ -1642,10 +1668,11 @@ int ncnn_moe_hip_sampler_speculative_verify(
             s, s->logits, s->logits_dtype, rows, s->logits_vocab, s->logits_stride,
             s->verify_input_mapped->params, s->verify_input_mapped->row_uniforms, nullptr, s->results, export_to, every_pass, s->stream);
         if (rc != NCNN_MOE_SAMPLER_SUCCESS)
-            return rc;
+            return give_up(s, rc);
         expect_outcome();
         hipLaunchKernelGGL(speculative_verify_dense_kernel, dim3(1), dim3(kReplayThreads), 0, s->stream, d);
-        SAMPLER_HIP_CHECK(s, hipGetLastError());
+        if (const int launched = check_launches(s); launched != NCNN_MOE_SAMPLER_SUCCESS)
+            return give_up(s, launched);
         SAMPLER_HIP_CHECK(s, await_outcome());
     }
     return take_outcome();
