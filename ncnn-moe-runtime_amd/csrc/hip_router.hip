@@ -101,6 +101,7 @@ void launch_select(const RouterArgs& args, hipStream_t stream)
 
 int enqueue(ncnn_moe_hip_router* r, const RouterArgs& args, hipStream_t stream)
 {
+    (void)hipGetLastError(); // (what an earlier call of this thread left is no error of these launches)
     const uint32_t slots = (args.experts + kWaveSize - 1) / kWaveSize;
     if (slots <= 1)
         launch_select<1>(args, stream);
@@ -275,7 +276,10 @@ int ncnn_moe_hip_router_dispatch(
         explicit_expert_ids != nullptr ? r->explicit_ids : nullptr, r->expert_offsets, r->routes, r->status, &host_status,
         r->stream);
     if (rc != NCNN_MOE_ROUTER_SUCCESS)
+    {
+        (void)hipStreamSynchronize(r->stream); // (the caller's operands may be read until then)
         return rc;
+    }
     ROUTER_HIP_CHECK(r, hipMemcpyAsync(r->host_status, r->status, sizeof(uint32_t), hipMemcpyDeviceToHost, r->stream));
     ROUTER_HIP_CHECK(r, hipMemcpyAsync(expert_offsets, r->expert_offsets, (static_cast<size_t>(options->expert_count) + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, r->stream));
     ROUTER_HIP_CHECK(r, hipMemcpyAsync(routes, r->routes, assignments * sizeof(ncnn_moe_expert_route), hipMemcpyDeviceToHost, r->stream));

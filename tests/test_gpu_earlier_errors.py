@@ -1,11 +1,13 @@
 """An error that an earlier, unrelated call left on the thread is no error of the calls behind it: they succeed, their results are right, and so are
 those of the calls that follow."""
+import contextlib
+
 import numpy as np
 import pytest
 
 import oracle_lib
 import parity_util
-from ncnn_moe_runtime_amd import hip_sampler
+from ncnn_moe_runtime_amd import hip_router, hip_sampler
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +93,20 @@ def test_device_entries():
             _leave_an_error(sampler._lib)
             assert hip_sampler.sample_device_static(0, pointers[0], hip_sampler.LOGITS_F32, rows, vocab, vocab, pointers[1], pointers[2], None, results.data_ptr(), stream.cuda_stream) == 0
             check("sample_device_static")
+
+
+@pytest.mark.parametrize("tokens", [40, 600])
+def test_router(tokens):
+    experts, top_k = 64, 6
+    rng = np.random.default_rng(tokens)
+    with contextlib.closing(hip_router.HipRouter(tokens, experts, top_k)) as router:
+        for turn in range(2):
+            print("[case] router behind an error, %d tokens, turn %d" % (tokens, turn), flush=True)
+            logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+            cpu_status, cpu_offsets, cpu_routes = oracle_lib.oracle_router_dispatch(logits, top_k)
+            _leave_an_error(hip_router.load_library())
+            status, offsets, routes = router.dispatch(logits, top_k)
+            assert status == cpu_status == 0 and np.array_equal(offsets, cpu_offsets)
+            for field in ("token_index", "rank"):
+                assert np.array_equal(routes[field], cpu_routes[field]), field
+            assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
