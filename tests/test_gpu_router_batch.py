@@ -60,11 +60,32 @@ def test_few_experts_match_the_oracle(tokens, experts, top_k):
                 assert np.array_equal(routes["weight"].view(np.uint32), cpu_routes["weight"].view(np.uint32))
 
 
-@pytest.mark.parametrize("tokens", [5, 263, 1030])
-@pytest.mark.parametrize("experts,top_k", [(17, 16), (64, 15), (130, 16), (256, 17), (512, 1), (1024, 16)])
+def _thresholds(logits, top_k):
+    """Where the kernels find each row's threshold: "quads", or by the search, since the rule asks for that ("searched"), two quads' largest are
+    the same ("tied") or too many experts lie above it ("many")."""
+    experts = logits.shape[1]
+    with_experts = min((experts + 3) // 4, 16)
+    if 4 * top_k > 3 * with_experts:
+        return ["searched"] * len(logits)
+    of_quad = np.arange(experts) % 64 // 4
+    largest = np.full((len(logits), 16), -np.inf, dtype=np.float32)
+    for quad in range(with_experts):
+        largest[:, quad] = logits[:, of_quad == quad].max(axis=1)
+    ways = []
+    for row, above in enumerate((largest[:, None, :] > largest[:, :, None]).sum(axis=2)):
+        kth = np.nonzero(above == top_k - 1)[0]
+        most = min(64, top_k + top_k // 2 + 8)
+        ways.append("tied" if kth.size == 0 else "many" if (logits[row] >= largest[row, kth[0]]).sum() > most else "quads")
+    return ways
+
+
+@pytest.mark.parametrize("tokens", [5, 263, 1030, 2111])
+@pytest.mark.parametrize("experts,top_k", [(17, 16), (64, 15), (130, 16), (256, 17), (512, 1), (1024, 16), (17, 3), (17, 4), (33, 6), (64, 12), (64, 13),
+                                           (65, 12), (130, 12), (256, 8), (256, 12), (512, 5), (1024, 2), (1024, 12)])
 def test_thresholds_of_quads_match_the_oracle(tokens, experts, top_k):
-    """The threshold is the top_k-th of the sixteen quads' largest (up to sixteen routes) or searched for: the best experts spread over the quads,
-    all in one quad, equal in two of them, and too many above the threshold; then a call with rejected rows, and one more."""
+    """The threshold is the top_k-th of the sixteen quads' largest (up to three quarters as many routes as there are quads with experts) or searched for:
+    the best experts spread over the quads, all in one quad, equal in two of them, and too many above the threshold; then a call with rejected rows, and one
+    more.  Above 2,048 tokens the softmax's sums of a workgroup's rows go side by side."""
     rng = np.random.default_rng(tokens * 31 + experts)
     logits = rng.standard_normal((tokens, experts)).astype(np.float32)
     lanes = np.arange(experts) % 64
@@ -77,6 +98,13 @@ def test_thresholds_of_quads_match_the_oracle(tokens, experts, top_k):
         elif row % 4 == 3:
             logits[row] = np.round(logits[row] * 2) / 2           # quads with the same largest
     print("[case] quads, %d tokens, %d experts, top %d" % (tokens, experts, top_k), flush=True)
+    if tokens >= 263:
+        ways = _thresholds(logits, top_k)
+        if 4 * top_k > 3 * min((experts + 3) // 4, 16):
+            assert set(ways) == {"searched"}
+        else:
+            assert ways[::4].count("quads") > ways[::4].count("many") and (top_k == 1 or "tied" in ways[3::4])
+            assert experts < 256 or top_k == 1 or set(ways[1::4]) == {"many"}
     bad = logits.copy()
     bad[tokens // 2, experts // 2] = np.nan
     with contextlib.closing(hip_router.HipRouter(tokens, experts, top_k)) as router:
