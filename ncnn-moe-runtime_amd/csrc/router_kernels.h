@@ -157,14 +157,17 @@ __host__ __device__ inline uint32_t ranks_quads(uint32_t experts, uint32_t top_k
     return 4u * top_k <= 3u * quads ? 1u : 0u;
 }
 
-// A wave's scratch for the routes of one token.
-struct RouteScratch
+// A wave's scratch for the routes of one token.  Its members are read in vectors of 16 bytes.
+struct alignas(16) RouteScratch
 {
     uint64_t candidates[kWaveSize + 4]; // ordered selection score (32 bits), complement of the expert id (32)
     float scores[kWaveSize + 4];        // the candidates' scores
     float selected[kWaveSize + 4];      // the selected scores, in rank order, then zeros
     uint32_t quads[kRankedQuads];       // the largest key of each four lanes
 };
+static_assert(offsetof(RouteScratch, candidates) % 16 == 0 && offsetof(RouteScratch, selected) % 16 == 0 && offsetof(RouteScratch, quads) % 16 == 0 &&
+                  sizeof(RouteScratch) % 16 == 0,
+              "vector reads of a token's scratch");
 
 // This wave's LDS accesses in front of it come before those behind it (a wave's LDS operations run in order: only the
 // compiler has to keep it).
@@ -623,6 +626,7 @@ struct RouterShared
     RouteScratch scratch[kStagedTokensPerBlock];
     uint64_t exp2_table[32];
 };
+static_assert(offsetof(RouterShared, scores) % 16 == 0 && offsetof(RouterShared, scratch) % 16 == 0, "vector reads of the tokens' scores and scratch");
 
 __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterShared& shared, uint32_t first_token)
 {
