@@ -693,7 +693,7 @@ __device__ __forceinline__ void stage_token_scores(const RouterArgs& r, RouterSh
 // expert); one workgroup per chunk then places its chunk's routes:
 //   position = routes of lower experts (all chunks) + this expert's routes in earlier chunks
 //              + this expert's routes earlier in the chunk.
-// The last workgroup to finish returns the scratch counters to zero for the next call.
+// The last workgroup to have read the scratch counters, perhaps while others place their routes, returns them to zero for the next call.
 struct GroupShared
 {
     uint32_t wave_base[kRouterWavesPerBlock][NCNN_MOE_ROUTER_MAX_EXPERTS];
