@@ -79,7 +79,11 @@ void launch_select(const RouterArgs& args, hipStream_t stream)
     }
     const auto batch = [&](auto waves) {
         constexpr int kWaves = decltype(waves)::value;
-        hipLaunchKernelGGL((router_batch_kernel<SLOTS, kWaves>), dim3((args.tokens + kWaves - 1u) / kWaves), dim3(kWaves * kWaveSize), 0, stream, args);
+        const dim3 grid((args.tokens + kWaves - 1u) / kWaves), threads(kWaves * kWaveSize);
+        if (args.rank_quads != 0u)
+            hipLaunchKernelGGL((router_batch_kernel<SLOTS, kWaves, true>), grid, threads, 0, stream, args);
+        else
+            hipLaunchKernelGGL((router_batch_kernel<SLOTS, kWaves, false>), grid, threads, 0, stream, args);
     };
     // (see kBatchWaves)
     bool few_waves = SLOTS > 8;

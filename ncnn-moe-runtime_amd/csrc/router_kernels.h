@@ -268,8 +268,8 @@ __device__ __forceinline__ float sequential_row_sums_ahead(const float* row_of_l
 constexpr uint32_t kRankedExperts = 8;
 
 template <int SLOTS>
-__device__ __forceinline__ float select_best(const RouterArgs& r, const float (&score)[SLOTS], const float (&bias)[SLOTS], RouteScratch& scratch,
-                                             int lane, uint32_t& my_expert, uint32_t& my_rank, float& my_score)
+__device__ __forceinline__ float select_best(const RouterArgs& r, bool rank_quads, const float (&score)[SLOTS], const float (&bias)[SLOTS],
+                                             RouteScratch& scratch, int lane, uint32_t& my_expert, uint32_t& my_rank, float& my_score)
 {
     const uint32_t top_k = r.top_k;
     uint32_t key[SLOTS];
@@ -310,7 +310,7 @@ __device__ __forceinline__ float select_best(const RouterArgs& r, const float (&
     const uint32_t most = min(static_cast<uint32_t>(kWaveSize), top_k + top_k / 2u + 8u);
     uint32_t threshold;
     uint32_t equals = 0xffffffffu; // how many scores that equal the threshold are taken
-    bool search = r.rank_quads == 0u;
+    bool search = !rank_quads;
     if (!search)
     {
         uint32_t of_quad = largest;
@@ -433,7 +433,8 @@ __device__ __forceinline__ bool take_explicit(const RouterArgs& r, const float* 
 // e / 64 of lane e % 64 (zeros past the last expert), and `counts` counts the routes to each expert.
 template <int SLOTS, bool FUSED>
 __device__ __forceinline__ void route_token(
-    const RouterArgs& r, const float* scores, const float (&held)[SLOTS], float divisor, RouteScratch& scratch, uint32_t* counts, uint32_t token, int lane)
+    const RouterArgs& r, bool rank_quads, const float* scores, const float (&held)[SLOTS], float divisor, RouteScratch& scratch, uint32_t* counts, uint32_t token,
+    int lane)
 {
     uint32_t my_expert, my_rank;
     float my_score, selected_sum;
@@ -458,7 +459,7 @@ __device__ __forceinline__ void route_token(
             for (int s = 0; s < SLOTS; ++s)
                 score[s] = score[s] / divisor;
         }
-        selected_sum = select_best<SLOTS>(r, score, bias, scratch, lane, my_expert, my_rank, my_score);
+        selected_sum = select_best<SLOTS>(r, rank_quads, score, bias, scratch, lane, my_expert, my_rank, my_score);
     }
     // ---- src/graph/expert_dispatcher.cpp:144-150
     if (r.renormalize != 0u && selected_sum <= 0.0f)
@@ -504,6 +505,10 @@ __device__ __forceinline__ void route_token(
 // What bounds it: instructions, some 400 per token of 256 experts under the softmax: 110 for the exponentials, 50 for
 // the divisions, 100 for the selection, 40 for its share of the sums.
 //
+// RANK_QUADS: ranks_quads' answer.  Decided inside the kernel it cost the calls that search up to 2 % (16,384 tokens, softmax and sigmoid: of 20 experts and
+// 10 routes 20.5 and 17.3 without quads, 20.7 and 17.6 decided inside, 20.65 and 17.5 so; of 12 and 9 20.4 and 18.2, 20.7 and 18.4, 20.5 and 18.3; of 16 and 8
+// 19.1 and 16.0, 19.4 and 16.3, 19.25 and 16.15).
+//
 // Waves of a workgroup: eight, which add their counts up together (16,384 tokens of 8 experts 14.8 us, with four 16.4).  But four
 // from 257 experts on where that gives every compute unit one at most (1,024 tokens): a token is then so much work that waves two to a SIMD
 // wait for each other (512 experts, sqrt softplus, 257 tokens 16.6 and 16.0, 1,024 17.3 and 16.4; 1,536 17.5 and 17.7), and from 513 on always
@@ -513,7 +518,7 @@ constexpr int kFewBatchWaves = 4;
 constexpr uint32_t kFewBatchTokens = 256u * kFewBatchWaves;
 constexpr uint32_t kChainsApart = 256u * kBatchWaves; // tokens
 
-template <int SLOTS, int WAVES>
+template <int SLOTS, int WAVES, bool RANK_QUADS>
 __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterArgs r)
 {
     constexpr int kThreads = WAVES * kWaveSize;
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void router_batch_kernel(RouterA
         wave_lds_fence();
     }
     if (routed)
-        route_token<SLOTS, false>(r, rows[wave], score, sum, scratch[wave], kCountsInLds ? workgroup_counts : chunk_counts, token, lane);
+        route_token<SLOTS, false>(r, RANK_QUADS, rows[wave], score, sum, scratch[wave], kCountsInLds ? workgroup_counts : chunk_counts, token, lane);
     if constexpr (kCountsInLds)
     {
         __syncthreads();
@@ -1017,7 +1022,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_select_kernel(RouterArg
         {
             const float sum = r.score_function == NCNN_MOE_ROUTER_SOFTMAX ? sequential_row_sums(shared.scores[wave], (r.experts + 15u) / 16u * 16u) : 1.0f;
             const float none[SLOTS] = {};
-            route_token<SLOTS, true>(r, shared.scores[wave], none, sum, shared.scratch[wave], nullptr, token, lane);
+            route_token<SLOTS, true>(r, r.rank_quads != 0u, shared.scores[wave], none, sum, shared.scratch[wave], nullptr, token, lane);
         }
     }
     // this workgroup's routes (written through), counts and error words (atomics) have landed once
