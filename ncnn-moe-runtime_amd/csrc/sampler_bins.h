@@ -1100,30 +1100,16 @@ __device__ __forceinline__ uint4 sum_of_part(
         const auto collect = [&](uint32_t first_vector, uint32_t (&all)[4], uint32_t (&in_front)[4]) {
             uint32_t* const counts = g.counts + static_cast<size_t>(slot * grid.parts) * 2u * kBins;
             const uint32_t bytes = grid.parts * 2u * kBins * 4u;
-            constexpr uint32_t kTogether = ACROSS ? kMaxBinParts : kPartsAtATime;
-            for (uint32_t first = 0; first < grid.parts; first += kTogether)
+            // (four parts' at a time: all sixteen's, in fours where a row has fewer parts, gave long rows nothing, and the code made every short one wait: 3 rows
+            // of 600 28.2 us so and 29.0, 5 of 5,000 37.5 and 38.4, 60 of 4,000 37.9 and 38.8, 8 of 151,936 86.9 and 87.4)
+            for (uint32_t first = 0; first < grid.parts; first += kPartsAtATime)
             {
-                uint4 of_part[kTogether];
-                // (all of a long row's together, where there are registers: 8 x 151,936 92.9 -> 90.3 us with the steps' change; a short one's two parts do not pay for
-                // sixteen: 3 x 2,500 37.3 us, 38.7 with sixteen, 37.6 so.  Two copies of the loop, one a way, cost the long rows all of it)
+                uint4 of_part[kPartsAtATime];
 #pragma unroll
-                for (uint32_t some = 0; some < kTogether; some += kPartsAtATime)
-                {
-                    if (some == 0u || some < grid.parts)
-                    {
+                for (uint32_t k = 0; k < kPartsAtATime; ++k)
+                    of_part[k] = taken_over_vector<ACROSS>(counts, bytes, min(first + k, grid.parts - 1u) * 2u * kBinQuads + first_vector);
 #pragma unroll
-                        for (uint32_t k = some; k < some + kPartsAtATime; ++k)
-                            of_part[k] = taken_over_vector<ACROSS>(counts, bytes, min(first + k, grid.parts - 1u) * 2u * kBinQuads + first_vector);
-                    }
-                    else
-                    {
-#pragma unroll
-                        for (uint32_t k = some; k < some + kPartsAtATime; ++k)
-                            of_part[k] = uint4{0u, 0u, 0u, 0u};
-                    }
-                }
-#pragma unroll
-                for (uint32_t k = 0; k < kTogether; ++k)
+                for (uint32_t k = 0; k < kPartsAtATime; ++k)
                 {
                     const uint32_t some = first + k < grid.parts ? 0xffffffffu : 0u;
                     const uint32_t some_before = first + k < grid.part ? 0xffffffffu : 0u;
