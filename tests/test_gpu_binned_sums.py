@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import parity_util
+import test_gpu_speculative as speculative
 from ncnn_moe_runtime_amd import hip_sampler, workloads
 
 pytestmark = pytest.mark.gpu
@@ -75,8 +76,9 @@ def test_draws_and_cuts_at_the_ends():
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("rows,vocab", [(12, 2049), (12, 16411), (300, 4099)])
 def test_quotients_and_finite_counts_at_the_ends_of_their_ranges(dtype, rows, vocab):
-    """Temperatures and logits on both sides of those whose quotients are made with corrections, a maximum next to zero among tiny logits,
-    and rows with NaN, -inf and the largest numbers at their ends and inside, in one launch and in four, in windows and without one."""
+    """Temperatures on both sides of those whose quotients are made with corrections, a maximum next to zero among tiny logits, and rows with NaN,
+    -inf and the largest numbers at their ends and inside, in one launch and in four, fp32 rows in windows and without one, bf16 rows in windows (the limits of
+    logits and maxima, and bf16 rows without a window: the tests behind this one)."""
     rng = np.random.default_rng(rows + vocab)
     print("[case] ends of quotients, %d x %d %s" % (rows, vocab, dtype), flush=True)
     logits = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
@@ -104,6 +106,101 @@ def test_quotients_and_finite_counts_at_the_ends_of_their_ranges(dtype, rows, vo
         sampler.upload_logits(data)
         gpu = sampler.sample(params, uniforms)
     parity_util.assert_results_match(gpu, cpu, dtype, "ends of quotients")
+
+
+# Terms are made with corrected quotients for temperatures of 2^-20 to 2^20 where no logit is beyond 2^60 and the maximum is 2^-20 at least: a row for each
+# side of each limit, its logits ordinary ones but for those that the limit is about.  `below` and `above`: the neighbours in the row's type.
+LIMIT_KINDS = ["ordinary", "logit 2^60", "logit above 2^60", "maximum 2^-20", "maximum below 2^-20", "maximum above 2^-20", "ends"]
+
+
+def _limit_row(rng, kind, vocab, temperature, spread, below, above):
+    row = (rng.standard_normal(vocab) * spread * temperature).astype(np.float32)
+    if kind.startswith("logit"):
+        limit = np.float32(2.0 ** 60)
+        row[vocab // 3] = -(limit if kind == "logit 2^60" else above(limit))
+    elif kind.startswith("maximum"):
+        # (the maximum is the largest logit by the temperature, which is a power of two in these rows)
+        limit = np.float32(2.0 ** -20) * np.float32(temperature)
+        row = -np.abs(row) - np.float32(temperature) * np.float32(0.01)
+        row[::997] = np.float32(-1e-39)  # (some hundred: rows of thousands of equal terms, which these all are to the maximum, are sorted)
+        row[1::997] = np.float32(2.0 ** -75)
+        row[vocab // 3] = below(limit) if "below" in kind else above(limit) if "above" in kind else limit
+    elif kind == "ends":
+        row[1::7] = -np.inf
+        row[0] = row[vocab // 2] = row[-1] = np.nan
+        row[2] = row[-2] = np.float32(-2.0 ** 60)
+    return row
+
+
+def _float_below(x):
+    return np.nextafter(np.float32(x), np.float32(0))
+
+
+def _float_above(x):
+    return np.nextafter(np.float32(x), np.float32(np.inf))
+
+
+# (one launch, and four)
+@pytest.mark.parametrize("rows,vocab", [(49, 4099), (5, 16411), (294, 2053)])
+def test_quotients_at_the_limits_of_logits_and_maxima(rows, vocab):
+    rng = np.random.default_rng(rows + vocab)
+    print("[case] limits of quotients, %d x %d" % (rows, vocab), flush=True)
+    temperatures = [1.0, 0.7, 1.3 * 2.0 ** 19, 2.0 ** 20, _float_above(2.0 ** 20), 2.0 ** -20, _float_below(2.0 ** -20)]
+    logits = np.empty((rows, vocab), dtype=np.float32)
+    params = hip_sampler.make_params(rows, 1.0, 0, 0.999, 0.0)
+    for row in range(rows):
+        kind = LIMIT_KINDS[row % 7]
+        temperature = np.float32(2.0 ** (row // 7 % 3 * 9) if kind.startswith("maximum") else temperatures[row // 7 % 7])
+        params["temperature"][row] = temperature
+        params["top_p"][row] = (0.9, 0.999, 1.0)[row // 49 % 3]
+        logits[row] = _limit_row(rng, kind, vocab, temperature, 2.0, _float_below, _float_above)
+    uniforms = rng.random(rows, dtype=np.float32)
+    cpu = parity_util.run_oracle(logits, params, uniforms)
+    assert (cpu["kept_count"] > 100).all()  # (the rows' sums are of many terms)
+    with hip_sampler.HipSampler(rows, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        sampler.upload_logits(logits)
+        gpu = sampler.sample(params, uniforms)
+        served = sampler.binned_rows(rows)
+    parity_util.assert_results_match(gpu, cpu, "f32", "limits of quotients")
+    assert served.sum() >= rows - 1 - rows // 5, (served, rows)
+
+
+# bf16 rows without a window come to these kernels by the verification.  (One launch, and four: parts of more than 20,000 logits.)
+@pytest.mark.parametrize("drafts,vocab", [(3, 4099), (1, 320103)])
+@pytest.mark.parametrize("temperature", [1.0, 0.7, 1.3 * 2.0 ** 19, 2.0 ** 20, 2.0 ** 21, 2.0 ** -20, 2.0 ** -21])
+def test_quotients_of_bf16_rows_at_their_limits(drafts, vocab, temperature):
+    rng = np.random.default_rng(drafts + vocab)
+    options = dict(temperature=temperature, top_p=0.999)
+    step = 2.0 ** -7
+
+    def below(x):
+        return np.float32(x) * np.float32(1 - step / 2)
+
+    def above(x):
+        return np.float32(x) * np.float32(1 + step)
+
+    def rounded(x):
+        return workloads.bf16_bits_to_float32(workloads.float32_to_bf16_bits(x))
+
+    kinds = LIMIT_KINDS if np.log2(temperature) % 1 == 0 else [kind for kind in LIMIT_KINDS if not kind.startswith("maximum")]
+    with hip_sampler.HipSampler(2 * drafts + 1, vocab, testing=True) as sampler:
+        sampler.binned_sums(True)
+        served = 0
+        for kind in kinds:
+            print("[case] limits of bf16 quotients, %d drafts over %d, temperature %g, %s" % (drafts, vocab, temperature, kind), flush=True)
+            target = rounded(np.stack([_limit_row(rng, kind, vocab, temperature, 2.0, below, above) for _ in range(drafts + 1)]))
+            noise = 1 + (0.1 * rng.standard_normal((drafts, vocab))).astype(np.float32)
+            draft = target[:drafts] * np.where(np.abs(target[:drafts]) > 2.0 ** 50, 1, noise).astype(np.float32)
+            if kind.startswith("maximum"):
+                draft[:, vocab // 3] = target[:drafts, vocab // 3]
+            draft = rounded(draft)
+            proposed = speculative._propose(rng, draft, options)
+            uniforms = rng.random(drafts + 1, dtype=np.float32)
+            speculative._compare(sampler, target, draft, proposed, uniforms, kind, bf16=True, **options)
+            served += int(sampler.filtered_rows(2 * drafts + 1).sum())
+    # (rows of hundreds of thousands of bf16 logits hold so many equal ones that some are left to the sort)
+    assert served >= (2 * drafts + 1) * len(kinds) // 2, served
 
 
 # Both sides of what decides whether the sums are one launch: elements a part (16 parts of 20,000 logits, and 6 of 80,000 where the call has
