@@ -572,9 +572,11 @@ def test_quotients_of_terms_are_correctly_rounded(exponent):
             assert np.array_equal(sampler.quotients(quotients, again).view(np.uint32), (quotients / again).view(np.uint32))
 
 
-@pytest.mark.parametrize("rows,vocab", [(2, 163839), (2, 163848), (2, 10239), (1, 10249), (260, 4100)])
+# (a trip of the chain's loads is 8,192 terms, here a sixteenth of the row's; of the four launches' 16,384 in the sum and 8,192 in the walks)
+@pytest.mark.parametrize("rows,vocab", [(2, 163839), (2, 163848), (2, 10239), (1, 10249), (260, 4100), (2, 131072), (2, 131080), (260, 8192), (260, 8200),
+                                        (260, 16384), (260, 16392)])
 def test_steps_at_the_ends_of_their_trips(rows, vocab):
-    """Parts that take one trip of their terms' loads and one element more, in one launch and in four: logits of eighths, whose equal terms and terms
+    """Parts that take one trip of their terms' loads and one group of eight more, in one launch and in four: logits of eighths, whose equal terms and terms
     half way between two sums reach every kind of bin, beside plain ones."""
     rng = np.random.default_rng(rows * 7 + vocab)
     print("[case] trips of steps, %d x %d" % (rows, vocab), flush=True)
