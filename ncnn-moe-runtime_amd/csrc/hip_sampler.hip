@@ -48,6 +48,7 @@ struct ncnn_moe_hip_sampler
     bool captured = false;       // a sample_device call has been captured: its replays are ordered behind nothing here
 
     void* device_memory = nullptr; // every device buffer below
+    uint8_t* pinned_memory = nullptr; // every pinned one but upload_host
     void* logits = nullptr;
     int logits_dtype = NCNN_MOE_LOGITS_F32;
     uint32_t logits_rows = 0;
@@ -1129,19 +1130,30 @@ int ncnn_moe_hip_sampler_create(int device, uint32_t max_rows, uint32_t max_voca
     // room for stop ids: 64 per row, or one list as long as the vocabulary, whichever is more
     s->input_stop_capacity = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(rows * 64, max_vocab), 1u << 28));
     const size_t input_bytes = s->input_stops_offset + static_cast<size_t>(s->input_stop_capacity) * sizeof(int32_t);
-    CREATE_CHECK(hipHostMalloc(&s->input_block_host, input_bytes, hipHostMallocDefault));
-    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->input_block_mapped), s->input_block_host, 0));
     s->upload_capacity = std::min<size_t>(rows * s->logits_stride_f32 * sizeof(float), kUploadStaging);
+    // Pinned memory comes in two allocations (13 us and more each: a handle of 1 x 32,000 takes 88 us to create, 127 with one for each buffer).  The
+    // staging memory of uploads has one of its own: with the operands at its front the first call of a new handle took 25 us longer.
+    size_t pinned_bytes = 0;
+    const auto pinned_place = [&](size_t size) { return std::exchange(pinned_bytes, pinned_bytes + round_up(size, 256)); };
+    const size_t input_at = pinned_place(input_bytes);
+    const size_t results_at = pinned_place(rows * sizeof(ncnn_moe_sample_result));
+    const size_t verify_input_at = pinned_place(sizeof(ncnn_moe_hip_sampler::VerifyInput));
+    const size_t verify_output_at = pinned_place(sizeof(ncnn_moe_hip_sampler::VerifyOutput));
+    uint8_t* mapped = nullptr;
+    CREATE_CHECK(hipHostMalloc(&s->pinned_memory, pinned_bytes, hipHostMallocDefault));
+    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&mapped), s->pinned_memory, 0));
+    s->input_block_host = s->pinned_memory + input_at;
+    s->input_block_mapped = mapped + input_at;
     CREATE_CHECK(hipHostMalloc(&s->upload_host, s->upload_capacity + sizeof(uint32_t), hipHostMallocDefault));
     CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->upload_mapped), s->upload_host, 0));
     s->upload_done_host = reinterpret_cast<uint32_t*>(s->upload_host + s->upload_capacity); // (rows are whole vectors)
     s->upload_done_mapped = reinterpret_cast<uint32_t*>(s->upload_mapped + s->upload_capacity);
-    CREATE_CHECK(hipHostMalloc(&s->results_host, rows * sizeof(ncnn_moe_sample_result), hipHostMallocDefault));
-    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->results_host_device), s->results_host, 0));
-    CREATE_CHECK(hipHostMalloc(&s->verify_input_host, sizeof(ncnn_moe_hip_sampler::VerifyInput), hipHostMallocDefault));
-    CREATE_CHECK(hipHostMalloc(&s->verify_output_host, sizeof(ncnn_moe_hip_sampler::VerifyOutput), hipHostMallocDefault));
-    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->verify_input_mapped), s->verify_input_host, 0));
-    CREATE_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&s->verify_output_mapped), s->verify_output_host, 0));
+    s->results_host = reinterpret_cast<ncnn_moe_sample_result*>(s->pinned_memory + results_at);
+    s->results_host_device = reinterpret_cast<ncnn_moe_sample_result*>(mapped + results_at);
+    s->verify_input_host = reinterpret_cast<ncnn_moe_hip_sampler::VerifyInput*>(s->pinned_memory + verify_input_at);
+    s->verify_input_mapped = reinterpret_cast<ncnn_moe_hip_sampler::VerifyInput*>(mapped + verify_input_at);
+    s->verify_output_host = reinterpret_cast<ncnn_moe_hip_sampler::VerifyOutput*>(s->pinned_memory + verify_output_at);
+    s->verify_output_mapped = reinterpret_cast<ncnn_moe_hip_sampler::VerifyOutput*>(mapped + verify_output_at);
     CREATE_CHECK(hipStreamSynchronize(s->stream));
 #undef CREATE_CHECK
     *out = s;
@@ -1171,16 +1183,10 @@ void ncnn_moe_hip_sampler_destroy(ncnn_moe_hip_sampler* s)
         (void)hipEventDestroy(s->cut_done);
     if (s->device_memory != nullptr)
         (void)hipFree(s->device_memory);
-    if (s->input_block_host != nullptr)
-        (void)hipHostFree(s->input_block_host);
+    if (s->pinned_memory != nullptr)
+        (void)hipHostFree(s->pinned_memory);
     if (s->upload_host != nullptr)
         (void)hipHostFree(s->upload_host);
-    if (s->results_host != nullptr)
-        (void)hipHostFree(s->results_host);
-    if (s->verify_input_host != nullptr)
-        (void)hipHostFree(s->verify_input_host);
-    if (s->verify_output_host != nullptr)
-        (void)hipHostFree(s->verify_output_host);
     delete s;
 }
 
