@@ -925,8 +925,8 @@ __device__ __forceinline__ uint32_t fit_plan(BinPlan& plan, const uint32_t (&fro
 //             odd steps of that value; then bit step % 32 for a term half way between `step` and the next.  The kWideBins bins
 //             from wide_first on have the same with 64 and 128 bits
 // What bounds it: instructions, and with two waves a SIMD the trips to LDS for the bins' entries: there (kFewWaves) four terms look theirs up
-// together, and their steps are made without a branch (a part of 9,500 terms by 512 threads, warm 5.0 -> 4.3 us, where the
-// instructions are new 5.7 -> 4.7; without the additions to the bins 4.9, without the parities 3.4).  With eight waves a SIMD branches cost less than what
+// together, and their steps are made without a branch (a part of 9,500 terms by 512 threads, warm 4.95 -> 4.45 us, where the
+// instructions are new 5.55 -> 5.05; of the 4.95, 0.1 were the additions to the bins and 1.5 the parities).  With eight waves a SIMD branches cost less than what
 // they pass by (512 workgroups of 1,024 threads, 30,400 terms each, 17.0 with a branch, 18.0 without).  Steps are made from the terms scaled to ulps of the
 // sum, with shifts of their mantissas both took 0.3 to 0.8 us more.
 template <int PHASE, int THREADS, bool ACROSS>
@@ -935,8 +935,8 @@ __device__ __forceinline__ void add_bin_steps(
     uint32_t* entries, uint32_t* steps, uint32_t* ties, uint32_t* masks, uint32_t wide_first, float* list_terms, uint32_t* list_tokens, bool near, int tid)
 {
     constexpr bool kFewWaves = THREADS < kBinThreads;
-    // (five, where there are registers, so that parts of up to 10,240 terms take one trip: 8 rows of 131,200 to 163,000 and of 151,936 the same within 0.6 %
-    // either way, 16 of 151,936 91.8 with four and 92.7 with five, 40 of 32,000 62.3 and 62.7)
+    // (five, where there are registers, gain where they save a trip only: by 512 threads parts of 8,193 to 10,240 terms 5.1 -> 4.85 us, of 2,000 1.39 -> 1.43,
+    // of 6,250 3.64 -> 3.69, of 12,500 6.26 -> 6.31)
     constexpr int kLoads = 4;
     const uint32_t bytes = (s.end + 7u) / 8u * 32u;
     const uint32_t first = s.first * 2u, last = s.last * 2u;
